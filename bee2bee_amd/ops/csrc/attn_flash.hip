@@ -1,0 +1,382 @@
+// Causal prompt attention: whole packed prompts, and query chunks against the
+// paged history (query row j of sequence b stands at hist + j, hist =
+// seq_lens[b] - its query length; the chunk's own keys are in the pages).
+//
+// What bounds it is the CU: the matrix cores, the exponentials beside them
+// and the LDS reads that feed them, about equal in time.
+//  * A workgroup takes the query rows of ALL heads that share a key head: row
+//    = position * group + head, so that any group size and any chunk length
+//    fill the 32-row tiles, and a key tile is read once for the group.
+//  * Scores are computed transposed, S^T = K Q^T on 32x32x16 tiles: a lane
+//    holds 16 keys of ONE query row, so that the row's maximum and sum are
+//    in-lane (one exchange with lane + 32), and its weights are, as they
+//    stand, the right operand of O^T = V^T P^T: no trip through LDS. That
+//    product takes its 16 keys in the order the score tile holds them, which
+//    the transposing LDS read of V follows.
+//  * Keys and values are staged in LDS row-major, 16-byte chunks xor-ed by
+//    the key so that both kinds of reads spread over the banks, two buffers,
+//    the next tile's global reads in flight over the current tile's products.
+//  * The running maximum is raised only by a score FL_SLACK powers of two
+//    above it: most tiles leave the sums as they are. Weights stay below
+//    2^FL_SLACK, whose bf16 rounding is as fine, and sums are fp32.
+// Scores are scaled in fp32 (queries enter the product unrounded). The kernel
+// before it (16-row tiles, weights and V transposed through LDS by 2-byte
+// writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
+// of 28 heads on 16384 keys 897 us instead of 5240 (940 TFLOP/s), 2048 tokens
+// of 32 heads 63 us instead of 386 (540), nine prompts of 112 to 901 tokens
+// 38 us instead of 140. Fetching key fragments two steps ahead by hand
+// changed nothing (979 us against 928 in one run).
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) short short4v;
+typedef __attribute__((ext_vector_type(2))) unsigned int uint2v;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((address_space(3))) short4v lds_short4v;
+
+constexpr int FL_KT = 64;   // keys per staged tile
+// a row's running maximum is raised only by a score this far (in powers of
+// two) above it
+constexpr float FL_SLACK = 8.f;
+
+// the values of lanes l and l + 32, in both: .x the lower lane's
+DEV_INLINE float2v lane_pair(float x) {
+    const unsigned int u = __builtin_bit_cast(unsigned int, x);
+    const uint2v r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    // (a bit cast of a vector's element would take element 0)
+    const unsigned int r0 = r[0], r1 = r[1];
+    return float2v{__builtin_bit_cast(float, r0),
+                   __builtin_bit_cast(float, r1)};
+}
+DEV_INLINE float pair_max(float x) {
+    const float2v p = lane_pair(x);
+    return fmaxf(p.x, p.y);
+}
+DEV_INLINE float pair_sum(float x) {
+    const float2v p = lane_pair(x);
+    return p.x + p.y;
+}
+
+template <int HD, int RW, int KSP, bool PAGED, typename KVT>
+__global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
+    const unsigned short* __restrict__ q, const KVT* __restrict__ k,
+    const KVT* __restrict__ v, const int* __restrict__ cu,
+    const int* __restrict__ block_table, const int* __restrict__ seq_lens,
+    unsigned short* __restrict__ out, int nq, int nkv, long s_q, long s_k,
+    long s_v, int W, int bs, int pairs, float scale_log2) {
+    constexpr int NW = RW * KSP;           // waves
+    constexpr int ROWS = RW * 32;          // query rows of a workgroup
+    constexpr int NF = 2 / KSP;            // 32-key tiles of a wave's step
+    constexpr int KS = HD / 16;            // k steps of a score tile
+    constexpr int DT = HD / 32;            // output tiles of 32 coordinates
+    constexpr int CPR = HD / 8;            // 16-byte chunks of a key row
+    constexpr int RB = HD * 2;             // bytes of a key row
+    constexpr int RPT = NW * 64 / CPR;     // key rows staged at once
+    constexpr int NST = FL_KT / RPT;       // staging steps of a tile
+    constexpr int TILE = FL_KT * RB;       // bytes of a K or V tile
+    static_assert(FL_KT % RPT == 0, "whole staging steps");
+
+    // workgroups go round the 8 dies in turn: heads fastest, so that a key
+    // head stays on few of them, long rows of tiles first, and the sequences
+    // rotated from one tile to the next, so that a long one is on all
+    const int nseq = pairs / nkv;
+    const int up = blockIdx.x / pairs, tile = gridDim.x / pairs - 1 - up;
+    const int seq =
+        (blockIdx.x % pairs / nkv + (nkv % 8 ? up : 0)) % nseq;
+    const int kvh = blockIdx.x % nkv;
+    const int G = nq / nkv;
+    const int s0 = cu[seq], QL = cu[seq + 1] - s0;
+    const int L = PAGED ? seq_lens[seq] : QL;
+    const int hist = L - QL;
+    const int row0 = tile * ROWS;
+    if (row0 >= QL * G) return;
+    const int* bt = PAGED ? block_table + (long)seq * W : nullptr;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31, hi = lane >> 5;
+    const int rw = KSP == 1 ? wid : wid % RW;     // row block of the wave
+    const int f0 = KSP == 1 ? 0 : wid / RW;       // its first 32-key tile
+
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    // two buffers of a K and a V tile each
+
+    // ---- this lane's query row
+    const int R = row0 + rw * 32 + lr;
+    const bool row_ok = R < QL * G;
+    const int pos = row_ok ? R / G : QL - 1;       // chunk position
+    const int head = kvh * G + (row_ok ? R % G : G - 1);
+    bf16x8 bq[KS];
+    {
+        const unsigned short* qr = q + (long)(s0 + pos) * s_q + (long)head * HD;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            bq[ks] = *reinterpret_cast<const bf16x8*>(qr + ks * 16 + hi * 8);
+    }
+    const int see = hist + pos;                    // last key this row sees
+    // of the wave: the earliest row's last key, and the end of all its keys
+    const int wr0 = row0 + rw * 32;
+    const int w_first = hist + min(wr0, QL * G - 1) / G;
+    const int w_end =
+        wr0 < QL * G ? hist + min(wr0 + 31, QL * G - 1) / G + 1 : 0;
+    const int kv_end = hist + min(row0 + ROWS - 1, QL * G - 1) / G + 1;
+
+    // ---- staging: thread -> (key row, chunk)
+    const int st_row = tid / CPR, st_c = tid % CPR;
+    bf16x8 rk[NST], rv[NST];
+    // pages of whole tiles: a tile's page is one scalar look-up
+    const bool whole_pages = PAGED && bs % FL_KT == 0;
+    auto load_tile = [&](int kb) {
+        long tile_off = 0;
+        if (whole_pages)
+            tile_off =
+                (((long)bt[kb / bs] * nkv + kvh) * bs + kb % bs) * HD;
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+            const int key = min(kb + st_row + i * RPT, kv_end - 1);
+            if (PAGED) {
+                const long off =
+                    (whole_pages
+                         ? tile_off + (long)(key - kb) * HD
+                         : (((long)bt[key / bs] * nkv + kvh) * bs +
+                            key % bs) * HD) +
+                    st_c * 8;
+                rk[i] = load_kv8_bf16(k + off);
+                rv[i] = load_kv8_bf16(v + off);
+            } else {
+                rk[i] = load_kv8_bf16(k + (long)(s0 + key) * s_k +
+                                      (long)kvh * HD + st_c * 8);
+                rv[i] = load_kv8_bf16(v + (long)(s0 + key) * s_v +
+                                      (long)kvh * HD + st_c * 8);
+            }
+        }
+    };
+    constexpr int VMASK = HD == 128 ? 7 : 3;
+    auto store_tile = [&](int buf) {
+        char* kd = smem + buf * 2 * TILE;
+        char* vd = kd + TILE;
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+            const int row = st_row + i * RPT;
+            *reinterpret_cast<bf16x8*>(kd + row * RB +
+                                       ((st_c ^ (row & 7)) << 4)) = rk[i];
+            *reinterpret_cast<bf16x8*>(
+                vd + row * RB + ((st_c ^ (2 * (row & VMASK))) << 4)) = rv[i];
+        }
+    };
+
+    // ---- fragment addresses
+    // K (rows = keys): lane reads key lr of a 32-key tile, chunk 2 ks + hi
+    const int k_base = lr * RB;
+    const int k_sw = lr & 7;
+    // V^T (rows = coordinates) through the transposing read: the 16 lanes of
+    // a group address 4 keys x 16 coordinates
+    const int v_key = 4 * hi + ((lane >> 2) & 3);
+    const int v_c0 = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+    const int v_sw = 2 * (v_key & VMASK);
+    int v_off[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+        v_off[d] = TILE + v_key * RB + (((d * 4 + v_c0) ^ v_sw) << 4) +
+                   (lane & 1) * 8;
+
+    f32x16 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
+    float m = -1e30f, l = 0.f;
+
+    if (kv_end > 0) {
+        load_tile(0);
+        store_tile(0);
+    }
+    int buf = 0;
+    for (int kb = 0; kb < kv_end; kb += FL_KT, buf ^= 1) {
+        __syncthreads();
+        const bool more = kb + FL_KT < kv_end;
+        if (more) load_tile(kb + FL_KT);
+        if (kb < w_end) {
+            const char* base = smem + buf * 2 * TILE;
+            // ---- S^T = K Q^T: column = query row, rows = keys
+            f32x16 s[NF];
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[f][r] = 0.f;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const bf16x8 ak = *reinterpret_cast<const bf16x8*>(
+                        base + (f0 + f) * 32 * RB + k_base +
+                        (((ks * 2 + hi) ^ k_sw) << 4));
+                    s[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        ak, bq[ks], s[f], 0, 0, 0);
+                }
+            }
+            if (kb + FL_KT - 1 > w_first) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key =
+                            kb + (f0 + f) * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+                        if (key > see) s[f][r] = -INFINITY;
+                    }
+            }
+            // ---- online softmax, in powers of two
+            float mx = s[0][0];
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[f][r]);
+            mx = pair_max(mx) * scale_log2;
+            if (__any(mx > m + FL_SLACK)) {
+                const float mn = fmaxf(m, mx);
+                const float alpha = __builtin_amdgcn_exp2f(m - mn);
+                m = mn;
+                l *= alpha;
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+            }
+            bf16x8 bp[NF * 2];
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float p = __builtin_amdgcn_exp2f(
+                        fmaf(s[f][r], scale_log2, -m));
+                    l += p;
+                    bp[f * 2 + r / 8][r % 8] = (__bf16)p;
+                }
+            // ---- O^T += V^T P^T; the keys of a step in the order the score
+            // tile holds them: 4 hi + {0..3}, then 8 + 4 hi + {0..3}
+#pragma unroll
+            for (int st = 0; st < NF * 2; ++st)
+#pragma unroll
+                for (int d = 0; d < DT; ++d) {
+                    const char* va =
+                        base + v_off[d] + (f0 * 2 + st) * 16 * RB;
+                    const short4v a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (lds_short4v*)va);
+                    const short4v a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (lds_short4v*)(va + 8 * RB));
+                    const short8 av = __builtin_shufflevector(
+                        a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, av), bp[st], o[d], 0, 0, 0);
+                }
+        }
+        if (more) store_tile(buf ^ 1);
+    }
+
+    l = pair_sum(l);
+    if (KSP == 2) {
+        // the halves' sums meet in LDS (over the tiles): [row block][lane]
+        // columns of DT * 16 sums, then m and l
+        float* mg = reinterpret_cast<float*>(smem) + rw * (DT * 16 + 2) * 64 +
+                    lane;
+        __syncthreads();
+        if (f0 == 1) {
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mg[(d * 16 + r) * 64] = o[d][r];
+            mg[DT * 16 * 64] = m;
+            mg[(DT * 16 + 1) * 64] = l;
+        }
+        __syncthreads();
+        if (f0 == 1) return;
+        const float m1 = mg[DT * 16 * 64];
+        const float mn = fmaxf(m, m1);
+        const float a0 = __builtin_amdgcn_exp2f(m - mn);
+        const float a1 = __builtin_amdgcn_exp2f(m1 - mn);
+        l = l * a0 + mg[(DT * 16 + 1) * 64] * a1;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                o[d][r] = o[d][r] * a0 + mg[(d * 16 + r) * 64] * a1;
+    }
+    if (!row_ok) return;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    unsigned short* orow = out + ((long)(s0 + pos) * nq + head) * HD;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            short4v w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                w[e] = (short)f2bf(o[d][r4 * 4 + e] * inv);
+            *reinterpret_cast<short4v*>(orow + d * 32 + r4 * 8 + hi * 4) = w;
+        }
+}
+
+// ------------------------------------------------------------- launchers
+
+static int flash_smem(int hd, int rw, int ksp) {
+    const int tiles = 4 * FL_KT * hd * 2;
+    const int merge = ksp == 2 ? rw * (hd / 2 + 2) * 64 * 4 : 0;
+    return tiles > merge ? tiles : merge;
+}
+
+// Shape of a workgroup by how many of 256 rows the step fills (`full`,
+// T * nq / 256; a CU holds one such workgroup at head size 128, two at 64):
+// 256 rows read a key tile from memory least often and win once there are
+// about two rounds of them; with fewer, 128 rows balance better; with less
+// than a chip of those, 64 rows whose two wave pairs share a tile's keys.
+// Measured (us; 256 / 128 / 64 rows), head size 128: full 1024 600/674/735,
+// 448 (with 12k cached) 897/1056/1146, 426 (nine short prompts) 39/38/50,
+// 256 70/63/63, 128 37/31/26, 64 23/18/15; head size 64: 2048 333/362/405,
+// 750 48/47/63, 125 25/21/17.
+static int flash_shape(int hd, long full) {
+    if (full >= (hd == 128 ? 440 : 1024)) return 0;
+    return full >= (hd == 128 ? 150 : 230) ? 1 : 2;
+}
+
+#define FL_ONE(HDV, RWV, KSPV, PG, KVT)                                       \
+    hipLaunchKernelGGL(                                                       \
+        (attn_flash_kernel<HDV, RWV, KSPV, PG, KVT>),                         \
+        dim3((unsigned)((rows + RWV * 32 - 1) / (RWV * 32) * pairs)),         \
+        dim3(RWV * KSPV * 64), flash_smem(HDV, RWV, KSPV), stream, q,         \
+        (const KVT*)k, (const KVT*)v, cu, block_table, seq_lens, out, nq,     \
+        nkv, s_q, s_k, s_v, W, bs, pairs, scale * LOG2E)
+#define FL_HD(HDV, PG, KVT)                                                   \
+    do {                                                                      \
+        if (shape == 0) FL_ONE(HDV, 8, 1, PG, KVT);                           \
+        else if (shape == 1) FL_ONE(HDV, 4, 1, PG, KVT);                      \
+        else FL_ONE(HDV, 2, 2, PG, KVT);                                      \
+    } while (0)
+
+constexpr float LOG2E = 1.44269504088896340736f;
+
+// Whole packed prompts, or (block_table given) query chunks whose keys come
+// from the pages only, bf16 or fp8 bytes. T: query tokens of the step. Head
+// size 64 or 128 and a positive scale (a row's maximum is taken before it);
+// nonzero for any other.
+extern "C" int launch_attn_flash(
+    const unsigned short* q, const void* k, const void* v, const int* cu,
+    const int* block_table, const int* seq_lens, unsigned short* out, long T,
+    int nseq, int nq, int nkv, int hd, long s_q, long s_k, long s_v, int W,
+    int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
+    if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
+    if (nseq == 0 || max_qlen <= 0) return 0;
+    const int pairs = nseq * nkv;
+    const long rows = (long)max_qlen * (nq / nkv);
+    const int shape = flash_shape(hd, T * nq / 256);
+    if (!block_table) {
+        if (hd == 128) FL_HD(128, false, unsigned short);
+        else FL_HD(64, false, unsigned short);
+    } else if (fp8) {
+        if (hd == 128) FL_HD(128, true, unsigned char);
+        else FL_HD(64, true, unsigned char);
+    } else {
+        if (hd == 128) FL_HD(128, true, unsigned short);
+        else FL_HD(64, true, unsigned short);
+    }
+    return 0;
+}
+#undef FL_HD
+#undef FL_ONE

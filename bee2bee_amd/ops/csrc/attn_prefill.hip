@@ -7,8 +7,9 @@
 // hist + j where hist = seq_lens[b] - query_len[b]). The chunk's own K/V
 // were stored to the cache by kv_store before this kernel runs.
 //
-// Two kernels:
-//  * attn_prefill_mfma — the production path for head_dim 64/128: per
+// The plain form with head_dim 64/128 is in attn_flash.hip. Two kernels here:
+//  * attn_prefill_mfma — head_dim 64/128: chunks of a few tokens, and the
+//    forms with sinks, windows, gates, biases and mixed heads: per
 //    workgroup 4 waves x 16 q-rows (64-row Q tile), 32-key K/V tiles staged
 //    in LDS (+8-element row padding => conflict-free ds_read_b128, guide
 //    T2/G4), QK^T and P.V on v_mfma_f32_16x16x32_bf16, online softmax in
@@ -27,17 +28,6 @@ __device__ __forceinline__ float kv_elem_f32(unsigned short x) {
 }
 __device__ __forceinline__ float kv_elem_f32(unsigned char x) {
     return fp8x2_2f((unsigned short)x).x;
-}
-__device__ __forceinline__ bf16x8 load_kv8_bf16(const unsigned short* p) {
-    return *reinterpret_cast<const bf16x8*>(p);
-}
-__device__ __forceinline__ bf16x8 load_kv8_bf16(const unsigned char* p) {
-    float f[8];
-    load_fp8x8(p, f);
-    bf16x8 r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (__bf16)f[e];
-    return r;
 }
 
 // ------------------------------------------------------------------ basic
@@ -463,27 +453,22 @@ static int prefill_mfma_smem(int hd, int hilo = 0) {
     return (k_bytes > p_bytes ? k_bytes : p_bytes) + vt_bytes;
 }
 
+// attn_flash.hip: head size 64 or 128 and a positive scale, nonzero otherwise
+extern "C" int launch_attn_flash(
+    const unsigned short* q, const void* k, const void* v, const int* cu,
+    const int* block_table, const int* seq_lens, unsigned short* out, long T,
+    int nseq, int nq, int nkv, int hd, long s_q, long s_k, long s_v, int W,
+    int bs, int max_qlen, float scale, int fp8, hipStream_t stream);
+
 extern "C" void launch_attn_prefill(
     const unsigned short* q, const unsigned short* k, const unsigned short* v,
-    const int* cu, unsigned short* out, int nseq, int nq, int nkv, int hd,
-    long s_q, long s_k, long s_v, int max_seqlen, float scale, int causal,
-    hipStream_t stream) {
-    if ((hd == 64 || hd == 128) && causal) {
-        const int tiles = (max_seqlen + PF_TM - 1) / PF_TM;
-        dim3 grid(tiles, nq, nseq);
-        const int smem = prefill_mfma_smem(hd);
-        if (hd == 128)
-            hipLaunchKernelGGL((attn_prefill_mfma<128, false, unsigned short>),
-                               grid, dim3(256), smem, stream, q, k, v, cu,
-                               nullptr, nullptr, out, nq, nkv, s_q, s_k, s_v,
-                               0, 0, scale, nullptr, 1.f, (long)nq * hd);
-        else
-            hipLaunchKernelGGL((attn_prefill_mfma<64, false, unsigned short>),
-                               grid, dim3(256), smem, stream, q, k, v, cu,
-                               nullptr, nullptr, out, nq, nkv, s_q, s_k, s_v,
-                               0, 0, scale, nullptr, 1.f, (long)nq * hd);
+    const int* cu, unsigned short* out, long T, int nseq, int nq, int nkv,
+    int hd, long s_q, long s_k, long s_v, int max_seqlen, float scale,
+    int causal, hipStream_t stream) {
+    if (causal && launch_attn_flash(q, k, v, cu, nullptr, nullptr, out, T,
+                                    nseq, nq, nkv, hd, s_q, s_k, s_v, 0, 1,
+                                    max_seqlen, scale, 0, stream) == 0)
         return;
-    }
     dim3 grid(nq, nseq);
     const int smem = (hd + WAVE) * 4;
     hipLaunchKernelGGL((attn_prefill_basic<false, unsigned short>), grid,
@@ -498,8 +483,14 @@ extern "C" void launch_attn_prefill(
 extern "C" void launch_attn_prefill_paged(
     const unsigned short* q, const void* k_cache, const void* v_cache,
     const int* cu, const int* block_table, const int* seq_lens,
-    unsigned short* out, int nseq, int nq, int nkv, int hd, long s_q, int W,
-    int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
+    unsigned short* out, long T, int nseq, int nq, int nkv, int hd, long s_q,
+    int W, int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
+    // (a few tokens a sequence fill a tile of neither kernel)
+    if (max_qlen * (nq / nkv) > 32 &&
+        launch_attn_flash(q, k_cache, v_cache, cu, block_table, seq_lens, out,
+                          T, nseq, nq, nkv, hd, s_q, 0, 0, W, bs, max_qlen,
+                          scale, fp8, stream) == 0)
+        return;
 #define PFP_LAUNCH(KVT)                                                        \
     do {                                                                       \
         const KVT* kc = reinterpret_cast<const KVT*>(k_cache);                 \

@@ -70,6 +70,19 @@ __device__ __forceinline__ void store_bf16x8(unsigned short* p, const float* in)
     *reinterpret_cast<short8*>(p) = raw;
 }
 
+// 8 cache elements (bf16, or OCP fp8 bytes widened) as a bf16 fragment
+__device__ __forceinline__ bf16x8 load_kv8_bf16(const unsigned short* p) {
+    return *reinterpret_cast<const bf16x8*>(p);
+}
+__device__ __forceinline__ bf16x8 load_kv8_bf16(const unsigned char* p) {
+    float f[8];
+    load_fp8x8(p, f);
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = (__bf16)f[e];
+    return r;
+}
+
 // full-wave (64-lane) reductions via xor shuffles
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll

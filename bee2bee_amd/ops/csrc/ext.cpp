@@ -39,12 +39,12 @@ void launch_attn_decode(const unsigned short*, const void*, const void*,
                         int, int, int, long, float, int, hipStream_t);
 void launch_attn_prefill(const unsigned short*, const unsigned short*,
                          const unsigned short*, const int*, unsigned short*,
-                         int, int, int, int, long, long, long, int, float,
-                         int, hipStream_t);
+                         long, int, int, int, int, long, long, long, int,
+                         float, int, hipStream_t);
 void launch_attn_prefill_paged(const unsigned short*, const void*,
                                const void*, const int*, const int*,
-                               const int*, unsigned short*, int, int, int,
-                               int, long, int, int, int, float, int,
+                               const int*, unsigned short*, long, int, int,
+                               int, int, long, int, int, int, float, int,
                                hipStream_t);
 void launch_mfma_probe(const unsigned short*, const unsigned short*, float*,
                        hipStream_t);
@@ -290,8 +290,8 @@ Tensor attn_prefill(const Tensor& q, const Tensor& k, const Tensor& v,
     TORCH_CHECK(v.stride(2) == 1 && v.stride(1) == hd);
     Tensor out = torch::empty({T, nq, hd}, q.options());
     launch_attn_prefill(bf16p(q), bf16p(k), bf16p(v),
-                        cu_seqlens.data_ptr<int>(), bf16p_mut(out), nseq, nq,
-                        nkv, hd, q.stride(0), k.stride(0), v.stride(0),
+                        cu_seqlens.data_ptr<int>(), bf16p_mut(out), T, nseq,
+                        nq, nkv, hd, q.stride(0), k.stride(0), v.stride(0),
                         (int)max_seqlen, (float)scale, causal ? 1 : 0,
                         stream());
     return out;
@@ -321,8 +321,8 @@ Tensor attn_prefill_paged(const Tensor& q, const Tensor& k_cache,
     launch_attn_prefill_paged(bf16p(q), k_cache.data_ptr(),
                               v_cache.data_ptr(), cu_q.data_ptr<int>(),
                               block_table.data_ptr<int>(),
-                              seq_lens.data_ptr<int>(), bf16p_mut(out), nseq,
-                              nq, nkv, hd, q.stride(0), W, bs, (int)max_qlen,
+                              seq_lens.data_ptr<int>(), bf16p_mut(out), T,
+                              nseq, nq, nkv, hd, q.stride(0), W, bs, (int)max_qlen,
                               (float)scale, fp8 ? 1 : 0, stream());
     return out;
 }

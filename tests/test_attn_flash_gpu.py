@@ -1,0 +1,107 @@
+"""The prompt-attention kernel (attn_flash.hip) at the edges of its tiles and
+of its three workgroup shapes, against the fp32 reference.
+
+Tolerance: a weight and an output element are rounded to bf16 once each
+(2^-9 relative), so an element is off by at most 2^-8 of the largest value;
+fp32 sums and exp2 add far less."""
+import pytest
+import torch
+
+from bee2bee_amd import ops
+from bee2bee_amd.ops import reference
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _qkv(T, nq, nkv, hd, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    qkv = torch.randn(T, (nq + 2 * nkv) * hd, generator=g,
+                      device=DEV).bfloat16()
+    q, k, v = qkv.split([nq * hd, nkv * hd, nkv * hd], -1)
+    return q.view(T, nq, hd), k.view(T, nkv, hd), v.view(T, nkv, hd)
+
+
+def _cu(lens):
+    return torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(),
+                        dtype=torch.int32, device=DEV)
+
+
+def _check(got, want, v):
+    assert torch.isfinite(got).all()
+    err = (got.float() - want.float()).abs().max().item()
+    assert err <= v.float().abs().max().item() * 2 ** -8, err
+
+
+@pytest.mark.parametrize("nq,nkv,hd,lens", [
+    (4, 4, 64, [1]), (4, 1, 128, [1, 63, 64, 65]), (7, 1, 128, [9, 10, 37]),
+    (32, 8, 64, [57, 0, 129]), (12, 12, 64, [31, 32, 33, 127, 128, 129]),
+    (24, 8, 128, [255, 256, 257]), (16, 1, 64, [2, 100]),
+    # 128- and 256-row workgroups
+    (28, 4, 128, [700, 513, 64, 300]), (32, 8, 128, [512] * 7 + [1]),
+    (12, 12, 64, [1000] * 6), (64, 8, 64, [513] * 8 + [63]),
+])
+def test_whole_prompts(nq, nkv, hd, lens):
+    q, k, v = _qkv(sum(lens), nq, nkv, hd, len(lens))
+    cu, scale = _cu(lens), 0.7 * hd ** -0.5
+    got = ops.attn_prefill(q, k, v, cu, max(lens), scale)
+    want = reference.attn_prefill(q.float(), k.float(), v.float(), cu,
+                                  max(lens), scale)
+    _check(got, want, v)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("nq,nkv,hd,lens,hist,bs", [
+    (32, 8, 128, [5, 5, 1], [1500, 255, 0], 256),
+    (28, 4, 128, [64, 40], [63, 64], 64), (32, 8, 64, [33, 2], [77, 1], 16),
+    (6, 2, 128, [40, 9], [100, 300], 24), (12, 12, 64, [130], [1000], 256),
+    (28, 4, 128, [2100], [500], 256), (32, 8, 128, [3600], [130], 256),
+])
+def test_chunks_against_pages(nq, nkv, hd, lens, hist, bs, fp8):
+    q, _, _ = _qkv(sum(lens), nq, nkv, hd, 3)
+    total = [a + b for a, b in zip(lens, hist)]
+    W = max(-(-n // bs) for n in total) + 1
+    nb = W * len(lens) + 2
+    g = torch.Generator(device=DEV).manual_seed(4)
+    table = torch.randperm(nb, generator=g, device=DEV)[: W * len(lens)]
+    table = table.int().view(len(lens), W)
+    kc = torch.randn(nb, nkv, bs, hd, generator=g, device=DEV).bfloat16()
+    vc = torch.randn(nb, nkv, bs, hd, generator=g, device=DEV).bfloat16()
+    if fp8:
+        kc = kc.to(torch.float8_e4m3fn).view(torch.uint8)
+        vc = vc.to(torch.float8_e4m3fn).view(torch.uint8)
+    cu, scale = _cu(lens), hd ** -0.5
+    lens_t = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    total_t = torch.tensor(total, dtype=torch.int32, device=DEV)
+    got = ops.attn_prefill_paged(q, kc, vc, table, total_t, cu, max(lens),
+                                 scale)
+    up = (lambda c: c.view(torch.float8_e4m3fn).float()) if fp8 else \
+        (lambda c: c.float())
+    want = reference.attn_decode_with_history(q.float(), up(kc), up(vc),
+                                              table, total_t, lens_t, scale)
+    _check(got, want, up(vc))
+
+
+def test_scores_that_climb():
+    """Scores that grow along the keys raise the running maximum tile by
+    tile, in steps below and above the kernel's slack."""
+    T, hd = 400, 128
+    q = torch.ones(T, 1, hd, device=DEV).bfloat16()
+    ramp = torch.arange(T, device=DEV, dtype=torch.float32)
+    for step in (0.02, 1.0):
+        k = (ramp * step / hd)[:, None, None].expand(T, 1, hd).bfloat16()
+        v = torch.randn(T, 1, hd, device=DEV).bfloat16()
+        got = ops.attn_prefill(q, k, v, _cu([T]), T, 1.0)
+        want = reference.attn_prefill(q.float(), k.float(), v.float(),
+                                      _cu([T]), T, 1.0)
+        _check(got, want, v)
+
+
+def test_a_scale_that_is_not_positive():
+    """Takes the plain kernel, as before."""
+    q, k, v = _qkv(70, 2, 1, 64, 9)
+    for scale in (0.0, -0.1):
+        got = ops.attn_prefill(q, k, v, _cu([70]), 70, scale)
+        want = reference.attn_prefill(q.float(), k.float(), v.float(),
+                                      _cu([70]), 70, scale)
+        _check(got, want, v)
