@@ -1,17 +1,8 @@
-// Paged GQA decode attention — three-stage flash-decoding.
-//
-// The decode step is memory-bound on KV reads (per key: 2*hd*2 B moved).
-// A single fused kernel could not reach the HBM roofline: its score phase
-// (lanes-over-keys) and PV phase (lanes-over-dims) have opposing register
-// needs, and together they pushed VGPRs past 100 -> 2 waves/SIMD -> too few
-// bytes in flight (measured 1.7-2.5 TB/s vs 6.0 TB/s for each access
-// pattern probed in isolation — see probe.hip bw_* kernels). Splitting into
-// per-chunk kernels keeps each at <=64 VGPRs with deep independent-load
-// batches:
+// Paged GQA decode attention for head sizes other than 64 and 128 (those are
+// attn_stream.hip's, at a positive scale) — three-stage flash-decoding:
 //   1. attn_scores:  S = q.K^T + chunk-level softmax -> p, (m,l) scratch
 //   2. attn_pv:      partial_o = p.V per chunk (p from scratch, LDS-staged)
 //   3. attn_combine: merge chunk partials, normalize, write bf16 out
-// Scratch p traffic is ~3% of KV traffic.
 //
 // Replaces: the reference's decode path inside transformers.generate()
 // (bee2bee/hf.py:84-108). Numerics reference: ops/reference.py attn_decode.
@@ -52,95 +43,7 @@ __device__ __forceinline__ float2v kv_pair_f32(kv_pair_t<unsigned char> p) {
     return fp8x2_2f(w);
 }
 
-// MFMA fragment plumbing for the scores kernel: bf16 caches feed the bf16
-// MFMA; fp8 caches feed v_mfma_f32_16x16x32_fp8_fp8 DIRECTLY (same lane
-// map, hardware-verified by test_mfma_fp8_fragment_map) — K bytes go
-// straight from the load into the matrix op, no convert VALU. q is
-// quantized to e4m3 once at fragment setup (the fp8 cache mode is already
-// approximate; documented).
-template <typename KVT> struct kfrag_of { using type = bf16x8; };
-template <> struct kfrag_of<unsigned char> { using type = long; };
-template <typename KVT>
-__device__ __forceinline__ typename kfrag_of<KVT>::type load_kfrag(
-    const KVT* p) {
-    return *reinterpret_cast<const typename kfrag_of<KVT>::type*>(p);
-}
-__device__ __forceinline__ bf16x8 qfrag_from_lds_bf16(
-    const unsigned short* p) {
-    return *reinterpret_cast<const bf16x8*>(p);
-}
-__device__ __forceinline__ long qfrag_from_lds_fp8(const unsigned short* p) {
-    unsigned short w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        w[i] = f2fp8x2(bf2f(p[2 * i]), bf2f(p[2 * i + 1]));
-    long r;
-    unsigned short* rp = reinterpret_cast<unsigned short*>(&r);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rp[i] = w[i];
-    return r;
-}
-template <typename KVT>
-__device__ __forceinline__ typename kfrag_of<KVT>::type qfrag_from_lds(
-    const unsigned short* p);
-template <>
-__device__ __forceinline__ bf16x8 qfrag_from_lds<unsigned short>(
-    const unsigned short* p) {
-    return qfrag_from_lds_bf16(p);
-}
-template <>
-__device__ __forceinline__ long qfrag_from_lds<unsigned char>(
-    const unsigned short* p) {
-    return qfrag_from_lds_fp8(p);
-}
-__device__ __forceinline__ f32x4 mfma_kq(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4 mfma_kq(long a, long b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a, b, c, 0, 0, 0);
-}
-
-template <typename KVT>
-__device__ __forceinline__ float2v load_kv_f32x2(const KVT* p);
-template <>
-__device__ __forceinline__ float2v load_kv_f32x2(const unsigned short* p) {
-    const short2v v = *reinterpret_cast<const short2v*>(p);
-    return float2v{bf2f((unsigned short)v[0]), bf2f((unsigned short)v[1])};
-}
-template <>
-__device__ __forceinline__ float2v load_kv_f32x2(const unsigned char* p) {
-    return fp8x2_2f(*reinterpret_cast<const unsigned short*>(p));
-}
-
 // ------------------------------------------------------------ stage 1: S
-// Whole K row staged into registers (HD/8 independent 16 B loads in one
-// burst), then G dot products against the LDS-held q. Compile-time HD keeps
-// the row array in registers (a runtime bound would spill it to scratch).
-template <int G, int HD, typename KVT>
-__device__ __forceinline__ void score_row(const KVT* kr,
-                                          const unsigned short* q_s,
-                                          float* s) {
-    bf16x8 krow[HD / 8];
-#pragma unroll
-    for (int ii = 0; ii < HD / 8; ++ii)
-        krow[ii] = load_kv_bf16x8<KVT>(kr + ii * 8);
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-        for (int ii = 0; ii < HD / 8; ++ii) {
-            const short8 qraw =
-                *reinterpret_cast<const short8*>(q_s + g * HD + ii * 8);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                s[g] = fmaf((float)krow[ii][j],
-                            bf2f((unsigned short)qraw[j]), s[g]);
-        }
-        // stop the scheduler hoisting every g's LDS q-reads to the top
-        // (otherwise G=4/HD=128 allocates 256 VGPRs -> 1 wave/SIMD)
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
 template <int G, typename KVT>
 __global__ __launch_bounds__(DEC_BLOCK) void attn_scores_kernel(
     const unsigned short* __restrict__ q,        // [B, nq, hd] (strided)
@@ -189,22 +92,16 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_scores_kernel(
             k_cache + (((long)page * nkv + kvh) * bs + key % bs) * hd;
 #pragma unroll
         for (int g = 0; g < G; ++g) s[g] = 0.f;
-        if (hd == 128) {
-            score_row<G, 128, KVT>(kr, q_s, s);
-        } else if (hd == 64) {
-            score_row<G, 64, KVT>(kr, q_s, s);
-        } else {
-            for (int d = 0; d < hd; d += 8) {  // tail models (hd 16/24/...)
-                const bf16x8 kraw = load_kv_bf16x8<KVT>(kr + d);
+        for (int d = 0; d < hd; d += 8) {
+            const bf16x8 kraw = load_kv_bf16x8<KVT>(kr + d);
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const short8 qraw =
-                        *reinterpret_cast<const short8*>(q_s + g * hd + d);
+            for (int g = 0; g < G; ++g) {
+                const short8 qraw =
+                    *reinterpret_cast<const short8*>(q_s + g * hd + d);
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        s[g] = fmaf((float)kraw[j],
-                                    bf2f((unsigned short)qraw[j]), s[g]);
-                }
+                for (int j = 0; j < 8; ++j)
+                    s[g] = fmaf((float)kraw[j],
+                                bf2f((unsigned short)qraw[j]), s[g]);
             }
         }
     }
@@ -263,166 +160,6 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_scores_kernel(
     }  // chunk loop
 }
 
-
-// MFMA variant of stage 1 (hd 64/128): the G dot products per key run on
-// the matrix pipe as S^T tiles = K_tile(16 keys) x q^T(16 cols, G used).
-// A-fragment rows map exactly to "lane reads its key row's 16 B segment",
-// so K streams from HBM straight into MFMA operands — no LDS staging, no
-// VALU fma chains, ~70 VGPRs -> high occupancy.
-// Fragment maps (verified on HW by tests/test_ops_gpu.py::test_mfma_fragment_map):
-//   A (16x32): lane = row (l&15), k = (l>>4)*8+e
-//   B (32x16): lane = col (l&15), k = (l>>4)*8+e
-//   C (16x16): lane = col (l&15), row = (l>>4)*4+r
-template <int G, int HD, typename KVT>
-__global__ __launch_bounds__(DEC_BLOCK) void attn_scores_mfma_kernel(
-    const unsigned short* __restrict__ q,
-    const KVT* __restrict__ k_cache,
-    const int* __restrict__ block_table,
-    const int* __restrict__ seq_lens,
-    unsigned short* __restrict__ p_out,  // bf16
-    float* __restrict__ part_ml,
-    int nkv, int W, int bs, int C, long q_stride, float scale) {
-    constexpr int KSTEPS = HD / 32;
-    constexpr int TILES = WAVE / 16;  // 4 key-tiles of 16 per wave
-    const int b = blockIdx.x;
-    const int kvh = blockIdx.y;
-    const int L = seq_lens[b];
-    if ((int)blockIdx.z * DEC_CHUNK >= L) return;
-    const int lane = threadIdx.x % WAVE;
-    const int wid = threadIdx.x / WAVE;
-    const int lg = lane >> 4;  // lane group 0..3
-    const int li = lane & 15;
-
-    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    unsigned short* q_s = reinterpret_cast<unsigned short*>(smem_raw);  // [G*HD]
-    float* red = reinterpret_cast<float*>(smem_raw + ((G * HD * 2 + 15) & ~15));
-    // red: [DEC_WAVES][G][2]
-
-    for (int i = threadIdx.x; i < G * HD; i += DEC_BLOCK) {
-        const int g = i / HD, d = i % HD;
-        q_s[i] = f2bf(
-            bf2f(q[(long)b * q_stride + (kvh * G + g) * (long)HD + d]) * scale);
-    }
-    __syncthreads();
-
-    // B-fragments: col = q head (li), k = dim lg*8+e within each kstep
-    using kfrag_t = typename kfrag_of<KVT>::type;
-    kfrag_t bq[KSTEPS];
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-        if (li < G) {
-            bq[ks] = qfrag_from_lds<KVT>(q_s + li * HD + ks * 32 + lg * 8);
-        } else {
-            bq[ks] = kfrag_t{};
-        }
-    }
-
-    const int* bt = block_table + (long)b * W;
-    // loop chunks with stride gridDim.z: the q staging amortizes and the
-    // per-chunk softmax tail overlaps other chunks' K bursts (single-chunk
-    // blocks measured ~66% memory-idle from cold-start/tail phases)
-    for (int chunk = blockIdx.z; chunk * DEC_CHUNK < L; chunk += gridDim.z) {
-    const int start = chunk * DEC_CHUNK;
-    const int wave_key0 = start + wid * WAVE;  // this wave covers 64 keys
-
-    // scores: all TILES*KSTEPS A-fragments issue before any MFMA (probe-
-    // style load batching: 16 independent 16 B loads in flight per wave)
-    f32x4 acc[TILES];
-    kfrag_t afr[TILES][KSTEPS];
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        const int key = wave_key0 + t * 16 + li;  // A row = li
-        const KVT* kr;
-        if (key < L) {
-            const int page = bt[key / bs];
-            kr = k_cache + (((long)page * nkv + kvh) * bs + key % bs) * HD;
-        } else {
-            // safe dummy row; masked later via the key<L score mask
-            kr = k_cache;
-        }
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
-            afr[t][ks] = load_kfrag<KVT>(kr + ks * 32 + lg * 8);
-    }
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        f32x4 c{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
-            c = mfma_kq(afr[t][ks], bq[ks], c);
-        acc[t] = c;
-    }
-
-    // this lane holds scores for g = li, keys (t*16 + lg*4 + r)
-    float sv[TILES * 4];
-    float lmax = -1e30f;
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int key = wave_key0 + t * 16 + lg * 4 + r;
-            float v = (key < L) ? acc[t][r] : -1e30f;
-            sv[t * 4 + r] = v;
-            lmax = fmaxf(lmax, v);
-        }
-    }
-    // reduce over the 4 lane groups holding the same g (stride-16 lanes)
-    lmax = fmaxf(lmax, __shfl_xor(lmax, 16));
-    lmax = fmaxf(lmax, __shfl_xor(lmax, 32));
-    if (lg == 0 && li < G) red[(wid * G + li) * 2] = lmax;
-    __syncthreads();
-    float M = -1e30f;  // chunk max for this lane's g
-    if (li < G) {
-#pragma unroll
-        for (int w2 = 0; w2 < DEC_WAVES; ++w2)
-            M = fmaxf(M, red[(w2 * G + li) * 2]);
-    }
-    float lsum = 0.f;
-#pragma unroll
-    for (int i = 0; i < TILES * 4; ++i) {
-        // round to bf16 BEFORE summing so l matches the p that PV consumes
-        const float pv =
-            (sv[i] <= -1e29f) ? 0.f : bf2f(f2bf(__expf(sv[i] - M)));
-        sv[i] = pv;
-        lsum += pv;
-    }
-    lsum += __shfl_xor(lsum, 16);
-    lsum += __shfl_xor(lsum, 32);
-    __syncthreads();  // red slot-0 reads done
-    if (lg == 0 && li < G) red[(wid * G + li) * 2 + 1] = lsum;
-
-    // p write-out: [key][G]; lanes with the same (t, r) write G consecutive
-    // floats for 4 key-groups -> 4 x 64 B segments per instruction
-    if (li < G) {
-        unsigned short* pbase =
-            p_out + (((long)b * nkv + kvh) * C + chunk) * DEC_CHUNK * G;
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int key = wid * WAVE + t * 16 + lg * 4 + r;
-                pbase[key * G + li] = f2bf(sv[t * 4 + r]);
-            }
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float* pml = part_ml + ((((long)b * nkv + kvh) * C + chunk) * G) * 2;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float ls = 0.f;
-            for (int w2 = 0; w2 < DEC_WAVES; ++w2)
-                ls += red[(w2 * G + g) * 2 + 1];
-            float mg = -1e30f;
-            for (int w2 = 0; w2 < DEC_WAVES; ++w2)
-                mg = fmaxf(mg, red[(w2 * G + g) * 2]);
-            pml[g * 2] = mg;
-            pml[g * 2 + 1] = ls;
-        }
-    }
-    __syncthreads();  // red reused by the next chunk iteration
-    }  // chunk loop
-}
 
 // ----------------------------------------------------------- stage 2: PV
 // When FOLD (launcher sets it iff gridDim.z == 1, i.e. every chunk of this
@@ -610,149 +347,6 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_pv_kernel(
     }
 }
 
-// ------------------------------------------- stage 2 (MFMA variant, hd 128)
-// P.V on the matrix pipe: out[g][d] = sum_k P[g][k] V[k][d] as 16x16x32
-// MFMA tiles (A = P rows staged transposed [g][key] in LDS, B = V^T staged
-// [d][key] in LDS). The waves SPLIT THE 128 OUTPUT DIMS (2 dim-groups of 16
-// each) and share one cooperative 32-key V subtile per iteration, so there
-// is no cross-wave merge and the per-wave state is 2 C-fragments (8 VGPRs).
-// Per lane per 32 keys this is ~25 ops vs ~420 for the VALU PV (2G-fma
-// chains + G LDS reads per key) — the G-proportional tail the roadmap
-// attributed the 4.2-4.7 TB/s plateau to.
-// vt row stride 40 elems: 80 B rows keep ds_read_b128 16 B-aligned and hit
-// 16 distinct banks at the 64-dword b128 modulus (bank math in the CDNA4
-// guide §2); the b16 scatter writes are 2-way conflicted (acceptable).
-#define PVM_PAD 8
-#define PVM_STRIDE (32 + PVM_PAD)
-
-template <int G>
-__global__ __launch_bounds__(DEC_BLOCK) void attn_pv_mfma_kernel(
-    const unsigned short* __restrict__ v_cache,  // [nb, nkv, bs, 128]
-    const int* __restrict__ block_table,
-    const int* __restrict__ seq_lens,
-    const unsigned short* __restrict__ p_in,     // [B,nkv,C,CHUNK,G] bf16
-    float* __restrict__ part_o,                  // [B, nkv, C, G, 128]
-    int nkv, int W, int bs, int C) {
-    constexpr int HD = 128;
-    constexpr int PT_STRIDE = DEC_CHUNK + 8;
-    const int b = blockIdx.x;
-    const int kvh = blockIdx.y;
-    const int L = seq_lens[b];
-    if ((int)blockIdx.z * DEC_CHUNK >= L) return;
-    const int tid = threadIdx.x;
-    const int lane = tid % WAVE;
-    const int wid = tid / WAVE;
-    const int lg = lane >> 4;
-    const int li = lane & 15;
-
-    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    unsigned short* p_t = reinterpret_cast<unsigned short*>(smem_raw);
-    const int off_v = (G * PT_STRIDE * 2 + 15) & ~15;
-    long* voff_s = reinterpret_cast<long*>(smem_raw + off_v);  // [CHUNK]
-    unsigned short* vt =
-        reinterpret_cast<unsigned short*>(smem_raw + off_v + DEC_CHUNK * 8);
-    // vt: double-buffered [2][HD][PVM_STRIDE]
-
-    for (int chunk = blockIdx.z; chunk * DEC_CHUNK < L; chunk += gridDim.z) {
-        const int start = chunk * DEC_CHUNK;
-        // stage p transposed ([key][G] -> [g][key]) and the V row offsets
-        {
-            const unsigned short* psrc =
-                p_in + (((long)b * nkv + kvh) * C + chunk) * DEC_CHUNK * G;
-            for (int i = tid; i < DEC_CHUNK * G; i += DEC_BLOCK)
-                p_t[(i % G) * PT_STRIDE + i / G] = psrc[i];
-            const int* btb = block_table + (long)b * W;
-            const int key = start + tid;
-            long vo = 0;
-            if (key < L)
-                vo = (((long)btb[key / bs] * nkv + kvh) * bs + key % bs) * HD;
-            voff_s[tid] = vo;
-        }
-        __syncthreads();
-
-        const int nkeys = min(DEC_CHUNK, L - start);
-        const int nsub = (nkeys + 31) / 32;
-        f32x4 acc[2];
-        acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-        // Cooperative 32-key x 128-dim V subtiles, transposed through LDS.
-        // T14 register staging (guide): loads for subtile t+2 issue BEFORE
-        // the LDS write of t+1 waits on t+1's loads, so each load has a full
-        // iteration (barrier + 2 MFMAs + epilogue traffic) to land. Two
-        // register sets = 2 subtiles of load latency in flight per thread.
-        // Thread t owns key t/8, dims [(t%8)*16, +16): two 16 B loads,
-        // sixteen b16 column writes.
-        const int st_key = tid >> 3;
-        const int st_d = (tid & 7) * 16;
-        short8 ra[2], rb[2];
-#define PVM_LOAD(SUB, SET)                                                     \
-    do {                                                                       \
-        const int k_ = (SUB) * 32 + st_key;                                    \
-        ra[SET] = short8{};                                                    \
-        rb[SET] = short8{};                                                    \
-        if (k_ < nkeys) {                                                      \
-            const unsigned short* vr_ = v_cache + voff_s[k_] + st_d;           \
-            ra[SET] = *reinterpret_cast<const short8*>(vr_);                   \
-            rb[SET] = *reinterpret_cast<const short8*>(vr_ + 8);               \
-        }                                                                      \
-    } while (0)
-#define PVM_WRITE(SET, BUF)                                                    \
-    do {                                                                       \
-        unsigned short* w_ = vt + (BUF) * HD * PVM_STRIDE + st_key;            \
-        _Pragma("unroll") for (int e = 0; e < 8; ++e)                          \
-            w_[(st_d + e) * PVM_STRIDE] = (unsigned short)ra[SET][e];          \
-        _Pragma("unroll") for (int e = 0; e < 8; ++e)                          \
-            w_[(st_d + 8 + e) * PVM_STRIDE] = (unsigned short)rb[SET][e];      \
-    } while (0)
-
-// one 32-key step: LDS-write reg set, prefetch 2 subtiles ahead, barrier,
-// 2 MFMAs. SET/BUF are LITERALS so the compiler tracks which outstanding
-// loads each write actually needs (a runtime-indexed set forced
-// vmcnt(0) at every write: measured 2.1 TB/s vs 4.1)
-#define PVM_STEP(SUB, SET)                                                     \
-    do {                                                                       \
-        PVM_WRITE(SET, SET);                                                   \
-        if ((SUB) + 2 < nsub) PVM_LOAD((SUB) + 2, SET);                        \
-        __syncthreads();                                                       \
-        const unsigned short* vb_ = vt + (SET) * HD * PVM_STRIDE;              \
-        const bf16x8 ap_ = *reinterpret_cast<const bf16x8*>(                   \
-            p_t + prow + (SUB) * 32 + lg * 8);                                 \
-        _Pragma("unroll") for (int dgi = 0; dgi < 2; ++dgi) {                  \
-            const bf16x8 bv_ = *reinterpret_cast<const bf16x8*>(               \
-                vb_ + ((wid * 2 + dgi) * 16 + li) * PVM_STRIDE + lg * 8);      \
-            acc[dgi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(                \
-                ap_, bv_, acc[dgi], 0, 0, 0);                                  \
-        }                                                                      \
-    } while (0)
-
-        PVM_LOAD(0, 0);
-        if (nsub > 1) PVM_LOAD(1, 1);
-        const int prow = (li < G ? li : G - 1) * PT_STRIDE;
-        int sub = 0;
-        for (; sub + 1 < nsub; sub += 2) {
-            PVM_STEP(sub, 0);
-            PVM_STEP(sub + 1, 1);
-        }
-        if (sub < nsub) PVM_STEP(sub, 0);
-#undef PVM_STEP
-#undef PVM_LOAD
-#undef PVM_WRITE
-
-        // C layout: lane holds rows g = lg*4 + r, col d = dgroup*16 + li
-        const long base = (((long)b * nkv + kvh) * C + chunk) * G;
-#pragma unroll
-        for (int dgi = 0; dgi < 2; ++dgi) {
-            const int d = (wid * 2 + dgi) * 16 + li;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int g = lg * 4 + r;
-                if (g < G) part_o[(base + g) * HD + d] = acc[dgi][r];
-            }
-        }
-        __syncthreads();  // p_t / voff_s reused by the next chunk
-    }
-}
-
 // ------------------------------------------------------ stage 3: combine
 template <int G>
 __global__ __launch_bounds__(DEC_BLOCK) void attn_decode_combine_kernel(
@@ -815,47 +409,15 @@ extern "C" void launch_attn_decode(
     const int smem_pv = DEC_CHUNK * G * 4 + DEC_CHUNK * 8 +
                         DEC_WAVES * G * hd * 4 +
                         G * hd * 4 + G * 8;  // + FOLD running state
-    const int smem_pvm = ((G * (DEC_CHUNK + 8) * 2 + 15) & ~15) +
-                         DEC_CHUNK * 8 + 2 * hd * PVM_STRIDE * 2;
-    // MFMA PV (attn_pv_mfma_kernel) measured 4.2 TB/s vs the VALU PV's
-    // 4.5 at B768/G4: the barrier-paced LDS pipeline loses more latency
-    // hiding than the matrix pipe saves (PV is latency-, not VALU-bound).
-    // Kept as opt-in infrastructure for future tr_b16 staging work.
-    static int pv_mfma = -1;
-    if (pv_mfma < 0) {
-        const char* e = getenv("BEE2BEE_PV_MFMA");
-        pv_mfma = (e != nullptr && e[0] == '1') ? 1 : 0;
-    }
 #define LAUNCH_T(GG, KVT)                                                      \
     do {                                                                       \
         const KVT* kc = reinterpret_cast<const KVT*>(k_cache);                 \
         const KVT* vc = reinterpret_cast<const KVT*>(v_cache);                 \
-        if (hd == 128)                                                         \
-            hipLaunchKernelGGL((attn_scores_mfma_kernel<GG, 128, KVT>), grid,  \
-                               dim3(DEC_BLOCK), smem_s, stream, q, kc,         \
-                               block_table, seq_lens, p_buf, part_ml, nkv, W,  \
-                               bs, C, q_stride, scale);                        \
-        else if (hd == 64)                                                     \
-            hipLaunchKernelGGL((attn_scores_mfma_kernel<GG, 64, KVT>), grid,   \
-                               dim3(DEC_BLOCK), smem_s, stream, q, kc,         \
-                               block_table, seq_lens, p_buf, part_ml, nkv, W,  \
-                               bs, C, q_stride, scale);                        \
-        else                                                                   \
-            hipLaunchKernelGGL((attn_scores_kernel<GG, KVT>), grid,            \
-                               dim3(DEC_BLOCK), smem_s, stream, q, kc,         \
-                               block_table, seq_lens, p_buf, part_ml, nkv, W,  \
-                               bs, hd, C, q_stride, scale);                    \
-        if (hd == 128 && pv_mfma && !fp8) {                                    \
-            hipLaunchKernelGGL(attn_pv_mfma_kernel<GG>, grid,                  \
-                               dim3(DEC_BLOCK), smem_pvm, stream,              \
-                               reinterpret_cast<const unsigned short*>(        \
-                                   v_cache),                                   \
-                               block_table, seq_lens, p_buf, part_o, nkv, W,   \
-                               bs, C);                                         \
-            hipLaunchKernelGGL(attn_decode_combine_kernel<GG>, cgrid,          \
-                               dim3(DEC_BLOCK), 0, stream, part_o, part_ml,    \
-                               seq_lens, out, out_ml, nkv, hd, C);             \
-        } else if (Z == 1) {                                                   \
+        hipLaunchKernelGGL((attn_scores_kernel<GG, KVT>), grid,                \
+                           dim3(DEC_BLOCK), smem_s, stream, q, kc,             \
+                           block_table, seq_lens, p_buf, part_ml, nkv, W, bs,  \
+                           hd, C, q_stride, scale);                            \
+        if (Z == 1) {                                                          \
             hipLaunchKernelGGL((attn_pv_kernel<GG, true, KVT>), grid,          \
                                dim3(DEC_BLOCK), smem_pv, stream, vc,           \
                                block_table, seq_lens, p_buf, part_o, part_ml,  \

@@ -30,32 +30,12 @@
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) short short4v;
-typedef __attribute__((ext_vector_type(2))) unsigned int uint2v;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((address_space(3))) short4v lds_short4v;
 
 constexpr int FL_KT = 64;   // keys per staged tile
 // a row's running maximum is raised only by a score this far (in powers of
 // two) above it
 constexpr float FL_SLACK = 8.f;
-
-// the values of lanes l and l + 32, in both: .x the lower lane's
-DEV_INLINE float2v lane_pair(float x) {
-    const unsigned int u = __builtin_bit_cast(unsigned int, x);
-    const uint2v r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    // (a bit cast of a vector's element would take element 0)
-    const unsigned int r0 = r[0], r1 = r[1];
-    return float2v{__builtin_bit_cast(float, r0),
-                   __builtin_bit_cast(float, r1)};
-}
-DEV_INLINE float pair_max(float x) {
-    const float2v p = lane_pair(x);
-    return fmaxf(p.x, p.y);
-}
-DEV_INLINE float pair_sum(float x) {
-    const float2v p = lane_pair(x);
-    return p.x + p.y;
-}
 
 template <int HD, int RW, int KSP, bool PAGED, typename KVT>
 __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(

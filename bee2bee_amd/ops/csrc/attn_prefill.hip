@@ -1,15 +1,17 @@
-// Varlen causal prefill attention (flash-style, no S x S materialization).
+// Varlen causal prefill attention (flash-style, no S x S materialization):
+// the launchers of the plain form (its kernel for head size 64/128 is in
+// attn_flash.hip) and the kernels of the forms with sinks, windows, gates,
+// biases and mixed heads.
 //
-// Both kernels are templated over PAGED: when true, K/V come from the paged
+// The first two kernels are templated over PAGED: when true, K/V come from the paged
 // KV cache ([nb, nkv, bs, hd] + block table) instead of the packed fresh
 // projections, and each query chunk attends to the full cached history
 // (chunked prefill: query row j of sequence b has absolute position
 // hist + j where hist = seq_lens[b] - query_len[b]). The chunk's own K/V
 // were stored to the cache by kv_store before this kernel runs.
 //
-// The plain form with head_dim 64/128 is in attn_flash.hip. Two kernels here:
-//  * attn_prefill_mfma — head_dim 64/128: chunks of a few tokens, and the
-//    forms with sinks, windows, gates, biases and mixed heads: per
+// Two kernels:
+//  * attn_prefill_mfma — head_dim 64/128 with fp32-grade weights: per
 //    workgroup 4 waves x 16 q-rows (64-row Q tile), 32-key K/V tiles staged
 //    in LDS (+8-element row padding => conflict-free ds_read_b128, guide
 //    T2/G4), QK^T and P.V on v_mfma_f32_16x16x32_bf16, online softmax in
@@ -123,10 +125,10 @@ __global__ __launch_bounds__(64) void attn_prefill_basic(
 #define PF_TN 64                     // kv tile (4 x 16-key fragments)
 #define PF_PAD 8                     // LDS row padding (bf16 elems)
 
-// HILO: the softmax weights enter the P V product as a bf16 PAIR (hi + lo,
-// two MFMAs, ~16 mantissa bits) instead of one bf16 rounding — for designs
-// whose attention weights are 32-bit quantities. sink (optional, [nq] fp32):
-// a per-head logit counted once in the softmax denominator, with no key and
+// The softmax weights enter the P V product as a bf16 PAIR (hi + lo, two
+// MFMAs, ~16 mantissa bits): the attention of designs whose weights are
+// 32-bit quantities (one bf16 rounding: attn_flash.hip). sink (optional, [nq]
+// fp32): a per-head logit counted once in the softmax denominator, with no key and
 // no value. The output row of token t, head h starts at out + t*s_o + h*HD
 // and is multiplied by out_scale. window > 0: the row at absolute position
 // p sees keys p - window < j <= p, and key tiles wholly before the tile's
@@ -134,8 +136,8 @@ __global__ __launch_bounds__(64) void attn_prefill_basic(
 // stride s_g): head h's output times sigmoid(head_gate[t, h]). DIST:
 // dist [2, nq] = (a, b), a_h ln(1 + b_h d) is taken off a score whose key
 // lies d positions back. KEEP: with a window, the first `keep` positions stay
-// visible to every later row (their tiles are visited first). HILO on packed
-// keys applies `scale` to the fp32 scores instead of the bf16 queries.
+// visible to every later row (their tiles are visited first). On packed keys
+// `scale` is applied to the fp32 scores instead of the bf16 queries.
 //
 // MODE 1 / MODE 2 split the kernel around a score buffer, for attention
 // whose scores are mixed across heads before the softmax: MODE 1 stops
@@ -147,12 +149,12 @@ __global__ __launch_bounds__(64) void attn_prefill_basic(
 // query rows [qt0 * 64, qt0 * 64 + qt_rows) of every chunk; entry `col` of
 // a row is key kv_lo + col, kv_lo being the first key the row's 64-query
 // tile visits. blockIdx.x counts tiles from qt0.
-template <int HD, bool PAGED, typename KVT, bool HILO = false, int MODE = 0,
-          bool DIST = false, bool KEEP = false>
+template <int HD, bool PAGED, int MODE = 0, bool DIST = false,
+          bool KEEP = false>
 __global__ __launch_bounds__(256) void attn_prefill_mfma(
     const unsigned short* __restrict__ q,
-    const KVT* __restrict__ k,  // PAGED: k_cache [nb,nkv,bs,hd]
-    const KVT* __restrict__ v,
+    const unsigned short* __restrict__ k,  // PAGED: k_cache [nb,nkv,bs,hd]
+    const unsigned short* __restrict__ v,
     const int* __restrict__ cu,            // [nseq+1] query tokens
     const int* __restrict__ block_table,   // PAGED only
     const int* __restrict__ seq_lens,      // PAGED only
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
     int qt_rows = 0, long ctx = 0, float softcap = 0.f,
     const float* __restrict__ dist = nullptr, int keep = 0) {
     constexpr int KSTEPS = HD / 32;
-    constexpr bool SCALE_S = HILO && !PAGED;
+    constexpr bool SCALE_S = !PAGED;
     const int seq = blockIdx.z;
     const int h = blockIdx.y;
     const int kvh = h / (nq / nkv);
@@ -190,7 +192,7 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
     constexpr int VT_STRIDE = PF_TN + PF_PAD;
     constexpr int K_ELEMS = PF_TN * (HD + PF_PAD);
     constexpr int P_TILE = PF_TM * VT_STRIDE;
-    constexpr int P_ELEMS = P_TILE * (HILO ? 2 : 1);
+    constexpr int P_ELEMS = P_TILE * 2;  // weights: hi, lo
     constexpr int VT_OFF = (K_ELEMS > P_ELEMS ? K_ELEMS : P_ELEMS);
     unsigned short* k_s = reinterpret_cast<unsigned short*>(smem_raw);
     unsigned short* vt_s = k_s + VT_OFF;
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
                     (wid * PF_QROWS + lg * 4 + r) * VT_STRIDE + f * 16 + li;
                 const unsigned short hi = f2bf(pv);
                 p_s[pi] = hi;
-                if (HILO) p_s[P_TILE + pi] = f2bf(pv - bf2f(hi));
+                p_s[P_TILE + pi] = f2bf(pv - bf2f(hi));
             }
         }
         // row sum across group lanes
@@ -397,13 +399,12 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
         // share the LDS buffer -> sync so K-tile reuse is safe)
         __syncthreads();
         bf16x8 a_p[PF_TN / 32];  // A k-dim = keys: 32 keys per fragment
-        bf16x8 a_pl[HILO ? PF_TN / 32 : 1];
+        bf16x8 a_pl[PF_TN / 32];
 #pragma unroll
         for (int ks2 = 0; ks2 < PF_TN / 32; ++ks2) {
             const int pi = (wid * PF_QROWS + li) * VT_STRIDE + ks2 * 32 + lg * 8;
             a_p[ks2] = *reinterpret_cast<const bf16x8*>(p_s + pi);
-            if (HILO)
-                a_pl[ks2] = *reinterpret_cast<const bf16x8*>(p_s + P_TILE + pi);
+            a_pl[ks2] = *reinterpret_cast<const bf16x8*>(p_s + P_TILE + pi);
         }
 #pragma unroll
         for (int nb = 0; nb < HD / 16; ++nb) {
@@ -413,9 +414,8 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
                     vt_s + (nb * 16 + li) * VT_STRIDE + ks2 * 32 + lg * 8);
                 o_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     a_p[ks2], bv, o_acc[nb], 0, 0, 0);
-                if (HILO)
-                    o_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        a_pl[ks2], bv, o_acc[nb], 0, 0, 0);
+                o_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a_pl[ks2], bv, o_acc[nb], 0, 0, 0);
             }
         }
     }
@@ -445,10 +445,10 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma(
     }
 }
 
-static int prefill_mfma_smem(int hd, int hilo = 0) {
-    // LDS: max(K tile, P tile(s)) + V^T tile, bf16; must match VT_OFF
+static int prefill_mfma_smem(int hd) {
+    // LDS: max(K tile, P tiles) + V^T tile, bf16; must match VT_OFF
     const int k_bytes = PF_TN * (hd + PF_PAD) * 2;
-    const int p_bytes = PF_TM * (PF_TN + PF_PAD) * 2 * (hilo ? 2 : 1);
+    const int p_bytes = PF_TM * (PF_TN + PF_PAD) * 2 * 2;
     const int vt_bytes = hd * (PF_TN + PF_PAD) * 2;
     return (k_bytes > p_bytes ? k_bytes : p_bytes) + vt_bytes;
 }
@@ -485,40 +485,16 @@ extern "C" void launch_attn_prefill_paged(
     const int* cu, const int* block_table, const int* seq_lens,
     unsigned short* out, long T, int nseq, int nq, int nkv, int hd, long s_q,
     int W, int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
-    // (a few tokens a sequence fill a tile of neither kernel)
-    if (max_qlen * (nq / nkv) > 32 &&
-        launch_attn_flash(q, k_cache, v_cache, cu, block_table, seq_lens, out,
+    if (launch_attn_flash(q, k_cache, v_cache, cu, block_table, seq_lens, out,
                           T, nseq, nq, nkv, hd, s_q, 0, 0, W, bs, max_qlen,
                           scale, fp8, stream) == 0)
         return;
-#define PFP_LAUNCH(KVT)                                                        \
-    do {                                                                       \
-        const KVT* kc = reinterpret_cast<const KVT*>(k_cache);                 \
-        const KVT* vc = reinterpret_cast<const KVT*>(v_cache);                 \
-        if (hd == 64 || hd == 128) {                                           \
-            const int tiles = (max_qlen + PF_TM - 1) / PF_TM;                  \
-            dim3 grid(tiles, nq, nseq);                                        \
-            const int smem = prefill_mfma_smem(hd);                            \
-            if (hd == 128)                                                     \
-                hipLaunchKernelGGL((attn_prefill_mfma<128, true, KVT>), grid,  \
-                                   dim3(256), smem, stream, q, kc, vc, cu,     \
-                                   block_table, seq_lens, out, nq, nkv, s_q,   \
-                                   0, 0, W, bs, scale, nullptr, 1.f,           \
-                                   (long)nq * hd);                             \
-            else                                                               \
-                hipLaunchKernelGGL((attn_prefill_mfma<64, true, KVT>), grid,   \
-                                   dim3(256), smem, stream, q, kc, vc, cu,     \
-                                   block_table, seq_lens, out, nq, nkv, s_q,   \
-                                   0, 0, W, bs, scale, nullptr, 1.f,           \
-                                   (long)nq * hd);                             \
-            return;                                                            \
-        }                                                                      \
-        dim3 grid(nq, nseq);                                                   \
-        const int smem = (hd + WAVE) * 4;                                      \
-        hipLaunchKernelGGL((attn_prefill_basic<true, KVT>), grid, dim3(WAVE),  \
-                           smem, stream, q, kc, vc, cu, block_table, seq_lens, \
-                           out, nq, nkv, hd, s_q, 0, 0, W, bs, scale, 1);      \
-    } while (0)
+#define PFP_LAUNCH(KVT)                                                       \
+    hipLaunchKernelGGL((attn_prefill_basic<true, KVT>), dim3(nq, nseq),       \
+                       dim3(WAVE), (hd + WAVE) * 4, stream, q,                \
+                       (const KVT*)k_cache, (const KVT*)v_cache, cu,          \
+                       block_table, seq_lens, out, nq, nkv, hd, s_q, 0, 0, W, \
+                       bs, scale, 1)
     if (fp8) PFP_LAUNCH(unsigned char);
     else PFP_LAUNCH(unsigned short);
 #undef PFP_LAUNCH
@@ -542,10 +518,10 @@ extern "C" int launch_attn_prefill_paged_sink(
     if (nseq == 0 || max_qlen == 0) return 0;
     const int tiles = (max_qlen + PF_TM - 1) / PF_TM;
     dim3 grid(tiles, nq, nseq);
-    const int smem = prefill_mfma_smem(hd, 1);
+    const int smem = prefill_mfma_smem(hd);
 #define PS_LAUNCH(HDV, DI, KP)                                                \
     hipLaunchKernelGGL(                                                       \
-        (attn_prefill_mfma<HDV, true, unsigned short, true, 0, DI, KP>),      \
+        (attn_prefill_mfma<HDV, true, 0, DI, KP>),                            \
         grid, dim3(256), smem, stream, q, k_cache, v_cache, cu, block_table,  \
         seq_lens, out, nq, nkv, s_q, 0, 0, W, bs, 1.f, sink, out_scale, s_o,  \
         window, head_gate, s_g, nullptr, 0, 0, 0, 0.f, dist, keep)
@@ -573,10 +549,10 @@ extern "C" int launch_attn_prefill_packed(
     if (hd != 64 && hd != 128) return 1;
     if (nseq == 0 || max_qlen == 0) return 0;
     const dim3 grid((max_qlen + PF_TM - 1) / PF_TM, nq, nseq);
-    const int smem = prefill_mfma_smem(hd, 1);
+    const int smem = prefill_mfma_smem(hd);
     const int* none = nullptr;
 #define PK_LAUNCH(HDV)                                                        \
-    hipLaunchKernelGGL((attn_prefill_mfma<HDV, false, unsigned short, true>), \
+    hipLaunchKernelGGL((attn_prefill_mfma<HDV, false>),                       \
                        grid, dim3(256), smem, stream, q, k, v, cu, none,      \
                        none, out, nq, nkv, s_q, s_k, s_v, 0, 0, scale,        \
                        (const float*)nullptr, out_scale, s_o, window,         \
@@ -644,7 +620,7 @@ extern "C" int launch_attn_prefill_paged_mixed(
     if (nseq == 0 || n_tiles == 0) return 0;
     const int qt_rows = n_tiles * PF_TM;
     const dim3 grid(n_tiles, nq, nseq);
-    const int smem = prefill_mfma_smem(hd, 1);
+    const int smem = prefill_mfma_smem(hd);
     const size_t mix_smem =
         ((size_t)nq * nq + (size_t)nq * 64 * SM_ROWS) * sizeof(float);
     if (mix_smem > 64 * 1024) return 1;
@@ -652,8 +628,8 @@ extern "C" int launch_attn_prefill_paged_mixed(
                      (qt_rows + SM_ROWS - 1) / SM_ROWS, nseq);
 #define PM_LAUNCH(HDV, M)                                                     \
     hipLaunchKernelGGL(                                                       \
-        (attn_prefill_mfma<HDV, true, unsigned short, true, M>), grid,        \
-        dim3(256), smem, stream, q, k_cache, v_cache, cu, block_table,        \
+        (attn_prefill_mfma<HDV, true, M>), grid, dim3(256),                   \
+        smem, stream, q, k_cache, v_cache, cu, block_table,        \
         seq_lens, out, nq, nkv, s_q, 0, 0, W, bs, 1.f, sink, 1.f, s_o,        \
         window, head_gate, s_g, score_buf, qt0, qt_rows, ctx, softcap)
     if (hd == 128) PM_LAUNCH(128, 1); else PM_LAUNCH(64, 1);
@@ -921,7 +897,7 @@ extern "C" int launch_attn_prefill_paged_cross(
     if (nseq == 0 || max_qlen == 0) return 0;
     const int tiles = (max_qlen + PF_TM - 1) / PF_TM;
     dim3 grid(tiles, nq, nseq);
-    const int smem = prefill_mfma_smem(hd, 1);
+    const int smem = prefill_mfma_smem(hd);
 #define PFC(HDV, NVV)                                                          \
     hipLaunchKernelGGL((attn_prefill_cross_mfma<HDV, NVV>), grid, dim3(256),   \
                        smem, stream, q, k_cache, v_cache, cu, block_table,     \

@@ -1,0 +1,453 @@
+// Paged attention of a few query rows per sequence: decode steps, and the
+// chunks of a few tokens that speculative decoding verifies.
+//
+// Bound by reading the cache once. A wave takes tiles of 32 keys on its own:
+// whole 16-byte chunks of neighbouring rows into registers (1 KB a load), on
+// to its part of LDS, the next tile's loads on their way over the products of
+// this one, no barrier before the end. Scores are S^T = K Q^T on 16x16x32
+// matrix tiles (a column is a query row; the rows of all heads that share the
+// key head, times the chunk's tokens), so that the weights are, as they
+// stand, the right operand of O^T = V^T P^T, whose keys follow the score
+// tile's order through the transposing LDS read. One pass over K and V: no
+// weights written, no second kernel unless the context is split over
+// workgroups (their fp32 sums, combined). fp8 rows are widened to bf16 on
+// their way into LDS (decode queries are rounded to fp8 like them, chunks'
+// are not).
+// Measured against the kernels before it (scores, weights through memory,
+// values, combine): 1536 sequences of 137..1100 tokens, 8 key heads of size
+// 128: 652 us (5.98 TB/s) instead of 778; fp8 361 instead of 588; 200
+// sequences of up to 3000 fp8 132 instead of 228; one of 3000 8.6 instead of
+// 15.3; 16 sequences' 5 tokens on 1500 26 instead of 166.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) short short4v;
+typedef __attribute__((address_space(3))) short4v lds_short4v;
+
+constexpr int ST_WAVES = 4;
+constexpr int ST_KEYS = 32;                      // keys of a wave's tile
+constexpr int ST_STEP = ST_WAVES * ST_KEYS;      // keys of a workgroup's step
+constexpr float ST_LOG2E = 1.44269504088896340736f;
+
+// 16 bytes of a bf16 row, or 8 of an fp8 row, as read
+template <typename KVT> struct st_raw { using type = short8; };
+template <> struct st_raw<unsigned char> { using type = uint2v; };
+DEV_INLINE short8 st_widen(short8 x) { return x; }
+DEV_INLINE short8 st_widen(uint2v x) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    bf16x8 r;
+    const unsigned int w[2] = {x[0], x[1]};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const bf16x2 a =
+            __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.f, false);
+        const bf16x2 b =
+            __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.f, true);
+        r[i * 4] = a[0];
+        r[i * 4 + 1] = a[1];
+        r[i * 4 + 2] = b[0];
+        r[i * 4 + 3] = b[1];
+    }
+    return __builtin_bit_cast(short8, r);
+}
+
+// 8 queries times the score scale, rounded to fp8
+DEV_INLINE bf16x8 st_round_fp8(bf16x8 x, float scale) {
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = (float)(__bf16)((float)x[e] * scale);
+    uint2v w;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        w[i] = f2fp8x2(f[i * 4], f[i * 4 + 1]) |
+               (unsigned int)f2fp8x2(f[i * 4 + 2], f[i * 4 + 3]) << 16;
+    return __builtin_bit_cast(bf16x8, st_widen(w));
+}
+
+// keys per split: whole steps of a workgroup, the same for every reader
+DEV_INLINE int split_keys(int L, int Z) {
+    return ((L + Z - 1) / Z + ST_STEP - 1) / ST_STEP * ST_STEP;
+}
+
+template <int HD, int QT, typename KVT>
+__global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
+    const unsigned short* __restrict__ q, const KVT* __restrict__ k_cache,
+    const KVT* __restrict__ v_cache, const int* __restrict__ cu,
+    const int* __restrict__ block_table, const int* __restrict__ seq_lens,
+    unsigned short* __restrict__ out, float* __restrict__ out_ml,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int nkv, int G,
+    int W, int bs, int Z, int max_rows, long s_q, float scale) {
+    constexpr int KS = HD / 32;          // k steps of a score tile
+    constexpr int DT = HD / 16;          // output tiles of 16 coordinates
+    constexpr int CPR = HD / 8;          // chunks of 8 elements of a key row
+    constexpr int RB = HD * 2;           // bytes of a staged row
+    constexpr int RPI = 64 / CPR;        // rows a wave loads at once
+    constexpr int NL = ST_KEYS / RPI;    // loads of a tile
+    constexpr int TILE = ST_KEYS * RB;
+    constexpr int VMASK = HD == 128 ? 7 : 3;
+    using raw_t = typename st_raw<KVT>::type;
+
+    const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
+    const int s0 = cu ? cu[b] : b;
+    const int rows = (cu ? cu[b + 1] - s0 : 1) * G;
+    const int row0 = blockIdx.z * QT * 16;
+    if (row0 >= rows) return;
+    const int L = seq_lens[b];
+    const int hist = L - rows / G;
+    const int per = split_keys(L, Z);
+    const int k0 = blockIdx.y * per, k1 = min(L, k0 + per);
+    if (k0 >= L && blockIdx.y > 0) return;
+    const int* bt = block_table + (long)b * W;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    char* kd = smem + wid * 2 * TILE;    // this wave's K tile, then its V tile
+
+    // decoding on an 8-bit cache, scaled queries are of its type too
+    const bool round_q = sizeof(KVT) == 1 && !cu;
+    const float scale_log2 = round_q ? ST_LOG2E : scale * ST_LOG2E;
+
+    // ---- query rows: column li of tile qt is row row0 + qt * 16 + li
+    bf16x8 bq[QT][KS];
+    int see[QT];                         // last key of the row
+    long q_off[QT];                      // of the row's output
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        const int r = min(row0 + t * 16 + li, rows - 1);
+        const int pos = r / G, head = kvh * G + r % G;
+        const unsigned short* qr =
+            q + (long)(s0 + pos) * s_q + (long)head * HD;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            bq[t][ks] =
+                *reinterpret_cast<const bf16x8*>(qr + ks * 32 + lg * 8);
+            if (round_q) bq[t][ks] = st_round_fp8(bq[t][ks], scale);
+        }
+        see[t] = hist + pos;
+        q_off[t] = (long)(s0 + pos) * nkv * G + head;
+    }
+    const int first_see = hist + row0 / G;
+
+    // ---- loading: lane -> (row of RPI, chunk)
+    const int ld_row = lane / CPR, ld_c = lane % CPR;
+    raw_t rk[NL], rv[NL];
+    const bool whole_pages = bs % ST_KEYS == 0;
+    auto load_tile = [&](int kb) {
+        // a tile inside one page: the page is a scalar look-up
+        long base = 0;
+        if (whole_pages) {
+            const int page = bt[kb / bs];
+            BB_KASSERT(page >= 0);
+            base = (((long)page * nkv + kvh) * bs + kb % bs) * HD;
+        }
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int key = min(kb + ld_row + i * RPI, k1 - 1);
+            long off;
+            if (whole_pages) {
+                off = base + (long)(key - kb) * HD;
+            } else {
+                const int page = bt[key / bs];
+                BB_KASSERT(page >= 0);
+                off = (((long)page * nkv + kvh) * bs + key % bs) * HD;
+            }
+            off += ld_c * 8;
+            rk[i] = *reinterpret_cast<const raw_t*>(k_cache + off);
+            rv[i] = *reinterpret_cast<const raw_t*>(v_cache + off);
+        }
+    };
+
+    // ---- fragment addresses: K row li (+ 16), chunk ks * 4 + lg; V through
+    // the transposing read, 16 lanes on 4 keys x 16 coordinates
+    const int k_base = li * RB, k_sw = li & 7;
+    const int v_key = lg * 4 + (li >> 2);
+    const int v_sw = 2 * (v_key & VMASK);
+    const int v_base = TILE + v_key * RB + (lane & 1) * 8;
+    const int v_c = (lane & 3) >> 1;
+
+    f32x4 o[DT][QT];
+    float m[QT], l[QT];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        m[t] = -1e30f;
+        l[t] = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[d][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    int kb = k0 + wid * ST_KEYS;
+    if (kb < k1) load_tile(kb);
+    for (; kb < k1; kb += ST_STEP) {
+        // ---- registers -> LDS (16-byte chunks xor-ed by the key), and the
+        // next tile's loads on their way over this tile's products
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int row = ld_row + i * RPI;
+            *reinterpret_cast<short8*>(kd + row * RB +
+                                       ((ld_c ^ (row & 7)) << 4)) =
+                st_widen(rk[i]);
+            *reinterpret_cast<short8*>(
+                kd + TILE + row * RB + ((ld_c ^ (2 * (row & VMASK))) << 4)) =
+                st_widen(rv[i]);
+        }
+        if (kb + ST_STEP < k1) load_tile(kb + ST_STEP);
+        WAVE_LDS_SYNC();
+
+        // ---- S^T = K Q^T: column = query row, rows = 16 keys
+        f32x4 s[2][QT];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 ak[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                ak[ks] = *reinterpret_cast<const bf16x8*>(
+                    kd + h * 16 * RB + k_base +
+                    (((ks * 4 + lg) ^ k_sw) << 4));
+#pragma unroll
+            for (int t = 0; t < QT; ++t) {
+                s[h][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    s[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        ak[ks], bq[t][ks], s[h][t], 0, 0, 0);
+            }
+        }
+        if (kb + ST_KEYS - 1 > first_see) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (kb + h * 16 + lg * 4 + r > see[t])
+                            s[h][t][r] = -INFINITY;
+        }
+
+        // ---- online softmax, in powers of two
+        bf16x8 bp[QT];
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            float mx = s[0][t][0];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                mx = fmaxf(fmaxf(mx, s[0][t][r]), s[1][t][r]);
+            mx = rows_max(mx) * scale_log2;
+            const float mn = fmaxf(m[t], mx);
+            if (__any(mn > m[t])) {
+                const float alpha = __builtin_amdgcn_exp2f(m[t] - mn);
+                m[t] = mn;
+                l[t] *= alpha;
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[d][t][r] *= alpha;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float p = __builtin_amdgcn_exp2f(
+                        fmaf(s[h][t][r], scale_log2, -m[t]));
+                    l[t] += p;
+                    bp[t][h * 4 + r] = (__bf16)p;
+                }
+        }
+        // ---- O^T += V^T P^T; keys in the order the score tiles hold them:
+        // lane group lg has 4 lg + {0..3}, then 16 + 4 lg + {0..3}
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            const char* va = kd + v_base + (((d * 2 + v_c) ^ v_sw) << 4);
+            const short4v a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_short4v*)va);
+            const short4v a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_short4v*)(va + 16 * RB));
+            const bf16x8 av = __builtin_bit_cast(
+                bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6,
+                                                7));
+#pragma unroll
+            for (int t = 0; t < QT; ++t)
+                o[d][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    av, bp[t], o[d][t], 0, 0, 0);
+        }
+        WAVE_LDS_SYNC();
+    }
+
+    // ---- the four waves' sums meet in LDS: each leaves m, l and O in its
+    // own tiles
+    float* mine = reinterpret_cast<float*>(kd);
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        l[t] = rows_sum(l[t]);
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+            *reinterpret_cast<f32x4*>(mine + ((t * DT + d) * 64 + lane) * 4) =
+                o[d][t];
+    }
+    float* ml_s = reinterpret_cast<float*>(smem + ST_WAVES * 2 * TILE);
+    if (lg == 0) {
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            ml_s[((t * 16 + li) * ST_WAVES + wid) * 2] = m[t];
+            ml_s[((t * 16 + li) * ST_WAVES + wid) * 2 + 1] = l[t];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        if (row0 + t * 16 + li >= rows) continue;
+        float wm[ST_WAVES], M = -1e30f, lsum = 0.f;
+#pragma unroll
+        for (int w = 0; w < ST_WAVES; ++w) {
+            wm[w] = ml_s[((t * 16 + li) * ST_WAVES + w) * 2];
+            M = fmaxf(M, wm[w]);
+        }
+#pragma unroll
+        for (int w = 0; w < ST_WAVES; ++w) {
+            wm[w] = __builtin_amdgcn_exp2f(wm[w] - M);
+            lsum += wm[w] * ml_s[((t * 16 + li) * ST_WAVES + w) * 2 + 1];
+        }
+        const long part =
+            ((long)blockIdx.x * Z + blockIdx.y) * max_rows + row0 + t * 16 +
+            li;
+        if (wid == 0 && lg == 0) {
+            if (Z > 1) {
+                part_ml[part * 2] = M;
+                part_ml[part * 2 + 1] = lsum;
+            } else if (out_ml) {
+                out_ml[q_off[t] * 2] = M / ST_LOG2E;
+                out_ml[q_off[t] * 2 + 1] = lsum;
+            }
+        }
+        const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+        for (int d = wid; d < DT; d += ST_WAVES) {
+            f32x4 a{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < ST_WAVES; ++w) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(
+                    smem + w * 2 * TILE + ((t * DT + d) * 64 + lane) * 16);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] += x[r] * wm[w];
+            }
+            if (Z > 1) {
+                *reinterpret_cast<f32x4*>(part_o + part * HD + d * 16 +
+                                          lg * 4) = a;
+            } else {
+                short4v w;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[r] = (short)f2bf(a[r] * inv);
+                *reinterpret_cast<short4v*>(out + q_off[t] * HD + d * 16 +
+                                            lg * 4) = w;
+            }
+        }
+    }
+}
+
+// The splits' sums of one row: workgroup = (sequence and key head, row), a
+// thread per coordinate.
+template <int HD>
+__global__ __launch_bounds__(HD) void attn_stream_combine_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const int* __restrict__ cu, const int* __restrict__ seq_lens,
+    unsigned short* __restrict__ out, float* __restrict__ out_ml, int nkv,
+    int G, int Z, int max_rows) {
+    const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
+    const int s0 = cu ? cu[b] : b;
+    const int row = blockIdx.y;
+    if (row >= (cu ? cu[b + 1] - s0 : 1) * G) return;
+    const int L = seq_lens[b];
+    const int per = split_keys(L, Z);
+    const int nz = L > 0 ? (L + per - 1) / per : 0;
+    const long p0 = (long)blockIdx.x * Z * max_rows + row;
+    float M = -1e30f, lsum = 0.f, acc = 0.f;
+    for (int z = 0; z < nz; ++z)
+        M = fmaxf(M, part_ml[(p0 + (long)z * max_rows) * 2]);
+#pragma unroll 8
+    for (int z = 0; z < nz; ++z) {
+        const long p = p0 + (long)z * max_rows;
+        const float w = __builtin_amdgcn_exp2f(part_ml[p * 2] - M);
+        lsum += w * part_ml[p * 2 + 1];
+        acc += w * part_o[p * HD + threadIdx.x];
+    }
+    const long o = (long)(s0 + row / G) * nkv * G + kvh * G + row % G;
+    out[o * HD + threadIdx.x] = f2bf(lsum > 0.f ? acc / lsum : 0.f);
+    if (out_ml && threadIdx.x == 0) {
+        out_ml[o * 2] = M / ST_LOG2E;
+        out_ml[o * 2 + 1] = lsum;
+    }
+}
+
+// Workgroups of a step that take one (sequence, key head) and up to 32 query
+// rows each.
+static long stream_groups(long pairs, long rows) {
+    return pairs * ((rows + 31) / 32);
+}
+
+// Query chunks against the pages: this kernel, or attn_flash.hip's. This one
+// fills the chip with splits of the context where there are few rows; the
+// other reads a key once for 64 rows and more. They cross at about 500
+// workgroups here (us, this / that, 8000 cached tokens, 8 key heads of size
+// 128: 5 rows x 1 sequence 24 / 158; 128 rows x 4 67 / 163; 128 rows x 16
+// 178 / 213; 256 rows x 16 365 / 243; 64 rows x 64 with 2000 cached 210 /
+// 104). Up to 32 rows stay here at any batch (64 sequences, 2000 cached: 109
+// / 101): tokens verified together get the sums that decoding gives them.
+extern "C" int attn_stream_takes(long pairs, long rows) {
+    return rows <= 32 || stream_groups(pairs, rows) <= 448;
+}
+
+// Splits of a context of up to `keys` keys (what the block table holds):
+// about a workgroup a CU. More cost more in the combine than they hide (192
+// (sequence, key head) pairs of up to 2000 keys: 25.1 us with 2 splits, 26.4
+// with 6, 28.9 with 16; 8 pairs of 3000: 35.7 with 1, 10.1 with 8, 8.6 with
+// 32); from 256 pairs on one split writes its result itself.
+extern "C" int attn_stream_splits(long pairs, long rows, long keys) {
+    const long groups = stream_groups(pairs, rows);
+    const long most = (keys + ST_STEP - 1) / ST_STEP;
+    long z = (256 + groups - 1) / groups;
+    if (z > 32) z = 32;
+    if (z > most) z = most;
+    return z < 1 ? 1 : (int)z;
+}
+
+// cu null: one row a sequence (decode). part_o [nseq * nkv, Z, max_rows, hd]
+// and part_ml [.., 2] fp32 when Z > 1; out_ml (optional) [T, nq, 2]: natural-
+// log (m, l) of every row. Head size 64 or 128 and a positive scale, nonzero
+// for any other.
+extern "C" int launch_attn_stream(
+    const unsigned short* q, const void* k_cache, const void* v_cache,
+    const int* cu, const int* block_table, const int* seq_lens,
+    unsigned short* out, float* out_ml, float* part_o, float* part_ml,
+    int nseq, int nkv, int G, int W, int bs, int hd, int Z, int max_qlen,
+    long s_q, float scale, int fp8, hipStream_t stream) {
+    if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
+    if (nseq == 0 || max_qlen <= 0) return 0;
+    const int max_rows = max_qlen * G;
+    const int qt = max_rows <= 16 ? 1 : 2;
+    const dim3 grid(nseq * nkv, Z, (max_rows + qt * 16 - 1) / (qt * 16));
+    const int smem = ST_WAVES * 2 * ST_KEYS * hd * 2 +
+                     qt * 16 * ST_WAVES * 2 * (int)sizeof(float);
+#define ST_ONE(HDV, QTV, KVT)                                                 \
+    hipLaunchKernelGGL((attn_stream_kernel<HDV, QTV, KVT>), grid,             \
+                       dim3(ST_WAVES * 64), smem, stream, q,                  \
+                       (const KVT*)k_cache, (const KVT*)v_cache, cu,          \
+                       block_table, seq_lens, out, out_ml, part_o, part_ml,   \
+                       nkv, G, W, bs, Z, max_rows, s_q, scale)
+#define ST_HD(HDV)                                                            \
+    do {                                                                      \
+        if (fp8 && qt == 1) ST_ONE(HDV, 1, unsigned char);                    \
+        else if (fp8) ST_ONE(HDV, 2, unsigned char);                          \
+        else if (qt == 1) ST_ONE(HDV, 1, unsigned short);                     \
+        else ST_ONE(HDV, 2, unsigned short);                                  \
+        if (Z > 1)                                                            \
+            hipLaunchKernelGGL((attn_stream_combine_kernel<HDV>),             \
+                               dim3(nseq * nkv, max_rows), dim3(HDV), 0,      \
+                               stream, part_o, part_ml, cu, seq_lens, out,    \
+                               out_ml, nkv, G, Z, max_rows);                  \
+    } while (0)
+    if (hd == 128) ST_HD(128);
+    else ST_HD(64);
+#undef ST_HD
+#undef ST_ONE
+    return 0;
+}

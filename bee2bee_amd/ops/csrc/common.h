@@ -16,6 +16,7 @@ typedef __attribute__((ext_vector_type(2))) short short2v;
 typedef __attribute__((ext_vector_type(2))) float float2v;
 typedef __attribute__((ext_vector_type(8))) unsigned char uchar8;
 typedef __attribute__((ext_vector_type(2))) unsigned char u8x2;
+typedef __attribute__((ext_vector_type(2))) unsigned int uint2v;
 
 // --- OCP fp8 (e4m3) helpers: gfx950's v_cvt_* work on packed pairs.
 // pack two floats into the low word of an int (2 x fp8 bytes)
@@ -97,6 +98,41 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 #define DEV_INLINE __device__ __forceinline__
+
+// the values of lanes l and l + 32, in both: .x the lower lane's
+DEV_INLINE float2v lane_pair(float x) {
+    const unsigned int u = __builtin_bit_cast(unsigned int, x);
+    const uint2v r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    // (a bit cast of a vector's element would take element 0)
+    const unsigned int r0 = r[0], r1 = r[1];
+    return float2v{__builtin_bit_cast(float, r0),
+                   __builtin_bit_cast(float, r1)};
+}
+DEV_INLINE float pair_max(float x) {
+    const float2v p = lane_pair(x);
+    return fmaxf(p.x, p.y);
+}
+DEV_INLINE float pair_sum(float x) {
+    const float2v p = lane_pair(x);
+    return p.x + p.y;
+}
+
+// the maximum / sum over the four 16-lane rows of a wave, in every lane
+DEV_INLINE float2v row_pair(float x) {
+    const unsigned int u = __builtin_bit_cast(unsigned int, x);
+    const uint2v r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned int r0 = r[0], r1 = r[1];
+    return float2v{__builtin_bit_cast(float, r0),
+                   __builtin_bit_cast(float, r1)};
+}
+DEV_INLINE float rows_max(float x) {
+    const float2v p = row_pair(x);
+    return pair_max(fmaxf(p.x, p.y));
+}
+DEV_INLINE float rows_sum(float x) {
+    const float2v p = row_pair(x);
+    return pair_sum(p.x + p.y);
+}
 
 // LDS hand-over inside ONE wave (no workgroup barrier): a wave's LDS
 // operations execute in order, so earlier writes of any lane are seen by

@@ -37,6 +37,12 @@ void launch_attn_decode(const unsigned short*, const void*, const void*,
                         const int*, const int*, unsigned short*, float*,
                         float*, unsigned short*, float*, int, int, int, int,
                         int, int, int, long, float, int, hipStream_t);
+int attn_stream_takes(long, long);
+int attn_stream_splits(long, long, long);
+int launch_attn_stream(const unsigned short*, const void*, const void*,
+                       const int*, const int*, const int*, unsigned short*,
+                       float*, float*, float*, int, int, int, int, int, int,
+                       int, int, long, float, int, hipStream_t);
 void launch_attn_prefill(const unsigned short*, const unsigned short*,
                          const unsigned short*, const int*, unsigned short*,
                          long, int, int, int, int, long, long, long, int,
@@ -210,6 +216,40 @@ Tensor swiglu(const Tensor& gu) {
     return out;
 }
 
+// A few query rows per sequence (cu null: one): the one-pass kernel, with
+// workspaces for the sums of a split context. False if it does not take the
+// head size or scale.
+bool attn_stream(const Tensor& q_in, const Tensor& k_cache,
+                 const Tensor& v_cache, const int* cu, int nseq,
+                 const Tensor& block_table, const Tensor& seq_lens,
+                 Tensor& out, float* out_ml, int max_qlen, double scale) {
+    // queries are read 16 bytes at a time
+    const bool aligned =
+        q_in.stride(0) % 8 == 0 &&
+        reinterpret_cast<uintptr_t>(q_in.data_ptr()) % 16 == 0;
+    const Tensor q =
+        aligned ? q_in : q_in.clone(at::MemoryFormat::Contiguous);
+    const int nq = q.size(1), hd = q.size(2), nkv = k_cache.size(1);
+    const int bs = k_cache.size(2), W = block_table.size(1);
+    const int G = nq / nkv;
+    const long pairs = (long)nseq * nkv, rows = (long)max_qlen * G;
+    const int Z = attn_stream_splits(pairs, rows, (long)W * bs);
+    auto fopt = q.options().dtype(torch::kFloat32);
+    Tensor part_o, part_ml;
+    if (Z > 1) {
+        part_o = torch::empty({pairs * Z * rows, hd}, fopt);
+        part_ml = torch::empty({pairs * Z * rows, 2}, fopt);
+    }
+    return launch_attn_stream(
+               bf16p(q), k_cache.data_ptr(), v_cache.data_ptr(), cu,
+               block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
+               bf16p_mut(out), out_ml,
+               Z > 1 ? part_o.data_ptr<float>() : nullptr,
+               Z > 1 ? part_ml.data_ptr<float>() : nullptr, nseq, nkv, G, W,
+               bs, hd, Z, max_qlen, q.stride(0), (float)scale,
+               k_cache.scalar_type() == torch::kUInt8, stream()) == 0;
+}
+
 std::vector<Tensor> attn_decode_impl(const Tensor& q, const Tensor& k_cache,
                                      const Tensor& v_cache,
                                      const Tensor& block_table,
@@ -238,15 +278,19 @@ std::vector<Tensor> attn_decode_impl(const Tensor& q, const Tensor& k_cache,
     const int C = (W * bs + kDecChunk - 1) / kDecChunk;
     TORCH_CHECK(C <= 128, "decode supports up to 32768-token contexts for now");
     auto fopt = q.options().dtype(torch::kFloat32);
-    Tensor p_buf = torch::empty({B, nkv, C, kDecChunk, G}, q.options());
-    Tensor part_o = torch::empty({B, nkv, C, G, hd}, fopt);
-    Tensor part_ml = torch::empty({B, nkv, C, G, 2}, fopt);
     Tensor out_ml;
     float* out_ml_p = nullptr;
     if (want_lse) {
         out_ml = torch::empty({B, nq, 2}, fopt);
         out_ml_p = out_ml.data_ptr<float>();
     }
+    if (attn_stream(q, k_cache, v_cache, nullptr, B, block_table, seq_lens,
+                    out, out_ml_p, 1, scale))
+        return want_lse ? std::vector<Tensor>{out, out_ml}
+                        : std::vector<Tensor>{out};
+    Tensor p_buf = torch::empty({B, nkv, C, kDecChunk, G}, q.options());
+    Tensor part_o = torch::empty({B, nkv, C, G, hd}, fopt);
+    Tensor part_ml = torch::empty({B, nkv, C, G, 2}, fopt);
     launch_attn_decode(bf16p(q), k_cache.data_ptr(), v_cache.data_ptr(),
                        block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
                        bf16p_mut(p_buf), part_o.data_ptr<float>(),
@@ -318,6 +362,11 @@ Tensor attn_prefill_paged(const Tensor& q, const Tensor& k_cache,
     TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous());
     TORCH_CHECK(block_table.size(0) == nseq && seq_lens.size(0) == nseq);
     Tensor out = torch::empty({T, nq, hd}, q.options());
+    if (T > 0 && attn_stream_takes((long)nseq * nkv, max_qlen * (nq / nkv)) &&
+        attn_stream(q, k_cache, v_cache, cu_q.data_ptr<int>(), nseq,
+                    block_table, seq_lens, out, nullptr, (int)max_qlen,
+                    scale))
+        return out;
     launch_attn_prefill_paged(bf16p(q), k_cache.data_ptr(),
                               v_cache.data_ptr(), cu_q.data_ptr<int>(),
                               block_table.data_ptr<int>(),

@@ -1,0 +1,127 @@
+"""The one-pass paged attention of few query rows (attn_stream.hip) at the
+edges of its tiles, row tiles and splits, against the fp32 reference.
+
+Tolerance: a weight and an output element are rounded to bf16 once each
+(2^-9 relative), so an element is off by at most 2^-8 of the largest value;
+fp32 sums and exp2 add far less. 8-bit cache rows are exact in bf16."""
+import pytest
+import torch
+
+from bee2bee_amd import ops
+from bee2bee_amd.ops import reference
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _pages(nkv, hd, bs, total, fp8, seed, width=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    counts = [-(-n // bs) for n in total]
+    table = torch.zeros(len(total), max(counts + [width, 1]),
+                        dtype=torch.int32, device=DEV)
+    nb = sum(counts) + 1
+    ids = torch.randperm(nb, generator=g, device=DEV).int()
+    at = 0
+    for i, c in enumerate(counts):
+        table[i, :c] = ids[at : at + c]
+        at += c
+    caches = []
+    for _ in range(2):
+        c = torch.randn(nb, nkv, bs, hd, generator=g, device=DEV).bfloat16()
+        caches.append(c.to(torch.float8_e4m3fn).view(torch.uint8) if fp8
+                      else c)
+    lens = torch.tensor(total, dtype=torch.int32, device=DEV)
+    return caches[0], caches[1], table, lens
+
+
+def _wide(c):
+    return (c.view(torch.float8_e4m3fn) if c.dtype == torch.uint8
+            else c).float()
+
+
+def _check(got, want, v):
+    assert torch.isfinite(got).all()
+    err = (got.float() - want.float()).abs().max().item()
+    assert err <= v.max().item() * 2 ** -8, err
+
+
+# (heads, key heads, head size, contexts, page size, table width)
+DECODE = [
+    (4, 4, 64, [1], 256, 1), (8, 1, 128, [31, 32, 33, 127, 128, 129], 64, 0),
+    (7, 1, 128, [1000, 1, 255, 256, 257], 256, 16), (12, 12, 64, [300], 16, 4),
+    (6, 2, 128, [77, 129], 24, 0), (16, 1, 64, [3000, 40], 256, 32),
+    (32, 8, 128, [5 + 37 * i for i in range(40)], 256, 0),
+    (28, 4, 128, [9000, 200], 256, 64),
+]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("nq,nkv,hd,total,bs,width", DECODE)
+def test_decode(nq, nkv, hd, total, bs, width, fp8):
+    kc, vc, table, lens = _pages(nkv, hd, bs, total, fp8, 1, width)
+    q = torch.randn(len(total), nq, hd, device=DEV).bfloat16()
+    scale = 0.8 * hd ** -0.5
+    got, ml = ops.attn_decode_lse(q, kc, vc, table, lens, scale)
+    qf = q.float()
+    if fp8:     # decode queries are rounded to the cache's type, scaled
+        qf = (qf * scale).bfloat16().to(torch.float8_e4m3fn).float() / scale
+    want, want_ml = reference.attn_decode_lse(
+        qf, _wide(kc), _wide(vc), table, lens, scale)
+    _check(got, want, _wide(vc))
+    # the (m, l) pair that ranks merge: l e^m is the sum of e^score
+    assert torch.allclose(ml[..., 0] + ml[..., 1].log(),
+                          want_ml[..., 0] + want_ml[..., 1].log(), atol=2e-3)
+    assert torch.equal(ops.attn_decode(q, kc, vc, table, lens, scale), got)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("nq,nkv,hd,new,old,bs", [
+    (32, 8, 128, [5, 1, 4], [1500, 0, 251], 256),
+    (32, 8, 64, [8, 3], [77, 1000], 16), (28, 4, 128, [8, 5, 2], [999, 3, 60],
+                                          256),
+    (6, 2, 128, [11, 0, 1], [100, 40, 300], 24),
+    (12, 12, 64, [17, 33], [300, 31], 64), (32, 8, 128, [64], [2000], 256),
+])
+def test_chunks_of_a_few_tokens(nq, nkv, hd, new, old, bs, fp8):
+    total = [a + b for a, b in zip(new, old)]
+    kc, vc, table, lens = _pages(nkv, hd, bs, total, fp8, 2)
+    q = torch.randn(sum(new), nq, hd, device=DEV).bfloat16()
+    cu = torch.tensor([0] + torch.tensor(new).cumsum(0).tolist(),
+                      dtype=torch.int32, device=DEV)
+    scale = hd ** -0.5
+    got = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, max(new), scale)
+    want = reference.attn_decode_with_history(
+        q.float(), _wide(kc), _wide(vc), table, lens,
+        torch.tensor(new, dtype=torch.int32), scale)
+    _check(got, want, _wide(vc))
+
+
+def test_a_verified_token_gets_the_sums_of_decoding():
+    """A row's result is the same whether its token is decoded or verified
+    with others (16 rows in one tile either way)."""
+    total, new = [700, 1300], 3
+    kc, vc, table, lens = _pages(8, 128, 256, total, False, 3)
+    q = torch.randn(2 * new, 32, 128, device=DEV).bfloat16()
+    cu = torch.tensor([0, new, 2 * new], dtype=torch.int32, device=DEV)
+    rows = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, new, 0.1)
+    last = ops.attn_decode(q[new - 1 :: new], kc, vc, table, lens, 0.1)
+    assert torch.equal(rows[new - 1 :: new], last)
+
+
+def test_queries_at_odd_addresses_and_other_scales():
+    kc, vc, table, lens = _pages(2, 64, 32, [70, 5], False, 4)
+    flat = torch.randn(2 * (4 * 64 + 1) + 1, device=DEV).bfloat16()
+    q = flat[1:].as_strided((2, 4, 64), (4 * 64 + 1, 64, 1), 1)
+    for scale in (0.2, 0.0, -0.1):
+        got = ops.attn_decode(q, kc, vc, table, lens, scale)
+        want = reference.attn_decode(q.float(), kc.float(), vc.float(), table,
+                                     lens, scale)
+        _check(got, want, vc.float())
+
+
+def test_an_empty_context_is_zero():
+    kc, vc, table, lens = _pages(1, 64, 32, [40, 40], False, 5)
+    lens[1] = 0
+    q = torch.randn(2, 4, 64, device=DEV).bfloat16()
+    out, ml = ops.attn_decode_lse(q, kc, vc, table, lens, 0.125)
+    assert (out[1] == 0).all() and (ml[1, :, 1] == 0).all()
