@@ -70,6 +70,14 @@ class Runner:
         self.rope_cos, self.rope_sin = cos, sin
 
     @property
+    def _rows_dims(self) -> bool:
+        """Stacks whose steps of a few rows run on ops.rows_linear: dense
+        ones with sizes of whole matrix-core steps."""
+        s = self.spec
+        return not (s.is_hybrid or s.is_moe or s.hidden_size % 32
+                    or s.q_size % 32 or s.intermediate_size % 32)
+
+    @property
     def is_first_stage(self) -> bool:
         return self.layer_lo == 0
 
@@ -122,9 +130,63 @@ class Runner:
                 hidden.contiguous(), self.weights.final_gain,
                 self.spec.rms_eps, self.dtype)
             return F.linear(normed, self.weights.lm_head)
-        normed = self._norm(hidden, self.weights.final_norm,
-                            self.weights.final_norm_bias)
-        return F.linear(normed, self.weights.lm_head)
+        W = self.weights
+        if self._rows_dims and ops.few_rows(hidden):
+            return ops.rows_linear(
+                hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
+                                         self.spec.rms_eps))
+        normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
+        return F.linear(normed, W.lm_head)
+
+    def _layer_rows(
+        self,
+        layer_idx: int,
+        x: torch.Tensor,
+        positions: torch.Tensor,
+        slot_mapping: torch.Tensor,
+        attn_fn,
+        paged: bool,
+    ) -> torch.Tensor:
+        """A dense layer on a few rows: five launches, each projection with
+        its norm, and bias, activation or residual add, folded in. paged:
+        attention reads the pages only, so rotation and store go into the
+        q|k|v projection too."""
+        s, lw = self.spec, self.weights.layers[layer_idx]
+        T = x.shape[0]
+        k_cache, v_cache = self.kv.layer(layer_idx)
+        norm = (lw.attn_norm, lw.attn_norm_bias, s.rms_eps)
+        rope = s.pos_type == "rope"
+        if paged and s.head_dim % 32 == 0:
+            k = v = None
+            q = ops.rows_qkv(x, lw.wqkv, lw.wqkv_bias, norm, s.n_heads,
+                             positions if rope else None, self.rope_cos,
+                             self.rope_sin, k_cache, v_cache, slot_mapping)
+        else:
+            qkv = ops.rows_linear(x, lw.wqkv, lw.wqkv_bias, norm=norm).view(
+                T, -1, s.head_dim)
+            q, k, v = qkv.split([s.n_heads, s.n_kv_heads, s.n_kv_heads], 1)
+            if rope:
+                ops.rope_inplace(q, k, positions, self.rope_cos,
+                                 self.rope_sin)
+            ops.kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
+        o = attn_fn(layer_idx, q, k, v, k_cache, v_cache)
+        x = self._rows_add(x, o.reshape(T, s.q_size), lw.wo, lw.wo_bias)
+        norm = (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps)
+        act = ops.rows_linear(x, lw.w_gate_up, lw.w_gate_up_bias, norm=norm,
+                              act="gelu" if s.act_type == "gelu" else "swiglu")
+        return self._rows_add(x, act, lw.w_down, lw.w_down_bias)
+
+    def _rows_add(self, x, y, w, bias) -> torch.Tensor:
+        """x + y w^T + bias; under tensor parallelism y and w are this rank's
+        part of the inner dimension."""
+        if self.tp_group is not None:
+            import torch.distributed as dist
+
+            if dist.get_world_size(self.tp_group) > 1:
+                part = ops.rows_linear(y, w, bias)
+                dist.all_reduce(part, group=self.tp_group)
+                return x + part
+        return ops.rows_linear(y, w, bias, x)
 
     def _layer(
         self,
@@ -385,7 +447,13 @@ class Runner:
         positions: torch.Tensor,
         slot_mapping: torch.Tensor,
         attn_fn,
+        paged: bool = True,
     ) -> torch.Tensor:
+        if self._rows_dims and ops.few_rows(hidden):
+            for layer_idx in range(self.layer_lo, self.layer_hi):
+                hidden = self._layer_rows(layer_idx, hidden, positions,
+                                          slot_mapping, attn_fn, paged)
+            return hidden
         residual = None
         for layer_idx in range(self.layer_lo, self.layer_hi):
             hidden, residual = self._layer(
@@ -435,7 +503,7 @@ class Runner:
             if self.is_first_stage
             else input_ids_or_hidden
         )
-        return self._run_layers(hidden, positions, slot_mapping, attn)
+        return self._run_layers(hidden, positions, slot_mapping, attn, chunked)
 
     def forward_decode(
         self,

@@ -222,6 +222,45 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     return reference.swiglu(gate_up)
 
 
+# ---------------------------------------------------- steps of a few rows
+# One launch a projection, with the norm before it and what follows it folded
+# in. norm: (weight, bias or None, eps) - with a bias layer norm, without RMS
+# norm.
+
+ROWS_MAX = 16
+
+
+def few_rows(x: torch.Tensor) -> bool:
+    """Steps that the few-row projections take: 1 to ROWS_MAX contiguous,
+    16-byte aligned bf16 rows on the GPU."""
+    return (x.dim() == 2 and 1 <= x.shape[0] <= ROWS_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous()
+            and x.data_ptr() % 16 == 0)
+
+
+def rows_linear(x, w, bias=None, resid=None, norm=None, act=None):
+    """act(norm(x) w^T + bias) + resid. act: None, "gelu" (tanh form), or
+    "swiglu" (w holds the gate's rows, then the values'; no bias)."""
+    if _use_hip(x):
+        nw, nb, eps = norm or (None, None, 0.0)
+        return require_hip().rows_linear(
+            x, w, bias, resid, nw, nb, eps,
+            {None: 0, "swiglu": 1, "gelu": 2}[act])
+    return reference.rows_linear(x, w, bias, resid, norm, act)
+
+
+def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
+             v_cache, slot_mapping):
+    """norm(x) w^T + bias split into q|k|v; q and k rotated (positions None:
+    not), k and v stored into their pages. -> q [T, n_heads, hd]."""
+    if _use_hip(x):
+        return require_hip().rows_qkv(x, w, bias, norm[0], norm[1], norm[2],
+                                      n_heads, positions, cos, sin, k_cache,
+                                      v_cache, slot_mapping)
+    return reference.rows_qkv(x, w, bias, norm, n_heads, positions, cos, sin,
+                              k_cache, v_cache, slot_mapping)
+
+
 def moe_topk_gate(logits: torch.Tensor, top_k: int):
     # gating math is tiny ([T, E]); torch ops are fine on both devices
     return reference.moe_topk_gate(logits, top_k)

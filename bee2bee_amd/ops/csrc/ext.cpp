@@ -454,6 +454,7 @@ void register_gated_ops(pybind11::module_& m);  // gated_ext.cpp
 void register_tanh_ops(pybind11::module_& m);  // tanh_ext.cpp
 void register_moe_ops(pybind11::module_& m);  // moe_ext.cpp
 void register_scaled_ops(pybind11::module_& m);  // scaled_ext.cpp
+void register_rows_ops(pybind11::module_& m);  // rows_ext.cpp
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     register_hybrid_ops(m);
@@ -462,6 +463,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     register_tanh_ops(m);
     register_moe_ops(m);
     register_scaled_ops(m);
+    register_rows_ops(m);
     m.def("rmsnorm", &rmsnorm, "fused RMSNorm (bf16)");
     m.def("fused_add_rmsnorm", &fused_add_rmsnorm,
           "residual += x; y = rmsnorm(residual)");

@@ -1,0 +1,143 @@
+// Torch bindings of the projections of a few rows (linear_rows.hip).
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+#include <hip/hip_runtime.h>
+
+using torch::Tensor;
+using c10::optional;
+
+extern "C" int launch_linear_rows(
+    const unsigned short*, const unsigned short*, const unsigned short*,
+    const unsigned short*, const unsigned short*, const unsigned short*,
+    unsigned short*, int, int, int, float, int, int, const int*, const float*,
+    const float*, const int*, void*, void*, int, int, int, int, int,
+    hipStream_t);
+
+namespace {
+
+enum { EPI_PLAIN = 0, EPI_GLU = 1, EPI_GELU = 2, EPI_QKV = 3 };
+
+hipStream_t stream() {
+    return at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+}
+
+// t as the kernel reads it: contiguous, 16-byte aligned (copied if it is not)
+Tensor dense(const Tensor& t, const char* name) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16, name,
+                " must be bf16 on the GPU");
+    if (t.is_contiguous() &&
+        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0)
+        return t;
+    return t.clone(at::MemoryFormat::Contiguous);
+}
+
+// one value a column; undefined without the tensor
+Tensor column(const optional<Tensor>& t, long n, const char* name) {
+    if (!t.has_value()) return Tensor();
+    TORCH_CHECK(t->numel() == n, name, " must have ", n, " values");
+    return dense(*t, name);
+}
+
+const unsigned short* ptr(const Tensor& t) {
+    return t.defined()
+               ? reinterpret_cast<const unsigned short*>(t.data_ptr())
+               : nullptr;
+}
+
+struct Rows {
+    Tensor x, w, norm_w, norm_b;
+    int M, N, K, norm;
+};
+
+Rows rows_of(const Tensor& x, const Tensor& w, const optional<Tensor>& norm_w,
+             const optional<Tensor>& norm_b) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
+                "x [M, K] and w [N, K]");
+    Rows r;
+    r.M = x.size(0);
+    r.K = x.size(1);
+    r.N = w.size(0);
+    TORCH_CHECK(r.M >= 1 && r.M <= 16, "1 to 16 rows");
+    TORCH_CHECK(r.K % 32 == 0, "K must be a multiple of 32");
+    TORCH_CHECK(norm_w.has_value() || !norm_b.has_value());
+    r.x = dense(x, "x");
+    r.w = dense(w, "w");
+    r.norm_w = column(norm_w, r.K, "norm weight");
+    r.norm_b = column(norm_b, r.K, "norm bias");
+    r.norm = !norm_w.has_value() ? 0 : norm_b.has_value() ? 2 : 1;
+    return r;
+}
+
+// norm_b given: layer norm; norm_w alone: RMS norm
+Tensor rows_linear(const Tensor& x, const Tensor& w,
+                   const optional<Tensor>& bias,
+                   const optional<Tensor>& resid,
+                   const optional<Tensor>& norm_w,
+                   const optional<Tensor>& norm_b, double eps, int64_t act) {
+    const Rows r = rows_of(x, w, norm_w, norm_b);
+    TORCH_CHECK(act == EPI_PLAIN || act == EPI_GLU || act == EPI_GELU);
+    TORCH_CHECK(act != EPI_GLU || (r.N % 32 == 0 && !bias.has_value()));
+    TORCH_CHECK(act == EPI_PLAIN || !resid.has_value());
+    const int N = act == EPI_GLU ? r.N / 2 : r.N;
+    if (resid.has_value())
+        TORCH_CHECK(resid->dim() == 2 && resid->size(0) == r.M &&
+                    resid->size(1) == N, "resid [M, N]");
+    const Tensor b = column(bias, N, "bias");
+    const Tensor add = resid.has_value() ? dense(*resid, "resid") : Tensor();
+    Tensor y = torch::empty({r.M, N}, x.options());
+    TORCH_CHECK(launch_linear_rows(
+                    ptr(r.x), ptr(r.norm_w), ptr(r.norm_b), ptr(r.w), ptr(b),
+                    ptr(add),
+                    reinterpret_cast<unsigned short*>(y.data_ptr()), r.M, N,
+                    r.K, (float)eps, r.norm, (int)act, nullptr, nullptr,
+                    nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0,
+                    stream()) == 0);
+    return y;
+}
+
+// -> rotated queries [M, nq, hd]; rotated keys and the values go to the pages
+Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
+                const Tensor& norm_w, const optional<Tensor>& norm_b,
+                double eps, int64_t nq, const optional<Tensor>& pos,
+                const optional<Tensor>& cos_t, const optional<Tensor>& sin_t,
+                Tensor& k_cache, Tensor& v_cache, const Tensor& slots) {
+    const Rows r = rows_of(x, w, norm_w, norm_b);
+    const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
+    TORCH_CHECK(k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
+                k_cache.scalar_type() == v_cache.scalar_type() &&
+                k_cache.is_contiguous() && v_cache.is_contiguous());
+    TORCH_CHECK(fp8 || k_cache.scalar_type() == torch::kBFloat16);
+    const int nkv = k_cache.size(1), bs = k_cache.size(2),
+              hd = k_cache.size(3);
+    TORCH_CHECK(hd % 32 == 0 && r.N == (nq + 2 * nkv) * hd);
+    TORCH_CHECK(slots.scalar_type() == torch::kInt32 &&
+                slots.is_contiguous() && slots.numel() == r.M);
+    if (pos.has_value()) {
+        TORCH_CHECK(pos->scalar_type() == torch::kInt32 &&
+                    pos->is_contiguous() && pos->numel() == r.M);
+        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
+            TORCH_CHECK(t->scalar_type() == torch::kFloat32 &&
+                        t->is_contiguous() && t->size(1) == hd / 2);
+    }
+    const Tensor b = column(bias, r.N, "bias");
+    Tensor q = torch::empty({r.M, nq, hd}, x.options());
+    TORCH_CHECK(launch_linear_rows(
+                    ptr(r.x), ptr(r.norm_w), ptr(r.norm_b), ptr(r.w), ptr(b),
+                    nullptr, reinterpret_cast<unsigned short*>(q.data_ptr()),
+                    r.M, r.N, r.K, (float)eps, r.norm, EPI_QKV,
+                    pos.has_value() ? pos->data_ptr<int>() : nullptr,
+                    pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
+                    pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
+                    slots.data_ptr<int>(), k_cache.data_ptr(),
+                    v_cache.data_ptr(), nq, nkv, hd, bs, fp8, stream()) == 0);
+    return q;
+}
+
+}  // namespace
+
+void register_rows_ops(pybind11::module_& m) {
+    m.def("rows_linear", &rows_linear,
+          "projection of a few rows: norm, product, bias, activation, residual");
+    m.def("rows_qkv", &rows_qkv,
+          "norm, q|k|v projection, rotation and page store of a few rows");
+}

@@ -293,6 +293,29 @@ def grouped_gemm(
     return out
 
 
+def rows_linear(x, w, bias=None, resid=None, norm=None, act=None):
+    """act(norm(x) w^T + bias) + resid; norm (weight, bias or None, eps)."""
+    if norm is not None:
+        x = (rmsnorm(x, norm[0], norm[2]) if norm[1] is None
+             else layernorm(x, *norm))
+    y = torch.nn.functional.linear(x, w, bias)
+    if act is not None:
+        y = gelu(y) if act == "gelu" else swiglu(y)
+    return y if resid is None else (y.float() + resid.float()).to(x.dtype)
+
+
+def rows_qkv(x, w, bias, norm, n_heads, positions, cos, sin, k_cache, v_cache,
+             slot_mapping):
+    """Normed q|k|v projection, rotation and page store; -> q [T, nq, hd]."""
+    nkv, hd = k_cache.shape[1], k_cache.shape[3]
+    qkv = rows_linear(x, w, bias, norm=norm).view(x.shape[0], -1, hd)
+    q, k, v = qkv.split([n_heads, nkv, nkv], dim=1)
+    if positions is not None:
+        rope_inplace(q, k, positions, cos, sin)
+    kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
+    return q.contiguous()
+
+
 def attn_decode_lse(
     q: torch.Tensor,
     k_cache: torch.Tensor,

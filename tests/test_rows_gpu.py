@@ -1,0 +1,144 @@
+"""Projections of a few rows (linear_rows.hip) at the edges of their tiles, of
+the waves' shares of K and of the kernel shapes, against fp32.
+
+Tolerance: the normed input and the output are rounded to bf16 (2^-9 relative,
+half of it more for the weight folded in first): an element is off by at most
+2^-8 of the sum of its products' magnitudes, carried through the activation
+(whose slope is below 1.13), and 2^-8 of itself."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from bee2bee_amd import ops
+from bee2bee_amd.ops import reference
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rand(*shape, std=1.0, mean=0.0):
+    return (torch.randn(*shape, device=DEV) * std + mean).bfloat16()
+
+
+def _norm(kind, K):
+    if kind is None:
+        return None
+    b = _rand(K, std=0.1) if kind == "layer" else None
+    return (_rand(K, std=0.1, mean=1.0), b, 1e-5)
+
+
+def _f32(norm):
+    return norm and (norm[0].float(),
+                     None if norm[1] is None else norm[1].float(), norm[2])
+
+
+def _products(x, w, norm):
+    """fp32 product and the sum of its terms' magnitudes."""
+    h = x.float()
+    if norm is not None:
+        n = _f32(norm)
+        h = (reference.rmsnorm(h, n[0], n[2]) if n[1] is None
+             else reference.layernorm(h, *n))
+    return h @ w.float().t(), h.abs() @ w.float().abs().t()
+
+
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K", [
+    (16, 32), (17, 64), (50257, 96), (768, 3072), (4096, 2048), (4112, 256),
+    (4608, 3584), (1000, 4096 + 32),
+])
+@pytest.mark.parametrize("kind", [None, "rms", "layer"])
+def test_plain(M, N, K, kind):
+    torch.manual_seed(M + N)
+    x, w, b, r = _rand(M, K), _rand(N, K, std=0.05), _rand(N), _rand(M, N)
+    norm = _norm(kind, K)
+    got = ops.rows_linear(x, w, b, r, norm).float()
+    y, mag = _products(x, w, norm)
+    want = y + b.float() + r.float()
+    assert ((got - want).abs() <= 2 ** -8 * (mag + want.abs()) + 1e-5).all()
+    if N > 16:    # bare, and rows at an odd address
+        flat = _rand(M * K + 1)
+        xo = flat[1:].view(M, K)
+        got = ops.rows_linear(xo, w).float()
+        y, mag = _products(xo, w, None)
+        assert ((got - y).abs() <= 2 ** -8 * (mag + y.abs()) + 1e-5).all()
+
+
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("I,K", [(16, 64), (8192, 2048), (48, 3072 + 96)])
+def test_activations(M, I, K):
+    torch.manual_seed(M + I)
+    x, w, norm = _rand(M, K), _rand(2 * I, K, std=0.03), _norm("rms", K)
+    got = ops.rows_linear(x, w, norm=norm, act="swiglu").float()
+    y, mag = _products(x, w, norm)
+    (g, u), (mg, mu) = y.chunk(2, -1), mag.chunk(2, -1)
+    want = F.silu(g) * u
+    bound = 2 ** -8 * (1.13 * mg * u.abs() + F.silu(g).abs() * mu
+                       + want.abs()) + 2 ** -16 * mg * mu
+    assert ((got - want).abs() <= bound + 1e-5).all()
+    norm, b = _norm("layer", K), _rand(2 * I)
+    got = ops.rows_linear(x, w, b, norm=norm, act="gelu").float()
+    y, mag = _products(x, w, norm)
+    want = F.gelu(y + b.float(), approximate="tanh")
+    assert ((got - want).abs()
+            <= 2 ** -8 * (1.13 * mag + want.abs()) + 1e-5).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,nq,nkv,hd,K,kind", [
+    (1, 32, 8, 128, 256, "rms"), (16, 7, 1, 64, 96, "rms"),
+    (3, 12, 12, 64, 768, "layer"), (2, 2, 1, 32, 64, "rms"),
+])
+def test_qkv(M, nq, nkv, hd, K, kind, fp8):
+    torch.manual_seed(M)
+    N = (nq + 2 * nkv) * hd
+    x, w, b, norm = _rand(M, K), _rand(N, K, std=0.1), _rand(N), \
+        _norm(kind, K)
+    cos, sin = reference.rope_tables(64, hd, 1e4, DEV)
+    pos = torch.arange(M, device=DEV, dtype=torch.int32) * 3 + 1
+    rope = kind == "rms"
+    nb, bs = 3, 24
+    dt = torch.uint8 if fp8 else torch.bfloat16
+    kc = torch.zeros(nb, nkv, bs, hd, device=DEV, dtype=dt)
+    vc = torch.zeros_like(kc)
+    slots = torch.randperm(nb * bs, device=DEV)[:M].int()
+    q = ops.rows_qkv(x, w, b, norm, nq, pos if rope else None, cos, sin, kc,
+                     vc, slots)
+    y, mag = _products(x, w, norm)
+    y = (y + b.float()).view(M, -1, hd)
+    # a rotated element mixes two products
+    mag = mag.view(M, -1, hd) + y.abs()
+    mag = mag + mag.roll(hd // 2, -1)
+    wq, wk, wv = (t.clone() for t in y.split([nq, nkv, nkv], 1))
+    if rope:
+        reference.rope_inplace(wq, wk, pos, cos, sin)
+    mq, mk, mv = mag.split([nq, nkv, nkv], 1)
+    assert ((q.float() - wq).abs() <= 2 ** -8 * mq + 1e-5).all()
+    s = slots.long()
+    for cache, want, m in ((kc, wk, mk), (vc, wv, mv)):
+        rows = cache[s // bs, :, s % bs]
+        step = 2 ** -8
+        if fp8:      # and one rounding to 3 mantissa bits
+            rows, step = rows.view(torch.float8_e4m3fn), 2 ** -8 + 2 ** -4
+        assert ((rows.float() - want).abs() <= step * m + 2 ** -9).all()
+        rest = cache.clone()
+        rest[s // bs, :, s % bs] = 0
+        assert (rest == 0).all()
+
+
+def test_a_row_does_not_depend_on_the_others():
+    torch.manual_seed(0)
+    x, w, norm = _rand(16, 4096), _rand(6144, 4096, std=0.02), \
+        _norm("rms", 4096)
+    full = ops.rows_linear(x, w, norm=norm)
+    for rows in (slice(0, 1), slice(7, 12)):
+        part = ops.rows_linear(x[rows].contiguous(), w, norm=norm)
+        assert torch.equal(part, full[rows])
+
+
+def test_refused():
+    x, w = _rand(17, 64), _rand(32, 64)
+    with pytest.raises(RuntimeError):
+        ops.rows_linear(x, w)
+    with pytest.raises(RuntimeError):
+        ops.rows_linear(x[:4, :40].contiguous(), w[:, :40].contiguous())
