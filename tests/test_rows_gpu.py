@@ -13,6 +13,10 @@ from bee2bee_amd import ops
 from bee2bee_amd.ops import reference
 
 pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
 DEV = "cuda"
 
 
