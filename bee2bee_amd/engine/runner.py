@@ -78,6 +78,21 @@ class Runner:
                     or s.q_size % 32 or s.intermediate_size % 32)
 
     @property
+    def _mid_dims(self) -> bool:
+        """Stacks whose steps of some tens of rows run on ops.mid_linear; a
+        tensor-parallel rank's rows are reduced before they are added."""
+        s = self.spec
+        if not self._rows_dims or s.hidden_size % 64 or s.q_size % 64 or \
+                s.intermediate_size % 64 or s.hidden_size > 8192 or \
+                s.head_dim % 16:
+            return False
+        if self.tp_group is None:
+            return True
+        import torch.distributed as dist
+
+        return dist.get_world_size(self.tp_group) == 1
+
+    @property
     def is_first_stage(self) -> bool:
         return self.layer_lo == 0
 
@@ -157,24 +172,73 @@ class Runner:
         norm = (lw.attn_norm, lw.attn_norm_bias, s.rms_eps)
         rope = s.pos_type == "rope"
         if paged and s.head_dim % 32 == 0:
-            k = v = None
             q = ops.rows_qkv(x, lw.wqkv, lw.wqkv_bias, norm, s.n_heads,
                              positions if rope else None, self.rope_cos,
                              self.rope_sin, k_cache, v_cache, slot_mapping)
+            o = attn_fn(layer_idx, q, None, None, k_cache, v_cache)
         else:
-            qkv = ops.rows_linear(x, lw.wqkv, lw.wqkv_bias, norm=norm).view(
-                T, -1, s.head_dim)
-            q, k, v = qkv.split([s.n_heads, s.n_kv_heads, s.n_kv_heads], 1)
-            if rope:
-                ops.rope_inplace(q, k, positions, self.rope_cos,
-                                 self.rope_sin)
-            ops.kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
-        o = attn_fn(layer_idx, q, k, v, k_cache, v_cache)
+            o = self._attend(layer_idx,
+                             ops.rows_linear(x, lw.wqkv, norm=norm),
+                             positions, slot_mapping, attn_fn)
         x = self._rows_add(x, o.reshape(T, s.q_size), lw.wo, lw.wo_bias)
         norm = (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps)
         act = ops.rows_linear(x, lw.w_gate_up, lw.w_gate_up_bias, norm=norm,
                               act="gelu" if s.act_type == "gelu" else "swiglu")
         return self._rows_add(x, act, lw.w_down, lw.w_down_bias)
+
+    def _attend(self, layer_idx: int, qkv, positions, slot_mapping, attn_fn):
+        """Attention of a layer on its projected q|k|v: rows [T, N], or their
+        parts [S, T, N]. Bias, rotation and page store are one kernel (head
+        sizes of whole 16-element pieces)."""
+        s, lw = self.spec, self.weights.layers[layer_idx]
+        k_cache, v_cache = self.kv.layer(layer_idx)
+        rope = s.pos_type == "rope"
+        fused = s.head_dim % 16 == 0
+        if fused:
+            qkv = ops.rope_store_qkv(
+                qkv, lw.wqkv_bias, s.n_heads, positions if rope else None,
+                self.rope_cos, self.rope_sin, k_cache, v_cache, slot_mapping)
+        elif lw.wqkv_bias is not None:
+            qkv = qkv + lw.wqkv_bias
+        q, k, v = qkv.view(qkv.shape[0], -1, s.head_dim).split(
+            [s.n_heads, s.n_kv_heads, s.n_kv_heads], 1)
+        if not fused:
+            if rope:
+                ops.rope_inplace(q, k, positions, self.rope_cos,
+                                 self.rope_sin)
+            ops.kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
+        return attn_fn(layer_idx, q, k, v, k_cache, v_cache)
+
+    def _run_layers_mid(
+        self,
+        x: torch.Tensor,
+        positions: torch.Tensor,
+        slot_mapping: torch.Tensor,
+        attn_fn,
+    ) -> torch.Tensor:
+        """Dense layers on some tens of rows: the narrow projections as parts
+        over K, summed by the kernels that read them."""
+        s, T = self.spec, x.shape[0]
+        layers = self.weights.layers
+        gelu = s.act_type == "gelu"
+        lw = layers[self.layer_lo]
+        normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
+        for i in range(self.layer_lo, self.layer_hi):
+            lw = layers[i]
+            o = self._attend(i, ops.mid_linear(normed, lw.wqkv), positions,
+                             slot_mapping, attn_fn)
+            normed, x = ops.add_norm_parts(
+                ops.mid_linear(o.reshape(T, s.q_size), lw.wo), lw.wo_bias, x,
+                (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps))
+            z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
+            z = ops.gelu(z) if gelu else ops.swiglu(z)
+            nxt = None
+            if i + 1 < self.layer_hi:
+                nxt = (layers[i + 1].attn_norm, layers[i + 1].attn_norm_bias,
+                       s.rms_eps)
+            normed, x = ops.add_norm_parts(ops.mid_linear(z, lw.w_down),
+                                           lw.w_down_bias, x, nxt)
+        return x
 
     def _rows_add(self, x, y, w, bias) -> torch.Tensor:
         """x + y w^T + bias; under tensor parallelism y and w are this rank's
@@ -208,18 +272,9 @@ class Runner:
             )
 
         qkv = F.linear(normed, lw.wqkv)  # column-parallel under TP
-        if lw.wqkv_bias is not None:  # Qwen2-style attention bias
-            qkv = qkv + lw.wqkv_bias
         T = qkv.shape[0]
-        q, k, v = qkv.split([s.q_size, s.kv_size, s.kv_size], dim=-1)
-        q = q.view(T, s.n_heads, s.head_dim)
-        k = k.view(T, s.n_kv_heads, s.head_dim)
-        v = v.view(T, s.n_kv_heads, s.head_dim)
-        if s.pos_type == "rope":
-            ops.rope_inplace(q, k, positions, self.rope_cos, self.rope_sin)
-        k_cache, v_cache = self.kv.layer(layer_idx)
-        ops.kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
-        attn_out = attn_fn(layer_idx, q, k, v, k_cache, v_cache)
+        attn_out = self._attend(layer_idx, qkv, positions, slot_mapping,
+                                attn_fn)
         attn_out = F.linear(attn_out.reshape(T, s.q_size), lw.wo, lw.wo_bias)
         if self.tp_group is not None:
             # row-parallel o-projection: sum the per-shard partials
@@ -454,6 +509,9 @@ class Runner:
                 hidden = self._layer_rows(layer_idx, hidden, positions,
                                           slot_mapping, attn_fn, paged)
             return hidden
+        if self._mid_dims and ops.mid_rows(hidden):
+            return self._run_layers_mid(hidden, positions, slot_mapping,
+                                        attn_fn)
         residual = None
         for layer_idx in range(self.layer_lo, self.layer_hi):
             hidden, residual = self._layer(

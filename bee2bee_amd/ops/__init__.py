@@ -261,6 +261,46 @@ def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
                               k_cache, v_cache, slot_mapping)
 
 
+# Steps of some tens of rows: narrow projections as fp32 parts over their inner
+# dimension, which the next kernel sums.
+
+MID_MAX = 128
+
+
+def mid_rows(x: torch.Tensor) -> bool:
+    """Steps of ROWS_MAX + 1 to MID_MAX contiguous bf16 rows on the GPU."""
+    return (x.dim() == 2 and ROWS_MAX < x.shape[0] <= MID_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous())
+
+
+def mid_linear(x, w):
+    """Parts [S, T, N] fp32 whose sum over S is x w^T."""
+    if _use_hip(x):
+        return require_hip().mid_linear(x, w)
+    return reference.mid_linear(x, w)
+
+
+def add_norm_parts(part, bias, resid, norm=None):
+    """-> (norm(resid + parts + bias) or None without a norm, that sum)."""
+    if _use_hip(resid):
+        nw, nb, eps = norm or (None, None, 0.0)
+        return require_hip().add_norm_parts(part, bias, resid, nw, nb, eps)
+    return reference.add_norm_parts(part, bias, resid, norm)
+
+
+def rope_store_qkv(qkv, bias, n_heads: int, positions, cos, sin, k_cache,
+                   v_cache, slot_mapping):
+    """qkv: rows [T, N] (changed in place) or parts [S, T, N]. Bias added, q
+    and k rotated (positions None: not), k and v stored into their pages. ->
+    [T, N]."""
+    if _use_hip(qkv):
+        return require_hip().rope_store_qkv(qkv, bias, n_heads, positions,
+                                            cos, sin, k_cache, v_cache,
+                                            slot_mapping)
+    return reference.rope_store_qkv(qkv, bias, n_heads, positions, cos, sin,
+                                    k_cache, v_cache, slot_mapping)
+
+
 def moe_topk_gate(logits: torch.Tensor, top_k: int):
     # gating math is tiny ([T, E]); torch ops are fine on both devices
     return reference.moe_topk_gate(logits, top_k)

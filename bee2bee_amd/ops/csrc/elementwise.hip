@@ -242,6 +242,108 @@ __global__ void kv_store_fp8_kernel(
     }
 }
 
+// ------------------------------------------------------------- rope_store
+// What stands between the q|k|v projection and attention, in one pass: the
+// projection's parts summed (S > 0: fp32 [S, T, N]) or its bf16 rows taken
+// (S == 0, in qkv itself), bias added, q and k rotated (pos null: not), the
+// result left in qkv [T, N] and k and v scattered into the paged pool (bf16,
+// or OCP fp8 bytes). A thread takes 8 coordinates of a head's first half and
+// their partners in the second. Bound by its bytes at thousands of tokens (8512
+// tokens of 28 + 2x4 heads of 128: 38 us with the bias; as an add, a rotation
+// of 2-byte accesses and a copy it was 44 + 64 + 12), by its launch at tens.
+template <typename CT>
+__global__ __launch_bounds__(256) void qkv_rope_store_kernel(
+    const float* __restrict__ part, int S, unsigned short* __restrict__ qkv,
+    const unsigned short* __restrict__ bias, const int* __restrict__ pos,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    CT* __restrict__ k_cache, CT* __restrict__ v_cache,
+    const int* __restrict__ slots, long T, int nq, int nkv, int hd, int bs) {
+    const int heads = nq + 2 * nkv, half = hd / 2, per = hd / 16;
+    const long idx = blockIdx.x * 256L + threadIdx.x;
+    const int c = idx % per;
+    const int h = idx / per % heads;
+    const long t = idx / per / heads;
+    if (t >= T) return;
+    const int N = heads * hd, d = c * 8, n = h * hd + d;
+    unsigned short* row = qkv + t * N + n;
+    float a[8], b[8];
+    if (S > 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.f;
+        for (int s = 0; s < S; ++s) {
+            const float* p = part + ((long)s * T + t) * N + n;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const f32x4 u = reinterpret_cast<const f32x4*>(p)[q];
+                const f32x4 w = reinterpret_cast<const f32x4*>(p + half)[q];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a[q * 4 + e] += u[e];
+                    b[q * 4 + e] += w[e];
+                }
+            }
+        }
+    } else {
+        load_bf16x8(row, a);
+        load_bf16x8(row + half, b);
+    }
+    if (bias) {
+        float u[8], w[8];
+        load_bf16x8(bias + n, u);
+        load_bf16x8(bias + n + half, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            a[e] += u[e];
+            b[e] += w[e];
+        }
+    }
+    const bool turns = pos && h < nq + nkv;
+    if (turns) {
+        const long tab = (long)pos[t] * half + d;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const f32x4 cs = reinterpret_cast<const f32x4*>(cos_t + tab)[q];
+            const f32x4 sn = reinterpret_cast<const f32x4*>(sin_t + tab)[q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = a[q * 4 + e], y = b[q * 4 + e];
+                a[q * 4 + e] = x * cs[e] - y * sn[e];
+                b[q * 4 + e] = y * cs[e] + x * sn[e];
+            }
+        }
+    }
+    if (S > 0 || bias || turns) {
+        store_bf16x8(row, a);
+        store_bf16x8(row + half, b);
+    }
+    if (h < nq) return;
+    const int kvh = (h - nq) % nkv, slot = slots[t];
+    const long dst =
+        (((long)(slot / bs) * nkv + kvh) * bs + slot % bs) * hd + d;
+    CT* cache = (h < nq + nkv ? k_cache : v_cache) + dst;
+    if (sizeof(CT) == 2) {
+        unsigned short* o = reinterpret_cast<unsigned short*>(cache);
+        store_bf16x8(o, a);
+        store_bf16x8(o + half, b);
+    } else {
+        unsigned int w[4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const float* x = q ? b : a;
+            float r[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] = bf2f(f2bf(x[e]));
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                w[q * 2 + e] =
+                    f2fp8x2(r[e * 4], r[e * 4 + 1]) |
+                    (unsigned int)f2fp8x2(r[e * 4 + 2], r[e * 4 + 3]) << 16;
+        }
+        *reinterpret_cast<uint2v*>(cache) = uint2v{w[0], w[1]};
+        *reinterpret_cast<uint2v*>(cache + half) = uint2v{w[2], w[3]};
+    }
+}
+
 // ----------------------------------------------------------------- swiglu
 // out[t, i] = silu(gu[t, i]) * gu[t, I + i]; grid-stride, short8 loads.
 __global__ void swiglu_kernel(
@@ -343,6 +445,26 @@ void launch_kv_store_fp8(const unsigned short* k, const unsigned short* v,
     hipLaunchKernelGGL(kv_store_fp8_kernel, dim3(blocks), dim3(256), 0,
                        stream, k, v, k_cache, v_cache, slots, T, nkv, hd, bs,
                        sk, sv);
+}
+
+// hd % 16 == 0; qkv, bias, tables and pools 16-byte aligned; nonzero otherwise
+int launch_qkv_rope_store(const float* part, int S, unsigned short* qkv,
+                      const unsigned short* bias, const int* pos,
+                      const float* cos_t, const float* sin_t, void* k_cache,
+                      void* v_cache, const int* slots, long T, int nq, int nkv,
+                      int hd, int bs, int fp8, hipStream_t stream) {
+    if (hd % 16) return 1;
+    const long n = T * (nq + 2 * nkv) * (hd / 16);
+    if (n == 0) return 0;
+#define RS_GO(CT)                                                             \
+    hipLaunchKernelGGL((qkv_rope_store_kernel<CT>), dim3((n + 255) / 256),        \
+                       dim3(256), 0, stream, part, S, qkv, bias, pos, cos_t,  \
+                       sin_t, (CT*)k_cache, (CT*)v_cache, slots, T, nq, nkv,  \
+                       hd, bs)
+    if (fp8) RS_GO(unsigned char);
+    else RS_GO(unsigned short);
+#undef RS_GO
+    return 0;
 }
 
 void launch_swiglu(const unsigned short* gu, unsigned short* out, long T,

@@ -1,4 +1,5 @@
-// Torch bindings of the projections of a few rows (linear_rows.hip).
+// Torch bindings of the projections of a few rows (linear_rows.hip) and of some
+// tens (linear_mid.hip), and of the pass between q|k|v and attention.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
@@ -12,6 +13,17 @@ extern "C" int launch_linear_rows(
     unsigned short*, int, int, int, float, int, int, const int*, const float*,
     const float*, const int*, void*, void*, int, int, int, int, int,
     hipStream_t);
+extern "C" int linear_mid_splits(int, int);
+extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
+                                 float*, int, int, int, int, hipStream_t);
+extern "C" int launch_add_norm_parts(
+    const float*, const unsigned short*, const unsigned short*,
+    const unsigned short*, const unsigned short*, unsigned short*,
+    unsigned short*, int, int, int, float, hipStream_t);
+extern "C" int launch_qkv_rope_store(
+    const float*, int, unsigned short*, const unsigned short*, const int*,
+    const float*, const float*, void*, void*, const int*, long, int, int, int,
+    int, int, hipStream_t);
 
 namespace {
 
@@ -133,6 +145,97 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
     return q;
 }
 
+unsigned short* mut(Tensor& t) {
+    return reinterpret_cast<unsigned short*>(t.data_ptr());
+}
+
+// parts [S, M, N] fp32, whose sum over S is x w^T
+Tensor mid_linear(const Tensor& x, const Tensor& w) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
+                "x [M, K] and w [N, K]");
+    const int M = x.size(0), K = x.size(1), N = w.size(0);
+    TORCH_CHECK(M >= 1 && M <= 128, "1 to 128 rows");
+    TORCH_CHECK(K % 64 == 0 && N % 4 == 0);
+    const Tensor xd = dense(x, "x"), wd = dense(w, "w");
+    const int S = linear_mid_splits(N, K);
+    Tensor part = torch::empty({S, M, N},
+                               x.options().dtype(torch::kFloat32));
+    TORCH_CHECK(launch_linear_mid(ptr(xd), ptr(wd), part.data_ptr<float>(), M,
+                                  N, K, S, stream()) == 0);
+    return part;
+}
+
+const float* parts(const Tensor& t, long M, long N) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
+                t.is_contiguous() && t.dim() == 3 && t.size(1) == M &&
+                t.size(2) == N, "parts [S, M, N] fp32");
+    return t.data_ptr<float>();
+}
+
+// -> norm(resid + sum of the parts + bias) (undefined without a norm), and
+// that sum in bf16
+std::vector<optional<Tensor>> add_norm_parts(
+    const Tensor& part, const optional<Tensor>& bias, const Tensor& resid,
+    const optional<Tensor>& norm_w, const optional<Tensor>& norm_b,
+    double eps) {
+    TORCH_CHECK(resid.dim() == 2);
+    TORCH_CHECK(norm_w.has_value() || !norm_b.has_value());
+    const int M = resid.size(0), H = resid.size(1);
+    TORCH_CHECK(M >= 1 && H % 8 == 0 && H <= 8192);
+    const Tensor r = dense(resid, "resid"), b = column(bias, H, "bias"),
+                 nw = column(norm_w, H, "norm weight"),
+                 nb = column(norm_b, H, "norm bias");
+    Tensor sum = torch::empty({M, H}, r.options()), y;
+    if (norm_w.has_value()) y = torch::empty({M, H}, r.options());
+    TORCH_CHECK(launch_add_norm_parts(
+                    parts(part, M, H), ptr(b), ptr(r), ptr(nw), ptr(nb),
+                    mut(sum), y.defined() ? mut(y) : nullptr, M, H,
+                    part.size(0), (float)eps, stream()) == 0);
+    return {y.defined() ? optional<Tensor>(y) : optional<Tensor>(), sum};
+}
+
+// qkv: the projection's bf16 rows [T, N], changed in place, or its fp32 parts
+// [S, T, N]; -> [T, N] with bias added and q, k rotated; k, v also stored
+Tensor rope_store_qkv(const Tensor& qkv, const optional<Tensor>& bias,
+                      int64_t nq, const optional<Tensor>& pos,
+                      const optional<Tensor>& cos_t,
+                      const optional<Tensor>& sin_t, Tensor& k_cache,
+                      Tensor& v_cache, const Tensor& slots) {
+    const bool split = qkv.dim() == 3;
+    const long T = qkv.size(-2), N = qkv.size(-1);
+    const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
+    TORCH_CHECK(k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
+                k_cache.scalar_type() == v_cache.scalar_type() &&
+                k_cache.is_contiguous() && v_cache.is_contiguous());
+    TORCH_CHECK(fp8 || k_cache.scalar_type() == torch::kBFloat16);
+    const int nkv = k_cache.size(1), bs = k_cache.size(2),
+              hd = k_cache.size(3);
+    TORCH_CHECK(hd % 16 == 0 && N == (nq + 2 * nkv) * hd);
+    TORCH_CHECK(slots.scalar_type() == torch::kInt32 &&
+                slots.is_contiguous() && slots.numel() == T);
+    if (pos.has_value()) {
+        TORCH_CHECK(pos->scalar_type() == torch::kInt32 &&
+                    pos->is_contiguous() && pos->numel() == T);
+        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
+            TORCH_CHECK(t->scalar_type() == torch::kFloat32 &&
+                        t->is_contiguous() && t->size(1) == hd / 2);
+    }
+    const Tensor b = column(bias, N, "bias");
+    const float* p = split ? parts(qkv, T, N) : nullptr;
+    Tensor out = split ? torch::empty({T, N}, qkv.options().dtype(
+                                                  torch::kBFloat16))
+                       : dense(qkv, "qkv");
+    TORCH_CHECK(launch_qkv_rope_store(
+                    p, split ? qkv.size(0) : 0, mut(out), ptr(b),
+                    pos.has_value() ? pos->data_ptr<int>() : nullptr,
+                    pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
+                    pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
+                    k_cache.data_ptr(), v_cache.data_ptr(),
+                    slots.data_ptr<int>(), T, nq, nkv, hd, bs, fp8,
+                    stream()) == 0);
+    return out;
+}
+
 }  // namespace
 
 void register_rows_ops(pybind11::module_& m) {
@@ -140,4 +243,10 @@ void register_rows_ops(pybind11::module_& m) {
           "projection of a few rows: norm, product, bias, activation, residual");
     m.def("rows_qkv", &rows_qkv,
           "norm, q|k|v projection, rotation and page store of a few rows");
+    m.def("mid_linear", &mid_linear,
+          "projection of some tens of rows as fp32 parts over K");
+    m.def("add_norm_parts", &add_norm_parts,
+          "residual add of a projection's parts, and the next norm");
+    m.def("rope_store_qkv", &rope_store_qkv,
+          "bias, rotation and page store of q|k|v rows or parts");
 }

@@ -316,6 +316,45 @@ def rows_qkv(x, w, bias, norm, n_heads, positions, cos, sin, k_cache, v_cache,
     return q.contiguous()
 
 
+def mid_linear(x, w):
+    return (x.float() @ w.float().t()).unsqueeze(0)
+
+
+def add_norm_parts(part, bias, resid, norm=None):
+    y = resid.float() + part.sum(0)
+    if bias is not None:
+        y = y + bias.float()
+    normed = None
+    if norm is not None:
+        w, b, eps = norm
+        normed = (rmsnorm(y, w, eps) if b is None
+                  else layernorm(y, w, b, eps)).to(resid.dtype)
+    return normed, y.to(resid.dtype)
+
+
+def rope_store_qkv(qkv, bias, n_heads, positions, cos, sin, k_cache, v_cache,
+                   slot_mapping):
+    if qkv.dim() == 3:
+        rows = qkv.sum(0)
+    else:
+        rows = qkv.float()
+    if bias is not None:
+        rows = rows + bias.float()
+    T, N = rows.shape
+    nkv, hd = k_cache.shape[1], k_cache.shape[3]
+    q, k, v = rows.view(T, -1, hd).split([n_heads, nkv, nkv], dim=1)
+    if positions is not None:
+        rope_inplace(q, k, positions, cos, sin)
+    dtype = qkv.dtype if qkv.dim() == 2 else k_cache.dtype
+    out = rows.to(dtype)
+    _, k, v = out.view(T, -1, hd).split([n_heads, nkv, nkv], dim=1)
+    kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
+    if qkv.dim() == 2:
+        qkv.copy_(out)
+        return qkv
+    return out
+
+
 def attn_decode_lse(
     q: torch.Tensor,
     k_cache: torch.Tensor,

@@ -1,10 +1,10 @@
 """Projections of a few rows (linear_rows.hip) at the edges of their tiles, of
 the waves' shares of K and of the kernel shapes, against fp32.
 
-Tolerance: the normed input and the output are rounded to bf16 (2^-9 relative,
-half of it more for the weight folded in first): an element is off by at most
-2^-8 of the sum of its products' magnitudes, carried through the activation
-(whose slope is below 1.13), and 2^-8 of itself."""
+Tolerance: the normed input and the output are rounded to bf16 once each (2^-8
+relative at most): an element is off by at most 2^-8 of the sum of its
+products' magnitudes, carried through the activation (whose slope is below
+1.13), and 2^-8 of itself."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -146,3 +146,88 @@ def test_refused():
         ops.rows_linear(x, w)
     with pytest.raises(RuntimeError):
         ops.rows_linear(x[:4, :40].contiguous(), w[:, :40].contiguous())
+
+
+# ------------------------------------------------- steps of some tens of rows
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("N,K", [(64, 64), (68, 1088), (3584, 960),
+                                 (4096, 2048), (512, 8192 + 64)])
+def test_parts_over_k(M, N, K):
+    """Products of bf16 numbers are exact in fp32: only the order of the sums
+    differs, at most K roundings of a partial sum."""
+    torch.manual_seed(M + N)
+    x, w = _rand(M, K), _rand(N, K, std=0.05)
+    part = ops.mid_linear(x, w)
+    want = x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t()
+    assert ((part.double().sum(0) - want).abs() <= 2 ** -24 * K * mag).all()
+
+
+@pytest.mark.parametrize("S,M,H", [(1, 17, 64), (8, 128, 4096), (4, 20, 8192),
+                                   (2, 33, 3592)])
+@pytest.mark.parametrize("kind", [None, "rms", "layer"])
+def test_add_norm_parts(S, M, H, kind):
+    torch.manual_seed(S)
+    part = torch.randn(S, M, H, device=DEV)
+    bias, resid = _rand(H) if S > 1 else None, _rand(M, H)
+    norm = _norm(kind, H)
+    y, total = ops.add_norm_parts(part, bias, resid, norm)
+    want_y, want = reference.add_norm_parts(
+        part, None if bias is None else bias.float(), resid.float(),
+        _f32(norm))
+    assert ((total.float() - want).abs() <= 2 ** -8 * want.abs()
+            + 1e-5).all()
+    assert (y is None) == (norm is None)
+    if y is not None:
+        assert ((y.float() - want_y).abs() <= 2 ** -8 * want_y.abs()
+                + 1e-4).all()
+
+
+@pytest.mark.parametrize("parts", [0, 1, 4])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,nq,nkv,hd,rope,biased", [
+    (1, 4, 2, 16, True, False), (57, 28, 4, 128, True, True),
+    (33, 12, 12, 64, False, True), (300, 3, 1, 96, True, False),
+    (65, 8, 8, 64, False, False),
+])
+def test_rope_store_qkv(T, nq, nkv, hd, rope, biased, parts, fp8):
+    torch.manual_seed(T)
+    N = (nq + 2 * nkv) * hd
+    qkv = torch.randn(parts, T, N, device=DEV) if parts else _rand(T, N)
+    bias = _rand(N) if biased else None
+    cos, sin = reference.rope_tables(512, hd, 1e4, DEV)
+    pos = torch.randint(0, 512, (T,), device=DEV, dtype=torch.int32)
+    bs, nb = 24, T // 24 + 2
+    dt = torch.uint8 if fp8 else torch.bfloat16
+    kc = torch.zeros(nb, nkv, bs, hd, device=DEV, dtype=dt)
+    vc = torch.zeros_like(kc)
+    slots = torch.randperm(nb * bs, device=DEV)[:T].int()
+    y = (qkv.sum(0) if parts else qkv.float().clone())
+    if biased:
+        y = y + bias.float()
+    want = y.view(T, -1, hd).clone()
+    wq, wk, _ = want.split([nq, nkv, nkv], 1)
+    if rope:
+        reference.rope_inplace(wq, wk, pos, cos, sin)
+    got = ops.rope_store_qkv(qkv, bias, nq, pos if rope else None, cos, sin,
+                             kc, vc, slots)
+    if not parts:
+        assert got.data_ptr() == qkv.data_ptr()
+    got = got.view(T, -1, hd)
+    # one rounding to bf16 (2^-8 relative at most) of a sum that fp32 holds to
+    # 2^-20 of its terms
+    mag = y.view(T, -1, hd).abs()
+    mag = mag + mag.roll(hd // 2, -1)
+    assert ((got.float() - want).abs()
+            <= 2 ** -8 * want.abs() + 2 ** -20 * mag + 1e-6).all()
+    s = slots.long()
+    for cache, rows in ((kc, got[:, nq : nq + nkv]), (vc, got[:, nq + nkv :])):
+        stored = cache[s // bs, :, s % bs]
+        if fp8:
+            rows = rows.float().to(torch.float8_e4m3fn).view(torch.uint8)
+        assert torch.equal(stored, rows)
+        rest = cache.clone()
+        rest[s // bs, :, s % bs] = 0
+        assert (rest == 0).all()
