@@ -13,19 +13,21 @@
 //    stand, the right operand of O^T = V^T P^T: no trip through LDS. That
 //    product takes its 16 keys in the order the score tile holds them, which
 //    the transposing LDS read of V follows.
-//  * Keys and values are staged in LDS row-major, 16-byte chunks xor-ed by
-//    the key so that both kinds of reads spread over the banks, two buffers,
-//    the next tile's global reads in flight over the current tile's products.
+//  * Keys and values are staged in LDS row-major (two buffers), 16-byte chunks
+//    xor-ed by the key, the next tile's global reads in flight over the
+//    current tile's products.
 //  * The running maximum is raised only by a score FL_SLACK powers of two
 //    above it: most tiles leave the sums as they are. Weights stay below
 //    2^FL_SLACK, whose bf16 rounding is as fine, and sums are fp32.
 // Scores are scaled in fp32 (queries enter the product unrounded). The kernel
 // before it (16-row tiles, weights and V transposed through LDS by 2-byte
 // writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
-// of 28 heads on 16384 keys 897 us instead of 5240 (940 TFLOP/s), 2048 tokens
+// of 28 heads on 16384 keys 860 us instead of 5240 (980 TFLOP/s), 2048 tokens
 // of 32 heads 63 us instead of 386 (540), nine prompts of 112 to 901 tokens
-// 38 us instead of 140. Fetching key fragments two steps ahead by hand
-// changed nothing (979 us against 928 in one run).
+// 38 us instead of 140. Neither fetching key fragments two steps ahead by hand
+// nor computing the next tile's scores beside this one's exponentials (with
+// or without a forced interleaving) made it faster: at 980 TFLOP/s the clock
+// has come down to 1.75 GHz.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -101,6 +103,15 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         wr0 < QL * G ? hist + min(wr0 + 31, QL * G - 1) / G + 1 : 0;
     const int kv_end = hist + min(row0 + ROWS - 1, QL * G - 1) / G + 1;
 
+    // Chunks of a staged row are xor-ed so that no two lanes served together
+    // meet in a bank. LDS serves 256 bytes a clock: 16 lanes of a 16-byte read
+    // (16 keys, one chunk), 32 lanes of a transposing read (4 keys, two pairs
+    // of chunks). With patterns made for 128 bytes a clock, 44% of the LDS
+    // cycles were conflicts and 8192 tokens of 32 heads took 578 us, not 561.
+    auto k_swz = [](int row) { return HD == 128 ? row & 15 : (row >> 1) & 7; };
+    auto v_swz = [](int row) {
+        return HD == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1);
+    };
     // ---- staging: thread -> (key row, chunk)
     const int st_row = tid / CPR, st_c = tid % CPR;
     bf16x8 rk[NST], rv[NST];
@@ -131,7 +142,6 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             }
         }
     };
-    constexpr int VMASK = HD == 128 ? 7 : 3;
     auto store_tile = [&](int buf) {
         char* kd = smem + buf * 2 * TILE;
         char* vd = kd + TILE;
@@ -139,21 +149,21 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         for (int i = 0; i < NST; ++i) {
             const int row = st_row + i * RPT;
             *reinterpret_cast<bf16x8*>(kd + row * RB +
-                                       ((st_c ^ (row & 7)) << 4)) = rk[i];
+                                       ((st_c ^ k_swz(row)) << 4)) = rk[i];
             *reinterpret_cast<bf16x8*>(
-                vd + row * RB + ((st_c ^ (2 * (row & VMASK))) << 4)) = rv[i];
+                vd + row * RB + ((st_c ^ v_swz(row)) << 4)) = rv[i];
         }
     };
 
     // ---- fragment addresses
     // K (rows = keys): lane reads key lr of a 32-key tile, chunk 2 ks + hi
     const int k_base = lr * RB;
-    const int k_sw = lr & 7;
+    const int k_sw = k_swz(lr);
     // V^T (rows = coordinates) through the transposing read: the 16 lanes of
     // a group address 4 keys x 16 coordinates
     const int v_key = 4 * hi + ((lane >> 2) & 3);
     const int v_c0 = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
-    const int v_sw = 2 * (v_key & VMASK);
+    const int v_sw = v_swz(v_key);
     int v_off[DT];
 #pragma unroll
     for (int d = 0; d < DT; ++d)

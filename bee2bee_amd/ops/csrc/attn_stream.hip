@@ -83,7 +83,13 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     constexpr int RPI = 64 / CPR;        // rows a wave loads at once
     constexpr int NL = ST_KEYS / RPI;    // loads of a tile
     constexpr int TILE = ST_KEYS * RB;
-    constexpr int VMASK = HD == 128 ? 7 : 3;
+    // chunks of a staged row are xor-ed so that the lanes LDS serves together
+    // (256 bytes a clock: 16 keys of one chunk; 8 keys of one pair of chunks)
+    // meet in no bank
+    auto k_swz = [](int row) { return HD == 128 ? row & 15 : (row >> 1) & 7; };
+    auto v_swz = [](int row) {
+        return 2 * (HD == 128 ? row & 7 : (row >> 1) & 3);
+    };
     using raw_t = typename st_raw<KVT>::type;
 
     const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
@@ -161,9 +167,9 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
 
     // ---- fragment addresses: K row li (+ 16), chunk ks * 4 + lg; V through
     // the transposing read, 16 lanes on 4 keys x 16 coordinates
-    const int k_base = li * RB, k_sw = li & 7;
+    const int k_base = li * RB, k_sw = k_swz(li);
     const int v_key = lg * 4 + (li >> 2);
-    const int v_sw = 2 * (v_key & VMASK);
+    const int v_sw = v_swz(v_key);
     const int v_base = TILE + v_key * RB + (lane & 1) * 8;
     const int v_c = (lane & 3) >> 1;
 
@@ -186,10 +192,10 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
         for (int i = 0; i < NL; ++i) {
             const int row = ld_row + i * RPI;
             *reinterpret_cast<short8*>(kd + row * RB +
-                                       ((ld_c ^ (row & 7)) << 4)) =
+                                       ((ld_c ^ k_swz(row)) << 4)) =
                 st_widen(rk[i]);
             *reinterpret_cast<short8*>(
-                kd + TILE + row * RB + ((ld_c ^ (2 * (row & VMASK))) << 4)) =
+                kd + TILE + row * RB + ((ld_c ^ v_swz(row)) << 4)) =
                 st_widen(rv[i]);
         }
         if (kb + ST_STEP < k1) load_tile(kb + ST_STEP);

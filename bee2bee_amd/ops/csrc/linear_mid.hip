@@ -7,7 +7,8 @@
 // the latency of a step. A workgroup takes 64 rows of W and a part of K: four
 // waves of 16 rows, twice, for the two halves of that part. Weights go from
 // memory into the left operand as they lie (three steps in flight), the input
-// rows through LDS, shared by the four waves, xor-ed against bank conflicts.
+// rows through LDS, shared by the four waves, xor-ed so that the 16 rows of a
+// read meet in no bank (LDS serves 256 bytes a clock).
 // Measured beside the library's product (us; 24 / 57 / 80 / 128 rows):
 // 4096x14336 27 / 30 / 34 / 42 (32 / 41 / 43 / 76), 4096x4096 10.8 / 12.5 /
 // 14 / 16 (13.7 / 13.8 / 17 / 24), 6144x4096 15.4 / 18 / 20.5 / 24 (15 / 18 /
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
         xs[j] = x + (long)min(row, M - 1) * K +
                 (long)(h ? c0 + first : c0) * 64 + c * 8;
         xlast[j] = (h ? c1 - c0 - first : first) - 1;
-        xd[j] = (h * MP + row) * 128 + ((c ^ (row & 7)) << 4);
+        xd[j] = (h * MP + row) * 128 + ((c ^ (row >> 1 & 7)) << 4);
     }
     // (a half without steps left loads, and ignores, a step of the other)
     bf16x8 xr[NLD];
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
                     for (int m = 0; m < MT; ++m) {
                         const bf16x8 bx = *reinterpret_cast<const bf16x8*>(
                             b + m * 16 * 128 +
-                            (((s * 4 + lg) ^ (li & 7)) << 4));
+                            (((s * 4 + lg) ^ (li >> 1)) << 4));
                         acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                             aw[j][s], bx, acc[m], 0, 0, 0);
                     }
