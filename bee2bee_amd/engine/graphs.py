@@ -18,6 +18,8 @@ from typing import Dict, Optional
 
 import torch
 
+from .. import ops
+
 logger = logging.getLogger("bee2bee_amd.engine")
 
 
@@ -25,9 +27,7 @@ def decode_slot_mapping(
     block_table: torch.Tensor, positions: torch.Tensor, block_size: int
 ) -> torch.Tensor:
     """slot[b] = block_table[b][pos//bs]*bs + pos%bs, computed on device."""
-    blk_idx = torch.div(positions, block_size, rounding_mode="floor")
-    blk = block_table.gather(1, blk_idx.unsqueeze(1).long()).squeeze(1)
-    return blk * block_size + positions % block_size
+    return ops.decode_slots(block_table, positions, block_size)
 
 
 class DecodeGraphs:

@@ -104,10 +104,10 @@ class Runner:
 
     def embed(self, input_ids: torch.Tensor,
               positions: Optional[torch.Tensor] = None) -> torch.Tensor:
-        h = F.embedding(input_ids, self.weights.embed)
         if self.spec.pos_type == "learned" and positions is not None:
-            h = h + F.embedding(positions.long(), self.weights.pos_embed)
-        return h
+            return ops.embed_positions(input_ids, self.weights.embed,
+                                       positions, self.weights.pos_embed)
+        return F.embedding(input_ids, self.weights.embed)
 
     def _norm(self, x, w, b):
         if self.spec.norm_type == "layernorm":

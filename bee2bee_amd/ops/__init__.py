@@ -301,6 +301,26 @@ def rope_store_qkv(qkv, bias, n_heads: int, positions, cos, sin, k_cache,
                                     k_cache, v_cache, slot_mapping)
 
 
+def decode_slots(block_table, positions, block_size: int):
+    """slot[b] = block_table[b][pos // bs] * bs + pos % bs."""
+    if (_use_hip(positions) and positions.dtype is torch.int32
+            and block_table.dtype is torch.int32 and positions.dim() == 1
+            and positions.is_contiguous() and block_table.stride(1) == 1):
+        return require_hip().decode_slots(block_table, positions, block_size)
+    return reference.decode_slots(block_table, positions, block_size)
+
+
+def embed_positions(ids, table, positions, pos_table):
+    """table[ids] + pos_table[positions]."""
+    if (_use_hip(table) and table.dtype is torch.bfloat16
+            and ids.dtype is torch.int64 and positions.dtype is torch.int32
+            and ids.dim() == 1 and ids.is_contiguous()
+            and positions.shape == ids.shape and positions.is_contiguous()
+            and pos_table.dtype is table.dtype and table.shape[1] % 8 == 0):
+        return require_hip().embed_positions(ids, table, positions, pos_table)
+    return reference.embed_positions(ids, table, positions, pos_table)
+
+
 def moe_topk_gate(logits: torch.Tensor, top_k: int):
     # gating math is tiny ([T, E]); torch ops are fine on both devices
     return reference.moe_topk_gate(logits, top_k)

@@ -25,6 +25,13 @@ extern "C" int launch_qkv_rope_store(
     const float*, const float*, void*, void*, const int*, long, int, int, int,
     int, int, hipStream_t);
 
+extern "C" void launch_decode_slots(const int*, const int*, int*, int, int,
+                                    long, int, hipStream_t);
+extern "C" void launch_embed_positions(const long*, const unsigned short*,
+                                       const int*, const unsigned short*,
+                                       unsigned short*, long, int, long, int,
+                                       hipStream_t);
+
 namespace {
 
 enum { EPI_PLAIN = 0, EPI_GLU = 1, EPI_GELU = 2, EPI_QKV = 3 };
@@ -236,6 +243,37 @@ Tensor rope_store_qkv(const Tensor& qkv, const optional<Tensor>& bias,
     return out;
 }
 
+Tensor decode_slots(const Tensor& table, const Tensor& pos, int64_t bs) {
+    TORCH_CHECK(table.is_cuda() && table.scalar_type() == torch::kInt32 &&
+                table.dim() == 2 && table.stride(1) == 1);
+    TORCH_CHECK(pos.is_cuda() && pos.scalar_type() == torch::kInt32 &&
+                pos.is_contiguous() && pos.dim() == 1 &&
+                pos.size(0) <= table.size(0) && bs > 0);
+    Tensor slots = torch::empty_like(pos);
+    launch_decode_slots(table.data_ptr<int>(), pos.data_ptr<int>(),
+                        slots.data_ptr<int>(), pos.size(0), table.size(1),
+                        table.stride(0), bs, stream());
+    return slots;
+}
+
+// [T, H] bf16 = embed[ids] + pos_embed[pos]
+Tensor embed_positions(const Tensor& ids, const Tensor& embed,
+                       const Tensor& pos, const Tensor& pos_embed) {
+    TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == torch::kInt64 &&
+                ids.is_contiguous() && ids.dim() == 1);
+    TORCH_CHECK(pos.is_cuda() && pos.scalar_type() == torch::kInt32 &&
+                pos.is_contiguous() && pos.sizes() == ids.sizes());
+    const Tensor e = dense(embed, "embed"), p = dense(pos_embed, "pos_embed");
+    TORCH_CHECK(e.dim() == 2 && p.dim() == 2 && e.size(1) == p.size(1) &&
+                e.size(1) % 8 == 0);
+    Tensor out = torch::empty({ids.size(0), e.size(1)}, e.options());
+    launch_embed_positions(reinterpret_cast<const long*>(ids.data_ptr()),
+                           ptr(e), pos.data_ptr<int>(), ptr(p), mut(out),
+                           ids.size(0), e.size(1), e.size(0), p.size(0),
+                           stream());
+    return out;
+}
+
 }  // namespace
 
 void register_rows_ops(pybind11::module_& m) {
@@ -247,6 +285,9 @@ void register_rows_ops(pybind11::module_& m) {
           "projection of some tens of rows as fp32 parts over K");
     m.def("add_norm_parts", &add_norm_parts,
           "residual add of a projection's parts, and the next norm");
+    m.def("decode_slots", &decode_slots, "page slots of a decode step's rows");
+    m.def("embed_positions", &embed_positions,
+          "token and learned position embeddings, added");
     m.def("rope_store_qkv", &rope_store_qkv,
           "bias, rotation and page store of q|k|v rows or parts");
 }

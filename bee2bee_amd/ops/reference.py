@@ -355,6 +355,17 @@ def rope_store_qkv(qkv, bias, n_heads, positions, cos, sin, k_cache, v_cache,
     return out
 
 
+def decode_slots(block_table, positions, block_size):
+    blk_idx = torch.div(positions, block_size, rounding_mode="floor")
+    blk = block_table.gather(1, blk_idx.unsqueeze(1).long()).squeeze(1)
+    return blk * block_size + positions % block_size
+
+
+def embed_positions(ids, table, positions, pos_table):
+    F = torch.nn.functional
+    return F.embedding(ids, table) + F.embedding(positions.long(), pos_table)
+
+
 def attn_decode_lse(
     q: torch.Tensor,
     k_cache: torch.Tensor,

@@ -231,3 +231,29 @@ def test_rope_store_qkv(T, nq, nkv, hd, rope, biased, parts, fp8):
         rest = cache.clone()
         rest[s // bs, :, s % bs] = 0
         assert (rest == 0).all()
+
+
+# ------------------------------------------------------ what a step starts with
+
+
+@pytest.mark.parametrize("B,W,bs", [(1, 1, 16), (257, 5, 24), (3, 128, 256)])
+def test_decode_slots(B, W, bs):
+    torch.manual_seed(B)
+    wide = torch.randint(0, 10000, (B + 1, W + 3), device=DEV,
+                         dtype=torch.int32)
+    table = wide[:, :W]           # rows at a stride, more of them than asked
+    pos = torch.randint(0, W * bs, (B,), device=DEV, dtype=torch.int32)
+    pos[0] = W * bs - 1
+    got = ops.decode_slots(table, pos, bs)
+    want = reference.decode_slots(table[:B], pos, bs)
+    assert got.dtype == want.dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,H", [(1, 8), (33, 768), (2, 2048)])
+def test_embed_positions(T, H):
+    torch.manual_seed(T)
+    table, pos_table = _rand(50, H), _rand(40, H)
+    ids = torch.randint(0, 50, (T,), device=DEV)
+    pos = torch.randint(0, 40, (T,), device=DEV, dtype=torch.int32)
+    got = ops.embed_positions(ids, table, pos, pos_table)
+    assert torch.equal(got, table[ids] + pos_table[pos.long()])
