@@ -11,6 +11,10 @@
 //    The waves of a workgroup share K and add up in LDS; there is no split
 //    over workgroups, so a row's result depends neither on the other rows nor
 //    on their number.
+//  * TC 8: 8 rows of W at two places along K, 128 bytes of a row together, as
+//    one left operand, 8 input rows at both places as the other; the two
+//    diagonal quarters of the product add up. Twice the workgroups where 16
+//    columns each leave CUs without one, and better pieces to load elsewhere.
 //  * RMS norm: the columns enter as bf16(x w), the sum of squares is taken on
 //    the way and 1/rms multiplies the fp32 sum: one rounding, as if the normed
 //    row had been written and read. Layer norm needs mean and deviation first:
@@ -19,10 +23,10 @@
 //    16 the registers cost more waves than the loads gain (output head of
 //    128256 x 4096, us: 4 tiles 182, 8 205, 16 230), and a streaming hint on
 //    the loads loses the half lines a 64-byte piece leaves (206 to 240).
-// Measured (us, one row, beside the library product alone): 6144x4096 14
-// (14.5), 4096x4096 9 (15.6), 2x14336x4096 48 (64), 4096x14336 24 (27),
-// 128256x4096 182 (190); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
-// 24, 182. With 16 rows 16, 11, 54, 31, 207: the input's reads add up, so
+// Measured (us, one row, beside the library product alone): 6144x4096 15.3
+// (14.5), 4096x4096 9.3 (15.6), 2x14336x4096 44 (64), 4096x14336 25 (27),
+// 128256x4096 183 (190); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
+// 24, 182. With 16 rows 17, 11.6, 57, 34, 216: the input's reads add up, so
 // more rows go to the library.
 #include "common.h"
 
@@ -64,7 +68,7 @@ DEV_INLINE void store_row4(void* cache, long at, int fp8, const float* z) {
 // LR_QKV: see QkvStore (W [N, K], bias optional). NT tiles of 16 columns of y
 // per workgroup (LR_GLU, LR_QKV: of each half; LR_QKV's halves are those of a
 // head).
-template <int NW, int NT, int NORM, int EPI>
+template <int NW, int NT, int TC, int G, int NORM, int EPI>
 __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
     const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ norm_w,
@@ -75,41 +79,50 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
     int M, int N, int K, float eps, QkvStore st) {
     constexpr bool PAIR = EPI == LR_GLU || EPI == LR_QKV;
     constexpr int WT = PAIR ? 2 * NT : NT;
-    constexpr int U = LR_U / WT > 0 ? LR_U / WT : 1;
+    constexpr int H = TC == 16 ? G : 1;        // tiles of W along K a step
+    constexpr int U = LR_U / (WT * H) > 0 ? LR_U / (WT * H) : 1;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    int n0 = blockIdx.x * NT * 16;             // first column of y
+    // TC 8: lanes 8..15 take the same weights' rows, and the same input rows,
+    // 32 further along K; the off-diagonal quarters of the tile are not read.
+    // G 2: TC 8: input rows 0-7 and 8-15; TC 16: K and K + 32, summed apart as
+    // TC 8 does
+    constexpr int KS = TC == 8 || G == 2 ? 64 : 32;    // K of a step
+    constexpr int RG = TC == 8 ? 8 : 0;        // rows from acc[0] to acc[1]
+    const int lj = li & (TC - 1), lk = (li - lj) * 4 + lg * 8;
+    int n0 = blockIdx.x * NT * TC;             // first column of y
     int half = N;                              // to the pair's other tile
     if (EPI == LR_QKV) {
-        const int per = st.hd / 32;            // workgroups of a head
-        n0 = blockIdx.x / per * st.hd + blockIdx.x % per * 16;
+        const int per = st.hd / (2 * TC);      // workgroups of a head
+        n0 = blockIdx.x / per * st.hd + blockIdx.x % per * TC;
         half = st.hd / 2;
     }
-    // this wave's steps of 32 along K
-    const int steps = K / 32;
+    const int steps = K / KS;                  // this wave's: s0 .. s1
     const int s0 = steps * wid / NW, s1 = steps * (wid + 1) / NW;
 
     const unsigned short* wp[WT];
 #pragma unroll
     for (int t = 0; t < WT; ++t) {
-        int n = n0 + (t % NT) * 16 + li;
+        int n = n0 + (t % NT) * TC + lj;
         if (!PAIR) n = min(n, N - 1);
-        wp[t] = w + (long)(t < NT ? n : half + n) * K + lg * 8;
+        wp[t] = w + (long)(t < NT ? n : half + n) * K + lk;
     }
-    bf16x8 aw[2][U][WT];
+    bf16x8 aw[2][U][H][WT];
     auto fetch = [&](int set, int s) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int t = 0; t < WT; ++t)
-                aw[set][u][t] = *reinterpret_cast<const bf16x8*>(
-                    wp[t] + (long)(s + u) * 32);
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int t = 0; t < WT; ++t)
+                    aw[set][u][h][t] = *reinterpret_cast<const bf16x8*>(
+                        wp[t] + (long)(s + u) * KS + h * 32);
     };
     int s = s0;
     if (s + U <= s1) fetch(0, s);
 
-    float mean = 0.f, dev = 1.f;               // LR_LAYER: of row li
+    float mean[G], dev[G];                     // LR_LAYER: of acc[g]'s row
     if (NORM == LR_LAYER) {
         __shared__ float stat[16][2];
         for (int m = wid; m < M; m += NW) {
@@ -131,41 +144,52 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
             }
         }
         __syncthreads();
-        mean = stat[min(li, M - 1)][0];
-        dev = stat[min(li, M - 1)][1];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            mean[g] = stat[min(lj + RG * g, M - 1)][0];
+            dev[g] = stat[min(lj + RG * g, M - 1)][1];
+        }
     }
 
-    const long x_off = (long)min(li, M - 1) * K + lg * 8;
-    f32x4 acc[WT];
-    float sq = 0.f;                            // LR_RMS
+    long x_off[G];
+    f32x4 acc[G][WT];
+    float sq[G];                               // LR_RMS
 #pragma unroll
-    for (int t = 0; t < WT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto products = [&](const bf16x8* a, int st_) {
-        const long k = (long)st_ * 32;
-        bf16x8 bx = *reinterpret_cast<const bf16x8*>(x + x_off + k);
-        if (NORM == LR_RMS) {
-            const bf16x8 g =
-                *reinterpret_cast<const bf16x8*>(norm_w + lg * 8 + k);
+    for (int g = 0; g < G; ++g) {
+        x_off[g] = (long)min(lj + RG * g, M - 1) * K + lk;
+        sq[g] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = (float)bx[e];
-                sq = fmaf(v, v, sq);
-                bx[e] = (__bf16)(v * (float)g[e]);
+        for (int t = 0; t < WT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto products = [&](const bf16x8 (*a)[WT], int st_) {
+        bf16x8 nw, nb;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const long k = (long)st_ * KS + (TC == 16 ? g * 32 : 0);
+            if (NORM != LR_NONE && (g == 0 || TC == 16))
+                nw = *reinterpret_cast<const bf16x8*>(norm_w + lk + k);
+            if (NORM == LR_LAYER && (g == 0 || TC == 16))
+                nb = *reinterpret_cast<const bf16x8*>(norm_b + lk + k);
+            bf16x8 bx = *reinterpret_cast<const bf16x8*>(x + x_off[g] + k);
+            if (NORM == LR_RMS) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = (float)bx[e];
+                    sq[g] = fmaf(v, v, sq[g]);
+                    bx[e] = (__bf16)(v * (float)nw[e]);
+                }
+            } else if (NORM == LR_LAYER) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    bx[e] = (__bf16)(((float)bx[e] - mean[g]) * dev[g] *
+                                         (float)nw[e] +
+                                     (float)nb[e]);
             }
-        } else if (NORM == LR_LAYER) {
-            const bf16x8 g =
-                *reinterpret_cast<const bf16x8*>(norm_w + lg * 8 + k);
-            const bf16x8 c =
-                *reinterpret_cast<const bf16x8*>(norm_b + lg * 8 + k);
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                bx[e] = (__bf16)(((float)bx[e] - mean) * dev * (float)g[e] +
-                                 (float)c[e]);
+            for (int t = 0; t < WT; ++t)
+                acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a[TC == 16 ? g : 0][t], bx, acc[g][t], 0, 0, 0);
         }
-#pragma unroll
-        for (int t = 0; t < WT; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], bx, acc[t],
-                                                             0, 0, 0);
     };
     for (; s + 2 * U <= s1; s += 2 * U) {
         fetch(1, s + U);
@@ -181,56 +205,79 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         s += U;
     }
     for (; s < s1; ++s) {
-        bf16x8 a[WT];
+        bf16x8 a[H][WT];
 #pragma unroll
-        for (int t = 0; t < WT; ++t)
-            a[t] = *reinterpret_cast<const bf16x8*>(wp[t] + (long)s * 32);
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int t = 0; t < WT; ++t)
+                a[h][t] = *reinterpret_cast<const bf16x8*>(
+                    wp[t] + (long)s * KS + h * 32);
         products(a, s);
     }
 
     // ---- the waves' sums; C layout: column li = row of x, rows lg * 4 + r =
     // columns of y
-    __shared__ f32x4 part[NW][WT][64];
-    __shared__ float sqp[NW][16];
-    if (NORM == LR_RMS) {
-        sq = rows_sum(sq);
-        if (lg == 0) sqp[wid][li] = sq;
-    }
+    __shared__ f32x4 part[NW][G][WT][64];
+    __shared__ float sqp[NW][G][16];
 #pragma unroll
-    for (int t = 0; t < WT; ++t) part[wid][t][lane] = acc[t];
+    for (int g = 0; g < G; ++g) {
+        if (NORM == LR_RMS) {
+            sq[g] = rows_sum(sq[g]);
+            if (lg == 0) sqp[wid][g][li] = sq[g];
+        }
+#pragma unroll
+        for (int t = 0; t < WT; ++t) part[wid][g][t][lane] = acc[g][t];
+    }
     __syncthreads();
-    const int m = li;
-    if (wid >= NT || m >= M) return;
+    if (wid >= NT * (TC == 8 ? G : 1) ||
+        (TC == 8 && (li >= 8 || lg >= 2))) return;
+    const int g = wid / NT, tile = wid % NT, m = li + RG * g;
+    if (m >= M) return;
+    // the sums over K and over K + 32, each of all waves, then together
+    constexpr bool TWO = KS == 64;
+    const int g2 = TC == 8 ? g : G - 1, up = TC == 8 ? 8 : 0;   // li + 8, and
+    const int up_lane = TC == 8 ? 40 : 0;                       // lg + 2
     float inv = 1.f;
     if (NORM == LR_RMS) {
         float v = 0.f;
 #pragma unroll
-        for (int k = 0; k < NW; ++k) v += sqp[k][m];
+        for (int k = 0; k < NW; ++k) {
+            v += sqp[k][g][li];
+            if (TWO) v += sqp[k][g2][li + up];
+        }
         inv = rsqrtf(v / (float)K + eps);
     }
     auto total = [&](int t, float* z) {
-        f32x4 v = part[0][t][lane];
+        f32x4 v = part[0][g][t][lane];
 #pragma unroll
         for (int k = 1; k < NW; ++k) {
-            const f32x4 p = part[k][t][lane];
+            const f32x4 p = part[k][g][t][lane];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] += p[r];
+        }
+        if (TWO) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k) {
+                const f32x4 p = part[k][g2][t][lane + up_lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] += p[r];
+            }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) z[r] = v[r] * inv;
     };
-    const int n = n0 + wid * 16 + lg * 4;      // (wid: the tile; NT <= NW)
+    const int n = n0 + tile * TC + lg * 4;     // (NT * G <= NW)
     if (!PAIR && n >= N) return;
     float z[4];
-    total(wid, z);
+    total(tile, z);
     if (EPI == LR_GLU) {
         float u[4];
-        total(NT + wid, u);
+        total(NT + tile, u);
 #pragma unroll
         for (int r = 0; r < 4; ++r) z[r] = z[r] / (1.f + __expf(-z[r])) * u[r];
     } else if (EPI == LR_QKV) {
         float u[4];
-        total(NT + wid, u);
+        total(NT + tile, u);
         if (bias) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -289,12 +336,27 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
 
 // x [M, K] and w rows of K, 1 <= M <= 16, K % 32 == 0, all contiguous and
 // 16-byte aligned; norm 0 none, 1 RMS, 2 layer norm; epi as above (LR_GLU: N %
-// 16 == 0, LR_QKV: hd % 32 == 0). Nonzero for anything else. The shape of a workgroup depends on N and K only. Measured (us, one
-// row; 16 columns and 8 waves / 16 and 16 / 32 and 8): 4096x4096 9.4 / 8.7 /
-// 12.3, 4096x14336 28.5 / 23.8 / 37, 3584x18944 33 / 30 / 42, 3072x2048 6.5 /
-// 6.5 / 7.9, 768x3072 6.0 / 6.3 / 9.4; 6144x4096 15.6 / 17 / 13.8, 4608x3584
-// 14.1 / 16 / 11.6, 128256x4096 198 / 260 / 182; gated, 2x14336x4096 48 with
-// 8 waves, 50 with 4, 2x8192x2048 16.1 and 14.8.
+// 16 == 0, LR_QKV: hd % 32 == 0). Nonzero for anything else.
+//
+// The shape of a workgroup (waves x tiles x columns of a tile) depends on N and
+// K only, or on M between shapes of the same sums: 16 columns with G 2 add as 8
+// do. Measured (us) at 1 / 8 / 16 rows:
+//   q, k, v: 3072x2048 8x1x8 6.5 / 7.1 / 8.3, 8x1x16 8.2 / 8.7 / 9.3 (96
+//    workgroups); 2304x768 5.8 / 6.2 / 7.8 and 6.0 / 6.6 / 7.5; but 5120x3072
+//    11.8 / 12.9 / 16.3 and 11.9 / 11.7 / 12.6, 6144x4096 15.2 / 17.0 / 20.3
+//    and 15.4 / 16.4 / 17.2;
+//   gated: 2x14336x4096 4x1x8 44 / 49 / 64, 4x1x16 50 / 52 / 57, 8x1x16 49 /
+//    50 / 55; 2x18944x3584 53 / 59 / 76, 54 / 57 / 63, 54 / 57 / 63;
+//    2x8192x2048 15.7 / 17.2 / 21.7, 16.0 / 16.2 / 17.4, 15.8 / 16.2 / 17.3;
+//   up to 2048 columns: 2048x8192 8x1x8 10 / 11.7 / 15.4, 8x2x8 13 / 14.7 /
+//    18.6, 16x1x16 14 / 16 / 18.7; 2048x2048 4.5 / 5.2 / 6.1, 5.3 / 5.9 / 6.8,
+//    5.3 / 6.1 / 6.8; 768x3072 5.6 / 6.3 / 7.8, 6.3 / 7.2 / 8.7, 6.8 / 7.9 /
+//    9.2;
+//   up to 4096: 3072x8192 14.1 / 19 / 25, 14.0 / 16.6 / 19.2, 15.4 / 18 / 19.7;
+//    4096x4096 8.6 / 10.9 / 14.4, 9.3 / 9.8 / 11.6, 9.2 / 10.4 / 11.9;
+//    4096x14336 24.9 / 32 / 44, 24.9 / 26.5 / 34.5, 25.4 / 29.3 / 34.6;
+//    3584x18944 31 / 41 / 56, 29 / 34 / 44, 32 / 40 / 46;
+//   above: 128256x4096 8x2x8 174 / 204 / 272, 8x2x16 184 / 194 / 217.
 extern "C" int launch_linear_rows(
     const unsigned short* x, const unsigned short* norm_w,
     const unsigned short* norm_b, const unsigned short* w,
@@ -308,25 +370,40 @@ extern "C" int launch_linear_rows(
     if (epi == LR_QKV && (hd % 32 || N != (nq + 2 * nkv) * hd)) return 1;
     const QkvStore st{pos,     cos_t, sin_t, slots, k_cache,
                       v_cache, nq,    nkv,   hd,    bs, fp8};
-#define LR_GO(NWV, NTV, NO, EP, COLS)                                         \
-    hipLaunchKernelGGL((linear_rows_kernel<NWV, NTV, NO, EP>),                \
-                       dim3((N + (COLS) - 1) / (COLS)), dim3(NWV * 64), 0,    \
-                       stream, x, norm_w, norm_b, w, bias, resid, y, M, N, K, \
-                       eps, st)
-#define LR_NORMS(NWV, NTV, EP, COLS)                                          \
+#define LR_COLS(NTV, TCV, EP) (NTV * TCV * (EP == LR_QKV ? 2 : 1))
+#define LR_GO(NWV, NTV, TCV, GV, NO, EP)                                      \
+    hipLaunchKernelGGL((linear_rows_kernel<NWV, NTV, TCV, GV, NO, EP>),       \
+                       dim3((N + LR_COLS(NTV, TCV, EP) - 1) /                 \
+                            LR_COLS(NTV, TCV, EP)),                           \
+                       dim3(NWV * 64), 0, stream, x, norm_w, norm_b, w, bias, \
+                       resid, y, M, N, K, eps, st)
+#define LR_NORMS(NWV, NTV, TCV, GV, EP)                                       \
     do {                                                                      \
-        if (norm == LR_RMS) LR_GO(NWV, NTV, LR_RMS, EP, COLS);                \
-        else if (norm == LR_LAYER) LR_GO(NWV, NTV, LR_LAYER, EP, COLS);       \
-        else LR_GO(NWV, NTV, LR_NONE, EP, COLS);                              \
+        if (norm == LR_RMS) LR_GO(NWV, NTV, TCV, GV, LR_RMS, EP);             \
+        else if (norm == LR_LAYER) LR_GO(NWV, NTV, TCV, GV, LR_LAYER, EP);    \
+        else LR_GO(NWV, NTV, TCV, GV, LR_NONE, EP);                           \
     } while (0)
-    if (epi == LR_QKV) LR_NORMS(8, 1, LR_QKV, 32);
-    else if (epi == LR_GLU && K >= 3072) LR_NORMS(8, 1, LR_GLU, 16);
-    else if (epi == LR_GLU) LR_NORMS(4, 1, LR_GLU, 16);
-    else if (epi == LR_GELU) LR_NORMS(8, 1, LR_GELU, 16);
-    else if (N > 4096) LR_NORMS(8, 2, LR_PLAIN, 32);
-    else if (K >= 2048) LR_NORMS(16, 1, LR_PLAIN, 16);
-    else LR_NORMS(8, 1, LR_PLAIN, 16);
+#define LR_16(NWV, NTV, EP) LR_NORMS(NWV, NTV, 16, 1, EP)
+#define LR_8(NWV, NTV, EP)                                                    \
+    do {                                                                      \
+        if (M > 8) LR_NORMS(NWV, NTV, 8, 2, EP);                              \
+        else LR_NORMS(NWV, NTV, 8, 1, EP);                                    \
+    } while (0)
+    const bool t8 = K % 64 == 0;
+    if (epi == LR_QKV && N <= 4096 && t8) LR_8(8, 1, LR_QKV);
+    else if (epi == LR_QKV) LR_16(8, 1, LR_QKV);
+    else if (epi == LR_GLU && t8 && M <= 8) LR_NORMS(4, 1, 8, 1, LR_GLU);
+    else if (epi == LR_GLU && t8) LR_NORMS(4, 1, 16, 2, LR_GLU);
+    else if (epi == LR_GLU) LR_16(4, 1, LR_GLU);
+    else if (epi == LR_GELU) LR_16(8, 1, LR_GELU);
+    else if (N > 4096) LR_16(8, 2, LR_PLAIN);
+    else if (N > 2048 && t8) LR_8(8, 2, LR_PLAIN);
+    else if (t8) LR_8(8, 1, LR_PLAIN);
+    else LR_16(8, 1, LR_PLAIN);
+#undef LR_8
+#undef LR_16
 #undef LR_NORMS
 #undef LR_GO
+#undef LR_COLS
     return 0;
 }

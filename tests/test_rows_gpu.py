@@ -46,10 +46,10 @@ def _products(x, w, norm):
     return h @ w.float().t(), h.abs() @ w.float().abs().t()
 
 
-@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("M", [1, 5, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [
     (16, 32), (17, 64), (50257, 96), (768, 3072), (4096, 2048), (4112, 256),
-    (4608, 3584), (1000, 4096 + 32),
+    (4608, 3584), (1000, 4096 + 32), (9, 64), (2052, 576),
 ])
 @pytest.mark.parametrize("kind", [None, "rms", "layer"])
 def test_plain(M, N, K, kind):
@@ -68,7 +68,7 @@ def test_plain(M, N, K, kind):
         assert ((got - y).abs() <= 2 ** -8 * (mag + y.abs()) + 1e-5).all()
 
 
-@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("M", [1, 5, 6, 16])
 @pytest.mark.parametrize("I,K", [(16, 64), (8192, 2048), (48, 3072 + 96)])
 def test_activations(M, I, K):
     torch.manual_seed(M + I)
@@ -88,10 +88,28 @@ def test_activations(M, I, K):
             <= 2 ** -8 * (1.13 * mag + want.abs()) + 1e-5).all()
 
 
+@pytest.mark.parametrize("N,K,act", [
+    (2048, 576, None), (4096, 576, None), (4112, 256, None), (64, 96, None),
+    (4096, 320, "swiglu"), (4096, 96, "swiglu"), (64, 256, "gelu"),
+])
+def test_rows_alone(N, K, act):
+    """A row's result is the same to the bit whatever rows are beside it."""
+    torch.manual_seed(N)
+    x, w, norm = _rand(16, K), _rand(N, K, std=0.05), _norm("rms", K)
+    b = _rand(N) if act == "gelu" else None
+    rows = lambda n: ops.rows_linear(x[:n].contiguous(), w, b, norm=norm,
+                                     act=act)
+    one = rows(1)
+    for n in (2, 8, 9, 16):
+        assert torch.equal(rows(n)[:1], one)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("M,nq,nkv,hd,K,kind", [
     (1, 32, 8, 128, 256, "rms"), (16, 7, 1, 64, 96, "rms"),
     (3, 12, 12, 64, 768, "layer"), (2, 2, 1, 32, 64, "rms"),
+    (8, 24, 4, 128, 320, "rms"), (9, 24, 4, 128, 320, "rms"),
+    (2, 32, 2, 128, 192, "layer"), (3, 32, 2, 128, 192, "rms"),
 ])
 def test_qkv(M, nq, nkv, hd, K, kind, fp8):
     torch.manual_seed(M)
