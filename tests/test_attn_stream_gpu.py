@@ -57,6 +57,10 @@ DECODE = [
     (6, 2, 128, [77, 129], 24, 0), (16, 1, 64, [3000, 40], 256, 32),
     (32, 8, 128, [5 + 37 * i for i in range(40)], 256, 0),
     (28, 4, 128, [9000, 200], 256, 64),
+    # 2 to 4 splits, and some sequences short of them
+    (16, 8, 128, [1 + 50 * i for i in range(20)], 256, 0),
+    (16, 8, 128, [1 + 80 * i for i in range(9)], 256, 0),
+    (12, 12, 64, [1 + 90 * i for i in range(7)], 16, 0),
 ]
 
 
