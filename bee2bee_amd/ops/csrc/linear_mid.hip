@@ -6,15 +6,19 @@
 // would leave three quarters idle at 4096 of them (hence the split), and by
 // the latency of a step. A workgroup takes 64 rows of W and a part of K: four
 // waves of 16 rows, twice, for the two halves of that part. Weights go from
-// memory into the left operand as they lie (three steps in flight), the input
-// rows through LDS, shared by the four waves, xor-ed so that the 16 rows of a
-// read meet in no bank (LDS serves 256 bytes a clock).
+// memory into the left operand as they lie, three steps ahead, the input rows
+// two steps ahead and then through LDS, shared by the four waves, xor-ed so
+// that the 16 rows of a read meet in no bank (LDS serves 256 bytes a clock).
 // Measured beside the library's product (us; 24 / 57 / 80 / 128 rows):
-// 4096x14336 27 / 30 / 34 / 42 (32 / 41 / 43 / 76), 4096x4096 10.8 / 12.5 /
-// 14 / 16 (13.7 / 13.8 / 17 / 24), 6144x4096 15.4 / 18 / 20.5 / 24 (15 / 18 /
-// 23 / 25). Wide outputs stay with the library (2x14336x4096: 66 here against
-// 56 at 24 rows), and so do more rows (200: 54 against 59, but 33 against 27).
+// 4096x14336 26 / 29 / 33 / 40 (32 / 41 / 43 / 76), 4096x4096 10.2 / 11.2 / 13
+// / 16 (13.7 / 13.8 / 17 / 24), 6144x4096 14.7 / 17 / 19 / 24 (15 / 18 / 23 /
+// 25); with the input one step ahead, and twice the workgroups to hide that,
+// 27 / 31 / 34 / 42, 10.6 / 13 / 14 / 16, 15.4 / 18 / 20.5 / 24.5. Wide
+// outputs stay with the library (2x14336x4096: 66 here against 56 at 24 rows),
+// and so do more rows (200: 54 against 59, but 33 against 27).
 #include "common.h"
+
+constexpr int LM_W = 4;     // steps of weights under way, and the current one's
 
 template <int MT>
 __global__ __launch_bounds__(512) void linear_mid_kernel(
@@ -51,19 +55,19 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
         xd[j] = (h * MP + row) * 128 + ((c ^ (row >> 1 & 7)) << 4);
     }
     // (a half without steps left loads, and ignores, a step of the other)
-    bf16x8 xr[NLD];
-    auto load_x = [&](int it) {
+    bf16x8 xr[2][NLD];
+    auto load_x = [&](int set, int it) {
 #pragma unroll
         for (int j = 0; j < NLD; ++j)
-            xr[j] = *reinterpret_cast<const bf16x8*>(
+            xr[set][j] = *reinterpret_cast<const bf16x8*>(
                 xs[j] + (long)min(it, xlast[j]) * 64);
     };
-    auto store_x = [&](int buf) {
+    auto store_x = [&](int set) {          // into the buffer of its number
 #pragma unroll
         for (int j = 0; j < NLD; ++j)
-            *reinterpret_cast<bf16x8*>(smem + buf * XB + xd[j]) = xr[j];
+            *reinterpret_cast<bf16x8*>(smem + set * XB + xd[j]) = xr[set][j];
     };
-    bf16x8 aw[3][2];
+    bf16x8 aw[LM_W][2];
     auto load_w = [&](int set, int it) {
         const long k = (long)min(my0 + it, CH - 1) * 64;
 #pragma unroll
@@ -74,36 +78,44 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    load_x(0);
-    load_w(0, 0);
-    load_w(1, 1);
+    load_x(0, 0);
+#pragma unroll
+    for (int i = 0; i < LM_W - 1; ++i) load_w(i, i);
+    load_x(1, 1);
     store_x(0);
     __syncthreads();
     const char* xb = smem + kh * MP * 128 + li * 128;
-    for (int it0 = 0; it0 < first; it0 += 3) {
+    // step `it` with `it` % LM_W == j: the input of the step after the next
+    // and weights of LM_W - 1 later ones set out, the next step's input goes
+    // to LDS. No load stands under a condition: what is under way would have
+    // to be waited for where the two ways meet.
+    auto step = [&](int j, int it) {
+        load_x(j & 1, it + 2);
+        load_w((j + LM_W - 1) % LM_W, it + LM_W - 1);
+        if (it < mine) {
+            const char* b = xb + (j & 1) * XB;
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int it = it0 + j;
-            if (it >= first) continue;     // (uniform over the workgroup)
-            if (it + 1 < first) load_x(it + 1);
-            load_w((j + 2) % 3, it + 2);
-            if (it < mine) {
-                const char* b = xb + (it & 1) * XB;
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                for (int m = 0; m < MT; ++m) {
+                    const bf16x8 bx = *reinterpret_cast<const bf16x8*>(
+                        b + m * 16 * 128 +
+                        (((s * 4 + lg) ^ (li >> 1)) << 4));
+                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        aw[j][s], bx, acc[m], 0, 0, 0);
+                }
+        }
+        store_x((j + 1) & 1);
+        __syncthreads();
+    };
+    for (int it = 0;;) {
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) {
-                        const bf16x8 bx = *reinterpret_cast<const bf16x8*>(
-                            b + m * 16 * 128 +
-                            (((s * 4 + lg) ^ (li >> 1)) << 4));
-                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            aw[j][s], bx, acc[m], 0, 0, 0);
-                    }
-            }
-            if (it + 1 < first) store_x((it + 1) & 1);
-            __syncthreads();
+        for (int j = 0; j < LM_W; ++j) {
+            step(j, it);
+            if (++it >= first) goto done;
         }
     }
+done:
     // ---- the halves' sums meet in LDS
     f32x4* mg = reinterpret_cast<f32x4*>(smem) + rw * MT * 64 + lane;
     if (kh == 1) {
@@ -126,11 +138,14 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     }
 }
 
-// Splits of K: up to two workgroups a CU, at least four steps of 64 a half.
+// Splits of K: up to a workgroup a CU, at least four steps of 64 a half. Two
+// workgroups a CU: 4096x14336 at 80 rows 36 us against 32.6, 6144x4096 21.5
+// against 18.9, 4096x4096 15.2 against 12.9, and the reader has twice the
+// parts.
 extern "C" int linear_mid_splits(int N, int K) {
     const int tiles = (N + 63) / 64;
     int S = 1;
-    while (S < 8 && tiles * S * 2 <= 512 && K / 64 >= S * 16) S *= 2;
+    while (S < 8 && tiles * S * 2 <= 256 && K / 64 >= S * 16) S *= 2;
     return S;
 }
 
