@@ -1,28 +1,24 @@
 """Op dispatch: hand-written CDNA4 HIP kernels on GPU, fp32 torch reference
 on CPU.
 
-Policy (deliberate, judge-visible): when the tensors live on a GPU the HIP
-extension `_bee2bee_hip` is REQUIRED — a missing/failed extension raises
-immediately rather than silently falling back to eager PyTorch. The torch
-reference path (ops/reference.py) runs only for CPU tensors (tests and
-GPU-less plumbing runs).
+Policy: when the tensors live on a GPU the HIP extension `_bee2bee_hip` is
+REQUIRED — a missing/failed extension raises immediately rather than silently
+falling back to eager PyTorch. The torch reference path (ops/reference.py) runs
+only for CPU tensors (tests and GPU-less plumbing runs).
 
 Kernels (ops/csrc/): fused (add+)RMSNorm, RoPE, paged KV store, paged GQA
-decode attention (flash-decoding style), MFMA flash prefill attention,
-SwiGLU, top-k gating, grouped expert GEMM. Plain projection GEMMs go
-through hipBLASLt via torch.nn.functional.linear — library GEMMs are the
-one place we use a vendor library; every fused hot op is hand-written HIP.
+decode attention, MFMA flash prefill attention, SwiGLU, top-k gating, grouped
+expert GEMM, projections of few rows with what stands around them. Other
+projection GEMMs go through hipBLASLt via torch.nn.functional.linear.
 
-The projection carve-out is MEASURED, not assumed (scripts/bench_skinny.py,
-round 2): across the four Llama-3-8B projection shapes at decode batches
-16/64/256/1536, hipBLASLt beats the hand-written grouped kernel driven as
-a single-segment GEMM on all 16 points (e.g. gate_up at M=64: 6.34 TB/s
-of W vs 3.91 — with one expert segment the grouped grid collapses to
-N/64 workgroups and starves the chip; hipBLASLt's split-K kernels keep
-all 256 CUs fed). The kernel stays the MoE winner because the E-way grid
-and the device-side segment offsets are exactly what the library cannot
-express (its batched path memory-faults at padded M ~1K, and padding an
-uneven routing to bmm shape costs a host sync that blocks hipGraph).
+Which projections are whose is measured: up to 16 rows (`few_rows`) the kernels
+of linear_rows.hip, one launch for norm, product and what follows; 17 to 128
+rows (`mid_rows`) narrow outputs by linear_mid.hip, split over K; wide outputs
+and more rows by the library (gate and up of 14336 x 4096 at 24 rows: 56 us
+there, 66 here). The grouped kernel driven as a single-segment GEMM loses to
+the library on all shapes (scripts/bench_skinny.py: N/64 workgroups starve the
+chip); it stays for experts because the E-way grid and the device-side segment
+offsets are what the library cannot express.
 """
 from __future__ import annotations
 
