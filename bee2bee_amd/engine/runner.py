@@ -217,19 +217,27 @@ class Runner:
         attn_fn,
     ) -> torch.Tensor:
         """Dense layers on some tens of rows: the narrow projections as parts
-        over K, summed by the kernels that read them."""
+        over K, summed by the kernels that read them; of more rows
+        (ops.deep_rows) the down projection alone."""
         s, T = self.spec, x.shape[0]
         layers = self.weights.layers
-        gelu = s.act_type == "gelu"
+        gelu, all_parts = s.act_type == "gelu", ops.mid_rows(x)
         lw = layers[self.layer_lo]
         normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
         for i in range(self.layer_lo, self.layer_hi):
             lw = layers[i]
-            o = self._attend(i, ops.mid_linear(normed, lw.wqkv), positions,
-                             slot_mapping, attn_fn)
-            normed, x = ops.add_norm_parts(
-                ops.mid_linear(o.reshape(T, s.q_size), lw.wo), lw.wo_bias, x,
-                (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps))
+            qkv = (ops.mid_linear(normed, lw.wqkv) if all_parts
+                   else F.linear(normed, lw.wqkv))
+            o = self._attend(i, qkv, positions, slot_mapping,
+                             attn_fn).reshape(T, s.q_size)
+            if all_parts:
+                normed, x = ops.add_norm_parts(
+                    ops.mid_linear(o, lw.wo), lw.wo_bias, x,
+                    (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps))
+            else:
+                normed, x = self._fused_add_norm(
+                    F.linear(o, lw.wo, lw.wo_bias), x, lw.mlp_norm,
+                    lw.mlp_norm_bias)
             z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
             z = ops.gelu(z) if gelu else ops.swiglu(z)
             nxt = None
@@ -509,7 +517,10 @@ class Runner:
                 hidden = self._layer_rows(layer_idx, hidden, positions,
                                           slot_mapping, attn_fn, paged)
             return hidden
-        if self._mid_dims and ops.mid_rows(hidden):
+        s = self.spec
+        if self._mid_dims and (
+                ops.mid_rows(hidden)
+                or ops.deep_rows(hidden, s.intermediate_size)):
             return self._run_layers_mid(hidden, positions, slot_mapping,
                                         attn_fn)
         residual = None

@@ -12,7 +12,7 @@ expert GEMM, projections of few rows with what stands around them. Other
 projection GEMMs go through hipBLASLt via torch.nn.functional.linear.
 
 Which projections are whose is measured: up to 16 rows (`few_rows`) the kernels
-of linear_rows.hip, one launch for norm, product and what follows; 17 to 128
+of linear_rows.hip, one launch for norm, product and what follows; 17 to 160
 rows (`mid_rows`) narrow outputs by linear_mid.hip, split over K; wide outputs
 and more rows by the library (gate and up of 14336 x 4096 at 24 rows: 56 us
 there, 66 here). The grouped kernel driven as a single-segment GEMM loses to
@@ -260,13 +260,22 @@ def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
 # Steps of some tens of rows: narrow projections as fp32 parts over their inner
 # dimension, which the next kernel sums.
 
-MID_MAX = 128
+MID_MAX = 160
+DEEP_MAX = 256
 
 
 def mid_rows(x: torch.Tensor) -> bool:
     """Steps of ROWS_MAX + 1 to MID_MAX contiguous bf16 rows on the GPU."""
     return (x.dim() == 2 and ROWS_MAX < x.shape[0] <= MID_MAX and _use_hip(x)
             and x.dtype is torch.bfloat16 and x.is_contiguous())
+
+
+def deep_rows(x: torch.Tensor, inner: int) -> bool:
+    """Steps of up to DEEP_MAX such rows whose down projection is at least
+    3.5 times as deep as wide."""
+    return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous()
+            and inner * 2 >= 7 * x.shape[1])
 
 
 def mid_linear(x, w):

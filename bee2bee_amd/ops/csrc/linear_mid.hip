@@ -1,5 +1,5 @@
-// Projections of 17 to 128 rows whose output is narrow (q|k|v, attention
-// output, feed-forward output): split over K, the splits' fp32 sums left to
+// Projections of 17 to 160 rows whose output is narrow (q|k|v, attention
+// output, feed-forward output; the last, where it is deep, to 256): split over K, the splits' fp32 sums left to
 // the kernel that reads them anyway (qkv_rope_store, add_norm_parts).
 //
 // Bound by reading the weights once, by a chip that 64 columns a workgroup
@@ -14,8 +14,13 @@
 // / 16 (13.7 / 13.8 / 17 / 24), 6144x4096 14.7 / 17 / 19 / 24 (15 / 18 / 23 /
 // 25); with the input one step ahead, and twice the workgroups to hide that,
 // 27 / 31 / 34 / 42, 10.6 / 13 / 14 / 16, 15.4 / 18 / 20.5 / 24.5. Wide
-// outputs stay with the library (2x14336x4096: 66 here against 56 at 24 rows),
-// and so do more rows (200: 54 against 59, but 33 against 27).
+// outputs stay with the library (2x14336x4096: 66 here against 56 at 24 rows).
+// At 160 / 200 / 256 rows 4096x14336 46 / 54 / 62 (84 / 57 / 63), 6144x4096 26
+// / 31 / 35 (28 / 26 / 40), 4096x4096 17.5 / 20.5 / 23 (27 / 22 / 22.5),
+// 3072x8192 27 / 32 / 36 (28 / 31 / 34), 3072x2048 11.6 / 13.7 / 15.5 (12 / 13
+// / 13), but 3584x18944 56 / 67 / 76 (107 / 123 / 127) and 2048x8192 18 / 21 /
+// 24 (26 / 27.5 / 26.5): above 160 rows only products 3.5 times as deep as
+// wide, and deeper.
 #include "common.h"
 
 constexpr int LM_W = 4;     // steps of weights under way, and the current one's
@@ -150,12 +155,12 @@ extern "C" int linear_mid_splits(int N, int K) {
 }
 
 // part [S, M, N] fp32: x [M, K] times rows of w [N, K] over S parts of K. x and
-// w contiguous and 16-byte aligned, 1 <= M <= 128, N % 4 == 0, K % 64 == 0, S
+// w contiguous and 16-byte aligned, 1 <= M <= 256, N % 4 == 0, K % 64 == 0, S
 // <= K / 64; nonzero for anything else.
 extern "C" int launch_linear_mid(const unsigned short* x,
                                  const unsigned short* w, float* part, int M,
                                  int N, int K, int S, hipStream_t stream) {
-    if (M < 1 || M > 128 || N < 4 || N % 4 || K < 64 || K % 64) return 1;
+    if (M < 1 || M > 256 || N < 4 || N % 4 || K < 64 || K % 64) return 1;
     if (S < 1 || S > K / 64) return 1;
     const dim3 grid((N + 63) / 64, S);
 #define LM_GO(MTV)                                                            \
@@ -164,7 +169,11 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     if (M <= 32) LM_GO(2);
     else if (M <= 64) LM_GO(4);
     else if (M <= 96) LM_GO(6);
-    else LM_GO(8);
+    else if (M <= 128) LM_GO(8);
+    else if (M <= 160) LM_GO(10);
+    else if (M <= 192) LM_GO(12);
+    else if (M <= 224) LM_GO(14);
+    else LM_GO(16);
 #undef LM_GO
     return 0;
 }

@@ -161,7 +161,7 @@ Tensor mid_linear(const Tensor& x, const Tensor& w) {
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
                 "x [M, K] and w [N, K]");
     const int M = x.size(0), K = x.size(1), N = w.size(0);
-    TORCH_CHECK(M >= 1 && M <= 128, "1 to 128 rows");
+    TORCH_CHECK(M >= 1 && M <= 256, "1 to 256 rows");
     TORCH_CHECK(K % 64 == 0 && N % 4 == 0);
     const Tensor xd = dense(x, "x"), wd = dense(w, "w");
     const int S = linear_mid_splits(N, K);

@@ -169,7 +169,8 @@ def test_refused():
 # ------------------------------------------------- steps of some tens of rows
 
 
-@pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128, 129, 160,
+                               161, 200, 256])
 @pytest.mark.parametrize("N,K", [(64, 64), (68, 1088), (3584, 960),
                                  (4096, 2048), (512, 8192 + 64)])
 def test_parts_over_k(M, N, K):
