@@ -22,7 +22,9 @@
 //  * two batches of weight loads, LR_U tiles each, are on their way: with 8 or
 //    16 the registers cost more waves than the loads gain (output head of
 //    128256 x 4096, us: 4 tiles 182, 8 205, 16 230), and a streaming hint on
-//    the loads loses the half lines a 64-byte piece leaves (206 to 240).
+//    the loads loses the half lines a 64-byte piece leaves (206 to 240). The
+//    input asked for as early as the weights costs registers too (a step of 8
+//    layers of 3584, two rows: 1220 to 1290 us; of 4096, one row: 1014 to 1034).
 // Measured (us, one row, beside the library product alone): 6144x4096 15.3
 // (14.5), 4096x4096 9.3 (15.6), 2x14336x4096 44 (64), 4096x14336 25 (27),
 // 128256x4096 183 (190); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
