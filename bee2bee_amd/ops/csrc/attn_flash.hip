@@ -290,7 +290,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 o[d][r] = o[d][r] * a0 + mg[(d * 16 + r) * 64] * a1;
     }
     if (!row_ok) return;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const float inv = l == 0.f ? 0.f : 1.f / l;
     unsigned short* orow = out + ((long)(s0 + pos) * nq + head) * HD;
 #pragma unroll
     for (int d = 0; d < DT; ++d)

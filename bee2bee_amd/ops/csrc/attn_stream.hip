@@ -326,7 +326,8 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
                 out_ml[q_off[t] * 2 + 1] = lsum;
             }
         }
-        const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+        // (no keys: zeros; a NaN is neither less nor greater and stays one)
+        const float inv = lsum == 0.f ? 0.f : 1.f / lsum;
         for (int d = wid; d < DT; d += ST_WAVES) {
             f32x4 a{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(HD / 4 * P) void attn_stream_combine_kernel(
     short4v y;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        y[r] = (short)f2bf(lsum > 0.f ? acc[r] / lsum : 0.f);
+        y[r] = (short)f2bf(lsum == 0.f ? 0.f : acc[r] / lsum);
     *reinterpret_cast<short4v*>(out + at * HD + c * 4) = y;
     if (out_ml && c == 0) {
         out_ml[at * 2] = M / ST_LOG2E;

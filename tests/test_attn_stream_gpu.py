@@ -134,3 +134,24 @@ def test_an_empty_context_is_zero():
     q = torch.randn(2, 4, 64, device=DEV).bfloat16()
     out, ml = ops.attn_decode_lse(q, kc, vc, table, lens, 0.125)
     assert (out[1] == 0).all() and (ml[1, :, 1] == 0).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("nseq", [2, 40])      # contexts split, and not
+def test_a_nan_reaches_the_output(nseq, fp8):
+    """A NaN in a key takes the rows of its head, one in a value its
+    coordinate, and nothing else, whatever the batch."""
+    kc, vc, table, lens = _pages(8, 128, 256, [600] * nseq, fp8, 6)
+    nan = 0x7F if fp8 else float("nan")
+    kc[table[0, 0], 3, 5, 17] = nan
+    vc[table[1, 2], 6, 600 - 512 - 1, 40] = nan
+    q = torch.randn(nseq, 32, 128, device=DEV).bfloat16()
+    got, ml = ops.attn_decode_lse(q, kc, vc, table, lens, 0.1)
+    want, want_ml = reference.attn_decode_lse(q.float(), _wide(kc), _wide(vc),
+                                              table, lens, 0.1)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert got.isnan().sum() == 4 * 128 + 4
+    assert torch.equal(ml[..., 1].isnan(), want_ml[..., 1].isnan())
+    rows = ops.attn_prefill_paged(q, kc, vc, table, lens, torch.arange(
+        nseq + 1, device=DEV, dtype=torch.int32), 1, 0.1)
+    assert torch.equal(rows.isnan(), want.isnan())
