@@ -96,7 +96,9 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     const int s0 = cu ? cu[b] : b;
     const int rows = (cu ? cu[b + 1] - s0 : 1) * G;
     const int row0 = blockIdx.z * QT * 16;
-    if (row0 >= rows) return;
+    // a chunk longer than the caller said has no room in the workspaces
+    const int live = min(rows, max_rows);
+    if (row0 >= live) return;
     const int L = seq_lens[b];
     const int hist = L - rows / G;
     const int per = split_keys(L, Z);
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-        if (row0 + t * 16 + li >= rows) continue;
+        if (row0 + t * 16 + li >= live) continue;
         float wm[ST_WAVES], M = -1e30f, lsum = 0.f;
 #pragma unroll
         for (int w = 0; w < ST_WAVES; ++w) {

@@ -155,3 +155,15 @@ def test_a_nan_reaches_the_output(nseq, fp8):
     rows = ops.attn_prefill_paged(q, kc, vc, table, lens, torch.arange(
         nseq + 1, device=DEV, dtype=torch.int32), 1, 0.1)
     assert torch.equal(rows.isnan(), want.isnan())
+
+
+def test_a_chunk_longer_than_said():
+    """Rows past max_qlen have no place in the splits' workspaces: they are
+    left out, and the rows before them are what they are without them."""
+    kc, vc, table, lens = _pages(2, 64, 256, [1500, 905], False, 8)
+    q = torch.randn(10, 8, 64, device=DEV).bfloat16()
+    cu = torch.tensor([0, 5, 10], dtype=torch.int32, device=DEV)
+    want = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, 5, 0.125)
+    got = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, 3, 0.125)
+    for at in (0, 5):
+        assert torch.equal(got[at : at + 3], want[at : at + 3])
