@@ -63,9 +63,10 @@ DEV_INLINE bf16x8 st_round_fp8(bf16x8 x, float scale) {
     return __builtin_bit_cast(bf16x8, st_widen(w));
 }
 
-// keys per split: whole steps of a workgroup, the same for every reader
-DEV_INLINE int split_keys(int L, int Z) {
-    return ((L + Z - 1) / Z + ST_STEP - 1) / ST_STEP * ST_STEP;
+// keys per split, the same for every reader: a context in `even` parts of whole
+// steps of a workgroup, none above `most` keys (whole steps too)
+DEV_INLINE int split_keys(int L, int even, int most) {
+    return min(((L + even - 1) / even + ST_STEP - 1) / ST_STEP * ST_STEP, most);
 }
 
 template <int HD, int QT, typename KVT>
@@ -75,7 +76,8 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     const int* __restrict__ block_table, const int* __restrict__ seq_lens,
     unsigned short* __restrict__ out, float* __restrict__ out_ml,
     float* __restrict__ part_o, float* __restrict__ part_ml, int nkv, int G,
-    int W, int bs, int Z, int max_rows, long s_q, float scale) {
+    int W, int bs, int Z, int even, int most, int max_rows, long s_q,
+    float scale) {
     constexpr int KS = HD / 32;          // k steps of a score tile
     constexpr int DT = HD / 16;          // output tiles of 16 coordinates
     constexpr int CPR = HD / 8;          // chunks of 8 elements of a key row
@@ -101,7 +103,8 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     if (row0 >= live) return;
     const int L = seq_lens[b];
     const int hist = L - rows / G;
-    const int per = split_keys(L, Z);
+    const int per = split_keys(L, even, most);
+    const bool split = L > per;          // or the result itself is written
     const int k0 = blockIdx.y * per, k1 = min(L, k0 + per);
     if (k0 >= L && blockIdx.y > 0) return;
     const int* bt = block_table + (long)b * W;
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
             ((long)blockIdx.x * Z + blockIdx.y) * max_rows + row0 + t * 16 +
             li;
         if (wid == 0 && lg == 0) {
-            if (Z > 1) {
+            if (split) {
                 part_ml[part * 2] = M;
                 part_ml[part * 2 + 1] = lsum;
             } else if (out_ml) {
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) a[r] += x[r] * wm[w];
             }
-            if (Z > 1) {
+            if (split) {
                 *reinterpret_cast<f32x4*>(part_o + part * HD + d * 16 +
                                           lg * 4) = a;
             } else {
@@ -366,15 +369,16 @@ __global__ __launch_bounds__(HD / 4 * P) void attn_stream_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
     const int* __restrict__ cu, const int* __restrict__ seq_lens,
     unsigned short* __restrict__ out, float* __restrict__ out_ml, int nkv,
-    int G, int Z, int max_rows) {
+    int G, int Z, int even, int most, int max_rows) {
     constexpr int C = HD / 4;                  // threads of a split
     const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
     const int s0 = cu ? cu[b] : b;
     const int row = blockIdx.y;
     if (row >= (cu ? cu[b + 1] - s0 : 1) * G) return;
     const int L = seq_lens[b];
-    const int per = split_keys(L, Z);
-    const int nz = L > 0 ? (L + per - 1) / per : 0;
+    const int per = split_keys(L, even, most);
+    if (L <= per) return;                      // written by its workgroup
+    const int nz = min((L + per - 1) / per, Z);
     const long p0 = (long)blockIdx.x * Z * max_rows + row;
     const int lane = threadIdx.x & 63, c = threadIdx.x % C;
     const int z0 = threadIdx.x / C;            // 0 .. P - 1
@@ -443,18 +447,43 @@ extern "C" int attn_stream_takes(long pairs, long rows) {
     return rows <= 32 || stream_groups(pairs, rows) <= 448;
 }
 
-// Splits of a context of up to `keys` keys (what the block table holds):
-// about a workgroup a CU. More cost more in the combine than they hide (192
-// (sequence, key head) pairs of up to 2000 keys: 25.1 us with 2 splits, 26.4
-// with 6, 28.9 with 16; 8 pairs of 3000: 35.7 with 1, 10.1 with 8, 8.6 with
-// 32); from 256 pairs on one split writes its result itself.
-extern "C" int attn_stream_splits(long pairs, long rows, long keys) {
-    const long groups = stream_groups(pairs, rows);
-    const long most = (keys + ST_STEP - 1) / ST_STEP;
-    long z = (256 + groups - 1) / groups;
-    if (z > 32) z = 32;                        // the combine's lanes
-    if (z > most) z = most;
-    return z < 1 ? 1 : (int)z;
+// Splits of the contexts of a step, of up to `keys` keys (what the block table
+// holds; their lengths are on the GPU). `even`: about a workgroup a CU where
+// there are few; more cost more in the combine than they hide (192 (sequence,
+// key head) pairs of up to 2000 keys: 25.1 us with 2 splits, 26.4 with 6, 28.9
+// with 16; 8 pairs of 3000: 35.7 with 1, 10.1 with 8, 8.6 with 32).
+// `most`: a workgroup takes 12 ns a key, so with one or two splits the longest
+// context of an uneven batch is read by a few CUs when the others are done.
+// There, a context is cut into parts of 2048 keys and more, as many as keep the
+// grid within ST_GRID workgroups (most leave at once). One long context among
+// short ones of 60 keys (us, 8 key heads of size 128; even splits alone / with
+// the limit / the three-stage kernels before, of 4096 workgroups): 4000 and 42
+// short ones 45.7 / 26.5 / 35.5, 8000 and 42 86.5 / 29.4 / 48.7; of 4 key
+// heads 8000 and 79 83 / 27 / 59, 30000 and 79 299 / 85 / 213. An even batch
+// may pay for the combine: 16 of 900 to 7000 61.3 / 64.9 / 88.8, 64 of 500 to
+// 4000 117.1 / 117.6 / 154, but 24 of 900 to 7000 89.9 / 82.4 / 105. From 768
+// groups on nothing is cut (200 of 400 to 3000 would take 237.8, not 232.9),
+// and the three stages had five workgroups a context or fewer, of 67 ns a key.
+constexpr long ST_GRID = 1536;
+extern "C" int attn_stream_splits(long pairs, long rows, long keys, int* even,
+                                  int* most) {
+    const long groups = pairs > 0 ? stream_groups(pairs, rows) : 1;
+    const long steps = (keys + ST_STEP - 1) / ST_STEP;
+    long e = (256 + groups - 1) / groups;
+    if (e > 32) e = 32;                        // the combine's lanes
+    if (e > steps) e = steps;
+    if (e < 1) e = 1;
+    long z = e;
+    if (e <= 2) {
+        z = (keys + 2047) / 2048;
+        if (z > ST_GRID / groups) z = ST_GRID / groups;
+        if (z > 32) z = 32;
+        if (z < e) z = e;
+    }
+    *even = (int)e;
+    // (a split of no more than its share of `keys`: never more than z)
+    *most = z > e ? (int)((steps + z - 1) / z) * ST_STEP : 1 << 30;
+    return (int)z;
 }
 
 // cu null: one row a sequence (decode). part_o [nseq * nkv, Z, max_rows, hd]
@@ -465,8 +494,8 @@ extern "C" int launch_attn_stream(
     const unsigned short* q, const void* k_cache, const void* v_cache,
     const int* cu, const int* block_table, const int* seq_lens,
     unsigned short* out, float* out_ml, float* part_o, float* part_ml,
-    int nseq, int nkv, int G, int W, int bs, int hd, int Z, int max_qlen,
-    long s_q, float scale, int fp8, hipStream_t stream) {
+    int nseq, int nkv, int G, int W, int bs, int hd, int Z, int even, int most,
+    int max_qlen, long s_q, float scale, int fp8, hipStream_t stream) {
     if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
     if (nseq == 0 || max_qlen <= 0) return 0;
     const int max_rows = max_qlen * G;
@@ -479,12 +508,12 @@ extern "C" int launch_attn_stream(
                        dim3(ST_WAVES * 64), smem, stream, q,                  \
                        (const KVT*)k_cache, (const KVT*)v_cache, cu,          \
                        block_table, seq_lens, out, out_ml, part_o, part_ml,   \
-                       nkv, G, W, bs, Z, max_rows, s_q, scale)
+                       nkv, G, W, bs, Z, even, most, max_rows, s_q, scale)
 #define ST_COMBINE(HDV, P, I)                                                 \
     hipLaunchKernelGGL((attn_stream_combine_kernel<HDV, P, I>),               \
                        dim3(nseq * nkv, max_rows), dim3(HDV / 4 * (P)), 0,    \
                        stream, part_o, part_ml, cu, seq_lens, out, out_ml,    \
-                       nkv, G, Z, max_rows)
+                       nkv, G, Z, even, most, max_rows)
 #define ST_HD(HDV)                                                            \
     do {                                                                      \
         if (fp8 && qt == 1) ST_ONE(HDV, 1, unsigned char);                    \

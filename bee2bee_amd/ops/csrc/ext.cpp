@@ -38,11 +38,11 @@ void launch_attn_decode(const unsigned short*, const void*, const void*,
                         float*, unsigned short*, float*, int, int, int, int,
                         int, int, int, long, float, int, hipStream_t);
 int attn_stream_takes(long, long);
-int attn_stream_splits(long, long, long);
+int attn_stream_splits(long, long, long, int*, int*);
 int launch_attn_stream(const unsigned short*, const void*, const void*,
                        const int*, const int*, const int*, unsigned short*,
                        float*, float*, float*, int, int, int, int, int, int,
-                       int, int, long, float, int, hipStream_t);
+                       int, int, int, int, long, float, int, hipStream_t);
 void launch_attn_prefill(const unsigned short*, const unsigned short*,
                          const unsigned short*, const int*, unsigned short*,
                          long, int, int, int, int, long, long, long, int,
@@ -233,7 +233,9 @@ bool attn_stream(const Tensor& q_in, const Tensor& k_cache,
     const int bs = k_cache.size(2), W = block_table.size(1);
     const int G = nq / nkv;
     const long pairs = (long)nseq * nkv, rows = (long)max_qlen * G;
-    const int Z = attn_stream_splits(pairs, rows, (long)W * bs);
+    int even, most;
+    const int Z =
+        attn_stream_splits(pairs, rows, (long)W * bs, &even, &most);
     auto fopt = q.options().dtype(torch::kFloat32);
     Tensor part_o, part_ml;
     if (Z > 1) {
@@ -246,7 +248,7 @@ bool attn_stream(const Tensor& q_in, const Tensor& k_cache,
                bf16p_mut(out), out_ml,
                Z > 1 ? part_o.data_ptr<float>() : nullptr,
                Z > 1 ? part_ml.data_ptr<float>() : nullptr, nseq, nkv, G, W,
-               bs, hd, Z, max_qlen, q.stride(0), (float)scale,
+               bs, hd, Z, even, most, max_qlen, q.stride(0), (float)scale,
                k_cache.scalar_type() == torch::kUInt8, stream()) == 0;
 }
 

@@ -61,6 +61,11 @@ DECODE = [
     (16, 8, 128, [1 + 50 * i for i in range(20)], 256, 0),
     (16, 8, 128, [1 + 80 * i for i in range(9)], 256, 0),
     (12, 12, 64, [1 + 90 * i for i in range(7)], 16, 0),
+    # long contexts among short ones: parts of limited length, and contexts
+    # of one part that write their result beside them
+    (16, 8, 128, [5000, 2048, 2049, 4096, 4097, 1] + [60] * 30, 256, 32),
+    (16, 8, 128, [60] * 14 + [7000, 300, 2048, 128], 256, 32),
+    (12, 12, 64, [2049, 33] + [33] * 20 + [4100], 64, 96),
 ]
 
 
