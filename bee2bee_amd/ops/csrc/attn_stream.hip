@@ -258,12 +258,12 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(
+                for (int r = 0; r < 4; ++r)
+                    bp[t][h * 4 + r] = (__bf16)__builtin_amdgcn_exp2f(
                         fmaf(s[h][t][r], scale_log2, -m[t]));
-                    l[t] += p;
-                    bp[t][h * 4 + r] = (__bf16)p;
-                }
+            // the sum that divides is of the weights as they are multiplied:
+            // what rounding does to both cancels
+            l[t] = add_bf16x8(bp[t], l[t]);
         }
         // ---- O^T += V^T P^T; keys in the order the score tiles hold them:
         // lane group lg has 4 lg + {0..3}, then 16 + 4 lg + {0..3}

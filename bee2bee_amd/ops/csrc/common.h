@@ -134,6 +134,17 @@ DEV_INLINE float rows_sum(float x) {
     return pair_sum(p.x + p.y);
 }
 
+// acc + the eight elements, in fp32
+DEV_INLINE float add_bf16x8(bf16x8 v, float acc) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    const bf16x2 ones{(__bf16)1.f, (__bf16)1.f};
+#pragma unroll
+    for (int e = 0; e < 8; e += 2)
+        acc = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{v[e], v[e + 1]}, ones,
+                                              acc, false);
+    return acc;
+}
+
 // LDS hand-over inside ONE wave (no workgroup barrier): a wave's LDS
 // operations execute in order, so earlier writes of any lane are seen by
 // later reads of any lane; the fences keep the compiler from moving them.

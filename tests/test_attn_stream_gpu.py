@@ -172,3 +172,26 @@ def test_a_chunk_longer_than_said():
     got = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, 3, 0.125)
     for at in (0, 5):
         assert torch.equal(got[at : at + 3], want[at : at + 3])
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("nseq", [1, 40])      # contexts split, and not
+def test_weights_add_up_to_one(nseq, hd):
+    """Where all values are 1 the output is 1: the sum that divides is of the
+    weights as they are multiplied. One key of a wave's 32 at the maximum, the
+    others where rounding to bf16 takes most (0.5 and 0.98 of half a unit), or
+    anywhere."""
+    for far in (True, False):
+        kc, vc, table, lens = _pages(8, hd, 256, [1000] * nseq, False, 7)
+        vc.fill_(1.0)
+        q = torch.randn(nseq, 8, hd, device=DEV).bfloat16()
+        scale = hd ** -0.5
+        if far:
+            q.zero_()
+            q[..., :2] = 1.0
+            kc.zero_()
+            kc[..., 0], kc[..., 1] = -1.0, 0.0055
+            kc[:, :, ::32, :2] = 0.0
+            scale = 0.6931471805599453
+        got = ops.attn_decode(q, kc, vc, table, lens, scale)
+        assert (got == 1).all(), (far, got.float().min().item())
