@@ -16,9 +16,10 @@
 //  * Keys and values are staged in LDS row-major (two buffers), 16-byte chunks
 //    xor-ed by the key, the next tile's global reads in flight over the
 //    current tile's products.
-//  * The running maximum is raised only by a score FL_SLACK powers of two
-//    above it: most tiles leave the sums as they are. Weights stay below
-//    2^FL_SLACK, whose bf16 rounding is as fine, and sums are fp32.
+//  * At head size 128 the running maximum is raised only by a score FL_SLACK
+//    powers of two above it: most tiles leave the sums as they are. Sums are
+//    fp32, of the weights as rounded for the product, so that most of what
+//    rounding does cancels.
 // Scores are scaled in fp32 (queries enter the product unrounded). The kernel
 // before it (16-row tiles, weights and V transposed through LDS by 2-byte
 // writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
@@ -36,8 +37,15 @@ typedef __attribute__((address_space(3))) short4v lds_short4v;
 
 constexpr int FL_KT = 64;   // keys per staged tile
 // a row's running maximum is raised only by a score this far (in powers of
-// two) above it
-constexpr float FL_SLACK = 8.f;
+// two) above it. A row's largest weight is then rounded like the others instead
+// of being 1: of rows that few keys dominate the error grows (random scores of
+// deviation 4, 300 keys, relative to 64 bits, before the output's rounding:
+// 0.0005 without slack, 0.0008 with it). The kernel before, which rounded the
+// scaled queries to bf16 and summed the unrounded weights, had 0.0033 at head
+// size 128, but 0.0005 at 64, where the scale is a power of two: slack at 128
+// only. It is worth 3 to 6% there (4096 queries on 16384 keys 918 us against
+// 945, 700 on 7700 160 against 171), 1 to 3% at 64.
+template <int HD> constexpr float FL_SLACK = HD == 128 ? 8.f : 0.f;
 
 template <int HD, int RW, int KSP, bool PAGED, typename KVT>
 __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
@@ -220,7 +228,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[f][r]);
             mx = pair_max(mx) * scale_log2;
-            if (__any(mx > m + FL_SLACK)) {
+            if (__any(mx > m + FL_SLACK<HD>)) {
                 const float mn = fmaxf(m, mx);
                 const float alpha = __builtin_amdgcn_exp2f(m - mn);
                 m = mn;
@@ -234,12 +242,12 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
 #pragma unroll
             for (int f = 0; f < NF; ++f)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(
+                for (int r = 0; r < 16; ++r)
+                    bp[f * 2 + r / 8][r % 8] = (__bf16)__builtin_amdgcn_exp2f(
                         fmaf(s[f][r], scale_log2, -m));
-                    l += p;
-                    bp[f * 2 + r / 8][r % 8] = (__bf16)p;
-                }
+            // the sum that divides is of the weights as they are multiplied
+#pragma unroll
+            for (int st = 0; st < NF * 2; ++st) l = add_bf16x8(bp[st], l);
             // ---- O^T += V^T P^T; the keys of a step in the order the score
             // tile holds them: 4 hi + {0..3}, then 8 + 4 hi + {0..3}
 #pragma unroll

@@ -110,3 +110,21 @@ def test_a_scale_that_is_not_positive():
         want = reference.attn_prefill(q.float(), k.float(), v.float(),
                                       _cu([70]), 70, scale)
         _check(got, want, v)
+
+
+@pytest.mark.parametrize("T", [300, 3000])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_weights_add_up_to_one(hd, T):
+    """Where all values are 1 the output is 1: the sum that divides is of the
+    weights as they are multiplied. Key 70's weight is 2^7 and 0.98 of half a
+    unit of bf16 above, within the kernel's slack."""
+    q = torch.zeros(T, 8, hd, device=DEV).bfloat16()
+    k = torch.zeros(T, 8, hd, device=DEV).bfloat16()
+    q[..., :2] = 1.0
+    k[70, :, 0], k[70, :, 1] = 7.0, 0.0055
+    v = torch.ones_like(k)
+    got = ops.attn_prefill(q, k, v, _cu([T]), T, 0.6931471805599453)
+    assert (got == 1).all(), got.float().min().item()
+    q, k, _ = _qkv(T, 8, 8, hd, 5)
+    got = ops.attn_prefill(q, k, v, _cu([T]), T, hd ** -0.5)
+    assert (got == 1).all(), got.float().min().item()
