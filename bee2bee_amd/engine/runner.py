@@ -153,38 +153,48 @@ class Runner:
         normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
         return F.linear(normed, W.lm_head)
 
-    def _layer_rows(
+    def _run_layers_rows(
         self,
-        layer_idx: int,
         x: torch.Tensor,
         positions: torch.Tensor,
         slot_mapping: torch.Tensor,
         attn_fn,
         paged: bool,
     ) -> torch.Tensor:
-        """A dense layer on a few rows: five launches, each projection with
-        its norm, and bias, activation or residual add, folded in. paged:
+        """Dense layers on a few rows: five launches each, every projection
+        with its norm, and bias, activation or residual add, folded in. paged:
         attention reads the pages only, so rotation and store go into the
-        q|k|v projection too."""
-        s, lw = self.spec, self.weights.layers[layer_idx]
-        T = x.shape[0]
-        k_cache, v_cache = self.kv.layer(layer_idx)
-        norm = (lw.attn_norm, lw.attn_norm_bias, s.rms_eps)
+        q|k|v projection too. The residual x stays in fp32 between the first
+        layer's input and the last one's result; rows and norm are what the
+        next projection reads."""
+        s, T = self.spec, x.shape[0]
+        layers = self.weights.layers
+        lw = layers[self.layer_lo]
+        rows, norm = x, (lw.attn_norm, lw.attn_norm_bias, s.rms_eps)
         rope = s.pos_type == "rope"
-        if paged and s.head_dim % 32 == 0:
-            q = ops.rows_qkv(x, lw.wqkv, lw.wqkv_bias, norm, s.n_heads,
-                             positions if rope else None, self.rope_cos,
-                             self.rope_sin, k_cache, v_cache, slot_mapping)
-            o = attn_fn(layer_idx, q, None, None, k_cache, v_cache)
-        else:
-            o = self._attend(layer_idx,
-                             ops.rows_linear(x, lw.wqkv, norm=norm),
-                             positions, slot_mapping, attn_fn)
-        x = self._rows_add(x, o.reshape(T, s.q_size), lw.wo, lw.wo_bias)
-        norm = (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps)
-        act = ops.rows_linear(x, lw.w_gate_up, lw.w_gate_up_bias, norm=norm,
-                              act="gelu" if s.act_type == "gelu" else "swiglu")
-        return self._rows_add(x, act, lw.w_down, lw.w_down_bias)
+        for i in range(self.layer_lo, self.layer_hi):
+            lw = layers[i]
+            k_cache, v_cache = self.kv.layer(i)
+            if paged and s.head_dim % 32 == 0:
+                q = ops.rows_qkv(rows, lw.wqkv, lw.wqkv_bias, norm, s.n_heads,
+                                 positions if rope else None, self.rope_cos,
+                                 self.rope_sin, k_cache, v_cache, slot_mapping)
+                o = attn_fn(i, q, None, None, k_cache, v_cache)
+            else:
+                o = self._attend(i, ops.rows_linear(rows, lw.wqkv, norm=norm),
+                                 positions, slot_mapping, attn_fn)
+            x, rows, norm = self._rows_add(
+                x, o.reshape(T, s.q_size), lw.wo, lw.wo_bias,
+                (lw.mlp_norm, lw.mlp_norm_bias))
+            act = ops.rows_linear(
+                rows, lw.w_gate_up, lw.w_gate_up_bias, norm=norm,
+                act="gelu" if s.act_type == "gelu" else "swiglu")
+            nxt = None
+            if i + 1 < self.layer_hi:
+                nxt = layers[i + 1].attn_norm, layers[i + 1].attn_norm_bias
+            x, rows, norm = self._rows_add(x, act, lw.w_down, lw.w_down_bias,
+                                           nxt)
+        return x
 
     def _attend(self, layer_idx: int, qkv, positions, slot_mapping, attn_fn):
         """Attention of a layer on its projected q|k|v: rows [T, N], or their
@@ -248,17 +258,29 @@ class Runner:
                                            lw.w_down_bias, x, nxt)
         return x
 
-    def _rows_add(self, x, y, w, bias) -> torch.Tensor:
-        """x + y w^T + bias; under tensor parallelism y and w are this rank's
-        part of the inner dimension."""
+    def _rows_add(self, x, y, w, bias, nxt):
+        """x + y w^T + bias, and the rows and norm of the projection that
+        reads it through `nxt`, a norm's (weight, bias) (None: the sum alone,
+        in bf16). Under tensor parallelism y and w are this rank's part of the
+        inner dimension."""
         if self.tp_group is not None:
             import torch.distributed as dist
 
             if dist.get_world_size(self.tp_group) > 1:
                 part = ops.rows_linear(y, w, bias)
                 dist.all_reduce(part, group=self.tp_group)
-                return x + part
-        return ops.rows_linear(y, w, bias, x)
+                if nxt is None:
+                    return x + part, None, None
+                normed, x = self._fused_add_norm(part, x, *nxt)
+                return x, normed, None
+        if nxt is None:
+            return ops.rows_linear(y, w, bias, x), None, None
+        if nxt[1] is not None:
+            x = ops.rows_linear(y, w, bias, x, keep32=True)
+            return x, x, (*nxt, self.spec.rms_eps)
+        x, scaled, squares = ops.rows_linear(y, w, bias, x, keep32=True,
+                                             then=nxt[0])
+        return x, scaled, (squares, self.spec.rms_eps)
 
     def _layer(
         self,
@@ -512,11 +534,11 @@ class Runner:
         attn_fn,
         paged: bool = True,
     ) -> torch.Tensor:
-        if self._rows_dims and ops.few_rows(hidden):
-            for layer_idx in range(self.layer_lo, self.layer_hi):
-                hidden = self._layer_rows(layer_idx, hidden, positions,
-                                          slot_mapping, attn_fn, paged)
+        if self.layer_lo >= self.layer_hi:
             return hidden
+        if self._rows_dims and ops.few_rows(hidden):
+            return self._run_layers_rows(hidden, positions, slot_mapping,
+                                         attn_fn, paged)
         s = self.spec
         if self._mid_dims and (
                 ops.mid_rows(hidden)

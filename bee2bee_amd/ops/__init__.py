@@ -221,7 +221,7 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
 # ---------------------------------------------------- steps of a few rows
 # One launch a projection, with the norm before it and what follows it folded
 # in. norm: (weight, bias or None, eps) - with a bias layer norm, without RMS
-# norm.
+# norm - or (squares, eps): RMS norm of rows that rows_linear's `then` made.
 
 ROWS_MAX = 16
 
@@ -234,15 +234,28 @@ def few_rows(x: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0)
 
 
-def rows_linear(x, w, bias=None, resid=None, norm=None, act=None):
+def _norm_args(norm):
+    """weight, bias, squares, eps of the bindings."""
+    if norm is None:
+        return None, None, None, 0.0
+    return (None, None, *norm) if len(norm) == 2 else (*norm[:2], None,
+                                                       norm[2])
+
+
+def rows_linear(x, w, bias=None, resid=None, norm=None, act=None,
+                keep32=False, then=None):
     """act(norm(x) w^T + bias) + resid. act: None, "gelu" (tanh form), or
-    "swiglu" (w holds the gate's rows, then the values'; no bias)."""
+    "swiglu" (w holds the gate's rows, then the values'; no bias). x of a layer
+    norm, and resid, may be fp32. Without act: keep32 leaves the result in
+    fp32; `then`, the weight of the RMS norm that reads it, adds what that
+    norm's projection takes: -> (result, result * then, sums of squares of 8
+    columns each)."""
     if _use_hip(x):
-        nw, nb, eps = norm or (None, None, 0.0)
-        return require_hip().rows_linear(
-            x, w, bias, resid, nw, nb, eps,
-            {None: 0, "swiglu": 1, "gelu": 2}[act])
-    return reference.rows_linear(x, w, bias, resid, norm, act)
+        out = require_hip().rows_linear(
+            x, w, bias, resid, *_norm_args(norm),
+            {None: 0, "swiglu": 1, "gelu": 2}[act], keep32, then)
+        return out[0] if then is None else tuple(out)
+    return reference.rows_linear(x, w, bias, resid, norm, act, keep32, then)
 
 
 def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
@@ -250,9 +263,9 @@ def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
     """norm(x) w^T + bias split into q|k|v; q and k rotated (positions None:
     not), k and v stored into their pages. -> q [T, n_heads, hd]."""
     if _use_hip(x):
-        return require_hip().rows_qkv(x, w, bias, norm[0], norm[1], norm[2],
-                                      n_heads, positions, cos, sin, k_cache,
-                                      v_cache, slot_mapping)
+        return require_hip().rows_qkv(x, w, bias, *_norm_args(norm), n_heads,
+                                      positions, cos, sin, k_cache, v_cache,
+                                      slot_mapping)
     return reference.rows_qkv(x, w, bias, norm, n_heads, positions, cos, sin,
                               k_cache, v_cache, slot_mapping)
 

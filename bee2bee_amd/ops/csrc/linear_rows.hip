@@ -15,6 +15,13 @@
 //    one left operand, 8 input rows at both places as the other; the two
 //    diagonal quarters of the product add up. Twice the workgroups where 16
 //    columns each leave CUs without one, and better pieces to load elsewhere.
+//  * Between two layers' projections the residual sum stays in fp32: the norm
+//    after an add takes the sum before it is rounded, as the kernel that adds
+//    and norms does. For an RMS norm the projection that adds leaves the sum
+//    times the norm's weight, in bf16, and sums of squares (Sum, LR_SCALED):
+//    reading fp32 rows instead cost 24 us of a step of 8 layers of 4096, one
+//    row (965 to 989). The error of such a step against 64 bits went from
+//    0.010 to 0.0053 of its norm. A layer norm reads the fp32 rows.
 //  * RMS norm: the columns enter as bf16(x w), the sum of squares is taken on
 //    the way and 1/rms multiplies the fp32 sum: one rounding, as if the normed
 //    row had been written and read. Layer norm needs mean and deviation first:
@@ -37,7 +44,8 @@ typedef __attribute__((ext_vector_type(4))) short short4v;
 constexpr int LR_U = 4;     // weight tiles of a batch of loads
 
 enum { LR_PLAIN = 0, LR_GLU = 1, LR_GELU = 2, LR_QKV = 3 };
-enum { LR_NONE = 0, LR_RMS = 1, LR_LAYER = 2 };
+// LR_SCALED: RMS norm of rows that come as what Sum below makes of them
+enum { LR_NONE = 0, LR_RMS = 1, LR_LAYER = 2, LR_SCALED = 3 };
 
 // What an LR_QKV epilogue reads and writes besides the rows: queries rotated
 // into q [M, nq, hd]; keys rotated, and values, into the pages (bf16 or fp8).
@@ -50,6 +58,29 @@ struct QkvStore {
     void* v_cache;
     int nq, nkv, hd, bs, fp8;
 };
+
+// What an LR_PLAIN epilogue adds, and what it leaves of the sum: bf16 or fp32
+// rows, and for the RMS norm that reads them next (then_w its weight) the rows
+// times that weight and the sums of squares of 8 columns each.
+struct Sum {
+    const void* resid;            // [M, N] bf16 or fp32, or null
+    int resid32, y32;
+    const unsigned short* then_w; // [N], or null
+    unsigned short* scaled;       // [M, N]
+    float* squares;               // [M, N / 8]
+};
+
+DEV_INLINE void load_x8(const unsigned short* p, float* v) {
+    load_bf16x8(p, v);
+}
+DEV_INLINE void load_x8(const float* p, float* v) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const f32x4 u = reinterpret_cast<const f32x4*>(p)[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[q * 4 + e] = u[e];
+    }
+}
 
 DEV_INLINE void store_row4(void* cache, long at, int fp8, const float* z) {
     if (fp8) {
@@ -70,15 +101,17 @@ DEV_INLINE void store_row4(void* cache, long at, int fp8, const float* z) {
 // LR_QKV: see QkvStore (W [N, K], bias optional). NT tiles of 16 columns of y
 // per workgroup (LR_GLU, LR_QKV: of each half; LR_QKV's halves are those of a
 // head).
-template <int NW, int NT, int TC, int G, int NORM, int EPI>
+// x is of type XT: bf16, or (LR_LAYER) fp32. squares: of LR_SCALED's rows.
+template <int NW, int NT, int TC, int G, int NORM, int EPI, typename XT>
 __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
-    const unsigned short* __restrict__ x,
+    const XT* __restrict__ x,
     const unsigned short* __restrict__ norm_w,
     const unsigned short* __restrict__ norm_b,
     const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias,
-    const unsigned short* __restrict__ resid, unsigned short* __restrict__ y,
-    int M, int N, int K, float eps, QkvStore st) {
+    const float* __restrict__ squares, Sum add,
+    unsigned short* __restrict__ y, int M, int N, int K, float eps,
+    QkvStore st) {
     constexpr bool PAIR = EPI == LR_GLU || EPI == LR_QKV;
     constexpr int WT = PAIR ? 2 * NT : NT;
     constexpr int H = TC == 16 ? G : 1;        // tiles of W along K a step
@@ -131,7 +164,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
             float sum = 0.f, sumsq = 0.f;
             for (int i = lane * 8; i < K; i += 512) {
                 float v[8];
-                load_bf16x8(x + (long)m * K + i, v);
+                load_x8(x + (long)m * K + i, v);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     sum += v[e];
@@ -168,24 +201,27 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const long k = (long)st_ * KS + (TC == 16 ? g * 32 : 0);
-            if (NORM != LR_NONE && (g == 0 || TC == 16))
+            if ((NORM == LR_RMS || NORM == LR_LAYER) && (g == 0 || TC == 16))
                 nw = *reinterpret_cast<const bf16x8*>(norm_w + lk + k);
             if (NORM == LR_LAYER && (g == 0 || TC == 16))
                 nb = *reinterpret_cast<const bf16x8*>(norm_b + lk + k);
-            bf16x8 bx = *reinterpret_cast<const bf16x8*>(x + x_off[g] + k);
-            if (NORM == LR_RMS) {
+            bf16x8 bx;
+            if (NORM == LR_NONE || NORM == LR_SCALED) {
+                bx = *reinterpret_cast<const bf16x8*>(x + x_off[g] + k);
+            } else {
+                float v[8];
+                load_x8(x + x_off[g] + k, v);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float v = (float)bx[e];
-                    sq[g] = fmaf(v, v, sq[g]);
-                    bx[e] = (__bf16)(v * (float)nw[e]);
+                    if (NORM == LR_RMS) {
+                        sq[g] = fmaf(v[e], v[e], sq[g]);
+                        bx[e] = (__bf16)(v[e] * (float)nw[e]);
+                    } else {
+                        bx[e] = (__bf16)((v[e] - mean[g]) * dev[g] *
+                                             (float)nw[e] +
+                                         (float)nb[e]);
+                    }
                 }
-            } else if (NORM == LR_LAYER) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    bx[e] = (__bf16)(((float)bx[e] - mean[g]) * dev[g] *
-                                         (float)nw[e] +
-                                     (float)nb[e]);
             }
 #pragma unroll
             for (int t = 0; t < WT; ++t)
@@ -215,6 +251,30 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
                 a[h][t] = *reinterpret_cast<const bf16x8*>(
                     wp[t] + (long)s * KS + h * 32);
         products(a, s);
+    }
+
+    // LR_SCALED: 1/rms, a wave a row (at one row a shorter chain than 16
+    // lanes: 3072x2048 6.4 us, not 6.8) or, of more rows than waves, 16 lanes.
+    // (Before the loop it keeps the first wave from its weights: 2x14336x4096,
+    // one row, 46.9 us, not 45.7.)
+    __shared__ float scale_s[16];
+    if (NORM == LR_SCALED) {
+        const bool wide = M <= NW;
+        const int m = wide ? wid : wid * 4 + lg;
+        float sum = 0.f;
+        if (m < M) {
+            const float* sp = squares + (long)m * (K / 8);
+#pragma unroll 4
+            for (int i = (wide ? lane : li) * 4; i < K / 8;
+                 i += wide ? 256 : 64) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(sp + i);
+                sum += (v[0] + v[1]) + (v[2] + v[3]);
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o);
+        if (wide) sum = rows_sum(sum);
+        if (m < M && li == 0) scale_s[m] = rsqrtf(sum / (float)K + eps);
     }
 
     // ---- the waves' sums; C layout: column li = row of x, rows lg * 4 + r =
@@ -249,6 +309,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         }
         inv = rsqrtf(v / (float)K + eps);
     }
+    if (NORM == LR_SCALED) inv = scale_s[m];
     auto total = [&](int t, float* z) {
         f32x4 v = part[0][g][t][lane];
 #pragma unroll
@@ -314,20 +375,57 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         store_row4(cache, at + half, st.fp8, u);
         return;
     } else {
+        const long at = (long)m * N + n;
+        if (EPI == LR_PLAIN && add.resid32 && N % 4 == 0) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(
+                reinterpret_cast<const float*>(add.resid) + at);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool in = n + r < N;
-            if (bias && in) z[r] += bf2f(bias[n + r]);
-            if (EPI == LR_GELU) {
-                const float c = 0.7978845608028654f *
-                                (z[r] + 0.044715f * z[r] * z[r] * z[r]);
-                z[r] = 0.5f * z[r] * (1.f + tanhf(c));
+            for (int r = 0; r < 4; ++r) {
+                if (bias) z[r] += bf2f(bias[n + r]);
+                z[r] += v[r];
             }
-            if (resid && in) z[r] += bf2f(resid[(long)m * N + n + r]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bool in = n + r < N;
+                if (bias && in) z[r] += bf2f(bias[n + r]);
+                if (EPI == LR_GELU) {
+                    const float c = 0.7978845608028654f *
+                                    (z[r] + 0.044715f * z[r] * z[r] * z[r]);
+                    z[r] = 0.5f * z[r] * (1.f + tanhf(c));
+                }
+                if (add.resid && in)
+                    z[r] += add.resid32
+                                ? reinterpret_cast<const float*>(
+                                      add.resid)[at + r]
+                                : bf2f(reinterpret_cast<const unsigned short*>(
+                                      add.resid)[at + r]);
+            }
         }
     }
     const long at = (long)m * N + n;
-    if (N % 4 == 0) {
+    if (EPI == LR_PLAIN && add.then_w) {       // (N % 8 == 0)
+        const short4v tw = *reinterpret_cast<const short4v*>(add.then_w + n);
+        float v[4], sq4 = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] = z[r] * bf2f((unsigned short)tw[r]);
+            sq4 += z[r] * z[r];
+        }
+        store_row4(add.scaled, at, 0, v);
+        sq4 += __shfl_xor(sq4, 16);            // the next 4 columns'
+        if (lg % 2 == 0) add.squares[(long)m * (N / 8) + n / 8] = sq4;
+    }
+    if (EPI == LR_PLAIN && add.y32) {
+        float* y32 = reinterpret_cast<float*>(y) + at;
+        if (N % 4 == 0) {
+            *reinterpret_cast<f32x4*>(y32) = f32x4{z[0], z[1], z[2], z[3]};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) y32[r] = z[r];
+        }
+    } else if (N % 4 == 0) {
         store_row4(y, at, 0, z);
     } else {
 #pragma unroll
@@ -337,8 +435,10 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
 }
 
 // x [M, K] and w rows of K, 1 <= M <= 16, K % 32 == 0, all contiguous and
-// 16-byte aligned; norm 0 none, 1 RMS, 2 layer norm; epi as above (LR_GLU: N %
-// 16 == 0, LR_QKV: hd % 32 == 0). Nonzero for anything else.
+// 16-byte aligned; x32: x is fp32 (norm 2); norm 0 none, 1 RMS, 2 layer norm, 3
+// RMS with `squares` [M, K / 8]; epi as above (LR_GLU: N % 16 == 0, LR_QKV: hd %
+// 32 == 0); resid32, y32: the residual, and LR_PLAIN's y, are fp32; then_w: see
+// Sum (N % 8 == 0). Nonzero for anything else.
 //
 // The shape of a workgroup (waves x tiles x columns of a tile) depends on N and
 // K only, or on M between shapes of the same sums: 16 columns with G 2 add as 8
@@ -360,30 +460,44 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
 //    3584x18944 31 / 41 / 56, 29 / 34 / 44, 32 / 40 / 46;
 //   above: 128256x4096 8x2x8 174 / 204 / 272, 8x2x16 184 / 194 / 217.
 extern "C" int launch_linear_rows(
-    const unsigned short* x, const unsigned short* norm_w,
+    const void* x, int x32, const unsigned short* norm_w,
     const unsigned short* norm_b, const unsigned short* w,
-    const unsigned short* bias, const unsigned short* resid,
-    unsigned short* y, int M, int N, int K, float eps, int norm, int epi,
+    const unsigned short* bias, const float* squares, const void* resid,
+    int resid32, void* y, int y32, const unsigned short* then_w,
+    unsigned short* scaled, float* squares_out, int M, int N, int K,
+    float eps, int norm, int epi,
     const int* pos, const float* cos_t, const float* sin_t, const int* slots,
     void* k_cache, void* v_cache, int nq, int nkv, int hd, int bs, int fp8,
     hipStream_t stream) {
     if (M < 1 || M > 16 || N < 1 || K < 32 || K % 32) return 1;
     if (epi == LR_GLU && N % 16) return 1;
+    if ((x32 && norm != LR_LAYER) || (norm == LR_SCALED && !squares)) return 1;
+    if ((y32 || then_w) && epi != LR_PLAIN) return 1;
+    if (then_w && N % 8) return 1;
+    const Sum add{resid, resid32, y32, then_w, scaled, squares_out};
     if (epi == LR_QKV && (hd % 32 || N != (nq + 2 * nkv) * hd)) return 1;
     const QkvStore st{pos,     cos_t, sin_t, slots, k_cache,
                       v_cache, nq,    nkv,   hd,    bs, fp8};
 #define LR_COLS(NTV, TCV, EP) (NTV * TCV * (EP == LR_QKV ? 2 : 1))
-#define LR_GO(NWV, NTV, TCV, GV, NO, EP)                                      \
-    hipLaunchKernelGGL((linear_rows_kernel<NWV, NTV, TCV, GV, NO, EP>),       \
+#define LR_GO(NWV, NTV, TCV, GV, NO, EP, XT)                                  \
+    hipLaunchKernelGGL((linear_rows_kernel<NWV, NTV, TCV, GV, NO, EP, XT>),   \
                        dim3((N + LR_COLS(NTV, TCV, EP) - 1) /                 \
                             LR_COLS(NTV, TCV, EP)),                           \
-                       dim3(NWV * 64), 0, stream, x, norm_w, norm_b, w, bias, \
-                       resid, y, M, N, K, eps, st)
+                       dim3(NWV * 64), 0, stream, (const XT*)x, norm_w,       \
+                       norm_b, w, bias, squares, add, (unsigned short*)y, M,  \
+                       N, K, eps, st)
 #define LR_NORMS(NWV, NTV, TCV, GV, EP)                                       \
     do {                                                                      \
-        if (norm == LR_RMS) LR_GO(NWV, NTV, TCV, GV, LR_RMS, EP);             \
-        else if (norm == LR_LAYER) LR_GO(NWV, NTV, TCV, GV, LR_LAYER, EP);    \
-        else LR_GO(NWV, NTV, TCV, GV, LR_NONE, EP);                           \
+        if (norm == LR_SCALED)                                                \
+            LR_GO(NWV, NTV, TCV, GV, LR_SCALED, EP, unsigned short);          \
+        else if (norm == LR_RMS)                                              \
+            LR_GO(NWV, NTV, TCV, GV, LR_RMS, EP, unsigned short);             \
+        else if (norm == LR_LAYER && x32)                                     \
+            LR_GO(NWV, NTV, TCV, GV, LR_LAYER, EP, float);                    \
+        else if (norm == LR_LAYER)                                            \
+            LR_GO(NWV, NTV, TCV, GV, LR_LAYER, EP, unsigned short);           \
+        else                                                                  \
+            LR_GO(NWV, NTV, TCV, GV, LR_NONE, EP, unsigned short);            \
     } while (0)
 #define LR_16(NWV, NTV, EP) LR_NORMS(NWV, NTV, 16, 1, EP)
 #define LR_8(NWV, NTV, EP)                                                    \

@@ -8,11 +8,11 @@ using torch::Tensor;
 using c10::optional;
 
 extern "C" int launch_linear_rows(
-    const unsigned short*, const unsigned short*, const unsigned short*,
-    const unsigned short*, const unsigned short*, const unsigned short*,
-    unsigned short*, int, int, int, float, int, int, const int*, const float*,
-    const float*, const int*, void*, void*, int, int, int, int, int,
-    hipStream_t);
+    const void*, int, const unsigned short*, const unsigned short*,
+    const unsigned short*, const unsigned short*, const float*, const void*,
+    int, void*, int, const unsigned short*, unsigned short*, float*, int, int,
+    int, float, int, int, const int*, const float*, const float*, const int*,
+    void*, void*, int, int, int, int, int, hipStream_t);
 extern "C" int linear_mid_splits(int, int);
 extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
                                  float*, int, int, int, int, hipStream_t);
@@ -40,10 +40,14 @@ hipStream_t stream() {
     return at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
 }
 
+bool is_f32(const Tensor& t) { return t.scalar_type() == torch::kFloat32; }
+
 // t as the kernel reads it: contiguous, 16-byte aligned (copied if it is not)
-Tensor dense(const Tensor& t, const char* name) {
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16, name,
-                " must be bf16 on the GPU");
+Tensor dense(const Tensor& t, const char* name, bool f32_too = false) {
+    TORCH_CHECK(t.is_cuda() && (t.scalar_type() == torch::kBFloat16 ||
+                                (f32_too && is_f32(t))),
+                name, f32_too ? " must be bf16 or fp32 on the GPU"
+                              : " must be bf16 on the GPU");
     if (t.is_contiguous() &&
         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0)
         return t;
@@ -63,13 +67,23 @@ const unsigned short* ptr(const Tensor& t) {
                : nullptr;
 }
 
+unsigned short* mut(Tensor& t) {
+    return reinterpret_cast<unsigned short*>(t.data_ptr());
+}
+
 struct Rows {
-    Tensor x, w, norm_w, norm_b;
+    Tensor x, w, norm_w, norm_b, squares;
     int M, N, K, norm;
+    const float* sq() const {
+        return squares.defined() ? squares.data_ptr<float>() : nullptr;
+    }
 };
 
+// norm_b given: layer norm; norm_w alone: RMS norm; squares: RMS norm of rows
+// that are multiplied by its weight already
 Rows rows_of(const Tensor& x, const Tensor& w, const optional<Tensor>& norm_w,
-             const optional<Tensor>& norm_b) {
+             const optional<Tensor>& norm_b,
+             const optional<Tensor>& squares) {
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
                 "x [M, K] and w [N, K]");
     Rows r;
@@ -79,48 +93,71 @@ Rows rows_of(const Tensor& x, const Tensor& w, const optional<Tensor>& norm_w,
     TORCH_CHECK(r.M >= 1 && r.M <= 16, "1 to 16 rows");
     TORCH_CHECK(r.K % 32 == 0, "K must be a multiple of 32");
     TORCH_CHECK(norm_w.has_value() || !norm_b.has_value());
-    r.x = dense(x, "x");
+    r.x = dense(x, "x", norm_b.has_value());
     r.w = dense(w, "w");
     r.norm_w = column(norm_w, r.K, "norm weight");
     r.norm_b = column(norm_b, r.K, "norm bias");
     r.norm = !norm_w.has_value() ? 0 : norm_b.has_value() ? 2 : 1;
+    if (squares.has_value()) {
+        TORCH_CHECK(r.norm == 0 && squares->is_cuda() && is_f32(*squares) &&
+                    squares->dim() == 2 && squares->size(0) == r.M &&
+                    squares->size(1) == r.K / 8 && squares->is_contiguous(),
+                    "squares [M, K / 8] fp32, in the norm's place");
+        r.squares = *squares;
+        r.norm = 3;
+    }
     return r;
 }
 
-// norm_b given: layer norm; norm_w alone: RMS norm
-Tensor rows_linear(const Tensor& x, const Tensor& w,
-                   const optional<Tensor>& bias,
-                   const optional<Tensor>& resid,
-                   const optional<Tensor>& norm_w,
-                   const optional<Tensor>& norm_b, double eps, int64_t act) {
-    const Rows r = rows_of(x, w, norm_w, norm_b);
+// x of a layer norm, and resid, may be fp32; keep32: so is the result. then_w,
+// the weight of the RMS norm that reads the result: -> also the result times it,
+// and the sums of squares of 8 columns each
+std::vector<Tensor> rows_linear(
+    const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
+    const optional<Tensor>& resid, const optional<Tensor>& norm_w,
+    const optional<Tensor>& norm_b, const optional<Tensor>& squares,
+    double eps, int64_t act, bool keep32, const optional<Tensor>& then_w) {
+    const Rows r = rows_of(x, w, norm_w, norm_b, squares);
     TORCH_CHECK(act == EPI_PLAIN || act == EPI_GLU || act == EPI_GELU);
     TORCH_CHECK(act != EPI_GLU || (r.N % 32 == 0 && !bias.has_value()));
-    TORCH_CHECK(act == EPI_PLAIN || !resid.has_value());
+    TORCH_CHECK(act == EPI_PLAIN ||
+                !(resid.has_value() || keep32 || then_w.has_value()));
     const int N = act == EPI_GLU ? r.N / 2 : r.N;
     if (resid.has_value())
         TORCH_CHECK(resid->dim() == 2 && resid->size(0) == r.M &&
                     resid->size(1) == N, "resid [M, N]");
     const Tensor b = column(bias, N, "bias");
-    const Tensor add = resid.has_value() ? dense(*resid, "resid") : Tensor();
-    Tensor y = torch::empty({r.M, N}, x.options());
+    const Tensor add =
+        resid.has_value() ? dense(*resid, "resid", true) : Tensor();
+    const auto bf16 = r.w.options();
+    const auto f32 = bf16.dtype(torch::kFloat32);
+    std::vector<Tensor> out{torch::empty({r.M, N}, keep32 ? f32 : bf16)};
+    const Tensor tw = column(then_w, N, "the next norm's weight");
+    if (tw.defined()) {
+        TORCH_CHECK(N % 8 == 0);
+        out.push_back(torch::empty({r.M, N}, bf16));
+        out.push_back(torch::empty({r.M, N / 8}, f32));
+    }
     TORCH_CHECK(launch_linear_rows(
-                    ptr(r.x), ptr(r.norm_w), ptr(r.norm_b), ptr(r.w), ptr(b),
-                    ptr(add),
-                    reinterpret_cast<unsigned short*>(y.data_ptr()), r.M, N,
+                    r.x.data_ptr(), is_f32(r.x), ptr(r.norm_w),
+                    ptr(r.norm_b), ptr(r.w), ptr(b), r.sq(),
+                    add.defined() ? add.data_ptr() : nullptr,
+                    add.defined() && is_f32(add), out[0].data_ptr(), keep32,
+                    ptr(tw), tw.defined() ? mut(out[1]) : nullptr,
+                    tw.defined() ? out[2].data_ptr<float>() : nullptr, r.M, N,
                     r.K, (float)eps, r.norm, (int)act, nullptr, nullptr,
                     nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0,
                     stream()) == 0);
-    return y;
+    return out;
 }
 
 // -> rotated queries [M, nq, hd]; rotated keys and the values go to the pages
 Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
-                const Tensor& norm_w, const optional<Tensor>& norm_b,
-                double eps, int64_t nq, const optional<Tensor>& pos,
+                const optional<Tensor>& norm_w, const optional<Tensor>& norm_b,
+                const optional<Tensor>& squares, double eps, int64_t nq, const optional<Tensor>& pos,
                 const optional<Tensor>& cos_t, const optional<Tensor>& sin_t,
                 Tensor& k_cache, Tensor& v_cache, const Tensor& slots) {
-    const Rows r = rows_of(x, w, norm_w, norm_b);
+    const Rows r = rows_of(x, w, norm_w, norm_b, squares);
     const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
     TORCH_CHECK(k_cache.dim() == 4 && k_cache.sizes() == v_cache.sizes() &&
                 k_cache.scalar_type() == v_cache.scalar_type() &&
@@ -139,21 +176,17 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
                         t->is_contiguous() && t->size(1) == hd / 2);
     }
     const Tensor b = column(bias, r.N, "bias");
-    Tensor q = torch::empty({r.M, nq, hd}, x.options());
+    Tensor q = torch::empty({r.M, nq, hd}, r.w.options());
     TORCH_CHECK(launch_linear_rows(
-                    ptr(r.x), ptr(r.norm_w), ptr(r.norm_b), ptr(r.w), ptr(b),
-                    nullptr, reinterpret_cast<unsigned short*>(q.data_ptr()),
-                    r.M, r.N, r.K, (float)eps, r.norm, EPI_QKV,
+                    r.x.data_ptr(), is_f32(r.x), ptr(r.norm_w),
+                    ptr(r.norm_b), ptr(r.w), ptr(b), r.sq(), nullptr, 0,
+                    q.data_ptr(), 0, nullptr, nullptr, nullptr, r.M, r.N, r.K, (float)eps, r.norm, EPI_QKV,
                     pos.has_value() ? pos->data_ptr<int>() : nullptr,
                     pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
                     pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
                     slots.data_ptr<int>(), k_cache.data_ptr(),
                     v_cache.data_ptr(), nq, nkv, hd, bs, fp8, stream()) == 0);
     return q;
-}
-
-unsigned short* mut(Tensor& t) {
-    return reinterpret_cast<unsigned short*>(t.data_ptr());
 }
 
 // parts [S, M, N] fp32, whose sum over S is x w^T

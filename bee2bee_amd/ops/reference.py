@@ -293,15 +293,27 @@ def grouped_gemm(
     return out
 
 
-def rows_linear(x, w, bias=None, resid=None, norm=None, act=None):
-    """act(norm(x) w^T + bias) + resid; norm (weight, bias or None, eps)."""
-    if norm is not None:
+def rows_linear(x, w, bias=None, resid=None, norm=None, act=None,
+                keep32=False, then=None):
+    """act(norm(x) w^T + bias) + resid; norm (weight, bias or None, eps), or
+    (squares, eps) for rows that `then` made."""
+    if norm is not None and len(norm) == 2:
+        x = x.float() * torch.rsqrt(
+            norm[0].sum(-1, keepdim=True) / x.shape[1] + norm[1])
+    elif norm is not None:
         x = (rmsnorm(x, norm[0], norm[2]) if norm[1] is None
              else layernorm(x, *norm))
-    y = torch.nn.functional.linear(x, w, bias)
+    y = torch.nn.functional.linear(x.to(w.dtype), w, bias)
     if act is not None:
         y = gelu(y) if act == "gelu" else swiglu(y)
-    return y if resid is None else (y.float() + resid.float()).to(x.dtype)
+    if resid is not None:
+        y = y.float() + resid.float()
+    out = y.float() if keep32 else y.to(w.dtype)
+    if then is None:
+        return out
+    y = y.float()
+    return (out, (y * then.float()).to(w.dtype),
+            y.square().view(y.shape[0], -1, 8).sum(-1))
 
 
 def rows_qkv(x, w, bias, norm, n_heads, positions, cos, sin, k_cache, v_cache,

@@ -1,0 +1,162 @@
+"""Steps of dense stacks at the row counts where the Runner changes its route
+(few rows, some tens, deep down projections, more), against the same steps in
+fp32 on the CPU.
+
+Tolerance: a layer rounds about eight tensors to bf16 (2^-9 relative at most,
+independent of each other) and adds their effects to a residual that is rounded
+once or twice; two layers and the head stay below 1% of the result's norm, and
+1.5% is asked for. 8-bit pages round keys, values and, in decoding, queries
+to 3 mantissa bits (2^-4 at most) on top: 5%."""
+import pytest
+import torch
+
+from bee2bee_amd.engine.graphs import decode_slot_mapping
+from bee2bee_amd.engine.kv import PagedKV
+from bee2bee_amd.engine.runner import Runner
+from bee2bee_amd.models.spec import ModelSpec
+from bee2bee_amd.models.weights import ModelWeights
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
+DEV, CPU = torch.device("cuda:0"), torch.device("cpu")
+SWIGLU = ModelSpec(name="t-swiglu", vocab_size=500, hidden_size=256,
+                   intermediate_size=1024, n_layers=2, n_heads=4, n_kv_heads=2,
+                   head_dim=64, max_seq_len=1024, qkv_bias=True)
+GELU = ModelSpec(name="t-gelu", vocab_size=500, hidden_size=256,
+                 intermediate_size=1024, n_layers=2, n_heads=4, n_kv_heads=4,
+                 head_dim=64, max_seq_len=1024, qkv_bias=True, arch="gpt2",
+                 norm_type="layernorm", act_type="gelu", pos_type="learned",
+                 attn_out_bias=True, mlp_bias=True)
+
+
+def _tensors(holder):
+    names = getattr(holder, "__slots__", None) or list(vars(holder))
+    pairs = [(n, getattr(holder, n, None)) for n in names]
+    return [(n, t) for n, t in pairs if isinstance(t, torch.Tensor)]
+
+
+def _weights(spec):
+    """The same random weights, biases and norms on GPU and CPU."""
+    W = ModelWeights(spec, CPU, torch.float32).random_init(seed=3)
+    g = torch.Generator().manual_seed(4)
+    W.embed.normal_(0.0, 1.0, generator=g)
+    for holder in [W, *W.layers]:
+        for name, t in _tensors(holder):
+            if name == "embed":
+                continue
+            if name.endswith("bias"):
+                t.normal_(0.0, 0.5, generator=g)
+            elif name.endswith("norm"):
+                t.normal_(1.0, 0.2, generator=g)
+            elif t.dim() == 2:
+                t.normal_(0.0, t.shape[1] ** -0.5, generator=g)
+    G = ModelWeights(spec, DEV, torch.bfloat16).random_init(seed=3)
+    for a, b in zip([W, *W.layers], [G, *G.layers]):
+        for name, t in _tensors(a):
+            t.copy_(t.bfloat16())
+            getattr(b, name).copy_(t)
+    return W, G
+
+
+class _Side:
+    """A stack with its pages on one device."""
+
+    def __init__(self, spec, weights, device, dtype, kv_dtype):
+        self.kv = PagedKV(spec, device, dtype, n_blocks=600, block_size=16,
+                          kv_dtype=kv_dtype)
+        self.runner = Runner(spec, weights, self.kv, device, dtype)
+        self.device, self.seqs = device, 0
+
+    def ints(self, x):
+        return torch.tensor(x, dtype=torch.int32, device=self.device)
+
+    def prompt(self, ids, lens, old=None):
+        """ids of new sequences of these lengths, or, with `old`, the next
+        portions of the last ones."""
+        chunked = old is not None
+        if not chunked:
+            old = [0] * len(lens)
+            self.rows = list(range(self.seqs, self.seqs + len(lens)))
+            self.seqs += len(lens)
+            for s in self.rows:
+                self.kv.new_seq(s)
+        pos, slots, cu = [], [], [0]
+        for s, n, o in zip(self.rows, lens, old):
+            self.kv.extend_seq(s, o + n)
+            pos += range(o, o + n)
+            slots += self.kv.slot_mapping(s, range(o, o + n))
+            cu.append(cu[-1] + n)
+        more = {}
+        if chunked:
+            more = {"block_table": self.kv.block_table(self.rows),
+                    "seq_lens": self.ints([o + n for o, n in zip(old, lens)]),
+                    "query_lens": self.ints(lens)}
+        return self.runner.forward_prefill(
+            ids.to(self.device), self.ints(pos), self.ints(slots),
+            self.ints(cu), max(lens), **more)
+
+    def decode(self, ids, n):
+        """One token for each of the last sequences, which hold n."""
+        for s in self.rows:
+            self.kv.extend_seq(s, n + 1)
+        table = self.kv.block_table(self.rows)
+        pos = self.ints([n] * len(self.rows))
+        return self.runner.forward_decode(
+            ids.to(self.device), pos,
+            decode_slot_mapping(table, pos, 16), table, pos + 1)
+
+
+def _rel(got, want):
+    got, want = got.double().cpu(), want.double().cpu()
+    return ((got - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("kv_dtype", ["native", "fp8"])
+@pytest.mark.parametrize("spec", [SWIGLU, GELU], ids=lambda s: s.name)
+@pytest.mark.parametrize("rows", [1, 9, 16, 17, 160, 161, 256, 257])
+@torch.no_grad()
+def test_steps(spec, rows, kv_dtype):
+    W, G = _weights(spec)
+    gpu = _Side(spec, G, DEV, torch.bfloat16, kv_dtype)
+    cpu = _Side(spec, W, CPU, torch.float32, kv_dtype)
+    g = torch.Generator().manual_seed(rows)
+    ids = lambda n: torch.randint(0, 500, (n,), generator=g)
+    lens = [n for n in (rows - rows // 3 - rows // 5, rows // 3, rows // 5)
+            if n]
+    steps = [("prompts", "prompt", ids(rows), lens),
+             ("histories", "prompt", ids(3 * rows), [3] * rows),
+             ("decode", "decode", ids(rows), 3),
+             ("history", "prompt", ids(40), [40]),
+             ("portion", "prompt", ids(rows), [rows], [40])]
+    for name, call, *args in steps:
+        got, want = (getattr(side, call)(*args) for side in (gpu, cpu))
+        limit = 0.015 if kv_dtype == "native" else 0.05
+        assert _rel(got, want) <= limit, (name, _rel(got, want))
+        last = slice(-min(rows, 20), None)
+        got, want = gpu.runner.lm_head(got[last]), cpu.runner.lm_head(
+            want[last])
+        assert _rel(got, want) <= limit, (name, _rel(got, want))
+
+
+@pytest.mark.parametrize("rows", [1, 9, 17])
+@torch.no_grad()
+def test_norms_see_the_unrounded_residual(rows):
+    """Where the residual stands at 256, a bf16 one moves in steps of 2: the
+    norm after a sum takes it before it is rounded."""
+    spec = GELU
+    W, G = _weights(spec)
+    for w in (W, G):
+        w.embed.fill_(256.0)
+        w.pos_embed.zero_()
+        for lw in w.layers:
+            lw.wo.zero_()
+            lw.w_down.copy_(100 * lw.w_down)
+    gpu = _Side(spec, G, DEV, torch.bfloat16, "native")
+    cpu = _Side(spec, W, CPU, torch.float32, "native")
+    ids = torch.arange(rows) % 7
+    got, want = (s.prompt(ids, [rows]) for s in (gpu, cpu))
+    # the first layer's norm of 256 + bias, through gelu and 100 w_down
+    assert _rel(got, want) <= 0.015, _rel(got, want)

@@ -148,6 +148,41 @@ def test_qkv(M, nq, nkv, hd, K, kind, fp8):
         assert (rest == 0).all()
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(64, 32), (2048, 576), (2080, 192),
+                                 (4104, 96), (4128, 64)])
+def test_sum_and_next_norm(M, N, K):
+    """The residual sum in fp32 and what the next RMS norm's projection takes
+    of it, through that projection; and a layer norm of fp32 rows. Their norm
+    stands at 256: rounded to bf16, rows would move in steps of 2."""
+    torch.manual_seed(M + N)
+    x, w, b = _rand(M, K), _rand(N, K, std=0.05), _rand(N)
+    resid = 256 + torch.randn(M, N, device=DEV)
+    then = _rand(N, std=0.1, mean=1.0)
+    total, scaled, squares = ops.rows_linear(x, w, b, resid, keep32=True,
+                                             then=then)
+    want = x.double() @ w.double().t() + b.double() + resid.double()
+    # fp32 sums of K exact products, and of values near 256
+    assert ((total.double() - want).abs() <= 2 ** -23 * (K + 300)).all()
+    t32 = total * then.float()
+    assert ((scaled.float() - t32).abs() <= 2 ** -8 * t32.abs()).all()
+    eights = total.double().square().view(M, -1, 8).sum(-1)
+    assert ((squares.double() - eights).abs() <= 2 ** -21 * eights).all()
+    if N % 32:
+        return
+    w2 = _rand(80, N, std=0.05)
+    for norm in ((then, None, 1e-5), (then, b, 1e-5)):
+        y, mag = _products(total, w2, norm)
+        args = (scaled, w2), {"norm": (squares, 1e-5)}
+        if norm[1] is not None:
+            args = (total, w2), {"norm": norm}
+            # mean and deviation of values near 256 from sums of fp32 squares:
+            # 2^-24 of 2^16, a few times, of a variance near 1
+            mag = mag * 1.5 + 2 ** -5 * y.abs()
+        got = ops.rows_linear(*args[0], **args[1]).float()
+        assert ((got - y).abs() <= 2 ** -8 * (mag + y.abs()) + 1e-5).all()
+
+
 def test_a_row_does_not_depend_on_the_others():
     torch.manual_seed(0)
     x, w, norm = _rand(16, 4096), _rand(6144, 4096, std=0.02), \
@@ -164,6 +199,10 @@ def test_refused():
         ops.rows_linear(x, w)
     with pytest.raises(RuntimeError):
         ops.rows_linear(x[:4, :40].contiguous(), w[:, :40].contiguous())
+    with pytest.raises(RuntimeError):       # fp32 rows without a layer norm
+        ops.rows_linear(x[:4].float(), w)
+    with pytest.raises(RuntimeError):       # squares of other rows
+        ops.rows_linear(x[:4], w, norm=(torch.ones(4, 4, device=DEV), 1e-5))
 
 
 # ------------------------------------------------- steps of some tens of rows
