@@ -306,6 +306,12 @@ class InferenceEngine:
         self.graphs: Optional[DecodeGraphs] = None
         if self.use_graphs:
             self.graphs = DecodeGraphs(self.runner, max_batch, blocks_per_seq)
+        # positions that the rotation or position table and, in captured
+        # steps, the block table have: a sequence that fills them is done
+        self._positions = self.spec.max_seq_len
+        if self.graphs is not None:
+            self._positions = min(self._positions,
+                                  blocks_per_seq * block_size)
         # scratch sequence backing pad rows of graph-bucket batches
         self._scratch_seq = -1
         self.kv.new_seq(self._scratch_seq)
@@ -366,6 +372,13 @@ class InferenceEngine:
         # empty prompts become [bos] at admission (engine loop); <1
         # max_new behaves as 1 (prefill completion always emits one token)
         req.max_new_tokens = max(1, int(req.max_new_tokens))
+        # ids past the vocabulary would be read from past the embedding, in
+        # a step that other requests share
+        if req.prompt_ids and not (
+                0 <= min(req.prompt_ids)
+                and max(req.prompt_ids) < self.spec.vocab_size):
+            raise ValueError("prompt_ids outside the vocabulary of "
+                             f"{self.spec.vocab_size}")
         self.start()
         self._pending.put(req)
         self._wake.set()
@@ -607,6 +620,7 @@ class InferenceEngine:
                     a.req.admitted_ts = now_admit
                 p = a.req.prompt_ids or [self.spec.bos_token_id]
                 p = p[: self.max_seq_len - a.req.max_new_tokens - 1] or p[:1]
+                p = p[: max(1, self._positions - 1)]
                 a.req.prompt_ids = p
             take = min(len(a.req.prompt_ids) - a.prefilled, budget)
             batch.append((a, a.prefilled, take))
@@ -1006,7 +1020,7 @@ class InferenceEngine:
             # keys get overwritten; attention never reads past seq_len)
             a.length += len(emitted)
             self.kv.extend_seq(a.seq_id, a.length)
-            for tok in emitted:
+            for j, tok in enumerate(emitted):
                 if r.done_ts is not None:
                     break
                 if r.first_token_ts is None:
@@ -1017,7 +1031,9 @@ class InferenceEngine:
                     pen_new_toks.append(tok)
                 n_emitted += 1
                 done = (r.cancelled or tok in r.stop_token_ids
-                        or len(r.output_ids) >= r.max_new_tokens)
+                        or len(r.output_ids) >= r.max_new_tokens
+                        or (j + 1 == len(emitted)
+                            and a.length >= self._positions))
                 if done:
                     r.done_ts = now
                 if r.on_emit is not None:
@@ -1185,7 +1201,8 @@ class InferenceEngine:
             r.output_ids.append(tok)
             n_emitted += 1
             done = (r.cancelled or tok in r.stop_token_ids
-                    or len(r.output_ids) >= r.max_new_tokens)
+                    or len(r.output_ids) >= r.max_new_tokens
+                    or a.length >= self._positions)
             if done:
                 r.done_ts = now
             if r.on_emit is not None:

@@ -438,3 +438,37 @@ def test_kv_pressure_queues_and_completes_all():
         assert eng.kv.free_blocks >= total - 1
     finally:
         eng.shutdown()
+
+
+@pytest.mark.parametrize("ids", [(1, 512), (-1, 2), (1 << 40,)])
+def test_ids_outside_the_vocabulary_are_refused(small_engine, ids):
+    """Before they share a step with other requests."""
+    beside = small_engine.submit(_req(6, (7, 8)))
+    with pytest.raises(ValueError):
+        small_engine.submit(_req(4, ids))
+    _drain(beside)
+    assert beside.error is None and len(beside.output_ids) == 6
+
+
+@pytest.mark.parametrize("spec_decode", [False, True])
+def test_a_sequence_that_fills_the_positions_is_done(spec_decode):
+    """It ends there, and the requests beside it go on."""
+    import dataclasses
+
+    from bee2bee_amd.models.spec import PRESETS
+
+    spec = dataclasses.replace(PRESETS["tiny"], max_seq_len=40)
+    eng = InferenceEngine(spec, device="cpu", max_batch=3, max_seq_len=40,
+                          seed=5, spec_decode=spec_decode)
+    try:
+        endless = eng.submit(_req(0, (1, 2, 3), max_new=1000))
+        long = eng.submit(_req(0, tuple(range(1, 300)) * 8, max_new=1000))
+        beside = eng.submit(_req(0, (9, 8, 7, 9, 8, 7), max_new=30))
+        for r in (endless, long, beside):
+            _drain(r)
+            assert r.error is None
+        assert len(endless.prompt_ids) + len(endless.output_ids) == 41
+        assert len(long.prompt_ids) + len(long.output_ids) == 41
+        assert len(beside.output_ids) == 30
+    finally:
+        eng.shutdown()
