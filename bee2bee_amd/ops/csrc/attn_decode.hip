@@ -55,7 +55,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_scores_kernel(
     int nkv, int W, int bs, int hd, int C, long q_stride, float scale) {
     const int b = blockIdx.x;
     const int kvh = blockIdx.y;
-    const int L = seq_lens[b];
+    const int L = min(seq_lens[b], W * bs);    // (what its pages hold)
     if ((int)blockIdx.z * DEC_CHUNK >= L) return;
     const int lane = threadIdx.x % WAVE;
     const int wid = threadIdx.x / WAVE;
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_pv_kernel(
     int nkv, int W, int bs, int hd, int C) {
     const int b = blockIdx.x;
     const int kvh = blockIdx.y;
-    const int L = seq_lens[b];
+    const int L = min(seq_lens[b], W * bs);    // (what its pages hold)
     if ((int)blockIdx.z * DEC_CHUNK >= L) return;
     const int lane = threadIdx.x % WAVE;
     const int wid = threadIdx.x / WAVE;
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_decode_combine_kernel(
     const int g = blockIdx.z;  // one block per (seq, kv head, q head)
     const int nq = nkv * G;
     const int L = seq_lens[b];
-    const int nc = (L + DEC_CHUNK - 1) / DEC_CHUNK;
+    const int nc = min((L + DEC_CHUNK - 1) / DEC_CHUNK, C);
     const long base = ((long)b * nkv + kvh) * C;
 
     // stage this head's (m, l) pairs once

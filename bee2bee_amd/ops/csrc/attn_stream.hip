@@ -101,7 +101,7 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     // a chunk longer than the caller said has no room in the workspaces
     const int live = min(rows, max_rows);
     if (row0 >= live) return;
-    const int L = seq_lens[b];
+    const int L = min(seq_lens[b], W * bs);    // (what its pages hold)
     const int hist = L - rows / G;
     const int per = split_keys(L, even, most);
     const bool split = L > per;          // or the result itself is written
@@ -369,16 +369,16 @@ __global__ __launch_bounds__(HD / 4 * P) void attn_stream_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
     const int* __restrict__ cu, const int* __restrict__ seq_lens,
     unsigned short* __restrict__ out, float* __restrict__ out_ml, int nkv,
-    int G, int Z, int even, int most, int max_rows) {
+    int G, int pages, int Z, int even, int most, int max_rows) {
     constexpr int C = HD / 4;                  // threads of a split
     const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
     const int s0 = cu ? cu[b] : b;
     const int row = blockIdx.y;
     if (row >= (cu ? cu[b + 1] - s0 : 1) * G) return;
-    const int L = seq_lens[b];
+    const int L = min(seq_lens[b], pages);
     const int per = split_keys(L, even, most);
     if (L <= per) return;                      // written by its workgroup
-    const int nz = min((L + per - 1) / per, Z);
+    const int nz = (L + per - 1) / per;
     const long p0 = (long)blockIdx.x * Z * max_rows + row;
     const int lane = threadIdx.x & 63, c = threadIdx.x % C;
     const int z0 = threadIdx.x / C;            // 0 .. P - 1
@@ -513,7 +513,7 @@ extern "C" int launch_attn_stream(
     hipLaunchKernelGGL((attn_stream_combine_kernel<HDV, P, I>),               \
                        dim3(nseq * nkv, max_rows), dim3(HDV / 4 * (P)), 0,    \
                        stream, part_o, part_ml, cu, seq_lens, out, out_ml,    \
-                       nkv, G, Z, even, most, max_rows)
+                       nkv, G, W * bs, Z, even, most, max_rows)
 #define ST_HD(HDV)                                                            \
     do {                                                                      \
         if (fp8 && qt == 1) ST_ONE(HDV, 1, unsigned char);                    \

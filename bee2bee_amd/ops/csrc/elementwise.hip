@@ -199,6 +199,7 @@ __global__ void kv_store_kernel(
     const int t = glob_wave / nkv;
     const int h = glob_wave % nkv;
     const int slot = slots[t];
+    if (slot < 0) return;            // no such position
     const int blk = slot / bs, off = slot % bs;
     const long dst = (((long)blk * nkv + h) * bs + off) * hd;
     const unsigned short* ks = k + (long)t * sk + (long)h * hd;
@@ -228,6 +229,7 @@ __global__ void kv_store_fp8_kernel(
     const int t = glob_wave / nkv;
     const int h = glob_wave % nkv;
     const int slot = slots[t];
+    if (slot < 0) return;            // no such position
     const int blk = slot / bs, off = slot % bs;
     const long dst = (((long)blk * nkv + h) * bs + off) * hd;
     const unsigned short* ks = k + (long)t * sk + (long)h * hd;
@@ -318,6 +320,7 @@ __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     }
     if (h < nq) return;
     const int kvh = (h - nq) % nkv, slot = slots[t];
+    if (slot < 0) return;            // no such position
     const long dst =
         (((long)(slot / bs) * nkv + kvh) * bs + slot % bs) * hd + d;
     CT* cache = (h < nq + nkv ? k_cache : v_cache) + dst;
@@ -350,7 +353,8 @@ __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
 // kernels), 501 -> 490 us at llama3.2-1b's (the slots alone).
 
 // slot[b] = table[b][pos / bs] * bs + pos % bs: where row b's new key and value
-// go. A position past the table is an error, as an index past its end is.
+// go; -1, which the kernels that store leave out, for a position that the table
+// does not have.
 __global__ void decode_slots_kernel(const int* __restrict__ table,
                                     const int* __restrict__ pos,
                                     int* __restrict__ slots, int B, int W,
@@ -358,24 +362,28 @@ __global__ void decode_slots_kernel(const int* __restrict__ table,
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
     const int p = pos[b], page = p / bs;
-    if (p < 0 || page >= W) __builtin_trap();
-    slots[b] = table[b * row_stride + page] * bs + p % bs;
+    slots[b] = p < 0 || page >= W
+                   ? -1
+                   : table[b * row_stride + page] * bs + p % bs;
 }
 
-// out[t] = embed[ids[t]] + pos_embed[pos[t]], one workgroup a token
+// out[t] = embed[ids[t]] + pos_embed[pos[t]], one workgroup a token; a row of
+// NaN for an id or a position that the tables do not have
 __global__ void embed_positions_kernel(
     const long* __restrict__ ids, const unsigned short* __restrict__ embed,
     const int* __restrict__ pos, const unsigned short* __restrict__ pos_embed,
     unsigned short* __restrict__ out, int H, long vocab, int positions) {
     const long t = blockIdx.x, id = ids[t];
     const int p = pos[t];
-    if (id < 0 || id >= vocab || p < 0 || p >= positions) __builtin_trap();
+    const bool known = id >= 0 && id < vocab && p >= 0 && p < positions;
     for (int i = threadIdx.x * 8; i < H; i += blockDim.x * 8) {
         float a[8], b[8];
-        load_bf16x8(embed + id * H + i, a);
-        load_bf16x8(pos_embed + (long)p * H + i, b);
+        if (known) {
+            load_bf16x8(embed + id * H + i, a);
+            load_bf16x8(pos_embed + (long)p * H + i, b);
+        }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) a[e] += b[e];
+        for (int e = 0; e < 8; ++e) a[e] = known ? a[e] + b[e] : NAN;
         store_bf16x8(out + t * H + i, a);
     }
 }

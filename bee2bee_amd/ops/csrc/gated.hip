@@ -232,6 +232,7 @@ rope_store_kernel(const TIN* q, long q_tok, T* q_out, long qo_tok, int H, const 
     const int pos = positions[t];
     const int half = dims / 2;
     const int slot = slot_mapping[t];
+    if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
     float* nb = buf[wid];
     // no workgroup barrier below, so waves past the end just leave

@@ -293,6 +293,7 @@ __global__ void latent_rope_store_kernel(
     const long t = blockIdx.x;
     const T* row = kv + t * kv_stride;
     const long slot = slot_mapping[t];
+    if (slot < 0) return;            // no such position
     T* dst = cache + slot * (long)(C + R);
     float ss = 0.f;
     for (int i = threadIdx.x; i < C; i += blockDim.x) {
@@ -491,6 +492,7 @@ qk_norm_rope_store_kernel(T* __restrict__ q, long q_tok, int H,
     const int pos = positions[t];
     const int half = dims / 2;
     const int slot = slot_mapping[t];
+    if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
     float* nb = buf[wid];
     for (int hh = wid; hh < H + G; hh += 4) {
@@ -568,6 +570,7 @@ head_norm_store_kernel(T* __restrict__ q, long q_tok, int H,
         dst = q + t * q_tok + (long)g * D;
     } else {
         const int slot = slot_mapping[t];
+        if (slot < 0) return;        // no such position
         const long row = ((long)(slot / bs) * G + g) * bs + slot % bs;
         dst = kind == 1 ? k_cache + row * D : v_cache + row * Dv;
     }

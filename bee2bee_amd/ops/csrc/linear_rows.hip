@@ -368,6 +368,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         const bool is_k = head < st.nq + st.nkv;
         const int kvh = head - st.nq - (is_k ? 0 : st.nkv);
         const int slot = st.slots[m];
+        if (slot < 0) return;                  // no such position
         const long at = (((long)(slot / st.bs) * st.nkv + kvh) * st.bs +
                          slot % st.bs) * st.hd + d;
         void* cache = is_k ? st.k_cache : st.v_cache;

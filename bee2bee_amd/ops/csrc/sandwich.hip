@@ -179,6 +179,7 @@ rope_unit_store_kernel(T* __restrict__ q, long q_tok, int H,
     const int pos = positions[t];
     const int half = dims / 2;
     const int slot = slot_mapping[t];
+    if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
     float* nb = buf[wid];
     // one head per wave: blockIdx.y walks the H + 2G heads four at a time

@@ -113,6 +113,7 @@ proj_norm_store_kernel(T* __restrict__ q, long q_tok, int H,
     __shared__ float red[TS_THREADS / WAVE];
     const long t = blockIdx.x;
     const int slot = slot_mapping[t];
+    if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
     const int nq = H * D, nk = G * D;
     T* qr = q + t * q_tok;

@@ -160,3 +160,26 @@ def test_norms_see_the_unrounded_residual(rows):
     got, want = (s.prompt(ids, [rows]) for s in (gpu, cpu))
     # the first layer's norm of 256 + bias, through gelu and 100 w_down
     assert _rel(got, want) <= 0.015, _rel(got, want)
+
+
+def test_a_captured_step_ends_at_its_block_table():
+    """48 positions in three pages of 16: a request that asks for more ends
+    there, and the one beside it goes on."""
+    from bee2bee_amd.engine.engine import GenerationRequest, InferenceEngine
+    from bee2bee_amd.engine.sampler import SamplingParams
+
+    eng = InferenceEngine("tiny", device="cuda:0", max_batch=2, max_seq_len=40,
+                          kv_block_size=16, kv_blocks=12)
+    try:
+        assert eng.graphs is not None
+        reqs = [eng.submit(GenerationRequest(
+            prompt_ids=[1, 2, 3], max_new_tokens=n,
+            sampling=SamplingParams(greedy=True))) for n in (1000, 30)]
+        for r in reqs:
+            while isinstance(r.out_queue.get(timeout=60), int):
+                pass
+            assert r.error is None
+        assert [len(r.prompt_ids) + len(r.output_ids) for r in reqs] == [49,
+                                                                         33]
+    finally:
+        eng.shutdown()

@@ -315,3 +315,45 @@ def test_embed_positions(T, H):
     pos = torch.randint(0, 40, (T,), device=DEV, dtype=torch.int32)
     got = ops.embed_positions(ids, table, pos, pos_table)
     assert torch.equal(got, table[ids] + pos_table[pos.long()])
+
+
+def test_ids_and_positions_that_the_tables_do_not_have():
+    """No slot and nothing stored, a row of NaN, keys of the pages alone; the
+    rows beside them are what they are."""
+    i32 = dict(device=DEV, dtype=torch.int32)
+    table = torch.tensor([[1, 3], [2, 0], [4, 5], [3, 1]], **i32)
+    pos = torch.tensor([31, 32, -1, 5], **i32)
+    slots = ops.decode_slots(table, pos, 16)
+    assert slots.tolist() == [63, -1, -1, 53]
+    emb, pemb = _rand(50, 64), _rand(40, 64)
+    ids = torch.tensor([3, 50, -1, 7, 8], device=DEV)
+    at = torch.tensor([1, 2, 3, 40, 39], **i32)
+    got = ops.embed_positions(ids, emb, at, pemb)
+    assert torch.equal(got[[0, 4]], emb[[3, 8]] + pemb[[1, 39]])
+    assert got[1:4].isnan().all()
+    nkv, hd = 2, 64
+    cos, sin = reference.rope_tables(64, hd, 1e4, DEV)
+    pos = pos.clamp(0)
+    for dt in (torch.bfloat16, torch.uint8):
+        qkv, x = _rand(4, 4 * nkv * hd), _rand(4, 64)
+        w, norm = _rand(4 * nkv * hd, 64), (_rand(64), None, 1e-5)
+        k = qkv.view(4, -1, hd)[:, :nkv]
+        for store in (
+                lambda c, v: ops.rope_store_qkv(
+                    qkv.clone(), None, 2 * nkv, pos, cos, sin, c, v, slots),
+                lambda c, v: ops.rows_qkv(x, w, None, norm, 2 * nkv, pos, cos,
+                                          sin, c, v, slots),
+                lambda c, v: ops.kv_cache_store(k, k, c, v, slots)):
+            # a page before the cache and one after it
+            flat = torch.zeros(2, 8, nkv, 16, hd, device=DEV, dtype=dt)
+            store(flat[0][1:7], flat[1][1:7])
+            rows = flat.transpose(2, 3).reshape(2, 8 * 16, nkv * hd)
+            used = (rows != 0).any(-1)
+            assert used.nonzero().tolist() == [
+                [c, 16 + s] for c in (0, 1) for s in (53, 63)]
+    kc, vc = _rand(6, nkv, 16, hd), _rand(6, nkv, 16, hd)
+    q = _rand(4, 4, hd)
+    past = torch.tensor([32, 33, 1000, 6], **i32)
+    assert torch.equal(ops.attn_decode(q, kc, vc, table, past, 0.1),
+                       ops.attn_decode(q, kc, vc, table, past.clamp(max=32),
+                                       0.1))
