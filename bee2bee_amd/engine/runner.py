@@ -146,7 +146,8 @@ class Runner:
                 self.spec.rms_eps, self.dtype)
             return F.linear(normed, self.weights.lm_head)
         W = self.weights
-        if self._rows_dims and ops.few_rows(hidden):
+        if self._rows_dims and ops.head_rows(
+                hidden, self.spec.norm_type == "layernorm"):
             return ops.rows_linear(
                 hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
                                          self.spec.rms_eps))

@@ -115,7 +115,8 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
     constexpr bool PAIR = EPI == LR_GLU || EPI == LR_QKV;
     constexpr int WT = PAIR ? 2 * NT : NT;
     constexpr int H = TC == 16 ? G : 1;        // tiles of W along K a step
-    constexpr int U = LR_U / (WT * H) > 0 ? LR_U / (WT * H) : 1;
+    // (4 tiles: whole 128-byte lines of W a batch, as with fewer)
+    constexpr int U = NT == 4 ? 2 : LR_U / (WT * H) > 0 ? LR_U / (WT * H) : 1;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -459,7 +460,15 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
 //    4096x4096 8.6 / 10.9 / 14.4, 9.3 / 9.8 / 11.6, 9.2 / 10.4 / 11.9;
 //    4096x14336 24.9 / 32 / 44, 24.9 / 26.5 / 34.5, 25.4 / 29.3 / 34.6;
 //    3584x18944 31 / 41 / 56, 29 / 34 / 44, 32 / 40 / 46;
-//   above: 128256x4096 8x2x8 174 / 204 / 272, 8x2x16 184 / 194 / 217.
+//   above: 128256x4096 8x2x8 174 / 204 / 272, 8x2x16 184 / 194 / 217;
+//   from 16384 on, K below 8192 (output heads): of 9 rows and more the input,
+//    read once for 32 columns, is half of what comes through L2, so 4 tiles;
+//    4 waves leave the registers for whole lines of 4 tiles, and add as 4 waves
+//    of 2 do (1 / 9 / 16 rows, 8x2x16 and 4x2x16 or 4x4x16): 128256x4096 186 /
+//    193 / 210 and 175 / 190 / 192, 128256x3072 140 / 147 / 165 and 137 / 147 /
+//    154, 152064x3584 189 / 207 / 224 and 184 / 198 / 207; 128256x8192 360 /
+//    372 / 396 and 394 / 420 / 428; 4608x4096, too few workgroups, 17 / 18 / 18
+//    and 17 / 24 / 26.
 extern "C" int launch_linear_rows(
     const void* x, int x32, const unsigned short* norm_w,
     const unsigned short* norm_b, const unsigned short* w,
@@ -513,6 +522,8 @@ extern "C" int launch_linear_rows(
     else if (epi == LR_GLU && t8) LR_NORMS(4, 1, 16, 2, LR_GLU);
     else if (epi == LR_GLU) LR_16(4, 1, LR_GLU);
     else if (epi == LR_GELU) LR_16(8, 1, LR_GELU);
+    else if (N >= 16384 && K < 8192 && M > 8) LR_16(4, 4, LR_PLAIN);
+    else if (N >= 16384 && K < 8192) LR_16(4, 2, LR_PLAIN);
     else if (N > 4096) LR_16(8, 2, LR_PLAIN);
     else if (N > 2048 && t8) LR_8(8, 2, LR_PLAIN);
     else if (t8) LR_8(8, 1, LR_PLAIN);

@@ -50,6 +50,7 @@ def _products(x, w, norm):
 @pytest.mark.parametrize("N,K", [
     (16, 32), (17, 64), (50257, 96), (768, 3072), (4096, 2048), (4112, 256),
     (4608, 3584), (1000, 4096 + 32), (9, 64), (2052, 576),
+    (16384, 160), (16421, 96), (16400, 8192),
 ])
 @pytest.mark.parametrize("kind", [None, "rms", "layer"])
 def test_plain(M, N, K, kind):
@@ -90,6 +91,7 @@ def test_activations(M, I, K):
 
 @pytest.mark.parametrize("N,K,act", [
     (2048, 576, None), (4096, 576, None), (4112, 256, None), (64, 96, None),
+    (16384, 96, None), (16421, 416, None), (4100, 8192, None),
     (4096, 320, "swiglu"), (4096, 96, "swiglu"), (64, 256, "gelu"),
 ])
 def test_rows_alone(N, K, act):
