@@ -295,12 +295,25 @@ def mid_rows(x: torch.Tensor) -> bool:
             and x.dtype is torch.bfloat16 and x.is_contiguous())
 
 
+def _deep(width: int, depth: int) -> bool:
+    return depth * 2 >= 7 * width
+
+
 def deep_rows(x: torch.Tensor, inner: int) -> bool:
     """Steps of up to DEEP_MAX such rows whose down projection is at least
     3.5 times as deep as wide."""
     return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
             and x.dtype is torch.bfloat16 and x.is_contiguous()
-            and inner * 2 >= 7 * x.shape[1])
+            and _deep(x.shape[1], inner))
+
+
+def mid_shape(w: torch.Tensor) -> bool:
+    """Projections that mid_linear takes: up to 6144 outputs, or deep ones.
+    Wider, K is split in two or not at all and the library wins: 10240 x 8192
+    with the rotation after it 55 us at 17 rows, 61 at 48, 80 at 128 (library
+    43, 48, 64), 8192 x 8192 with the add and norm 43, 44, 52 (36, 40, 56);
+    but 8192 x 28672 95, 110, 155 (99, 179, 210)."""
+    return w.shape[0] <= 6144 or _deep(*w.shape)
 
 
 def mid_linear(x, w):

@@ -32,6 +32,16 @@ GELU = ModelSpec(name="t-gelu", vocab_size=500, hidden_size=256,
                  attn_out_bias=True, mlp_bias=True)
 
 
+# outputs too wide for the split projections of some tens of rows: q|k|v, and
+# attention output and down projection
+WIDE = [ModelSpec(name="t-wide-qkv", vocab_size=500, hidden_size=128,
+                  intermediate_size=256, n_layers=2, n_heads=64,
+                  n_kv_heads=32, head_dim=64, max_seq_len=1024),
+        ModelSpec(name="t-wide", vocab_size=500, hidden_size=6208,
+                  intermediate_size=128, n_layers=2, n_heads=2, n_kv_heads=2,
+                  head_dim=64, max_seq_len=1024)]
+
+
 def _tensors(holder):
     names = getattr(holder, "__slots__", None) or list(vars(holder))
     pairs = [(n, getattr(holder, n, None)) for n in names]
@@ -114,9 +124,12 @@ def _rel(got, want):
     return ((got - want).norm() / want.norm()).item()
 
 
-@pytest.mark.parametrize("kv_dtype", ["native", "fp8"])
-@pytest.mark.parametrize("spec", [SWIGLU, GELU], ids=lambda s: s.name)
-@pytest.mark.parametrize("rows", [1, 9, 16, 17, 160, 161, 256, 257])
+@pytest.mark.parametrize("spec,rows,kv_dtype", [
+    (spec, rows, kv_dtype) for spec in (SWIGLU, GELU)
+    for rows in (1, 9, 16, 17, 160, 161, 256, 257)
+    for kv_dtype in ("native", "fp8")
+] + [(spec, rows, "native") for spec in WIDE for rows in (17, 200)],
+    ids=lambda v: getattr(v, "name", str(v)))
 @torch.no_grad()
 def test_steps(spec, rows, kv_dtype):
     W, G = _weights(spec)
