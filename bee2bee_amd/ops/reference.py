@@ -346,18 +346,22 @@ def add_norm_parts(part, bias, resid, norm=None):
 
 def rope_store_qkv(qkv, bias, n_heads, positions, cos, sin, k_cache, v_cache,
                    slot_mapping):
-    if qkv.dim() == 3:
-        rows = qkv.sum(0)
-    else:
-        rows = qkv.float()
+    rows = qkv.sum(0) if qkv.dim() == 3 else qkv
+    if rows.dtype != torch.float64:
+        rows = rows.float()
     if bias is not None:
-        rows = rows + bias.float()
+        rows = rows + bias
     T, N = rows.shape
     nkv, hd = k_cache.shape[1], k_cache.shape[3]
     q, k, v = rows.view(T, -1, hd).split([n_heads, nkv, nkv], dim=1)
     if positions is not None:
         rope_inplace(q, k, positions, cos, sin)
-    dtype = qkv.dtype if qkv.dim() == 2 else k_cache.dtype
+    # parts are fp32 whatever the model computes in: its pages' type, and bf16
+    # beside 8-bit pages
+    dtype = qkv.dtype
+    if qkv.dim() == 3:
+        dtype = (k_cache.dtype if k_cache.dtype.is_floating_point
+                 else torch.bfloat16)
     out = rows.to(dtype)
     _, k, v = out.view(T, -1, hd).split([n_heads, nkv, nkv], dim=1)
     kv_cache_store(k, v, k_cache, v_cache, slot_mapping)

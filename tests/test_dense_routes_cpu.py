@@ -1,0 +1,156 @@
+"""The Runner's routes for dense steps of few rows and of some tens, on the CPU
+with the reference ops in the kernels' places, against the plain route."""
+import dataclasses
+import multiprocessing as mp
+import pickle
+
+import pytest
+import torch
+
+from bee2bee_amd import ops
+from bee2bee_amd.engine.graphs import decode_slot_mapping
+from bee2bee_amd.engine.kv import PagedKV
+from bee2bee_amd.engine.runner import Runner
+from bee2bee_amd.models.spec import PRESETS
+from bee2bee_amd.models.weights import ModelWeights
+from bee2bee_amd.ops import reference
+
+CPU = torch.device("cpu")
+TINY = dataclasses.replace(PRESETS["tiny"], qkv_bias=True, head_dim=32)
+ROUTES = {"few": {"few_rows": True}, "mid": {"mid_rows": True},
+          "deep": {"deep_rows": True}}
+
+
+def _weights(spec):
+    W = ModelWeights(spec, CPU, torch.float32).random_init(seed=3)
+    g = torch.Generator().manual_seed(4)
+    W.embed.normal_(0.0, 1.0, generator=g)
+    for lw in W.layers:
+        for name in lw.__slots__:
+            t = getattr(lw, name, None)
+            if isinstance(t, torch.Tensor):
+                std = 0.5 if name.endswith("bias") else 0.2
+                t.normal_(float(name.endswith("norm")), std, generator=g)
+    return W
+
+
+def _steps(spec, W):
+    """Hidden rows of two prompts, a decode step and a portion."""
+    kv = PagedKV(spec, CPU, torch.float32, n_blocks=16, block_size=16)
+    r = Runner(spec, W, kv, CPU, torch.float32)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32)
+    ids = torch.arange(30) * 7 % 500
+
+    def chunk(lens, old, more):
+        pos, slots, cu = [], [], [0]
+        for s, (n, o) in enumerate(zip(lens, old)):
+            if not o:
+                kv.new_seq(s)
+            kv.extend_seq(s, o + n)
+            pos += range(o, o + n)
+            slots += kv.slot_mapping(s, range(o, o + n))
+            cu.append(cu[-1] + n)
+        if more:
+            more = {"block_table": kv.block_table([0, 1]),
+                    "seq_lens": ints([a + b for a, b in zip(lens, old)]),
+                    "query_lens": ints(lens)}
+        return r.forward_prefill(ids[: cu[-1]], ints(pos), ints(slots),
+                                 ints(cu), max(lens), **(more or {}))
+
+    out = [chunk([5, 18], [0, 0], False)]
+    for s, n in enumerate((6, 19)):
+        kv.extend_seq(s, n)
+    table, pos = kv.block_table([0, 1]), ints([5, 18])
+    out.append(r.forward_decode(ids[:2], pos,
+                                decode_slot_mapping(table, pos, 16), table,
+                                pos + 1))
+    out.append(chunk([4, 3], [6, 19], True))
+    out.append(r.lm_head(out[-1]))
+    return out
+
+
+@pytest.mark.parametrize("route", list(ROUTES))
+@pytest.mark.parametrize("spec", [TINY, PRESETS["tiny-gpt2"]],
+                         ids=["swiglu", "gelu"])
+@torch.no_grad()
+def test_a_route_computes_what_the_plain_one_does(spec, route, monkeypatch):
+    W = _weights(spec)
+    want = _steps(spec, W)
+    taken = []
+    for name in ("few_rows", "mid_rows", "deep_rows"):
+        on = ROUTES[route].get(name, False)
+        monkeypatch.setattr(ops, name, lambda *a, on=on: on)
+    for name in ("rows_linear", "rows_qkv", "mid_linear"):
+        op = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, op=op, name=name, **k: (
+            taken.append(name), op(*a, **k))[1])
+    got = _steps(spec, W)
+    few = {"rows_linear"} | ({"rows_qkv"} if spec.head_dim == 32 else set())
+    assert set(taken) == (few if route == "few" else {"mid_linear"})
+    for a, b in zip(got, want):
+        # fp32 sums in another order
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_parts_beside_8_bit_pages(fp8):
+    """Parts give rows of the pages' type, and bf16 beside 8-bit pages."""
+    g = torch.Generator().manual_seed(1)
+    parts = torch.randn(3, 4, 8 * 16, generator=g)
+    dt = torch.uint8 if fp8 else torch.bfloat16
+    kc, vc = torch.zeros(2, 2, 16, 16, dtype=dt), torch.zeros(2, 2, 16, 16,
+                                                              dtype=dt)
+    slots = torch.tensor([3, 17, 0, 31], dtype=torch.int32)
+    got = reference.rope_store_qkv(parts, None, 4, None, None, None, kc, vc,
+                                   slots)
+    assert got.dtype == torch.bfloat16
+    assert torch.equal(got, parts.sum(0).bfloat16())
+    rows = kc[slots.long() // 16, :, slots.long() % 16]
+    want = got.view(4, 8, 16)[:, 4:6]
+    assert torch.equal(rows, reference._kv_quant_like(want, kc) if fp8
+                       else want)
+
+
+def _tp_worker(rank, world, port, few, out_path):
+    import torch.distributed as dist
+
+    from bee2bee_amd.parallel.tp import TPEngine
+
+    dist.init_process_group(
+        backend="gloo", init_method=f"tcp://127.0.0.1:{port}", rank=rank,
+        world_size=world)
+    try:
+        if few:
+            ops.few_rows = lambda x: x.dim() == 2 and x.shape[0] <= 16
+        eng = TPEngine(TINY, device="cpu", max_batch=4, max_seq_len=64, seed=5)
+        out, lm_head = [], eng.runner.lm_head
+        eng.runner.lm_head = lambda h: (out.append(lm_head(h)), out[-1])[1]
+        tokens = eng.generate([[5, 6, 7, 8, 9], [100, 101]], 4)
+        if rank == 0:
+            with open(out_path, "wb") as f:
+                pickle.dump((tokens, out), f)
+    finally:
+        dist.destroy_process_group()
+
+
+@pytest.mark.timeout(300)
+def test_few_rows_under_tensor_parallelism(tmp_path):
+    """Two ranks, each with its part of the inner dimensions: the reduced rows
+    are added and normed as on the plain route."""
+    results = []
+    for few, port in ((False, 29741), (True, 29742)):
+        path = str(tmp_path / f"tp{few}.pkl")
+        ctx = mp.get_context("spawn")
+        procs = [ctx.Process(target=_tp_worker, args=(r, 2, port, few, path))
+                 for r in range(2)]
+        for p in procs:
+            p.start()
+        for p in procs:
+            p.join(timeout=140)
+            assert p.exitcode == 0
+        with open(path, "rb") as f:
+            results.append(pickle.load(f))
+    (t0, l0), (t1, l1) = results
+    assert t0 == t1
+    for a, b in zip(l0, l1):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
