@@ -322,16 +322,37 @@ static int flash_smem(int hd, int rw, int ksp) {
 
 // Shape of a workgroup by how many of 256 rows the step fills (`full`,
 // T * nq / 256; a CU holds one such workgroup at head size 128, two at 64):
-// 256 rows read a key tile from memory least often and win once there are
-// about two rounds of them; with fewer, 128 rows balance better; with less
-// than a chip of those, 64 rows whose two wave pairs share a tile's keys.
-// Measured (us; 256 / 128 / 64 rows), head size 128: full 1024 600/674/735,
-// 448 (with 12k cached) 897/1056/1146, 426 (nine short prompts) 39/38/50,
-// 256 70/63/63, 128 37/31/26, 64 23/18/15; head size 64: 2048 333/362/405,
-// 750 48/47/63, 125 25/21/17.
-static int flash_shape(int hd, long full) {
-    if (full >= (hd == 128 ? 440 : 1024)) return 0;
-    return full >= (hd == 128 ? 150 : 230) ? 1 : 2;
+// 256 rows read a key tile from memory least often and win where there are
+// enough of them and their tiles are about as long as each other (one long
+// prompt's, in falling order, or portions behind long histories); with fewer,
+// 128 rows balance better, with less than a chip of those 64 rows, whose two
+// wave pairs share a tile's keys. Prompts of different lengths leave tiles of
+// every length to balance: 256 rows need 256 fillings a prompt.
+// Measured (us, 256 / 128 / 64 rows; heads 32/8 unless stated), head size 128:
+//   one prompt: full 150 42/34/30, 256 70/57/63, 350 92/85/101, 400 107/108/127,
+//    450 121/135/159, 600 218/214/268, 1000 534/549/709;
+//   9 prompts of an eighth to 1: 100 12.9/12.3/10.4, 149 15/14/17, 450
+//    38/34/46 (28/4: 59/45/71), 1000 116/102/141 (28/4: 215/167/248), 1400
+//    191/183/247; 4 prompts: 124 22/19/24, 600 171/161/224, 1000 412/405/561,
+//    2000 1525/1521/2078;
+//   8000 cached: 100 263/220/186, 150 275/288/347, 256 322/346/421, 300
+//    518/503/559, 350 548/527/619, 400 573/632/767, 600 946/930/1143, 1000
+//    1537/1681/2123;
+// head size 64:
+//   one prompt: 300 54/46/45 (12/12: 140/117/107), 350 64/55/56, 600
+//    135/132/147, 750 184/191/221; 9 prompts: 200 15.2/10.7/11 (12/12:
+//    23/21/17), 600 31/30/34, 1000 59/60/72 (12/12: 151/146/180); 2: 600
+//    157/171/202;
+//   8000 cached: 150 193/187/169, 200 205/195/215, 300 297/272/303, 400
+//    338/391/402, 520 491/476/543, 1000 863/951/1127.
+static int flash_shape(int hd, long full, int nseq, bool pages) {
+    const bool lone = !pages && nseq == 1;
+    if (hd == 128) {
+        if (full >= 400 && (pages || full >= 256L * nseq)) return 0;
+        return full >= (lone ? 230 : pages ? 140 : 115) ? 1 : 2;
+    }
+    if (full >= (pages ? 400 : 700)) return 0;
+    return full >= (lone ? 320 : pages ? 185 : 230) ? 1 : 2;
 }
 
 #define FL_ONE(HDV, RWV, KSPV, PG, KVT)                                       \
@@ -363,7 +384,7 @@ extern "C" int launch_attn_flash(
     if (nseq == 0 || max_qlen <= 0) return 0;
     const int pairs = nseq * nkv;
     const long rows = (long)max_qlen * (nq / nkv);
-    const int shape = flash_shape(hd, T * nq / 256);
+    const int shape = flash_shape(hd, T * nq / 256, nseq, block_table);
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

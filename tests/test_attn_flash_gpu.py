@@ -45,6 +45,7 @@ def _check(got, want, v):
     # 128- and 256-row workgroups
     (28, 4, 128, [700, 513, 64, 300]), (32, 8, 128, [512] * 7 + [1]),
     (12, 12, 64, [1000] * 6), (64, 8, 64, [513] * 8 + [63]),
+    (32, 8, 128, [3300]), (32, 8, 128, [300, 1, 257]), (12, 12, 64, [7000]),
 ])
 def test_whole_prompts(nq, nkv, hd, lens):
     q, k, v = _qkv(sum(lens), nq, nkv, hd, len(lens))
