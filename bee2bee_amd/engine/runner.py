@@ -233,12 +233,16 @@ class Runner:
         s, T = self.spec, x.shape[0]
         layers = self.weights.layers
         gelu, all_parts = s.act_type == "gelu", ops.mid_rows(x)
+        H = s.hidden_size
+        qkv_parts = all_parts and ops.mid_shape(s.q_size + 2 * s.kv_size, H)
+        o_parts = all_parts and ops.mid_shape(H, s.q_size)
+        down_parts = ops.mid_shape(H, s.intermediate_size)
         lw = layers[self.layer_lo]
         normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
 
         def add_norm(rows, w, bias, nxt, parts):
             """x + rows w^T + bias, and its norm by nxt (None: no norm)."""
-            if parts and ops.mid_shape(w):
+            if parts:
                 return ops.add_norm_parts(ops.mid_linear(rows, w), bias, x,
                                           nxt and (*nxt, s.rms_eps))
             y = F.linear(rows, w, bias)
@@ -247,19 +251,19 @@ class Runner:
 
         for i in range(self.layer_lo, self.layer_hi):
             lw = layers[i]
-            qkv = (ops.mid_linear(normed, lw.wqkv)
-                   if all_parts and ops.mid_shape(lw.wqkv)
+            qkv = (ops.mid_linear(normed, lw.wqkv) if qkv_parts
                    else F.linear(normed, lw.wqkv))
             o = self._attend(i, qkv, positions, slot_mapping,
                              attn_fn).reshape(T, s.q_size)
             normed, x = add_norm(o, lw.wo, lw.wo_bias,
-                                 (lw.mlp_norm, lw.mlp_norm_bias), all_parts)
+                                 (lw.mlp_norm, lw.mlp_norm_bias), o_parts)
             z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
             z = ops.gelu(z) if gelu else ops.swiglu(z)
             nxt = None
             if i + 1 < self.layer_hi:
                 nxt = layers[i + 1].attn_norm, layers[i + 1].attn_norm_bias
-            normed, x = add_norm(z, lw.w_down, lw.w_down_bias, nxt, True)
+            normed, x = add_norm(z, lw.w_down, lw.w_down_bias, nxt,
+                                 down_parts)
         return x
 
     def _rows_add(self, x, y, w, bias, nxt):

@@ -241,17 +241,23 @@ def head_rows(x: torch.Tensor, layer_norm: bool) -> bool:
     at 16; 152064 of 3584 207 / 239 at 16; of 8192 373 / 371 at 8, 415 / 363 at
     16, 201088 of 8192 603 / 609 at 12, 623 / 593 at 16. A layer norm's mean and
     deviation are taken by each of the hundreds of workgroups: 50257 of 768 22.0
-    / 21.8 at 1 row, 30 / 23 at 16; of 1600 42 / 38 and 59 / 37."""
-    return few_rows(x) and not layer_norm and (x.shape[0] <= 12
-                                               or x.shape[1] < 8192)
+    / 21.8 at 1 row, 22.8 / 22.1 at 4 (a launch less for the host: 20 us of a
+    step that is not captured), 25 / 22.5 at 8, 30 / 23 at 16."""
+    if layer_norm:
+        return few_rows(x) and x.shape[0] <= 4
+    return few_rows(x) and (x.shape[0] <= 12 or x.shape[1] < 8192)
+
+
+_ACTS = {None: 0, "swiglu": 1, "gelu": 2}
 
 
 def _norm_args(norm):
     """weight, bias, squares, eps of the bindings."""
     if norm is None:
         return None, None, None, 0.0
-    return (None, None, *norm) if len(norm) == 2 else (*norm[:2], None,
-                                                       norm[2])
+    if len(norm) == 2:
+        return None, None, norm[0], norm[1]
+    return norm[0], norm[1], None, norm[2]
 
 
 def rows_linear(x, w, bias=None, resid=None, norm=None, act=None,
@@ -263,10 +269,12 @@ def rows_linear(x, w, bias=None, resid=None, norm=None, act=None,
     norm's projection takes: -> (result, result * then, sums of squares of 8
     columns each)."""
     if _use_hip(x):
-        out = require_hip().rows_linear(
-            x, w, bias, resid, *_norm_args(norm),
-            {None: 0, "swiglu": 1, "gelu": 2}[act], keep32, then)
-        return out[0] if then is None else tuple(out)
+        nw, nb, squares, eps = _norm_args(norm)
+        if then is None:
+            return require_hip().rows_linear(x, w, bias, resid, nw, nb,
+                                             squares, eps, _ACTS[act], keep32)
+        return require_hip().rows_sum(x, w, bias, resid, nw, nb, squares, eps,
+                                      keep32, then)
     return reference.rows_linear(x, w, bias, resid, norm, act, keep32, then)
 
 
@@ -307,13 +315,13 @@ def deep_rows(x: torch.Tensor, inner: int) -> bool:
             and _deep(x.shape[1], inner))
 
 
-def mid_shape(w: torch.Tensor) -> bool:
+def mid_shape(width: int, depth: int) -> bool:
     """Projections that mid_linear takes: up to 6144 outputs, or deep ones.
     Wider, K is split in two or not at all and the library wins: 10240 x 8192
     with the rotation after it 55 us at 17 rows, 61 at 48, 80 at 128 (library
     43, 48, 64), 8192 x 8192 with the add and norm 43, 44, 52 (36, 40, 56);
     but 8192 x 28672 95, 110, 155 (99, 179, 210)."""
-    return w.shape[0] <= 6144 or _deep(*w.shape)
+    return width <= 6144 or _deep(width, depth)
 
 
 def mid_linear(x, w):

@@ -110,18 +110,20 @@ Rows rows_of(const Tensor& x, const Tensor& w, const optional<Tensor>& norm_w,
 }
 
 // x of a layer norm, and resid, may be fp32; keep32: so is the result. then_w,
-// the weight of the RMS norm that reads the result: -> also the result times it,
-// and the sums of squares of 8 columns each
-std::vector<Tensor> rows_linear(
-    const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
-    const optional<Tensor>& resid, const optional<Tensor>& norm_w,
-    const optional<Tensor>& norm_b, const optional<Tensor>& squares,
-    double eps, int64_t act, bool keep32, const optional<Tensor>& then_w) {
+// the weight of the RMS norm that reads the result: also the result times it, and
+// the sums of squares of 8 columns each, in scaled and squares_out
+Tensor rows_product(const Tensor& x, const Tensor& w,
+                    const optional<Tensor>& bias,
+                    const optional<Tensor>& resid,
+                    const optional<Tensor>& norm_w,
+                    const optional<Tensor>& norm_b,
+                    const optional<Tensor>& squares, double eps, int64_t act,
+                    bool keep32, const optional<Tensor>& then_w,
+                    Tensor& scaled, Tensor& squares_out) {
     const Rows r = rows_of(x, w, norm_w, norm_b, squares);
     TORCH_CHECK(act == EPI_PLAIN || act == EPI_GLU || act == EPI_GELU);
     TORCH_CHECK(act != EPI_GLU || (r.N % 32 == 0 && !bias.has_value()));
-    TORCH_CHECK(act == EPI_PLAIN ||
-                !(resid.has_value() || keep32 || then_w.has_value()));
+    TORCH_CHECK(act == EPI_PLAIN || !(resid.has_value() || keep32));
     const int N = act == EPI_GLU ? r.N / 2 : r.N;
     if (resid.has_value())
         TORCH_CHECK(resid->dim() == 2 && resid->size(0) == r.M &&
@@ -131,24 +133,48 @@ std::vector<Tensor> rows_linear(
         resid.has_value() ? dense(*resid, "resid", true) : Tensor();
     const auto bf16 = r.w.options();
     const auto f32 = bf16.dtype(torch::kFloat32);
-    std::vector<Tensor> out{torch::empty({r.M, N}, keep32 ? f32 : bf16)};
+    Tensor y = torch::empty({r.M, N}, keep32 ? f32 : bf16);
     const Tensor tw = column(then_w, N, "the next norm's weight");
     if (tw.defined()) {
         TORCH_CHECK(N % 8 == 0);
-        out.push_back(torch::empty({r.M, N}, bf16));
-        out.push_back(torch::empty({r.M, N / 8}, f32));
+        scaled = torch::empty({r.M, N}, bf16);
+        squares_out = torch::empty({r.M, N / 8}, f32);
     }
     TORCH_CHECK(launch_linear_rows(
                     r.x.data_ptr(), is_f32(r.x), ptr(r.norm_w),
                     ptr(r.norm_b), ptr(r.w), ptr(b), r.sq(),
                     add.defined() ? add.data_ptr() : nullptr,
-                    add.defined() && is_f32(add), out[0].data_ptr(), keep32,
-                    ptr(tw), tw.defined() ? mut(out[1]) : nullptr,
-                    tw.defined() ? out[2].data_ptr<float>() : nullptr, r.M, N,
-                    r.K, (float)eps, r.norm, (int)act, nullptr, nullptr,
-                    nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0,
-                    stream()) == 0);
-    return out;
+                    add.defined() && is_f32(add), y.data_ptr(), keep32,
+                    ptr(tw), tw.defined() ? mut(scaled) : nullptr,
+                    tw.defined() ? squares_out.data_ptr<float>() : nullptr,
+                    r.M, N, r.K, (float)eps, r.norm, (int)act, nullptr,
+                    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0,
+                    0, stream()) == 0);
+    return y;
+}
+
+Tensor rows_linear(const Tensor& x, const Tensor& w,
+                   const optional<Tensor>& bias,
+                   const optional<Tensor>& resid,
+                   const optional<Tensor>& norm_w,
+                   const optional<Tensor>& norm_b,
+                   const optional<Tensor>& squares, double eps, int64_t act,
+                   bool keep32) {
+    Tensor none;
+    return rows_product(x, w, bias, resid, norm_w, norm_b, squares, eps, act,
+                        keep32, optional<Tensor>(), none, none);
+}
+
+// -> the result, its rows times then_w, the sums of squares
+std::tuple<Tensor, Tensor, Tensor> rows_sum(
+    const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
+    const optional<Tensor>& resid, const optional<Tensor>& norm_w,
+    const optional<Tensor>& norm_b, const optional<Tensor>& squares,
+    double eps, bool keep32, const Tensor& then_w) {
+    Tensor scaled, sums;
+    Tensor y = rows_product(x, w, bias, resid, norm_w, norm_b, squares, eps,
+                            EPI_PLAIN, keep32, then_w, scaled, sums);
+    return {y, scaled, sums};
 }
 
 // -> rotated queries [M, nq, hd]; rotated keys and the values go to the pages
@@ -312,6 +338,8 @@ Tensor embed_positions(const Tensor& ids, const Tensor& embed,
 void register_rows_ops(pybind11::module_& m) {
     m.def("rows_linear", &rows_linear,
           "projection of a few rows: norm, product, bias, activation, residual");
+    m.def("rows_sum", &rows_sum,
+          "the same without activation, and what the next RMS norm takes");
     m.def("rows_qkv", &rows_qkv,
           "norm, q|k|v projection, rotation and page store of a few rows");
     m.def("mid_linear", &mid_linear,
