@@ -589,8 +589,9 @@ class Runner:
             if chunked:
                 # chunked prefill: this chunk's K/V were just stored, so the
                 # kernel reads K/V exclusively from the paged cache and masks
-                # causally at absolute positions (HIP attn_prefill_mfma
-                # <HD, PAGED=true>; reference attn_decode_with_history on CPU)
+                # causally at absolute positions (HIP attn_stream for few
+                # rows, attn_flash for more; reference
+                # attn_decode_with_history on CPU)
                 return ops.attn_prefill_paged(
                     q, k_cache, v_cache, block_table, seq_lens, cu_seqlens,
                     max_seqlen, self.scale,

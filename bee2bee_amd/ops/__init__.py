@@ -11,11 +11,11 @@ decode attention, MFMA flash prefill attention, SwiGLU, top-k gating, grouped
 expert GEMM, projections of few rows with what stands around them. Other
 projection GEMMs go through hipBLASLt via torch.nn.functional.linear.
 
-Which projections are whose is measured: up to 16 rows (`few_rows`) the kernels
-of linear_rows.hip, one launch for norm, product and what follows; 17 to 160
-rows (`mid_rows`) narrow outputs by linear_mid.hip, split over K; wide outputs
-and more rows by the library (gate and up of 14336 x 4096 at 24 rows: 56 us
-there, 66 here). The grouped kernel driven as a single-segment GEMM loses to
+Which projections are whose is measured: up to 16 rows (`few_rows`; logits:
+`head_rows`) the kernels of linear_rows.hip, one launch for norm, product and
+what follows; 17 to 160 rows (`mid_rows`) outputs of `mid_shape` by
+linear_mid.hip, split over K; wide outputs and more rows by the library (gate
+and up of 14336 x 4096 at 24 rows: 56 us there, 66 here). The grouped kernel driven as a single-segment GEMM loses to
 the library on all shapes (scripts/bench_skinny.py: N/64 workgroups starve the
 chip); it stays for experts because the E-way grid and the device-side segment
 offsets are what the library cannot express.
@@ -309,7 +309,8 @@ def _deep(width: int, depth: int) -> bool:
 
 def deep_rows(x: torch.Tensor, inner: int) -> bool:
     """Steps of up to DEEP_MAX such rows whose down projection is at least
-    3.5 times as deep as wide."""
+    3.5 times as deep as wide (where the library's product is weak at these
+    rows; a matter of its choice of kernels, measured in linear_mid.hip)."""
     return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
             and x.dtype is torch.bfloat16 and x.is_contiguous()
             and _deep(x.shape[1], inner))

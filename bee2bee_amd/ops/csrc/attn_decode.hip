@@ -163,8 +163,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void attn_scores_kernel(
 
 // ----------------------------------------------------------- stage 2: PV
 // When FOLD (launcher sets it iff gridDim.z == 1, i.e. every chunk of this
-// (b, kvh) runs serially in THIS workgroup — always true at flagship batch
-// sizes where B*nkv >= 4096), the kernel carries the running flash-decoding
+// (b, kvh) runs serially in THIS workgroup: B*nkv >= 4096), the kernel carries the running flash-decoding
 // merge (M, l, acc) across chunks in registers and writes the normalized
 // bf16 output directly: no part_o round-trip, no combine kernel.
 template <int G, bool FOLD, typename KVT>

@@ -1,6 +1,7 @@
-// Projections of 17 to 160 rows whose output is narrow (q|k|v, attention
-// output, feed-forward output; the last, where it is deep, to 256): split over K, the splits' fp32 sums left to
-// the kernel that reads them anyway (qkv_rope_store, add_norm_parts).
+// Projections of 17 to 160 rows of up to 6144 outputs, or 3.5 times as deep as
+// wide (q|k|v, attention output, feed-forward output; the last, where it is
+// deep, to 256 rows): split over K, the splits' fp32 sums left to the kernel
+// that reads them anyway (qkv_rope_store, add_norm_parts).
 //
 // Bound by reading the weights once, by a chip that 64 columns a workgroup
 // would leave three quarters idle at 4096 of them (hence the split), and by
@@ -20,7 +21,15 @@
 // 3072x8192 27 / 32 / 36 (28 / 31 / 34), 3072x2048 11.6 / 13.7 / 15.5 (12 / 13
 // / 13), but 3584x18944 56 / 67 / 76 (107 / 123 / 127) and 2048x8192 18 / 21 /
 // 24 (26 / 27.5 / 26.5): above 160 rows only products 3.5 times as deep as
-// wide, and deeper.
+// wide, and deeper. Where that line lies is the library's doing and not a
+// property of the shapes: between 160 and 256 rows its products of 3584x18944
+// and 2048x8192 are half as fast as those of 4096x14336, where the gain of a
+// whole step is within 1%. Wider outputs (us, with the kernel that reads them;
+// 17 / 48 / 80 / 128 / 160 rows, the library's in brackets): 10240x8192, K not
+// split, 55 / 61 / 67 / 80 / 86 (43 / 48 / 80 / 64 / 72), 8192x8192 43 / 44 /
+// 46 / 52 / 57 (36 / 40 / 44 / 56 / 61), 8192x4096 23 / 24 / 27 / 32 / 34 (22 /
+// 24 / 30 / 33 / 35), 8192x28672 95 / 110 / 128 / 155 / 169 (99 / 179 / 198 /
+// 210 / 224).
 #include "common.h"
 
 constexpr int LM_W = 4;     // steps of weights under way, and the current one's

@@ -34,8 +34,8 @@
 //    layers of 3584, two rows: 1220 to 1290 us; of 4096, one row: 1014 to 1034).
 // Measured (us, one row, beside the library product alone): 6144x4096 15.3
 // (14.5), 4096x4096 9.3 (15.6), 2x14336x4096 44 (64), 4096x14336 25 (27),
-// 128256x4096 183 (190); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
-// 24, 182. With 16 rows 17, 11.6, 57, 34, 216: the input's reads add up, so
+// 128256x4096 182 (194); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
+// 24, 182. With 16 rows 17, 11.6, 57, 34, 200: the input's reads add up, so
 // more rows go to the library.
 #include "common.h"
 

@@ -110,9 +110,10 @@ def test_chunks_of_a_few_tokens(nq, nkv, hd, new, old, bs, fp8):
     _check(got, want, _wide(vc))
 
 
-def test_a_verified_token_gets_the_sums_of_decoding():
-    """A row's result is the same whether its token is decoded or verified
-    with others (16 rows in one tile either way)."""
+def test_the_last_verified_token_gets_the_sums_of_decoding():
+    """On bf16 pages, beside as many sequences in a table as wide, the result
+    of a sequence's last token is the same to the bit whether it is decoded or
+    verified with others (16 rows in one tile either way)."""
     total, new = [700, 1300], 3
     kc, vc, table, lens = _pages(8, 128, 256, total, False, 3)
     q = torch.randn(2 * new, 32, 128, device=DEV).bfloat16()
