@@ -368,17 +368,19 @@ class InferenceEngine:
 
     # -------------------------------------------------------------- serving
 
+    def _check_ids(self, ids) -> None:
+        """Ids past the vocabulary would be read from past the embedding, in
+        a step that other requests share."""
+        V = self.spec.vocab_size
+        if ids is not None and len(ids) and not (
+                0 <= min(ids) and max(ids) < V):
+            raise ValueError(f"token ids outside the vocabulary of {V}")
+
     def submit(self, req: GenerationRequest) -> GenerationRequest:
         # empty prompts become [bos] at admission (engine loop); <1
         # max_new behaves as 1 (prefill completion always emits one token)
         req.max_new_tokens = max(1, int(req.max_new_tokens))
-        # ids past the vocabulary would be read from past the embedding, in
-        # a step that other requests share
-        if req.prompt_ids and not (
-                0 <= min(req.prompt_ids)
-                and max(req.prompt_ids) < self.spec.vocab_size):
-            raise ValueError("prompt_ids outside the vocabulary of "
-                             f"{self.spec.vocab_size}")
+        self._check_ids(req.prompt_ids)
         self.start()
         self._pending.put(req)
         self._wake.set()
@@ -731,6 +733,8 @@ class InferenceEngine:
         after the call. Returns fp32 logits [n_wanted, vocab] in entry
         order (None if nothing is wanted). Not to be mixed with submit()
         traffic on the same engine."""
+        for _, toks, _ in entries:
+            self._check_ids(toks)
         fed = self.__dict__.setdefault("_fed", {})
         chunks, rows, base = [], [], 0
         for rid, toks, want in entries:

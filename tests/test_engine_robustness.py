@@ -448,6 +448,10 @@ def test_ids_outside_the_vocabulary_are_refused(small_engine, ids):
         small_engine.submit(_req(4, ids))
     _drain(beside)
     assert beside.error is None and len(beside.output_ids) == 6
+    eng = InferenceEngine("tiny", device="cpu", max_batch=2, max_seq_len=64)
+    with pytest.raises(ValueError):
+        eng.feed([(0, [1, 2], [1]), (1, list(ids), [0])])
+    assert not eng.__dict__.get("_fed")
 
 
 @pytest.mark.parametrize("spec_decode", [False, True])
