@@ -126,6 +126,9 @@ def _tp_worker(rank, world, port, few, out_path):
         out, lm_head = [], eng.runner.lm_head
         eng.runner.lm_head = lambda h: (out.append(lm_head(h)), out[-1])[1]
         tokens = eng.generate([[5, 6, 7, 8, 9], [100, 101]], 4)
+        # (a cycle would keep the engine, and so the process group's threads,
+        # until the interpreter is gone)
+        del eng.runner.lm_head
         if rank == 0:
             with open(out_path, "wb") as f:
                 pickle.dump((tokens, out), f)
