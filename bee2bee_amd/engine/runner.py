@@ -240,30 +240,33 @@ class Runner:
         lw = layers[self.layer_lo]
         normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
 
-        def add_norm(rows, w, bias, nxt, parts):
-            """x + rows w^T + bias, and its norm by nxt (None: no norm)."""
-            if parts:
-                return ops.add_norm_parts(ops.mid_linear(rows, w), bias, x,
-                                          nxt and (*nxt, s.rms_eps))
-            y = F.linear(rows, w, bias)
-            return ((None, x + y) if nxt is None
-                    else self._fused_add_norm(y, x, *nxt))
-
         for i in range(self.layer_lo, self.layer_hi):
             lw = layers[i]
             qkv = (ops.mid_linear(normed, lw.wqkv) if qkv_parts
                    else F.linear(normed, lw.wqkv))
             o = self._attend(i, qkv, positions, slot_mapping,
                              attn_fn).reshape(T, s.q_size)
-            normed, x = add_norm(o, lw.wo, lw.wo_bias,
-                                 (lw.mlp_norm, lw.mlp_norm_bias), o_parts)
+            if o_parts:
+                normed, x = ops.add_norm_parts(
+                    ops.mid_linear(o, lw.wo), lw.wo_bias, x,
+                    (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps))
+            else:
+                normed, x = self._fused_add_norm(
+                    F.linear(o, lw.wo, lw.wo_bias), x, lw.mlp_norm,
+                    lw.mlp_norm_bias)
             z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
             z = ops.gelu(z) if gelu else ops.swiglu(z)
-            nxt = None
-            if i + 1 < self.layer_hi:
-                nxt = layers[i + 1].attn_norm, layers[i + 1].attn_norm_bias
-            normed, x = add_norm(z, lw.w_down, lw.w_down_bias, nxt,
-                                 down_parts)
+            nxt = layers[i + 1] if i + 1 < self.layer_hi else None
+            if down_parts:
+                normed, x = ops.add_norm_parts(
+                    ops.mid_linear(z, lw.w_down), lw.w_down_bias, x,
+                    nxt and (nxt.attn_norm, nxt.attn_norm_bias, s.rms_eps))
+            else:
+                z = F.linear(z, lw.w_down, lw.w_down_bias)
+                if nxt is None:
+                    return x + z
+                normed, x = self._fused_add_norm(z, x, nxt.attn_norm,
+                                                 nxt.attn_norm_bias)
         return x
 
     def _rows_add(self, x, y, w, bias, nxt):

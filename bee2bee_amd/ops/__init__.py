@@ -15,10 +15,11 @@ Which projections are whose is measured: up to 16 rows (`few_rows`; logits:
 `head_rows`) the kernels of linear_rows.hip, one launch for norm, product and
 what follows; 17 to 160 rows (`mid_rows`) outputs of `mid_shape` by
 linear_mid.hip, split over K; wide outputs and more rows by the library (gate
-and up of 14336 x 4096 at 24 rows: 56 us there, 66 here). The grouped kernel driven as a single-segment GEMM loses to
-the library on all shapes (scripts/bench_skinny.py: N/64 workgroups starve the
-chip); it stays for experts because the E-way grid and the device-side segment
-offsets are what the library cannot express.
+and up of 14336 x 4096 at 24 rows: 56 us there, 66 here). The grouped kernel
+driven as a single-segment GEMM loses to the library on all shapes
+(scripts/bench_skinny.py: N/64 workgroups starve the chip); it stays for experts
+because the E-way grid and the device-side segment offsets are what the library
+cannot express.
 """
 from __future__ import annotations
 

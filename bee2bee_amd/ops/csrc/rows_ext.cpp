@@ -180,7 +180,8 @@ std::tuple<Tensor, Tensor, Tensor> rows_sum(
 // -> rotated queries [M, nq, hd]; rotated keys and the values go to the pages
 Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
                 const optional<Tensor>& norm_w, const optional<Tensor>& norm_b,
-                const optional<Tensor>& squares, double eps, int64_t nq, const optional<Tensor>& pos,
+                const optional<Tensor>& squares, double eps, int64_t nq,
+                const optional<Tensor>& pos,
                 const optional<Tensor>& cos_t, const optional<Tensor>& sin_t,
                 Tensor& k_cache, Tensor& v_cache, const Tensor& slots) {
     const Rows r = rows_of(x, w, norm_w, norm_b, squares);
@@ -206,7 +207,8 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
     TORCH_CHECK(launch_linear_rows(
                     r.x.data_ptr(), is_f32(r.x), ptr(r.norm_w),
                     ptr(r.norm_b), ptr(r.w), ptr(b), r.sq(), nullptr, 0,
-                    q.data_ptr(), 0, nullptr, nullptr, nullptr, r.M, r.N, r.K, (float)eps, r.norm, EPI_QKV,
+                    q.data_ptr(), 0, nullptr, nullptr, nullptr, r.M, r.N, r.K,
+                    (float)eps, r.norm, EPI_QKV,
                     pos.has_value() ? pos->data_ptr<int>() : nullptr,
                     pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
                     pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
