@@ -152,6 +152,10 @@ class Runner:
                 hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
                                          self.spec.rms_eps))
         normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
+        if self._mid_dims and (ops.mid_rows(normed) or ops.deep_rows(
+                normed, W.lm_head.shape[0])) and ops.mid_head(
+                    normed.shape[0], *W.lm_head.shape):
+            return ops.mid_rows_linear(normed, W.lm_head)
         return F.linear(normed, W.lm_head)
 
     def _run_layers_rows(
@@ -227,16 +231,19 @@ class Runner:
         slot_mapping: torch.Tensor,
         attn_fn,
     ) -> torch.Tensor:
-        """Dense layers on some tens of rows: the narrow projections
-        (ops.mid_shape) as parts over K, summed by the kernels that read them;
-        of more rows (ops.deep_rows) the down projection alone."""
+        """Dense layers on some tens of rows: projections as parts over K,
+        summed by the kernels that read them (ops.mid_shape), or activated where
+        they are made (ops.mid_gated, ops.mid_gelu)."""
         s, T = self.spec, x.shape[0]
         layers = self.weights.layers
-        gelu, all_parts = s.act_type == "gelu", ops.mid_rows(x)
-        H = s.hidden_size
-        qkv_parts = all_parts and ops.mid_shape(s.q_size + 2 * s.kv_size, H)
-        o_parts = all_parts and ops.mid_shape(H, s.q_size)
-        down_parts = ops.mid_shape(H, s.intermediate_size)
+        H, I = s.hidden_size, s.intermediate_size
+        qkv_parts = ops.mid_shape(T, s.q_size + 2 * s.kv_size, H)
+        o_parts = ops.mid_shape(T, H, s.q_size)
+        down_parts = ops.mid_shape(T, H, I)
+        gelu = s.act_type == "gelu"
+        act = "gelu" if gelu else "swiglu"
+        own_act = (ops.mid_gelu if gelu else ops.mid_gated)(T, I, H) and (
+            gelu or not s.mlp_bias)
         lw = layers[self.layer_lo]
         normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
 
@@ -254,8 +261,12 @@ class Runner:
                 normed, x = self._fused_add_norm(
                     F.linear(o, lw.wo, lw.wo_bias), x, lw.mlp_norm,
                     lw.mlp_norm_bias)
-            z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
-            z = ops.gelu(z) if gelu else ops.swiglu(z)
+            if own_act:
+                z = ops.mid_rows_linear(normed, lw.w_gate_up,
+                                        lw.w_gate_up_bias, act)
+            else:
+                z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
+                z = ops.gelu(z) if gelu else ops.swiglu(z)
             nxt = layers[i + 1] if i + 1 < self.layer_hi else None
             if down_parts:
                 normed, x = ops.add_norm_parts(

@@ -291,11 +291,12 @@ def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
                               k_cache, v_cache, slot_mapping)
 
 
-# Steps of some tens of rows: narrow projections as fp32 parts over their inner
-# dimension, which the next kernel sums.
+# Steps of some tens of rows: projections as fp32 parts over their inner
+# dimension, which the next kernel sums, or as activated bf16 rows.
 
-MID_MAX = 160
+MID_MAX = 128
 DEEP_MAX = 256
+DEEP_SIZE = 9_000_000
 
 
 def mid_rows(x: torch.Tensor) -> bool:
@@ -304,26 +305,71 @@ def mid_rows(x: torch.Tensor) -> bool:
             and x.dtype is torch.bfloat16 and x.is_contiguous())
 
 
-def _deep(width: int, depth: int) -> bool:
-    return depth * 2 >= 7 * width
-
-
 def deep_rows(x: torch.Tensor, inner: int) -> bool:
-    """Steps of up to DEEP_MAX such rows whose down projection is at least
-    3.5 times as deep as wide (where the library's product is weak at these
-    rows; a matter of its choice of kernels, measured in linear_mid.hip)."""
+    """Steps of up to DEEP_MAX such rows whose down projection has DEEP_SIZE
+    weights or more; mid_shape picks among the others."""
     return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
             and x.dtype is torch.bfloat16 and x.is_contiguous()
-            and _deep(x.shape[1], inner))
+            and x.shape[1] * inner >= DEEP_SIZE)
 
 
-def mid_shape(width: int, depth: int) -> bool:
-    """Projections that mid_linear takes: up to 6144 outputs, or deep ones.
-    Wider, K is split in two or not at all and the library wins: 10240 x 8192
-    with the rotation after it 55 us at 17 rows, 61 at 48, 80 at 128 (library
-    43, 48, 64), 8192 x 8192 with the add and norm 43, 44, 52 (36, 40, 56);
-    but 8192 x 28672 95, 110, 155 (99, 179, 210)."""
-    return width <= 6144 or _deep(width, depth)
+def mid_shape(rows: int, width: int, depth: int) -> bool:
+    """Projections that mid_linear takes, all up to MID_MAX rows, above it
+    those that outweigh their parts. Measured with the kernel that reads them
+    (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 16.9 (19.1)
+    / 26.1 (30.0) / 30.0 (30.4), 4096x14336 26.6 (32.8) / 35.3 (79) / 42.4
+    (59.6), 3584x18944 28.7 (112) / 39 (103) / 50 (127), 8192x8192 35.1 (34.6) /
+    44 (52.6) / 49 (57), 2048x2048 8.3 (10.9) / 12.0 (11.2) / 14.8 (12.2),
+    3072x2048 9.9 (15.0) / 14.7 (18.1) / 18.0 (16.6), 5120x3072 14.6 (16.4) /
+    22.5 (25.1) / 27.4 (24.1), 768x3072 7.7 (11.9) / 10.8 (10.4) / 12.8
+    (11.3)."""
+    return rows <= MID_MAX or width * depth >= (
+        16_000_000 if width > depth else DEEP_SIZE)
+
+
+def mid_gated(rows: int, width: int, depth: int) -> bool:
+    """Gated projections that mid_rows_linear takes (width: of one half). What
+    ends it is L2, from which a CU draws all input rows beside its share of the
+    weights. Measured beside the library's product and swiglu (us): 2x14336x4096
+    36.9 (56.7) at 24 rows, 50.8 (57.8) at 128, 64 (69.6) at 200, 78.6 (71.6) at
+    256; 2x18944x3584 44.6 (56.8), 60 (71.6), 68.6 (75.5) at 160, 113 (83) at
+    200; 2x8192x2048 14.2 (19.4), 20 (23.5), 26 (30), 29 (33) at 256; 2x2048x768
+    6.9 (9.4), 9.7 (10.4), 11.9 (10.3). More than 12 tiles of 8 columns a CU go
+    in rounds, each with a start of its own: 2x27648x5120 96 (100), 107 (105) at
+    48, 134 (123) at 128, but 2x28672x8192 141 (181), 153 (186), 194 (211)."""
+    tiles = -(-width // 2048)           # of 8 columns, a CU
+    if width * depth >= 1 << 30:        # the kernel's offsets are of 32 bits
+        return False
+    if tiles > 12:
+        return rows <= (MID_MAX if depth >= 8192 else 32)
+    if rows <= MID_MAX:
+        return True
+    if tiles > 8:
+        return rows <= 160
+    return width * depth >= 16_000_000 and rows <= (256 if tiles <= 4 else 224)
+
+
+def mid_gelu(rows: int, width: int, depth: int) -> bool:
+    """Projections with bias and gelu that mid_rows_linear takes: 3072x768 7.7 us
+    at 24 rows, 9.8 at 64 (library 9.8, 10.1), 8192x2048 12.3, 15.9 (15.9, 16.4),
+    20480x5120 45, 53 (45, 51)."""
+    return rows <= 64 and width <= 8192
+
+
+def mid_head(rows: int, width: int, depth: int) -> bool:
+    """Logits that mid_rows_linear takes. Groups of 8 tiles of 16 columns, a
+    CU's one after the other: where the last round leaves more than a twentieth
+    of the chip idle (152064 columns) the library is ahead above 64 rows. Beside
+    the library's product (us): 128256x4096 168 (193) at 24 rows, 195 (218) at
+    80, 230 (245) at 160, 304 (297) at 256; 152064x3584 172 (242), 218 (213);
+    32000x4096 41 (63), 48 (66), 58 (64); 128256x2048 84 (121), 103 (129); of
+    rows of 768 17.0 (18.6), 22.6 (20.8)."""
+    tiles = -(-width // 16)
+    rounds = -(-tiles // 2048)
+    full = 256 * rounds * -(-tiles // (256 * rounds))
+    if width % 4 or rows > 160 or (depth < 1024 and rows > 48):
+        return False
+    return rows <= 64 or tiles * 20 >= full * 19
 
 
 def mid_linear(x, w):
@@ -331,6 +377,14 @@ def mid_linear(x, w):
     if _use_hip(x):
         return require_hip().mid_linear(x, w)
     return reference.mid_linear(x, w)
+
+
+def mid_rows_linear(x, w, bias=None, act=None):
+    """act(x w^T + bias) of up to DEEP_MAX rows; act as in rows_linear (swiglu:
+    no bias)."""
+    if _use_hip(x):
+        return require_hip().mid_rows_linear(x, w, bias, _ACTS[act])
+    return reference.rows_linear(x, w, bias, act=act)
 
 
 def add_norm_parts(part, bias, resid, norm=None):

@@ -1,190 +1,398 @@
-// Projections of 17 to 160 rows of up to 6144 outputs, or 3.5 times as deep as
-// wide (q|k|v, attention output, feed-forward output; the last, where it is
-// deep, to 256 rows): split over K, the splits' fp32 sums left to the kernel
-// that reads them anyway (qkv_rope_store, add_norm_parts).
+// Projections of 17 to 256 rows, and the gated or activated ones and the output
+// head of such steps: x [M, K] times rows of w [N, K]. Three forms of result:
+//  parts   fp32 sums over S parts of K, left to the kernel that reads them
+//          anyway (qkv_rope_store, add_norm_parts): narrow projections, which
+//          would leave most of the chip idle unsplit;
+//  gated   silu(gate) * value in bf16 from w's two halves: the row tiles of w
+//          take 8 rows of each half, and lanes l and l + 32 hold a pair;
+//  rows    bf16, with bias and tanh-gelu where wanted (the output head, the
+//          feed-forward of the GPT-2 family).
 //
-// Bound by reading the weights once, by a chip that 64 columns a workgroup
-// would leave three quarters idle at 4096 of them (hence the split), and by
-// the latency of a step. A workgroup takes 64 rows of W and a part of K: four
-// waves of 16 rows, twice, for the two halves of that part. Weights go from
-// memory into the left operand as they lie, three steps ahead, the input rows
-// two steps ahead and then through LDS, shared by the four waves, xor-ed so
-// that the 16 rows of a read meet in no bank (LDS serves 256 bytes a clock).
-// Measured beside the library's product (us; 24 / 57 / 80 / 128 rows):
-// 4096x14336 26 / 29 / 33 / 40 (32 / 41 / 43 / 76), 4096x4096 10.2 / 11.2 / 13
-// / 16 (13.7 / 13.8 / 17 / 24), 6144x4096 14.7 / 17 / 19 / 24 (15 / 18 / 23 /
-// 25); with the input one step ahead, and twice the workgroups to hide that,
-// 27 / 31 / 34 / 42, 10.6 / 13 / 14 / 16, 15.4 / 18 / 20.5 / 24.5. Wide
-// outputs stay with the library (2x14336x4096: 66 here against 56 at 24 rows).
-// At 160 / 200 / 256 rows 4096x14336 46 / 54 / 62 (84 / 57 / 63), 6144x4096 26
-// / 31 / 35 (28 / 26 / 40), 4096x4096 17.5 / 20.5 / 23 (27 / 22 / 22.5),
-// 3072x8192 27 / 32 / 36 (28 / 31 / 34), 3072x2048 11.6 / 13.7 / 15.5 (12 / 13
-// / 13), but 3584x18944 56 / 67 / 76 (107 / 123 / 127) and 2048x8192 18 / 21 /
-// 24 (26 / 27.5 / 26.5): above 160 rows only products 3.5 times as deep as
-// wide, and deeper. Where that line lies is the library's doing and not a
-// property of the shapes: between 160 and 256 rows its products of 3584x18944
-// and 2048x8192 are half as fast as those of 4096x14336, where the gain of a
-// whole step is within 1%. Wider outputs (us, with the kernel that reads them;
-// 17 / 48 / 80 / 128 / 160 rows, the library's in brackets): 10240x8192, K not
-// split, 55 / 61 / 67 / 80 / 86 (43 / 48 / 80 / 64 / 72), 8192x8192 43 / 44 /
-// 46 / 52 / 57 (36 / 40 / 44 / 56 / 61), 8192x4096 23 / 24 / 27 / 32 / 34 (22 /
-// 24 / 30 / 33 / 35), 8192x28672 95 / 110 / 128 / 155 / 169 (99 / 179 / 198 /
-// 210 / 224).
+// Bound by reading the weights once, up to about 128 rows; beyond, by what a CU
+// draws from its L2 (weights and all input rows: about 19 bytes a clock and CU
+// at 200 rows). A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
+// workgroup's rows of w, and by all input rows. Four waves fill the one, four
+// the other, straight from memory (global_load_lds: no registers, so 100 KB of
+// loads are under way in each CU), and all eight multiply: the fragments of the
+// next half step are read while this one's products run. The weights carry the
+// streaming hint, so that they do not push the input out of L2 (2x14336x4096 at
+// 24 rows 40.8 us without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128
+// bytes in LDS are xor-ed by half their number: no two of a read's 16 rows meet
+// in a bank. Unsplit, workgroups start at different places of K (ROT): in step
+// they would all ask for the same few channels (44.8 -> 41.3 us at 24 rows, 53
+// -> 44.5 at 80; split, K = 14336, it loses: 22.9 -> 26.8).
+//
+// Measured beside the library's product and the kernel that reads it (us, 24 /
+// 80 / 128 / 200 / 256 rows; in brackets, the form before this one, which took
+// weights through registers):
+//   @T_PARTS@
 #include "common.h"
 
-constexpr int LM_W = 4;     // steps of weights under way, and the current one's
+enum { LM_PARTS = 0, LM_GATED = 1, LM_ROWS = 2 };
 
-template <int MT>
+DEV_INLINE unsigned lm_lds(const void* p) {
+    return (unsigned)(unsigned long)(
+        __attribute__((address_space(3))) const char*)p;
+}
+// 16 bytes a lane from base + off to LDS at `to` + lane * 16. The compiler does
+// not see these loads: lm_wait counts them. (M0 is set where it is used.)
+template <bool STREAM>
+DEV_INLINE void lm_load(const void* base, unsigned off, unsigned to) {
+    if constexpr (STREAM)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %0, %1 nt"
+                     ::"v"(off), "s"(base), "s"(to) : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %0, %1"
+                     ::"v"(off), "s"(base), "s"(to) : "memory");
+}
+// until at most `left` stages (R at most) of PER loads each are under way
+template <int PER, int R>
+DEV_INLINE void lm_wait(int left) {
+    if constexpr (R == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+        if (left >= R)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * R) : "memory");
+        else
+            lm_wait<PER, R - 1>(left);
+    }
+}
+
+// Waves: WN groups of TW tiles of 16 rows of w, by WM groups of MW tiles of 16
+// input rows, by WK halves of a step. DW, DX: slots of the rings. `tiles` of
+// the TW * WN are used. WK 1: a workgroup takes every gridDim.x-th group of
+// tiles, loading the next one's first steps under this one's last.
+template <int TW, int MW, int WN, int WM, int WK, int DW, int DX, int OUT>
 __global__ __launch_bounds__(512) void linear_mid_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
-    float* __restrict__ part, int M, int N, int K, int S) {
-    constexpr int MP = MT * 16;
-    constexpr int XB = 2 * MP * 128;       // bytes of a staged buffer: [half]
-                                           // [row][64 of K]
-    constexpr int NLD = MT / 2;            // 16-byte chunks a thread stages
+    const unsigned short* __restrict__ bias, void* __restrict__ out, int M,
+    int N, int K, int S, int tiles, int gelu) {
+    constexpr int T = TW * WN, MT = MW * WM;
+    static_assert(WN * WM * WK == 8 && DW >= 2 && DX >= 2, "");
+    constexpr int NLW = T / 2, NLX = (MT + 1) / 2;  // loads of a wave a step
+    constexpr int WB = NLW * 4096, XB = NLX * 4096; // bytes of a slot
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    const int rw = wid & 3, kh = wid >> 2; // row tile, half of the K part
-    const int n0 = blockIdx.x * 64 + rw * 16;
-    // steps of 64 along K: of the workgroup, of its first half, of this wave
-    const int CH = K / 64;
-    const int c0 = CH * blockIdx.y / S, c1 = CH * (blockIdx.y + 1) / S;
-    const int first = (c1 - c0 + 1) / 2;
-    const int my0 = kh ? c0 + first : c0;
-    const int mine = kh ? c1 - c0 - first : first;
-
+    const int wn = wid % WN, wm = wid / WN % WM, wk = wid / WN / WM;
+    const int NT = OUT == LM_GATED ? N / 8 : (N + 15) / 16;
+    const int NG = (NT + tiles - 1) / tiles;
+    const int CH = K / 64;                     // steps of 64: of them
+    const int c0 = CH * blockIdx.y / S, n = CH * (blockIdx.y + 1) / S - c0;
+    const int rot = (blockIdx.x / 8) % n;      // where it starts
+    int g = blockIdx.x;
+    const int total = n * ((NG - 1 - g) / (int)gridDim.x + 1);
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const unsigned short* wp = w + (long)min(n0 + li, N - 1) * K + lg * 8;
-    const unsigned short* xs[NLD];
-    int xd[NLD], xlast[NLD];
+    // ---- loads: a wave's load is 8 rows of 128 bytes, lane l the chunk of 16
+    // bytes that belongs at l * 16
+    const bool of_w = wid < 4;
+    const int r8 = lane >> 3, p8 = lane & 7;
+    unsigned off[NLW > NLX ? NLW : NLX];
+    const char* src = reinterpret_cast<const char*>(of_w ? w : x);
+    auto rows_of = [&](int grp) {              // (tiles past the last: its)
+        const int t0 = grp * tiles;
+        if (OUT != LM_GATED)
+            src = reinterpret_cast<const char*>(w + (long)t0 * 16 * K);
 #pragma unroll
-    for (int j = 0; j < NLD; ++j) {
-        const int i = tid + 512 * j, c = i & 7;
-        const int row = (i >> 3) % MP, h = (i >> 3) / MP;
-        xs[j] = x + (long)min(row, M - 1) * K +
-                (long)(h ? c0 + first : c0) * 64 + c * 8;
-        xlast[j] = (h ? c1 - c0 - first : first) - 1;
-        xd[j] = (h * MP + row) * 128 + ((c ^ (row >> 1 & 7)) << 4);
+        for (int j = 0; j < NLW; ++j) {
+            const int i = wid * NLW + j;
+            const int r = (i & 1) * 8 + r8;
+            const int t = min(t0 + min(i >> 1, tiles - 1), NT - 1);
+            const long row = OUT == LM_GATED
+                                 ? (long)t * 8 + r8 + (i & 1) * (long)N
+                                 : min(t * 16 + r, N - 1) - t0 * 16;
+            off[j] = (unsigned)((row * K + (p8 ^ (r >> 1 & 7)) * 8) * 2);
+        }
+    };
+    if (of_w) {
+        rows_of(g);
+    } else {
+#pragma unroll
+        for (int j = 0; j < NLX; ++j) {
+            const int r = ((wid - 4) * NLX + j) * 8 + r8;
+            off[j] = (unsigned)(((long)min(r, M - 1) * K +
+                                 (p8 ^ (r >> 1 & 7)) * 8) * 2);
+        }
     }
-    // (a half without steps left loads, and ignores, a step of the other)
-    bf16x8 xr[2][NLD];
-    auto load_x = [&](int set, int it) {
+    const unsigned to0 = lm_lds(smem) +
+                         (of_w ? wid * NLW * 1024
+                               : DW * WB + (wid - 4) * NLX * 1024);
+    int lk = rot, lleft = n, lgrp = g, lslot = 0;
+    auto issue = [&]() {                       // the next stage's loads
+        const char* b = src + (long)(c0 + lk) * 128;
+        if (of_w) {
 #pragma unroll
-        for (int j = 0; j < NLD; ++j)
-            xr[set][j] = *reinterpret_cast<const bf16x8*>(
-                xs[j] + (long)min(it, xlast[j]) * 64);
+            for (int j = 0; j < NLW; ++j)
+                lm_load<true>(b, off[j], to0 + lslot * WB + j * 1024);
+            if (++lslot == DW) lslot = 0;
+        } else {
+#pragma unroll
+            for (int j = 0; j < NLX; ++j)
+                lm_load<false>(b, off[j], to0 + lslot * XB + j * 1024);
+            if (++lslot == DX) lslot = 0;
+        }
+        if (++lk == n) lk = 0;
+        if (WK == 1 && --lleft == 0) {
+            lleft = n;
+            lgrp += gridDim.x;
+            if (of_w && lgrp < NG) rows_of(lgrp);
+        }
     };
-    auto store_x = [&](int set) {          // into the buffer of its number
-#pragma unroll
-        for (int j = 0; j < NLD; ++j)
-            *reinterpret_cast<bf16x8*>(smem + set * XB + xd[j]) = xr[set][j];
-    };
-    bf16x8 aw[LM_W][2];
-    auto load_w = [&](int set, int it) {
-        const long k = (long)min(my0 + it, CH - 1) * 64;
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            aw[set][s] = *reinterpret_cast<const bf16x8*>(wp + k + s * 32);
-    };
-    f32x4 acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int D = of_w ? DW : DX;
+    for (int i = 0; i < D && i < total; ++i) issue();
 
-    load_x(0, 0);
+    // ---- products
+    f32x4 acc[TW][MW];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < LM_W - 1; ++i) load_w(i, i);
-    load_x(1, 1);
-    store_x(0);
-    __syncthreads();
-    const char* xb = smem + kh * MP * 128 + li * 128;
-    // step `it` with `it` % LM_W == j: the input of the step after the next
-    // and weights of LM_W - 1 later ones set out, the next step's input goes
-    // to LDS. No load stands under a condition: what is under way would have
-    // to be waited for where the two ways meet.
-    auto step = [&](int j, int it) {
-        load_x(j & 1, it + 2);
-        load_w((j + LM_W - 1) % LM_W, it + LM_W - 1);
-        if (it < mine) {
-            const char* b = xb + (j & 1) * XB;
+        for (int t = 0; t < TW; ++t)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    const bf16x8 bx = *reinterpret_cast<const bf16x8*>(
-                        b + m * 16 * 128 +
-                        (((s * 4 + lg) ^ (li >> 1)) << 4));
-                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        aw[j][s], bx, acc[m], 0, 0, 0);
-                }
-        }
-        store_x((j + 1) & 1);
-        __syncthreads();
+            for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
-    for (int it = 0;;) {
+    clear();
+    bf16x8 fw[2][TW], fx[2][MW];
+    const char* wf = smem + (wn * TW * 16 + li) * 128;
+    const char* xf = smem + DW * WB + (wm * MW * 16 + li) * 128;
+    int ws = 0, xs = 0;                        // slots read from
+    auto read = [&](int set, int half) {
+        const int pos = ((half * 4 + lg) ^ (li >> 1)) << 4;
 #pragma unroll
-        for (int j = 0; j < LM_W; ++j) {
-            step(j, it);
-            if (++it >= first) goto done;
+        for (int t = 0; t < TW; ++t)
+            fw[set][t] = *reinterpret_cast<const bf16x8*>(
+                wf + ws * WB + pos + t * 2048);
+#pragma unroll
+        for (int m = 0; m < MW; ++m)
+            fx[set][m] = *reinterpret_cast<const bf16x8*>(
+                xf + xs * XB + pos + m * 2048);
+    };
+    auto products = [&](int set) {
+#pragma unroll
+        for (int m = 0; m < MW; ++m)
+#pragma unroll
+            for (int t = 0; t < TW; ++t)
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    fw[set][t], fx[set][m], acc[t][m], 0, 0, 0);
+    };
+    // (the builtin: the compiler has to know that nothing is under way, or it
+    // waits for what was only just asked for)
+    auto fragments_here = [&]() { __builtin_amdgcn_s_waitcnt(0xc07f); };
+    // Stage s is read by everyone, so its slot is free; stage s + 1 has come.
+    // (Loads of min(total, s + D) stages have been issued.)
+    auto advance = [&](int s) {
+        if (++ws == DW) ws = 0;
+        if (++xs == DX) xs = 0;
+        if (s + 1 == total) return false;
+        const int left = min(total - 2 - s, D - 2);
+        if (of_w) lm_wait<NLW, DW - 2>(left);
+        else lm_wait<NLX, DX - 2>(left);
+        asm volatile("s_barrier" ::: "memory");
+        if (s + D < total) issue();
+        return true;
+    };
+    auto finish = [&](int grp) {
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int tt = wn * TW + t, tile = grp * tiles + tt;
+            if (tt >= tiles || tile >= NT) continue;
+            // C layout: column li = input row, rows lg * 4 + r = columns
+            const int col = OUT == LM_GATED ? tile * 8 + lg * 4
+                                            : tile * 16 + lg * 4;
+#pragma unroll
+            for (int m = 0; m < MW; ++m) {
+                const int row = (wm * MW + m) * 16 + li;
+                f32x4 z = acc[t][m];
+                if (OUT == LM_GATED) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float2v p = lane_pair(acc[t][m][r]);
+                        z[r] = p.x / (1.f + __expf(-p.x)) * p.y;
+                    }
+                }
+                if (row >= M || (OUT == LM_GATED ? lane >= 32 : col >= N))
+                    continue;
+                if (OUT == LM_PARTS) {
+                    *reinterpret_cast<f32x4*>(
+                        reinterpret_cast<float*>(out) +
+                        ((long)blockIdx.y * M + row) * N + col) = z;
+                    continue;
+                }
+                if (OUT == LM_ROWS) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (bias) z[r] += bf2f(bias[col + r]);
+                        if (gelu) {
+                            // (1 + tanh c) / 2 = 1 / (1 + exp(-2 c))
+                            const float c = 0.7978845608028654f *
+                                            (z[r] + 0.044715f * z[r] * z[r] *
+                                                        z[r]);
+                            z[r] = z[r] / (1.f + __expf(-2.f * c));
+                        }
+                    }
+                }
+                *reinterpret_cast<uint2v*>(
+                    reinterpret_cast<unsigned short*>(out) + (long)row * N +
+                    col) =
+                    uint2v{f2bf(z[0]) | (unsigned)f2bf(z[1]) << 16,
+                           f2bf(z[2]) | (unsigned)f2bf(z[3]) << 16};
+            }
         }
+    };
+    if (of_w) lm_wait<NLW, DW - 1>(min(total, DW) - 1);
+    else lm_wait<NLX, DX - 1>(min(total, DX) - 1);
+    asm volatile("s_barrier" ::: "memory");
+    read(0, WK == 2 ? wk : 0);
+    int left = n;                              // steps of this group
+    auto step = [&](int set, int s) {
+        fragments_here();
+        if (WK == 2) {
+            if (advance(s)) read(set ^ 1, wk);
+            products(set);
+            return;
+        }
+        read(1, 1);
+        products(0);
+        fragments_here();
+        if (advance(s)) read(0, 0);
+        products(1);
+        if (--left == 0) {
+            finish(g);
+            g += gridDim.x;
+            left = n;
+            clear();
+        }
+    };
+    for (int s = 0;;) {
+        step(0, s);
+        if (++s >= total) break;
+        step(1, s);
+        if (++s >= total) break;
     }
-done:
-    // ---- the halves' sums meet in LDS
-    f32x4* mg = reinterpret_cast<f32x4*>(smem) + rw * MT * 64 + lane;
-    if (kh == 1) {
+    if (WK == 1) return;
+    // the halves' sums meet in LDS (every load has come, and been read)
+    __syncthreads();
+    f32x4* mg = reinterpret_cast<f32x4*>(smem) +
+                wid % (WN * WM) * TW * MW * 64 + lane;
+    if (wk == 1) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) mg[m * 64] = acc[m];
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int m = 0; m < MW; ++m) mg[(t * MW + m) * 64] = acc[t][m];
     }
     __syncthreads();
-    const int n = n0 + lg * 4;
-    if (kh == 1 || n >= N) return;
+    if (wk == 1) return;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int row = m * 16 + li;
-        if (row >= M) continue;
-        const f32x4 p = mg[m * 64];
-        f32x4 v;
+    for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = acc[m][r] + p[r];
-        *reinterpret_cast<f32x4*>(
-            part + ((long)blockIdx.y * M + row) * N + n) = v;
-    }
+        for (int m = 0; m < MW; ++m) {
+            const f32x4 p = mg[(t * MW + m) * 64];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][m][r] += p[r];
+        }
+    finish(g);
 }
 
-// Splits of K: up to a workgroup a CU, at least four steps of 64 a half. Two
-// workgroups a CU: 4096x14336 at 80 rows 36 us against 32.6, 6144x4096 21.5
-// against 18.9, 4096x4096 15.2 against 12.9, and the reader has twice the
-// parts.
+// Tiles of 16 rows of w in a workgroup, as few as a chip of 256 CUs leaves it
+// with `S` parts of K; `most` of them at most (then more workgroups than CUs,
+// or rounds).
+static int lm_tiles(int NT, int S, int most) {
+    const int cus = 256 / S;
+    const int rounds = (NT + cus * most - 1) / (cus * most);
+    return (NT + cus * rounds - 1) / (cus * rounds);
+}
+
+// Parts of K: as many as leave a workgroup at most 8 tiles and, of K, twice as
+// many steps of 64 as it has tiles (and 6), so that the parts, written and read
+// once more, stay below the weights. Measured with the kernel that reads them
+// (us, 24 / 200 rows): @T_SPLIT@
 extern "C" int linear_mid_splits(int N, int K) {
-    const int tiles = (N + 63) / 64;
+    const int NT = (N + 15) / 16;
     int S = 1;
-    while (S < 8 && tiles * S * 2 <= 256 && K / 64 >= S * 16) S *= 2;
+    for (int s = 2; s <= 8; s *= 2) {
+        const int tiles = (NT + 256 / s - 1) / (256 / s);
+        const int n = K / 64 / s;
+        if (tiles <= 8 && n >= 6 && n >= 2 * tiles) S = s;
+    }
     return S;
 }
 
-// part [S, M, N] fp32: x [M, K] times rows of w [N, K] over S parts of K. x and
-// w contiguous and 16-byte aligned, 1 <= M <= 256, N % 4 == 0, K % 64 == 0, S
-// <= K / 64; nonzero for anything else.
+// x [M, K] and w contiguous and 16-byte aligned, 1 <= M <= 256, K % 64 == 0.
+// out: form LM_PARTS [S, M, N] fp32, 1 <= S <= K / 64; LM_GATED [M, N] bf16, w
+// [2N, K], N % 8 == 0, S 1, no bias; LM_ROWS [M, N] bf16, S 1. N % 4 == 0.
+// Nonzero for anything else.
 extern "C" int launch_linear_mid(const unsigned short* x,
-                                 const unsigned short* w, float* part, int M,
-                                 int N, int K, int S, hipStream_t stream) {
+                                 const unsigned short* w,
+                                 const unsigned short* bias, void* out, int M,
+                                 int N, int K, int S, int form, int gelu,
+                                 hipStream_t stream) {
     if (M < 1 || M > 256 || N < 4 || N % 4 || K < 64 || K % 64) return 1;
-    if (S < 1 || S > K / 64) return 1;
-    const dim3 grid((N + 63) / 64, S);
-#define LM_GO(MTV)                                                            \
-    hipLaunchKernelGGL((linear_mid_kernel<MTV>), grid, dim3(512),             \
-                       2 * 2 * MTV * 16 * 128, stream, x, w, part, M, N, K, S)
-    if (M <= 32) LM_GO(2);
-    else if (M <= 64) LM_GO(4);
-    else if (M <= 96) LM_GO(6);
-    else if (M <= 128) LM_GO(8);
-    else if (M <= 160) LM_GO(10);
-    else if (M <= 192) LM_GO(12);
-    else if (M <= 224) LM_GO(14);
-    else LM_GO(16);
+    if (S < 1 || S > K / 64 || (form != LM_PARTS && S != 1)) return 1;
+    if (form == LM_GATED && N % 8) return 1;
+    // offsets are of 32 bits
+    if (form == LM_GATED && ((long)2 * N * K * 2) >> 32) return 1;
+    const int NT = form == LM_GATED ? N / 8 : (N + 15) / 16;
+    // 12 tiles and all rows' sums fit the registers of up to 160 rows
+    const int most = form == LM_GATED && M <= 160 && NT > 2048 && NT <= 3072
+                         ? 12 : 8;
+    const int tiles = lm_tiles(NT, S, most);
+    const int NG = (NT + tiles - 1) / tiles;
+    const bool once = NG * S <= 256;           // no second group of tiles
+#define LM_GO(TW, MW, WN, WM, WK, DW, DX, F)                                  \
+    do {                                                                      \
+        constexpr int lds =                                                   \
+            DW * (TW * WN / 2) * 4096 + DX * ((MW * WM + 1) / 2) * 4096;      \
+        static_assert(lds <= 163840, "LDS of a CU");                          \
+        static_assert(WK == 1 || TW * MW * 1024 * 4 <= lds, "halves");        \
+        hipLaunchKernelGGL(                                                   \
+            (linear_mid_kernel<TW, MW, WN, WM, WK, DW, DX, F>),               \
+            dim3(WK == 1 && !once ? 256 / S : NG, S), dim3(512),              \
+            lds, stream, x, w, bias, out, M, N, K, S, tiles, gelu);           \
+        return 0;                                                             \
+    } while (0)
+#define LM_4(F)                                                               \
+    do {                                                                      \
+        if (M <= 32) LM_GO(1, 2, 4, 1, 2, 12, 6, F);                          \
+        if (M <= 64) LM_GO(1, 4, 4, 1, 2, 12, 6, F);                          \
+        if (M <= 96) LM_GO(2, 3, 2, 2, 2, 10, 5, F);                          \
+        if (M <= 128) LM_GO(2, 4, 2, 2, 2, 10, 4, F);                         \
+        if (M <= 160) LM_GO(2, 5, 2, 2, 2, 8, 4, F);                          \
+        if (M <= 192) LM_GO(2, 6, 2, 2, 2, 8, 4, F);                          \
+        if (M <= 224) LM_GO(2, 7, 2, 2, 2, 7, 3, F);                          \
+        LM_GO(2, 8, 2, 2, 2, 7, 3, F);                                        \
+    } while (0)
+#define LM_8(F)                                                               \
+    do {                                                                      \
+        if (M <= 32) LM_GO(1, 2, 8, 1, 1, 7, 4, F);                           \
+        if (M <= 64) LM_GO(1, 4, 8, 1, 1, 7, 4, F);                           \
+        if (M <= 96 && once) LM_GO(2, 6, 4, 1, 2, 7, 3, F);                   \
+        if (M <= 96) LM_GO(1, 6, 8, 1, 1, 7, 3, F);                           \
+        if (M <= 128) LM_GO(2, 4, 4, 2, 1, 6, 3, F);                          \
+        if (M <= 160) LM_GO(2, 5, 4, 2, 1, 6, 3, F);                          \
+        if (M <= 192 && once) LM_GO(4, 6, 2, 2, 2, 5, 3, F);                  \
+        if (M <= 224 && once) LM_GO(4, 7, 2, 2, 2, 4, 3, F);                  \
+        if (M <= 192) LM_GO(2, 6, 4, 2, 1, 5, 3, F);                          \
+        if (M <= 224) LM_GO(2, 7, 4, 2, 1, 4, 3, F);                          \
+        LM_GO(2, 8, 4, 2, 1, 4, 3, F);                                        \
+    } while (0)
+    if (form == LM_GATED && tiles > 8) {
+        if (M <= 32) LM_GO(3, 2, 4, 1, 2, 6, 3, LM_GATED);
+        if (M <= 64) LM_GO(3, 4, 4, 1, 2, 5, 3, LM_GATED);
+        if (M <= 96) LM_GO(3, 3, 4, 2, 1, 5, 3, LM_GATED);
+        if (M <= 128) LM_GO(3, 4, 4, 2, 1, 4, 3, LM_GATED);
+        LM_GO(3, 5, 4, 2, 1, 4, 3, LM_GATED);
+    }
+    if (form == LM_GATED && tiles <= 4) LM_4(LM_GATED);
+    if (form == LM_GATED) LM_8(LM_GATED);
+    if (form == LM_ROWS && tiles <= 4) LM_4(LM_ROWS);
+    if (form == LM_ROWS) LM_8(LM_ROWS);
+    if (tiles <= 4) LM_4(LM_PARTS);
+    LM_8(LM_PARTS);
+#undef LM_8
+#undef LM_4
 #undef LM_GO
-    return 0;
+    return 1;
 }
 
 // ----------------------------------------------------------- add_norm_parts

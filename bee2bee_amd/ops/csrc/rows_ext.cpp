@@ -15,7 +15,8 @@ extern "C" int launch_linear_rows(
     void*, void*, int, int, int, int, int, hipStream_t);
 extern "C" int linear_mid_splits(int, int);
 extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
-                                 float*, int, int, int, int, hipStream_t);
+                                 const unsigned short*, void*, int, int, int,
+                                 int, int, int, hipStream_t);
 extern "C" int launch_add_norm_parts(
     const float*, const unsigned short*, const unsigned short*,
     const unsigned short*, const unsigned short*, unsigned short*,
@@ -228,9 +229,30 @@ Tensor mid_linear(const Tensor& x, const Tensor& w) {
     const int S = linear_mid_splits(N, K);
     Tensor part = torch::empty({S, M, N},
                                x.options().dtype(torch::kFloat32));
-    TORCH_CHECK(launch_linear_mid(ptr(xd), ptr(wd), part.data_ptr<float>(), M,
-                                  N, K, S, stream()) == 0);
+    TORCH_CHECK(launch_linear_mid(ptr(xd), ptr(wd), nullptr, part.data_ptr(),
+                                  M, N, K, S, 0, 0, stream()) == 0);
     return part;
+}
+
+// act(x w^T + bias) in bf16; act swiglu: w holds the gate's rows, then the
+// values'
+Tensor mid_rows_linear(const Tensor& x, const Tensor& w,
+                       const optional<Tensor>& bias, int64_t act) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
+                "x [M, K] and w [N, K]");
+    TORCH_CHECK(act == EPI_PLAIN || act == EPI_GLU || act == EPI_GELU);
+    const bool glu = act == EPI_GLU;
+    TORCH_CHECK(!glu || (w.size(0) % 16 == 0 && !bias.has_value()));
+    const int M = x.size(0), K = x.size(1), N = w.size(0) / (glu ? 2 : 1);
+    TORCH_CHECK(M >= 1 && M <= 256, "1 to 256 rows");
+    TORCH_CHECK(K % 64 == 0 && N % 4 == 0);
+    const Tensor xd = dense(x, "x"), wd = dense(w, "w"),
+                 b = column(bias, N, "bias");
+    Tensor y = torch::empty({M, N}, xd.options());
+    TORCH_CHECK(launch_linear_mid(ptr(xd), ptr(wd), ptr(b), y.data_ptr(), M,
+                                  N, K, 1, glu ? 1 : 2, act == EPI_GELU,
+                                  stream()) == 0);
+    return y;
 }
 
 const float* parts(const Tensor& t, long M, long N) {
@@ -346,6 +368,8 @@ void register_rows_ops(pybind11::module_& m) {
           "norm, q|k|v projection, rotation and page store of a few rows");
     m.def("mid_linear", &mid_linear,
           "projection of some tens of rows as fp32 parts over K");
+    m.def("mid_rows_linear", &mid_rows_linear,
+          "projection of some tens of rows, with bias and activation");
     m.def("add_norm_parts", &add_norm_parts,
           "residual add of a projection's parts, and the next norm");
     m.def("decode_slots", &decode_slots, "page slots of a decode step's rows");

@@ -213,7 +213,8 @@ def test_refused():
 @pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128, 129, 160,
                                161, 200, 256])
 @pytest.mark.parametrize("N,K", [(64, 64), (68, 1088), (3584, 960),
-                                 (4096, 2048), (512, 8192 + 64)])
+                                 (4096, 2048), (512, 8192 + 64), (6148, 3072),
+                                 (33004, 64)])
 def test_parts_over_k(M, N, K):
     """Products of bf16 numbers are exact in fp32: only the order of the sums
     differs, at most K roundings of a partial sum."""
@@ -223,6 +224,38 @@ def test_parts_over_k(M, N, K):
     want = x.double() @ w.double().t()
     mag = x.double().abs() @ w.double().abs().t()
     assert ((part.double().sum(0) - want).abs() <= 2 ** -24 * K * mag).all()
+
+
+# (tiles a workgroup takes: 1 to 4, 5 to 8, 9 to 12, and several groups of
+# them; steps of K fewer than the rings' slots, and more)
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128, 129, 160,
+                               161, 192, 193, 224, 225, 256])
+@pytest.mark.parametrize("N,K,act", [
+    (8, 64, "swiglu"), (2056, 1088, "swiglu"), (9000, 192, "swiglu"),
+    (17000, 704, "swiglu"), (25000, 128, "swiglu"), (4, 64, None),
+    (3072, 768, "gelu"), (8204, 320, "gelu"), (33004, 576, None)])
+def test_activated_rows(M, N, K, act):
+    """Products are exact in fp32, their sums off by K roundings at most; an
+    activation's slope is below 1.13, and the result is rounded to bf16."""
+    torch.manual_seed(M + N)
+    x, w = _rand(M, K), _rand(2 * N if act == "swiglu" else N, K, std=0.1)
+    bias = _rand(N) if act == "gelu" else None
+    got = ops.mid_rows_linear(x, w, bias, act).double()
+    z = x.double() @ w.double().t()
+    e = 2 ** -24 * K * (x.double().abs() @ w.double().abs().t())
+    if act == "swiglu":
+        g, u = z.chunk(2, -1)
+        eg, eu = e.chunk(2, -1)
+        want = F.silu(g) * u
+        e = 1.13 * eg * u.abs() + F.silu(g).abs() * eu + 1.13 * eg * eu
+    elif act == "gelu":
+        want = F.gelu(z + bias.double(), approximate="tanh")
+        e = 1.13 * (e + 2 ** -23 * (z.abs() + bias.double().abs()))
+    else:
+        want = z
+    # (exp in fp32: 2^-20 covers its argument's rounding)
+    assert ((got - want).abs() <= e + (2 ** -8 + 2 ** -20) * want.abs()
+            + 1e-6).all()
 
 
 @pytest.mark.parametrize("S,M,H", [(1, 17, 64), (8, 128, 4096), (4, 20, 8192),
