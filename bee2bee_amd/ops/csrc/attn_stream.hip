@@ -2,8 +2,9 @@
 // chunks of a few tokens that speculative decoding verifies.
 //
 // Bound by reading the cache once. A wave takes tiles of 32 keys on its own:
-// whole 16-byte chunks of neighbouring rows into registers (1 KB a load), on
-// to its part of LDS, the next tile's loads on their way over the products of
+// whole 16-byte chunks of neighbouring rows into registers (1 KB a load, with
+// the streaming hint: 1536 sequences below 653 us without it), on to its part
+// of LDS, the next tile's loads on their way over the products of
 // this one, no barrier before the end. Scores are S^T = K Q^T on 16x16x32
 // matrix tiles (a column is a query row; the rows of all heads that share the
 // key head, times the chunk's tokens), so that the weights are, as they
@@ -15,9 +16,11 @@
 // are not).
 // Measured against the kernels before it (scores, weights through memory,
 // values, combine): 1536 sequences of 137..1100 tokens, 8 key heads of size
-// 128: 652 us (5.98 TB/s) instead of 778; fp8 361 instead of 588; 200
-// sequences of up to 3000 fp8 132 instead of 228; one of 3000 8.6 instead of
-// 15.3; 16 sequences' 5 tokens on 1500 26 instead of 166.
+// 128: 595 us (6.55 TB/s) instead of 778; fp8 337 (5.8) instead of 588; 200
+// sequences of up to 3000 fp8 120 instead of 228 (122.8 with 8 bytes a lane);
+// one of 3000 8.5 instead of 15.3; 16 sequences' 5 tokens on 1500 24 instead
+// of 166. Loads two tiles ahead gain nothing on fp8 rows (121) and spill on
+// others.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) short short4v;
@@ -28,10 +31,9 @@ constexpr int ST_KEYS = 32;                      // keys of a wave's tile
 constexpr int ST_STEP = ST_WAVES * ST_KEYS;      // keys of a workgroup's step
 constexpr float ST_LOG2E = 1.44269504088896340736f;
 
-// 16 bytes of a bf16 row, or 8 of an fp8 row, as read
-template <typename KVT> struct st_raw { using type = short8; };
-template <> struct st_raw<unsigned char> { using type = uint2v; };
-DEV_INLINE short8 st_widen(short8 x) { return x; }
+// 16 bytes of a row, as read
+typedef __attribute__((ext_vector_type(4))) unsigned int st_raw;
+
 DEV_INLINE short8 st_widen(uint2v x) {
     typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
     bf16x8 r;
@@ -48,6 +50,12 @@ DEV_INLINE short8 st_widen(uint2v x) {
         r[i * 4 + 3] = b[1];
     }
     return __builtin_bit_cast(short8, r);
+}
+
+// elements 8 p .. 8 p + 7 of a load, in bf16
+template <typename KVT> DEV_INLINE short8 st_piece(st_raw x, int p) {
+    if constexpr (sizeof(KVT) == 2) return __builtin_bit_cast(short8, x);
+    else return st_widen(uint2v{x[p * 2], x[p * 2 + 1]});
 }
 
 // 8 queries times the score scale, rounded to fp8
@@ -80,7 +88,8 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     float scale) {
     constexpr int KS = HD / 32;          // k steps of a score tile
     constexpr int DT = HD / 16;          // output tiles of 16 coordinates
-    constexpr int CPR = HD / 8;          // chunks of 8 elements of a key row
+    constexpr int PC = 2 / sizeof(KVT);  // chunks of 8 elements of a load
+    constexpr int CPR = HD / 8 / PC;     // loads of a key row
     constexpr int RB = HD * 2;           // bytes of a staged row
     constexpr int RPI = 64 / CPR;        // rows a wave loads at once
     constexpr int NL = ST_KEYS / RPI;    // loads of a tile
@@ -92,7 +101,6 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     auto v_swz = [](int row) {
         return 2 * (HD == 128 ? row & 7 : (row >> 1) & 3);
     };
-    using raw_t = typename st_raw<KVT>::type;
 
     const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
     const int s0 = cu ? cu[b] : b;
@@ -141,9 +149,10 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     }
     const int first_see = hist + row0 / G;
 
-    // ---- loading: lane -> (row of RPI, chunk)
-    const int ld_row = lane / CPR, ld_c = lane % CPR;
-    raw_t rk[NL], rv[NL];
+    // ---- loading: lane -> (row of RPI, PC chunks). Each row is read once on
+    // the chip (query rows past 32 aside), so it is only streamed through L2.
+    const int ld_row = lane / CPR, ld_c = lane % CPR * PC;
+    st_raw rk[NL], rv[NL];
     const bool whole_pages = bs % ST_KEYS == 0;
     auto load_tile = [&](int kb) {
         // a tile inside one page: the page is a scalar look-up
@@ -165,8 +174,10 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
                 off = (((long)page * nkv + kvh) * bs + key % bs) * HD;
             }
             off += ld_c * 8;
-            rk[i] = *reinterpret_cast<const raw_t*>(k_cache + off);
-            rv[i] = *reinterpret_cast<const raw_t*>(v_cache + off);
+            rk[i] = __builtin_nontemporal_load(
+                reinterpret_cast<const st_raw*>(k_cache + off));
+            rv[i] = __builtin_nontemporal_load(
+                reinterpret_cast<const st_raw*>(v_cache + off));
         }
     };
 
@@ -196,12 +207,15 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int row = ld_row + i * RPI;
-            *reinterpret_cast<short8*>(kd + row * RB +
-                                       ((ld_c ^ k_swz(row)) << 4)) =
-                st_widen(rk[i]);
-            *reinterpret_cast<short8*>(
-                kd + TILE + row * RB + ((ld_c ^ v_swz(row)) << 4)) =
-                st_widen(rv[i]);
+#pragma unroll
+            for (int p = 0; p < PC; ++p) {
+                *reinterpret_cast<short8*>(
+                    kd + row * RB + (((ld_c + p) ^ k_swz(row)) << 4)) =
+                    st_piece<KVT>(rk[i], p);
+                *reinterpret_cast<short8*>(
+                    kd + TILE + row * RB + (((ld_c + p) ^ v_swz(row)) << 4)) =
+                    st_piece<KVT>(rv[i], p);
+            }
         }
         if (kb + ST_STEP < k1) load_tile(kb + ST_STEP);
         WAVE_LDS_SYNC();
