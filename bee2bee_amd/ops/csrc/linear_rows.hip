@@ -11,8 +11,10 @@
 //    The waves of a workgroup share K and add up in LDS; there is no split
 //    over workgroups, so a row's result depends neither on the other rows nor
 //    on their number.
-//  * TC 8: 8 rows of W at two places along K, 128 bytes of a row together, as
-//    one left operand, 8 input rows at both places as the other; the two
+//  * TC 8: 8 rows of W at two places along K, 128 bytes of a row together (whole
+//    lines, so these loads carry the streaming hint: 2x14336x4096 41 us without
+//    and 36.5 with, 4096x14336 24.2 and 22.1, 3584x18944 27.8 and 26), as one
+//    left operand, 8 input rows at both places as the other; the two
 //    diagonal quarters of the product add up. Twice the workgroups where 16
 //    columns each leave CUs without one, and better pieces to load elsewhere.
 //  * Between two layers' projections the residual sum stays in fp32: the norm
@@ -28,15 +30,15 @@
 //    each workgroup takes them from the rows itself (they are in L2).
 //  * two batches of weight loads, LR_U tiles each, are on their way: with 8 or
 //    16 the registers cost more waves than the loads gain (output head of
-//    128256 x 4096, us: 4 tiles 182, 8 205, 16 230), and a streaming hint on
-//    the loads loses the half lines a 64-byte piece leaves (206 to 240). The
+//    128256 x 4096, us: 4 tiles 182, 8 205, 16 230), and the streaming hint on
+//    16-row tiles loses the half lines a 64-byte piece leaves (206 to 240). The
 //    input asked for as early as the weights costs registers too (a step of 8
 //    layers of 3584, two rows: 1220 to 1290 us; of 4096, one row: 1014 to 1034).
-// Measured (us, one row, beside the library product alone): 6144x4096 15.3
-// (14.5), 4096x4096 9.3 (15.6), 2x14336x4096 44 (64), 4096x14336 25 (27),
-// 128256x4096 182 (194); floor at 5.9 TB/s and 4 us a launch: 12.5, 9.7, 44,
-// 24, 182. With 16 rows 17, 11.6, 57, 34, 200: the input's reads add up, so
-// more rows go to the library.
+// Measured (us, one row, beside the library product alone): 6144x4096 13.8
+// (14.5), 4096x4096 8.5 (15.6), 2x14336x4096 36.5 (64), 4096x14336 22.1 (27),
+// 128256x4096 178 (194); bytes at 6.5 TB/s: 7.7, 5.2, 36, 18, 162. With 16 rows
+// 15.5, 10.8, 52, 31, 188: the input's reads add up, so more rows, the longest
+// gated projections and most output heads are linear_mid.hip's.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) short short4v;
@@ -96,6 +98,14 @@ DEV_INLINE void store_row4(void* cache, long at, int fp8, const float* z) {
     }
 }
 
+// (see above: TC 8 reads whole lines, which are only streamed through L2)
+template <int TC> DEV_INLINE bf16x8 lr_weights(const unsigned short* p) {
+    if constexpr (TC == 8)
+        return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+    else
+        return *reinterpret_cast<const bf16x8*>(p);
+}
+
 // EPI LR_PLAIN: y = n(x) W^T [+ bias] [+ resid]; LR_GLU: y = silu(g) u, g and
 // u from the halves of W [2N, K]; LR_GELU: y = gelu_tanh(n(x) W^T + bias);
 // LR_QKV: see QkvStore (W [N, K], bias optional). NT tiles of 16 columns of y
@@ -152,7 +162,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
             for (int h = 0; h < H; ++h)
 #pragma unroll
                 for (int t = 0; t < WT; ++t)
-                    aw[set][u][h][t] = *reinterpret_cast<const bf16x8*>(
+                    aw[set][u][h][t] = lr_weights<TC>(
                         wp[t] + (long)(s + u) * KS + h * 32);
     };
     int s = s0;
@@ -249,8 +259,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         for (int h = 0; h < H; ++h)
 #pragma unroll
             for (int t = 0; t < WT; ++t)
-                a[h][t] = *reinterpret_cast<const bf16x8*>(
-                    wp[t] + (long)s * KS + h * 32);
+                a[h][t] = lr_weights<TC>(wp[t] + (long)s * KS + h * 32);
         products(a, s);
     }
 
