@@ -146,16 +146,17 @@ class Runner:
                 self.spec.rms_eps, self.dtype)
             return F.linear(normed, self.weights.lm_head)
         W = self.weights
+        if self._mid_dims and ops.ring_rows(hidden) and ops.mid_head(
+                hidden.shape[0], *W.lm_head.shape):
+            return ops.mid_rows_linear(
+                self._norm(hidden, W.final_norm, W.final_norm_bias),
+                W.lm_head)
         if self._rows_dims and ops.head_rows(
                 hidden, self.spec.norm_type == "layernorm"):
             return ops.rows_linear(
                 hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
                                          self.spec.rms_eps))
         normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
-        if self._mid_dims and (ops.mid_rows(normed) or ops.deep_rows(
-                normed, W.lm_head.shape[0])) and ops.mid_head(
-                    normed.shape[0], *W.lm_head.shape):
-            return ops.mid_rows_linear(normed, W.lm_head)
         return F.linear(normed, W.lm_head)
 
     def _run_layers_rows(

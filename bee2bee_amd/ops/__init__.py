@@ -236,14 +236,13 @@ def few_rows(x: torch.Tensor) -> bool:
 
 
 def head_rows(x: torch.Tensor, layer_norm: bool) -> bool:
-    """Few rows whose logits are rows_linear's; the others' are a norm and the
-    library's. Measured (us, rows_linear / norm and library): 128256 columns of
-    4096 182 / 194 at 1 row, 198 / 196 at 12, 200 / 194 at 16; of 3072 155 / 153
-    at 16; 152064 of 3584 207 / 239 at 16; of 8192 373 / 371 at 8, 415 / 363 at
-    16, 201088 of 8192 603 / 609 at 12, 623 / 593 at 16. A layer norm's mean and
-    deviation are taken by each of the hundreds of workgroups: 50257 of 768 22.0
-    / 21.8 at 1 row, 22.8 / 22.1 at 4 (a launch less for the host: 20 us of a
-    step that is not captured), 25 / 22.5 at 8, 30 / 23 at 16."""
+    """Few rows whose logits are rows_linear's, where mid_head does not take
+    them; the others' are a norm and the library's. Measured (us, rows_linear /
+    norm and library): 128256 columns of 8192 373 / 371 at 8 rows, 415 / 363 at
+    16. A layer norm's mean and deviation are taken by each of the hundreds of
+    workgroups: 50257 of 768 22.0 / 21.8 at 1 row, 22.8 / 22.1 at 4 (a launch
+    less for the host: 20 us of a step that is not captured), 25 / 22.5 at 8, 30
+    / 23 at 16."""
     if layer_norm:
         return few_rows(x) and x.shape[0] <= 4
     return few_rows(x) and (x.shape[0] <= 12 or x.shape[1] < 8192)
@@ -305,6 +304,13 @@ def mid_rows(x: torch.Tensor) -> bool:
             and x.dtype is torch.bfloat16 and x.is_contiguous())
 
 
+def ring_rows(x: torch.Tensor) -> bool:
+    """Rows that mid_rows_linear takes: 1 to DEEP_MAX contiguous bf16 rows on the
+    GPU."""
+    return (x.dim() == 2 and 1 <= x.shape[0] <= DEEP_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous())
+
+
 def deep_rows(x: torch.Tensor, inner: int) -> bool:
     """Steps of up to DEEP_MAX such rows whose down projection has DEEP_SIZE
     weights or more; mid_shape picks among the others."""
@@ -363,7 +369,11 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     the library's product (us): 128256x4096 168 (193) at 24 rows, 195 (218) at
     80, 230 (245) at 160, 304 (297) at 256; 152064x3584 172 (242), 218 (213);
     32000x4096 41 (63), 48 (66), 58 (64); 128256x2048 84 (121), 103 (129); of
-    rows of 768 17.0 (18.6), 22.6 (20.8)."""
+    rows of 768 17.0 (18.6), 22.6 (20.8). Few rows (one launch of rows_linear in
+    brackets; a norm takes 2.5 us): 1 / 16 rows 128256x4096 168 (178) / 166
+    (188), 152064x3584 158 (182) / 164 (204), 128256x2048 77 (93) / 81 (101)."""
+    if rows <= ROWS_MAX and width * depth < 100_000_000:
+        return False
     tiles = -(-width // 16)
     rounds = -(-tiles // 2048)
     full = 256 * rounds * -(-tiles // (256 * rounds))

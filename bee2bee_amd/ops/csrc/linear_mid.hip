@@ -1,5 +1,5 @@
-// Projections of 17 to 256 rows, and the gated or activated ones and the output
-// head of such steps: x [M, K] times rows of w [N, K]. Three forms of result:
+// Projections of 17 to 256 rows, and of fewer the longest gated ones and most
+// output heads: x [M, K] times rows of w [N, K]. Three forms of result:
 //  parts   fp32 sums over S parts of K, left to the kernel that reads them
 //          anyway (qkv_rope_store, add_norm_parts): narrow projections, which
 //          would leave most of the chip idle unsplit;
@@ -18,14 +18,20 @@
 // streaming hint, so that they do not push the input out of L2 (2x14336x4096 at
 // 24 rows 40.8 us without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128
 // bytes in LDS are xor-ed by half their number: no two of a read's 16 rows meet
-// in a bank. Unsplit, workgroups start at different places of K (ROT): in step
-// they would all ask for the same few channels (44.8 -> 41.3 us at 24 rows, 53
-// -> 44.5 at 80; split, K = 14336, it loses: 22.9 -> 26.8).
+// in a bank. Workgroups start at different places of K: in step they would all
+// ask for the same few channels (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 ->
+// 44.5 at 80). The input needs three slots (with two, and more of weights, 44 ->
+// 61 us at 80 rows); more, or its rows apart by an odd number of lines, change
+// nothing.
 //
-// Measured beside the library's product and the kernel that reads it (us, 24 /
-// 80 / 128 / 200 / 256 rows; in brackets, the form before this one, which took
-// weights through registers):
-//   @T_PARTS@
+// Measured with the kernel that reads them (us, 24 / 80 / 128 / 200 / 256 rows;
+// in brackets this file's form before, which took weights through registers):
+//   4096x14336 26.6 / 33.2 / 35.3 / 42.4 / 48.4 (30.1 / 36.1 / 43.9 / 56 / 64)
+//   4096x4096  13.7 / 16.9 / 19.7 / 23.7 / 25.1 (14.5 / 17.3 / 20.7 / 25.5 / 29)
+//   6144x4096  16.9 / 22.9 / 26.1 / 30.0 / 32.1 (19.5 / 24.0 / 29.1 / 36.5 / 41)
+//   3584x18944 28.7 / 35.4 / 39.0 / 50.2 / 56.6 (33.7 / 43.1 / 52.2 / 69 / 78)
+//   2048x8192  13.2 / 16.5 / 19.3 / 22.3 / 24.6 (14.4 / 17.1 / 20.3 / 25.5 / 29)
+// The library's figures are at the rules in ops/__init__.py.
 #include "common.h"
 
 enum { LM_PARTS = 0, LM_GATED = 1, LM_ROWS = 2 };
@@ -64,11 +70,13 @@ DEV_INLINE void lm_wait(int left) {
 // input rows, by WK halves of a step. DW, DX: slots of the rings. `tiles` of
 // the TW * WN are used. WK 1: a workgroup takes every gridDim.x-th group of
 // tiles, loading the next one's first steps under this one's last.
-template <int TW, int MW, int WN, int WM, int WK, int DW, int DX, int OUT>
+template <int TW, int MW, int WN, int WM, int WK, int DW, int DX, int OUT,
+          bool SCALED = false>
 __global__ __launch_bounds__(512) void linear_mid_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias, void* __restrict__ out, int M,
-    int N, int K, int S, int tiles, int gelu) {
+    int N, int K, int S, int tiles, int gelu,
+    const float* __restrict__ squares, float eps) {
     constexpr int T = TW * WN, MT = MW * WM;
     static_assert(WN * WM * WK == 8 && DW >= 2 && DX >= 2, "");
     constexpr int NLW = T / 2, NLX = (MT + 1) / 2;  // loads of a wave a step
@@ -129,6 +137,8 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
                 lm_load<true>(b, off[j], to0 + lslot * WB + j * 1024);
             if (++lslot == DW) lslot = 0;
         } else {
+            // (MT 1: two waves' loads are all)
+            if (MT > 1 || wid < 6)
 #pragma unroll
             for (int j = 0; j < NLX; ++j)
                 lm_load<false>(b, off[j], to0 + lslot * XB + j * 1024);
@@ -143,6 +153,21 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     };
     const int D = of_w ? DW : DX;
     for (int i = 0; i < D && i < total; ++i) issue();
+    // 1 / rms of each row, while the weights are on their way: the waves of
+    // the input, whose few stages the compiler's wait may include
+    __shared__ float inv_s[16];
+    if (SCALED && !of_w) {
+        for (int row = wid - 4; row < M; row += 4) {
+            float v = 0.f;
+            for (int c = lane * 4; c < K / 8; c += 256) {
+                const f32x4 q = *reinterpret_cast<const f32x4*>(
+                    squares + (long)row * (K / 8) + c);
+                v += (q[0] + q[1]) + (q[2] + q[3]);
+            }
+            v = wave_sum(v);
+            if (lane == 0) inv_s[row] = rsqrtf(v / (float)K + eps);
+        }
+    }
 
     // ---- products
     f32x4 acc[TW][MW];
@@ -193,6 +218,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
         return true;
     };
     auto finish = [&](int grp) {
+        const float inv = SCALED ? inv_s[min(li, M - 1)] : 1.f;
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
             const int tt = wn * TW + t, tile = grp * tiles + tt;
@@ -207,7 +233,8 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
                 if (OUT == LM_GATED) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float2v p = lane_pair(acc[t][m][r]);
+                        const float2v p = lane_pair(
+                            SCALED ? acc[t][m][r] * inv : acc[t][m][r]);
                         z[r] = p.x / (1.f + __expf(-p.x)) * p.y;
                     }
                 }
@@ -242,6 +269,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     };
     if (of_w) lm_wait<NLW, DW - 1>(min(total, DW) - 1);
     else lm_wait<NLX, DX - 1>(min(total, DX) - 1);
+    fragments_here();                          // (and inv_s is written)
     asm volatile("s_barrier" ::: "memory");
     read(0, WK == 2 ? wk : 0);
     int left = n;                              // steps of this group
@@ -305,8 +333,12 @@ static int lm_tiles(int NT, int S, int most) {
 
 // Parts of K: as many as leave a workgroup at most 8 tiles and, of K, twice as
 // many steps of 64 as it has tiles (and 6), so that the parts, written and read
-// once more, stay below the weights. Measured with the kernel that reads them
-// (us, 24 / 200 rows): @T_SPLIT@
+// once more, stay well below the weights. Measured with the kernel that reads
+// them (us, 24 / 200 rows, before the streaming hint): 6144x4096 2 parts of 3
+// tiles 19.6 / 30.9, 4 of 6 17.6 / 28.5, 8 of 12 20.1 / 33.9; 4096x4096 2 16.7 /
+// 27.7, 4 14.5 / 22.4, 8 15.3 / 24.5; 4096x14336 4 28.1 / 48.2, 8 28.4 / 43.1;
+// 3072x8192 4 18.9 / 30.7, 8 17.2 / 28.1; 2048x2048 2 10.1 / 16.7, 4 8.4 / 14.8,
+// 8 8.6 / 17.1.
 extern "C" int linear_mid_splits(int N, int K) {
     const int NT = (N + 15) / 16;
     int S = 1;
@@ -321,11 +353,14 @@ extern "C" int linear_mid_splits(int N, int K) {
 // x [M, K] and w contiguous and 16-byte aligned, 1 <= M <= 256, K % 64 == 0.
 // out: form LM_PARTS [S, M, N] fp32, 1 <= S <= K / 64; LM_GATED [M, N] bf16, w
 // [2N, K], N % 8 == 0, S 1, no bias; LM_ROWS [M, N] bf16, S 1. N % 4 == 0.
+// squares [M, K / 8] (LM_GATED, M <= 16; else null): RMS norm of
+// rows that come multiplied by its weight, whose sums of squares these are.
 // Nonzero for anything else.
 extern "C" int launch_linear_mid(const unsigned short* x,
                                  const unsigned short* w,
                                  const unsigned short* bias, void* out, int M,
                                  int N, int K, int S, int form, int gelu,
+                                 const float* squares, float eps,
                                  hipStream_t stream) {
     if (M < 1 || M > 256 || N < 4 || N % 4 || K < 64 || K % 64) return 1;
     if (S < 1 || S > K / 64 || (form != LM_PARTS && S != 1)) return 1;
@@ -348,7 +383,8 @@ extern "C" int launch_linear_mid(const unsigned short* x,
         hipLaunchKernelGGL(                                                   \
             (linear_mid_kernel<TW, MW, WN, WM, WK, DW, DX, F>),               \
             dim3(WK == 1 && !once ? 256 / S : NG, S), dim3(512),              \
-            lds, stream, x, w, bias, out, M, N, K, S, tiles, gelu);           \
+            lds, stream, x, w, bias, out, M, N, K, S, tiles, gelu, nullptr,   \
+            0.f);                                                             \
         return 0;                                                             \
     } while (0)
 #define LM_4(F)                                                               \
@@ -376,6 +412,23 @@ extern "C" int launch_linear_mid(const unsigned short* x,
         if (M <= 224) LM_GO(2, 7, 4, 2, 1, 4, 3, F);                          \
         LM_GO(2, 8, 4, 2, 1, 4, 3, F);                                        \
     } while (0)
+#define LM_SCALED(TW, MW, WN, WM, WK, DW, DX)                                 \
+    do {                                                                      \
+        constexpr int lds =                                                   \
+            DW * (TW * WN / 2) * 4096 + DX * ((MW * WM + 1) / 2) * 4096;      \
+        static_assert(lds + 64 <= 163840, "LDS of a CU");                     \
+        hipLaunchKernelGGL(                                                   \
+            (linear_mid_kernel<TW, MW, WN, WM, WK, DW, DX, LM_GATED, true>),  \
+            dim3(WK == 1 && !once ? 256 : NG), dim3(512), lds, stream, x, w,  \
+            nullptr, out, M, N, K, 1, tiles, 0, squares, eps);                \
+        return 0;                                                             \
+    } while (0)
+    if (squares) {
+        if (form != LM_GATED || M > 16) return 1;
+        if (tiles > 8) LM_SCALED(3, 1, 4, 1, 2, 6, 3);
+        if (tiles > 4) LM_SCALED(1, 1, 8, 1, 1, 8, 4);
+        LM_SCALED(1, 1, 4, 1, 2, 12, 6);
+    }
     if (form == LM_GATED && tiles > 8) {
         if (M <= 32) LM_GO(3, 2, 4, 1, 2, 6, 3, LM_GATED);
         if (M <= 64) LM_GO(3, 4, 4, 1, 2, 5, 3, LM_GATED);
@@ -389,6 +442,7 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     if (form == LM_ROWS) LM_8(LM_ROWS);
     if (tiles <= 4) LM_4(LM_PARTS);
     LM_8(LM_PARTS);
+#undef LM_SCALED
 #undef LM_8
 #undef LM_4
 #undef LM_GO

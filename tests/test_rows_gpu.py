@@ -258,6 +258,33 @@ def test_activated_rows(M, N, K, act):
             + 1e-6).all()
 
 
+# (a workgroup's tiles of 8 columns: up to 4, 8, 12, and two groups of 7)
+@pytest.mark.parametrize("N,K", [(8192, 6144), (12552, 4096), (17000, 3008),
+                                 (25000, 2048)])
+def test_long_gated_projections_of_few_rows(N, K):
+    """Rows that come with their sums of squares: 1 / rms in fp32 (a relative
+    2^-20 of the products, with the slopes of the activation), a row's result
+    the same to the bit whatever rows are beside it."""
+    torch.manual_seed(N)
+    x, w = _rand(16, K), _rand(2 * N, K, std=0.05)
+    squares = torch.rand(16, K // 8, device=DEV) * 16 + 1
+    rows = lambda at: ops.rows_linear(
+        x[at].contiguous(), w, norm=(squares[at].contiguous(), 1e-5),
+        act="swiglu")
+    got = rows(slice(0, 16))
+    inv = torch.rsqrt(squares.double().sum(-1, keepdim=True) / K + 1e-5)
+    z = x.double() @ w.double().t() * inv
+    mag = (x.double().abs() @ w.double().abs().t()) * inv
+    e = (2 ** -24 * K + 2 ** -20) * mag
+    (g, u), (eg, eu) = z.chunk(2, -1), e.chunk(2, -1)
+    want = F.silu(g) * u
+    bound = 1.13 * eg * u.abs() + F.silu(g).abs() * eu + 1.13 * eg * eu
+    assert ((got.double() - want).abs() <= bound + (2 ** -8 + 2 ** -20)
+            * want.abs() + 1e-6).all()
+    for at in (slice(0, 1), slice(3, 5), slice(7, 16)):
+        assert torch.equal(rows(at), got[at])
+
+
 @pytest.mark.parametrize("S,M,H", [(1, 17, 64), (8, 128, 4096), (4, 20, 8192),
                                    (2, 33, 3592)])
 @pytest.mark.parametrize("kind", [None, "rms", "layer"])
