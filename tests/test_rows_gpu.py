@@ -259,8 +259,8 @@ def test_activated_rows(M, N, K, act):
 
 
 # (a workgroup's tiles of 8 columns: up to 4, 8, 12, and two groups of 7)
-@pytest.mark.parametrize("N,K", [(8192, 6144), (12552, 4096), (17000, 3008),
-                                 (25000, 2048)])
+@pytest.mark.parametrize("N,K", [(8192, 6144), (12560, 4096), (17008, 3008),
+                                 (25008, 2048)])
 def test_long_gated_projections_of_few_rows(N, K):
     """Rows that come with their sums of squares: 1 / rms in fp32 (a relative
     2^-20 of the products, with the slopes of the activation), a row's result
