@@ -157,6 +157,10 @@ class Runner:
                 hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
                                          self.spec.rms_eps))
         normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
+        if self._mid_dims and ops.wide_rows(hidden):
+            plan = ops.wide_plan(hidden.shape[0], *W.lm_head.shape, "rows")
+            if plan:
+                return ops.wide_linear(normed, W.lm_head, plan)
         return F.linear(normed, W.lm_head)
 
     def _run_layers_rows(
@@ -225,6 +229,17 @@ class Runner:
             ops.kv_cache_store(k, v, k_cache, v_cache, slot_mapping)
         return attn_fn(layer_idx, q, k, v, k_cache, v_cache)
 
+    def _parts_product(self, rows: int, width: int, depth: int,
+                       bias: bool = False):
+        """The product of a projection whose reader sums parts, or takes rows:
+        a function of its input and weights, or None for the library."""
+        if rows <= ops.DEEP_MAX:
+            return ops.mid_linear if ops.mid_shape(rows, width, depth) else None
+        plan = ops.wide_plan(rows, width, depth, "parts")
+        if not plan or (bias and plan < 16):      # (rows come without bias)
+            return None
+        return lambda x, w: ops.wide_linear(x, w, plan)
+
     def _run_layers_mid(
         self,
         x: torch.Tensor,
@@ -232,53 +247,55 @@ class Runner:
         slot_mapping: torch.Tensor,
         attn_fn,
     ) -> torch.Tensor:
-        """Dense layers on some tens of rows: projections as parts over K,
-        summed by the kernels that read them (ops.mid_shape), or activated where
-        they are made (ops.mid_gated, ops.mid_gelu)."""
+        """Dense layers on some tens of rows and more: projections as parts over
+        K, summed by the kernels that read them (ops.mid_shape, ops.wide_plan),
+        or activated where they are made (ops.mid_gated, ops.mid_gelu)."""
         s, T = self.spec, x.shape[0]
         layers = self.weights.layers
         H, I = s.hidden_size, s.intermediate_size
-        qkv_parts = ops.mid_shape(T, s.q_size + 2 * s.kv_size, H)
-        o_parts = ops.mid_shape(T, H, s.q_size)
-        down_parts = ops.mid_shape(T, H, I)
-        gelu = s.act_type == "gelu"
-        act = "gelu" if gelu else "swiglu"
-        own_act = (ops.mid_gelu if gelu else ops.mid_gated)(T, I, H) and (
-            gelu or not s.mlp_bias)
         lw = layers[self.layer_lo]
+        make_qkv = self._parts_product(T, s.q_size + 2 * s.kv_size, H)
+        make_o = self._parts_product(T, H, s.q_size, lw.wo_bias is not None)
+        make_down = self._parts_product(T, H, I, lw.w_down_bias is not None)
+        gelu = s.act_type == "gelu"
+        act, plan = "gelu" if gelu else "swiglu", 0
+        own_act = T <= ops.DEEP_MAX and (
+            ops.mid_gelu if gelu else ops.mid_gated)(T, I, H) and (
+            gelu or not s.mlp_bias)
+        if T > ops.MID_MAX and not (own_act or gelu or s.mlp_bias):
+            plan = ops.wide_plan(T, I, H, "gated")
         normed = self._norm(x, lw.attn_norm, lw.attn_norm_bias)
+
+        def add(part, bias, x, norm):
+            """Residual add and the next norm of a product without its bias."""
+            if part.dim() == 3:
+                return ops.add_norm_parts(part, bias, x,
+                                          norm and (*norm, s.rms_eps))
+            if norm is None:
+                return None, x + part
+            return self._fused_add_norm(part, x, *norm)
 
         for i in range(self.layer_lo, self.layer_hi):
             lw = layers[i]
-            qkv = (ops.mid_linear(normed, lw.wqkv) if qkv_parts
-                   else F.linear(normed, lw.wqkv))
+            qkv = (make_qkv or F.linear)(normed, lw.wqkv)
             o = self._attend(i, qkv, positions, slot_mapping,
                              attn_fn).reshape(T, s.q_size)
-            if o_parts:
-                normed, x = ops.add_norm_parts(
-                    ops.mid_linear(o, lw.wo), lw.wo_bias, x,
-                    (lw.mlp_norm, lw.mlp_norm_bias, s.rms_eps))
-            else:
-                normed, x = self._fused_add_norm(
-                    F.linear(o, lw.wo, lw.wo_bias), x, lw.mlp_norm,
-                    lw.mlp_norm_bias)
+            o = make_o(o, lw.wo) if make_o else F.linear(o, lw.wo, lw.wo_bias)
+            normed, x = add(o, lw.wo_bias, x,
+                            (lw.mlp_norm, lw.mlp_norm_bias))
             if own_act:
                 z = ops.mid_rows_linear(normed, lw.w_gate_up,
                                         lw.w_gate_up_bias, act)
+            elif plan:
+                z = ops.wide_linear(normed, lw.w_gate_up, plan, act)
             else:
                 z = F.linear(normed, lw.w_gate_up, lw.w_gate_up_bias)
                 z = ops.gelu(z) if gelu else ops.swiglu(z)
+            z = (make_down(z, lw.w_down) if make_down
+                 else F.linear(z, lw.w_down, lw.w_down_bias))
             nxt = layers[i + 1] if i + 1 < self.layer_hi else None
-            if down_parts:
-                normed, x = ops.add_norm_parts(
-                    ops.mid_linear(z, lw.w_down), lw.w_down_bias, x,
-                    nxt and (nxt.attn_norm, nxt.attn_norm_bias, s.rms_eps))
-            else:
-                z = F.linear(z, lw.w_down, lw.w_down_bias)
-                if nxt is None:
-                    return x + z
-                normed, x = self._fused_add_norm(z, x, nxt.attn_norm,
-                                                 nxt.attn_norm_bias)
+            normed, x = add(z, lw.w_down_bias, x,
+                            nxt and (nxt.attn_norm, nxt.attn_norm_bias))
         return x
 
     def _rows_add(self, x, y, w, bias, nxt):
@@ -563,9 +580,7 @@ class Runner:
             return self._run_layers_rows(hidden, positions, slot_mapping,
                                          attn_fn, paged)
         s = self.spec
-        if self._mid_dims and (
-                ops.mid_rows(hidden)
-                or ops.deep_rows(hidden, s.intermediate_size)):
+        if self._mid_dims and (ops.mid_rows(hidden) or ops.wide_rows(hidden)):
             return self._run_layers_mid(hidden, positions, slot_mapping,
                                         attn_fn)
         residual = None

@@ -311,14 +311,6 @@ def ring_rows(x: torch.Tensor) -> bool:
             and x.dtype is torch.bfloat16 and x.is_contiguous())
 
 
-def deep_rows(x: torch.Tensor, inner: int) -> bool:
-    """Steps of up to DEEP_MAX such rows whose down projection has DEEP_SIZE
-    weights or more; mid_shape picks among the others."""
-    return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
-            and x.dtype is torch.bfloat16 and x.is_contiguous()
-            and x.shape[1] * inner >= DEEP_SIZE)
-
-
 def mid_shape(rows: int, width: int, depth: int) -> bool:
     """Projections that mid_linear takes, all up to MID_MAX rows, above it
     those that outweigh their parts. Measured with the kernel that reads them
@@ -380,6 +372,30 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     if width % 4 or rows > 160 or (depth < 1024 and rows > 48):
         return False
     return rows <= 64 or tiles * 20 >= full * 19
+
+
+def wide_rows(x: torch.Tensor) -> bool:
+    """Steps of more than MID_MAX contiguous bf16 rows on the GPU."""
+    return (x.dim() == 2 and x.shape[0] > MID_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous())
+
+
+_FORMS = {"rows": 0, "gated": 1, "parts": 2}
+
+
+def wide_plan(rows: int, width: int, depth: int, form: str) -> int:
+    """How wide_linear takes a projection on the GPU; 0: it is left to the
+    library. form: "rows", "gated" (width: of one half) or "parts", whose reader
+    sums parts or takes rows."""
+    return require_hip().wide_plan(rows, width, depth, _FORMS[form])
+
+
+def wide_linear(x, w, plan: int, act=None):
+    """x w^T in bf16, or as parts [S, T, N] fp32 where the plan has several; act
+    "swiglu" as in rows_linear."""
+    if _use_hip(x):
+        return require_hip().wide_linear(x, w, plan, act == "swiglu")
+    return reference.rows_linear(x, w, act=act)
 
 
 def mid_linear(x, w):

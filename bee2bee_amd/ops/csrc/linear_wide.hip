@@ -1,0 +1,382 @@
+// Projections of many rows: x [M, K] times rows of w [N, K], in bf16 with fp32
+// sums. Three forms of result:
+//  rows    x w^T in bf16;
+//  gated   silu(gate) * value from w's two halves, so that the pass that reads
+//          both and writes their product is gone, and neither is rounded;
+//  parts   fp32 sums over S parts of K, left to the kernel that reads them
+//          anyway (qkv_rope_store, add_norm_parts): where whole tiles would
+//          leave much of the chip idle.
+//
+// Bound by the matrix cores (at the clock that the power limit leaves them:
+// 8192x8192x8192 704 us, 1560 TFLOP/s). A workgroup a CU: 256 rows of x by 256
+// of w, 64 of K at a time in one of two buffers of 64 KB, filled straight from
+// memory. Eight waves, two a SIMD: 128 x 64 sums each, in four quarters of 64 x
+// 32. Waves 0-3 read a quarter's fragments while 4-7 multiply, and the other way
+// round, so that the matrix cores always have one of a SIMD's two waves; a
+// barrier at each change keeps them apart. What a quarter has read is loaded
+// again at once, for the step after next: 3500 clocks ahead, 6 of 8 regions
+// always under way. An XCD's workgroups take neighbouring tiles (8 by 4 at a
+// time), which share what its L2 holds.
+//
+// Measured (us; in brackets the library's product, and of gated ones its swiglu):
+//   gated 9216x2x18944x3584 1666 (1972), 4096x2x18944x3584 761 (874),
+//    4559x2x8192x3072 323 (468), 1536x2x14336x4096 258 (288), 500x 92 (115);
+//   rows 9216x3584x18944 800 (807), 4096x3584x18944 372 (531), 4096x4608x3584
+//    110 (122), 1536x6144x4096 63 (70), 1536x128256x4096 1104 (1216);
+//   parts, with the norm that adds them: 1536x4096x14336 141 (179), 1100x 126
+//    (158), 500x 68 (101), 800x2048x8192 36 (48).
+// Tried and slower: workgroups that stay and take tile after tile (3 to 6%: no
+// balance between them), tiles split over K inside one launch, the last to come
+// adding (256 KB a tile and part written and read: 40 to 80 us a product).
+#include "common.h"
+
+#include <type_traits>
+
+enum { LW_ROWS = 0, LW_GATED = 1, LW_PARTS = 2 };
+
+DEV_INLINE unsigned lw_lds(const void* p) {
+    return (unsigned)(unsigned long)(
+        __attribute__((address_space(3))) const char*)p;
+}
+// 16 bytes a lane from base + off to LDS at `to` + lane * 16. The compiler does
+// not see these loads: lw_wait counts them.
+DEV_INLINE void lw_load(const void* base, unsigned off, unsigned to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, %1"
+                 ::"v"(off), "s"(base), "s"(to) : "memory");
+}
+template <int N> DEV_INLINE void lw_wait() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+DEV_INLINE void lw_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+constexpr int LW_REGION = 128 * 128;           // 128 rows of 64 of K
+constexpr int LW_LDS = 8 * LW_REGION;
+
+// MT: tiles of 16 rows of x that a wave takes in each half of a tile's 64 * MT
+template <int FORM, int MT>
+__global__ __launch_bounds__(512) void linear_wide_kernel(
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
+    void* __restrict__ out, int M, int N, int K, int S, int TM, int TN,
+    int strip) {
+    constexpr int BM = MT * 64, HM = MT * 32;          // rows, of a half
+    constexpr int BN = FORM == LW_GATED ? 128 : 256;   // columns of a tile
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int wm = wid >> 2, wn = wid & 3;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+
+    // ---- the tile: an XCD's workgroups (every eighth) take neighbours, in
+    // strips of `strip` row tiles
+    int t;
+    {
+        const int total = gridDim.x, b = blockIdx.x;
+        const int xcd = b & 7, q = total >> 3, r = total & 7;
+        t = xcd * q + min(xcd, r) + (b >> 3);
+    }
+    const int part = t / (TM * TN);
+    t -= part * TM * TN;
+    const int s0 = t / (strip * TN), h = min(strip, TM - s0 * strip);
+    t -= s0 * strip * TN;
+    const int m0 = (s0 * strip + t % h) * BM, n0 = t / h * BN;
+    const int k0 = K / 64 * part / S, n = K / 64 * (part + 1) / S - k0;
+
+    // ---- loads: a wave's are 8 rows of 128 bytes, lane l the 16 bytes that
+    // belong at l * 16 (xor-ed by half the row's number: no two of a read's 16
+    // rows meet in a bank)
+    const char* xb = reinterpret_cast<const char*>(x + (long)m0 * K + k0 * 64);
+    const char* wb = reinterpret_cast<const char*>(w + (long)n0 * K + k0 * 64);
+    const char* wb1 = FORM == LW_GATED ? wb + (long)N * K * 2 : wb;
+    // Of each half of w's 256 rows a wave loads 16, of x's MT / 2 times 8 (MT 3:
+    // two of one half, one of the other, waves 4-7 the other way round).
+    auto first = [&](int g) {                  // its first 8 rows of x's half
+        return MT == 4 ? wid * 2 : MT == 2 ? wid
+               : (wid < 4) == (g == 0) ? wid % 4 * 2 : 8 + wid % 4;
+    };
+    unsigned xo[2][2], wo[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int r8 = lane >> 3;
+        const unsigned c = ((lane & 7) ^ (r8 >> 1)) * 16, c1 = c ^ 64;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int f = first(g) + j, xr = g * HM + f * 8 + r8;
+            xo[g][j] = (unsigned)min(xr, M - 1 - m0) * K * 2 + (f & 1 ? c1 : c);
+            // (rows past the last: its)
+            const int wr = (FORM == LW_GATED ? 0 : g * 128) + wid * 16 + j * 8 +
+                           r8;
+            wo[g][j] = (unsigned)min(wr, N - 1 - n0) * K * 2 + (j ? c1 : c);
+        }
+    }
+    const unsigned to = lw_lds(smem);
+    // regions of a buffer: x's halves, w's halves
+    auto load_x = [&](int buf, int g, int step) {
+        const char* b = xb + (long)step * 128;
+        const unsigned at = to + (buf * 4 + g) * LW_REGION + first(g) * 1024;
+        lw_load(b, xo[g][0], at);
+        if (MT == 4 || (MT == 3 && (wid < 4) == (g == 0)))
+            lw_load(b, xo[g][1], at + 1024);
+    };
+    auto load_w = [&](int buf, int g, int step) {
+        const char* b = (g ? wb1 : wb) + (long)step * 128;
+        const unsigned at = to + (buf * 4 + 2 + g) * LW_REGION + wid * 2048;
+        lw_load(b, wo[g][0], at);
+        lw_load(b, wo[g][1], at + 1024);
+    };
+    // until at most R regions' loads are under way (in the order w, x 0, w, x 1
+    // of a step, the last of them x 1 where AT 1; MT 3: as the wave has it that
+    // issued fewer)
+    auto wait = [&](auto regions, auto at1) {
+        constexpr int R = decltype(regions)::value;
+        constexpr bool A = decltype(at1)::value;
+        constexpr int W = A ? R / 2 : (R + 1) / 2, X = R - W;
+        lw_wait<W * 2 + (MT == 4 ? X * 2 : MT == 2 ? X : X * 3 / 2)>();
+    };
+
+    f32x4 acc[2][2][MT][2];                    // half of x, of w, tiles
+#pragma unroll
+    for (int i = 0; i < MT * 8; ++i)
+        acc[i / (4 * MT)][i / (2 * MT) & 1][i / 2 % MT][i & 1] =
+            f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 fa[MT][2], fb[2][2][2];
+    const int p0 = (lg ^ (li >> 1)) * 16;      // of K 0-31; 32-63: ^ 64
+    const char* af = smem + (wm * MT * 16 + li) * 128;
+    const char* bf = smem + (wn * 32 + li) * 128;
+    auto read_x = [&](int buf, int g) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                fa[i][k] = *reinterpret_cast<const bf16x8*>(
+                    af + (p0 ^ k * 64) + (buf * 4 + g) * LW_REGION + i * 2048);
+    };
+    auto read_w = [&](int buf, int g) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                fb[g][i][k] = *reinterpret_cast<const bf16x8*>(
+                    bf + (p0 ^ k * 64) + (buf * 4 + 2 + g) * LW_REGION +
+                    i * 2048);
+    };
+    auto products = [&](int gx, int gw) {
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[gx][gw][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        fb[gw][j][k], fa[i][k], acc[gx][gw][i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+    };
+    // (the builtin: the compiler has to know that nothing is under way)
+    auto here = [&]() {
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        lw_barrier();
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using I4 = std::integral_constant<int, 4>;
+    using I5 = std::integral_constant<int, 5>;
+    using I6 = std::integral_constant<int, 6>;
+    using No = std::false_type;
+    using Yes = std::true_type;
+
+    // Step s of parity P = (s + n) & 1 lies in buffer P. Its regions are read in
+    // the order w P, x 0, w !P, x 1, the first in the step before; each is loaded
+    // again, for step s + 2, where all waves have read it, seven reads ahead.
+    auto step = [&](auto par, auto ahead, int s) {
+        constexpr int P = decltype(par)::value, L = decltype(ahead)::value;
+        // L: steps after this one, 2 standing for more
+        read_x(P, 0);
+        if (L == 2) load_w(P, P, s + 2);
+        if (L == 2) wait(I6(), No());
+        else if (L == 1) wait(I5(), Yes());
+        else wait(I1(), Yes());
+        here();
+        products(0, P);
+        lw_barrier();
+        read_w(P, !P);
+        if (L == 2) load_x(P, 0, s + 2);
+        if (L == 2) wait(I6(), No());
+        else if (L == 1) wait(I4(), Yes());
+        else wait(I0(), Yes());
+        here();
+        products(0, !P);
+        lw_barrier();
+        read_x(P, 1);
+        if (L == 2) load_w(P, !P, s + 2);
+        if (L == 2) wait(I6(), No());
+        else if (L == 1) wait(I3(), Yes());
+        here();
+        products(1, !P);
+        lw_barrier();
+        if (L) read_w(!P, !P);
+        if (L == 2) load_x(P, 1, s + 2);
+        if (L == 2) wait(I6(), No());
+        else if (L == 1) wait(I2(), Yes());
+        here();
+        products(1, P);
+        lw_barrier();
+    };
+    auto start = [&](int P) {
+        load_w(P, P, 0);
+        load_x(P, 0, 0);
+        load_w(P, !P, 0);
+        load_x(P, 1, 0);
+        load_w(!P, !P, 1);
+        load_x(!P, 0, 1);
+        load_w(!P, P, 1);
+        load_x(!P, 1, 1);
+        wait(I6(), No());
+        lw_barrier();
+        read_w(P, P);
+        here();
+        // waves 4-7 read while 0-3 multiply, and the other way round
+        if (wid >= 4) lw_barrier();
+    };
+    int s = 0;
+    if (n & 1) {
+        start(1);
+        step(I1(), I2(), 0);
+        s = 1;
+    } else {
+        start(0);
+    }
+    for (; s + 2 < n; s += 2) {
+        step(I0(), I2(), s);
+        step(I1(), I2(), s + 1);
+    }
+    step(I0(), I1(), s);
+    step(I1(), I0(), s + 1);
+    if (wid < 4) lw_barrier();
+
+    // ---- rows to LDS, a half of x's at a time, then out in whole lines.
+    // C layout: column li = row of x, rows lg * 4 + r = columns
+    constexpr int LD = BN + (FORM == LW_PARTS ? 4 : 8);
+    using E = std::conditional_t<FORM == LW_PARTS, float, unsigned short>;
+    E* os = reinterpret_cast<E*>(smem);
+#pragma unroll
+    for (int gx = 0; gx < 2; ++gx) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int gw = 0; gw < (FORM == LW_GATED ? 1 : 2); ++gw)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    f32x4 z = acc[gx][gw][i][j];
+                    E* p = os + ((wm * MT + i) * 16 + li) * LD + gw * 128 +
+                           wn * 32 + j * 16 + lg * 4;
+                    if constexpr (FORM == LW_PARTS) {
+                        *reinterpret_cast<f32x4*>(p) = z;
+                        continue;
+                    }
+                    if (FORM == LW_GATED) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            z[r] = z[r] *
+                                   __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
+                                   acc[gx][1][i][j][r];
+                    }
+                    *reinterpret_cast<uint2v*>(p) =
+                        uint2v{f2bf(z[0]) | (unsigned)f2bf(z[1]) << 16,
+                               f2bf(z[2]) | (unsigned)f2bf(z[3]) << 16};
+                }
+        __syncthreads();
+        constexpr int V = 16 / sizeof(E), CH = BN / V;
+        E* to_row = reinterpret_cast<E*>(out) +
+                    (FORM == LW_PARTS ? (long)part * M * N : 0) +
+                    (long)(m0 + gx * HM) * N + n0;
+#pragma unroll
+        for (int c = tid; c < HM * CH; c += 512) {
+            const int r = c / CH, col = c % CH * V;
+            if (m0 + gx * HM + r < M && n0 + col < N)
+                *reinterpret_cast<f32x4*>(to_row + (long)r * N + col) =
+                    *reinterpret_cast<const f32x4*>(os + r * LD + col);
+        }
+    }
+}
+
+// Microseconds of a launch as the planner sees it: rounds of 256 workgroups,
+// each with its start and end, a last one that leaves CUs idle a little faster
+// a step. (The steps of 128-row tiles are bound by what L2 gives, not by their
+// products: 0.82 us against 1.26 for twice the rows.)
+static double lw_time(int M, int N, int K, int form, int tall, int S) {
+    const double step = tall == 4 ? 1.26 : tall == 3 ? 1.0 : 0.82;
+    const int BN = form == LW_GATED ? 128 : 256;
+    const long tiles = ((M + tall * 64L - 1) / (tall * 64)) *
+                       ((N + BN - 1) / BN) * S;
+    const double steps = K / 64 / S, full = tiles / 256,
+                 left = (tiles % 256) / 256.0;
+    double t = full * (steps * step + tall + 3);
+    if (left > 0) t += steps * step * (0.7 + 0.3 * left) + tall + 3;
+    // the parts, written and read in place of bf16 rows
+    if (form == LW_PARTS) t += (double)M * N * (4 * S - 2) / 2.2e6;
+    return t;
+}
+
+// The tile's height and number of parts (1: rows) that are fastest: tall + 8 *
+// parts, or 0: left to the library. Parts only where LW_PARTS is asked for.
+extern "C" int linear_wide_plan(int M, int N, int K, int form) {
+    if (M < 1 || N < 8 || N % 8 || K < 256 || K % 64 || K > 1 << 22) return 0;
+    int best = 0;
+    double least = 1e30;
+    for (int tall = 2; tall <= 4; ++tall)
+        for (int S = 1; S <= (form == LW_PARTS ? 8 : 1); S *= 2) {
+            if (K / 64 / S < 8 && S > 1) break;
+            const double t = lw_time(M, N, K, S == 1 && form == LW_PARTS
+                                                  ? LW_ROWS : form, tall, S);
+            if (t < least) {
+                least = t;
+                best = tall + 8 * S;
+            }
+        }
+    if (form == LW_GATED || K >= 8192) return best;
+    const double library = 2.0 * M * N * K / 1.45e9;
+    return least <= library * 1.25 + 8 ? best : 0;
+}
+
+// x [M, K], w [N, K] (LW_GATED [2N, K]) and out [M, N] (LW_PARTS [S, M, N] fp32)
+// contiguous, 16-byte aligned; K % 64 == 0, K >= 128 S, N % 8 == 0; S 1 but for
+// LW_PARTS; tall: 2, 3 or 4 times 64 rows a tile. Nonzero for anything else.
+extern "C" int launch_linear_wide(const unsigned short* x,
+                                  const unsigned short* w, void* out, int M,
+                                  int N, int K, int S, int form, int tall,
+                                  hipStream_t stream) {
+    if (M < 1 || N < 8 || N % 8 || S < 1 || K < 128 * S || K % 64) return 1;
+    if (form != LW_PARTS && S != 1) return 1;
+    if (K > 1 << 22) return 1;                 // offsets in a tile: 32 bits
+    const int BN = form == LW_GATED ? 128 : 256, BM = tall * 64;
+    const int TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
+    if ((long)TM * TN * S > 1 << 30) return 1;
+    const int strips = (TM + 7) / 8, strip = (TM + strips - 1) / strips;
+#define LW_GO(F, T)                                                           \
+    if (form == F && tall == T) {                                             \
+        constexpr int lds = F == LW_PARTS && T == 4 ? 128 * 260 * 4 : LW_LDS; \
+        hipLaunchKernelGGL((linear_wide_kernel<F, T>), dim3(TM * TN * S),     \
+                           dim3(512), lds, stream, x, w, out, M, N, K, S, TM, \
+                           TN, strip);                                        \
+        return 0;                                                             \
+    }
+    LW_GO(LW_ROWS, 2)
+    LW_GO(LW_ROWS, 3)
+    LW_GO(LW_ROWS, 4)
+    LW_GO(LW_GATED, 2)
+    LW_GO(LW_GATED, 3)
+    LW_GO(LW_GATED, 4)
+    LW_GO(LW_PARTS, 2)
+    LW_GO(LW_PARTS, 3)
+    LW_GO(LW_PARTS, 4)
+#undef LW_GO
+    return 1;
+}

@@ -1,8 +1,9 @@
 // Torch bindings of the projections of a few rows (linear_rows.hip) and of some
-// tens (linear_mid.hip), and of the pass between q|k|v and attention.
+// tens (linear_mid.hip) and more (linear_wide.hip), and of the pass between q|k|v and attention.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
+#include <limits>
 
 using torch::Tensor;
 using c10::optional;
@@ -18,6 +19,10 @@ extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
                                  const unsigned short*, void*, int, int, int,
                                  int, int, int, const float*, float,
                                  hipStream_t);
+extern "C" int linear_wide_plan(int, int, int, int);
+extern "C" int launch_linear_wide(const unsigned short*, const unsigned short*,
+                                  void*, int, int, int, int, int, int,
+                                  hipStream_t);
 extern "C" int launch_add_norm_parts(
     const float*, const unsigned short*, const unsigned short*,
     const unsigned short*, const unsigned short*, unsigned short*,
@@ -274,6 +279,38 @@ Tensor mid_rows_linear(const Tensor& x, const Tensor& w,
     return y;
 }
 
+// Wide products: forms of linear_wide.hip
+enum { WIDE_ROWS = 0, WIDE_GATED = 1, WIDE_PARTS = 2 };
+
+int64_t wide_plan(int64_t M, int64_t N, int64_t K, int64_t form) {
+    TORCH_CHECK(form >= WIDE_ROWS && form <= WIDE_PARTS);
+    const int64_t most = std::numeric_limits<int>::max();
+    if (M > most || N > most || K > most) return 0;
+    return linear_wide_plan(M, N, K, form);
+}
+
+// x w^T in bf16; silu(gate) * value of w's two halves (gated); or, where the
+// plan has several parts, [S, M, N] fp32
+Tensor wide_linear(const Tensor& x, const Tensor& w, int64_t plan,
+                   bool gated) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
+                "x [M, K] and w [N, K]");
+    const int64_t tall = plan % 8, S = plan / 8;
+    TORCH_CHECK(tall >= 2 && tall <= 4 && S >= 1 && S <= 8, "a plan");
+    TORCH_CHECK(!gated || (S == 1 && w.size(0) % 16 == 0));
+    TORCH_CHECK(x.size(0) >= 1 && x.size(1) % 64 == 0 &&
+                x.size(1) >= 128 * S && w.size(0) % 8 == 0);
+    const Tensor xd = dense(x, "x"), wd = dense(w, "w");
+    const int M = x.size(0), K = x.size(1), N = w.size(0) / (gated ? 2 : 1);
+    const int form = gated ? WIDE_GATED : S > 1 ? WIDE_PARTS : WIDE_ROWS;
+    Tensor y = S > 1 ? torch::empty({S, M, N},
+                                    x.options().dtype(torch::kFloat32))
+                     : torch::empty({M, N}, xd.options());
+    TORCH_CHECK(launch_linear_wide(ptr(xd), ptr(wd), y.data_ptr(), M, N, K,
+                                   S, form, tall, stream()) == 0);
+    return y;
+}
+
 const float* parts(const Tensor& t, long M, long N) {
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
                 t.is_contiguous() && t.dim() == 3 && t.size(1) == M &&
@@ -389,6 +426,10 @@ void register_rows_ops(pybind11::module_& m) {
           "projection of some tens of rows as fp32 parts over K");
     m.def("mid_rows_linear", &mid_rows_linear,
           "projection of some tens of rows, with bias and activation");
+    m.def("wide_plan", &wide_plan,
+          "tile and parts of a projection of many rows, 0 for the library");
+    m.def("wide_linear", &wide_linear,
+          "projection of many rows, gated or as parts where wanted");
     m.def("add_norm_parts", &add_norm_parts,
           "residual add of a projection's parts, and the next norm");
     m.def("decode_slots", &decode_slots, "page slots of a decode step's rows");

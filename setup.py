@@ -27,6 +27,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "rows_ext.cpp"),
         os.path.join(CSRC, "linear_rows.hip"),
         os.path.join(CSRC, "linear_mid.hip"),
+        os.path.join(CSRC, "linear_wide.hip"),
         os.path.join(CSRC, "probe.hip"),
         os.path.join(CSRC, "grouped_gemm.hip"),
         os.path.join(CSRC, "hybrid_ext.cpp"),

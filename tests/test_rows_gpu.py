@@ -285,6 +285,33 @@ def test_long_gated_projections_of_few_rows(N, K):
         assert torch.equal(rows(at), got[at])
 
 
+# (rows: edges of halves and of tiles of 128, 192 and 256; 256 columns a tile,
+# 128 gated; 2 steps of K a part, the least, and odd numbers of them)
+@pytest.mark.parametrize("tall", [2, 3, 4])
+@pytest.mark.parametrize("M", [1, 64, 97, 129, 256, 2100])
+@pytest.mark.parametrize("N,K,act,S", [
+    (8, 128, None, 1), (264, 192, None, 1), (2304, 1088, None, 1),
+    (8, 192, "swiglu", 1), (136, 128, "swiglu", 1), (1160, 832, "swiglu", 1),
+    (264, 256, None, 2), (512, 1088, None, 3), (1032, 4096, None, 8)])
+def test_wide_products(M, N, K, act, S, tall):
+    """As the activated rows and the parts above."""
+    torch.manual_seed(M + N)
+    x, w = _rand(M, K), _rand(2 * N if act else N, K, std=0.1)
+    got = ops.wide_linear(x, w, tall + 8 * S, act).double()
+    want = x.double() @ w.double().t()
+    e = 2 ** -24 * K * (x.double().abs() @ w.double().abs().t())
+    if S > 1:
+        assert got.shape == (S, M, N)
+        assert ((got.sum(0) - want).abs() <= e).all()
+        return
+    if act:
+        (g, u), (eg, eu) = want.chunk(2, -1), e.chunk(2, -1)
+        want = F.silu(g) * u
+        e = 1.13 * eg * u.abs() + F.silu(g).abs() * eu + 1.13 * eg * eu
+    assert ((got - want).abs() <= e + (2 ** -8 + 2 ** -20) * want.abs()
+            + 1e-6).all()
+
+
 @pytest.mark.parametrize("S,M,H", [(1, 17, 64), (8, 128, 4096), (4, 20, 8192),
                                    (2, 33, 3592)])
 @pytest.mark.parametrize("kind", [None, "rms", "layer"])
