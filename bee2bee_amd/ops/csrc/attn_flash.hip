@@ -16,6 +16,14 @@
 //  * Keys and values are staged in LDS row-major (two buffers), 16-byte chunks
 //    xor-ed by the key, the next tile's global reads in flight over the
 //    current tile's products.
+//  * 256 rows at head size 128 (TURNS): eight waves, two a SIMD, that take
+//    turns: while one multiplies (O of the last tile, S of the next), the other
+//    takes its maximum, weights and sum, with a barrier at each change. Left to
+//    themselves both multiply, then both wait for the vector units: the sum of
+//    the two times was 4400 clocks a tile of 64 keys, where each takes 2000 of
+//    both waves; in turns it is 3400. Fragments are read two groups of products
+//    ahead, tiles go straight to one of four LDS buffers two and three tiles
+//    ahead (no registers, no divisions by the page size in the loop).
 //  * At head size 128 the running maximum is raised only by a score FL_SLACK
 //    powers of two above it: most tiles leave the sums as they are. Sums are
 //    fp32, of the weights as rounded for the product, so that most of what
@@ -23,13 +31,14 @@
 // Scores are scaled in fp32 (queries enter the product unrounded). The kernel
 // before it (16-row tiles, weights and V transposed through LDS by 2-byte
 // writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
-// of 28 heads on 16384 keys 860 us instead of 5240 (980 TFLOP/s), 2048 tokens
-// of 32 heads 63 us instead of 386 (540), nine prompts of 112 to 901 tokens
-// 38 us instead of 140. Neither fetching key fragments two steps ahead by hand
-// nor computing the next tile's scores beside this one's exponentials (with
-// or without a forced interleaving) made it faster: at 980 TFLOP/s the clock
-// has come down to 1.75 GHz.
+// of 28 heads on 16384 keys 763 us (1100 TFLOP/s; 890 without turns), four
+// prompts of 512 to 4096 tokens of 28 heads 245 (284 as 128 rows without
+// turns), 2048 tokens of 32 heads 55 (59), nine prompts of 112 to 901 tokens
+// 35. How much of the weights is left to the turn that multiplies them makes no
+// difference; without s_setprio for the multiplying waves 1 to 2% are lost.
 #include "common.h"
+
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) short short4v;
@@ -47,7 +56,25 @@ constexpr int FL_KT = 64;   // keys per staged tile
 // 945, 700 on 7700 160 against 171), 1 to 3% at 64.
 template <int HD> constexpr float FL_SLACK = HD == 128 ? 8.f : 0.f;
 
-template <int HD, int RW, int KSP, bool PAGED, typename KVT>
+// 8 cache elements as they lie, widened when they are stored
+DEV_INLINE bf16x8 fl_raw(const unsigned short* p) { return load_kv8_bf16(p); }
+DEV_INLINE uint2v fl_raw(const unsigned char* p) {
+    return *reinterpret_cast<const uint2v*>(p);
+}
+DEV_INLINE bf16x8 fl_bf16(bf16x8 r) { return r; }
+DEV_INLINE bf16x8 fl_bf16(uint2v r) {
+    return load_kv8_bf16(reinterpret_cast<const unsigned char*>(&r));
+}
+
+// 16 bytes a lane to LDS at `to` + lane * 16, from base + off. The compiler
+// does not see these loads: the kernel waits for them itself.
+DEV_INLINE void fl_load(const char* base, unsigned off, unsigned to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, %1"
+                 ::"v"(off), "s"(base), "s"(to) : "memory");
+}
+
+template <int HD, int RW, int KSP, bool PAGED, bool TURNS, typename KVT>
 __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k,
     const KVT* __restrict__ v, const int* __restrict__ cu,
@@ -64,6 +91,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     constexpr int RPT = NW * 64 / CPR;     // key rows staged at once
     constexpr int NST = FL_KT / RPT;       // staging steps of a tile
     constexpr int TILE = FL_KT * RB;       // bytes of a K or V tile
+    static_assert(!TURNS || (HD == 128 && RW == 8 && KSP == 1), "");
     static_assert(FL_KT % RPT == 0, "whole staging steps");
 
     // workgroups go round the 8 dies in turn: heads fastest, so that a key
@@ -89,7 +117,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const int f0 = KSP == 1 ? 0 : wid / RW;       // its first 32-key tile
 
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    // two buffers of a K and a V tile each
+    // two buffers, or four, of a K and a V tile each
 
     // ---- this lane's query row
     const int R = row0 + rw * 32 + lr;
@@ -106,10 +134,12 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const int see = hist + pos;                    // last key this row sees
     // of the wave: the earliest row's last key, and the end of all its keys
     const int wr0 = row0 + rw * 32;
-    const int w_first = hist + min(wr0, QL * G - 1) / G;
-    const int w_end =
-        wr0 < QL * G ? hist + min(wr0 + 31, QL * G - 1) / G + 1 : 0;
-    const int kv_end = hist + min(row0 + ROWS - 1, QL * G - 1) / G + 1;
+    const int w_first =
+        __builtin_amdgcn_readfirstlane(hist + min(wr0, QL * G - 1) / G);
+    const int w_end = __builtin_amdgcn_readfirstlane(
+        wr0 < QL * G ? hist + min(wr0 + 31, QL * G - 1) / G + 1 : 0);
+    const int kv_end = __builtin_amdgcn_readfirstlane(
+        hist + min(row0 + ROWS - 1, QL * G - 1) / G + 1);
 
     // Chunks of a staged row are xor-ed so that no two lanes served together
     // meet in a bank. LDS serves 256 bytes a clock: 16 lanes of a 16-byte read
@@ -122,32 +152,40 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     };
     // ---- staging: thread -> (key row, chunk)
     const int st_row = tid / CPR, st_c = tid % CPR;
-    bf16x8 rk[NST], rv[NST];
-    // pages of whole tiles: a tile's page is one scalar look-up
+    typedef decltype(fl_raw((const KVT*)nullptr)) Raw;
+    Raw rk[NST], rv[NST];
+    // Tiles are loaded in order. Pages of whole tiles: a tile's page is one
+    // scalar look-up, made a tile ahead.
     const bool whole_pages = PAGED && bs % FL_KT == 0;
+    int page = 0, in_page = 0, page_at = 0;
+    if (whole_pages && kv_end > 0) page = bt[0];
     auto load_tile = [&](int kb) {
-        long tile_off = 0;
-        if (whole_pages)
-            tile_off =
-                (((long)bt[kb / bs] * nkv + kvh) * bs + kb % bs) * HD;
+        if (PAGED && !whole_pages) {
+#pragma unroll
+            for (int i = 0; i < NST; ++i) {
+                const int key = min(kb + st_row + i * RPT, kv_end - 1);
+                const long off = (((long)bt[key / bs] * nkv + kvh) * bs +
+                                  key % bs) * HD + st_c * 8;
+                rk[i] = fl_raw(k + off);
+                rv[i] = fl_raw(v + off);
+            }
+            return;
+        }
+        const long off = PAGED ? (((long)page * nkv + kvh) * bs + in_page) * HD
+                               : (long)kvh * HD;
+        const KVT* kt = k + (PAGED ? off : off + (long)(s0 + kb) * s_k);
+        const KVT* vt = v + (PAGED ? off : off + (long)(s0 + kb) * s_v);
 #pragma unroll
         for (int i = 0; i < NST; ++i) {
-            const int key = min(kb + st_row + i * RPT, kv_end - 1);
-            if (PAGED) {
-                const long off =
-                    (whole_pages
-                         ? tile_off + (long)(key - kb) * HD
-                         : (((long)bt[key / bs] * nkv + kvh) * bs +
-                            key % bs) * HD) +
-                    st_c * 8;
-                rk[i] = load_kv8_bf16(k + off);
-                rv[i] = load_kv8_bf16(v + off);
-            } else {
-                rk[i] = load_kv8_bf16(k + (long)(s0 + key) * s_k +
-                                      (long)kvh * HD + st_c * 8);
-                rv[i] = load_kv8_bf16(v + (long)(s0 + key) * s_v +
-                                      (long)kvh * HD + st_c * 8);
-            }
+            const int row = min(st_row + i * RPT, kv_end - 1 - kb);
+            rk[i] = fl_raw(kt + (unsigned)(row * (PAGED ? HD : (int)s_k) +
+                                           st_c * 8));
+            rv[i] = fl_raw(vt + (unsigned)(row * (PAGED ? HD : (int)s_v) +
+                                           st_c * 8));
+        }
+        if (PAGED && kb + FL_KT < kv_end && (in_page += FL_KT) == bs) {
+            in_page = 0;
+            page = bt[++page_at];
         }
     };
     auto store_tile = [&](int buf) {
@@ -156,10 +194,10 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
 #pragma unroll
         for (int i = 0; i < NST; ++i) {
             const int row = st_row + i * RPT;
-            *reinterpret_cast<bf16x8*>(kd + row * RB +
-                                       ((st_c ^ k_swz(row)) << 4)) = rk[i];
             *reinterpret_cast<bf16x8*>(
-                vd + row * RB + ((st_c ^ v_swz(row)) << 4)) = rv[i];
+                kd + row * RB + ((st_c ^ k_swz(row)) << 4)) = fl_bf16(rk[i]);
+            *reinterpret_cast<bf16x8*>(
+                vd + row * RB + ((st_c ^ v_swz(row)) << 4)) = fl_bf16(rv[i]);
         }
     };
 
@@ -185,88 +223,304 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
     float m = -1e30f, l = 0.f;
 
-    if (kv_end > 0) {
-        load_tile(0);
-        store_tile(0);
-    }
-    int buf = 0;
-    for (int kb = 0; kb < kv_end; kb += FL_KT, buf ^= 1) {
-        __syncthreads();
-        const bool more = kb + FL_KT < kv_end;
-        if (more) load_tile(kb + FL_KT);
-        if (kb < w_end) {
-            const char* base = smem + buf * 2 * TILE;
-            // ---- S^T = K Q^T: column = query row, rows = keys
-            f32x16 s[NF];
+    // ---- S^T = K Q^T: column = query row, rows = keys
+    f32x16 s[NF];
+    auto scores = [&](const char* base) {
 #pragma unroll
-            for (int f = 0; f < NF; ++f) {
+        for (int f = 0; f < NF; ++f) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[f][r] = 0.f;
+            for (int r = 0; r < 16; ++r) s[f][r] = 0.f;
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    const bf16x8 ak = *reinterpret_cast<const bf16x8*>(
-                        base + (f0 + f) * 32 * RB + k_base +
-                        (((ks * 2 + hi) ^ k_sw) << 4));
-                    s[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        ak, bq[ks], s[f], 0, 0, 0);
-                }
+            for (int ks = 0; ks < KS; ++ks) {
+                const bf16x8 ak = *reinterpret_cast<const bf16x8*>(
+                    base + (f0 + f) * 32 * RB + k_base +
+                    (((ks * 2 + hi) ^ k_sw) << 4));
+                s[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ak, bq[ks],
+                                                               s[f], 0, 0, 0);
             }
-            if (kb + FL_KT - 1 > w_first) {
-#pragma unroll
-                for (int f = 0; f < NF; ++f)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int key =
-                            kb + (f0 + f) * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                        if (key > see) s[f][r] = -INFINITY;
-                    }
-            }
-            // ---- online softmax, in powers of two
-            float mx = s[0][0];
+        }
+    };
+    // ---- online softmax, in powers of two, of the tile at key kb
+    bf16x8 bp[NF * 2];
+    auto weights = [&](int kb) {
+        if (kb + FL_KT - 1 > w_first) {
 #pragma unroll
             for (int f = 0; f < NF; ++f)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[f][r]);
-            mx = pair_max(mx) * scale_log2;
-            if (__any(mx > m + FL_SLACK<HD>)) {
-                const float mn = fmaxf(m, mx);
-                const float alpha = __builtin_amdgcn_exp2f(m - mn);
-                m = mn;
-                l *= alpha;
-#pragma unroll
-                for (int d = 0; d < DT; ++d)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-            }
-            bf16x8 bp[NF * 2];
-#pragma unroll
-            for (int f = 0; f < NF; ++f)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    bp[f * 2 + r / 8][r % 8] = (__bf16)__builtin_amdgcn_exp2f(
-                        fmaf(s[f][r], scale_log2, -m));
-            // the sum that divides is of the weights as they are multiplied
-#pragma unroll
-            for (int st = 0; st < NF * 2; ++st) l = add_bf16x8(bp[st], l);
-            // ---- O^T += V^T P^T; the keys of a step in the order the score
-            // tile holds them: 4 hi + {0..3}, then 8 + 4 hi + {0..3}
-#pragma unroll
-            for (int st = 0; st < NF * 2; ++st)
-#pragma unroll
-                for (int d = 0; d < DT; ++d) {
-                    const char* va =
-                        base + v_off[d] + (f0 * 2 + st) * 16 * RB;
-                    const short4v a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (lds_short4v*)va);
-                    const short4v a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (lds_short4v*)(va + 8 * RB));
-                    const short8 av = __builtin_shufflevector(
-                        a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, av), bp[st], o[d], 0, 0, 0);
+                for (int r = 0; r < 16; ++r) {
+                    const int key =
+                        kb + (f0 + f) * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+                    if (key > see) s[f][r] = -INFINITY;
                 }
         }
-        if (more) store_tile(buf ^ 1);
+        float mx = s[0][0];
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[f][r]);
+        mx = pair_max(mx) * scale_log2;
+        if (__any(mx > m + FL_SLACK<HD>)) {
+            const float mn = fmaxf(m, mx);
+            const float alpha = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                bp[f * 2 + r / 8][r % 8] = (__bf16)__builtin_amdgcn_exp2f(
+                    fmaf(s[f][r], scale_log2, -m));
+        // the sum that divides is of the weights as they are multiplied
+#pragma unroll
+        for (int st = 0; st < NF * 2; ++st) l = add_bf16x8(bp[st], l);
+    };
+    // ---- O^T += V^T P^T; the keys of a step in the order the score tile holds
+    // them: 4 hi + {0..3}, then 8 + 4 hi + {0..3}
+    auto outputs = [&](const char* base) {
+#pragma unroll
+        for (int st = 0; st < NF * 2; ++st)
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const char* va = base + v_off[d] + (f0 * 2 + st) * 16 * RB;
+                const short4v a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_short4v*)va);
+                const short4v a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_short4v*)(va + 8 * RB));
+                const short8 av = __builtin_shufflevector(a0, a1, 0, 1, 2, 3,
+                                                          4, 5, 6, 7);
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, av), bp[st], o[d], 0, 0, 0);
+            }
+    };
+
+    if constexpr (TURNS) {
+        // Two waves a SIMD: while one multiplies, O of the last tile and S of
+        // this one, the other takes its weights.
+        constexpr bool DIRECT = sizeof(KVT) == 2;
+        auto turn = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto at = [&](int t) { return smem + (t & 3) * 2 * TILE; };
+        // bf16 goes straight to LDS: a wave's loads are 4 rows of 256 bytes,
+        // lane l the 16 bytes that belong at l * 16
+        const int nt = (kv_end + FL_KT - 1) / FL_KT;
+        unsigned off[2][2][NST];               // K, V; a whole tile, the last
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+            const int row = (i * 8 + wid) * 4 + (lane >> 4);
+            const int left = kv_end - 1 - (nt - 1) * FL_KT;
+            const int kc = ((lane & 15) ^ k_swz(row)) << 4;
+            const int vc = ((lane & 15) ^ v_swz(row)) << 4;
+            const int ks = PAGED ? RB : (int)s_k * 2;
+            const int vs = PAGED ? RB : (int)s_v * 2;
+            off[0][0][i] = row * ks + kc;
+            off[1][0][i] = row * vs + vc;
+            // (rows past the last: its)
+            off[0][1][i] = min(row, left) * ks + kc;
+            off[1][1][i] = min(row, left) * vs + vc;
+        }
+        const unsigned lds =
+            (unsigned)(unsigned long)(__attribute__((address_space(3)))
+                                          const char*)smem + wid * 1024;
+        // Tiles are asked for in order, K's one ahead of V's: where the next
+        // ones lie in memory and in LDS, and what is left of K's page.
+        const char *k_src = nullptr, *v_src = nullptr, *v_next = nullptr;
+        int k_to = 0, v_to = TILE, k_left = 0, k_at = 0;
+        auto page_of = [&](const KVT* pool, int b) {
+            return reinterpret_cast<const char*>(
+                pool + ((long)b * nkv + kvh) * bs * HD);
+        };
+        if (DIRECT && nt > 0) {
+            if (PAGED) {
+                const int b = bt[0];
+                k_src = page_of(k, b);
+                v_src = page_of(v, b);
+                k_left = bs;
+            } else {
+                k_src = reinterpret_cast<const char*>(
+                    k + (long)s0 * s_k + (long)kvh * HD);
+                v_src = reinterpret_cast<const char*>(
+                    v + (long)s0 * s_v + (long)kvh * HD);
+            }
+            v_next = v_src;
+        }
+        int new_page = 0;                      // asked for a turn ahead
+        auto load_k = [&](int t) {
+            if (t >= nt) return;
+            if (t + 1 == nt)
+#pragma unroll
+                for (int i = 0; i < NST; ++i) off[0][0][i] = off[0][1][i];
+            if (PAGED && k_left == 0) {
+                k_src = page_of(k, new_page);
+                v_next = page_of(v, new_page);
+                k_left = bs;
+            }
+#pragma unroll
+            for (int i = 0; i < NST; ++i)
+                fl_load(k_src, off[0][0][i], lds + k_to + i * 8192);
+            k_to = (k_to + 2 * TILE) & (8 * TILE - 1);
+            k_src += PAGED ? FL_KT * RB : s_k * FL_KT * 2;
+            if (PAGED && (k_left -= FL_KT) == 0 && t + 1 < nt)
+                new_page = bt[++k_at];
+        };
+        auto load_v = [&](int t) {
+            if (t >= nt) return;
+            if (t + 1 == nt)
+#pragma unroll
+                for (int i = 0; i < NST; ++i) off[1][0][i] = off[1][1][i];
+            v_src = v_next;
+#pragma unroll
+            for (int i = 0; i < NST; ++i)
+                fl_load(v_src, off[1][0][i], lds + v_to + i * 8192);
+            v_to = (v_to + 2 * TILE) & (8 * TILE - 1);
+            v_next = v_src + (PAGED ? FL_KT * RB : s_v * FL_KT * 2);
+        };
+        // Fragments: four groups of V for the products of O, then KS / 2 of K
+        // for S, each read two groups ahead.
+        bf16x8 fr[3][4];
+        auto read_v = [&](const char* base, int g) {
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const char* va = base + v_off[d] + g * 16 * RB;
+                const short4v a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_short4v*)va);
+                const short4v a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds_short4v*)(va + 8 * RB));
+                fr[g % 3][d] = __builtin_bit_cast(
+                    bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5,
+                                                    6, 7));
+            }
+        };
+        auto read_k = [&](const char* base, int g) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)        // two steps of both key tiles
+                fr[(g + 4) % 3][e] = *reinterpret_cast<const bf16x8*>(
+                    base + (e & 1) * 32 * RB + k_base +
+                    (((g * 4 + e / 2 * 2 + hi) ^ k_sw) << 4));
+        };
+        auto make_o = [&](const char* vb, auto more, const char* kb_) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                if (g < 2) read_v(vb, g + 2);
+                else if (decltype(more)::value) read_k(kb_, g - 2);
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+                    o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        fr[g % 3][d], bp[g], o[d], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto make_s = [&](const char* kb_) {
+#pragma unroll
+            for (int g = 0; g < KS / 2; ++g) {
+                if (g + 2 < KS / 2) read_k(kb_, g + 2);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f32x16 z;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) z[r] = 0.f;
+                    s[e & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        fr[(g + 4) % 3][e], bq[g * 2 + e / 2],
+                        g == 0 && e < 2 ? z : s[e & 1], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // the first half of the weights is taken here, not where they are
+        // multiplied; the others between the products
+        auto pin = [&]() {
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                f32x4 u = __builtin_bit_cast(f32x4, bp[st]);
+                asm volatile("" : "+v"(u));
+                bp[st] = __builtin_bit_cast(bf16x8, u);
+            }
+        };
+        if (nt > 0) {
+            if (DIRECT) {
+                load_k(0);
+                load_v(0);
+                load_k(1);
+                load_v(1);
+                load_k(2);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else {
+                load_tile(0);
+                store_tile(0);
+                if (nt > 1) {
+                    load_tile(FL_KT);
+                    store_tile(1);
+                }
+                if (nt > 2) load_tile(2 * FL_KT);
+                __builtin_amdgcn_s_waitcnt(0xc07f);
+            }
+            turn();
+            if (wid >= 4) turn();
+            read_k(at(0), 0);
+            read_k(at(0), 1);
+            make_s(at(0));
+            turn();
+            for (int t = 0; t + 1 < nt; ++t) {
+                // V of tile t + 2 takes the place of t - 2's, K of t + 3 that
+                // of t - 1's: their last readers were in the turn before. What
+                // the last such turn asked for has come by the end of this.
+                if (DIRECT) {
+                    load_v(t + 2);
+                    load_k(t + 3);
+                } else {
+                    if (t + 2 < nt) store_tile((t + 2) & 3);
+                    if (t + 3 < nt) load_tile((t + 3) * FL_KT);
+                }
+                weights(t * FL_KT);
+                pin();
+                if (!DIRECT) __builtin_amdgcn_s_waitcnt(0xc07f);
+                read_v(at(t), 0);
+                read_v(at(t), 1);
+                if (DIRECT) {
+                    if (t + 3 < nt)
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NST)
+                                     : "memory");
+                    else
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+                turn();
+                __builtin_amdgcn_s_setprio(1);
+                make_o(at(t), std::true_type(), at(t + 1));
+                make_s(at(t + 1));
+                __builtin_amdgcn_s_setprio(0);
+                turn();
+            }
+            weights((nt - 1) * FL_KT);
+            read_v(at(nt - 1), 0);
+            read_v(at(nt - 1), 1);
+            make_o(at(nt - 1), std::false_type(), nullptr);
+            if (wid < 4) turn();
+        }
+    } else {
+        if (kv_end > 0) {
+            load_tile(0);
+            store_tile(0);
+        }
+        int buf = 0;
+        for (int kb = 0; kb < kv_end; kb += FL_KT, buf ^= 1) {
+            __syncthreads();
+            const bool more = kb + FL_KT < kv_end;
+            if (more) load_tile(kb + FL_KT);
+            if (kb < w_end) {
+                const char* base = smem + buf * 2 * TILE;
+                scores(base);
+                weights(kb);
+                outputs(base);
+            }
+            if (more) store_tile(buf ^ 1);
+        }
     }
 
     l = pair_sum(l);
@@ -314,59 +568,65 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
 
 // ------------------------------------------------------------- launchers
 
-static int flash_smem(int hd, int rw, int ksp) {
-    const int tiles = 4 * FL_KT * hd * 2;
+static int flash_smem(int hd, int rw, int ksp, bool turns) {
+    const int tiles = (turns ? 8 : 4) * FL_KT * hd * 2;
     const int merge = ksp == 2 ? rw * (hd / 2 + 2) * 64 * 4 : 0;
     return tiles > merge ? tiles : merge;
 }
 
 // Shape of a workgroup by how many of 256 rows the step fills (`full`,
 // T * nq / 256; a CU holds one such workgroup at head size 128, two at 64):
-// 256 rows read a key tile from memory least often and win where there are
-// enough of them and their tiles are about as long as each other (one long
-// prompt's, in falling order, or portions behind long histories); with fewer,
-// 128 rows balance better, with less than a chip of those 64 rows, whose two
-// wave pairs share a tile's keys. Prompts of different lengths leave tiles of
-// every length to balance: 256 rows need 256 fillings a prompt.
+// 256 rows read a key tile from memory least often, at head size 128 take
+// turns at the matrix cores, and win where there are enough of them and their
+// tiles are about as long as each other (one long prompt's, in falling order, or
+// portions behind long histories); with fewer, 128 rows balance better, with
+// less than a chip of those 64 rows, whose two wave pairs share a tile's keys.
+// Prompts of different lengths leave tiles of every length to balance: 256 rows
+// need more of them the more prompts there are.
 // Measured (us, 256 / 128 / 64 rows; heads 32/8 unless stated), head size 128:
-//   one prompt: full 150 42/34/30, 256 70/57/63, 350 92/85/101, 400 107/108/127,
-//    450 121/135/159, 600 218/214/268, 1000 534/549/709;
-//   9 prompts of an eighth to 1: 100 12.9/12.3/10.4, 149 15/14/17, 450
-//    38/34/46 (28/4: 59/45/71), 1000 116/102/141 (28/4: 215/167/248), 1400
-//    191/183/247; 4 prompts: 124 22/19/24, 600 171/161/224, 1000 412/405/561,
-//    2000 1525/1521/2078;
-//   8000 cached: 100 263/220/186, 150 275/288/347, 256 322/346/421, 300
-//    518/503/559, 350 548/527/619, 400 573/632/767, 600 946/930/1143, 1000
-//    1537/1681/2123;
+//   one prompt: full 150 35/34/30, 190 42/44/40, 230 50/53/56, 350 77/83/102,
+//    600 192/212/261, 1000 466/553/687; 2 prompts of an eighth to 1: 150
+//    30/32/39, 600 232/285/396; 4: 149 20.5/19.5/27.6 (28/4: 23/22/20), 299
+//    50/52/71 (28/4: 37/42/50), 1000 316/395/558;
+//   9 prompts: 149 14/13.6/16, 449 39/34/46 (28/4: 54/44/69), 999 109/102/141,
+//    1399 172/181/239 (28/4: 311/289/441), 2000 319/360/468 (28/4:
+//    586/580/840); 30 prompts: 1000 66/61/79, 2000 165/159/221;
+//   8000 cached: 120 206/206/187, 140 210/261/334, 256 287/330/393, 400
+//    489/597/732, 1000 1372/1612/1999; 500 cached: 120 42/37/33, 140 45/44/40,
+//    185 54/53/59, 300 82/84/106, 600 235/250/307;
 // head size 64:
-//   one prompt: 300 54/46/45 (12/12: 140/117/107), 350 64/55/56, 600
-//    135/132/147, 750 184/191/221; 9 prompts: 200 15.2/10.7/11 (12/12:
-//    23/21/17), 600 31/30/34, 1000 59/60/72 (12/12: 151/146/180); 2: 600
-//    157/171/202;
-//   8000 cached: 150 193/187/169, 200 205/195/215, 300 297/272/303, 400
-//    338/391/402, 520 491/476/543, 1000 863/951/1127.
+//   one prompt: 300 53/47/44 (12/12: 139/121/106), 350 64/56/57, 600
+//    134/128/144, 1000 306/313/373; 9 prompts: 300 17/15/16 (12/12: 34/30/26),
+//    600 30/29/34, 1000 61/60/76 (12/12: 146/137/169); 2: 600 152/155/193;
+//   8000 cached: 150 176/177/160, 230 193/192/216, 300 286/264/286, 400
+//    328/357/386, 1000 843/914/1083.
 static int flash_shape(int hd, long full, int nseq, bool pages) {
     const bool lone = !pages && nseq == 1;
     if (hd == 128) {
-        if (full >= 400 && (pages || full >= 256L * nseq)) return 0;
-        return full >= (lone ? 230 : pages ? 140 : 115) ? 1 : 2;
+        if (full >= (pages  ? 140
+                     : lone ? 210
+                            : (nseq <= 4 ? 75 : 150) * (long)nseq))
+            return 0;
+        return full >= 115 && !pages && !lone ? 1 : 2;
     }
     if (full >= (pages ? 400 : 700)) return 0;
     return full >= (lone ? 320 : pages ? 185 : 230) ? 1 : 2;
 }
 
-#define FL_ONE(HDV, RWV, KSPV, PG, KVT)                                       \
+#define FL_ONE(HDV, RWV, KSPV, PG, TU, KVT)                                     \
     hipLaunchKernelGGL(                                                       \
-        (attn_flash_kernel<HDV, RWV, KSPV, PG, KVT>),                         \
+        (attn_flash_kernel<HDV, RWV, KSPV, PG, TU, KVT>),                        \
         dim3((unsigned)((rows + RWV * 32 - 1) / (RWV * 32) * pairs)),         \
-        dim3(RWV * KSPV * 64), flash_smem(HDV, RWV, KSPV), stream, q,         \
+        dim3(RWV * KSPV * 64), flash_smem(HDV, RWV, KSPV, TU), stream, q,     \
         (const KVT*)k, (const KVT*)v, cu, block_table, seq_lens, out, nq,     \
         nkv, s_q, s_k, s_v, W, bs, pairs, scale * LOG2E)
 #define FL_HD(HDV, PG, KVT)                                                   \
     do {                                                                      \
-        if (shape == 0) FL_ONE(HDV, 8, 1, PG, KVT);                           \
-        else if (shape == 1) FL_ONE(HDV, 4, 1, PG, KVT);                      \
-        else FL_ONE(HDV, 2, 2, PG, KVT);                                      \
+        if (shape == 0 && HDV == 128 && turns)                                \
+            FL_ONE(HDV, 8, 1, PG, HDV == 128, KVT);                           \
+        else if (shape == 0) FL_ONE(HDV, 8, 1, PG, false, KVT);               \
+        else if (shape == 1) FL_ONE(HDV, 4, 1, PG, false, KVT);               \
+        else FL_ONE(HDV, 2, 2, PG, false, KVT);                               \
     } while (0)
 
 constexpr float LOG2E = 1.44269504088896340736f;
@@ -385,6 +645,9 @@ extern "C" int launch_attn_flash(
     const int pairs = nseq * nkv;
     const long rows = (long)max_qlen * (nq / nkv);
     const int shape = flash_shape(hd, T * nq / 256, nseq, block_table);
+    // whole tiles in a page; offsets in a tile are of 32 bits
+    const bool turns = block_table ? bs % FL_KT == 0
+                                   : s_k < 1 << 24 && s_v < 1 << 24;
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

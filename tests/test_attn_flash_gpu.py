@@ -88,6 +88,48 @@ def test_chunks_against_pages(nq, nkv, hd, lens, hist, bs, fp8):
     _check(got, want, up(vc))
 
 
+# 256-row workgroups whose waves take turns: 1 to 5 and more tiles of keys, last
+# tiles of 1, 63 and 64, new pages within a workgroup's tiles; scores that climb
+# along the keys raise the maximum in every tile
+@pytest.mark.parametrize("pages", [None, "bf16", "fp8"])
+@pytest.mark.parametrize("nq,nkv,lens,hist,bs", [
+    (64, 64, [1, 65, 130, 520], [0, 63, 62, 1], 64),
+    (64, 8, [300, 300], [5, 700], 256), (28, 4, [1300], [191], 64),
+    (64, 64, [900], [1], 128), (64, 4, [577, 600], [0, 40], 192),
+])
+def test_waves_in_turn(nq, nkv, lens, hist, bs, pages):
+    hd, T = 128, sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q, k, v = _qkv(T, nq, nkv, hd, 5)
+    cu, scale = _cu(lens), hd ** -0.5
+    if pages is None:
+        k = k * torch.linspace(0.5, 3, T, device=DEV)[:, None, None].bfloat16()
+        got = ops.attn_prefill(q, k, v, cu, max(lens), scale)
+        want = reference.attn_prefill(q.float(), k.float(), v.float(), cu,
+                                      max(lens), scale)
+        _check(got, want, v)
+        return
+    total = [a + b for a, b in zip(lens, hist)]
+    W = max(-(-n // bs) for n in total)
+    table = torch.randperm(W * len(lens), generator=g, device=DEV).int()
+    table = table.view(len(lens), W)
+    kc, vc = (torch.randn(W * len(lens), nkv, bs, hd, generator=g,
+                          device=DEV) for _ in range(2))
+    for row in table.tolist():
+        for at, page in enumerate(row):
+            kc[page] *= 0.5 + 2.5 * at / W
+    dt = torch.bfloat16 if pages == "bf16" else torch.float8_e4m3fn
+    kc, vc = kc.to(dt), vc.to(dt)
+    lens_t = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    total_t = torch.tensor(total, dtype=torch.int32, device=DEV)
+    raw = (lambda c: c) if pages == "bf16" else (lambda c: c.view(torch.uint8))
+    got = ops.attn_prefill_paged(q, raw(kc), raw(vc), table, total_t, cu,
+                                 max(lens), scale)
+    want = reference.attn_decode_with_history(
+        q.float(), kc.float(), vc.float(), table, total_t, lens_t, scale)
+    _check(got, want, vc)
+
+
 def test_scores_that_climb():
     """Scores that grow along the keys raise the running maximum tile by
     tile, in steps below and above the kernel's slack."""
