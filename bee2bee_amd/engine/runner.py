@@ -236,7 +236,7 @@ class Runner:
         if rows <= ops.DEEP_MAX:
             return ops.mid_linear if ops.mid_shape(rows, width, depth) else None
         plan = ops.wide_plan(rows, width, depth, "parts")
-        if not plan or (bias and plan < 16):      # (rows come without bias)
+        if not plan or (bias and plan % 128 < 16):    # rows have no bias
             return None
         return lambda x, w: ops.wide_linear(x, w, plan)
 

@@ -308,25 +308,33 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
 }
 
 // Microseconds of a launch as the planner sees it: rounds of 256 workgroups,
-// each with its start and end, a last one that leaves CUs idle a little faster
-// a step. (The steps of 128-row tiles are bound by what L2 gives, not by their
-// products: 0.82 us against 1.26 for twice the rows.)
+// each with its start and end, a last one that leaves CUs idle faster a step.
+// Fitted to 50 sizes of 300 to 9216 rows: the choice below was the fastest of
+// its own in all but one (4% behind). Steps of 128-row tiles take 0.82 us, of 256
+// rows 1.26: they draw 48 KB from L2, not 64, for half the products.
 static double lw_time(int M, int N, int K, int form, int tall, int S) {
-    const double step = tall == 4 ? 1.26 : tall == 3 ? 1.0 : 0.82;
-    const int BN = form == LW_GATED ? 128 : 256;
+    static const double step[] = {0.82, 1.0, 1.26}, idle[] = {0.48, 0.45, 0.56},
+                        busy[] = {0.45, 0.58, 0.46};
+    const int BN = form == LW_GATED ? 128 : 256, i = tall - 2;
     const long tiles = ((M + tall * 64L - 1) / (tall * 64)) *
                        ((N + BN - 1) / BN) * S;
-    const double steps = K / 64 / S, full = tiles / 256,
+    const double steps = K / 64 / S * step[i], full = tiles / 256,
                  left = (tiles % 256) / 256.0;
-    double t = full * (steps * step + tall + 3);
-    if (left > 0) t += steps * step * (0.7 + 0.3 * left) + tall + 3;
+    double t = full * (steps + tall + 3);
+    if (left > 0) {
+        const double f = idle[i] + busy[i] * left;
+        t += steps * (f < 1 ? f : 1) + tall + 3;
+    }
     // the parts, written and read in place of bf16 rows
     if (form == LW_PARTS) t += (double)M * N * (4 * S - 2) / 2.2e6;
     return t;
 }
 
 // The tile's height and number of parts (1: rows) that are fastest: tall + 8 *
-// parts, or 0: left to the library. Parts only where LW_PARTS is asked for.
+// parts, or 0: left to the library. Parts only where LW_PARTS is asked for. +
+// 128: the rows past the last whole tile are linear_mid.hip's, which reads the
+// weights once more for them: where they would begin a round of their own
+// (9217x3584x18944: 37 rows of tiles by 14 are 518 workgroups).
 extern "C" int linear_wide_plan(int M, int N, int K, int form) {
     if (M < 1 || N < 8 || N % 8 || K < 256 || K % 64 || K > 1 << 22) return 0;
     int best = 0;
@@ -334,16 +342,25 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
     for (int tall = 2; tall <= 4; ++tall)
         for (int S = 1; S <= (form == LW_PARTS ? 8 : 1); S *= 2) {
             if (K / 64 / S < 8 && S > 1) break;
-            const double t = lw_time(M, N, K, S == 1 && form == LW_PARTS
-                                                  ? LW_ROWS : form, tall, S);
+            const int f = S == 1 && form == LW_PARTS ? LW_ROWS : form;
+            const double t = lw_time(M, N, K, f, tall, S);
             if (t < least) {
                 least = t;
                 best = tall + 8 * S;
             }
+            const int tail = M % (tall * 64);
+            const double bytes = (f == LW_GATED ? 4.0 : 2.0) * N * K;
+            if (S > 1 || tail == 0 || tail == M || bytes >= 1LL << 32) continue;
+            const double t2 = lw_time(M - tail, N, K, f, tall, 1) + 8 +
+                              bytes / 5.2e6 * (1 + 0.0035 * tail);
+            if (t2 < 0.97 * least) {
+                least = t2;
+                best = tall + 8 + 128;
+            }
         }
     if (form == LW_GATED || K >= 8192) return best;
     const double library = 2.0 * M * N * K / 1.45e9;
-    return least <= library * 1.25 + 8 ? best : 0;
+    return least <= library * 1.25 + 14 ? best : 0;
 }
 
 // x [M, K], w [N, K] (LW_GATED [2N, K]) and out [M, N] (LW_PARTS [S, M, N] fp32)

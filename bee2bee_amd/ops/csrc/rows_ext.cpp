@@ -295,7 +295,7 @@ Tensor wide_linear(const Tensor& x, const Tensor& w, int64_t plan,
                    bool gated) {
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
                 "x [M, K] and w [N, K]");
-    const int64_t tall = plan % 8, S = plan / 8;
+    const int64_t tall = plan % 8, S = plan / 8 % 16;
     TORCH_CHECK(tall >= 2 && tall <= 4 && S >= 1 && S <= 8, "a plan");
     TORCH_CHECK(!gated || (S == 1 && w.size(0) % 16 == 0));
     TORCH_CHECK(x.size(0) >= 1 && x.size(1) % 64 == 0 &&
@@ -306,8 +306,16 @@ Tensor wide_linear(const Tensor& x, const Tensor& w, int64_t plan,
     Tensor y = S > 1 ? torch::empty({S, M, N},
                                     x.options().dtype(torch::kFloat32))
                      : torch::empty({M, N}, xd.options());
-    TORCH_CHECK(launch_linear_wide(ptr(xd), ptr(wd), y.data_ptr(), M, N, K,
-                                   S, form, tall, stream()) == 0);
+    // rows past the last whole tile, if the plan has them apart
+    const int tail = plan >= 128 ? M % (tall * 64) : 0;
+    TORCH_CHECK(plan < 256 && (tail == 0 || (S == 1 && tail < M)), "a plan");
+    TORCH_CHECK(launch_linear_wide(ptr(xd), ptr(wd), y.data_ptr(), M - tail,
+                                   N, K, S, form, tall, stream()) == 0);
+    if (tail)
+        TORCH_CHECK(launch_linear_mid(
+                        ptr(xd) + (long)(M - tail) * K, ptr(wd), nullptr,
+                        mut(y) + (long)(M - tail) * N, tail, N, K, 1,
+                        gated ? 1 : 2, 0, nullptr, 0.f, stream()) == 0);
     return y;
 }
 
