@@ -16,17 +16,21 @@
 // barrier at each change keeps them apart. What a quarter has read is loaded
 // again at once, for the step after next: 3500 clocks ahead, 6 of 8 regions
 // always under way. An XCD's workgroups take neighbouring tiles (8 by 4 at a
-// time), which share what its L2 holds.
+// time), which share what its L2 holds. Where there are more tiles than CUs a
+// workgroup takes several: the next one's first steps are loaded under the last
+// ones of this, whose rows go out from the registers (9216x2x18944x3584 1719 ->
+// 1666 us, 4096x2x18944x3584 776 -> 757, 4559x2x8192x3072 328 -> 316; without
+// swiglu less: 9216x3584x18944 830 -> 822, 1536x128256x4096 1131 -> 1124).
 //
 // Measured (us; in brackets the library's product, and of gated ones its swiglu):
-//   gated 9216x2x18944x3584 1666 (1972), 4096x2x18944x3584 761 (874),
-//    4559x2x8192x3072 323 (468), 1536x2x14336x4096 258 (288), 500x 92 (115);
+//   gated 9216x2x18944x3584 1666 (1972), 4096x2x18944x3584 757 (874),
+//    4559x2x8192x3072 316 (468), 1536x2x14336x4096 257 (288), 500x 92 (115);
 //   rows 9216x3584x18944 800 (807), 4096x3584x18944 372 (531), 4096x4608x3584
 //    110 (122), 1536x6144x4096 63 (70), 1536x128256x4096 1104 (1216);
 //   parts, with the norm that adds them: 1536x4096x14336 141 (179), 1100x 126
 //    (158), 500x 68 (101), 800x2048x8192 36 (48).
-// Tried and slower: workgroups that stay and take tile after tile (3 to 6%: no
-// balance between them), tiles split over K inside one launch, the last to come
+// Tried and slower: an XCD's tiles as one stretch for its workgroups (3 to 6%: some
+// have a round more), tiles split over K inside one launch, the last to come
 // adding (256 KB a tile and part written and read: 40 to 80 us a product).
 #include "common.h"
 
@@ -45,6 +49,12 @@ DEV_INLINE void lw_load(const void* base, unsigned off, unsigned to) {
                  "global_load_lds_dwordx4 %0, %1"
                  ::"v"(off), "s"(base), "s"(to) : "memory");
 }
+// the lane, as a value that is not kept in a register from one use to the next
+DEV_INLINE int lw_lane() {
+    int z = 0;
+    asm volatile("" : "+v"(z));
+    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
 template <int N> DEV_INLINE void lw_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
@@ -62,7 +72,7 @@ template <int FORM, int MT>
 __global__ __launch_bounds__(512) void linear_wide_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
     void* __restrict__ out, int M, int N, int K, int S, int TM, int TN,
-    int strip) {
+    int strip, int stride) {
     constexpr int BM = MT * 64, HM = MT * 32;          // rows, of a half
     constexpr int BN = FORM == LW_GATED ? 128 : 256;   // columns of a tile
     const int tid = threadIdx.x, lane = tid & 63;
@@ -71,27 +81,29 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     const int wm = wid >> 2, wn = wid & 3;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    // ---- the tile: an XCD's workgroups (every eighth) take neighbours, in
-    // strips of `strip` row tiles
-    int t;
-    {
-        const int total = gridDim.x, b = blockIdx.x;
-        const int xcd = b & 7, q = total >> 3, r = total & 7;
-        t = xcd * q + min(xcd, r) + (b >> 3);
-    }
-    const int part = t / (TM * TN);
-    t -= part * TM * TN;
-    const int s0 = t / (strip * TN), h = min(strip, TM - s0 * strip);
-    t -= s0 * strip * TN;
-    const int m0 = (s0 * strip + t % h) * BM, n0 = t / h * BN;
-    const int k0 = K / 64 * part / S, n = K / 64 * (part + 1) / S - k0;
+    // ---- tiles: an XCD's workgroups (every eighth) take neighbours, in strips
+    // of `strip` row tiles; workgroup b its XCD's b / 8, b / 8 + stride, ..
+    const int total = TM * TN * S, xcd = blockIdx.x & 7;
+    const int mine = (total >> 3) + (xcd < (total & 7));       // of this XCD
+    const int t0 = (total >> 3) * xcd + min(xcd, total & 7);
+    int idx = blockIdx.x >> 3;
+    const int n = K / 64 / S;                  // steps of 64: even
+    int part, m0, n0;
+    auto tile = [&](int i) {
+        int t = t0 + i;
+        part = t / (TM * TN);
+        t -= part * TM * TN;
+        const int s0 = t / (strip * TN), h = min(strip, TM - s0 * strip);
+        t -= s0 * strip * TN;
+        m0 = (s0 * strip + t % h) * BM;
+        n0 = t / h * BN;
+    };
+    tile(idx);
 
     // ---- loads: a wave's are 8 rows of 128 bytes, lane l the 16 bytes that
     // belong at l * 16 (xor-ed by half the row's number: no two of a read's 16
     // rows meet in a bank)
-    const char* xb = reinterpret_cast<const char*>(x + (long)m0 * K + k0 * 64);
-    const char* wb = reinterpret_cast<const char*>(w + (long)n0 * K + k0 * 64);
-    const char* wb1 = FORM == LW_GATED ? wb + (long)N * K * 2 : wb;
+    const char *xb, *wb, *wb1;
     // Of each half of w's 256 rows a wave loads 16, of x's MT / 2 times 8 (MT 3:
     // two of one half, one of the other, waves 4-7 the other way round).
     auto first = [&](int g) {                  // its first 8 rows of x's half
@@ -99,21 +111,28 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
                : (wid < 4) == (g == 0) ? wid % 4 * 2 : 8 + wid % 4;
     };
     unsigned xo[2][2], wo[2][2];
+    auto aim = [&]() {                         // at the tile
+        xb = reinterpret_cast<const char*>(x + (long)m0 * K + part * n * 64);
+        wb = reinterpret_cast<const char*>(w + (long)n0 * K + part * n * 64);
+        wb1 = FORM == LW_GATED ? wb + (long)N * K * 2 : wb;
+        const int l = lw_lane(), r8 = l >> 3;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int r8 = lane >> 3;
-        const unsigned c = ((lane & 7) ^ (r8 >> 1)) * 16, c1 = c ^ 64;
+        for (int j = 0; j < 2; ++j) {
+            const unsigned c = ((l & 7) ^ (r8 >> 1)) * 16, c1 = c ^ 64;
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int f = first(g) + j, xr = g * HM + f * 8 + r8;
-            xo[g][j] = (unsigned)min(xr, M - 1 - m0) * K * 2 + (f & 1 ? c1 : c);
-            // (rows past the last: its)
-            const int wr = (FORM == LW_GATED ? 0 : g * 128) + wid * 16 + j * 8 +
-                           r8;
-            wo[g][j] = (unsigned)min(wr, N - 1 - n0) * K * 2 + (j ? c1 : c);
+            for (int g = 0; g < 2; ++g) {
+                const int f = first(g) + j, xr = g * HM + f * 8 + r8;
+                xo[g][j] = (unsigned)min(xr, M - 1 - m0) * K * 2 +
+                           (f & 1 ? c1 : c);
+                // (rows past the last: its)
+                const int wr = (FORM == LW_GATED ? 0 : g * 128) + wid * 16 +
+                               j * 8 + r8;
+                wo[g][j] = (unsigned)min(wr, N - 1 - n0) * K * 2 + (j ? c1 : c);
+            }
         }
-    }
-    const unsigned to = lw_lds(smem);
+    };
+    aim();
+    const unsigned to = __builtin_amdgcn_readfirstlane(lw_lds(smem));
     // regions of a buffer: x's halves, w's halves
     auto load_x = [&](int buf, int g, int step) {
         const char* b = xb + (long)step * 128;
@@ -130,19 +149,27 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     };
     // until at most R regions' loads are under way (in the order w, x 0, w, x 1
     // of a step, the last of them x 1 where AT 1; MT 3: as the wave has it that
-    // issued fewer)
+    // issued fewer), and, behind a whole tile's `stores`, those
+    constexpr int STORES = FORM == LW_GATED ? 2 * MT
+                           : FORM == LW_ROWS ? 4 * MT : 8 * MT;
+    bool stores = false;
     auto wait = [&](auto regions, auto at1) {
         constexpr int R = decltype(regions)::value;
         constexpr bool A = decltype(at1)::value;
         constexpr int W = A ? R / 2 : (R + 1) / 2, X = R - W;
-        lw_wait<W * 2 + (MT == 4 ? X * 2 : MT == 2 ? X : X * 3 / 2)>();
+        constexpr int L = W * 2 + (MT == 4 ? X * 2 : MT == 2 ? X : X * 3 / 2);
+        if (!A && stores) lw_wait<L + STORES>();
+        else lw_wait<L>();
     };
 
     f32x4 acc[2][2][MT][2];                    // half of x, of w, tiles
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < MT * 8; ++i)
-        acc[i / (4 * MT)][i / (2 * MT) & 1][i / 2 % MT][i & 1] =
-            f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MT * 8; ++i)
+            acc[i / (4 * MT)][i / (2 * MT) & 1][i / 2 % MT][i & 1] =
+                f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
     bf16x8 fa[MT][2], fb[2][2][2];
     const int p0 = (lg ^ (li >> 1)) * 16;      // of K 0-31; 32-63: ^ 64
     const char* af = smem + (wm * MT * 16 + li) * 128;
@@ -191,14 +218,14 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     using No = std::false_type;
     using Yes = std::true_type;
 
-    // Step s of parity P = (s + n) & 1 lies in buffer P. Its regions are read in
-    // the order w P, x 0, w !P, x 1, the first in the step before; each is loaded
-    // again, for step s + 2, where all waves have read it, seven reads ahead.
-    auto step = [&](auto par, auto ahead, int s) {
+    // Step s of parity P lies in buffer P. Its regions are read in the order w P, x 0, w !P, x 1, the first in the step before; each is loaded
+    // again, for step s + 2 (`nx`), where all waves have read it, seven reads
+    // ahead. half: after two of the four `stores` have to be done
+    auto step = [&](auto par, auto ahead, int nx, bool half) {
         constexpr int P = decltype(par)::value, L = decltype(ahead)::value;
         // L: steps after this one, 2 standing for more
         read_x(P, 0);
-        if (L == 2) load_w(P, P, s + 2);
+        if (L == 2) load_w(P, P, nx);
         if (L == 2) wait(I6(), No());
         else if (L == 1) wait(I5(), Yes());
         else wait(I1(), Yes());
@@ -206,81 +233,61 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
         products(0, P);
         lw_barrier();
         read_w(P, !P);
-        if (L == 2) load_x(P, 0, s + 2);
+        if (L == 2) load_x(P, 0, nx);
         if (L == 2) wait(I6(), No());
         else if (L == 1) wait(I4(), Yes());
         else wait(I0(), Yes());
         here();
         products(0, !P);
         lw_barrier();
+        if (half) stores = false;
         read_x(P, 1);
-        if (L == 2) load_w(P, !P, s + 2);
+        if (L == 2) load_w(P, !P, nx);
         if (L == 2) wait(I6(), No());
         else if (L == 1) wait(I3(), Yes());
         here();
         products(1, !P);
         lw_barrier();
         if (L) read_w(!P, !P);
-        if (L == 2) load_x(P, 1, s + 2);
+        if (L == 2) load_x(P, 1, nx);
         if (L == 2) wait(I6(), No());
         else if (L == 1) wait(I2(), Yes());
         here();
         products(1, P);
         lw_barrier();
     };
-    auto start = [&](int P) {
-        load_w(P, P, 0);
-        load_x(P, 0, 0);
-        load_w(P, !P, 0);
-        load_x(P, 1, 0);
-        load_w(!P, !P, 1);
-        load_x(!P, 0, 1);
-        load_w(!P, P, 1);
-        load_x(!P, 1, 1);
-        wait(I6(), No());
-        lw_barrier();
-        read_w(P, P);
-        here();
-        // waves 4-7 read while 0-3 multiply, and the other way round
-        if (wid >= 4) lw_barrier();
-    };
-    int s = 0;
-    if (n & 1) {
-        start(1);
-        step(I1(), I2(), 0);
-        s = 1;
-    } else {
-        start(0);
-    }
-    for (; s + 2 < n; s += 2) {
-        step(I0(), I2(), s);
-        step(I1(), I2(), s + 1);
-    }
-    step(I0(), I1(), s);
-    step(I1(), I0(), s + 1);
-    if (wid < 4) lw_barrier();
-
-    // ---- rows to LDS, a half of x's at a time, then out in whole lines.
-    // C layout: column li = row of x, rows lg * 4 + r = columns
-    constexpr int LD = BN + (FORM == LW_PARTS ? 4 : 8);
-    using E = std::conditional_t<FORM == LW_PARTS, float, unsigned short>;
-    E* os = reinterpret_cast<E*>(smem);
+    // ---- C layout: column li = row of x, rows lg * 4 + r = columns. Two tiles of
+    // 16 columns side by side: lane rows swapped so that a lane has 8 columns of
+    // one of them
+    auto finish = [&](int fm, int fn, int fp) {
+        const bool whole = fm + BM <= M && fn + BN <= N;
+        const int l = lw_lane(), lg = l >> 4;
+        const int r0 = fm + wm * MT * 16 + (l & 15);
+        const int c0 = fn + wn * 32 +
+                       (FORM == LW_PARTS ? lg * 4
+                                         : (lg & 1) * 16 + (lg >> 1) * 8);
+        auto put = [&](int row, int col, f32x4 v) {
+            const long at = (long)row * N + col;
+            if (FORM == LW_PARTS)
+                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) +
+                                          (long)fp * M * N + at) = v;
+            else
+                *reinterpret_cast<f32x4*>(
+                    reinterpret_cast<unsigned short*>(out) + at) = v;
+        };
+        auto rows = [&](int gx, int i, int gw, auto all) {
+            const int row = r0 + gx * HM + i * 16, col = c0 + gw * 128;
+            if constexpr (FORM == LW_PARTS) {
 #pragma unroll
-    for (int gx = 0; gx < 2; ++gx) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int gw = 0; gw < (FORM == LW_GATED ? 1 : 2); ++gw)
+                for (int j = 0; j < 2; ++j)
+                    if (decltype(all)::value ||
+                        (row < M && col + j * 16 < N))
+                        put(row, col + j * 16, acc[gx][gw][i][j]);
+            } else {
+                uint2v u[2];
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     f32x4 z = acc[gx][gw][i][j];
-                    E* p = os + ((wm * MT + i) * 16 + li) * LD + gw * 128 +
-                           wn * 32 + j * 16 + lg * 4;
-                    if constexpr (FORM == LW_PARTS) {
-                        *reinterpret_cast<f32x4*>(p) = z;
-                        continue;
-                    }
                     if (FORM == LW_GATED) {
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
@@ -288,23 +295,72 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
                                    __builtin_amdgcn_rcpf(1.f + __expf(-z[r])) *
                                    acc[gx][1][i][j][r];
                     }
-                    *reinterpret_cast<uint2v*>(p) =
-                        uint2v{f2bf(z[0]) | (unsigned)f2bf(z[1]) << 16,
-                               f2bf(z[2]) | (unsigned)f2bf(z[3]) << 16};
+                    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+                    u[j] = __builtin_bit_cast(
+                        uint2v, bf16x4{(__bf16)z[0], (__bf16)z[1], (__bf16)z[2],
+                                       (__bf16)z[3]});
                 }
-        __syncthreads();
-        constexpr int V = 16 / sizeof(E), CH = BN / V;
-        E* to_row = reinterpret_cast<E*>(out) +
-                    (FORM == LW_PARTS ? (long)part * M * N : 0) +
-                    (long)(m0 + gx * HM) * N + n0;
+                const uint2v a =
+                    __builtin_amdgcn_permlane16_swap(u[0][0], u[1][0], false,
+                                                     false);
+                const uint2v b =
+                    __builtin_amdgcn_permlane16_swap(u[0][1], u[1][1], false,
+                                                     false);
+                typedef __attribute__((ext_vector_type(4))) unsigned uint4v;
+                if (decltype(all)::value || (row < M && col < N))
+                    put(row, col, __builtin_bit_cast(
+                                      f32x4, uint4v{a[0], b[0], a[1], b[1]}));
+            }
+        };
+        auto tiles = [&](auto all) {
 #pragma unroll
-        for (int c = tid; c < HM * CH; c += 512) {
-            const int r = c / CH, col = c % CH * V;
-            if (m0 + gx * HM + r < M && n0 + col < N)
-                *reinterpret_cast<f32x4*>(to_row + (long)r * N + col) =
-                    *reinterpret_cast<const f32x4*>(os + r * LD + col);
-        }
+            for (int gx = 0; gx < 2; ++gx)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int gw = 0; gw < (FORM == LW_GATED ? 1 : 2); ++gw)
+                        rows(gx, i, gw, all);
+        };
+        if (whole) tiles(Yes());
+        else tiles(No());
+        stores = whole;
+    };
+    for (int i = 0; i < 2; ++i) {
+        load_w(i, i, i);
+        load_x(i, 0, i);
+        load_w(i, !i, i);
+        load_x(i, 1, i);
     }
+    wait(I6(), No());
+    lw_barrier();
+    read_w(0, 0);
+    here();
+    // waves 4-7 read while 0-3 multiply, and the other way round
+    if (wid >= 4) lw_barrier();
+    int nx = 2;
+    for (;;) {
+        const int fm = m0, fn = n0, fp = part;
+        const bool more = idx + stride < mine;
+        for (int s = 0; s + 2 < n + 2 * more; s += 2) {
+            if (nx == n) {
+                idx += stride;
+                tile(idx);
+                aim();
+                nx = 0;
+            }
+            step(I0(), I2(), nx, false);
+            step(I1(), I2(), nx + 1, true);
+            nx += 2;
+        }
+        if (!more) {
+            step(I0(), I1(), 0, false);
+            step(I1(), I0(), 0, false);
+        }
+        finish(fm, fn, fp);
+        if (!more) break;
+        clear();
+    }
+    if (wid < 4) lw_barrier();
 }
 
 // Microseconds of a launch as the planner sees it: rounds of 256 workgroups,
@@ -336,12 +392,12 @@ static double lw_time(int M, int N, int K, int form, int tall, int S) {
 // weights once more for them: where they would begin a round of their own
 // (9217x3584x18944: 37 rows of tiles by 14 are 518 workgroups).
 extern "C" int linear_wide_plan(int M, int N, int K, int form) {
-    if (M < 1 || N < 8 || N % 8 || K < 256 || K % 64 || K > 1 << 22) return 0;
+    if (M < 1 || N < 8 || N % 8 || K < 256 || K % 128 || K > 1 << 22) return 0;
     int best = 0;
     double least = 1e30;
     for (int tall = 2; tall <= 4; ++tall)
         for (int S = 1; S <= (form == LW_PARTS ? 8 : 1); S *= 2) {
-            if (K / 64 / S < 8 && S > 1) break;
+            if (S > 1 && (K / 64 / S < 8 || K % (128 * S))) break;
             const int f = S == 1 && form == LW_PARTS ? LW_ROWS : form;
             const double t = lw_time(M, N, K, f, tall, S);
             if (t < least) {
@@ -364,25 +420,27 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
 }
 
 // x [M, K], w [N, K] (LW_GATED [2N, K]) and out [M, N] (LW_PARTS [S, M, N] fp32)
-// contiguous, 16-byte aligned; K % 64 == 0, K >= 128 S, N % 8 == 0; S 1 but for
-// LW_PARTS; tall: 2, 3 or 4 times 64 rows a tile. Nonzero for anything else.
+// contiguous, 16-byte aligned; K % (128 S) == 0, N % 8 == 0; S 1 but for LW_PARTS;
+// tall: 2, 3 or 4 times 64 rows a tile. Nonzero for anything else.
 extern "C" int launch_linear_wide(const unsigned short* x,
                                   const unsigned short* w, void* out, int M,
                                   int N, int K, int S, int form, int tall,
                                   hipStream_t stream) {
-    if (M < 1 || N < 8 || N % 8 || S < 1 || K < 128 * S || K % 64) return 1;
+    if (M < 1 || N < 8 || N % 8 || S < 1 || K < 1 || K % (128L * S)) return 1;
     if (form != LW_PARTS && S != 1) return 1;
     if (K > 1 << 22) return 1;                 // offsets in a tile: 32 bits
     const int BN = form == LW_GATED ? 128 : 256, BM = tall * 64;
     const int TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
     if ((long)TM * TN * S > 1 << 30) return 1;
     const int strips = (TM + 7) / 8, strip = (TM + strips - 1) / strips;
+    const bool stay = TM * TN * S > 256;       // a workgroup a CU
+    const dim3 grid(stay ? 256 : TM * TN * S);
+    const int stride = stay ? 32 : 1 << 30;
 #define LW_GO(F, T)                                                           \
     if (form == F && tall == T) {                                             \
-        constexpr int lds = F == LW_PARTS && T == 4 ? 128 * 260 * 4 : LW_LDS; \
-        hipLaunchKernelGGL((linear_wide_kernel<F, T>), dim3(TM * TN * S),     \
-                           dim3(512), lds, stream, x, w, out, M, N, K, S, TM, \
-                           TN, strip);                                        \
+        hipLaunchKernelGGL((linear_wide_kernel<F, T>), grid, dim3(512),       \
+                           LW_LDS, stream, x, w, out, M, N, K, S, TM, TN,     \
+                           strip, stride);                                    \
         return 0;                                                             \
     }
     LW_GO(LW_ROWS, 2)

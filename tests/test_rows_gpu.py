@@ -286,13 +286,17 @@ def test_long_gated_projections_of_few_rows(N, K):
 
 
 # (rows: edges of halves and of tiles of 128, 192 and 256; 256 columns a tile,
-# 128 gated; 2 steps of K a part, the least, and odd numbers of them)
+# 128 gated; 2 steps of K a part, the least, and more. The last four: more tiles
+# than CUs at 2100 rows, so that a workgroup takes several, the loads of one
+# under the last steps and the stores of another.)
 @pytest.mark.parametrize("tall", [2, 3, 4])
 @pytest.mark.parametrize("M", [1, 64, 97, 129, 256, 2100])
 @pytest.mark.parametrize("N,K,act,S", [
-    (8, 128, None, 1), (264, 192, None, 1), (2304, 1088, None, 1),
-    (8, 192, "swiglu", 1), (136, 128, "swiglu", 1), (1160, 832, "swiglu", 1),
-    (264, 256, None, 2), (512, 1088, None, 3), (1032, 4096, None, 8)])
+    (8, 128, None, 1), (264, 256, None, 1), (2304, 1152, None, 1),
+    (8, 256, "swiglu", 1), (136, 128, "swiglu", 1), (1160, 896, "swiglu", 1),
+    (264, 256, None, 2), (512, 1152, None, 3), (1032, 4096, None, 8),
+    (9000, 128, None, 1), (8712, 640, None, 1), (4616, 256, "swiglu", 1),
+    (4104, 768, None, 2)])
 def test_wide_products(M, N, K, act, S, tall):
     """As the activated rows and the parts above."""
     torch.manual_seed(M + N)
