@@ -414,9 +414,17 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
                 best = tall + 8 + 128;
             }
         }
-    if (form == LW_GATED || K >= 8192) return best;
-    const double library = 2.0 * M * N * K / 1.45e9;
-    return least <= library * 1.25 + 14 ? best : 0;
+    if (form == LW_GATED || (form == LW_PARTS && K >= 8192)) return best;
+    double library = 2.0 * M * N * K / 1.45e9 * 1.25 + 14;
+    if (form == LW_ROWS) {
+        // output heads of a few hundred rows are bound by their weights (200
+        // rows, us, the library's in brackets: 32000x4096 76 (71), 128256x4096
+        // 232 (293))
+        const double bytes = 2.0 * N * K;
+        if (least < bytes / 5.05e6 + 24) least = bytes / 5.05e6 + 24;
+        if (library < bytes / 3.7e6) library = bytes / 3.7e6;
+    }
+    return least <= library ? best : 0;
 }
 
 // x [M, K], w [N, K] (LW_GATED [2N, K]) and out [M, N] (LW_PARTS [S, M, N] fp32)

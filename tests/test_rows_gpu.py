@@ -319,6 +319,27 @@ def test_wide_products(M, N, K, act, S, tall):
         assert ((got - want).abs() <= bound).all()
 
 
+def test_wide_plans_are_what_the_kernel_takes():
+    """Whole pairs of steps a part, parts only for a reader that sums them, rows
+    apart only beside whole tiles; sizes that the kernel does not take stay with
+    the library."""
+    for M in (1, 129, 257, 300, 1000, 1536, 4097, 9217, 16384):
+        for N, K in ((8, 256), (768, 3072), (3584, 18944), (4608, 3584),
+                     (14336, 4096), (128256, 4096), (4096, 14336)):
+            for form in ("rows", "gated", "parts"):
+                plan = ops.wide_plan(M, N, K, form)
+                if plan == 0:
+                    assert form != "gated"
+                    continue
+                tall, S, apart = plan % 8, plan // 8 % 16, plan >= 128
+                assert 2 <= tall <= 4 and S in (1, 2, 4, 8) and plan < 256
+                assert K % (128 * S) == 0 and (S == 1 or form == "parts")
+                assert not apart or (S == 1 and 0 < M % (64 * tall) < M)
+    for N, K in ((12, 4096), (4096, 4160), (4096, 128), (4096, 1 << 23)):
+        for form in ("rows", "gated", "parts"):
+            assert ops.wide_plan(4096, N, K, form) == 0
+
+
 @pytest.mark.parametrize("S,M,H", [(1, 17, 64), (8, 128, 4096), (4, 20, 8192),
                                    (2, 33, 3592)])
 @pytest.mark.parametrize("kind", [None, "rms", "layer"])
