@@ -2,8 +2,8 @@
 
 This is the replacement for the reference's `transformers.generate()` hot
 loop (bee2bee/hf.py:84-108): explicit prefill/decode forwards over fused
-weights, paged KV, and the HIP kernel set. Projection GEMMs go through
-F.linear (hipBLASLt); everything fused is ops.* (HIP on GPU).
+weights, paged KV, and the HIP kernel set. Projections of dense stacks are
+ops.* (HIP on GPU) where those are the faster, F.linear (hipBLASLt) otherwise.
 
 Pipeline parallelism: a Runner can own a contiguous layer range; the first
 stage embeds tokens, the last stage applies the final norm + lm_head

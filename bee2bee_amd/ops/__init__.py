@@ -8,14 +8,15 @@ only for CPU tensors (tests and GPU-less plumbing runs).
 
 Kernels (ops/csrc/): fused (add+)RMSNorm, RoPE, paged KV store, paged GQA
 decode attention, MFMA flash prefill attention, SwiGLU, top-k gating, grouped
-expert GEMM, projections of few rows with what stands around them. Other
-projection GEMMs go through hipBLASLt via torch.nn.functional.linear.
+expert GEMM, projections with what stands around them. Other projection GEMMs go
+through hipBLASLt via torch.nn.functional.linear.
 
 Which projections are whose is measured: up to 16 rows (`few_rows`; logits:
 `head_rows`) the kernels of linear_rows.hip, one launch for norm, product and
-what follows; 17 to 160 rows (`mid_rows`) outputs of `mid_shape` by
-linear_mid.hip, split over K; wide outputs and more rows by the library (gate
-and up of 14336 x 4096 at 24 rows: 56 us there, 66 here). The grouped kernel
+what follows; 17 to 256 rows (`mid_rows`, `mid_shape`, `mid_gated`) linear_mid.hip,
+split over K or activated; more rows linear_wide.hip where `wide_plan` says so:
+all gated ones and deep ones, and others unless they leave much of the chip
+idle. The grouped kernel
 driven as a single-segment GEMM loses to the library on all shapes
 (scripts/bench_skinny.py: N/64 workgroups starve the chip); it stays for experts
 because the E-way grid and the device-side segment offsets are what the library
@@ -327,8 +328,9 @@ def mid_shape(rows: int, width: int, depth: int) -> bool:
 
 def mid_gated(rows: int, width: int, depth: int) -> bool:
     """Gated projections that mid_rows_linear takes (width: of one half). What
-    ends it is L2, from which a CU draws all input rows beside its share of the
-    weights. Measured beside the library's product and swiglu (us): 2x14336x4096
+    ends it are the input rows, which each CU draws beside its share of the
+    weights; wide_linear takes the others. Measured beside the library's product
+    and swiglu (us): 2x14336x4096
     36.9 (56.7) at 24 rows, 50.8 (57.8) at 128, 64 (69.6) at 200, 78.6 (71.6) at
     256; 2x18944x3584 44.6 (56.8), 60 (71.6), 68.6 (75.5) at 160, 113 (83) at
     200; 2x8192x2048 14.2 (19.4), 20 (23.5), 26 (30), 29 (33) at 256; 2x2048x768

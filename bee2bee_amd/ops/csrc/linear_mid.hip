@@ -8,9 +8,13 @@
 //  rows    bf16, with bias and tanh-gelu where wanted (the output head, the
 //          feed-forward of the GPT-2 family).
 //
-// Bound by reading the weights once, up to about 128 rows; beyond, by what a CU
-// draws from its L2 (weights and all input rows: about 19 bytes a clock and CU
-// at 200 rows). A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
+// Bound by reading the weights once, up to about 128 rows; beyond, a CU draws 38
+// to 40 GB/s of weights and input rows together at any number of rows (from L2
+// alone it draws 120; at 200 rows a step takes 1900 clocks, of which products
+// 900). Neither halves that read and multiply in turn (200 rows 3 to 7% faster,
+// fewer 2 to 15% slower), nor weights in registers and the input in all of LDS,
+// nor tiles of 128 rows of w in turns with three buffers of both changed that by
+// more. A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
 // workgroup's rows of w, and by all input rows. Four waves fill the one, four
 // the other, straight from memory (global_load_lds: no registers, so 100 KB of
 // loads are under way in each CU), and all eight multiply: the fragments of the
