@@ -157,7 +157,8 @@ class Runner:
                 hidden, W.lm_head, norm=(W.final_norm, W.final_norm_bias,
                                          self.spec.rms_eps))
         normed = self._norm(hidden, W.final_norm, W.final_norm_bias)
-        if self._mid_dims and ops.wide_rows(hidden):
+        if self._mid_dims and hidden.shape[0] > ops.MID_MAX and (
+                ops.deep_rows(hidden) or ops.wide_rows(hidden)):
             plan = ops.wide_plan(hidden.shape[0], *W.lm_head.shape, "rows")
             if plan:
                 return ops.wide_linear(normed, W.lm_head, plan)
@@ -580,7 +581,8 @@ class Runner:
             return self._run_layers_rows(hidden, positions, slot_mapping,
                                          attn_fn, paged)
         s = self.spec
-        if self._mid_dims and (ops.mid_rows(hidden) or ops.wide_rows(hidden)):
+        if self._mid_dims and (ops.mid_rows(hidden) or ops.deep_rows(hidden)
+                               or ops.wide_rows(hidden)):
             return self._run_layers_mid(hidden, positions, slot_mapping,
                                         attn_fn)
         residual = None

@@ -376,9 +376,15 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     return rows <= 64 or tiles * 20 >= full * 19
 
 
+def deep_rows(x: torch.Tensor) -> bool:
+    """Steps of MID_MAX + 1 to DEEP_MAX contiguous bf16 rows on the GPU."""
+    return (x.dim() == 2 and MID_MAX < x.shape[0] <= DEEP_MAX and _use_hip(x)
+            and x.dtype is torch.bfloat16 and x.is_contiguous())
+
+
 def wide_rows(x: torch.Tensor) -> bool:
-    """Steps of more than MID_MAX contiguous bf16 rows on the GPU."""
-    return (x.dim() == 2 and x.shape[0] > MID_MAX and _use_hip(x)
+    """Steps of more than DEEP_MAX contiguous bf16 rows on the GPU."""
+    return (x.dim() == 2 and x.shape[0] > DEEP_MAX and _use_hip(x)
             and x.dtype is torch.bfloat16 and x.is_contiguous())
 
 
@@ -397,6 +403,8 @@ def wide_linear(x, w, plan: int, act=None):
     "swiglu" as in rows_linear."""
     if _use_hip(x):
         return require_hip().wide_linear(x, w, plan, act == "swiglu")
+    if plan // 8 % 16 > 1:
+        return reference.mid_linear(x, w)
     return reference.rows_linear(x, w, act=act)
 
 

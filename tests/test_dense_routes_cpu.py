@@ -92,6 +92,35 @@ def test_a_route_computes_what_the_plain_one_does(spec, route, monkeypatch):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
 
 
+# plans: left to the library, whole rows, 4 parts, rows past the last tile apart
+@pytest.mark.parametrize("plan", [0, 12, 36, 140])
+@pytest.mark.parametrize("spec", [TINY, PRESETS["tiny-gpt2"]],
+                         ids=["swiglu", "gelu"])
+@torch.no_grad()
+def test_steps_of_many_rows_compute_what_the_plain_route_does(spec, plan,
+                                                              monkeypatch):
+    W = _weights(spec)
+    want = _steps(spec, W)
+    taken = []
+    for name in ("few_rows", "mid_rows", "deep_rows"):
+        monkeypatch.setattr(ops, name, lambda *a: False)
+    monkeypatch.setattr(ops, "wide_rows", lambda x: True)
+    for name in ("MID_MAX", "DEEP_MAX"):
+        monkeypatch.setattr(ops, name, 0)
+    monkeypatch.setattr(ops, "wide_plan", lambda rows, width, depth, form: (
+        plan if form == "parts" or plan != 36 else 12))
+    op = ops.wide_linear
+    monkeypatch.setattr(ops, "wide_linear", lambda x, w, plan, act=None: (
+        taken.append((plan, act)), op(x, w, plan, act))[1])
+    got = _steps(spec, W)
+    acts = {act for _, act in taken}
+    assert taken if plan else not taken
+    assert not plan or acts == {None} | (
+        set() if spec.act_type == "gelu" else {"swiglu"})
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_parts_beside_8_bit_pages(fp8):
     """Parts give rows of the pages' type, and bf16 beside 8-bit pages."""
