@@ -31,11 +31,10 @@
 // Scores are scaled in fp32 (queries enter the product unrounded). The kernel
 // before it (16-row tiles, weights and V transposed through LDS by 2-byte
 // writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
-// of 28 heads on 16384 keys 763 us (1100 TFLOP/s; 890 without turns), four
+// of 28 heads on 16384 keys 728 us (1155 TFLOP/s; 890 without turns), four
 // prompts of 512 to 4096 tokens of 28 heads 245 (284 as 128 rows without
 // turns), 2048 tokens of 32 heads 55 (59), nine prompts of 112 to 901 tokens
-// 35. How much of the weights is left to the turn that multiplies them makes no
-// difference; without s_setprio for the multiplying waves 1 to 2% are lost.
+// 35. Without s_setprio for the multiplying waves 1 to 2% are lost.
 #include "common.h"
 
 #include <type_traits>
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     };
     // ---- online softmax, in powers of two, of the tile at key kb
     bf16x8 bp[NF * 2];
-    auto weights = [&](int kb) {
+    auto maximum = [&](int kb) {
         if (kb + FL_KT - 1 > w_first) {
 #pragma unroll
             for (int f = 0; f < NF; ++f)
@@ -269,12 +268,17 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
         }
+    };
+    auto weight = [&](int st, int e) {
+        bp[st][e] = (__bf16)__builtin_amdgcn_exp2f(
+            fmaf(s[st / 2][st % 2 * 8 + e], scale_log2, -m));
+    };
+    auto weights = [&](int kb) {
+        maximum(kb);
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
+        for (int st = 0; st < NF * 2; ++st)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                bp[f * 2 + r / 8][r % 8] = (__bf16)__builtin_amdgcn_exp2f(
-                    fmaf(s[f][r], scale_log2, -m));
+            for (int e = 0; e < 8; ++e) weight(st, e);
         // the sum that divides is of the weights as they are multiplied
 #pragma unroll
         for (int st = 0; st < NF * 2; ++st) l = add_bf16x8(bp[st], l);
@@ -302,6 +306,14 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         // Two waves a SIMD: while one multiplies, O of the last tile and S of
         // this one, the other takes its weights.
         constexpr bool DIRECT = sizeof(KVT) == 2;
+        // The first 32 keys' weights are taken before the turn ends, and kept from
+        // moving to where they are multiplied. Against pages the other 32 keys'
+        // follow two after each product of the first, in its shadow: 4096 queries
+        // of 28 heads on 16384 keys 743 -> 728 us (fp8 776 -> 762), two portions
+        // of 700 on 8400 198 -> 190, 512 of 32 heads on 8512 197 -> 188. Whole
+        // prompts are faster with them before the turn's end, as far as the
+        // compiler leaves them there (four of 512 to 4096 236, against 242).
+        constexpr bool SHADOW = PAGED;
         auto turn = [&]() {
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_barrier" ::: "memory");
@@ -411,9 +423,18 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 if (g < 2) read_v(vb, g + 2);
                 else if (decltype(more)::value) read_k(kb_, g - 2);
 #pragma unroll
-                for (int d = 0; d < DT; ++d)
+                for (int d = 0; d < DT; ++d) {
                     o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                         fr[g % 3][d], bp[g], o[d], 0, 0, 0);
+                    if (!SHADOW) continue;
+                    if (g < 2) {
+                        weight(g + 2, d * 2);
+                        weight(g + 2, d * 2 + 1);
+                    } else if (d == 0) {
+                        l = add_bf16x8(bp[g], l);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -433,15 +454,21 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        // the first half of the weights is taken here, not where they are
-        // multiplied; the others between the products
-        auto pin = [&]() {
+        auto first_weights = [&](int kb) {
+            maximum(kb);
+#pragma unroll
+            for (int st = 0; st < (SHADOW ? 2 : 4); ++st)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) weight(st, e);
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 f32x4 u = __builtin_bit_cast(f32x4, bp[st]);
                 asm volatile("" : "+v"(u));
                 bp[st] = __builtin_bit_cast(bf16x8, u);
             }
+#pragma unroll
+            for (int st = 0; st < (SHADOW ? 2 : 4); ++st)
+                l = add_bf16x8(bp[st], l);
         };
         if (nt > 0) {
             if (DIRECT) {
@@ -478,8 +505,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                     if (t + 2 < nt) store_tile((t + 2) & 3);
                     if (t + 3 < nt) load_tile((t + 3) * FL_KT);
                 }
-                weights(t * FL_KT);
-                pin();
+                first_weights(t * FL_KT);
                 if (!DIRECT) __builtin_amdgcn_s_waitcnt(0xc07f);
                 read_v(at(t), 0);
                 read_v(at(t), 1);
@@ -497,7 +523,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 __builtin_amdgcn_s_setprio(0);
                 turn();
             }
-            weights((nt - 1) * FL_KT);
+            first_weights((nt - 1) * FL_KT);
             read_v(at(nt - 1), 0);
             read_v(at(nt - 1), 1);
             make_o(at(nt - 1), std::false_type(), nullptr);
