@@ -660,20 +660,24 @@ constexpr float LOG2E = 1.44269504088896340736f;
 // Whole packed prompts, or (block_table given) query chunks whose keys come
 // from the pages only, bf16 or fp8 bytes. T: query tokens of the step. Head
 // size 64 or 128 and a positive scale (a row's maximum is taken before it);
-// nonzero for any other.
+// keys and values of packed prompts 16-byte aligned, row strides multiples of 8
+// below 2^24 (a tile's offsets are of 32 bits). Nonzero for any other.
 extern "C" int launch_attn_flash(
     const unsigned short* q, const void* k, const void* v, const int* cu,
     const int* block_table, const int* seq_lens, unsigned short* out, long T,
     int nseq, int nq, int nkv, int hd, long s_q, long s_k, long s_v, int W,
     int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
     if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
+    const bool aligned = ((unsigned long)k | (unsigned long)v) % 16 == 0;
+    if (!block_table && (!aligned || s_k % 8 || s_v % 8 || s_k >= 1 << 24 ||
+                         s_v >= 1 << 24))
+        return 1;
     if (nseq == 0 || max_qlen <= 0) return 0;
     const int pairs = nseq * nkv;
     const long rows = (long)max_qlen * (nq / nkv);
     const int shape = flash_shape(hd, T * nq / 256, nseq, block_table);
-    // whole tiles in a page; offsets in a tile are of 32 bits
-    const bool turns = block_table ? bs % FL_KT == 0
-                                   : s_k < 1 << 24 && s_v < 1 << 24;
+    // whole tiles in a page, in pieces that go straight to LDS
+    const bool turns = !block_table || (bs % FL_KT == 0 && aligned);
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

@@ -320,20 +320,30 @@ std::vector<Tensor> attn_decode_lse(const Tensor& q, const Tensor& k_cache,
                             scale, true);
 }
 
-Tensor attn_prefill(const Tensor& q, const Tensor& k, const Tensor& v,
+// Keys or values as attn_flash.hip loads them: pieces of 16 bytes, straight to
+// LDS, at 32-bit offsets in a tile of 64 rows. Others are copied.
+Tensor flash_rows(const Tensor& t) {
+    const bool as_is =
+        t.stride(0) % 8 == 0 && t.stride(0) < 1L << 24 &&
+        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    return as_is ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
+Tensor attn_prefill(const Tensor& q, const Tensor& k_in, const Tensor& v_in,
                     const Tensor& cu_seqlens, long max_seqlen, double scale,
                     bool causal) {
     check_bf16(q, "q");
-    check_bf16(k, "k");
+    check_bf16(k_in, "k");
     TORCH_CHECK(cu_seqlens.scalar_type() == torch::kInt32 &&
                 cu_seqlens.is_contiguous());
     const int T = q.size(0), nq = q.size(1), hd = q.size(2);
-    const int nkv = k.size(1);
+    const int nkv = k_in.size(1);
     const int nseq = cu_seqlens.size(0) - 1;
     TORCH_CHECK(nq % nkv == 0);
     TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == hd);
-    TORCH_CHECK(k.stride(2) == 1 && k.stride(1) == hd);
-    TORCH_CHECK(v.stride(2) == 1 && v.stride(1) == hd);
+    TORCH_CHECK(k_in.stride(2) == 1 && k_in.stride(1) == hd);
+    TORCH_CHECK(v_in.stride(2) == 1 && v_in.stride(1) == hd);
+    const Tensor k = flash_rows(k_in), v = flash_rows(v_in);
     Tensor out = torch::empty({T, nq, hd}, q.options());
     launch_attn_prefill(bf16p(q), bf16p(k), bf16p(v),
                         cu_seqlens.data_ptr<int>(), bf16p_mut(out), T, nseq,

@@ -56,6 +56,45 @@ def test_whole_prompts(nq, nkv, hd, lens):
     _check(got, want, v)
 
 
+# rows that are not 16-byte aligned, and rows 2^27 elements apart: 32 of them
+# are 2^32
+@pytest.mark.parametrize("lens,stride,offset", [
+    ([700], 1024 + 16, 1), ([300, 600], 1024 + 3, 0), ([70], 1024 + 4, 4),
+    ([40], 1 << 27, 0)])
+def test_keys_of_any_stride_and_alignment(lens, stride, offset):
+    nq, nkv, hd, T = 64, 8, 128, sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q = torch.randn(T, nq, hd, generator=g, device=DEV).bfloat16()
+    at = lambda: torch.empty(T * stride + offset, dtype=torch.bfloat16,
+                             device=DEV)[offset:].as_strided(
+        (T, nkv, hd), (stride, hd, 1))
+    k, v = at(), at()
+    for t in (k, v):
+        t.copy_(torch.randn(T, nkv, hd, generator=g, device=DEV))
+    cu, scale = _cu(lens), hd ** -0.5
+    got = ops.attn_prefill(q, k, v, cu, max(lens), scale)
+    want = reference.attn_prefill(q.float(), k.float(), v.float(), cu,
+                                  max(lens), scale)
+    _check(got, want, v)
+
+
+def test_pages_that_are_not_aligned():
+    nq, nkv, hd, bs, n = 64, 8, 128, 64, 700
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn(n, nq, hd, generator=g, device=DEV).bfloat16()
+    size = 16 * nkv * bs * hd
+    kc, vc = (torch.randn(size + 4, generator=g, device=DEV).bfloat16()[4:]
+              .view(16, nkv, bs, hd) for _ in range(2))
+    table = torch.randperm(16, generator=g, device=DEV).int().view(1, 16)
+    total = torch.tensor([n + 99], dtype=torch.int32, device=DEV)
+    got = ops.attn_prefill_paged(q, kc, vc, table, total, _cu([n]), n,
+                                 hd ** -0.5)
+    want = reference.attn_decode_with_history(
+        q.float(), kc.float(), vc.float(), table, total,
+        torch.tensor([n], dtype=torch.int32, device=DEV), hd ** -0.5)
+    _check(got, want, vc)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("nq,nkv,hd,lens,hist,bs", [
     (32, 8, 128, [5, 5, 1], [1500, 255, 0], 256),
