@@ -70,7 +70,7 @@ DEV_INLINE bf16x8 fl_bf16(uint2v r) {
 DEV_INLINE void fl_load(const char* base, unsigned off, unsigned to) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %0, %1"
-                 ::"v"(off), "s"(base), "s"(to) : "memory");
+                 ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
 }
 
 template <int HD, int RW, int KSP, bool PAGED, bool TURNS, typename KVT>

@@ -51,11 +51,11 @@ DEV_INLINE void lm_load(const void* base, unsigned off, unsigned to) {
     if constexpr (STREAM)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                      "global_load_lds_dwordx4 %0, %1 nt"
-                     ::"v"(off), "s"(base), "s"(to) : "memory");
+                     ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
     else
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                      "global_load_lds_dwordx4 %0, %1"
-                     ::"v"(off), "s"(base), "s"(to) : "memory");
+                     ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
 }
 // until at most `left` stages (R at most) of PER loads each are under way
 template <int PER, int R>

@@ -47,7 +47,7 @@ DEV_INLINE unsigned lw_lds(const void* p) {
 DEV_INLINE void lw_load(const void* base, unsigned off, unsigned to) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %0, %1"
-                 ::"v"(off), "s"(base), "s"(to) : "memory");
+                 ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
 }
 // the lane, as a value that is not kept in a register from one use to the next
 DEV_INLINE int lw_lane() {

@@ -1,6 +1,7 @@
 """The BEE2BEE_DEBUG_KERNELS=1 build: BB_KASSERT compiles into the kernels
 (hipcc cross-compiles gfx950 without a GPU, so this runs in CPU CI)."""
 import os
+import re
 import shutil
 import subprocess
 
@@ -44,3 +45,19 @@ def test_debug_macro_traps_in_isa(tmp_path):
     assert r.returncode == 0, r.stderr[-2000:]
     asm = out.read_text()
     assert "s_trap" in asm or "llvm.trap" in asm or "s_endpgm" in asm
+
+
+def test_asm_that_sets_m0_says_so():
+    """An asm statement that writes M0 names it among its clobbers, or the
+    compiler may keep a value of its own there across the statement."""
+    folder, seen = os.path.dirname(SRC), 0
+    for name in sorted(os.listdir(folder)):
+        if not name.endswith(".hip") or name.endswith("_hip.hip"):
+            continue
+        with open(os.path.join(folder, name)) as f:
+            text = f.read()
+        for statement in re.findall(r"\basm volatile\(.*?\);", text, re.S):
+            if re.search(r"s_\w+ m0\b", statement):
+                seen += 1
+                assert '"m0"' in statement.rsplit(":", 1)[1], (name, statement)
+    assert seen
