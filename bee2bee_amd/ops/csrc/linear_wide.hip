@@ -363,26 +363,48 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     if (wid < 4) lw_barrier();
 }
 
-// Microseconds of a launch as the planner sees it: rounds of 256 workgroups,
-// each with its start and end, a last one that leaves CUs idle faster a step.
-// Fitted to 50 sizes of 300 to 9216 rows: the choice below was the fastest of
-// its own in all but one (4% behind). Steps of 128-row tiles take 0.82 us, of 256
-// rows 1.26: they draw 48 KB from L2, not 64, for half the products.
-static double lw_time(int M, int N, int K, int form, int tall, int S) {
+// Microseconds of a launch as the planner sees it: rounds of 256 workgroups, a
+// last one that leaves CUs idle faster a step, each with a start and an end.
+// Steps of 128-row tiles take less than those of 256 rows: they draw 48 KB from
+// L2, not 64, for half the products. Gated ones and output heads, which outweigh
+// the caches: fitted to 50 sizes of 300 to 9216 rows, the choice the fastest of
+// its own in all but one (4% behind).
+static double lw_time(int M, int N, int K, int form, int tall) {
     static const double step[] = {0.82, 1.0, 1.26}, idle[] = {0.48, 0.45, 0.56},
                         busy[] = {0.45, 0.58, 0.46};
     const int BN = form == LW_GATED ? 128 : 256, i = tall - 2;
     const long tiles = ((M + tall * 64L - 1) / (tall * 64)) *
-                       ((N + BN - 1) / BN) * S;
-    const double steps = K / 64 / S * step[i], full = tiles / 256,
+                       ((N + BN - 1) / BN);
+    const double steps = K / 64 * step[i], full = tiles / 256,
                  left = (tiles % 256) / 256.0;
     double t = full * (steps + tall + 3);
     if (left > 0) {
         const double f = idle[i] + busy[i] * left;
         t += steps * (f < 1 ? f : 1) + tall + 3;
     }
-    // the parts, written and read in place of bf16 rows
-    if (form == LW_PARTS) t += (double)M * N * (4 * S - 2) / 2.2e6;
+    return t;
+}
+
+// The same of the narrow projections (S parts; 1: rows), fitted to 437 products
+// of 4M weights and more, 257 to 6000 rows, every launch with weights that no
+// cache holds, as in a model's step: a round starts slower and few workgroups
+// gain less than above. Parts are written, and read in place of bf16 rows.
+static double lw_time_parts(int M, int N, int K, int tall, int S) {
+    static const double step[] = {0.84, 1.05, 1.36}, idle[] = {0.75, 0.71, 0.63},
+                        busy[] = {0.42, 0.23, 0.28}, start[] = {3.6, 5.1, 4.4},
+                        round[] = {0, 2.1, 6.0}, store[] = {0.22, 0.14, 0.08};
+    const int i = tall - 2;
+    const long tiles = ((M + tall * 64L - 1) / (tall * 64)) *
+                       ((N + 255) / 256) * S;
+    const double steps = K / 64 / S * step[i], full = tiles / 256,
+                 left = (tiles % 256) / 256.0;
+    double t = start[i] + full * (steps + round[i]);
+    if (left > 0) {
+        const double f = idle[i] + busy[i] * left;
+        t += steps * (f < 1 ? f : 1) + round[i];
+    }
+    if (S > 1)
+        t += (double)M * N / 1e6 * (4 * S * store[i] + 0.2 * (4 * S - 2));
     return t;
 }
 
@@ -391,6 +413,17 @@ static double lw_time(int M, int N, int K, int form, int tall, int S) {
 // 128: the rows past the last whole tile are linear_mid.hip's, which reads the
 // weights once more for them: where they would begin a round of their own
 // (9217x3584x18944: 37 rows of tiles by 14 are 518 workgroups).
+//
+// The library's time is fitted to the same products: its rounds of 256 x 256
+// tiles, operations and weights. Of 208 other products (330 to 12000 rows) the
+// choice is more than 3% behind the library in one and 0.7% from the best on
+// average; the times that were fitted to cached weights left it behind in 18,
+// with the norm that follows, us, those in brackets: 512x3072x2048 20.6 (26.0),
+// 512x2048x2048 16.3 (21.0), 1200x3072x3072 40.4 (47.2), 1400x2560x2560 36.3
+// (46.4). Products of fewer weights stay here, up to 5 us behind the library:
+// steps of such a stack that are not captured are bound by the host, which takes
+// 6 us to launch one and 20 for the library's (six layers of 768, prompts of 300
+// to 1023 tokens: 580 us against 770).
 extern "C" int linear_wide_plan(int M, int N, int K, int form) {
     if (M < 1 || N < 8 || N % 8 || K < 256 || K % 128 || K > 1 << 22) return 0;
     int best = 0;
@@ -398,32 +431,39 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
     for (int tall = 2; tall <= 4; ++tall)
         for (int S = 1; S <= (form == LW_PARTS ? 8 : 1); S *= 2) {
             if (S > 1 && (K / 64 / S < 8 || K % (128 * S))) break;
-            const int f = S == 1 && form == LW_PARTS ? LW_ROWS : form;
-            const double t = lw_time(M, N, K, f, tall, S);
+            auto time = [&](int rows) {
+                return form == LW_PARTS ? lw_time_parts(rows, N, K, tall, S)
+                                        : lw_time(rows, N, K, form, tall);
+            };
+            const double t = time(M);
             if (t < least) {
                 least = t;
                 best = tall + 8 * S;
             }
             const int tail = M % (tall * 64);
-            const double bytes = (f == LW_GATED ? 4.0 : 2.0) * N * K;
+            const double bytes = (form == LW_GATED ? 4.0 : 2.0) * N * K;
             if (S > 1 || tail == 0 || tail == M || bytes >= 1LL << 32) continue;
-            const double t2 = lw_time(M - tail, N, K, f, tall, 1) + 8 +
+            const double t2 = time(M - tail) + (form == LW_PARTS ? 12 : 8) +
                               bytes / 5.2e6 * (1 + 0.0035 * tail);
             if (t2 < 0.97 * least) {
                 least = t2;
                 best = tall + 8 + 128;
             }
         }
-    if (form == LW_GATED || (form == LW_PARTS && K >= 8192)) return best;
-    double library = 2.0 * M * N * K / 1.45e9 * 1.25 + 14;
-    if (form == LW_ROWS) {
-        // output heads of a few hundred rows are bound by their weights (200
-        // rows, us, the library's in brackets: 32000x4096 76 (71), 128256x4096
-        // 232 (293))
-        const double bytes = 2.0 * N * K;
-        if (least < bytes / 5.05e6 + 24) least = bytes / 5.05e6 + 24;
-        if (library < bytes / 3.7e6) library = bytes / 3.7e6;
+    const double flops = 2.0 * M * N * K, bytes = 2.0 * N * K;
+    if (form == LW_GATED) return best;
+    if (form == LW_PARTS) {
+        if ((long)N * K < 4 << 20) return best;
+        const long tiles = ((M + 255L) / 256) * ((N + 255) / 256);
+        const double library = 5.3 + (tiles + 255) / 256 * (K * 2.29e-3) +
+                               flops * 0.73e-9 + bytes * 0.173e-6;
+        return least <= library ? best : 0;
     }
+    // output heads of a few hundred rows are bound by their weights (200 rows,
+    // us, the library's in brackets: 32000x4096 76 (71), 128256x4096 232 (293))
+    double library = flops / 1.45e9 * 1.25 + 14;
+    if (least < bytes / 5.05e6 + 24) least = bytes / 5.05e6 + 24;
+    if (library < bytes / 3.7e6) library = bytes / 3.7e6;
     return least <= library ? best : 0;
 }
 

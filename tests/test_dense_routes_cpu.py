@@ -186,3 +186,26 @@ def test_few_rows_under_tensor_parallelism(tmp_path):
     assert t0 == t1
     for a, b in zip(l0, l1):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
+# rows, outputs, depth: measured with the norm that follows (us, the library's
+# product, the best of linear_wide.hip's own)
+@pytest.mark.skipif(not ops.hip_available(), reason="the extension is not built")
+@pytest.mark.parametrize("M,N,K,library,own", [
+    (300, 3072, 2048, 17.8, 20.3), (400, 2048, 2048, 15.1, 17.6),
+    (700, 2048, 2048, 17.6, 19.0), (1024, 2048, 2048, 20.9, 23.4),
+    (1536, 3072, 2048, 34.4, 37.4), (384, 2560, 2560, 19.9, 22.8),
+    (560, 5120, 3072, 34.9, 36.9), (300, 4096, 11008, 67.9, 80.3),
+    (330, 1536, 8960, 39.6, 64.7), (3000, 3072, 3072, 77.9, 65.5),
+    (512, 2048, 8192, 39.6, 29.6), (1536, 4096, 14336, 184.7, 144.5),
+    (800, 5120, 27648, 334.9, 248.7), (600, 1024, 4096, 21.8, 18.4),
+    (9217, 5120, 3072, 395.3, 282.8), (650, 4096, 11008, 96.7, 80.6)])
+def test_plans_follow_what_was_measured(M, N, K, library, own):
+    assert bool(ops.wide_plan(M, N, K, "parts")) == (own < library)
+
+
+@pytest.mark.skipif(not ops.hip_available(), reason="the extension is not built")
+def test_small_products_keep_their_kernel():
+    for M in (257, 600, 1023, 4096):
+        for N, K in ((768, 768), (2304, 768), (768, 3072), (3072, 1024)):
+            assert ops.wide_plan(M, N, K, "parts")
