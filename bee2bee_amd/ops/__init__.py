@@ -313,8 +313,13 @@ def ring_rows(x: torch.Tensor) -> bool:
 
 
 def mid_shape(rows: int, width: int, depth: int) -> bool:
-    """Projections that mid_linear takes, all up to MID_MAX rows, above it
-    those that outweigh their parts. Measured with the kernel that reads them
+    """Projections that mid_linear takes: all up to MID_MAX rows, above it those
+    that outweigh their parts, and of at most 4M weights all up to 160 rows and
+    deep ones: the library is up to 2 us ahead on these, but its launches cost the
+    host 20 us and not 6, which is what a step of such a stack takes if it is not
+    captured (six layers of 768, prompts of 140 / 200 / 256 tokens 480 / 680 / 675
+    us, with the library's 770; captured, 335 / 350 / 355 and 328 / 345 / 347).
+    Measured with the kernel that reads them
     (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 16.9 (19.1)
     / 26.1 (30.0) / 30.0 (30.4), 4096x14336 26.6 (32.8) / 35.3 (79) / 42.4
     (59.6), 3584x18944 28.7 (112) / 39 (103) / 50 (127), 8192x8192 35.1 (34.6) /
@@ -322,6 +327,8 @@ def mid_shape(rows: int, width: int, depth: int) -> bool:
     3072x2048 9.9 (15.0) / 14.7 (18.1) / 18.0 (16.6), 5120x3072 14.6 (16.4) /
     22.5 (25.1) / 27.4 (24.1), 768x3072 7.7 (11.9) / 10.8 (10.4) / 12.8
     (11.3)."""
+    if width * depth <= 4 << 20 and (rows <= 160 or 2 * depth >= 7 * width):
+        return True
     return rows <= MID_MAX or width * depth >= (
         16_000_000 if width > depth else DEEP_SIZE)
 

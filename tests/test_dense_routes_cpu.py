@@ -209,3 +209,14 @@ def test_small_products_keep_their_kernel():
     for M in (257, 600, 1023, 4096):
         for N, K in ((768, 768), (2304, 768), (768, 3072), (3072, 1024)):
             assert ops.wide_plan(M, N, K, "parts")
+
+
+@pytest.mark.parametrize("rows,width,depth,own", [
+    (129, 2304, 768, True), (160, 768, 768, True), (160, 2048, 2048, True),
+    (161, 768, 768, False), (161, 768, 3072, True), (256, 1024, 4096, True),
+    (129, 3072, 2048, False), (256, 2048, 2048, False), (128, 3072, 2048, True),
+    (256, 4096, 14336, True), (200, 5120, 3072, False)])
+def test_small_products_of_129_to_256_rows(rows, width, depth, own):
+    """Steps of small stacks are bound by the host, which a library product
+    costs three times as much."""
+    assert ops.mid_shape(rows, width, depth) == own
