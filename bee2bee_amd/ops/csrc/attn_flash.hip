@@ -608,35 +608,75 @@ static int flash_smem(int hd, int rw, int ksp, bool turns) {
 // portions behind long histories); with fewer, 128 rows balance better, with
 // less than a chip of those 64 rows, whose two wave pairs share a tile's keys.
 // Prompts of different lengths leave tiles of every length to balance: 256 rows
-// need more of them the more prompts there are.
+// need more of them the more prompts there are, and, as measured, more again
+// from eight prompts on where seven or eight heads share a key head. Three
+// prompts, and few of one length (`level`), want more of them than two or four
+// of different lengths.
 // Measured (us, 256 / 128 / 64 rows; heads 32/8 unless stated), head size 128:
 //   one prompt: full 150 35/34/30, 190 42/44/40, 230 50/53/56, 350 77/83/102,
-//    600 192/212/261, 1000 466/553/687; 2 prompts of an eighth to 1: 150
-//    30/32/39, 600 232/285/396; 4: 149 20.5/19.5/27.6 (28/4: 23/22/20), 299
-//    50/52/71 (28/4: 37/42/50), 1000 316/395/558;
-//   9 prompts: 149 14/13.6/16, 449 39/34/46 (28/4: 54/44/69), 999 109/102/141,
-//    1399 172/181/239 (28/4: 311/289/441), 2000 319/360/468 (28/4:
-//    586/580/840); 30 prompts: 1000 66/61/79, 2000 165/159/221;
+//    600 192/212/261, 1000 466/553/687;
+//   2 of an eighth to 1: 150 31/32/39, 600 233/286/399; of one length 150
+//    22/20/18, 230 29/30/33, 450 62/74/88;
+//   3: 229 33/31/30 (28/4: 37/35/34), 299 46/46/50 (45/46/49), 600 104/110/139;
+//   4: 149 21/20/28 (28/4: 23/22/20), 189 27/28/36 (26/27/27), 299 50/52/71
+//    (36/41/49), 1000 317/392/550; of one length 230 20/19/24, 300 26/24/34, 450
+//    42/45/56;
+//   9: 149 14/13.6/16, 449 39/34/46 (28/4: 53/45/69), 999 106/99/140, 1399
+//    170/179/242 (28/4: 311/285/439, 64/8: 113/107/150; of one length 149/147/200,
+//    28/4 157/162/224), 2000 322/349/470 (28/4: 590/582/833, 64/8: 207/197/276),
+//    2800 581/664/871 (976/1106/1561, 346/361/492); 16: 2000 246/250/355 (28/4:
+//    249/242/338, 64/8: 179/160/229), 2800 409/456/648 (429/460/618, 277/272/395);
+//   30: 1000 65/59/78, 2000 165/156/220, 2800 267/263/375;
 //   8000 cached: 120 206/206/187, 140 210/261/334, 256 287/330/393, 400
 //    489/597/732, 1000 1372/1612/1999; 500 cached: 120 42/37/33, 140 45/44/40,
-//    185 54/53/59, 300 82/84/106, 600 235/250/307;
+//    185 54/53/59, 300 82/84/106, 600 235/250/307; without turns (pages of 48):
+//    8000 140 269/295/359, 300 534/517/596, 350 579/545/678, 400 605/655/827;
+//    500 140 54/49/45, 185 66/59/68, 256 90/78/90, 300 95/91/118, 350
+//    112/121/146, 600 272/269/354;
 // head size 64:
 //   one prompt: 300 53/47/44 (12/12: 139/121/106), 350 64/56/57, 600
 //    134/128/144, 1000 306/313/373; 9 prompts: 300 17/15/16 (12/12: 34/30/26),
 //    600 30/29/34, 1000 61/60/76 (12/12: 146/137/169); 2: 600 152/155/193;
 //   8000 cached: 150 176/177/160, 230 193/192/216, 300 286/264/286, 400
 //    328/357/386, 1000 843/914/1083.
-static int flash_shape(int hd, long full, int nseq, bool pages) {
+static int flash_shape(int hd, long T, int nseq, int nq, int nkv, int max_qlen,
+                       bool pages, bool turns) {
+    const long full = T * nq / 256;
     const bool lone = !pages && nseq == 1;
+    if (hd == 128 && pages) {
+        if (full >= (turns ? 140 : 380)) return 0;
+        return full >= 140 ? 1 : 2;
+    }
     if (hd == 128) {
-        if (full >= (pages  ? 140
-                     : lone ? 210
-                            : (nseq <= 4 ? 75 : 150) * (long)nseq))
-            return 0;
-        return full >= 115 && !pages && !lone ? 1 : 2;
+        const bool level = 4 * T >= 3L * nseq * max_qlen;
+        long least = 150L * nseq;
+        if (lone) least = 210;
+        else if (nseq <= 4 && (level || nseq == 3)) least = 90 * nseq;
+        else if (nseq <= 4) least = nseq == 2 ? 150 : 180;
+        else if (nseq >= 8 && nq >= 7 * nkv && !level) {
+            const long more = 240L * nseq < 2200 ? 240L * nseq : 2200;
+            least = more > least ? more : least;
+        }
+        if (full >= least) return 0;
+        return full >= 115 && !lone ? 1 : 2;
     }
     if (full >= (pages ? 400 : 700)) return 0;
     return full >= (lone ? 320 : pages ? 185 : 230) ? 1 : 2;
+}
+
+// whole tiles in a page, in pieces that go straight to LDS
+static bool flash_turns(int hd, bool pages, int bs, bool aligned) {
+    return hd == 128 && (!pages || (bs % FL_KT == 0 && aligned));
+}
+
+// What a step of these sizes runs on: the workgroup's rows (256, 128 or 64), + 1
+// where its waves take turns. bs: keys of a page, 0 for packed prompts.
+extern "C" int attn_flash_form(long T, int nseq, int nq, int nkv, int hd,
+                               int max_qlen, int bs) {
+    const bool turns = flash_turns(hd, bs > 0, bs, true);
+    const int shape =
+        flash_shape(hd, T, nseq, nq, nkv, max_qlen, bs > 0, turns);
+    return (256 >> shape) + (shape == 0 && turns);
 }
 
 #define FL_ONE(HDV, RWV, KSPV, PG, TU, KVT)                                     \
@@ -675,9 +715,9 @@ extern "C" int launch_attn_flash(
     if (nseq == 0 || max_qlen <= 0) return 0;
     const int pairs = nseq * nkv;
     const long rows = (long)max_qlen * (nq / nkv);
-    const int shape = flash_shape(hd, T * nq / 256, nseq, block_table);
-    // whole tiles in a page, in pieces that go straight to LDS
-    const bool turns = !block_table || (bs % FL_KT == 0 && aligned);
+    const bool turns = flash_turns(hd, block_table, bs, aligned);
+    const int shape =
+        flash_shape(hd, T, nseq, nq, nkv, max_qlen, block_table, turns);
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

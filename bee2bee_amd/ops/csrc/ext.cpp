@@ -37,6 +37,7 @@ void launch_attn_decode(const unsigned short*, const void*, const void*,
                         const int*, const int*, unsigned short*, float*,
                         float*, unsigned short*, float*, int, int, int, int,
                         int, int, int, long, float, int, hipStream_t);
+int attn_flash_form(long, int, int, int, int, int, int);
 int attn_stream_takes(long, long);
 int attn_stream_splits(long, long, long, int*, int*);
 int launch_attn_stream(const unsigned short*, const void*, const void*,
@@ -492,6 +493,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attn_prefill", &attn_prefill, "varlen causal flash prefill");
     m.def("attn_prefill_paged", &attn_prefill_paged,
           "chunked prefill vs paged history");
+    m.def("attn_flash_form", &attn_flash_form,
+          "rows of prompt attention's workgroups, + 1 where waves take turns");
     m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA layout probe");
     m.def("mfma_probe_fp8", &mfma_probe_fp8,
           "16x16x32 fp8 MFMA layout probe");

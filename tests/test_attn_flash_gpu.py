@@ -101,6 +101,9 @@ def test_pages_that_are_not_aligned():
     (28, 4, 128, [64, 40], [63, 64], 64), (32, 8, 64, [33, 2], [77, 1], 16),
     (6, 2, 128, [40, 9], [100, 300], 24), (12, 12, 64, [130], [1000], 256),
     (28, 4, 128, [2100], [500], 256), (32, 8, 128, [3600], [130], 256),
+    # pages of no whole tiles: 128- and 256-row workgroups without turns
+    (32, 8, 128, [1300], [200], 48), (28, 4, 128, [900, 1100], [70, 0], 16),
+    (64, 8, 128, [1700], [30], 48),
 ])
 def test_chunks_against_pages(nq, nkv, hd, lens, hist, bs, fp8):
     q, _, _ = _qkv(sum(lens), nq, nkv, hd, 3)
