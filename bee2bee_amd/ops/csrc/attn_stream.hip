@@ -3,9 +3,13 @@
 //
 // Bound by reading the cache once. A wave takes tiles of 32 keys on its own:
 // whole 16-byte chunks of neighbouring rows into registers (1 KB a load, with
-// the streaming hint: 1536 sequences below 653 us without it), on to its part
-// of LDS, the next tile's loads on their way over the products of
-// this one, no barrier before the end. Scores are S^T = K Q^T on 16x16x32
+// the streaming hint where the block table has room for more than 6 MB of keys
+// and values: 1536 sequences below 653 us without it; 8 of 500 tokens, 8 heads of
+// 128, 8.8 against 10.0 where no cache holds them. One sequence of 300 or 1000
+// tokens takes the same time with it, 6.4 to 7.5, but a step that finds its pages
+// in a cache is slower: six layers of 12 heads of 64, 300 keys, 190 us against
+// 187), on to its part of LDS, the next tile's loads on their way over the
+// products of this one, no barrier before the end. Scores are S^T = K Q^T on 16x16x32
 // matrix tiles (a column is a query row; the rows of all heads that share the
 // key head, times the chunk's tokens), so that the weights are, as they
 // stand, the right operand of O^T = V^T P^T, whose keys follow the score
@@ -52,6 +56,11 @@ DEV_INLINE short8 st_widen(uint2v x) {
     return __builtin_bit_cast(short8, r);
 }
 
+template <bool STREAM> DEV_INLINE st_raw st_load(const st_raw* p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
 // elements 8 p .. 8 p + 7 of a load, in bf16
 template <typename KVT> DEV_INLINE short8 st_piece(st_raw x, int p) {
     if constexpr (sizeof(KVT) == 2) return __builtin_bit_cast(short8, x);
@@ -77,7 +86,7 @@ DEV_INLINE int split_keys(int L, int even, int most) {
     return min(((L + even - 1) / even + ST_STEP - 1) / ST_STEP * ST_STEP, most);
 }
 
-template <int HD, int QT, typename KVT>
+template <int HD, int QT, typename KVT, bool STREAM>
 __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k_cache,
     const KVT* __restrict__ v_cache, const int* __restrict__ cu,
@@ -174,9 +183,9 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
                 off = (((long)page * nkv + kvh) * bs + key % bs) * HD;
             }
             off += ld_c * 8;
-            rk[i] = __builtin_nontemporal_load(
+            rk[i] = st_load<STREAM>(
                 reinterpret_cast<const st_raw*>(k_cache + off));
-            rv[i] = __builtin_nontemporal_load(
+            rv[i] = st_load<STREAM>(
                 reinterpret_cast<const st_raw*>(v_cache + off));
         }
     };
@@ -520,8 +529,15 @@ extern "C" int launch_attn_stream(
     const dim3 grid(nseq * nkv, Z, (max_rows + qt * 16 - 1) / (qt * 16));
     const int smem = ST_WAVES * 2 * ST_KEYS * hd * 2 +
                      qt * 16 * ST_WAVES * 2 * (int)sizeof(float);
+    const bool streamed =
+        (long)nseq * nkv * W * bs * hd * (fp8 ? 2 : 4) > 6 << 20;
 #define ST_ONE(HDV, QTV, KVT)                                                 \
-    hipLaunchKernelGGL((attn_stream_kernel<HDV, QTV, KVT>), grid,             \
+    do {                                                                      \
+        if (streamed) ST_GO(HDV, QTV, KVT, true);                             \
+        else ST_GO(HDV, QTV, KVT, false);                                     \
+    } while (0)
+#define ST_GO(HDV, QTV, KVT, STR)                                             \
+    hipLaunchKernelGGL((attn_stream_kernel<HDV, QTV, KVT, STR>), grid,        \
                        dim3(ST_WAVES * 64), smem, stream, q,                  \
                        (const KVT*)k_cache, (const KVT*)v_cache, cu,          \
                        block_table, seq_lens, out, out_ml, part_o, part_ml,   \
@@ -545,5 +561,6 @@ extern "C" int launch_attn_stream(
 #undef ST_HD
 #undef ST_COMBINE
 #undef ST_ONE
+#undef ST_GO
     return 0;
 }

@@ -12,11 +12,18 @@
 //    over workgroups, so a row's result depends neither on the other rows nor
 //    on their number.
 //  * TC 8: 8 rows of W at two places along K, 128 bytes of a row together (whole
-//    lines, so these loads carry the streaming hint: 2x14336x4096 41 us without
-//    and 36.5 with, 4096x14336 24.2 and 22.1, 3584x18944 27.8 and 26), as one
-//    left operand, 8 input rows at both places as the other; the two
-//    diagonal quarters of the product add up. Twice the workgroups where 16
+//    lines), as one left operand, 8 input rows at both places as the other; the
+//    two diagonal quarters of the product add up. Twice the workgroups where 16
 //    columns each leave CUs without one, and better pieces to load elsewhere.
+//    These loads carry the streaming hint (STREAM): weights that no cache holds
+//    come 3 to 9% sooner (2x14336x4096 41 us without and 36.5 with, 4096x14336
+//    24.2 and 22.1, 2048x2048 5.0 and 4.6), but those that the 256 MB memory-side
+//    cache has kept since the last step 5 to 15% later, at the time of those that
+//    it has not. So not where the sides are those of stacks of 768 (sides up to
+//    768 and 4096), which fit there whole: distilgpt2, one row, repeated 199.6 us
+//    with the hint on all and 187.2, a first step on new weights 230 and 218;
+//    with three such stacks in turn, which do not fit, 205 and 212. 1024x1024
+//    belongs to stacks that do not fit: 3.4 us with it and 3.8.
 //  * Between two layers' projections the residual sum stays in fp32: the norm
 //    after an add takes the sum before it is rounded, as the kernel that adds
 //    and norms does. For an RMS norm the projection that adds leaves the sum
@@ -98,9 +105,9 @@ DEV_INLINE void store_row4(void* cache, long at, int fp8, const float* z) {
     }
 }
 
-// (see above: TC 8 reads whole lines, which are only streamed through L2)
-template <int TC> DEV_INLINE bf16x8 lr_weights(const unsigned short* p) {
-    if constexpr (TC == 8)
+// (see above)
+template <bool STREAM> DEV_INLINE bf16x8 lr_weights(const unsigned short* p) {
+    if constexpr (STREAM)
         return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
     else
         return *reinterpret_cast<const bf16x8*>(p);
@@ -112,7 +119,8 @@ template <int TC> DEV_INLINE bf16x8 lr_weights(const unsigned short* p) {
 // per workgroup (LR_GLU, LR_QKV: of each half; LR_QKV's halves are those of a
 // head).
 // x is of type XT: bf16, or (LR_LAYER) fp32. squares: of LR_SCALED's rows.
-template <int NW, int NT, int TC, int G, int NORM, int EPI, typename XT>
+template <int NW, int NT, int TC, int G, int NORM, int EPI, typename XT,
+          bool STREAM>
 __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
     const XT* __restrict__ x,
     const unsigned short* __restrict__ norm_w,
@@ -162,7 +170,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
             for (int h = 0; h < H; ++h)
 #pragma unroll
                 for (int t = 0; t < WT; ++t)
-                    aw[set][u][h][t] = lr_weights<TC>(
+                    aw[set][u][h][t] = lr_weights<STREAM>(
                         wp[t] + (long)(s + u) * KS + h * 32);
     };
     int s = s0;
@@ -259,7 +267,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         for (int h = 0; h < H; ++h)
 #pragma unroll
             for (int t = 0; t < WT; ++t)
-                a[h][t] = lr_weights<TC>(wp[t] + (long)s * KS + h * 32);
+                a[h][t] = lr_weights<STREAM>(wp[t] + (long)s * KS + h * 32);
         products(a, s);
     }
 
@@ -497,14 +505,23 @@ extern "C" int launch_linear_rows(
     if (epi == LR_QKV && (hd % 32 || N != (nq + 2 * nkv) * hd)) return 1;
     const QkvStore st{pos,     cos_t, sin_t, slots, k_cache,
                       v_cache, nq,    nkv,   hd,    bs, fp8};
+    // (see above: stacks of more than 768)
+    const int WN = epi == LR_GLU ? 2 * N : N;
+    const bool streamed = (WN < K ? WN : K) > 768 || (WN < K ? K : WN) > 4096;
 #define LR_COLS(NTV, TCV, EP) (NTV * TCV * (EP == LR_QKV ? 2 : 1))
+#define LR_ONE(NWV, NTV, TCV, GV, NO, EP, XT, STR)                            \
+    hipLaunchKernelGGL(                                                       \
+        (linear_rows_kernel<NWV, NTV, TCV, GV, NO, EP, XT, STR>),             \
+        dim3((N + LR_COLS(NTV, TCV, EP) - 1) / LR_COLS(NTV, TCV, EP)),        \
+        dim3(NWV * 64), 0, stream, (const XT*)x, norm_w, norm_b, w, bias,     \
+        squares, add, (unsigned short*)y, M, N, K, eps, st)
 #define LR_GO(NWV, NTV, TCV, GV, NO, EP, XT)                                  \
-    hipLaunchKernelGGL((linear_rows_kernel<NWV, NTV, TCV, GV, NO, EP, XT>),   \
-                       dim3((N + LR_COLS(NTV, TCV, EP) - 1) /                 \
-                            LR_COLS(NTV, TCV, EP)),                           \
-                       dim3(NWV * 64), 0, stream, (const XT*)x, norm_w,       \
-                       norm_b, w, bias, squares, add, (unsigned short*)y, M,  \
-                       N, K, eps, st)
+    do {                                                                      \
+        if (TCV == 8 && streamed)                                             \
+            LR_ONE(NWV, NTV, TCV, GV, NO, EP, XT, TCV == 8);                  \
+        else                                                                  \
+            LR_ONE(NWV, NTV, TCV, GV, NO, EP, XT, false);                     \
+    } while (0)
 #define LR_NORMS(NWV, NTV, TCV, GV, EP)                                       \
     do {                                                                      \
         if (norm == LR_SCALED)                                                \
@@ -541,6 +558,7 @@ extern "C" int launch_linear_rows(
 #undef LR_16
 #undef LR_NORMS
 #undef LR_GO
+#undef LR_ONE
 #undef LR_COLS
     return 0;
 }

@@ -106,6 +106,23 @@ def test_rows_alone(N, K, act):
         assert torch.equal(rows(n)[:1], one)
 
 
+# (sides up to 768 and 4096: loads without the streaming hint)
+@pytest.mark.parametrize("M", [1, 9])
+@pytest.mark.parametrize("N,K,act", [
+    (768, 4096, None), (776, 4096, None), (768, 4160, None), (4096, 768, None),
+    (2048, 768, "swiglu"), (2064, 768, "swiglu"), (2048, 832, "swiglu")])
+def test_both_sides_of_the_streaming_hint(M, N, K, act):
+    torch.manual_seed(N + K)
+    x, w = _rand(M, K), _rand(2 * N if act else N, K, std=0.05)
+    got = ops.rows_linear(x, w, act=act).float()
+    want, mag = _products(x, w, None)
+    if act:
+        (g, u), (mg, mu) = want.chunk(2, -1), mag.chunk(2, -1)
+        want = F.silu(g) * u
+        mag = 1.13 * mg * u.abs() + F.silu(g).abs() * mu
+    assert ((got - want).abs() <= 2 ** -8 * (mag + want.abs()) + 1e-5).all()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("M,nq,nkv,hd,K,kind", [
     (1, 32, 8, 128, 256, "rms"), (16, 7, 1, 64, 96, "rms"),
