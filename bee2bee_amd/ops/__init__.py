@@ -239,8 +239,8 @@ def few_rows(x: torch.Tensor) -> bool:
 def head_rows(x: torch.Tensor, layer_norm: bool) -> bool:
     """Few rows whose logits are rows_linear's, where mid_head does not take
     them; the others' are a norm and the library's. Measured (us, rows_linear /
-    norm and library): 128256 columns of 8192 373 / 371 at 8 rows, 415 / 363 at
-    16. A layer norm's mean and deviation are taken by each of the hundreds of
+    norm and library): 128256 columns of 8192 359 / 374 at 8 rows, 376 / 365 at
+    12, 402 / 364 at 16, 152064 459 / 464 at 12. A layer norm's mean and deviation are taken by each of the hundreds of
     workgroups: 50257 of 768 22.0 / 21.8 at 1 row, 22.8 / 22.1 at 4 (a launch
     less for the host: 20 us of a step that is not captured), 25 / 22.5 at 8, 30
     / 23 at 16."""
@@ -372,8 +372,12 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     32000x4096 41 (63), 48 (66), 58 (64); 128256x2048 84 (121), 103 (129); of
     rows of 768 17.0 (18.6), 22.6 (20.8). Few rows (one launch of rows_linear in
     brackets; a norm takes 2.5 us): 1 / 16 rows 128256x4096 168 (178) / 166
-    (188), 152064x3584 158 (182) / 164 (204), 128256x2048 77 (93) / 81 (101)."""
+    (188), 152064x3584 158 (182) / 164 (204), 128256x2048 77 (93) / 81 (101); of
+    rows of 8192 1 / 8 / 12 rows 128256 370 (363) / 371 (359) / 370 (376), 152064
+    454 (427) / 458 (438) / 454 (459)."""
     if rows <= ROWS_MAX and width * depth < 100_000_000:
+        return False
+    if rows <= 8 and depth >= 8192:
         return False
     tiles = -(-width // 16)
     rounds = -(-tiles // 2048)

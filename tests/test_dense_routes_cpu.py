@@ -220,3 +220,13 @@ def test_small_products_of_129_to_256_rows(rows, width, depth, own):
     """Steps of small stacks are bound by the host, which a library product
     costs three times as much."""
     assert ops.mid_shape(rows, width, depth) == own
+
+
+# us as measured: the rings behind a norm, rows_linear
+@pytest.mark.parametrize("rows,width,depth,rings,alone", [
+    (1, 128256, 8192, 370, 363), (8, 128256, 8192, 371, 359),
+    (12, 128256, 8192, 370, 376), (1, 152064, 8192, 454, 427),
+    (12, 152064, 8192, 454, 459), (1, 152064, 5120, 244, 277),
+    (8, 128256, 4096, 174, 187), (1, 32000, 4096, 48, 50)])
+def test_output_heads_of_few_rows(rows, width, depth, rings, alone):
+    assert ops.mid_head(rows, width, depth) == (rings < alone)
