@@ -1,6 +1,6 @@
 """Steps of dense stacks at the row counts where the Runner changes its route
-(few rows, some tens, deep down projections, more), against the same steps in
-fp32 on the CPU.
+(few rows, some tens, a few hundred, more), against the same steps in fp32 on
+the CPU.
 
 Tolerance: a layer rounds about eight tensors to bf16 (2^-9 relative at most,
 independent of each other) and adds their effects to a residual that is rounded
@@ -32,8 +32,8 @@ GELU = ModelSpec(name="t-gelu", vocab_size=500, hidden_size=256,
                  attn_out_bias=True, mlp_bias=True)
 
 
-# outputs too wide for the split projections of some tens of rows: q|k|v, and
-# attention output and down projection
+# long q|k|v and attention output, and rows longer than 4096: few parts of K, or
+# one; from 129 rows on some of their products are the library's
 WIDE = [ModelSpec(name="t-wide-qkv", vocab_size=500, hidden_size=128,
                   intermediate_size=256, n_layers=2, n_heads=64,
                   n_kv_heads=32, head_dim=64, max_seq_len=1024),
@@ -126,9 +126,9 @@ def _rel(got, want):
 
 @pytest.mark.parametrize("spec,rows,kv_dtype", [
     (spec, rows, kv_dtype) for spec in (SWIGLU, GELU)
-    for rows in (1, 9, 16, 17, 160, 161, 256, 257)
+    for rows in (1, 9, 16, 17, 128, 129, 160, 161, 256, 257)
     for kv_dtype in ("native", "fp8")
-] + [(spec, rows, "native") for spec in WIDE for rows in (17, 200)],
+] + [(spec, rows, "native") for spec in WIDE for rows in (17, 129, 200, 257)],
     ids=lambda v: getattr(v, "name", str(v)))
 @torch.no_grad()
 def test_steps(spec, rows, kv_dtype):
@@ -152,6 +152,44 @@ def test_steps(spec, rows, kv_dtype):
         got, want = gpu.runner.lm_head(got[last]), cpu.runner.lm_head(
             want[last])
         assert _rel(got, want) <= limit, (name, _rel(got, want))
+
+
+def test_wide_specs_leave_products_to_the_library():
+    """What WIDE above is for: each has one that is left, and one that is not."""
+    from bee2bee_amd import ops
+
+    for spec in WIDE:
+        H, I, Q = spec.hidden_size, spec.intermediate_size, spec.q_size
+        shapes = [(Q + 2 * spec.kv_size, H), (H, Q), (H, I)]
+        assert len({ops.mid_shape(200, *s) for s in shapes}) == 2, spec.name
+        assert all(ops.mid_shape(128, *s) for s in shapes)
+
+
+# logits that are linear_wide's, the rings' (up to 160 rows) and the library's
+@pytest.mark.parametrize("vocab,hidden,rows,wide", [
+    (100000, 2048, 129, True), (100000, 2048, 200, True),
+    (65536, 1024, 700, True), (65536, 1024, 160, False),
+    (65536, 1024, 161, False)])
+@torch.no_grad()
+def test_output_heads_of_many_rows(vocab, hidden, rows, wide):
+    from bee2bee_amd import ops
+
+    spec = ModelSpec(name="t-head", vocab_size=vocab, hidden_size=hidden,
+                     intermediate_size=128, n_layers=1, n_heads=2,
+                     n_kv_heads=2, head_dim=64, max_seq_len=64)
+    W = ModelWeights(spec, DEV, torch.bfloat16).random_init(seed=3)
+    kv = PagedKV(spec, DEV, torch.bfloat16, n_blocks=4, block_size=16)
+    runner = Runner(spec, W, kv, DEV, torch.bfloat16)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, hidden, generator=g, device=DEV).bfloat16()
+    assert bool(ops.wide_plan(rows, vocab, hidden, "rows")) == wide
+    got = runner.lm_head(x).double()
+    x, w = x.double(), W.lm_head.double()
+    normed = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + spec.rms_eps)
+    normed = normed * W.final_norm.double()
+    want, mag = normed @ w.t(), normed.abs() @ w.abs().t()
+    # the normed rows and the logits are rounded to bf16 once each
+    assert ((got - want).abs() <= 2 ** -8 * (mag + want.abs()) + 1e-5).all()
 
 
 @pytest.mark.parametrize("rows", [1, 9, 17])
