@@ -135,12 +135,14 @@ def test_chunks_against_pages(nq, nkv, hd, lens, hist, bs, fp8):
 # along the keys raise the maximum in every tile
 @pytest.mark.parametrize("pages", [None, "bf16", "fp8"])
 @pytest.mark.parametrize("nq,nkv,lens,hist,bs", [
-    (64, 64, [1, 65, 130, 520], [0, 63, 62, 1], 64),
-    (64, 8, [300, 300], [5, 700], 256), (28, 4, [1300], [191], 64),
+    (64, 64, [1, 65, 130, 1020], [0, 63, 62, 1], 64),
+    (64, 8, [400, 400], [5, 700], 256), (28, 4, [1950], [191], 64),
     (64, 64, [900], [1], 128), (64, 4, [577, 600], [0, 40], 192),
 ])
 def test_waves_in_turn(nq, nkv, lens, hist, bs, pages):
     hd, T = 128, sum(lens)
+    assert ops.require_hip().attn_flash_form(
+        T, len(lens), nq, nkv, hd, max(lens), bs if pages else 0) == 257
     g = torch.Generator(device=DEV).manual_seed(T)
     q, k, v = _qkv(T, nq, nkv, hd, 5)
     cu, scale = _cu(lens), hd ** -0.5
