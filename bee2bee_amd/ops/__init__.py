@@ -15,8 +15,8 @@ Which projections are whose is measured: up to 16 rows (`few_rows`; logits:
 `head_rows`) the kernels of linear_rows.hip, one launch for norm, product and
 what follows; 17 to 256 rows (`mid_rows`, `mid_shape`, `mid_gated`) linear_mid.hip,
 split over K or activated; more rows linear_wide.hip where `wide_plan` says so:
-all gated ones and deep ones, and others unless they leave much of the chip
-idle. The grouped kernel
+all gated ones, and others where its times are below the library's. The grouped
+kernel
 driven as a single-segment GEMM loses to the library on all shapes
 (scripts/bench_skinny.py: N/64 workgroups starve the chip); it stays for experts
 because the E-way grid and the device-side segment offsets are what the library

@@ -8,7 +8,7 @@
 //          leave much of the chip idle.
 //
 // Bound by the matrix cores (at the clock that the power limit leaves them:
-// 8192x8192x8192 704 us, 1560 TFLOP/s). A workgroup a CU: 256 rows of x by 256
+// 8192x8192x8192 704 to 729 us from card to card, 1510 to 1560 TFLOP/s). A workgroup a CU: 256 rows of x by 256
 // of w, 64 of K at a time in one of two buffers of 64 KB, filled straight from
 // memory. Eight waves, two a SIMD: 128 x 64 sums each, in four quarters of 64 x
 // 32. Waves 0-3 read a quarter's fragments while 4-7 multiply, and the other way
@@ -18,17 +18,17 @@
 // always under way. An XCD's workgroups take neighbouring tiles (8 by 4 at a
 // time), which share what its L2 holds. Where there are more tiles than CUs a
 // workgroup takes several: the next one's first steps are loaded under the last
-// ones of this, whose rows go out from the registers (9216x2x18944x3584 1719 ->
-// 1666 us, 4096x2x18944x3584 776 -> 757, 4559x2x8192x3072 328 -> 316; without
-// swiglu less: 9216x3584x18944 830 -> 822, 1536x128256x4096 1131 -> 1124).
+// ones of this, whose rows go out from the registers (2 to 4% of a gated product,
+// 1% of others).
 //
-// Measured (us; in brackets the library's product, and of gated ones its swiglu):
-//   gated 9216x2x18944x3584 1666 (1972), 4096x2x18944x3584 757 (874),
-//    4559x2x8192x3072 316 (468), 1536x2x14336x4096 257 (288), 500x 92 (115);
-//   rows 9216x3584x18944 800 (807), 4096x3584x18944 372 (531), 4096x4608x3584
-//    110 (122), 1536x6144x4096 63 (70), 1536x128256x4096 1104 (1216);
-//   parts, with the norm that adds them: 1536x4096x14336 141 (179), 1100x 126
-//    (158), 500x 68 (101), 800x2048x8192 36 (48).
+// Measured with weights that no cache holds (us, on a card of the slower kind; in
+// brackets the library's product, and of gated ones its swiglu):
+//   gated 9216x2x18944x3584 1715 (2059), 4096x2x18944x3584 788 (911),
+//    4559x2x8192x3072 340 (481), 1536x2x14336x4096 278 (318), 500x 95 (112);
+//   rows 9216x3584x18944 848 (845), 4096x3584x18944 393 (498), 4096x4608x3584
+//    116 (129), 1536x6144x4096 68 (74), 1536x128256x4096 1150 (1268);
+//   parts, or rows, with the norm that follows: 1536x4096x14336 164 (190), 1100x
+//    137 (168), 500x 71 (102), 800x2048x8192 40 (53), 1536x4096x4096 62 (64).
 // Tried and slower: an XCD's tiles as one stretch for its workgroups (3 to 6%: some
 // have a round more), tiles split over K inside one launch, the last to come
 // adding (256 KB a tile and part written and read: 40 to 80 us a product).
@@ -218,9 +218,9 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     using No = std::false_type;
     using Yes = std::true_type;
 
-    // Step s of parity P lies in buffer P. Its regions are read in the order w P, x 0, w !P, x 1, the first in the step before; each is loaded
-    // again, for step s + 2 (`nx`), where all waves have read it, seven reads
-    // ahead. half: after two of the four `stores` have to be done
+    // Step s of parity P lies in buffer P. Its regions are read in the order w P,
+    // x 0, w !P, x 1, the first in the step before; each is loaded again, for step
+    // s + 2 (`nx`), where all waves have read it, seven reads ahead. half: after two of the four `stores` have to be done
     auto step = [&](auto par, auto ahead, int nx, bool half) {
         constexpr int P = decltype(par)::value, L = decltype(ahead)::value;
         // L: steps after this one, 2 standing for more

@@ -1,5 +1,6 @@
-// Torch bindings of the projections of a few rows (linear_rows.hip) and of some
-// tens (linear_mid.hip) and more (linear_wide.hip), and of the pass between q|k|v and attention.
+// Torch bindings of the projections of a few rows (linear_rows.hip), of some tens
+// (linear_mid.hip) and more (linear_wide.hip), and of the pass between q|k|v and
+// attention.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
