@@ -317,8 +317,8 @@ def mid_shape(rows: int, width: int, depth: int) -> bool:
     that outweigh their parts, and of at most 4M weights all up to 160 rows and
     deep ones: the library is up to 2 us ahead on these, but its launches cost the
     host 20 us and not 6, which is what a step of such a stack takes if it is not
-    captured (six layers of 768, prompts of 140 / 200 / 256 tokens 480 / 680 / 675
-    us, with the library's 770; captured, 335 / 350 / 355 and 328 / 345 / 347).
+    captured (six layers of 768, prompts of 140 / 200 / 256 tokens 490 / 685 / 685
+    us, with the library's 770; captured, 332 / 355 / 358 and 329 / 347 / 345).
     Measured with the kernel that reads them
     (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 16.9 (19.1)
     / 26.1 (30.0) / 30.0 (30.4), 4096x14336 26.6 (32.8) / 35.3 (79) / 42.4

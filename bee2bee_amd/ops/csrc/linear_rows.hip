@@ -17,12 +17,12 @@
 //    columns each leave CUs without one, and better pieces to load elsewhere.
 //    These loads carry the streaming hint (STREAM): weights that no cache holds
 //    come 3 to 9% sooner (2x14336x4096 41 us without and 36.5 with, 4096x14336
-//    24.2 and 22.1, 2048x2048 5.0 and 4.6), but those that the 256 MB memory-side
+//    24.2 and 22.1, 2048x2048 4.4 and 4.1), but those that the 256 MB memory-side
 //    cache has kept since the last step 5 to 15% later, at the time of those that
 //    it has not. So not where the sides are those of stacks of 768 (sides up to
 //    768 and 4096), which fit there whole: distilgpt2, one row, repeated 199.6 us
 //    with the hint on all and 187.2, a first step on new weights 230 and 218;
-//    with three such stacks in turn, which do not fit, 205 and 212. 1024x1024
+//    with three such stacks in turn, which do not fit, 205 and 213. 1024x1024
 //    belongs to stacks that do not fit: 3.4 us with it and 3.8.
 //  * Between two layers' projections the residual sum stays in fp32: the norm
 //    after an add takes the sum before it is rounded, as the kernel that adds
