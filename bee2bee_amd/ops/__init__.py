@@ -291,6 +291,32 @@ def rows_qkv(x, w, bias, norm, n_heads: int, positions, cos, sin, k_cache,
                               k_cache, v_cache, slot_mapping)
 
 
+def stack_rows(spec) -> int:
+    """Most rows of a decode step whose layers decode_stack takes, 0 for stacks
+    that it does not: dense ones with sizes of whole steps of 64, heads of 64 or
+    128, a layer norm of up to 1024 columns, and as many rows as fit into a CU's
+    LDS."""
+    return require_hip().stack_rows(
+        spec.hidden_size, spec.n_heads, spec.n_kv_heads, spec.head_dim,
+        spec.intermediate_size, spec.norm_type == "layernorm")
+
+
+def decode_stack(x, layers, pages, n_heads: int, act: str, eps: float,
+                 scale: float, positions, cos, sin, slot_mapping, block_table,
+                 seq_lens, workgroups: int = 256):
+    """Decoder layers of one token of each of x's rows [M, H], on the GPU:
+    q|k|v (rotated unless positions is None) with its page store, attention
+    against the pages, output, feed-forward. layers: their weights; pages: their
+    (keys, values). workgroups: fewer than 256 compute the same."""
+    return require_hip().decode_stack(
+        x, [[w.wqkv, w.wo, w.w_gate_up, w.w_down, w.wqkv_bias, w.wo_bias,
+             w.w_gate_up_bias, w.w_down_bias, w.attn_norm, w.mlp_norm,
+             w.attn_norm_bias, w.mlp_norm_bias, *kv]
+            for w, kv in zip(layers, pages)],
+        n_heads, act == "gelu", eps, scale, positions, cos, sin, slot_mapping,
+        block_table, seq_lens, workgroups)
+
+
 # Steps of some tens of rows: projections as fp32 parts over their inner
 # dimension, which the next kernel sums, or as activated bf16 rows.
 

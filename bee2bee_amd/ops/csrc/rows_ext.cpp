@@ -1,10 +1,12 @@
 // Torch bindings of the projections of a few rows (linear_rows.hip), of some tens
-// (linear_mid.hip) and more (linear_wide.hip), and of the pass between q|k|v and
-// attention.
+// (linear_mid.hip) and more (linear_wide.hip), of the pass between q|k|v and
+// attention, and of a decode step's layers in one launch (decode_stack.hip).
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <limits>
+#include "decode_stack.h"
 
 using torch::Tensor;
 using c10::optional;
@@ -15,6 +17,10 @@ extern "C" int launch_linear_rows(
     int, void*, int, const unsigned short*, unsigned short*, float*, int, int,
     int, float, int, int, const int*, const float*, const float*, const int*,
     void*, void*, int, int, int, int, int, hipStream_t);
+extern "C" int decode_stack_rows(int, int);
+extern "C" int decode_stack_splits(long, long);
+extern "C" int launch_decode_stack(const StackArgs*, int, int, int, int,
+                                   hipStream_t);
 extern "C" int linear_mid_splits(int, int);
 extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
                                  const unsigned short*, void*, int, int, int,
@@ -243,6 +249,152 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
     return q;
 }
 
+// Most rows of a decode step whose layers decode_stack takes, 0 for a stack that
+// it does not take.
+int64_t stack_rows(int64_t hidden, int64_t nq, int64_t nkv, int64_t hd,
+                   int64_t inner, bool layer_norm) {
+    const int64_t deepest = std::max(std::max(hidden, nq * hd), inner);
+    if ((hd != 64 && hd != 128) || nkv < 1 || nq % nkv || nq / nkv > 16 ||
+        hidden % 64 || inner % 64 || deepest > 1 << 16 ||
+        (layer_norm && hidden > DS_LAYER_NORM))
+        return 0;
+    return decode_stack_rows((int)deepest, (int)hd);
+}
+
+// The layers of a decode step, x [M, H] to the last one's result. A layer is 14
+// tensors: w_qkv, w_o, w_up, w_down, their biases, the two norms' weights, their
+// biases (layer norm: all given), pages of keys and of values. wgs: workgroups
+// (DS_WGS; fewer do the work of the others).
+Tensor decode_stack(const Tensor& x,
+                    const std::vector<std::vector<optional<Tensor>>>& layers,
+                    int64_t nq, bool gelu, double eps, double scale,
+                    const optional<Tensor>& pos, const optional<Tensor>& cos_t,
+                    const optional<Tensor>& sin_t, const Tensor& slots,
+                    const Tensor& table, const Tensor& seq_lens, int64_t wgs) {
+    const int L = layers.size();
+    TORCH_CHECK(L >= 1 && layers[0].size() == 14);
+    const Tensor xd = dense(x, "x");
+    TORCH_CHECK(xd.dim() == 2);
+    const Tensor& k0 = layers[0][12].value();
+    TORCH_CHECK(k0.dim() == 4);
+    const int M = xd.size(0), H = xd.size(1), nkv = k0.size(1),
+              bs = k0.size(2), hd = k0.size(3);
+    const bool fp8 = k0.scalar_type() == torch::kUInt8;
+    TORCH_CHECK(fp8 || k0.scalar_type() == torch::kBFloat16);
+    const bool norm_b = layers[0][10].has_value();
+    const int Q = nq * hd, N = (nq + 2 * nkv) * hd;
+    const int I = layers[0][3].value().size(1);
+    TORCH_CHECK(M >= 1 && M <= stack_rows(H, nq, nkv, hd, I, norm_b), "rows");
+    auto ints = [&](const Tensor& t, long n, const char* name) {
+        TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt32 &&
+                    t.is_contiguous() && t.numel() == n, name);
+        return t.data_ptr<int>();
+    };
+    TORCH_CHECK(table.dim() == 2 && table.size(0) == M && table.size(1) > 0);
+
+    StackArgs a{};
+    a.M = M;
+    a.gelu = gelu;
+    a.nq = nq;
+    a.nkv = nkv;
+    a.G = nq / nkv;
+    a.bs = bs;
+    a.W = table.size(1);
+    a.eps = (float)eps;
+    a.scale = (float)scale;
+    a.all = L;
+    a.slots = ints(slots, M, "slots");
+    a.table = ints(table, (long)M * a.W, "table");
+    a.seq_lens = ints(seq_lens, M, "seq_lens");
+    if (pos.has_value()) {
+        a.pos = ints(*pos, M, "positions");
+        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
+            TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kFloat32 &&
+                        t->is_contiguous() && t->size(1) == hd / 2);
+        a.cos_t = cos_t->data_ptr<float>();
+        a.sin_t = sin_t->data_ptr<float>();
+    }
+    const int up = gelu ? I : 2 * I;
+    const int K[4] = {H, Q, H, I}, rows[4] = {N, H, up, H};
+    for (int k = 0; k < 4; ++k) {
+        a.K[k] = K[k];
+        a.octets[k] = rows[k] / 8;
+        a.half[k] = k == DS_QKV ? hd / 2 : k == DS_UP && !gelu ? I : 4;
+    }
+    // (as linear_rows.hip: stacks of more than 768)
+    a.streamed = std::min(H, I) > 768 || std::max(up, I) > 4096;
+    a.Z = decode_stack_splits((long)M * nkv, (long)a.W * bs);
+
+    // words that pass, a layer's after the other's: queries, the step's own keys
+    // and values, attention's result, the rows after attention, activations, the
+    // rows after the layer
+    const long after = norm_b ? (long)M * H : (long)M * H / 2 + M * H / 8;
+    a.new_kv = M * Q / 2;
+    a.att = a.new_kv + M * nkv * hd;
+    a.o = a.att + M * Q / 2;
+    a.up = a.o + after;
+    a.down = a.up + M * I / 2;
+    a.stride = (a.down + after + 31) / 32 * 32;
+    const int launches = (L + DS_LAYERS - 1) / DS_LAYERS;
+    a.items = M * nkv * a.Z;
+    const long parts = a.Z > 1 ? (long)a.items * a.G * (hd / 16 * 18) : 0;
+    const long claims = (long)launches * DS_CLAIMS;
+    Tensor work = torch::full({claims + (long)L * a.stride + parts}, -1,
+                              xd.options().dtype(torch::kInt32));
+    unsigned* words = reinterpret_cast<unsigned*>(work.data_ptr());
+    a.words = words + claims;
+    a.parts = a.words + (long)L * a.stride;
+    Tensor x32 = torch::empty({M, H}, xd.options().dtype(torch::kFloat32));
+    Tensor out = torch::empty({M, H}, xd.options());
+    a.x = ptr(xd);
+    a.x32 = x32.data_ptr<float>();
+    a.out = reinterpret_cast<unsigned*>(out.data_ptr());
+
+    std::vector<StackLayer> told(L + 1);
+    std::vector<Tensor> kept;                  // copies of what is not dense
+    auto keep = [&](const Tensor& t) {
+        kept.push_back(t);
+        return ptr(t);
+    };
+    for (int l = 0; l < L; ++l) {
+        const auto& t = layers[l];
+        TORCH_CHECK(t.size() == 14);
+        StackLayer& s = told[l];
+        for (int k = 0; k < 4; ++k) {
+            const Tensor w = dense(t[k].value(), "weights");
+            TORCH_CHECK(w.dim() == 2 && w.size(0) == rows[k] &&
+                        w.size(1) == K[k], "sizes of the layer's products");
+            s.w[k] = keep(w);
+            TORCH_CHECK(k != DS_UP || gelu || !t[4 + k].has_value());
+            s.bias[k] = keep(column(t[4 + k], rows[k], "bias"));
+        }
+        for (int i = 0; i < 2; ++i) {
+            TORCH_CHECK(t[8 + i].has_value() &&
+                        t[10 + i].has_value() == norm_b, "norms");
+            s.norm[i] = keep(column(t[8 + i], H, "norm weight"));
+            s.norm_bias[i] = keep(column(t[10 + i], H, "norm bias"));
+        }
+        for (int i = 12; i < 14; ++i) {
+            const Tensor& c = t[i].value();
+            TORCH_CHECK(c.is_cuda() && c.sizes() == k0.sizes() &&
+                        c.scalar_type() == k0.scalar_type() &&
+                        c.is_contiguous() &&
+                        reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0,
+                        "pages");
+            (i == 12 ? s.k_cache : s.v_cache) = c.data_ptr();
+        }
+    }
+    for (int i = 0; i < launches; ++i) {
+        a.lo = i * DS_LAYERS;
+        a.hi = std::min(L, a.lo + DS_LAYERS);
+        a.claims = words + (long)i * DS_CLAIMS;
+        std::copy(told.begin() + a.lo, told.begin() + a.hi + 1, a.layer);
+        TORCH_CHECK(launch_decode_stack(&a, hd, fp8, norm_b, (int)wgs,
+                                        stream()) == 0);
+    }
+    return out;
+}
+
 // parts [S, M, N] fp32, whose sum over S is x w^T
 Tensor mid_linear(const Tensor& x, const Tensor& w) {
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1),
@@ -431,6 +583,9 @@ void register_rows_ops(pybind11::module_& m) {
           "the same without activation, and what the next RMS norm takes");
     m.def("rows_qkv", &rows_qkv,
           "norm, q|k|v projection, rotation and page store of a few rows");
+    m.def("stack_rows", &stack_rows,
+          "most rows of a decode step whose layers are one launch");
+    m.def("decode_stack", &decode_stack, "the layers of a decode step");
     m.def("mid_linear", &mid_linear,
           "projection of some tens of rows as fp32 parts over K");
     m.def("mid_rows_linear", &mid_rows_linear,

@@ -26,6 +26,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "attn_stream.hip"),
         os.path.join(CSRC, "rows_ext.cpp"),
         os.path.join(CSRC, "linear_rows.hip"),
+        os.path.join(CSRC, "decode_stack.hip"),
         os.path.join(CSRC, "linear_mid.hip"),
         os.path.join(CSRC, "linear_wide.hip"),
         os.path.join(CSRC, "probe.hip"),

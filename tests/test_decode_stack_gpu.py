@@ -1,0 +1,270 @@
+"""A decode step's layers in one launch (decode_stack.hip) against the reference
+ops in fp64: sizes at the edges of its octets, waves and tiles, contexts that one
+workgroup reads and such as are split, one row to the most, and fewer workgroups
+than there are numbers.
+
+Tolerance: what passes between the products is rounded to bf16 (2^-9 relative at
+most each, independent of each other), about eight times a layer, into a residual
+that is not: 1.5% of the result's norm, as the steps' tests ask for. 8-bit pages
+round the step's own keys and values, and queries, to 3 mantissa bits: 5%."""
+import types
+
+import pytest
+import torch
+
+from bee2bee_amd import ops
+from bee2bee_amd.ops import reference
+
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
+DEV = torch.device("cuda:0")
+
+
+def _spec(H, nq, nkv, hd, I, kind):
+    return types.SimpleNamespace(
+        hidden_size=H, n_heads=nq, n_kv_heads=nkv, head_dim=hd,
+        intermediate_size=I, norm_type=kind)
+
+
+def _layer(s, biased, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def rand(*shape, std=1.0, mean=0.0):
+        t = torch.empty(*shape, device=DEV).normal_(mean, std, generator=g)
+        return t.bfloat16()
+
+    H, I, Q = s.hidden_size, s.intermediate_size, s.n_heads * s.head_dim
+    gelu = s.norm_type == "layernorm"
+    N = Q + 2 * s.n_kv_heads * s.head_dim
+    up = I if gelu else 2 * I
+    lw = types.SimpleNamespace(
+        wo=rand(H, Q, std=2 * Q ** -0.5), w_gate_up=rand(up, H, std=H ** -0.5),
+        w_down=rand(H, I, std=2 * I ** -0.5), wqkv=rand(N, H, std=H ** -0.5))
+    for name in ("attn_norm", "mlp_norm"):
+        setattr(lw, name, rand(H, std=0.2, mean=1.0))
+        setattr(lw, name + "_bias", rand(H, std=0.2) if gelu else None)
+    for name, n in (("wo_bias", H), ("w_gate_up_bias", up if gelu else 0),
+                    ("w_down_bias", H), ("wqkv_bias", N)):
+        setattr(lw, name, rand(n, std=0.5) if biased and n else None)
+    return lw
+
+
+def _wide(lw):
+    return types.SimpleNamespace(**{
+        k: None if v is None else v.double() for k, v in vars(lw).items()})
+
+
+def _rel(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+class _Step:
+    """A stack with its pages; `lens` counts the step's own tokens."""
+
+    def __init__(self, spec, layers, lens, bs, biased=False, fp8=False, W=None):
+        self.spec, self.fp8, M = spec, fp8, len(lens)
+        self.layers = [_layer(spec, biased, i) for i in range(layers)]
+        g = torch.Generator(device=DEV).manual_seed(M)
+        W = W or max(-(-n // bs) for n in lens)
+        nb, nkv, hd = M * W + 1, spec.n_kv_heads, spec.head_dim
+        self.pages = []
+        for _ in range(layers):
+            kv = [torch.empty(nb, nkv, bs, hd, device=DEV).normal_(
+                generator=g) for _ in range(2)]
+            self.pages.append([
+                t.to(torch.float8_e4m3fn).view(torch.uint8) if fp8
+                else t.bfloat16() for t in kv])
+        self.table = 1 + torch.randperm(M * W, generator=g, device=DEV).int(
+            ).view(M, W)
+        self.lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        self.pos = self.lens - 1
+        at = self.pos.long()
+        self.slots = (self.table.gather(1, (at // bs)[:, None]).squeeze(1) * bs
+                      + at % bs).int()
+        self.x = torch.randn(M, spec.hidden_size, generator=g,
+                             device=DEV).bfloat16()
+        self.cos, self.sin = reference.rope_tables(max(lens), hd, 1e4, DEV)
+        self.rope = spec.norm_type == "rmsnorm"
+        self.act = "swiglu" if self.rope else "gelu"
+
+    def run(self, rows=None, workgroups=256, pages=None):
+        rows = list(range(len(self.x))) if rows is None else rows
+        pages = pages or [[t.clone() for t in kv] for kv in self.pages]
+        s = self.spec
+        out = ops.decode_stack(
+            self.x[rows], self.layers, pages, s.n_heads, self.act, 1e-5,
+            s.head_dim ** -0.5, self.pos[rows] if self.rope else None,
+            self.cos, self.sin, self.slots[rows], self.table[rows],
+            self.lens[rows], workgroups)
+        return out, pages
+
+    def want(self):
+        s, x = self.spec, self.x.double()
+        pages = []
+        for lw, kv in zip(self.layers, self.pages):
+            lw = _wide(lw)
+            kv = [(t.view(torch.float8_e4m3fn) if self.fp8 else t).double()
+                  for t in kv]
+            q = reference.rows_qkv(
+                x, lw.wqkv, lw.wqkv_bias, (lw.attn_norm, lw.attn_norm_bias,
+                                           1e-5), s.n_heads,
+                self.pos if self.rope else None, self.cos.double(),
+                self.sin.double(), *kv, self.slots)
+            o = _attention(q, *kv, self.table, self.lens)
+            x = reference.rows_linear(o, lw.wo, lw.wo_bias, x)
+            z = reference.rows_linear(
+                x, lw.w_gate_up, lw.w_gate_up_bias,
+                norm=(lw.mlp_norm, lw.mlp_norm_bias, 1e-5), act=self.act)
+            x = reference.rows_linear(z, lw.w_down, lw.w_down_bias, x)
+            pages.append(kv)
+        return x, pages
+
+
+def _attention(q, kc, vc, table, lens):
+    M, nq, hd = q.shape
+    nkv, bs = kc.shape[1:3]
+    out = []
+    for m in range(M):
+        k, v = (t[table[m].long()].transpose(0, 1).reshape(nkv, -1, hd)
+                [:, : lens[m]].repeat_interleave(nq // nkv, 0)
+                for t in (kc, vc))
+        p = torch.softmax((k @ q[m][:, :, None])[..., 0] * hd ** -0.5, -1)
+        out.append((p[:, None] @ v)[:, 0].reshape(-1))
+    return torch.stack(out)
+
+
+# H, query heads, key heads, head size, inner width, norm, biases, page size,
+# contexts: one octet to several a workgroup, waves without a step of K, sizes
+# that leave workgroups without an octet of some products; contexts of one key,
+# at the ends of tiles and pages, and split ones
+CASES = [
+    (64, 1, 1, 64, 64, "rmsnorm", False, 16, [1]),
+    (256, 4, 2, 64, 1024, "rmsnorm", True, 16, [33, 1, 16, 700, 32]),
+    (256, 2, 1, 128, 704, "rmsnorm", False, 24, [1025, 31, 2000]),
+    (768, 12, 12, 64, 3072, "layernorm", True, 256, [300]),
+    (768, 12, 12, 64, 3072, "layernorm", True, 32, [64, 1500, 257, 1024]),
+    (1024, 8, 8, 128, 704, "layernorm", False, 16, [5, 1030]),
+    (2048, 32, 8, 64, 8192, "rmsnorm", False, 256, [1000]),
+    (2048, 32, 8, 64, 2048, "rmsnorm", False, 256, [3000, 255, 256, 9, 1, 1024,
+                                                    1025, 2100]),
+    (3584, 28, 4, 128, 18944, "rmsnorm", True, 256, [5000, 8192]),
+    (4160, 32, 2, 128, 1088, "rmsnorm", False, 256, [31, 4000, 97]),
+]
+
+
+@pytest.mark.parametrize("workgroups", [256, 100, 3])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}-{c[8]}")
+def test_stack(case, fp8, workgroups):
+    H, nq, nkv, hd, I, kind, biased, bs, lens = case
+    if workgroups == 3 and (H > 1024 or fp8):
+        pytest.skip("long")
+    spec = _spec(H, nq, nkv, hd, I, kind)
+    assert len(lens) <= ops.stack_rows(spec)
+    step = _Step(spec, 2, lens, bs, biased, fp8)
+    got, pages = step.run(workgroups=workgroups)
+    want, want_pages = step.want()
+    limit = 0.05 if fp8 else 0.015
+    error = _rel(got, want)
+    assert error <= limit
+    s = step.slots.long()
+    for kv, kv_want, before in zip(pages, want_pages, step.pages):
+        for t, w, b in zip(kv, kv_want, before):
+            rows = (t.view(torch.float8_e4m3fn) if fp8 else t).double()
+            error = _rel(rows[s // bs, :, s % bs], w[s // bs, :, s % bs])
+            assert error <= limit
+            t[s // bs, :, s % bs] = b[s // bs, :, s % bs]
+            assert torch.equal(t, b)           # and nothing else
+
+
+def test_rows_and_workgroups_do_not_change_a_row():
+    """Contexts that are not split: a row is the same to the bit beside others,
+    and whoever computes it."""
+    spec = _spec(1024, 16, 4, 64, 2816, "rmsnorm")
+    step = _Step(spec, 2, [40, 1000, 7, 513, 64, 1, 300, 999], 16)
+    full, _ = step.run()
+    for rows in ([3], [5, 2], [7, 0, 1, 4, 6]):
+        assert torch.equal(step.run(rows)[0], full[rows])
+        assert torch.equal(step.run(rows, 77)[0], full[rows])
+
+
+def test_more_layers_than_a_launch_takes():
+    spec = _spec(128, 2, 1, 64, 128, "rmsnorm")
+    step = _Step(spec, 64, [70, 1], 16)
+    for lw in step.layers:
+        lw.wo *= 0.2
+        lw.w_down *= 0.2
+    got, want = step.run()[0], step.want()[0]
+    error = _rel(got, want)
+    assert error <= 0.03
+
+
+def test_values_that_are_not_numbers_pass():
+    """A NaN in one row is that row's alone, and nothing waits for it; so with
+    all bits set, the mark of words that are not there yet."""
+    spec = _spec(256, 4, 2, 64, 1024, "rmsnorm")
+    step = _Step(spec, 2, [5, 1200, 40], 16)
+    step.x.view(torch.int16)[1] = -1
+    got = step.run()[0]
+    assert got[1].isnan().all() and not got[[0, 2]].isnan().any()
+    # in what a page holds behind the context's end
+    step = _Step(spec, 2, [5, 1200, 40], 16)
+    want = step.run()[0]
+    for kv in step.pages:
+        for t in kv:
+            for m, n in enumerate(step.lens.tolist()):
+                page = t[step.table[m, (n - 1) // 16].item()]
+                page[:, (n - 1) % 16 :] = float("nan")
+    assert torch.equal(step.run()[0], want)
+
+
+def test_a_token_without_a_position():
+    """Slot -1: nothing is stored, and attention reads what the pages hold, as
+    the plain route does."""
+    spec = _spec(256, 4, 2, 64, 1024, "rmsnorm")
+    step = _Step(spec, 1, [48, 20], 16)
+    step.slots[0] = -1
+    step.lens[0] = 49                          # past its three pages
+    got, pages = step.run()
+    s = step.slots.clone()
+    step.slots[0] = 0                          # (page 0 is nobody's)
+    step.lens[0] = 48
+    want = step.want()[0]
+    error = _rel(got, want)
+    assert error <= 0.015
+    before = [[t.clone() for t in kv] for kv in step.pages]
+    for kv, b in zip(pages, before):
+        for t, old in zip(kv, b):
+            t[s[1] // 16, :, s[1] % 16] = old[s[1] // 16, :, s[1] % 16]
+            assert torch.equal(t, old)
+
+
+def test_refused():
+    spec = _spec(256, 4, 2, 64, 1024, "rmsnorm")
+    step = _Step(spec, 1, [5, 12], 16)
+    ok = dict(x=step.x, table=step.table, lens=step.lens, slots=step.slots,
+              layers=step.layers, pages=step.pages)
+
+    def call(**change):
+        a = {**ok, **change}
+        return ops.decode_stack(a["x"], a["layers"], a["pages"], 4, "swiglu",
+                                1e-5, 0.125, step.pos, step.cos, step.sin,
+                                a["slots"], a["table"], a["lens"])
+
+    call()
+    narrow = types.SimpleNamespace(**{**vars(step.layers[0]),
+                                      "wo": step.layers[0].wo[:, :128]})
+    for bad in [dict(x=step.x[:1]), dict(x=step.x.float()),
+                dict(x=step.x[:, :192]), dict(lens=step.lens.long()),
+                dict(slots=step.slots[:1]), dict(table=step.table[:1]),
+                dict(layers=[narrow]), dict(layers=[], pages=[]),
+                dict(pages=[[t[:, :1] for t in step.pages[0]]])]:
+        with pytest.raises((RuntimeError, TypeError, IndexError)):
+            call(**bad)
+    assert ops.stack_rows(_spec(2048, 2, 2, 64, 256, "layernorm")) == 0
+    assert ops.stack_rows(_spec(256, 4, 2, 96, 256, "rmsnorm")) == 0
+    assert ops.stack_rows(_spec(288, 4, 2, 64, 256, "rmsnorm")) == 0
+    assert ops.stack_rows(_spec(256, 34, 2, 64, 256, "rmsnorm")) == 0
