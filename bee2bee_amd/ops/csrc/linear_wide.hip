@@ -8,9 +8,10 @@
 //          leave much of the chip idle.
 //
 // Bound by the matrix cores (at the clock that the power limit leaves them:
-// 8192x8192x8192 704 to 729 us from card to card, 1510 to 1560 TFLOP/s). A workgroup a CU: 256 rows of x by 256
-// of w, 64 of K at a time in one of two buffers of 64 KB, filled straight from
-// memory. Eight waves, two a SIMD: 128 x 64 sums each, in four quarters of 64 x
+// 8192x8192x8192 704 to 729 us from card to card, 1510 to 1560 TFLOP/s). A
+// workgroup a CU: 256 rows of x (or 128, 160, 192, 224: so many as fill the last
+// round) by 256 of w, 64 of K at a time in one of two buffers of 64 KB, filled
+// straight from memory. Eight waves, two a SIMD: 128 x 64 sums each, in four quarters of 64 x
 // 32. Waves 0-3 read a quarter's fragments while 4-7 multiply, and the other way
 // round, so that the matrix cores always have one of a SIMD's two waves; a
 // barrier at each change keeps them apart. What a quarter has read is loaded
@@ -64,16 +65,35 @@ DEV_INLINE void lw_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Fewest loads of a wave in X regions of x that follow one another, the last of
+// them of the second half, or of either
+constexpr int lw_loads(int MA, int MB, int X, bool second) {
+    int least = 1 << 30;
+    for (int early = 0; early < 2; ++early)    // waves 0-3, 4-7
+        for (int last = second; last < 2; ++last) {
+            int sum = 0;
+            for (int i = 0; i < X; ++i) {
+                const int g = (last + i) % 2, mt = g ? MB : MA;
+                sum += mt == 4 || (mt == 3 && (early == 0) == (g == 0)) ? 2 : 1;
+            }
+            least = sum < least ? sum : least;
+        }
+    return least;
+}
+
 constexpr int LW_REGION = 128 * 128;           // 128 rows of 64 of K
 constexpr int LW_LDS = 8 * LW_REGION;
 
-// MT: tiles of 16 rows of x that a wave takes in each half of a tile's 64 * MT
-template <int FORM, int MT>
+// MA, MB: tiles of 16 rows of x that a wave takes in either half of a tile's
+// 32 * (MA + MB) rows
+template <int FORM, int MA, int MB>
 __global__ __launch_bounds__(512) void linear_wide_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
     void* __restrict__ out, int M, int N, int K, int S, int TM, int TN,
     int strip, int stride) {
-    constexpr int BM = MT * 64, HM = MT * 32;          // rows, of a half
+    constexpr int BM = (MA + MB) * 32, HM = MA * 32;   // rows, of the first half
+    static_assert(MA >= MB && MB >= 2 && MA <= 4, "");
+    auto MT = [](int g) { return g ? MB : MA; };
     constexpr int BN = FORM == LW_GATED ? 128 : 256;   // columns of a tile
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -104,10 +124,11 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     // belong at l * 16 (xor-ed by half the row's number: no two of a read's 16
     // rows meet in a bank)
     const char *xb, *wb, *wb1;
-    // Of each half of w's 256 rows a wave loads 16, of x's MT / 2 times 8 (MT 3:
-    // two of one half, one of the other, waves 4-7 the other way round).
+    // Of each half of w's 256 rows a wave loads 16, of x's twice 8, or once (of
+    // halves of 96 rows four waves twice: of the first half 0-3, of the other
+    // 4-7).
     auto first = [&](int g) {                  // its first 8 rows of x's half
-        return MT == 4 ? wid * 2 : MT == 2 ? wid
+        return MT(g) == 4 ? wid * 2 : MT(g) == 2 ? wid
                : (wid < 4) == (g == 0) ? wid % 4 * 2 : 8 + wid % 4;
     };
     unsigned xo[2][2], wo[2][2];
@@ -138,7 +159,7 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
         const char* b = xb + (long)step * 128;
         const unsigned at = to + (buf * 4 + g) * LW_REGION + first(g) * 1024;
         lw_load(b, xo[g][0], at);
-        if (MT == 4 || (MT == 3 && (wid < 4) == (g == 0)))
+        if (MT(g) == 4 || (MT(g) == 3 && (wid < 4) == (g == 0)))
             lw_load(b, xo[g][1], at + 1024);
     };
     auto load_w = [&](int buf, int g, int step) {
@@ -148,39 +169,44 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
         lw_load(b, wo[g][1], at + 1024);
     };
     // until at most R regions' loads are under way (in the order w, x 0, w, x 1
-    // of a step, the last of them x 1 where AT 1; MT 3: as the wave has it that
-    // issued fewer), and, behind a whole tile's `stores`, those
-    constexpr int STORES = FORM == LW_GATED ? 2 * MT
-                           : FORM == LW_ROWS ? 4 * MT : 8 * MT;
+    // of a step; the last of them x 1 where AT 1, and either kind elsewhere: R is
+    // 6 there; as the wave has it that issued fewest), and, behind a whole tile's
+    // `stores`, those
+    constexpr int STORES = (FORM == LW_GATED ? 1 : FORM == LW_ROWS ? 2 : 4) *
+                           (MA + MB);
     bool stores = false;
     auto wait = [&](auto regions, auto at1) {
         constexpr int R = decltype(regions)::value;
         constexpr bool A = decltype(at1)::value;
         constexpr int W = A ? R / 2 : (R + 1) / 2, X = R - W;
-        constexpr int L = W * 2 + (MT == 4 ? X * 2 : MT == 2 ? X : X * 3 / 2);
+        static_assert(A || R == 6, "");
+        constexpr int L = W * 2 + lw_loads(MA, MB, X, A);
         if (!A && stores) lw_wait<L + STORES>();
         else lw_wait<L>();
     };
 
-    f32x4 acc[2][2][MT][2];                    // half of x, of w, tiles
+    f32x4 acc[2][2][MA][2];                    // half of x, of w, tiles
     auto clear = [&]() {
 #pragma unroll
-        for (int i = 0; i < MT * 8; ++i)
-            acc[i / (4 * MT)][i / (2 * MT) & 1][i / 2 % MT][i & 1] =
+        for (int i = 0; i < MA * 8; ++i)
+            acc[i / (4 * MA)][i / (2 * MA) & 1][i / 2 % MA][i & 1] =
                 f32x4{0.f, 0.f, 0.f, 0.f};
     };
     clear();
-    bf16x8 fa[MT][2], fb[2][2][2];
+    bf16x8 fa[MA][2], fb[2][2][2];
     const int p0 = (lg ^ (li >> 1)) * 16;      // of K 0-31; 32-63: ^ 64
-    const char* af = smem + (wm * MT * 16 + li) * 128;
+    const char* af = smem + (wm * MB * 16 + li) * 128;
     const char* bf = smem + (wn * 32 + li) * 128;
+    const char* af0 = smem + (wm * MA * 16 + li) * 128;
     auto read_x = [&](int buf, int g) {
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-                fa[i][k] = *reinterpret_cast<const bf16x8*>(
-                    af + (p0 ^ k * 64) + (buf * 4 + g) * LW_REGION + i * 2048);
+            for (int i = 0; i < MA; ++i)
+                if (i < MT(g))
+                    fa[i][k] = *reinterpret_cast<const bf16x8*>(
+                        (MA == MB || g ? af : af0) + (p0 ^ k * 64) +
+                        (buf * 4 + g) * LW_REGION + i * 2048);
     };
     auto read_w = [&](int buf, int g) {
 #pragma unroll
@@ -196,7 +222,7 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT(gx); ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
                     acc[gx][gw][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -262,7 +288,7 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
     auto finish = [&](int fm, int fn, int fp) {
         const bool whole = fm + BM <= M && fn + BN <= N;
         const int l = lw_lane(), lg = l >> 4;
-        const int r0 = fm + wm * MT * 16 + (l & 15);
+        const int r0 = fm + (l & 15);
         const int c0 = fn + wn * 32 +
                        (FORM == LW_PARTS ? lg * 4
                                          : (lg & 1) * 16 + (lg >> 1) * 8);
@@ -276,7 +302,8 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
                     reinterpret_cast<unsigned short*>(out) + at) = v;
         };
         auto rows = [&](int gx, int i, int gw, auto all) {
-            const int row = r0 + gx * HM + i * 16, col = c0 + gw * 128;
+            const int row = r0 + gx * HM + (wm * MT(gx) + i) * 16;
+            const int col = c0 + gw * 128;
             if constexpr (FORM == LW_PARTS) {
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
@@ -316,7 +343,7 @@ __global__ __launch_bounds__(512) void linear_wide_kernel(
 #pragma unroll
             for (int gx = 0; gx < 2; ++gx)
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
+                for (int i = 0; i < MT(gx); ++i)
 #pragma unroll
                     for (int gw = 0; gw < (FORM == LW_GATED ? 1 : 2); ++gw)
                         rows(gx, i, gw, all);
@@ -408,6 +435,47 @@ static double lw_time_parts(int M, int N, int K, int tall, int S) {
     return t;
 }
 
+// Heights between those of 64 rows: a third fit, of all five in one run (174
+// products of 4M weights and more and 86 gated ones, 257 to 12000 rows, weights
+// that no cache holds), that only compares heights.
+static double lw_time_rows(int M, int N, int K, int S, bool gated, int rows) {
+    struct Fit { double step, idle, busy, start, round, store; };
+    static const Fit fits[2][5] = {
+        {{0.754, 0.722, 0.989, 5.7, 0, 0.244}, {0.88, 0.807, 0.148, 8.3, 0, 0.183},
+         {0.998, 0.709, 0.231, 9.3, 0.6, 0.144},
+         {1.137, 0.68, 0.214, 9.6, 1.9, 0.124},
+         {1.285, 0.684, 0.184, 13.4, 0.2, 0.139}},
+        {{0.821, 0.595, 0.746, 6.8, 0, 0}, {0.935, 0.707, 0.313, 6.6, 0, 0},
+         {1.031, 0.748, 0.672, 3.2, 0.9, 0}, {1.181, 0.717, 0.239, 6.1, 0.8, 0},
+         {1.345, 0.632, 0.315, 8.2, 0, 0}}};
+    const Fit& f = fits[gated][rows / 32 - 4];
+    const int BN = gated ? 128 : 256;
+    const long tiles = ((M + rows - 1L) / rows) * ((N + BN - 1) / BN) * S;
+    const double steps = K / 64 / S * f.step, full = tiles / 256,
+                 left = (tiles % 256) / 256.0;
+    double t = f.start + full * (steps + f.round);
+    if (left > 0) {
+        const double part = f.idle + f.busy * left;
+        t += steps * (part < 1 ? part : 1) + f.round;
+    }
+    return S > 1 ? t + (double)M * N / 1e6 * 4 * S * f.store : t;
+}
+
+// Rows of a tile of a plan's 64 * tall: 160 for 192 and 224 for 256 where fewer
+// of them stand over in the last round, and 3% of the time (4559x3072x8192: 18 by
+// 12 tiles of 256 rows leave 40 CUs idle, 170 us; 21 by 12 of 224 154). A product
+// that would take the height tall - 1 takes these, too, if they beat it by as
+// much. Of the 260 products, 77 are 7% faster for it and one is 2% slower; all
+// heights' results are the same.
+static bool lw_between(int M, int N, int K, int S, bool gated, int tall) {
+    return tall > 2 && lw_time_rows(M, N, K, S, gated, tall * 64 - 32) <
+                           0.97 * lw_time_rows(M, N, K, S, gated, tall * 64);
+}
+extern "C" int linear_wide_rows(int M, int N, int K, int S, int form, int tall) {
+    return tall * 64 -
+           (lw_between(M, N, K, S, form == LW_GATED, tall) ? 32 : 0);
+}
+
 // The tile's height and number of parts (1: rows) that are fastest: tall + 8 *
 // parts, or 0: left to the library. Parts only where LW_PARTS is asked for. +
 // 128: the rows past the last whole tile are linear_mid.hip's, which reads the
@@ -450,6 +518,20 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
                 best = tall + 8 + 128;
             }
         }
+    if (best < 128) {
+        const bool gated = form == LW_GATED;
+        const int S = best / 8;
+        const int rows = linear_wide_rows(M, N, K, S, form, best % 8);
+        const double own = lw_time_rows(M, N, K, S, gated, best % 8 * 64);
+        double now = lw_time_rows(M, N, K, S, gated, rows);
+        for (int tall = 3; tall <= 4; ++tall) {
+            if (!lw_between(M, N, K, S, gated, tall)) continue;
+            const double t = lw_time_rows(M, N, K, S, gated, tall * 64 - 32);
+            if (t >= 0.97 * own || t >= now) continue;
+            now = t;
+            best = tall + 8 * S;
+        }
+    }
     const double flops = 2.0 * M * N * K, bytes = 2.0 * N * K;
     if (form == LW_GATED) return best;
     if (form == LW_PARTS) {
@@ -469,37 +551,41 @@ extern "C" int linear_wide_plan(int M, int N, int K, int form) {
 
 // x [M, K], w [N, K] (LW_GATED [2N, K]) and out [M, N] (LW_PARTS [S, M, N] fp32)
 // contiguous, 16-byte aligned; K % (128 S) == 0, N % 8 == 0; S 1 but for LW_PARTS;
-// tall: 2, 3 or 4 times 64 rows a tile. Nonzero for anything else.
+// rows of a tile: 128, 160 .. 256. Nonzero for anything else.
 extern "C" int launch_linear_wide(const unsigned short* x,
                                   const unsigned short* w, void* out, int M,
-                                  int N, int K, int S, int form, int tall,
+                                  int N, int K, int S, int form, int rows,
                                   hipStream_t stream) {
     if (M < 1 || N < 8 || N % 8 || S < 1 || K < 1 || K % (128L * S)) return 1;
     if (form != LW_PARTS && S != 1) return 1;
+    if (rows < 128 || rows > 256 || rows % 32) return 1;
     if (K > 1 << 22) return 1;                 // offsets in a tile: 32 bits
-    const int BN = form == LW_GATED ? 128 : 256, BM = tall * 64;
-    const int TM = (M + BM - 1) / BM, TN = (N + BN - 1) / BN;
+    const int BN = form == LW_GATED ? 128 : 256;
+    const int TM = (M + rows - 1) / rows, TN = (N + BN - 1) / BN;
     if ((long)TM * TN * S > 1 << 30) return 1;
     const int strips = (TM + 7) / 8, strip = (TM + strips - 1) / strips;
     const bool stay = TM * TN * S > 256;       // a workgroup a CU
     const dim3 grid(stay ? 256 : TM * TN * S);
     const int stride = stay ? 32 : 1 << 30;
-#define LW_GO(F, T)                                                           \
-    if (form == F && tall == T) {                                             \
-        hipLaunchKernelGGL((linear_wide_kernel<F, T>), grid, dim3(512),       \
+#define LW_ONE(F, A, B)                                                       \
+    if (rows == (A + B) * 32) {                                               \
+        hipLaunchKernelGGL((linear_wide_kernel<F, A, B>), grid, dim3(512),    \
                            LW_LDS, stream, x, w, out, M, N, K, S, TM, TN,     \
                            strip, stride);                                    \
         return 0;                                                             \
     }
-    LW_GO(LW_ROWS, 2)
-    LW_GO(LW_ROWS, 3)
-    LW_GO(LW_ROWS, 4)
-    LW_GO(LW_GATED, 2)
-    LW_GO(LW_GATED, 3)
-    LW_GO(LW_GATED, 4)
-    LW_GO(LW_PARTS, 2)
-    LW_GO(LW_PARTS, 3)
-    LW_GO(LW_PARTS, 4)
+#define LW_GO(F)                                                              \
+    if (form == F) {                                                          \
+        LW_ONE(F, 2, 2)                                                       \
+        LW_ONE(F, 3, 2)                                                       \
+        LW_ONE(F, 3, 3)                                                       \
+        LW_ONE(F, 4, 3)                                                       \
+        LW_ONE(F, 4, 4)                                                       \
+    }
+    LW_GO(LW_ROWS)
+    LW_GO(LW_GATED)
+    LW_GO(LW_PARTS)
+#undef LW_ONE
 #undef LW_GO
     return 1;
 }

@@ -27,6 +27,7 @@ extern "C" int launch_linear_mid(const unsigned short*, const unsigned short*,
                                  int, int, int, const float*, float,
                                  hipStream_t);
 extern "C" int linear_wide_plan(int, int, int, int);
+extern "C" int linear_wide_rows(int, int, int, int, int, int);
 extern "C" int launch_linear_wide(const unsigned short*, const unsigned short*,
                                   void*, int, int, int, int, int, int,
                                   hipStream_t);
@@ -442,6 +443,13 @@ int64_t wide_plan(int64_t M, int64_t N, int64_t K, int64_t form) {
     return linear_wide_plan(M, N, K, form);
 }
 
+// rows of a tile of that plan
+int64_t wide_height(int64_t M, int64_t N, int64_t K, int64_t plan, bool gated) {
+    TORCH_CHECK(M >= 1 && plan % 8 >= 2 && plan % 8 <= 4 && plan >= 8);
+    return linear_wide_rows(M, N, K, plan / 8 % 16,
+                            gated ? WIDE_GATED : WIDE_ROWS, plan % 8);
+}
+
 // x w^T in bf16; silu(gate) * value of w's two halves (gated); or, where the
 // plan has several parts, [S, M, N] fp32
 Tensor wide_linear(const Tensor& x, const Tensor& w, int64_t plan,
@@ -463,7 +471,10 @@ Tensor wide_linear(const Tensor& x, const Tensor& w, int64_t plan,
     const int tail = plan >= 128 ? M % (tall * 64) : 0;
     TORCH_CHECK(plan < 256 && (tail == 0 || (S == 1 && tail < M)), "a plan");
     TORCH_CHECK(launch_linear_wide(ptr(xd), ptr(wd), y.data_ptr(), M - tail,
-                                   N, K, S, form, tall, stream()) == 0);
+                                   N, K, S, form,
+                                   linear_wide_rows(M - tail, N, K, S, form,
+                                                    tall),
+                                   stream()) == 0);
     if (tail)
         TORCH_CHECK(launch_linear_mid(
                         ptr(xd) + (long)(M - tail) * K, ptr(wd), nullptr,
@@ -592,6 +603,7 @@ void register_rows_ops(pybind11::module_& m) {
           "projection of some tens of rows, with bias and activation");
     m.def("wide_plan", &wide_plan,
           "tile and parts of a projection of many rows, 0 for the library");
+    m.def("wide_height", &wide_height, "rows of a tile of a plan");
     m.def("wide_linear", &wide_linear,
           "projection of many rows, gated or as parts where wanted");
     m.def("add_norm_parts", &add_norm_parts,

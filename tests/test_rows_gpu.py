@@ -336,6 +336,34 @@ def test_wide_products(M, N, K, act, S, tall):
         assert ((got - want).abs() <= bound).all()
 
 
+# (tiles of 160 and 224 rows, whose halves differ: one row or one short of a tile
+# past the last, rows that end in either half; several tiles a workgroup)
+@pytest.mark.parametrize("M,N,K,act,S,tall", [
+    (161, 264, 256, None, 1, 3), (449, 8712, 768, None, 1, 3),
+    (2242, 1032, 768, None, 1, 3), (4559, 4104, 512, None, 1, 3),
+    (321, 3072, 768, None, 2, 3), (2242, 264, 512, None, 2, 3),
+    (449, 4104, 768, "swiglu", 1, 3), (4559, 3072, 512, "swiglu", 1, 3),
+    (225, 264, 512, None, 1, 4), (1121, 1032, 512, None, 1, 4),
+    (2241, 3072, 256, None, 1, 4), (4481, 4104, 256, None, 1, 4),
+    (1345, 3072, 256, None, 2, 4), (321, 9000, 256, "swiglu", 1, 4),
+    (3001, 3072, 256, "swiglu", 1, 4)])
+def test_heights_between(M, N, K, act, S, tall):
+    """As above, and to the bit what tiles of 128 rows give."""
+    plan = tall + 8 * S
+    hip = ops.require_hip()
+    assert hip.wide_height(M, N, K, plan, bool(act)) == 64 * tall - 32
+    assert hip.wide_height(M, N, K, 2 + 8 * S, bool(act)) == 128
+    torch.manual_seed(M + N)
+    x, w = _rand(M, K), _rand(2 * N if act else N, K, std=0.1)
+    got = ops.wide_linear(x, w, plan, act)
+    assert torch.equal(got, ops.wide_linear(x, w, 2 + 8 * S, act))
+    if S == 1 and not act:
+        want = x.double() @ w.double().t()
+        e = 2 ** -24 * K * (x.double().abs() @ w.double().abs().t())
+        bound = e + (2 ** -8 + 2 ** -20) * want.abs() + 1e-6
+        assert ((got.double() - want).abs() <= bound).all()
+
+
 def test_wide_plans_are_what_the_kernel_takes():
     """Whole pairs of steps a part, parts only for a reader that sums them, rows
     apart only beside whole tiles; sizes that the kernel does not take stay with
