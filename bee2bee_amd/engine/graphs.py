@@ -77,9 +77,8 @@ class DecodeGraphs:
         pos = self.positions[:B]
         bt = self.block_table[:B]
         lens = self.seq_lens[:B]
-        slots = decode_slot_mapping(bt, pos, self.runner.kv.block_size)
         st = None if self.state_slots is None else self.state_slots[:B]
-        hidden = self.runner.forward_decode(ids, pos, slots, bt, lens,
+        hidden = self.runner.forward_decode(ids, pos, None, bt, lens,
                                             state_slots=st)
         return self.runner.lm_head(hidden)
 

@@ -92,8 +92,8 @@ class Runner:
 
         return dist.get_world_size(self.tp_group) == 1
 
-    def _one_launch(self, x: torch.Tensor, slot_mapping, block_table,
-                    seq_lens) -> bool:
+    def _one_launch(self, x: torch.Tensor, positions, slot_mapping,
+                    block_table, seq_lens) -> bool:
         """Decode steps whose layers are one launch (ops.decode_stack); a tensor-
         parallel rank's rows are reduced between its products. What it saves,
         about 2 us a launch, is a layer's; what passes between its workgroups
@@ -108,8 +108,8 @@ class Runner:
         return (x.is_cuda and self.decode_attn_fn is None and self._mid_dims
                 and ops.few_rows(x) and self.layer_lo < self.layer_hi
                 and (s.act_type == "gelu" or not s.mlp_bias)
-                and slot_mapping.dtype is block_table.dtype is seq_lens.dtype
-                is torch.int32
+                and all(t is None or t.dtype is torch.int32 for t in (
+                    positions, slot_mapping, block_table, seq_lens))
                 and x.shape[0] <= min(4, ops.stack_rows(s)))
 
     @property
@@ -661,13 +661,17 @@ class Runner:
         self,
         input_ids_or_hidden: torch.Tensor,
         positions: torch.Tensor,
-        slot_mapping: torch.Tensor,
+        slot_mapping: Optional[torch.Tensor],
         block_table: torch.Tensor,
         seq_lens: torch.Tensor,
         state_slots: Optional[torch.Tensor] = None,
     ) -> torch.Tensor:
         """One-token-per-sequence step. input [B] ids (or [B, H] hidden for
-        later pipeline stages); returns final hidden [B, H]."""
+        later pipeline stages); returns final hidden [B, H]. slot_mapping
+        None: where block_table has the positions."""
+        if slot_mapping is None and self.spec.is_hybrid:
+            slot_mapping = ops.decode_slots(block_table, positions,
+                                            self.kv.block_size)
         if self.spec.is_hybrid:
             B = input_ids_or_hidden.shape[0]
             cu = torch.arange(B + 1, dtype=torch.int32, device=self.device)
@@ -691,15 +695,19 @@ class Runner:
             if self.is_first_stage
             else input_ids_or_hidden
         )
-        if self._one_launch(hidden, slot_mapping, block_table, seq_lens):
+        if self._one_launch(hidden, positions, slot_mapping, block_table,
+                            seq_lens):
             s, layers = self.spec, range(self.layer_lo, self.layer_hi)
             return ops.decode_stack(
                 hidden, [self.weights.layers[i] for i in layers],
                 [self.kv.layer(i) for i in layers], s.n_heads,
                 "gelu" if s.act_type == "gelu" else "swiglu", s.rms_eps,
-                self.scale, positions if s.pos_type == "rope" else None,
-                self.rope_cos, self.rope_sin, slot_mapping,
-                block_table.contiguous(), seq_lens)
+                self.scale, positions.contiguous(),
+                self.rope_cos if s.pos_type == "rope" else None, self.rope_sin,
+                slot_mapping, block_table.contiguous(), seq_lens)
+        if slot_mapping is None:
+            slot_mapping = ops.decode_slots(block_table, positions,
+                                            self.kv.block_size)
         return self._run_layers(hidden, positions, slot_mapping, attn)
 
     # --------------------------------------------------------- hybrid stacks

@@ -305,9 +305,10 @@ def decode_stack(x, layers, pages, n_heads: int, act: str, eps: float,
                  scale: float, positions, cos, sin, slot_mapping, block_table,
                  seq_lens, workgroups: int = 256):
     """Decoder layers of one token of each of x's rows [M, H], on the GPU:
-    q|k|v (rotated unless positions is None) with its page store, attention
-    against the pages, output, feed-forward. layers: their weights; pages: their
-    (keys, values). workgroups: fewer than 256 compute the same."""
+    q|k|v (rotated where positions and cos are given) with its page store,
+    attention against the pages, output, feed-forward. layers: their weights;
+    pages: their (keys, values); slot_mapping None: decode_slots'. workgroups:
+    fewer than 256 compute the same."""
     return require_hip().decode_stack(
         x, [[w.wqkv, w.wo, w.w_gate_up, w.w_down, w.wqkv_bias, w.wo_bias,
              w.w_gate_up_bias, w.w_down_bias, w.attn_norm, w.mlp_norm,

@@ -38,10 +38,10 @@ struct StackHead {
     const unsigned short* x;        // [M, H] bf16: the first layer's input
     float* x32;                     // [M, H]: the residual between
     unsigned* out;                  // [M, H] bf16: the last layer's result
-    const int* pos;                 // null: no rotation
-    const float* cos_t;             // [max_len, hd / 2]
+    const int* pos;
+    const float* cos_t;             // [max_len, hd / 2]; null: no rotation
     const float* sin_t;
-    const int* slots;
+    const int* slots;               // null: where the table has the positions
     const int* table;               // [M, W]
     const int* seq_lens;
 };

@@ -98,7 +98,11 @@ DEV_INLINE bool ds_again(bool there, int& spins) {
     return true;
 }
 // Until the word at p is there: one request a wave, where all the words that it
-// will read would be asked for in vain (a hop takes 2.1 us then, not 1.8).
+// will read would be asked for in vain. Where those are few, asking for them all
+// saves the second request: up to 768 bytes of a wave's input (DS_FEW steps) a
+// layer of 768 columns takes 25.0 us and not 25.9, of 2048 34.9 and 35.4, but of
+// 4096, at up to 1 KB, 83.5 and 82.7.
+constexpr int DS_FEW = 6;
 DEV_INLINE void ds_until(const unsigned* p) {
     int spins = 0;
     while (ds_again(__hip_atomic_load(p, __ATOMIC_RELAXED,
@@ -251,7 +255,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             told + offsetof(StackArgs, layer))[i];
     int lo = args.lo, hi = args.hi, M = args.M;
     float* const turns = reinterpret_cast<float*>(area + args.turns);
-    const bool rope = args.pos != nullptr;
+    const bool rope = args.cos_t != nullptr;
     int* const pages = reinterpret_cast<int*>(area + args.pages);
     const bool paged = args.area;
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(kw), "+s"(lo), "+s"(hi), "+s"(M)
@@ -319,9 +323,17 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         // have them with their next barrier.
         int slot = 0, len = 0, position = 0;
         if (lane < M) {
-            slot = DS_PTR(slots)[lane];
+            const int *slots = DS_PTR(slots), *pos = DS_PTR(pos);
+            const int W = DS_INT(W), bs = DS_INT(bs);
+            if (pos) position = pos[lane];
             len = DS_PTR(seq_lens)[lane];
-            if (rope) position = DS_PTR(pos)[lane];
+            if (slots)
+                slot = slots[lane];
+            else
+                slot = position < 0 || position / bs >= W
+                           ? -1             // (no such position)
+                           : DS_PTR(table)[lane * W + position / bs] * bs +
+                                 position % bs;
         }
         const bool own = claim(mine);
         if (lane < M) {
@@ -363,7 +375,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     }
                 }
                 const float* q = squares + row * Q;
-                if (l || k)
+                if ((l || k) && Q > 256)
                     ds_until(reinterpret_cast<const unsigned*>(q) + Q - 1);
                 for (int i0 = 0; i0 < Q && (l || k); i0 += 1024) {
                     unsigned long v[8];
@@ -760,7 +772,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             unsigned long v[DS_ROWS];
             bool ok;
             int spins = 0;
-            if (!raw && n > 0) ds_until(from - col + (M - 1) * H + s0 * 64 +
+            if (!raw && n > 0 && M > 2) ds_until(from - col + (M - 1) * H + s0 * 64 +
                                         n * 64 - 1);
             do {
                 ok = true;
@@ -831,7 +843,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             const int last = n * 128 - 8;
             int i = 0;
             unsigned out = 0, in = 0;          // of a load's part of a row
-            if (!raw)
+            if (!raw && M * n > DS_FEW)
                 ds_until(reinterpret_cast<const unsigned*>(
                     x + (long)(M - 1) * K * 2 + n * 128 - 4));
             constexpr int B = 10;
@@ -1080,7 +1092,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             const unsigned* qw =
                 at(l, 0) + (((m * nq + kvh * G + min(li, G - 1)) << hd_log2) +
                             lg * 8) / 2;
-            ds_until(qw + HD / 2 - 4 - lg * 4);
             unsigned long q[KS][2];
             bool ok;
             int spins = 0;

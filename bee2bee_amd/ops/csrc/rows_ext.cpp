@@ -270,8 +270,8 @@ Tensor decode_stack(const Tensor& x,
                     const std::vector<std::vector<optional<Tensor>>>& layers,
                     int64_t nq, bool gelu, double eps, double scale,
                     const optional<Tensor>& pos, const optional<Tensor>& cos_t,
-                    const optional<Tensor>& sin_t, const Tensor& slots,
-                    const Tensor& table, const Tensor& seq_lens, int64_t wgs) {
+                    const optional<Tensor>& sin_t,
+                    const optional<Tensor>& slots, const Tensor& table, const Tensor& seq_lens, int64_t wgs) {
     const int L = layers.size();
     TORCH_CHECK(L >= 1 && layers[0].size() == 14);
     const Tensor xd = dense(x, "x");
@@ -304,11 +304,14 @@ Tensor decode_stack(const Tensor& x,
     a.eps = (float)eps;
     a.scale = (float)scale;
     a.all = L;
-    a.slots = ints(slots, M, "slots");
+    TORCH_CHECK(slots.has_value() || pos.has_value(), "slots or positions");
+    if (slots.has_value()) a.slots = ints(*slots, M, "slots");
     a.table = ints(table, (long)M * a.W, "table");
     a.seq_lens = ints(seq_lens, M, "seq_lens");
     if (pos.has_value()) {
         a.pos = ints(*pos, M, "positions");
+    }
+    if (pos.has_value() && cos_t.has_value()) {
         for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
             TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kFloat32 &&
                         t->is_contiguous() && t->size(1) == hd / 2);

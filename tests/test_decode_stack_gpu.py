@@ -242,6 +242,35 @@ def test_a_token_without_a_position():
             assert torch.equal(t, old)
 
 
+@pytest.mark.parametrize("kind", ["rmsnorm", "layernorm"])
+def test_slots_of_the_positions(kind):
+    """No slots: where the table has the positions, and nowhere behind its end or
+    before its start."""
+    spec = _spec(256, 4, 2, 64, 1024, kind)
+    step = _Step(spec, 2, [33, 1, 48, 300], 16, W=19)
+    step.pos[1], step.pos[2] = -1, 19 * 16
+    step.slots[1] = step.slots[2] = -1
+    step.cos, step.sin = reference.rope_tables(400, 64, 1e4, DEV)
+    step.rope, want = False, step.run() if kind == "layernorm" else None
+    pages = [[t.clone() for t in kv] for kv in step.pages]
+    cos = step.cos if kind == "rmsnorm" else None
+
+    def run(slots, pages):
+        return ops.decode_stack(
+            step.x, step.layers, pages, 4, step.act, 1e-5, 0.125,
+            step.pos.clamp(min=0) if slots is not None else step.pos, cos,
+            step.sin, slots, step.table, step.lens)
+
+    if want is None:
+        step.pos[1] = 19 * 16 + 5              # (rotated by a row of the table)
+        want = [[t.clone() for t in kv] for kv in step.pages]
+        want = run(step.slots, want), want
+    assert torch.equal(run(None, pages), want[0])
+    for kv, kv_want in zip(pages, want[1]):
+        for t, w in zip(kv, kv_want):
+            assert torch.equal(t, w)
+
+
 def test_refused():
     spec = _spec(256, 4, 2, 64, 1024, "rmsnorm")
     step = _Step(spec, 1, [5, 12], 16)
