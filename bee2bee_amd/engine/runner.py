@@ -92,6 +92,18 @@ class Runner:
 
         return dist.get_world_size(self.tp_group) == 1
 
+    def _few_on_rings(self, rows: int) -> bool:
+        """Steps of few rows that run like those of some tens: of wide stacks,
+        from where a row more costs more than the launches that it saves. Time of
+        a step of 8 layers, on rows_linear over on the rings:
+          hidden 3584  8 / 9 / 10 / 16 rows   1.00 / 1.03 / 1.06 / 1.10
+          4096         8 / 9 / 10 / 16        0.97 / 1.02 / 1.03 / 1.06
+          3072         8 / 11 / 13 / 16       0.98 / 0.99 / 1.01 / 1.03
+          2048         8 / 10 / 12 / 16       0.88 / 0.95 / 0.97 / 0.99"""
+        hidden = self.spec.hidden_size
+        return (self._mid_dims and hidden >= 3072
+                and rows > (8 if hidden > 3072 else 11))
+
     def _one_launch(self, x: torch.Tensor, positions, slot_mapping,
                     block_table, seq_lens) -> bool:
         """Decode steps whose layers are one launch (ops.decode_stack); a tensor-
@@ -597,11 +609,13 @@ class Runner:
     ) -> torch.Tensor:
         if self.layer_lo >= self.layer_hi:
             return hidden
-        if self._rows_dims and ops.few_rows(hidden):
+        few = self._rows_dims and ops.few_rows(hidden)
+        if few and not self._few_on_rings(hidden.shape[0]):
             return self._run_layers_rows(hidden, positions, slot_mapping,
                                          attn_fn, paged)
         s = self.spec
-        if self._mid_dims and (ops.mid_rows(hidden) or ops.deep_rows(hidden)
+        if self._mid_dims and (few or ops.mid_rows(hidden)
+                               or ops.deep_rows(hidden)
                                or ops.wide_rows(hidden)):
             return self._run_layers_mid(hidden, positions, slot_mapping,
                                         attn_fn)

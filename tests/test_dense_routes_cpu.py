@@ -92,6 +92,25 @@ def test_a_route_computes_what_the_plain_one_does(spec, route, monkeypatch):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("spec", [TINY, PRESETS["tiny-gpt2"]],
+                         ids=["swiglu", "gelu"])
+@torch.no_grad()
+def test_few_rows_on_the_rings(spec, monkeypatch):
+    W = _weights(spec)
+    want = _steps(spec, W)
+    taken = []
+    monkeypatch.setattr(ops, "few_rows", lambda x: True)
+    monkeypatch.setattr(Runner, "_few_on_rings", lambda self, rows: True)
+    op = ops.mid_linear
+    monkeypatch.setattr(ops, "mid_linear", lambda *a: (
+        taken.append(1), op(*a))[1])
+    got = _steps(spec, W)
+    assert len(taken) == 9 * spec.n_layers     # three steps of three
+    for a, b in zip(got, want):
+        # fp32 sums in another order
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
 # plans: left to the library, whole rows, 4 parts, rows past the last tile apart
 @pytest.mark.parametrize("plan", [0, 12, 36, 140])
 @pytest.mark.parametrize("spec", [TINY, PRESETS["tiny-gpt2"]],

@@ -154,6 +154,19 @@ def test_steps(spec, rows, kv_dtype):
         assert _rel(got, want) <= limit, (name, _rel(got, want))
 
 
+@pytest.mark.parametrize("hidden,rows,rings", [
+    (3072, 11, False), (3072, 12, True), (4096, 8, False), (4096, 9, True),
+    (4096, 16, True)])
+def test_few_rows_of_wide_stacks(hidden, rows, rings):
+    spec = ModelSpec(name="t-few", vocab_size=512, hidden_size=hidden,
+                     intermediate_size=1024, n_layers=2, n_heads=8,
+                     n_kv_heads=2, head_dim=64, max_seq_len=128)
+    side = _Side(spec, ModelWeights(spec, DEV, torch.bfloat16).random_init(
+        seed=3), DEV, torch.bfloat16, "native")
+    assert side.runner._few_on_rings(rows) == rings
+    test_steps(spec, rows, "native")
+
+
 def test_wide_specs_leave_products_to_the_library():
     """What WIDE above is for: each has one that is left, and one that is not."""
     from bee2bee_amd import ops
