@@ -111,18 +111,19 @@ class Runner:
         about 2 us a launch, is a layer's; what passes between its workgroups
         grows with the rows. Time of a step of 8 layers (of 6: 768 columns),
         launch by launch over one launch:
-          4096 columns, 1 / 2 rows   1.12 / 1.09
-          3584 columns, 1 / 2        1.09 / 1.07
-          3072 columns, 1 / 3 / 4    1.05 / 1.08 / 1.03
-          2048 columns, 1 / 3 / 4    1.14 / 1.06 / 1.00
-          768 columns, layer norm, 1 / 4 / 6   1.15 / 1.13 / 1.00"""
+          4096 columns, 1 / 2 rows       1.14 / 1.10
+          3584 columns, 1 / 2            1.10 / 1.08
+          3072 columns, 1 / 3 / 4        1.09 / 1.08 / 1.07
+          2048 columns, 1 / 3 / 4        1.15 / 1.12 / 1.11
+          768 columns, 1 / 4 / 6 / 8     1.03 / 1.02 / 1.01 / 1.00
+          768 columns, layer norm, 1 / 4 / 6 / 8   1.21 / 1.16 / 1.03 / 1.00"""
         s = self.spec
         return (x.is_cuda and self.decode_attn_fn is None and self._mid_dims
                 and ops.few_rows(x) and self.layer_lo < self.layer_hi
                 and (s.act_type == "gelu" or not s.mlp_bias)
                 and all(t is None or t.dtype is torch.int32 for t in (
                     positions, slot_mapping, block_table, seq_lens))
-                and x.shape[0] <= min(4, ops.stack_rows(s)))
+                and x.shape[0] <= min(6, ops.stack_rows(s)))
 
     @property
     def is_first_stage(self) -> bool:

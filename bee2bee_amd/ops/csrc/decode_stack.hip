@@ -364,42 +364,63 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 (k == DS_QKV ? at(l - 1, DS_INT(down)) : at(l, DS_INT(o))) +
                 M * H / 2);
             float scale = 1.f;
-            for (int row = 0; row < M; ++row) {
-                float sum = 0.f;
-                if (l == 0 && k == DS_QKV) {
+            auto keep = [&](int row, float sum) __attribute__((always_inline)) {
+                sum = ds_wave_sum(sum);
+                if (m == row) scale = rsqrtf(sum / (float)H + told_s.eps);
+            };
+            if (l == 0 && k == DS_QKV) {
+                for (int row = 0; row < M; ++row) {
+                    float sum = 0.f;
                     for (int i = lane * 8; i < H; i += 512) {
                         float v[8];
                         load_bf16x8(DS_PTR(x) + row * H + i, v);
 #pragma unroll
                         for (int e = 0; e < 8; ++e) sum = fmaf(v[e], v[e], sum);
                     }
+                    keep(row, sum);
                 }
-                const float* q = squares + row * Q;
-                if ((l || k) && Q > 256)
-                    ds_until(reinterpret_cast<const unsigned*>(q) + Q - 1);
-                for (int i0 = 0; i0 < Q && (l || k); i0 += 1024) {
-                    unsigned long v[8];
-                    bool ok;
-                    int spins = 0;
-                    do {
-                        ok = true;
-#pragma unroll
-                        for (int u = 0; u < 8; ++u)
-                            if (i0 + u * 128 < Q)
-                                v[u] = ds_load(q + min(i0 + u * 128 + lane * 2,
-                                                       Q - 2));
-#pragma unroll
-                        for (int u = 0; u < 8; ++u)
-                            if (i0 + u * 128 < Q) ok = ok && ds_there(v[u]);
-                    } while (ds_again(ok, spins));
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        if (i0 + u * 128 + lane * 2 < Q)
-                            sum += ds_low(v[u]) + ds_high(v[u]);
-                }
-                sum = ds_wave_sum(sum);
-                if (m == row) scale = rsqrtf(sum / (float)H + told_s.eps);
+                return scale;
             }
+            // 16 loads at a time: of U for 128 sums each, rows beside each other
+            // (one after the other, 4 rows of 768 columns take 2 us more a layer)
+            auto rows = [&](auto u) __attribute__((always_inline)) {
+                constexpr int U = decltype(u)::value, R = 16 / U;
+                for (int r0 = 0; r0 < M; r0 += R) {
+                    float sum[R] = {};
+                    for (int i0 = 0; i0 < Q; i0 += U * 128) {
+                        unsigned long v[R][U];
+                        bool ok;
+                        int spins = 0;
+                        do {
+                            ok = true;
+#pragma unroll
+                            for (int i = 0; i < R * U; ++i)
+                                if (r0 + i / U < M && i0 + i % U * 128 < Q)
+                                    v[i / U][i % U] = ds_load(
+                                        squares + (r0 + i / U) * Q +
+                                        min(i0 + i % U * 128 + lane * 2,
+                                            Q - 2));
+#pragma unroll
+                            for (int i = 0; i < R * U; ++i)
+                                if (r0 + i / U < M && i0 + i % U * 128 < Q)
+                                    ok = ok && ds_there(v[i / U][i % U]);
+                        } while (ds_again(ok, spins));
+#pragma unroll
+                        for (int i = 0; i < R * U; ++i)
+                            if (r0 + i / U < M &&
+                                i0 + i % U * 128 + lane * 2 < Q)
+                                sum[i / U] += ds_low(v[i / U][i % U]) +
+                                              ds_high(v[i / U][i % U]);
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (r0 + r < M) keep(r0 + r, sum[r]);
+                }
+            };
+            if (M * Q > 256)
+                ds_until(reinterpret_cast<const unsigned*>(squares) + M * Q - 1);
+            if (M > 2 && Q <= 256) rows(std::integral_constant<int, 2>());
+            else rows(std::integral_constant<int, 8>());
             return scale;
         };
         bool passed = false;
