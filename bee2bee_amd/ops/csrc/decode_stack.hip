@@ -1113,11 +1113,21 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             const unsigned* qw =
                 at(l, 0) + (((m * nq + kvh * G + min(li, G - 1)) << hd_log2) +
                             lg * 8) / 2;
-            unsigned long q[KS][2];
+            // (the step's own key and value beside them, for the wave that has
+            // their tile)
+            const int of = lane / (HD / 4) % 2, e2 = lane % (HD / 4) * 2;
+            const unsigned* own =
+                at(l, DS_INT(new_kv)) +
+                ((((m * 2 + of) * nkv + kvh) << hd_log2) / 2 + e2);
+            unsigned long q[KS][2], fresh_word = 0;
             bool ok;
             int spins = 0;
             do {
                 ok = true;
+                if (mine) {
+                    fresh_word = ds_load(own);
+                    ok = ds_there(fresh_word);
+                }
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -1126,6 +1136,10 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                         ok = ok && ds_there(q[ks][e]);
                     }
             } while (ds_again(ok, spins));
+            if (mine) {
+                *reinterpret_cast<unsigned long*>(&fresh_s[of][e2]) = fresh_word;
+                WAVE_LDS_SYNC();
+            }
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 bq[ks] = __builtin_bit_cast(
@@ -1160,21 +1174,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         for (; kb < s.to; kb += DS_STEP) {
             const bool more = kb + DS_STEP < s.to;
             const long base = more && whole ? page_row(kb + DS_STEP) : 0;
-            // the tile with the step's own key and value, which are words
+            // the tile with the step's own key and value
             const bool patch = mine && newest < kb + DS_KEYS;
-            if (patch) {
-                const int of = lane / (HD / 4), e = lane % (HD / 4) * 2;
-                const unsigned* p =
-                    at(l, DS_INT(new_kv)) +
-                    (((m * 2 + of) * nkv + kvh) << hd_log2) / 2 + e;
-                unsigned long v;
-                int spins = 0;
-                do v = of < 2 ? ds_load(p) : 0;
-                while (ds_again(ds_there(v), spins));
-                if (of < 2)
-                    *reinterpret_cast<unsigned long*>(&fresh_s[of][e]) = v;
-                WAVE_LDS_SYNC();
-            }
             // values to LDS, 16-byte pieces xor-ed by the key
             const int to = ds_own(v_to), from = ds_own(v_from);
 #pragma unroll
