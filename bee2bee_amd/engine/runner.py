@@ -283,8 +283,11 @@ class Runner:
     ) -> torch.Tensor:
         """Dense layers on some tens of rows and more: projections as parts over
         K, summed by the kernels that read them (ops.mid_shape, ops.wide_plan),
-        or activated where they are made (ops.mid_gated, ops.mid_gelu)."""
-        s, T = self.spec, x.shape[0]
+        or activated where they are made (ops.mid_gated, ops.mid_gelu). Up to
+        MID_MAX rows the residual stays in fp32 between the first layer's input
+        and the last one's result."""
+        s, T, dtype = self.spec, x.shape[0], x.dtype
+        between = torch.float32 if T <= ops.MID_MAX else None
         layers = self.weights.layers
         H, I = s.hidden_size, s.intermediate_size
         lw = layers[self.layer_lo]
@@ -303,8 +306,9 @@ class Runner:
         def add(part, bias, x, norm):
             """Residual add and the next norm of a product without its bias."""
             if part.dim() == 3:
-                return ops.add_norm_parts(part, bias, x,
-                                          norm and (*norm, s.rms_eps))
+                return ops.add_norm_parts(
+                    part, bias, x, norm and (*norm, s.rms_eps),
+                    between if norm else dtype)
             if norm is None:
                 return None, x + part
             return self._fused_add_norm(part, x, *norm)

@@ -461,12 +461,15 @@ def mid_rows_linear(x, w, bias=None, act=None):
     return reference.rows_linear(x, w, bias, act=act)
 
 
-def add_norm_parts(part, bias, resid, norm=None):
-    """-> (norm(resid + parts + bias) or None without a norm, that sum)."""
-    if _use_hip(resid):
+def add_norm_parts(part, bias, resid, norm=None, dtype=None):
+    """-> (norm(resid + parts + bias) or None without a norm, that sum in dtype,
+    resid's by default). bf16 or fp32."""
+    dtype = dtype or resid.dtype
+    if _use_hip(part):
         nw, nb, eps = norm or (None, None, 0.0)
-        return require_hip().add_norm_parts(part, bias, resid, nw, nb, eps)
-    return reference.add_norm_parts(part, bias, resid, norm)
+        return require_hip().add_norm_parts(part, bias, resid, nw, nb, eps,
+                                            dtype is torch.float32)
+    return reference.add_norm_parts(part, bias, resid, norm, dtype)
 
 
 def rope_store_qkv(qkv, bias, n_heads: int, positions, cos, sin, k_cache,

@@ -252,8 +252,10 @@ __global__ void kv_store_fp8_kernel(
 // or OCP fp8 bytes). A thread takes 8 coordinates of a head's first half and
 // their partners in the second. Bound by its bytes at thousands of tokens (8512
 // tokens of 28 + 2x4 heads of 128: 38 us with the bias; as an add, a rotation
-// of 2-byte accesses and a copy it was 44 + 64 + 12), by its launch at tens.
-template <typename CT>
+// of 2-byte accesses and a copy it was 44 + 64 + 12), by the latency of its parts
+// at tens: all of them (PARTS; 0: rows, -1: a number that is not known) are asked
+// for before the first is added, by a wave a workgroup.
+template <typename CT, int PARTS>
 __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     const float* __restrict__ part, int S, unsigned short* __restrict__ qkv,
     const unsigned short* __restrict__ bias, const int* __restrict__ pos,
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     CT* __restrict__ k_cache, CT* __restrict__ v_cache,
     const int* __restrict__ slots, long T, int nq, int nkv, int hd, int bs) {
     const int heads = nq + 2 * nkv, half = hd / 2, per = hd / 16;
-    const long idx = blockIdx.x * 256L + threadIdx.x;
+    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
     const int c = idx % per;
     const int h = idx / per % heads;
     const long t = idx / per / heads;
@@ -269,7 +271,26 @@ __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     const int N = heads * hd, d = c * 8, n = h * hd + d;
     unsigned short* row = qkv + t * N + n;
     float a[8], b[8];
-    if (S > 0) {
+    if constexpr (PARTS > 0) {
+        f32x4 u[PARTS][2], w[PARTS][2];
+#pragma unroll
+        for (int s = 0; s < PARTS; ++s)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const float* p = part + ((long)s * T + t) * N + n;
+                u[s][q] = reinterpret_cast<const f32x4*>(p)[q];
+                w[s][q] = reinterpret_cast<const f32x4*>(p + half)[q];
+            }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            a[e] = b[e] = 0.f;
+#pragma unroll
+            for (int s = 0; s < PARTS; ++s) {
+                a[e] += u[s][e / 4][e % 4];
+                b[e] += w[s][e / 4][e % 4];
+            }
+        }
+    } else if (PARTS < 0) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.f;
         for (int s = 0; s < S; ++s) {
@@ -516,13 +537,23 @@ int launch_qkv_rope_store(const float* part, int S, unsigned short* qkv,
     if (hd % 16) return 1;
     const long n = T * (nq + 2 * nkv) * (hd / 16);
     if (n == 0) return 0;
+    const int threads = n < 256 * 256 ? 64 : 256;
+#define RS_ONE(CT, P)                                                         \
+    hipLaunchKernelGGL((qkv_rope_store_kernel<CT, P>),                        \
+                       dim3((n + threads - 1) / threads), dim3(threads), 0,   \
+                       stream, part, S, qkv, bias, pos, cos_t, sin_t,         \
+                       (CT*)k_cache, (CT*)v_cache, slots, T, nq, nkv, hd, bs)
 #define RS_GO(CT)                                                             \
-    hipLaunchKernelGGL((qkv_rope_store_kernel<CT>), dim3((n + 255) / 256),        \
-                       dim3(256), 0, stream, part, S, qkv, bias, pos, cos_t,  \
-                       sin_t, (CT*)k_cache, (CT*)v_cache, slots, T, nq, nkv,  \
-                       hd, bs)
+    do {                                                                      \
+        if (S == 0) RS_ONE(CT, 0);                                            \
+        else if (S == 1) RS_ONE(CT, 1);                                       \
+        else if (S == 2) RS_ONE(CT, 2);                                       \
+        else if (S == 4) RS_ONE(CT, 4);                                       \
+        else RS_ONE(CT, -1);                                                  \
+    } while (0)
     if (fp8) RS_GO(unsigned char);
     else RS_GO(unsigned short);
+#undef RS_ONE
 #undef RS_GO
     return 0;
 }

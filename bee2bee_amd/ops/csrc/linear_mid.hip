@@ -454,53 +454,96 @@ extern "C" int launch_linear_mid(const unsigned short* x,
 }
 
 // ----------------------------------------------------------- add_norm_parts
-// resid_out = resid + sum of the parts [+ bias]; y = norm(resid_out) (RMS, or
-// layer norm with norm_b), both from the fp32 sum; y null: the sum only. One
-// workgroup a row; the row stays in registers between its two uses.
-constexpr int ANP_T = 256;
-template <int S>
-__global__ __launch_bounds__(ANP_T) void add_norm_parts_kernel(
+// sum = resid + the parts [+ bias], either in bf16 or fp32; y = norm(sum) (RMS, or
+// layer norm with norm_b), from the fp32 sum; y null: the sum only. One
+// workgroup of T threads a row, which stays in registers between its two uses; a
+// thread takes V columns at a time. Many rows are bound by their bytes; of few, a
+// row's workgroup by the latency of its parts, which come from other XCDs: 1024
+// threads that ask for all of them at once. Behind the product that makes them,
+// us, with 256 threads of 8 columns / as now: 8 parts of 24x4096 5.2 / 4.6, of
+// 80x4096 6.8 / 5.9, of 24x3072 4.8 / 3.9, 4 parts of 24x4096 4.0 / 3.5, of 57x2048
+// 3.4 / 3.3; 2 of 1536x4096 14.6 and with 1024 threads 15.9.
+constexpr int ANP_MOST = 8192;              // columns
+template <int V> DEV_INLINE void anp_load(const unsigned short* p, float* to) {
+    if constexpr (V == 8) {
+        load_bf16x8(p, to);
+    } else {
+        const uint2v u = *reinterpret_cast<const uint2v*>(p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            to[e] = bf2f((unsigned short)(u[e / 2] >> e % 2 * 16));
+    }
+}
+template <int V>
+DEV_INLINE void anp_store(unsigned short* p, const float* from) {
+    if constexpr (V == 8)
+        store_bf16x8(p, from);
+    else
+        *reinterpret_cast<uint2v*>(p) =
+            uint2v{f2bf(from[0]) | (unsigned)f2bf(from[1]) << 16,
+                   f2bf(from[2]) | (unsigned)f2bf(from[3]) << 16};
+}
+template <int S, int T, int V>
+__global__ __launch_bounds__(T) void add_norm_parts_kernel(
     const float* __restrict__ part, const unsigned short* __restrict__ bias,
-    const unsigned short* __restrict__ resid,
+    const void* __restrict__ resid, int resid32,
     const unsigned short* __restrict__ norm_w,
-    const unsigned short* __restrict__ norm_b,
-    unsigned short* __restrict__ resid_out, unsigned short* __restrict__ y,
-    int M, int H, float eps) {
-    constexpr int MAXC = 4;                 // chunks of 8 a thread holds
+    const unsigned short* __restrict__ norm_b, void* __restrict__ sum_out,
+    int sum32, unsigned short* __restrict__ y, int M, int H, float eps) {
+    constexpr int MAXC = ANP_MOST / (T * V);    // chunks of V a thread holds
     const long row = blockIdx.x;
-    float v[MAXC][8], sum = 0.f, sumsq = 0.f;
+    __attribute__((aligned(16))) float v[MAXC][V];
+    float sum = 0.f, sumsq = 0.f;
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
-        const int i = (c * ANP_T + threadIdx.x) * 8;
+        const int i = (c * T + threadIdx.x) * V;
         if (i >= H) break;
-        load_bf16x8(resid + row * H + i, v[c]);
-        if (bias) {
-            float b[8];
-            load_bf16x8(bias + i, b);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[c][e] += b[e];
-        }
         // all parts on their way before the first is added
-        f32x4 p[S][2];
+        f32x4 p[S][V / 4];
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
+            for (int q = 0; q < V / 4; ++q)
                 p[s][q] = reinterpret_cast<const f32x4*>(
                     part + ((long)s * M + row) * H + i)[q];
+        if (resid32) {
+#pragma unroll
+            for (int q = 0; q < V / 4; ++q)
+                *reinterpret_cast<f32x4*>(v[c] + q * 4) =
+                    reinterpret_cast<const f32x4*>(
+                        reinterpret_cast<const float*>(resid) + row * H + i)[q];
+        } else {
+            anp_load<V>(reinterpret_cast<const unsigned short*>(resid) +
+                            row * H + i, v[c]);
+        }
+        if (bias) {
+            float b[V];
+            anp_load<V>(bias + i, b);
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[c][e] += b[e];
+        }
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[c][e] += p[s][e / 4][e % 4];
-        store_bf16x8(resid_out + row * H + i, v[c]);
+            for (int e = 0; e < V; ++e) v[c][e] += p[s][e / 4][e % 4];
+        if (sum32) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+            for (int q = 0; q < V / 4; ++q)
+                reinterpret_cast<f32x4*>(reinterpret_cast<float*>(sum_out) +
+                                         row * H + i)[q] =
+                    *reinterpret_cast<const f32x4*>(v[c] + q * 4);
+        } else {
+            anp_store<V>(reinterpret_cast<unsigned short*>(sum_out) + row * H +
+                             i, v[c]);
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
             sum += v[c][e];
             sumsq += v[c][e] * v[c][e];
         }
     }
     if (!y) return;
-    __shared__ float red[ANP_T / WAVE][2];
+    __shared__ float red[T / WAVE][2];
     sum = wave_sum(sum);
     sumsq = wave_sum(sumsq);
     if (threadIdx.x % WAVE == 0) {
@@ -510,7 +553,7 @@ __global__ __launch_bounds__(ANP_T) void add_norm_parts_kernel(
     __syncthreads();
     sum = sumsq = 0.f;
 #pragma unroll
-    for (int w = 0; w < ANP_T / WAVE; ++w) {
+    for (int w = 0; w < T / WAVE; ++w) {
         sum += red[w][0];
         sumsq += red[w][1];
     }
@@ -518,34 +561,38 @@ __global__ __launch_bounds__(ANP_T) void add_norm_parts_kernel(
     const float inv = rsqrtf(sumsq / (float)H - mean * mean + eps);
 #pragma unroll
     for (int c = 0; c < MAXC; ++c) {
-        const int i = (c * ANP_T + threadIdx.x) * 8;
+        const int i = (c * T + threadIdx.x) * V;
         if (i >= H) break;
-        float w[8], o[8];
-        load_bf16x8(norm_w + i, w);
+        float w[V], o[V];
+        anp_load<V>(norm_w + i, w);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (v[c][e] - mean) * inv * w[e];
+        for (int e = 0; e < V; ++e) o[e] = (v[c][e] - mean) * inv * w[e];
         if (norm_b) {
-            float b[8];
-            load_bf16x8(norm_b + i, b);
+            float b[V];
+            anp_load<V>(norm_b + i, b);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] += b[e];
+            for (int e = 0; e < V; ++e) o[e] += b[e];
         }
-        store_bf16x8(y + row * H + i, o);
+        anp_store<V>(y + row * H + i, o);
     }
 }
 
 // H % 8 == 0, H <= 8192, S 1, 2, 4 or 8; nonzero otherwise
 extern "C" int launch_add_norm_parts(
-    const float* part, const unsigned short* bias, const unsigned short* resid,
-    const unsigned short* norm_w, const unsigned short* norm_b,
-    unsigned short* resid_out, unsigned short* y, int M, int H, int S,
-    float eps, hipStream_t stream) {
-    if (M < 1 || H % 8 || H > ANP_T * 32) return 1;
+    const float* part, const unsigned short* bias, const void* resid,
+    int resid32, const unsigned short* norm_w, const unsigned short* norm_b,
+    void* sum, int sum32, unsigned short* y, int M, int H, int S, float eps,
+    hipStream_t stream) {
+    if (M < 1 || H % 8 || H > ANP_MOST) return 1;
+#define ANP_ONE(SV, T, V)                                                     \
+    hipLaunchKernelGGL((add_norm_parts_kernel<SV, T, V>), dim3(M), dim3(T),   \
+                       0, stream, part, bias, resid, resid32, norm_w, norm_b, \
+                       sum, sum32, y, M, H, eps)
 #define ANP_GO(SV)                                                            \
     case SV:                                                                  \
-        hipLaunchKernelGGL((add_norm_parts_kernel<SV>), dim3(M), dim3(ANP_T), \
-                           0, stream, part, bias, resid, norm_w, norm_b,      \
-                           resid_out, y, M, H, eps);                          \
+        if (M > 256) ANP_ONE(SV, 256, 8);                                     \
+        else if (H > 2048) ANP_ONE(SV, 1024, 4);                              \
+        else ANP_ONE(SV, 512, 4);                                             \
         return 0
     switch (S) {
         ANP_GO(1);
@@ -553,6 +600,7 @@ extern "C" int launch_add_norm_parts(
         ANP_GO(4);
         ANP_GO(8);
     }
+#undef ANP_ONE
 #undef ANP_GO
     return 1;
 }

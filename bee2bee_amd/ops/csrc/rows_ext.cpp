@@ -32,9 +32,9 @@ extern "C" int launch_linear_wide(const unsigned short*, const unsigned short*,
                                   void*, int, int, int, int, int, int,
                                   hipStream_t);
 extern "C" int launch_add_norm_parts(
-    const float*, const unsigned short*, const unsigned short*,
-    const unsigned short*, const unsigned short*, unsigned short*,
-    unsigned short*, int, int, int, float, hipStream_t);
+    const float*, const unsigned short*, const void*, int,
+    const unsigned short*, const unsigned short*, void*, int, unsigned short*,
+    int, int, int, float, hipStream_t);
 extern "C" int launch_qkv_rope_store(
     const float*, int, unsigned short*, const unsigned short*, const int*,
     const float*, const float*, void*, void*, const int*, long, int, int, int,
@@ -271,7 +271,8 @@ Tensor decode_stack(const Tensor& x,
                     int64_t nq, bool gelu, double eps, double scale,
                     const optional<Tensor>& pos, const optional<Tensor>& cos_t,
                     const optional<Tensor>& sin_t,
-                    const optional<Tensor>& slots, const Tensor& table, const Tensor& seq_lens, int64_t wgs) {
+                    const optional<Tensor>& slots, const Tensor& table,
+                    const Tensor& seq_lens, int64_t wgs) {
     const int L = layers.size();
     TORCH_CHECK(L >= 1 && layers[0].size() == 14);
     const Tensor xd = dense(x, "x");
@@ -494,23 +495,26 @@ const float* parts(const Tensor& t, long M, long N) {
 }
 
 // -> norm(resid + sum of the parts + bias) (undefined without a norm), and
-// that sum in bf16
+// that sum in bf16 or fp32; resid is either
 std::vector<optional<Tensor>> add_norm_parts(
     const Tensor& part, const optional<Tensor>& bias, const Tensor& resid,
     const optional<Tensor>& norm_w, const optional<Tensor>& norm_b,
-    double eps) {
+    double eps, bool sum32) {
     TORCH_CHECK(resid.dim() == 2);
     TORCH_CHECK(norm_w.has_value() || !norm_b.has_value());
     const int M = resid.size(0), H = resid.size(1);
     TORCH_CHECK(M >= 1 && H % 8 == 0 && H <= 8192);
-    const Tensor r = dense(resid, "resid"), b = column(bias, H, "bias"),
+    const Tensor r = dense(resid, "resid", true), b = column(bias, H, "bias"),
                  nw = column(norm_w, H, "norm weight"),
                  nb = column(norm_b, H, "norm bias");
-    Tensor sum = torch::empty({M, H}, r.options()), y;
-    if (norm_w.has_value()) y = torch::empty({M, H}, r.options());
+    const auto bf16 = r.options().dtype(torch::kBFloat16);
+    Tensor sum = torch::empty({M, H}, sum32 ? r.options().dtype(torch::kFloat32)
+                                            : bf16), y;
+    if (norm_w.has_value()) y = torch::empty({M, H}, bf16);
     TORCH_CHECK(launch_add_norm_parts(
-                    parts(part, M, H), ptr(b), ptr(r), ptr(nw), ptr(nb),
-                    mut(sum), y.defined() ? mut(y) : nullptr, M, H,
+                    parts(part, M, H), ptr(b), r.data_ptr(), is_f32(r), ptr(nw),
+                    ptr(nb), sum.data_ptr(), sum32,
+                    y.defined() ? mut(y) : nullptr, M, H,
                     part.size(0), (float)eps, stream()) == 0);
     return {y.defined() ? optional<Tensor>(y) : optional<Tensor>(), sum};
 }

@@ -332,7 +332,7 @@ def mid_linear(x, w):
     return (x.float() @ w.float().t()).unsqueeze(0)
 
 
-def add_norm_parts(part, bias, resid, norm=None):
+def add_norm_parts(part, bias, resid, norm=None, dtype=None):
     y = resid.float() + part.sum(0)
     if bias is not None:
         y = y + bias.float()
@@ -340,8 +340,8 @@ def add_norm_parts(part, bias, resid, norm=None):
     if norm is not None:
         w, b, eps = norm
         normed = (rmsnorm(y, w, eps) if b is None
-                  else layernorm(y, w, b, eps)).to(resid.dtype)
-    return normed, y.to(resid.dtype)
+                  else layernorm(y, w, b, eps)).to(w.dtype)
+    return normed, y.to(dtype or resid.dtype)
 
 
 def rope_store_qkv(qkv, bias, n_heads, positions, cos, sin, k_cache, v_cache,

@@ -405,6 +405,27 @@ def test_add_norm_parts(S, M, H, kind):
                 + 1e-4).all()
 
 
+# (256 rows and more: another kernel; 2048 columns and more: another's threads)
+@pytest.mark.parametrize("S,M,H", [(2, 256, 2048), (8, 9, 2056), (4, 257, 4096),
+                                   (1, 300, 72)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_add_norm_parts_in_fp32(S, M, H, dtype):
+    """A residual in fp32, as fp32 or bf16: fp32 sums of S + 2 numbers."""
+    torch.manual_seed(S)
+    part, resid = (torch.randn(*s, M, H, device=DEV) for s in ((S,), ()))
+    norm = _norm("rms", H)
+    y, total = ops.add_norm_parts(part, _rand(H), resid, norm, dtype)
+    torch.manual_seed(S)
+    part, resid = (torch.randn(*s, M, H, device=DEV) for s in ((S,), ()))
+    norm = _norm("rms", H)
+    want_y, want = reference.add_norm_parts(part, _rand(H).float(), resid,
+                                            _f32(norm))
+    assert total.dtype is dtype and y.dtype is torch.bfloat16
+    step = 2 ** -8 if dtype is torch.bfloat16 else 0
+    assert ((total.float() - want).abs() <= step * want.abs() + 1e-5).all()
+    assert ((y.float() - want_y).abs() <= 2 ** -8 * want_y.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("parts", [0, 1, 4])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("T,nq,nkv,hd,rope,biased", [
