@@ -382,8 +382,7 @@ __global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
 // The splits' sums of one row: workgroup = (sequence and key head, row). A
 // chain of loads and nothing else, so each wave takes the at most 32 maxima
 // and sums in one load, a lane a split, and P splits are read at once, 4
-// coordinates a thread: every load is under way before the first is used, and
-// before the length that says which of them are. With
+// coordinates a thread: every load is under way before the first is used. With
 // a thread a coordinate and a loop over the splits 32 splits of 7 rows took
 // 10.8 us, 8 groups of them, and 4.7 now; 6.2 and 4.8 with 4 rows. Up to 4
 // splits take one wave a row (2 splits of 20 rows, 128 groups: 4.9, 5.6 with
@@ -396,28 +395,31 @@ __global__ __launch_bounds__(HD / 4 * P) void attn_stream_combine_kernel(
     int G, int pages, int Z, int even, int most, int max_rows) {
     constexpr int C = HD / 4;                  // threads of a split
     const int b = blockIdx.x / nkv, kvh = blockIdx.x % nkv;
-    const int row = blockIdx.y;
-    const long p0 = (long)blockIdx.x * Z * max_rows + row;
-    const int lane = threadIdx.x & 63, c = threadIdx.x % C;
-    const int z0 = threadIdx.x / C;            // 0 .. P - 1
-    // (also of splits that there are not: what they hold is not used)
-    f32x4 o[I];                                // P * I >= Z
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-        o[i] = *reinterpret_cast<const f32x4*>(
-            part_o + (p0 + (long)min(z0 + i * P, Z - 1) * max_rows) * HD + c * 4);
-    const float2 ml = *reinterpret_cast<const float2*>(
-        part_ml + (p0 + (long)min(lane, Z - 1) * max_rows) * 2);
     const int s0 = cu ? cu[b] : b;
+    const int row = blockIdx.y;
     if (row >= (cu ? cu[b + 1] - s0 : 1) * G) return;
     const int L = min(seq_lens[b], pages);
     const int per = split_keys(L, even, most);
     if (L <= per) return;                      // written by its workgroup
     const int nz = (L + per - 1) / per;
+    const long p0 = (long)blockIdx.x * Z * max_rows + row;
+    const int lane = threadIdx.x & 63, c = threadIdx.x % C;
+    const int z0 = threadIdx.x / C;            // 0 .. P - 1
+    f32x4 o[I];                                // P * I >= Z
 #pragma unroll
-    for (int i = 0; i < I; ++i)
-        if (z0 + i * P >= nz) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float m = lane < nz ? ml.x : -1e30f, l = lane < nz ? ml.y : 0.f;
+    for (int i = 0; i < I; ++i) {
+        o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (z0 + i * P < nz)
+            o[i] = *reinterpret_cast<const f32x4*>(
+                part_o + (p0 + (long)(z0 + i * P) * max_rows) * HD + c * 4);
+    }
+    float m = -1e30f, l = 0.f;
+    if (lane < nz) {
+        const float2 ml = *reinterpret_cast<const float2*>(
+            part_ml + (p0 + (long)lane * max_rows) * 2);
+        m = ml.x;
+        l = ml.y;
+    }
     const float M = wave_max(m);
     const float w = __builtin_amdgcn_exp2f(m - M);
     const float lsum = wave_sum(w * l);
