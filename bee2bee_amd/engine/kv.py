@@ -201,11 +201,11 @@ class PagedKV:
         """Grow a sequence to new_len tokens, allocating blocks as needed."""
         blocks = self._seq_blocks[seq_id]
         need = (new_len + self.block_size - 1) // self.block_size
+        if need - len(blocks) > len(self._free):      # (all of them or none)
+            raise RuntimeError(
+                f"KV pool exhausted ({self.n_blocks} blocks of {self.block_size})"
+            )
         while len(blocks) < need:
-            if not self._free:
-                raise RuntimeError(
-                    f"KV pool exhausted ({self.n_blocks} blocks of {self.block_size})"
-                )
             blocks.append(self._free.pop())
         self._seq_len[seq_id] = new_len
 
