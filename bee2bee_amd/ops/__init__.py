@@ -11,9 +11,10 @@ decode attention, MFMA flash prefill attention, SwiGLU, top-k gating, grouped
 expert GEMM, projections with what stands around them. Other projection GEMMs go
 through hipBLASLt via torch.nn.functional.linear.
 
-Which projections are whose is measured: up to 16 rows (`few_rows`; logits:
-`head_rows`) the kernels of linear_rows.hip, one launch for norm, product and
-what follows; 17 to 256 rows (`mid_rows`, `mid_shape`, `mid_gated`) linear_mid.hip,
+Which projections are whose is measured: decode steps of one to six rows are one
+launch of decode_stack.hip; else up to 16 rows (`few_rows`; logits: `head_rows`) the
+kernels of linear_rows.hip, one launch for norm, product and what follows; 17 to 256
+rows, of wide stacks fewer (`mid_rows`, `mid_shape`, `mid_gated`) linear_mid.hip,
 split over K or activated; more rows linear_wide.hip where `wide_plan` says so:
 all gated ones, and others where its times are below the library's. The grouped
 kernel
@@ -347,12 +348,12 @@ def mid_shape(rows: int, width: int, depth: int) -> bool:
     captured (six layers of 768, prompts of 140 / 200 / 256 tokens 490 / 685 / 685
     us, with the library's 770; captured, 332 / 355 / 358 and 329 / 347 / 345).
     Measured with the kernel that reads them
-    (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 16.9 (19.1)
-    / 26.1 (30.0) / 30.0 (30.4), 4096x14336 26.6 (32.8) / 35.3 (79) / 42.4
-    (59.6), 3584x18944 28.7 (112) / 39 (103) / 50 (127), 8192x8192 35.1 (34.6) /
-    44 (52.6) / 49 (57), 2048x2048 8.3 (10.9) / 12.0 (11.2) / 14.8 (12.2),
-    3072x2048 9.9 (15.0) / 14.7 (18.1) / 18.0 (16.6), 5120x3072 14.6 (16.4) /
-    22.5 (25.1) / 27.4 (24.1), 768x3072 7.7 (11.9) / 10.8 (10.4) / 12.8
+    (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 15.1 (19.1)
+    / 25.4 (30.0) / 31.0 (30.4), 4096x14336 26.2 (32.8) / 34.9 (79) / 43.1
+    (59.6), 3584x18944 28.9 (112) / 39.5 (103) / 49.7 (127), 8192x8192 34.5 (34.6)
+    / 41.2 (52.6) / 49.1 (57), 2048x2048 8.7 (10.9) / 12.3 (11.2) / 15.2 (12.2),
+    3072x2048 9.5 (15.0) / 14.6 (18.1) / 18.2 (16.6), 5120x3072 12.9 (16.4) /
+    21.8 (25.1) / 28.0 (24.1), 768x3072 7.8 (11.9) / 10.6 (10.4) / 13.0
     (11.3)."""
     if width * depth <= 4 << 20 and (rows <= 160 or 2 * depth >= 7 * width):
         return True

@@ -1,5 +1,5 @@
-// Projections of 17 to 256 rows, and of fewer the longest gated ones and most
-// output heads: x [M, K] times rows of w [N, K]. Three forms of result:
+// Projections of 17 to 256 rows, of wide stacks from 9 or 12 on, and of fewer the
+// longest gated ones and most output heads: x [M, K] times rows of w [N, K]. Three forms of result:
 //  parts   fp32 sums over S parts of K, left to the kernel that reads them
 //          anyway (qkv_rope_store, add_norm_parts): narrow projections, which
 //          would leave most of the chip idle unsplit;
@@ -30,11 +30,11 @@
 //
 // Measured with the kernel that reads them (us, 24 / 80 / 128 / 200 / 256 rows;
 // in brackets this file's form before, which took weights through registers):
-//   4096x14336 26.6 / 33.2 / 35.3 / 42.4 / 48.4 (30.1 / 36.1 / 43.9 / 56 / 64)
-//   4096x4096  13.7 / 16.9 / 19.7 / 23.7 / 25.1 (14.5 / 17.3 / 20.7 / 25.5 / 29)
-//   6144x4096  16.9 / 22.9 / 26.1 / 30.0 / 32.1 (19.5 / 24.0 / 29.1 / 36.5 / 41)
-//   3584x18944 28.7 / 35.4 / 39.0 / 50.2 / 56.6 (33.7 / 43.1 / 52.2 / 69 / 78)
-//   2048x8192  13.2 / 16.5 / 19.3 / 22.3 / 24.6 (14.4 / 17.1 / 20.3 / 25.5 / 29)
+//   4096x14336 26.2 / 31.9 / 34.9 / 43.1 / 49.1 (30.1 / 36.1 / 43.9 / 56 / 64)
+//   4096x4096  13.1 / 16.8 / 19.6 / 24.1 / 26.0 (14.5 / 17.3 / 20.7 / 25.5 / 29)
+//   6144x4096  15.1 / 21.5 / 25.4 / 31.0 / 33.6 (19.5 / 24.0 / 29.1 / 36.5 / 41)
+//   3584x18944 28.9 / 34.3 / 39.5 / 49.7 / 56.8 (33.7 / 43.1 / 52.2 / 69 / 78)
+//   2048x8192  13.2 / 16.8 / 19.4 / 22.4 / 25.0 (14.4 / 17.1 / 20.3 / 25.5 / 29)
 // The library's figures are at the rules in ops/__init__.py.
 #include "common.h"
 
