@@ -9,8 +9,8 @@
 // stack; weights depend on nothing, so the next product's are asked for under
 // the last steps of this one, and what crosses the chip between products are a
 // few KB of rows. A step with its logits, us, launch by launch / in one: 6 layers
-// of 768 columns, 300 keys 213 / 185; 8 of 2048, 1000 keys 414 / 370; 8 of 4096,
-// 3000 keys 926 / 834; 8 of 3584, two rows of 24000 keys 1059 / 1015.
+// of 768 columns, 300 keys 213 / 173; 8 of 2048, 1000 keys 413 / 361; 8 of 4096,
+// 3000 keys 925 / 827; 8 of 3584, two rows of 24000 keys 1057 / 1005.
 //  * Rows pass from workgroup to workgroup as words that say themselves whether
 //    they are there: buffers are filled with DS_EMPTY (a NaN) before, a word is
 //    stored once, and readers load it until it is something else. Every such
@@ -50,8 +50,11 @@ constexpr int DS_BATCH = 2;                    // steps that are read at once
 constexpr unsigned DS_EMPTY = 0xffffffffu;
 constexpr int DS_KEYS = 32;                    // of a wave's tile
 constexpr int DS_STEP = DS_WAVES * DS_KEYS;
-constexpr int DS_ALONE = 512;                  // keys that are not split
-constexpr int DS_LEAST = 128;                  // keys of a split
+// Keys that are not split, a tile of each wave (of 300 keys, a layer of 768 columns
+// 24.7 us split and 25.2 not, 400 of 4096 columns 81.7 and 84.0), and least keys of
+// a split (64: the same; 256: 1000 keys of 2048 columns 35.7 us, not 34.9).
+constexpr int DS_ALONE = 256;
+constexpr int DS_LEAST = 128;
 constexpr int DS_PART = 18;                    // words: 16 columns of a split's
                                                // result, its maximum and sum
 constexpr int DS_KEPT = 4;                     // octets of which much is in LDS
