@@ -9,8 +9,8 @@
 // stack; weights depend on nothing, so the next product's are asked for under
 // the last steps of this one, and what crosses the chip between products are a
 // few KB of rows. A step with its logits, us, launch by launch / in one: 6 layers
-// of 768 columns, 300 keys 213 / 173; 8 of 2048, 1000 keys 413 / 361; 8 of 4096,
-// 3000 keys 925 / 827; 8 of 3584, two rows of 24000 keys 1057 / 1005.
+// of 768 columns, 300 keys 213 / 171; 8 of 2048, 1000 keys 413 / 357; 8 of 4096,
+// 3000 keys 924 / 820; 8 of 3584, two rows of 24000 keys 1057 / 1003.
 //  * Rows pass from workgroup to workgroup as words that say themselves whether
 //    they are there: buffers are filled with DS_EMPTY (a NaN) before, a word is
 //    stored once, and readers load it until it is something else. Every such
@@ -46,7 +46,10 @@ typedef __attribute__((ext_vector_type(4))) unsigned int ds_raw;
 
 constexpr int DS_WAVES = 8;                    // that stream
 constexpr int DS_RING = 8;                     // weight loads under way in each
-constexpr int DS_BATCH = 2;                    // steps that are read at once
+// Steps that are read at once (1 / 2 / 3 / 4: us a layer of 768 columns 25.0 /
+// 24.6 / 24.2 / 24.2, of 2048 35.3 / 35.2 / 34.7 / 35.0, of 4096 83.6 / 82.2 / 81.7 /
+// 81.9)
+constexpr int DS_BATCH = 3;
 constexpr unsigned DS_EMPTY = 0xffffffffu;
 constexpr int DS_KEYS = 32;                    // of a wave's tile
 constexpr int DS_STEP = DS_WAVES * DS_KEYS;
