@@ -344,7 +344,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         const bool own = claim(mine);
         if (lane < M) {
             slot_s[lane] = slot;
-            len_s[lane] = min(len, DS_INT(W) * DS_INT(bs));
+            len_s[lane] = max(min(len, DS_INT(W) * DS_INT(bs)), 0);
         }
         if (paged)
             for (int i = lane; i < M * DS_INT(W); i += 64)
@@ -1333,7 +1333,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         const int nq = DS_INT(nq), G = DS_INT(G);
         const int m = it / nq, head = it % nq;
         const int nz = ds_span(ds_same(len_s[m]), DS_INT(Z), 0).splits();
-        if (nz == 1 || wid >= DT) return;
+        if (nz <= 1 || wid >= DT) return;      // (0: no keys, attention's zeros)
         constexpr int U = DS_SPLITS / 8;
         const int lane = ds_own(tid & 63);
         const int z0 = lane >> 3, c = lane & 7;

@@ -242,6 +242,23 @@ def test_a_token_without_a_position():
             assert torch.equal(t, old)
 
 
+@pytest.mark.parametrize("length", [0, -3])
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_a_row_without_keys(at, length):
+    """Beside contexts that are split: zeros from its attention, as the plain
+    route gives, and the other rows as they are beside a row with keys."""
+    spec = _spec(256, 4, 2, 64, 1024, "rmsnorm")
+    step = _Step(spec, 2, [1500, 48, 2000], 16)
+    beside = step.run()[0]
+    step.lens[at] = length
+    step.slots[at] = -1
+    got = step.run()[0]
+    others = [m for m in range(3) if m != at]
+    assert torch.equal(got[others], beside[others])
+    step.lens[at] = step.slots[at] = 0         # (page 0 is nobody's)
+    assert _rel(got, step.want()[0]) <= 0.015
+
+
 @pytest.mark.parametrize("kind", ["rmsnorm", "layernorm"])
 def test_slots_of_the_positions(kind):
     """No slots: where the table has the positions, and nowhere behind its end or
