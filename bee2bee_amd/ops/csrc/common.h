@@ -41,6 +41,12 @@ __device__ __forceinline__ void load_fp8x8(const unsigned char* p,
     out[4] = c.x; out[5] = c.y; out[6] = d.x; out[7] = d.y;
 }
 
+// The row of a rotation's tables of a position: of one that they do not have,
+// their first or last. Callers' positions are not looked at on the host.
+__device__ __forceinline__ long turn_row(int pos, int rows) {
+    return max(min(pos, rows - 1), 0);
+}
+
 // bf16 (as ushort bits) <-> float
 __device__ __forceinline__ float bf2f(unsigned short u) {
     union { unsigned int i; float f; } v;

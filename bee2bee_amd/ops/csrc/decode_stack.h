@@ -32,6 +32,7 @@ struct StackHead {
     // words that pass between workgroups: [layers] of `stride`, and in each
     int stride, new_kv, att, o, up, down;    // (queries at 0)
     int turns, pages, area;         // in LDS (launch_decode_stack)
+    int turn_rows;                  // of cos_t and sin_t
     unsigned* words;
     unsigned* parts;                // [M * nkv, Z, G, hd / 16, 18]
     unsigned* claims;               // [DS_CLAIMS]
@@ -39,7 +40,7 @@ struct StackHead {
     float* x32;                     // [M, H]: the residual between
     unsigned* out;                  // [M, H] bf16: the last layer's result
     const int* pos;
-    const float* cos_t;             // [max_len, hd / 2]; null: no rotation
+    const float* cos_t;             // [turn_rows, hd / 2]; null: no rotation
     const float* sin_t;
     const int* slots;               // null: where the table has the positions
     const int* table;               // [M, W]

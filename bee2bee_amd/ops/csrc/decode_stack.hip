@@ -352,7 +352,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         if (rope)
             for (int i = lane; i < M * (HD / 2); i += 64) {
                 const int row = i / (HD / 2), d = i % (HD / 2);
-                const long from = (long)__shfl(position, row) * (HD / 2) + d;
+                const long from = turn_row(__shfl(position, row),
+                                           DS_INT(turn_rows)) * (HD / 2) + d;
                 turns[row * HD + d] = DS_PTR(cos_t)[from];
                 turns[row * HD + HD / 2 + d] = DS_PTR(sin_t)[from];
             }

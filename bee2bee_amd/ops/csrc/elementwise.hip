@@ -161,8 +161,8 @@ __global__ void rope_kernel(
     unsigned short* __restrict__ q,  // [T, nq, hd], token stride sq
     unsigned short* __restrict__ k,  // [T, nkv, hd], token stride sk
     const int* __restrict__ pos,     // [T]
-    const float* __restrict__ cos_t, // [max_len, hd/2]
-    const float* __restrict__ sin_t,
+    const float* __restrict__ cos_t, // [table, hd/2]
+    const float* __restrict__ sin_t, int table,
     int T, int nq, int nkv, int hd, long sq, long sk) {
     const int glob_wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
     const int lane = threadIdx.x % WAVE;
@@ -173,7 +173,7 @@ __global__ void rope_kernel(
     unsigned short* base = (h < nq) ? q + (long)t * sq + (long)h * hd
                                     : k + (long)t * sk + (long)(h - nq) * hd;
     const int half = hd / 2;
-    const long tab = (long)pos[t] * half;
+    const long tab = turn_row(pos[t], table) * half;
     for (int d = lane; d < half; d += WAVE) {
         float c = cos_t[tab + d];
         float s = sin_t[tab + d];
@@ -259,7 +259,7 @@ template <typename CT, int PARTS>
 __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     const float* __restrict__ part, int S, unsigned short* __restrict__ qkv,
     const unsigned short* __restrict__ bias, const int* __restrict__ pos,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table,
     CT* __restrict__ k_cache, CT* __restrict__ v_cache,
     const int* __restrict__ slots, long T, int nq, int nkv, int hd, int bs) {
     const int heads = nq + 2 * nkv, half = hd / 2, per = hd / 16;
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256) void qkv_rope_store_kernel(
     }
     const bool turns = pos && h < nq + nkv;
     if (turns) {
-        const long tab = (long)pos[t] * half + d;
+        const long tab = turn_row(pos[t], table) * half + d;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const f32x4 cs = reinterpret_cast<const f32x4*>(cos_t + tab)[q];
@@ -483,12 +483,12 @@ void launch_fused_add_rmsnorm(const unsigned short* x,
 }
 
 void launch_rope(unsigned short* q, unsigned short* k, const int* pos,
-                 const float* cos_t, const float* sin_t, int T, int nq,
+                 const float* cos_t, const float* sin_t, int table, int T, int nq,
                  int nkv, int hd, long sq, long sk, hipStream_t stream) {
     const long waves = (long)T * (nq + nkv);
     const long blocks = (waves + 3) / 4;
     hipLaunchKernelGGL(rope_kernel, dim3(blocks), dim3(256), 0, stream, q, k,
-                       pos, cos_t, sin_t, T, nq, nkv, hd, sq, sk);
+                       pos, cos_t, sin_t, table, T, nq, nkv, hd, sq, sk);
 }
 
 void launch_kv_store(const unsigned short* k, const unsigned short* v,
@@ -531,8 +531,8 @@ void launch_embed_positions(const long* ids, const unsigned short* embed,
 // hd % 16 == 0; qkv, bias, tables and pools 16-byte aligned; nonzero otherwise
 int launch_qkv_rope_store(const float* part, int S, unsigned short* qkv,
                       const unsigned short* bias, const int* pos,
-                      const float* cos_t, const float* sin_t, void* k_cache,
-                      void* v_cache, const int* slots, long T, int nq, int nkv,
+                      const float* cos_t, const float* sin_t, int table,
+                      void* k_cache, void* v_cache, const int* slots, long T, int nq, int nkv,
                       int hd, int bs, int fp8, hipStream_t stream) {
     if (hd % 16) return 1;
     const long n = T * (nq + 2 * nkv) * (hd / 16);
@@ -541,7 +541,7 @@ int launch_qkv_rope_store(const float* part, int S, unsigned short* qkv,
 #define RS_ONE(CT, P)                                                         \
     hipLaunchKernelGGL((qkv_rope_store_kernel<CT, P>),                        \
                        dim3((n + threads - 1) / threads), dim3(threads), 0,   \
-                       stream, part, S, qkv, bias, pos, cos_t, sin_t,         \
+                       stream, part, S, qkv, bias, pos, cos_t, sin_t, table,  \
                        (CT*)k_cache, (CT*)v_cache, slots, T, nq, nkv, hd, bs)
 #define RS_GO(CT)                                                             \
     do {                                                                      \

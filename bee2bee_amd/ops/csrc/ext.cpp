@@ -6,6 +6,7 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime.h>
+#include <algorithm>
 
 using torch::Tensor;
 
@@ -24,7 +25,8 @@ void launch_fused_add_layernorm(const unsigned short*, const unsigned short*,
                                 float, hipStream_t);
 void launch_gelu(const unsigned short*, unsigned short*, long, hipStream_t);
 void launch_rope(unsigned short*, unsigned short*, const int*, const float*,
-                 const float*, int, int, int, int, long, long, hipStream_t);
+                 const float*, int, int, int, int, int, long, long,
+                 hipStream_t);
 void launch_kv_store(const unsigned short*, const unsigned short*,
                      unsigned short*, unsigned short*, const int*, int, int,
                      int, int, long, long, hipStream_t);
@@ -132,10 +134,12 @@ void rope_inplace(Tensor& q, Tensor& k, const Tensor& pos, const Tensor& cos_t,
     TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == hd);
     TORCH_CHECK(k.stride(2) == 1 && k.stride(1) == hd);
     TORCH_CHECK(cos_t.size(1) == hd / 2 && cos_t.is_contiguous() &&
-                sin_t.is_contiguous());
+                sin_t.is_contiguous() && sin_t.size(1) == hd / 2);
+    const int table = (int)std::min(cos_t.size(0), sin_t.size(0));
+    TORCH_CHECK(table >= 1);
     launch_rope(bf16p_mut(q), bf16p_mut(k), pos.data_ptr<int>(),
-                cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), T, nq, nkv,
-                hd, q.stride(0), k.stride(0), stream());
+                cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), table, T, nq,
+                nkv, hd, q.stride(0), k.stride(0), stream());
 }
 
 void kv_cache_store(const Tensor& k, const Tensor& v, Tensor& k_cache,

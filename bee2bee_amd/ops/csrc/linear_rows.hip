@@ -60,8 +60,9 @@ enum { LR_NONE = 0, LR_RMS = 1, LR_LAYER = 2, LR_SCALED = 3 };
 // into q [M, nq, hd]; keys rotated, and values, into the pages (bf16 or fp8).
 struct QkvStore {
     const int* pos;           // null: no rotation
-    const float* cos_t;       // [max_len, hd / 2]
+    const float* cos_t;       // [table, hd / 2]
     const float* sin_t;
+    int table;
     const int* slots;
     void* k_cache;            // [nb, nkv, bs, hd]
     void* v_cache;
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(NW * 64) void linear_rows_kernel(
         }
         const int head = n / st.hd, d = n % st.hd;
         if (st.pos && head < st.nq + st.nkv) {
-            const long tab = (long)st.pos[m] * half + d;
+            const long tab = turn_row(st.pos[m], st.table) * half + d;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float c = st.cos_t[tab + r], sn = st.sin_t[tab + r];
@@ -493,8 +494,8 @@ extern "C" int launch_linear_rows(
     int resid32, void* y, int y32, const unsigned short* then_w,
     unsigned short* scaled, float* squares_out, int M, int N, int K,
     float eps, int norm, int epi,
-    const int* pos, const float* cos_t, const float* sin_t, const int* slots,
-    void* k_cache, void* v_cache, int nq, int nkv, int hd, int bs, int fp8,
+    const int* pos, const float* cos_t, const float* sin_t, int table,
+    const int* slots, void* k_cache, void* v_cache, int nq, int nkv, int hd, int bs, int fp8,
     hipStream_t stream) {
     if (M < 1 || M > 16 || N < 1 || K < 32 || K % 32) return 1;
     if (epi == LR_GLU && N % 16) return 1;
@@ -503,8 +504,8 @@ extern "C" int launch_linear_rows(
     if (then_w && N % 8) return 1;
     const Sum add{resid, resid32, y32, then_w, scaled, squares_out};
     if (epi == LR_QKV && (hd % 32 || N != (nq + 2 * nkv) * hd)) return 1;
-    const QkvStore st{pos,     cos_t, sin_t, slots, k_cache,
-                      v_cache, nq,    nkv,   hd,    bs, fp8};
+    const QkvStore st{pos,     cos_t, sin_t, table, slots, k_cache,
+                      v_cache, nq,    nkv,   hd,    bs,    fp8};
     // (see above: stacks of more than 768)
     const int WN = epi == LR_GLU ? 2 * N : N;
     const bool streamed = (WN < K ? WN : K) > 768 || (WN < K ? K : WN) > 4096;

@@ -15,8 +15,8 @@ extern "C" int launch_linear_rows(
     const void*, int, const unsigned short*, const unsigned short*,
     const unsigned short*, const unsigned short*, const float*, const void*,
     int, void*, int, const unsigned short*, unsigned short*, float*, int, int,
-    int, float, int, int, const int*, const float*, const float*, const int*,
-    void*, void*, int, int, int, int, int, hipStream_t);
+    int, float, int, int, const int*, const float*, const float*, int,
+    const int*, void*, void*, int, int, int, int, int, hipStream_t);
 extern "C" int decode_stack_rows(int, int);
 extern "C" int decode_stack_splits(long, long);
 extern "C" int launch_decode_stack(const StackArgs*, int, int, int, int,
@@ -37,8 +37,8 @@ extern "C" int launch_add_norm_parts(
     int, int, int, float, hipStream_t);
 extern "C" int launch_qkv_rope_store(
     const float*, int, unsigned short*, const unsigned short*, const int*,
-    const float*, const float*, void*, void*, const int*, long, int, int, int,
-    int, int, hipStream_t);
+    const float*, const float*, int, void*, void*, const int*, long, int, int,
+    int, int, int, hipStream_t);
 
 extern "C" void launch_decode_slots(const int*, const int*, int*, int, int,
                                     long, int, hipStream_t);
@@ -84,6 +84,23 @@ const unsigned short* ptr(const Tensor& t) {
 
 unsigned short* mut(Tensor& t) {
     return reinterpret_cast<unsigned short*>(t.data_ptr());
+}
+
+// The rotation's tables as kernels read them, [rows, hd / 2] each.
+struct Turns {
+    const float *cos_t = nullptr, *sin_t = nullptr;
+    int rows = 0;
+};
+Turns turns(const optional<Tensor>& cos_t, const optional<Tensor>& sin_t,
+            long hd) {
+    const Tensor &c = cos_t.value(), &s = sin_t.value();
+    for (const Tensor* t : {&c, &s})
+        TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kFloat32 &&
+                    t->is_contiguous() && t->dim() == 2 && t->size(0) >= 1 &&
+                    t->size(1) == hd / 2,
+                    "rotation tables [rows, head size / 2] fp32");
+    return {c.data_ptr<float>(), s.data_ptr<float>(),
+            (int)std::min(c.size(0), s.size(0))};
 }
 
 struct Rows {
@@ -181,8 +198,8 @@ Tensor rows_product(const Tensor& x, const Tensor& w,
                     ptr(tw), tw.defined() ? mut(scaled) : nullptr,
                     tw.defined() ? squares_out.data_ptr<float>() : nullptr,
                     r.M, N, r.K, (float)eps, r.norm, (int)act, nullptr,
-                    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0,
-                    0, stream()) == 0);
+                    nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0, 0, 0,
+                    0, 0, stream()) == 0);
     return y;
 }
 
@@ -228,12 +245,11 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
     TORCH_CHECK(hd % 32 == 0 && r.N == (nq + 2 * nkv) * hd);
     TORCH_CHECK(slots.scalar_type() == torch::kInt32 &&
                 slots.is_contiguous() && slots.numel() == r.M);
+    Turns by;
     if (pos.has_value()) {
         TORCH_CHECK(pos->scalar_type() == torch::kInt32 &&
                     pos->is_contiguous() && pos->numel() == r.M);
-        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
-            TORCH_CHECK(t->scalar_type() == torch::kFloat32 &&
-                        t->is_contiguous() && t->size(1) == hd / 2);
+        by = turns(cos_t, sin_t, hd);
     }
     const Tensor b = column(bias, r.N, "bias");
     Tensor q = torch::empty({r.M, nq, hd}, r.w.options());
@@ -243,8 +259,7 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
                     q.data_ptr(), 0, nullptr, nullptr, nullptr, r.M, r.N, r.K,
                     (float)eps, r.norm, EPI_QKV,
                     pos.has_value() ? pos->data_ptr<int>() : nullptr,
-                    pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
-                    pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
+                    by.cos_t, by.sin_t, by.rows,
                     slots.data_ptr<int>(), k_cache.data_ptr(),
                     v_cache.data_ptr(), nq, nkv, hd, bs, fp8, stream()) == 0);
     return q;
@@ -313,11 +328,10 @@ Tensor decode_stack(const Tensor& x,
         a.pos = ints(*pos, M, "positions");
     }
     if (pos.has_value() && cos_t.has_value()) {
-        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
-            TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kFloat32 &&
-                        t->is_contiguous() && t->size(1) == hd / 2);
-        a.cos_t = cos_t->data_ptr<float>();
-        a.sin_t = sin_t->data_ptr<float>();
+        const Turns by = turns(cos_t, sin_t, hd);
+        a.cos_t = by.cos_t;
+        a.sin_t = by.sin_t;
+        a.turn_rows = by.rows;
     }
     const int up = gelu ? I : 2 * I;
     const int K[4] = {H, Q, H, I}, rows[4] = {N, H, up, H};
@@ -538,12 +552,11 @@ Tensor rope_store_qkv(const Tensor& qkv, const optional<Tensor>& bias,
     TORCH_CHECK(hd % 16 == 0 && N == (nq + 2 * nkv) * hd);
     TORCH_CHECK(slots.scalar_type() == torch::kInt32 &&
                 slots.is_contiguous() && slots.numel() == T);
+    Turns by;
     if (pos.has_value()) {
         TORCH_CHECK(pos->scalar_type() == torch::kInt32 &&
                     pos->is_contiguous() && pos->numel() == T);
-        for (const Tensor* t : {&cos_t.value(), &sin_t.value()})
-            TORCH_CHECK(t->scalar_type() == torch::kFloat32 &&
-                        t->is_contiguous() && t->size(1) == hd / 2);
+        by = turns(cos_t, sin_t, hd);
     }
     const Tensor b = column(bias, N, "bias");
     const float* p = split ? parts(qkv, T, N) : nullptr;
@@ -553,8 +566,7 @@ Tensor rope_store_qkv(const Tensor& qkv, const optional<Tensor>& bias,
     TORCH_CHECK(launch_qkv_rope_store(
                     p, split ? qkv.size(0) : 0, mut(out), ptr(b),
                     pos.has_value() ? pos->data_ptr<int>() : nullptr,
-                    pos.has_value() ? cos_t->data_ptr<float>() : nullptr,
-                    pos.has_value() ? sin_t->data_ptr<float>() : nullptr,
+                    by.cos_t, by.sin_t, by.rows,
                     k_cache.data_ptr(), v_cache.data_ptr(),
                     slots.data_ptr<int>(), T, nq, nkv, hd, bs, fp8,
                     stream()) == 0);

@@ -5,6 +5,8 @@ Tolerance: the normed input and the output are rounded to bf16 once each (2^-8
 relative at most): an element is off by at most 2^-8 of the sum of its
 products' magnitudes, carried through the activation (whose slope is below
 1.13), and 2^-8 of itself."""
+import types
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -540,3 +542,47 @@ def test_ids_and_positions_that_the_tables_do_not_have():
     assert torch.equal(ops.attn_decode(q, kc, vc, table, past, 0.1),
                        ops.attn_decode(q, kc, vc, table, past.clamp(max=32),
                                        0.1))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_positions_that_the_rotation_has_not(hd):
+    """Its first row for positions before the tables, its last for those behind
+    them, in every kernel that rotates."""
+    M, nq, nkv, K, rows = 6, 4, 2, 256, 40
+    torch.manual_seed(hd)
+    N = (nq + 2 * nkv) * hd
+    x, w, norm = _rand(M, K), _rand(N, K, std=0.1), _norm("rms", K)
+    qkv = _rand(M, N)
+    cos, sin = (t[:rows] for t in reference.rope_tables(rows + 24, hd, 1e4, DEV))
+    pos = torch.tensor([-1, 39, 40, 63, -2 ** 31, 2 ** 31 - 1],
+                       dtype=torch.int32, device=DEV)
+    table = torch.arange(M, dtype=torch.int32, device=DEV).view(M, 1)
+    slots = table.view(-1) * 16
+    wo, up, down = (_rand(*s, std=0.1) for s in ((K, nq * hd), (1024, K),
+                                                 (K, 512)))
+    layer = types.SimpleNamespace(
+        wqkv=w, wo=wo, w_gate_up=up, w_down=down, attn_norm=norm[0],
+        mlp_norm=norm[0], **{n + "_bias": None for n in (
+            "wqkv", "wo", "w_gate_up", "w_down", "attn_norm", "mlp_norm")})
+
+    def inplace(pos, k, v):
+        y = qkv.clone().view(M, -1, hd)
+        ops.rope_inplace(y[:, :nq], y[:, nq : nq + nkv], pos, cos, sin)
+        return y
+
+    for op in (
+            lambda p, k, v: ops.rows_qkv(x, w, None, norm, nq, p, cos, sin, k,
+                                         v, slots),
+            lambda p, k, v: ops.rope_store_qkv(qkv.clone(), None, nq, p, cos,
+                                               sin, k, v, slots),
+            inplace,
+            lambda p, k, v: ops.decode_stack(
+                x, [layer], [(k, v)], nq, "swiglu", 1e-5, 0.125, p, cos, sin,
+                slots, table, torch.ones_like(slots))):
+        results = []
+        for p in (pos, pos.clamp(0, rows - 1)):
+            pages = [torch.zeros(M, nkv, 16, hd, device=DEV,
+                                 dtype=torch.bfloat16) for _ in range(2)]
+            results.append([op(p, *pages), *pages])
+        for a, b in zip(*results):
+            assert torch.equal(a, b)
