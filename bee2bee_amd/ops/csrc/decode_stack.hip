@@ -28,8 +28,9 @@
 //  * Attention is attn_stream.hip's tile of 32 keys a wave, eight waves a
 //    workgroup, with keys straight into the operand's registers. Contexts of up
 //    to DS_ALONE keys take one workgroup a key head; longer ones are split, and
-//    waves of their own add the splits up. The step's own key and value are
-//    taken from the words, not from the page that they are stored to.
+//    waves of their own add the splits up. The step's own keys and values, of
+//    all rows whose pages a context has, are taken from the words, not from
+//    the pages that they are stored to meanwhile.
 //  * Number c's octets of a product are c, c + DS_WGS and so on. Nothing has to
 //    be resident together for that: a workgroup claims its number when it
 //    starts, and after the first product each one sees that all numbers are
@@ -239,7 +240,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     __shared__ unsigned operands[DS_KEPT][2][64];
     __shared__ float residual[DS_KEPT][64];
     __shared__ int slot_s[DS_ROWS], len_s[DS_ROWS];
-    __shared__ __attribute__((aligned(16))) unsigned fresh_s[2][HD / 2];
+    __shared__ int own_s[DS_ROWS];             // attention: keys of this step
     __shared__ int ncols, begin, gate;
     constexpr int LW = sizeof(StackLayer) / 4;
     __shared__ __attribute__((aligned(16))) int layers[(DS_LAYERS + 1) * LW];
@@ -261,6 +262,11 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             told + offsetof(StackArgs, layer))[i];
     int lo = args.lo, hi = args.hi, M = args.M;
     float* const turns = reinterpret_cast<float*>(area + args.turns);
+    // the step's own keys and values: [row][2][HD / 2]
+    auto fresh_at = [&](int n, int of) __attribute__((always_inline)) {
+        return reinterpret_cast<unsigned*>(turns) + M * HD +
+               (n * 2 + of) * (HD / 2);
+    };
     const bool rope = args.cos_t != nullptr;
     int* const pages = reinterpret_cast<int*>(area + args.pages);
     const bool paged = args.area;
@@ -1010,7 +1016,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     // (of the first item, the only one where there are no more than workgroups:
     // the same in every layer)
     int i_at = -1, i_m = 0, i_kvh = 0, i_z = 0;
-    bool i_fresh = false;
+    unsigned i_mine = 0;
     long i_base = 0;
     auto attention = [&](int l, int it) __attribute__((always_inline)) {
         const int bs = DS_INT(bs);
@@ -1020,13 +1026,31 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             i_m = it / DS_INT(Z) / DS_INT(nkv);
             i_kvh = it / DS_INT(Z) % DS_INT(nkv);
             const Span s = ds_span(ds_same(len_s[i_m]), DS_INT(Z), i_z);
-            const int newest = s.len - 1, kb = s.from + wid * DS_KEYS;
+            const int kb = s.from + wid * DS_KEYS;
             if (!s.none(i_z)) {
-                // the step's own key, unless it is stored elsewhere
-                i_fresh = s.to == s.len &&
-                          ds_same(slot_s[i_m]) ==
-                              ds_same(page_of(i_m, newest / bs)) * bs +
-                                  newest % bs;
+                // Which of its keys the step's rows store, -1: none; all waves
+                // find the same. (Slots that several rows store to are this
+                // row's, if it is one of them.)
+                int own = -1;
+                for (int p0 = s.from / bs; p0 * bs < s.to; p0 += 64) {
+                    const int p = p0 + lane;
+                    const int page = p * bs < s.to ? page_of(i_m, p) : -1;
+                    for (int n = 0; n < M; ++n) {
+                        const int slot = ds_same(slot_s[n]);
+                        const int key = p * bs + slot % bs;
+                        const unsigned long hit = __ballot(
+                            slot >= 0 && page == slot / bs && key >= s.from &&
+                            key < s.to);
+                        if (hit && lane == n)
+                            own = (p0 + __builtin_ctzl(hit)) * bs + slot % bs;
+                    }
+                }
+                if (lane != i_m && own == __builtin_amdgcn_readlane(own, i_m))
+                    own = -1;
+                if (lane < M) own_s[lane] = own;
+                // (of these, the ones in this wave's tiles)
+                i_mine = __ballot(own >= kb &&
+                                  (unsigned)(own - kb) % DS_STEP < DS_KEYS);
                 if (whole && kb < s.to)        // the first tile's
                     i_base = (((long)ds_same(page_of(i_m, kb / bs)) *
                                    DS_INT(nkv) + i_kvh) * bs + kb % bs) * HD;
@@ -1036,8 +1060,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         const Span s = ds_span(ds_same(len_s[m]), DS_INT(Z), i_z);
         if (s.none(i_z)) return;
         const int G = DS_INT(G), nq = DS_INT(nq), nkv = DS_INT(nkv);
-        const int newest = s.len - 1;
-        const bool fresh = i_fresh;
         const char* kc = pointer(l, 12);
         const char* vc = pointer(l, 13);
         auto v_swz = [](int row) {
@@ -1114,25 +1136,28 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 
         // queries
         bf16x8 bq[KS];
-        const bool mine = fresh && newest >= kb && (newest - kb) % DS_STEP <
-                                                       DS_KEYS;
+        const unsigned mine = i_mine;          // rows
+        int own = -1;                          // their keys
         if (kb < s.to) {                       // (others have nothing to ask)
             const unsigned* qw =
                 at(l, 0) + (((m * nq + kvh * G + min(li, G - 1)) << hd_log2) +
                             lg * 8) / 2;
             // (the step's own key and value beside them, for the wave that has
-            // their tile)
+            // their tile; of more rows than one after that)
             const int of = lane / (HD / 4) % 2, e2 = lane % (HD / 4) * 2;
-            const unsigned* own =
-                at(l, DS_INT(new_kv)) +
-                ((((m * 2 + of) * nkv + kvh) << hd_log2) / 2 + e2);
+            auto fresh_of = [&](int n) __attribute__((always_inline)) {
+                return at(l, DS_INT(new_kv)) +
+                       ((((n * 2 + of) * nkv + kvh) << hd_log2) / 2 + e2);
+            };
+            const int first = mine ? __builtin_ctz(mine) : 0;
+            const unsigned* from = fresh_of(first);
             unsigned long q[KS][2], fresh_word = 0;
             bool ok;
             int spins = 0;
             do {
                 ok = true;
                 if (mine) {
-                    fresh_word = ds_load(own);
+                    fresh_word = ds_load(from);
                     ok = ds_there(fresh_word);
                 }
 #pragma unroll
@@ -1144,7 +1169,18 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     }
             } while (ds_again(ok, spins));
             if (mine) {
-                *reinterpret_cast<unsigned long*>(&fresh_s[of][e2]) = fresh_word;
+                if (lane < M) own = own_s[lane];
+                *reinterpret_cast<unsigned long*>(fresh_at(first, of) + e2) =
+                    fresh_word;
+#pragma unroll 1
+                for (unsigned b = mine & (mine - 1); b; b &= b - 1) {
+                    const int n = __builtin_ctz(b);
+                    spins = 0;
+                    do fresh_word = ds_load(fresh_of(n));
+                    while (ds_again(ds_there(fresh_word), spins));
+                    *reinterpret_cast<unsigned long*>(fresh_at(n, of) + e2) =
+                        fresh_word;
+                }
                 WAVE_LDS_SYNC();
             }
 #pragma unroll
@@ -1181,13 +1217,13 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         for (; kb < s.to; kb += DS_STEP) {
             const bool more = kb + DS_STEP < s.to;
             const long base = more && whole ? page_row(kb + DS_STEP) : 0;
-            // the tile with the step's own key and value
-            const bool patch = mine && newest < kb + DS_KEYS;
+            // rows whose keys are in this tile
+            unsigned patch = 0;
+            if (mine) patch = __ballot(own >= kb && own < kb + DS_KEYS);
             // values to LDS, 16-byte pieces xor-ed by the key
             const int to = ds_own(v_to), from = ds_own(v_from);
 #pragma unroll
             for (int i = 0; i < NL; ++i) {
-                const int row = ld_row + i * RPI;
 #pragma unroll
                 for (int p = 0; p < PC; ++p) {
                     ds_raw x = rv[i];
@@ -1195,9 +1231,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                         x = __builtin_bit_cast(
                             ds_raw, ds_widen(uint2v{rv[i][p * 2],
                                                     rv[i][p * 2 + 1]}));
-                    if (patch && kb + row >= newest)
-                        x = *reinterpret_cast<const ds_raw*>(
-                            &fresh_s[1][(ld_c + p) * 4]);
                     // (of keys RPI apart the same, or every other one's)
                     const int other = HD == 128 && RPI == 4 ? i % 2 * 128 : 0;
                     *reinterpret_cast<ds_raw*>(vt + (to ^ other) +
@@ -1205,6 +1238,23 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 }
             }
             if (more) values(kb + DS_STEP, base);
+            // (the last key's value stands in the tile's rows behind it, too)
+            const unsigned* fresh_k[2] = {nullptr, nullptr};
+#pragma unroll 1
+            for (unsigned b = patch; b; b &= b - 1) {
+                const int n = __builtin_ctz(b);
+                const int key = __builtin_amdgcn_readlane(own, n);
+                const int row = key - kb, c = lane % (HD / 8);
+                const int end = key == s.to - 1 ? DS_KEYS : row + 1;
+                const ds_raw x = *reinterpret_cast<const ds_raw*>(
+                    fresh_at(n, 1) + c * 4);
+                for (int r = row + lane / (HD / 8); r < end; r += 512 / HD)
+                    *reinterpret_cast<ds_raw*>(
+                        vt + r * RB + ((c ^ v_swz(r)) << 4)) = x;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (row == h * 16 + li) fresh_k[h] = fresh_at(n, 0);
+            }
             f32x4 sc[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -1214,9 +1264,9 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     bf16x8 ak;
                     if constexpr (sizeof(KVT) == 1) ak = ds_widen(rk[h][ks]);
                     else ak = __builtin_bit_cast(bf16x8, rk[h][ks]);
-                    if (patch && kb + h * 16 + li >= newest)
+                    if (patch && fresh_k[h])
                         ak = *reinterpret_cast<const bf16x8*>(
-                            &fresh_s[0][ks * 16 + lg * 4]);
+                            fresh_k[h] + ks * 16 + lg * 4);
                     sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                         ak, bq[ks], sc[h], 0, 0, 0);
                 }
@@ -1464,14 +1514,15 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 }
 
 // LDS of the rings; of the rows of `K` columns or the attention's tiles; of the
-// rows' rotation and, where there are few, their pages (up to 2 KB)
+// rows' rotation, new keys and values and, where there are few, their pages (up
+// to 2 KB)
 static long ds_area(int M, int K, int hd) {
     const long rows = (long)M * (K * 2 + DS_WAVES * 16);
     const long tiles = (long)DS_WAVES * DS_KEYS * hd * 2;
     return rows > tiles ? rows : tiles;
 }
 static long ds_lds(int M, int K, int hd) {
-    return DS_WAVES * DS_RING * 1024 + ds_area(M, K, hd) + M * hd * 4 + 2048;
+    return DS_WAVES * DS_RING * 1024 + ds_area(M, K, hd) + M * hd * 8 + 2048;
 }
 // ... beside what the kernel has without being asked
 constexpr long DS_LDS = 160 * 1024 - 17 * 1024;
@@ -1516,7 +1567,7 @@ extern "C" int launch_decode_stack(const StackArgs* args, int hd, int fp8,
     const dim3 grid(wgs), block((DS_WAVES + 1) * 64);
     const int lds = (int)ds_lds(a.M, deepest, hd);
     a.turns = (int)ds_area(a.M, deepest, hd);
-    a.pages = a.turns + a.M * hd * 4;
+    a.pages = a.turns + a.M * hd * 8;
     a.area = a.pages + ((long)a.M * a.W * 4 <= 2048 ? 1 : 0);
 #define DS_ONE(L, HD, T)                                                      \
     hipLaunchKernelGGL((decode_stack_kernel<L, HD, T>), grid, block, lds,     \

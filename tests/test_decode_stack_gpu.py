@@ -80,15 +80,19 @@ class _Step:
         self.table = 1 + torch.randperm(M * W, generator=g, device=DEV).int(
             ).view(M, W)
         self.lens = torch.tensor(lens, dtype=torch.int32, device=DEV)
-        self.pos = self.lens - 1
-        at = self.pos.long()
-        self.slots = (self.table.gather(1, (at // bs)[:, None]).squeeze(1) * bs
-                      + at % bs).int()
+        self.pos, self.bs = self.lens - 1, bs
+        self.place()
         self.x = torch.randn(M, spec.hidden_size, generator=g,
                              device=DEV).bfloat16()
         self.cos, self.sin = reference.rope_tables(max(lens), hd, 1e4, DEV)
         self.rope = spec.norm_type == "rmsnorm"
         self.act = "swiglu" if self.rope else "gelu"
+
+    def place(self):
+        """Slots of the positions."""
+        at, bs = self.pos.long(), self.bs
+        self.slots = (self.table.gather(1, (at // bs)[:, None]).squeeze(1) * bs
+                      + at % bs).int()
 
     def run(self, rows=None, workgroups=256, pages=None):
         rows = list(range(len(self.x))) if rows is None else rows
@@ -240,6 +244,36 @@ def test_a_token_without_a_position():
         for t, old in zip(kv, b):
             t[s[1] // 16, :, s[1] % 16] = old[s[1] // 16, :, s[1] % 16]
             assert torch.equal(t, old)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hd,bs,lens", [(64, 32, [34, 34, 34, 7]),
+                                        (128, 16, [254, 254, 254, 1000]),
+                                        (64, 24, [1500, 1500, 1500, 300]),
+                                        (128, 256, [2049, 2049, 2049, 20])])
+def test_new_tokens_anywhere_in_the_contexts(hd, bs, lens, fp8):
+    """Each row's attention has the step's own token of all rows whose pages it
+    reads: of three that follow each other in one sequence, and of one that is
+    stored inside its context; not behind a context's end."""
+    spec = _spec(256, 4, 2, hd, 1024, "rmsnorm")
+    step = _Step(spec, 2, lens, bs, fp8=fp8)
+    step.table[1] = step.table[2] = step.table[0]
+    for m in (0, 1):                           # row 2 has the last of the three
+        step.lens[m] -= 2 - m
+    step.pos = step.lens - 1
+    step.pos[3] = lens[3] // 2
+    step.place()
+    got, pages = step.run()
+    want, want_pages = step.want()
+    limit = 0.05 if fp8 else 0.015
+    for m in range(4):
+        error = _rel(got[m], want[m])
+        assert error <= limit, m
+    s = step.slots.long()
+    for kv, kv_want in zip(pages, want_pages):
+        for t, w in zip(kv, kv_want):
+            rows = (t.view(torch.float8_e4m3fn) if fp8 else t).double()
+            assert _rel(rows[s // bs, :, s % bs], w[s // bs, :, s % bs]) <= limit
 
 
 @pytest.mark.parametrize("length", [0, -3])
