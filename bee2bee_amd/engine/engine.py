@@ -1195,6 +1195,7 @@ class InferenceEngine:
             # invariance property test).
             self._last_sampled = next_dev
         next_ids = next_dev.cpu()  # the one host sync per step (emission)
+        self.runner.check_steps()
         now = time.time()
         n_emitted = 0
         for i, a in enumerate(acts):

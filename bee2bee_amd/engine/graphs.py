@@ -130,6 +130,7 @@ class DecodeGraphs:
         """Replay (capturing on first use) and return logits [bucket, V].
         Caller must have filled rows [:batch] of the static buffers and
         padded rows [batch:bucket] with safe scratch values."""
+        self.runner.check_steps()
         B = self.bucket_for(batch)
         if B not in self._graphs:
             self._capture(B)

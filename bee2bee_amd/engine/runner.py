@@ -60,6 +60,13 @@ class Runner:
         self._rope_by_cfg = {}
         self._zeros = {}        # fp32 zero vectors by length (zero-logit sinks)
         self.layer_tap = None
+        # set by a decode step's launch that could not be finished; the host
+        # reads it without a copy (check_steps)
+        self.step_status = None
+        if torch.device(device).type == "cuda":
+            self.step_status = torch.zeros(1, dtype=torch.int32,
+                                           pin_memory=True)
+            self._step_status = self.step_status.numpy()
         if spec.is_hybrid:
             self.rope_cos = self.rope_sin = None
             return
@@ -124,6 +131,17 @@ class Runner:
                 and all(t is None or t.dtype is torch.int32 for t in (
                     positions, slot_mapping, block_table, seq_lens))
                 and x.shape[0] <= min(6, ops.stack_rows(s)))
+
+    def check_steps(self) -> None:
+        """Raises if a decode step that has ended (the caller knows of that, by a
+        synchronisation or a copy of results) gave up a wait between its
+        workgroups: its hidden states, and those of steps behind it, are not
+        valid. Once for each such step; forward_decode looks by itself."""
+        if self.step_status is not None and self._step_status[0]:
+            self._step_status[0] = 0
+            raise RuntimeError(
+                "a decode step ended without all of its results: workgroups of "
+                "its launch waited for others that did not get on")
 
     @property
     def is_first_stage(self) -> bool:
@@ -688,6 +706,7 @@ class Runner:
         """One-token-per-sequence step. input [B] ids (or [B, H] hidden for
         later pipeline stages); returns final hidden [B, H]. slot_mapping
         None: where block_table has the positions."""
+        self.check_steps()
         if slot_mapping is None and self.spec.is_hybrid:
             slot_mapping = ops.decode_slots(block_table, positions,
                                             self.kv.block_size)
@@ -723,7 +742,8 @@ class Runner:
                 "gelu" if s.act_type == "gelu" else "swiglu", s.rms_eps,
                 self.scale, positions.contiguous(),
                 self.rope_cos if s.pos_type == "rope" else None, self.rope_sin,
-                slot_mapping, block_table.contiguous(), seq_lens)
+                slot_mapping, block_table.contiguous(), seq_lens,
+                status=self.step_status)
         if slot_mapping is None:
             slot_mapping = ops.decode_slots(block_table, positions,
                                             self.kv.block_size)

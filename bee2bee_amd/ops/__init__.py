@@ -304,19 +304,25 @@ def stack_rows(spec) -> int:
 
 def decode_stack(x, layers, pages, n_heads: int, act: str, eps: float,
                  scale: float, positions, cos, sin, slot_mapping, block_table,
-                 seq_lens, workgroups: int = 256):
+                 seq_lens, workgroups: int = 256, status=None,
+                 patience: int = 1 << 22, absent: int = 0):
     """Decoder layers of one token of each of x's rows [M, H], on the GPU:
     q|k|v (rotated where positions and cos are given) with its page store,
     attention against the pages, output, feed-forward. layers: their weights;
     pages: their (keys, values); slot_mapping None: decode_slots'. workgroups:
-    fewer than 256 compute the same."""
+    fewer than 256 compute the same. status: a pinned int32 on the host, which is
+    1 after a launch whose workgroups gave up a wait for each other, after
+    `patience` polls in which none got on: its result is not valid then, and what
+    depends on words that did not come is in no page. absent: so many of the 256
+    shares are marked as taken, though nobody takes them, so that such a wait
+    ends."""
     return require_hip().decode_stack(
         x, [[w.wqkv, w.wo, w.w_gate_up, w.w_down, w.wqkv_bias, w.wo_bias,
              w.w_gate_up_bias, w.w_down_bias, w.attn_norm, w.mlp_norm,
              w.attn_norm_bias, w.mlp_norm_bias, *kv]
             for w, kv in zip(layers, pages)],
         n_heads, act == "gelu", eps, scale, positions, cos, sin, slot_mapping,
-        block_table, seq_lens, workgroups)
+        block_table, seq_lens, workgroups, status, patience, absent)
 
 
 # Steps of some tens of rows: projections as fp32 parts over their inner

@@ -38,6 +38,12 @@
 //    (another kernel holds CUs) it claims free ones itself and does their work
 //    too. One that starts late and finds its number taken leaves. So a workgroup
 //    only ever waits for others that run.
+//  * A wait ends all the same: after DS_PATIENCE polls in which no workgroup with
+//    several numbers, which take their time, got on (the share of one is done in
+//    a millisecond). The host is told then (status), and from there on nothing is
+//    stored that depends on a word that did not come, to pages in particular: the
+//    others' waits end with it, and rows that no one is left to compute are NaN
+//    or as they were.
 #include "common.h"
 #include "decode_stack.h"
 
@@ -64,8 +70,6 @@ constexpr int DS_PART = 18;                    // words: 16 columns of a split's
 constexpr int DS_KEPT = 4;                     // octets of which much is in LDS
 constexpr float DS_LOG2E = 1.44269504088896340736f;
 enum { DS_LEAVE = -3, DS_OPEN = -2, DS_GO_ON = -1 };
-constexpr int DS_SPINS = 1 << 22;              // seconds: words that never come
-                                               // are taken as the NaN they are
 
 DEV_INLINE unsigned long ds_load(const void* p) {
     return __hip_atomic_load(reinterpret_cast<const unsigned long*>(p),
@@ -96,26 +100,11 @@ DEV_INLINE float ds_low(unsigned long v) {
 DEV_INLINE float ds_high(unsigned long v) {
     return __builtin_bit_cast(float, (unsigned)(v >> 32));
 }
-// Are all lanes' words there? If not, some clocks are left to the others before
-// they are asked for again: eight waves that ask without a pause keep the ninth
-// from issuing loads and stores at all.
-DEV_INLINE bool ds_again(bool there, int& spins) {
-    if (__all(there) || ++spins >= DS_SPINS) return false;
-    __builtin_amdgcn_s_sleep(1);
-    return true;
+DEV_INLINE unsigned ds_load4(const unsigned* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Until the word at p is there: one request a wave, where all the words that it
-// will read would be asked for in vain. Where those are few, asking for them all
-// saves the second request: up to 768 bytes of a wave's input (DS_FEW steps) a
-// layer of 768 columns takes 25.0 us and not 25.9, of 2048 34.9 and 35.4, but of
-// 4096, at up to 1 KB, 83.5 and 82.7.
+// Steps of a wave's input up to which all words are asked for at once (see until)
 constexpr int DS_FEW = 6;
-DEV_INLINE void ds_until(const unsigned* p) {
-    int spins = 0;
-    while (ds_again(__hip_atomic_load(p, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) != DS_EMPTY,
-                    spins)) {}
-}
 DEV_INLINE int ds_same(int v) { return __builtin_amdgcn_readfirstlane(v); }
 DEV_INLINE unsigned ds_pack(float a, float b) {
     return f2bf(a) | (unsigned)f2bf(b) << 16;
@@ -242,6 +231,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     __shared__ int slot_s[DS_ROWS], len_s[DS_ROWS];
     __shared__ int own_s[DS_ROWS];             // attention: keys of this step
     __shared__ int ncols, begin, gate;
+    __shared__ int gone;                       // a wait has been given up
+    __shared__ unsigned seen[DS_WAVES + 1];    // progress, when a wave last looked
     constexpr int LW = sizeof(StackLayer) / 4;
     __shared__ __attribute__((aligned(16))) int layers[(DS_LAYERS + 1) * LW];
 
@@ -297,7 +288,52 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     auto at = [&](int l, int off) __attribute__((always_inline)) {
         return DS_PTR(words) + (long)l * DS_INT(stride) + off;
     };
+    if (tid == 0) gone = 0;
+    if (lane == 0) seen[wid] = DS_EMPTY;
     ds_barrier();                              // (0) all of it is there
+
+    // Has this wait lasted long enough, or has another one?
+    auto enough = [&](int& polls) __attribute__((always_inline)) {
+        unsigned* const state = DS_PTR(state);
+        bool end =
+            ds_same(__hip_atomic_load(&gone, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_WORKGROUP)) ||
+            (unsigned)ds_same(ds_load4(state + 32)) != DS_EMPTY;
+        if (!end && polls >= DS_INT(patience)) {
+            const unsigned now = ds_same(ds_load4(state));
+            end = now == (unsigned)ds_same(seen[wid]);
+            if (lane == 0) seen[wid] = now;
+            polls = 0;
+        }
+        if (end && lane == 0) {
+            __hip_atomic_store(&gone, 1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_store(state + 32, 0u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            if (int* const status = DS_PTR(status))
+                __hip_atomic_store(status, 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return end;
+    };
+    // Are all lanes' words there? If not, some clocks are left to the others
+    // before they are asked for again: eight waves that ask without a pause keep
+    // the ninth from issuing loads and stores at all.
+    auto again = [&](bool there, int& polls) __attribute__((always_inline)) {
+        if (__all(there)) return false;
+        if (__builtin_expect((++polls & 31) == 0, 0) && enough(polls)) return false;
+        __builtin_amdgcn_s_sleep(1);
+        return true;
+    };
+    // Until the word at p is there: one request a wave, where all the words that
+    // it will read would be asked for in vain. Where those are few, asking for
+    // them all saves the second request: up to 768 bytes of a wave's input
+    // (DS_FEW steps) a layer of 768 columns takes 25.0 us and not 25.9, of 2048
+    // 34.9 and 35.4, but of 4096, at up to 1 KB, 83.5 and 82.7.
+    auto until = [&](const unsigned* p) __attribute__((always_inline)) {
+        int polls = 0;
+        while (again(ds_load4(p) != DS_EMPTY, polls)) {}
+    };
 
     if (wid == DS_WAVES) {
         // ------------------------------------------------ the ninth wave
@@ -403,7 +439,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     for (int i0 = 0; i0 < Q; i0 += U * 128) {
                         unsigned long v[R][U];
                         bool ok;
-                        int spins = 0;
+                        int polls = 0;
                         do {
                             ok = true;
 #pragma unroll
@@ -417,7 +453,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                             for (int i = 0; i < R * U; ++i)
                                 if (r0 + i / U < M && i0 + i % U * 128 < Q)
                                     ok = ok && ds_there(v[i / U][i % U]);
-                        } while (ds_again(ok, spins));
+                        } while (again(ok, polls));
 #pragma unroll
                         for (int i = 0; i < R * U; ++i)
                             if (r0 + i / U < M &&
@@ -431,10 +467,15 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 }
             };
             if (M * Q > 256)
-                ds_until(reinterpret_cast<const unsigned*>(squares) + M * Q - 1);
+                until(reinterpret_cast<const unsigned*>(squares) + M * Q - 1);
             if (M > 2 && Q <= 256) rows(std::integral_constant<int, 2>());
             else rows(std::integral_constant<int, 8>());
             return scale;
+        };
+        auto got_on = [&]() __attribute__((always_inline)) {
+            if (lane == 0)
+                __hip_atomic_fetch_add(DS_PTR(state), 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
         };
         bool passed = false;
         int nc = 1, parts = -1;
@@ -524,12 +565,13 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll
                 for (int w = 0; w < n; ++w) p[w] += p[w + n];
             buf ^= 1;
+            const bool sound = !gone, put = on && sound;
             float z = p[0] * inv;
             if (k == DS_UP && !gelu) {
                 const float u = ds_xor4(z);
                 const float v = z / (1.f + __expf(-z)) * u;
                 const float v1 = ds_xor1(v);
-                if (on && j < 4 && j % 2 == 0)
+                if (put && j < 4 && j % 2 == 0)
                     ds_store(dst + (m * N / 2 + o * 4 + j) / 2, ds_pack(v, v1));
                 return;
             }
@@ -540,20 +582,21 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 if (ends) {
                     const float y = ds_xor1(z);
                     if (on && j % 2 == 0)
-                        DS_PTR(out)[where / 2] = ds_pack(z, y);
+                        DS_PTR(out)[where / 2] = sound ? ds_pack(z, y)
+                                                       : 0x7fff7fffu;
                     return;
                 }
                 if (LAYER) {
-                    if (on) ds_store(dst + where, z);
+                    if (put) ds_store(dst + where, z);
                 } else {
                     const float v = z * times, v1 = ds_xor1(v);
-                    if (on && j % 2 == 0)
+                    if (put && j % 2 == 0)
                         ds_store(dst + where / 2, ds_pack(v, v1));
                     float sq = z * z;
                     sq += ds_xor1(sq);
                     sq += ds_xor2(sq);
                     sq += ds_xor4(sq);
-                    if (on && j == 0)
+                    if (put && j == 0)
                         ds_store(dst + M * H / 2 + where / 8, sq);
                 }
                 // (also for the next launch)
@@ -564,13 +607,13 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                                 (z + 0.044715f * z * z * z);
                 z = 0.5f * z * (1.f + tanhf(e));
                 const float y = ds_xor1(z);
-                if (on && j % 2 == 0) ds_store(dst + where / 2, ds_pack(z, y));
+                if (put && j % 2 == 0) ds_store(dst + where / 2, ds_pack(z, y));
             } else {
                 const int nq = DS_INT(nq), nkv = DS_INT(nkv);
                 z += add;
                 z = z * cosine + ds_xor4(z) * sine;
                 const float y = ds_xor1(z);
-                if (!on || j % 2) return;
+                if (!put || j % 2) return;
                 const int d = d0 + (j >> 2) * (HD / 2);
                 if (head < nq) {
                     ds_store(dst + (((m * nq + head) << hd_log2) + d) / 2,
@@ -627,6 +670,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     if (start && i == 0 && q == n - 1) decide();
                     if (own) octet(l, k, c + q * DS_WGS, i, q, bias, norm, dst);
                     else ds_barrier();
+                    if (nc > 1) got_on();
                 }
             }
             if (k < 3) fetch(l, k + 1);
@@ -681,6 +725,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 for (int i = 0; i < parts; ++i) {
                     ds_barrier();              // (A)
                     ds_barrier();              // (B)
+                    if (nc > 1) got_on();
                 }
             }
             if (++k == 4) k = 0, ++l;
@@ -805,9 +850,9 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 col;
             unsigned long v[DS_ROWS];
             bool ok;
-            int spins = 0;
-            if (!raw && n > 0 && M > 2) ds_until(from - col + (M - 1) * H + s0 * 64 +
-                                        n * 64 - 1);
+            int polls = 0;
+            if (!raw && n > 0 && M > 2)
+                until(from - col + (M - 1) * H + s0 * 64 + n * 64 - 1);
             do {
                 ok = true;
 #pragma unroll
@@ -826,7 +871,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll
                 for (int row = 0; row < DS_ROWS; ++row)
                     if (row < M) ok = ok && ds_there(v[row]);
-            } while (!raw && ds_again(ok, spins));
+            } while (!raw && again(ok, polls));
 #pragma unroll
             for (int row = 0; row < DS_ROWS; ++row)
                 if (row < M) {
@@ -878,7 +923,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             int i = 0;
             unsigned out = 0, in = 0;          // of a load's part of a row
             if (!raw && M * n > DS_FEW)
-                ds_until(reinterpret_cast<const unsigned*>(
+                until(reinterpret_cast<const unsigned*>(
                     x + (long)(M - 1) * K * 2 + n * 128 - 4));
             constexpr int B = 10;
             for (int l0 = 0; l0 < loads; l0 += B) {
@@ -898,7 +943,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     i = over ? 0 : i;
                 }
                 bool ok;
-                int spins = 0;
+                int polls = 0;
                 do {
                     ok = true;
 #pragma unroll
@@ -907,7 +952,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll
                     for (int u = 0; u < B; ++u)
                         if (l0 + u < loads) ok = ok && ds_there(v[u]);
-                } while (!raw && ds_again(ok, spins));
+                } while (!raw && again(ok, polls));
 #pragma unroll
                 for (int u = 0; u < B; ++u) {
                     if (l0 + u >= loads) continue;
@@ -1153,7 +1198,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             const unsigned* from = fresh_of(first);
             unsigned long q[KS][2], fresh_word = 0;
             bool ok;
-            int spins = 0;
+            int polls = 0;
             do {
                 ok = true;
                 if (mine) {
@@ -1167,7 +1212,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                         q[ks][e] = ds_load(qw + ks * 16 + e * 2);
                         ok = ok && ds_there(q[ks][e]);
                     }
-            } while (ds_again(ok, spins));
+            } while (again(ok, polls));
             if (mine) {
                 if (lane < M) own = own_s[lane];
                 *reinterpret_cast<unsigned long*>(fresh_at(first, of) + e2) =
@@ -1175,9 +1220,9 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll 1
                 for (unsigned b = mine & (mine - 1); b; b &= b - 1) {
                     const int n = __builtin_ctz(b);
-                    spins = 0;
+                    polls = 0;
                     do fresh_word = ds_load(fresh_of(n));
-                    while (ds_again(ds_there(fresh_word), spins));
+                    while (again(ds_there(fresh_word), polls));
                     *reinterpret_cast<unsigned long*>(fresh_at(n, of) + e2) =
                         fresh_word;
                 }
@@ -1342,6 +1387,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                                           wid * 16 + lg * 4) / 2;
         ds_barrier();                          // (A)
         if (wid < DT) {
+            const bool put = li < G && !gone;
             float wm[DS_WAVES], ws[DS_WAVES], top = -1e30f, all = 0.f;
             f32x4 x[DS_WAVES], y{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1362,7 +1408,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r) y[r] = fmaf(x[w][r], wm[w], y[r]);
             }
-            if (li < G) {
+            if (put) {
                 if (split) {
                     ds_store(to, y[0], y[1]);
                     ds_store(to + 2, y[2], y[3]);
@@ -1397,8 +1443,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             at(l, DS_INT(att)) + ((it << hd_log2) + wid * 16 + c * 2) / 2;
         unsigned long v[U], e[U];
         bool ok;
-        int spins = 0;
-        ds_until(from + (long)(nz - 1) * step + 17);
+        int polls = 0;
+        until(from + (long)(nz - 1) * step + 17);
         do {
             ok = true;
 #pragma unroll
@@ -1412,7 +1458,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 ok = ok && ds_there(v[u]) && ds_there(e[u]);
-        } while (ds_again(ok, spins));
+        } while (again(ok, polls));
+        if (!__all(ok)) return;
         auto empty = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -1542,9 +1589,9 @@ extern "C" int decode_stack_splits(long pairs, long keys) {
     return Z > DS_SPLITS ? DS_SPLITS : Z < 1 ? 1 : (int)Z;
 }
 
-// The fields of `args` as decode_stack.h says, every word that passes and the
-// claims DS_EMPTY, all rows 16-byte aligned. Nonzero for sizes that the kernel
-// does not take.
+// The fields of `args` as decode_stack.h says, every word that passes, the
+// claims and the state DS_EMPTY, all rows 16-byte aligned. Nonzero for sizes that
+// the kernel does not take.
 extern "C" int launch_decode_stack(const StackArgs* args, int hd, int fp8,
                                    int layer_norm, int wgs,
                                    hipStream_t stream) {
@@ -1554,7 +1601,7 @@ extern "C" int launch_decode_stack(const StackArgs* args, int hd, int fp8,
     if (wgs < 1 || wgs > DS_WGS || (hd != 64 && hd != 128)) return 1;
     if (a.nkv < 1 || a.nq != a.G * a.nkv || a.G > 16 || a.Z < 1) return 1;
     if (a.items != a.M * a.nkv * a.Z) return 1;
-    if (a.Z > DS_SPLITS || !(a.scale > 0.f)) return 1;
+    if (a.Z > DS_SPLITS || !(a.scale > 0.f) || a.patience < 1) return 1;
     int deepest = 0;
     for (int k = 0; k < 4; ++k) {
         const long K = a.K[k];

@@ -280,14 +280,17 @@ int64_t stack_rows(int64_t hidden, int64_t nq, int64_t nkv, int64_t hd,
 // The layers of a decode step, x [M, H] to the last one's result. A layer is 14
 // tensors: w_qkv, w_o, w_up, w_down, their biases, the two norms' weights, their
 // biases (layer norm: all given), pages of keys and of values. wgs: workgroups
-// (DS_WGS; fewer do the work of the others).
+// (DS_WGS; fewer do the work of the others). status: see decode_stack.h, pinned.
+// absent: so many of the last numbers are marked as taken, by nobody.
 Tensor decode_stack(const Tensor& x,
                     const std::vector<std::vector<optional<Tensor>>>& layers,
                     int64_t nq, bool gelu, double eps, double scale,
                     const optional<Tensor>& pos, const optional<Tensor>& cos_t,
                     const optional<Tensor>& sin_t,
                     const optional<Tensor>& slots, const Tensor& table,
-                    const Tensor& seq_lens, int64_t wgs) {
+                    const Tensor& seq_lens, int64_t wgs,
+                    const optional<Tensor>& status, int64_t patience,
+                    int64_t absent) {
     const int L = layers.size();
     TORCH_CHECK(L >= 1 && layers[0].size() == 14);
     const Tensor xd = dense(x, "x");
@@ -358,11 +361,27 @@ Tensor decode_stack(const Tensor& x,
     a.items = M * nkv * a.Z;
     const long parts = a.Z > 1 ? (long)a.items * a.G * (hd / 16 * 18) : 0;
     const long claims = (long)launches * DS_CLAIMS;
-    Tensor work = torch::full({claims + (long)L * a.stride + parts}, -1,
+    Tensor work = torch::full({claims + DS_STATE + (long)L * a.stride + parts},
+                              -1,
                               xd.options().dtype(torch::kInt32));
     unsigned* words = reinterpret_cast<unsigned*>(work.data_ptr());
-    a.words = words + claims;
+    a.state = words + claims;
+    a.words = a.state + DS_STATE;
     a.parts = a.words + (long)L * a.stride;
+    TORCH_CHECK(absent >= 0 && absent < DS_WGS && patience >= 1 &&
+                patience <= DS_PATIENCE);
+    for (int i = 0; i < launches; ++i)
+        for (int c = DS_WGS - absent; c < DS_WGS; ++c) {
+            work[(long)i * DS_CLAIMS + c].zero_();
+            work[(long)i * DS_CLAIMS + DS_WGS + c % 8 * 32].add_(1);
+        }
+    a.patience = (int)patience;
+    if (status.has_value()) {
+        TORCH_CHECK(status->device().is_cpu() && status->numel() == 1 &&
+                    status->scalar_type() == torch::kInt32 &&
+                    status->is_pinned(), "status: one pinned int32");
+        a.status = status->data_ptr<int>();
+    }
     Tensor x32 = torch::empty({M, H}, xd.options().dtype(torch::kFloat32));
     Tensor out = torch::empty({M, H}, xd.options());
     a.x = ptr(xd);

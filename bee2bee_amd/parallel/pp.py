@@ -200,7 +200,9 @@ class PipelineEngine:
         else:
             logits = self.runner.lm_head(hidden)
             next_ids = sample(logits, sampling).cpu()
-        return self._bcast_ids(next_ids, B)
+        ids = self._bcast_ids(next_ids, B)
+        self.runner.check_steps()              # (every stage's has ended)
+        return ids
 
     @torch.no_grad()
     def generate(

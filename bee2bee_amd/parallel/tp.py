@@ -215,8 +215,10 @@ class TPEngine:
         hidden = self.runner.forward_decode(
             ids.to(dev), positions, slots, bt, lens_t
         )
-        return sample(self.runner.lm_head(hidden), sampling,
-                      generator=self.sample_gen).cpu()
+        ids = sample(self.runner.lm_head(hidden), sampling,
+                     generator=self.sample_gen).cpu()
+        self.runner.check_steps()
+        return ids
 
     @torch.no_grad()
     def reset(self) -> None:

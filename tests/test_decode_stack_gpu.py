@@ -94,7 +94,7 @@ class _Step:
         self.slots = (self.table.gather(1, (at // bs)[:, None]).squeeze(1) * bs
                       + at % bs).int()
 
-    def run(self, rows=None, workgroups=256, pages=None):
+    def run(self, rows=None, workgroups=256, pages=None, **more):
         rows = list(range(len(self.x))) if rows is None else rows
         pages = pages or [[t.clone() for t in kv] for kv in self.pages]
         s = self.spec
@@ -102,7 +102,7 @@ class _Step:
             self.x[rows], self.layers, pages, s.n_heads, self.act, 1e-5,
             s.head_dim ** -0.5, self.pos[rows] if self.rope else None,
             self.cos, self.sin, self.slots[rows], self.table[rows],
-            self.lens[rows], workgroups)
+            self.lens[rows], workgroups, **more)
         return out, pages
 
     def want(self):
@@ -291,6 +291,46 @@ def test_a_row_without_keys(at, length):
     assert torch.equal(got[others], beside[others])
     step.lens[at] = step.slots[at] = 0         # (page 0 is nobody's)
     assert _rel(got, step.want()[0]) <= 0.015
+
+
+@pytest.mark.parametrize("kind", ["rmsnorm", "layernorm"])
+@pytest.mark.parametrize("lens", [[40, 7], [1500, 2000, 300]])
+@pytest.mark.parametrize("absent", [1, 30, 255])
+def test_a_wait_that_ends(kind, lens, absent):
+    """For shares that nobody has: the launch ends, the host is told, and the
+    pages have what they had, or what a sound step stores."""
+    inner = 1024 if kind == "rmsnorm" else 2048          # of 256 octets
+    spec = _spec(256, 4, 2, 64, inner, kind)
+    step = _Step(spec, 2, lens, 16)
+    status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    want, sound = step.run(status=status)
+    torch.cuda.synchronize()
+    assert status.item() == 0
+    _, pages = step.run(status=status, patience=256, absent=absent)
+    torch.cuda.synchronize()
+    assert status.item() == 1
+    for layer in range(2):
+        for t, good, before in zip(pages[layer], sound[layer],
+                                   step.pages[layer]):
+            same = (t == before) | ((t == good) & (layer == 0))
+            assert same.all(), layer
+    status.zero_()
+    assert torch.equal(step.run(status=status)[0], want)
+    assert status.item() == 0
+
+
+def test_waits_last_while_others_get_on():
+    """Three workgroups with some 85 numbers each, of which one takes up to 150 us
+    of a product: a launch of 20 ms with a patience of a millisecond at most (of
+    64 polls, it gives up now and then)."""
+    spec = _spec(8192, 64, 8, 128, 28672, "rmsnorm")
+    step = _Step(spec, 1, [300], 256)
+    status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    want = step.run(status=status)[0]
+    got = step.run(workgroups=3, status=status, patience=512)[0]
+    torch.cuda.synchronize()
+    assert status.item() == 0
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("kind", ["rmsnorm", "layernorm"])

@@ -167,6 +167,20 @@ def test_few_rows_of_wide_stacks(hidden, rows, rings):
     test_steps(spec, rows, "native")
 
 
+def test_a_step_that_gave_up_is_told():
+    """What such a launch leaves on the host (test_decode_stack_gpu.py): the next
+    call raises, and the ones after it do not."""
+    W = ModelWeights(SWIGLU, DEV, torch.bfloat16).random_init(seed=3)
+    side = _Side(SWIGLU, W, DEV, torch.bfloat16, "native")
+    side.prompt(torch.arange(3), [3])
+    want = side.decode(torch.tensor([1]), 3)
+    side.runner.step_status.fill_(1)
+    with pytest.raises(RuntimeError, match="without all"):
+        side.decode(torch.tensor([1]), 3)
+    side.runner.check_steps()
+    assert torch.equal(side.decode(torch.tensor([1]), 3), want)
+
+
 def test_wide_specs_leave_products_to_the_library():
     """What WIDE above is for: each has one that is left, and one that is not."""
     from bee2bee_amd import ops
