@@ -740,9 +740,10 @@ class Runner:
                 hidden, [self.weights.layers[i] for i in layers],
                 [self.kv.layer(i) for i in layers], s.n_heads,
                 "gelu" if s.act_type == "gelu" else "swiglu", s.rms_eps,
-                self.scale, positions.contiguous(),
+                self.scale,
+                positions if s.pos_type == "rope" else positions.contiguous(),
                 self.rope_cos if s.pos_type == "rope" else None, self.rope_sin,
-                slot_mapping, block_table.contiguous(), seq_lens,
+                slot_mapping, block_table, seq_lens,
                 status=self.step_status)
         if slot_mapping is None:
             slot_mapping = ops.decode_slots(block_table, positions,

@@ -266,11 +266,12 @@ Tensor rows_qkv(const Tensor& x, const Tensor& w, const optional<Tensor>& bias,
 }
 
 // Most rows of a decode step whose layers decode_stack takes, 0 for a stack that
-// it does not take.
+// it does not take (among them the group sizes that attn_decode refuses).
 int64_t stack_rows(int64_t hidden, int64_t nq, int64_t nkv, int64_t hd,
                    int64_t inner, bool layer_norm) {
     const int64_t deepest = std::max(std::max(hidden, nq * hd), inner);
-    if ((hd != 64 && hd != 128) || nkv < 1 || nq % nkv || nq / nkv > 16 ||
+    const int64_t G = nkv < 1 || nq % nkv ? 0 : nq / nkv;
+    if ((hd != 64 && hd != 128) || !((G >= 1 && G <= 8) || G == 16) ||
         hidden % 64 || inner % 64 || deepest > 1 << 16 ||
         (layer_norm && hidden > DS_LAYER_NORM))
         return 0;
@@ -307,10 +308,13 @@ Tensor decode_stack(const Tensor& x,
     TORCH_CHECK(M >= 1 && M <= stack_rows(H, nq, nkv, hd, I, norm_b), "rows");
     auto ints = [&](const Tensor& t, long n, const char* name) {
         TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt32 &&
-                    t.is_contiguous() && t.numel() == n, name);
+                    t.is_contiguous() && t.numel() >= n, name);
         return t.data_ptr<int>();
     };
-    TORCH_CHECK(table.dim() == 2 && table.size(0) == M && table.size(1) > 0);
+    // tables and lengths may be of more rows, contexts as long as attn_decode's
+    TORCH_CHECK(table.dim() == 2 && table.size(1) > 0);
+    TORCH_CHECK(table.size(1) * bs <= 32768,
+                "decode supports up to 32768-token contexts for now");
 
     StackArgs a{};
     a.M = M;
@@ -324,11 +328,15 @@ Tensor decode_stack(const Tensor& x,
     a.scale = (float)scale;
     a.all = L;
     TORCH_CHECK(slots.has_value() || pos.has_value(), "slots or positions");
-    if (slots.has_value()) a.slots = ints(*slots, M, "slots");
+    if (slots.has_value()) {
+        a.slots = ints(*slots, M, "slots");
+        TORCH_CHECK(slots->numel() == M, "slots");
+    }
     a.table = ints(table, (long)M * a.W, "table");
     a.seq_lens = ints(seq_lens, M, "seq_lens");
     if (pos.has_value()) {
         a.pos = ints(*pos, M, "positions");
+        TORCH_CHECK(pos->numel() == M, "positions");
     }
     if (pos.has_value() && cos_t.has_value()) {
         const Turns by = turns(cos_t, sin_t, hd);

@@ -167,6 +167,41 @@ def test_few_rows_of_wide_stacks(hidden, rows, rings):
     test_steps(spec, rows, "native")
 
 
+@torch.no_grad()
+def test_what_few_rows_take_and_refuse():
+    """As steps of more rows do: tables and lengths of more rows than there are;
+    no contexts past 32768 tokens, and not every group of query heads."""
+    W = ModelWeights(SWIGLU, DEV, torch.bfloat16).random_init(seed=3)
+    side = _Side(SWIGLU, W, DEV, torch.bfloat16, "native")
+    side.prompt(torch.arange(9), [1] * 9)
+    table = side.kv.block_table(side.rows)
+    lens = side.ints([2] * 9)
+
+    def step(rows, table=table, lens=lens):
+        pos = lens[:rows] - 1
+        return side.runner.forward_decode(
+            torch.ones(rows, dtype=torch.int64, device=DEV), pos,
+            decode_slot_mapping(table[:rows], pos, 16), table, lens)
+
+    for rows in (2, 7):
+        assert torch.equal(step(rows), step(rows, table[:rows].contiguous(),
+                                            lens[:rows]))
+        wide = torch.zeros(rows, 2049, dtype=torch.int32, device=DEV)
+        wide[:, 0] = table[:rows, 0]
+        assert step(rows, wide[:, :2048].contiguous()).isfinite().all()
+        with pytest.raises(RuntimeError, match="32768"):
+            step(rows, wide)
+        with pytest.raises(RuntimeError):
+            step(rows, wide[:, :2048])         # (not contiguous)
+    from bee2bee_amd import ops
+
+    for heads, rows in ((8, 8), (9, 0), (15, 0), (16, 8)):
+        spec = ModelSpec(name="t-group", vocab_size=64, hidden_size=576,
+                         intermediate_size=128, n_layers=1, n_heads=heads,
+                         n_kv_heads=1, head_dim=64, max_seq_len=64)
+        assert ops.stack_rows(spec) == rows
+
+
 def test_a_step_that_gave_up_is_told():
     """What such a launch leaves on the host (test_decode_stack_gpu.py): the next
     call raises, and the ones after it do not."""
