@@ -60,8 +60,8 @@ def serve_hf(model, model_path, port, region, api_port, device):
 @click.option("--api-port", default=8000, type=int)
 @click.option("--device", default=None)
 @click.option("--spec-decode", is_flag=True,
-              help="speculative decoding (prompt-lookup + exact greedy "
-                   "verification; output-invariant)")
+              help="speculative decoding (prompt-lookup + greedy "
+                   "verification; the same tokens but for ties)")
 @click.option("--kv-fp8", is_flag=True,
               help="fp8 (OCP e4m3) KV cache: half the decode-attention "
                    "bytes at a small quantization cost")

@@ -215,9 +215,11 @@ class InferenceEngine:
         # -token for requests behind a burst (they decode while later
         # arrivals prefill)
         self.max_prefill_tokens = max_prefill_tokens
-        # speculative decoding (prompt-lookup / n-gram proposer + exact
-        # greedy verification over the paged-history prefill path); output-
-        # invariant: verified tokens equal plain greedy decode
+        # speculative decoding (prompt-lookup / n-gram proposer + greedy
+        # verification over the paged-history prefill path): the tokens of
+        # plain greedy decode but for ties. In bf16 on the GPU a verification
+        # and a decode step sum in other orders, and of two logits that are
+        # equal but for that either may be the larger.
         self.spec_decode = spec_decode
         self.spec_k = spec_k
         self.spec_ngram = spec_ngram
@@ -896,8 +898,8 @@ class InferenceEngine:
     def _decode_spec_once(self) -> None:
         """One speculative step: each greedy sequence verifies its pending
         token plus up to spec_k proposed tokens in ONE forward through the
-        chunked-prefill (paged-history) path; the accepted prefix is exactly
-        what plain greedy decode would emit (verification is exact)."""
+        chunked-prefill (paged-history) path; the accepted prefix is what
+        plain greedy decode would emit, but for ties (see __init__)."""
         dev = self.device
         acts = self._active
         # propose first: when nothing is speculatable this step, take the

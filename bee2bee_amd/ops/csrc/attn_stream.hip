@@ -465,10 +465,11 @@ static long stream_groups(long pairs, long rows) {
 // 128: 5 rows x 1 sequence 24 / 158; 128 rows x 4 67 / 163; 128 rows x 16
 // 178 / 213; 256 rows x 16 365 / 243; 64 rows x 64 with 2000 cached 210 /
 // 104). Up to 32 rows stay here at any batch (64 sequences, 2000 cached: 109
-// / 101), so that verified tokens are computed as decoded ones are; to the bit
-// only the last token of each sequence, beside as many sequences in a table as
-// wide (the splits' borders follow from them) and on bf16 pages (decoding
-// rounds its queries on 8-bit ones).
+// / 101), so that verified tokens attend as decoded ones do in steps of more
+// rows than decode_stack.hip takes; to the bit only the last token of each
+// sequence, beside as many sequences in a table as wide (the splits' borders
+// follow from them) and on bf16 pages (decoding rounds its queries on 8-bit
+// ones).
 extern "C" int attn_stream_takes(long pairs, long rows) {
     return rows <= 32 || stream_groups(pairs, rows) <= 448;
 }

@@ -556,6 +556,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 sine = j < 4 ? -t[HD / 2] : t[HD / 2];
             }
             ds_barrier();                      // the waves' sums are there
+            // (one order of three whose errors against 64 bits are the same)
             float p[DS_WAVES];
 #pragma unroll
             for (int w = 0; w < DS_WAVES; ++w)

@@ -209,20 +209,51 @@ def test_chunked_prefill_matches_whole_gpu(engine):
     assert torch.isfinite(chunked).all()
 
 
+def decoded_gaps(engine, prompt, tokens):
+    """How far each of `tokens`, which follow the prompt, is below the largest
+    logit of a plain decode step on the tokens before it, over the logits' root
+    mean square: 0 for what greedy decoding gives, 4 or so for any other token of
+    a random model."""
+    from bee2bee_amd.engine.kv import PagedKV
+    from bee2bee_amd.engine.runner import Runner
+
+    dev = torch.device("cuda:0")
+    kv = PagedKV(engine.spec, dev, torch.bfloat16, n_blocks=8)
+    runner = Runner(engine.spec, engine.weights, kv, dev, torch.bfloat16)
+
+    def ints(*x):
+        return torch.tensor(x, dtype=torch.int32, device=dev)
+
+    n = len(prompt)
+    kv.new_seq(0)
+    kv.extend_seq(0, n + len(tokens))
+    table = kv.block_table([0])
+    hidden = runner.forward_prefill(
+        torch.tensor(prompt, device=dev), ints(*range(n)),
+        ints(*kv.slot_mapping(0, range(n))), ints(0, n), n)[-1:]
+    gaps = []
+    for i, token in enumerate(tokens):
+        logits = runner.lm_head(hidden).float()[0]
+        gaps.append(((logits.max() - logits[token])
+                     / logits.square().mean().sqrt()).item())
+        hidden = runner.forward_decode(
+            torch.tensor([token], device=dev), ints(n + i), None, table,
+            ints(n + i + 1))
+    return gaps
+
+
+# Two computations of a logit in bf16 differ by 1% of the logits' root mean square
+# (the tolerance of one step's error), four of them decide which of two tokens is
+# the greater one: 2% as a deviation, five times that as a limit.
+NEAR_TIE = 0.1
+
+
 def test_spec_decode_gpu():
-    """Speculative decoding on the HIP path: greedy output must match the
-    plain engine exactly (verification guarantees it for identical logits;
-    both paths compute the verify forward with the same kernels here since
-    spec mode disables graphs — compare against an eager engine)."""
+    """Speculative decoding on the HIP path emits what plain decode steps do, but
+    for ties: verification sums in another order than steps of few rows do, and
+    whichever of two logits that are equal to 1% is the larger one there, is as
+    good."""
     prompt = [11, 500, 77] * 8
-    plain = InferenceEngine(
-        "llama3.2-1b", device="cuda:0", max_batch=4, max_seq_len=512,
-        seed=11, use_graphs=False,
-    )
-    try:
-        exp = _greedy(plain, prompt, 24)
-    finally:
-        plain.shutdown()
     spec = InferenceEngine(
         "llama3.2-1b", device="cuda:0", max_batch=4, max_seq_len=512,
         seed=11, spec_decode=True,
@@ -230,12 +261,11 @@ def test_spec_decode_gpu():
     try:
         got = _greedy(spec, prompt, 24)
         stats = dict(spec.spec_stats)
+        gaps = decoded_gaps(spec, prompt, got)
+        other = decoded_gaps(spec, prompt, [t + 1 for t in got])
     finally:
         spec.shutdown()
     assert len(got) == 24
-    # bf16 near-ties can flip tokens between the decode kernel (plain) and
-    # the paged-prefill kernel (spec verify), so require a long matching
-    # prefix rather than full equality
-    match = sum(1 for x, y in zip(got, exp) if x == y)
-    assert match >= 12, f"only {match}/24 tokens match: {got} vs {exp}"
+    assert max(gaps) <= NEAR_TIE, gaps
+    assert min(other) > 10 * NEAR_TIE, other   # (what the limit tells apart)
     assert stats["steps"] <= 24

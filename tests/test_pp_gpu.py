@@ -1,6 +1,7 @@
 """Pipeline parallelism on the HIP path: two processes share one MI355X
-(gloo transport staging through host) and must produce the same greedy
-tokens as the single-process GPU engine."""
+(gloo transport staging through host) and must produce greedy tokens of the
+single-process GPU stack, but for ties: a stage's rows are rounded to bf16 on
+their way to the next."""
 import multiprocessing as mp
 import pickle
 
@@ -55,30 +56,16 @@ def test_pp2_gpu_matches_single(tmp_path):
     with open(out_path, "rb") as f:
         pp_outs = pickle.load(f)
 
-    # single-process reference on the same GPU/weights (bf16: compare with
-    # tolerance at token level — identical kernels, so expect exact match)
-    from bee2bee_amd.engine.engine import GenerationRequest, InferenceEngine
-    from bee2bee_amd.engine.sampler import SamplingParams
+    # the logits of a single process on the same GPU and weights decide
+    from bee2bee_amd.engine.engine import InferenceEngine
+
+    from tests.test_engine_gpu import NEAR_TIE, decoded_gaps
 
     eng = InferenceEngine("llama3.2-1b", device="cuda:0", max_batch=4,
                           max_seq_len=128, seed=SEED, use_graphs=False)
     try:
-        ref = []
-        for prompt in PROMPTS:
-            req = GenerationRequest(prompt_ids=list(prompt), max_new_tokens=N_NEW,
-                                    sampling=SamplingParams(greedy=True))
-            eng.submit(req)
-            while True:
-                item = req.out_queue.get(timeout=300)
-                if not isinstance(item, int):
-                    break
-            ref.append(req.output_ids)
+        gaps = [decoded_gaps(eng, p, out) for p, out in zip(PROMPTS, pp_outs)]
     finally:
         eng.shutdown()
-    # batched-vs-solo GEMM tilings can flip near-tied argmaxes; require the
-    # first tokens to agree and the rest to mostly agree
-    agree = sum(
-        a == b for pa, pb in zip(pp_outs, ref) for a, b in zip(pa, pb)
-    )
-    total = sum(len(x) for x in ref)
-    assert agree / total >= 0.75, (pp_outs, ref)
+    assert [len(g) for g in gaps] == [N_NEW] * len(PROMPTS)
+    assert max(map(max, gaps)) <= NEAR_TIE, gaps
