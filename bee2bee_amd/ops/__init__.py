@@ -310,7 +310,8 @@ def decode_stack(x, layers, pages, n_heads: int, act: str, eps: float,
     q|k|v (rotated where positions and cos are given) with its page store,
     attention against the pages, output, feed-forward. layers: their weights;
     pages: their (keys, values); slot_mapping None: decode_slots'. workgroups:
-    fewer than 256 compute the same. status: a pinned int32 on the host, which is
+    fewer than 256 compute the same, and up to 256 more find their share taken.
+    status: a pinned int32 on the host, which is
     1 after a launch whose workgroups gave up a wait for each other, after
     `patience` polls in which none got on: its result is not valid then, and what
     depends on words that did not come is in no page. absent: so many of the 256

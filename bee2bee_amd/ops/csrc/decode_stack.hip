@@ -218,6 +218,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     StackArgs args) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int number = blockIdx.x % DS_WGS;
     // the rings; then input rows, or the attention waves' tiles
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* const area = smem + DS_WAVES * DS_RING * 1024;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                        DS_WGS / 8 - 1;
             return (bool)__all(full);
         };
-        const int mine = blockIdx.x;
+        const int mine = number;
         // What the step's rows are: slots, lengths, pages, rotation. The others
         // have them with their next barrier.
         int slot = 0, len = 0, position = 0;
@@ -765,7 +766,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                : f == 6 ? K * 2
                         : (int)((unsigned)told_s.half[k] * K * 2);
     };
-    prepare(blockIdx.x);
+    prepare(number);
     auto planned = [&](int k, int f) __attribute__((always_inline)) {
         return __builtin_amdgcn_readlane(plan, k * 8 + f);
     };
@@ -794,7 +795,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 }
                 continue;
             }
-            if (gnc > 1) prepare(gi ? ds_same(cols[gi]) : (int)blockIdx.x);
+            if (gnc > 1) prepare(gi ? ds_same(cols[gi]) : number);
             goct = planned(gk, 0);
             if (!goct) continue;
             gleft = gn = planned(gk, 1) & 0xffff;
@@ -1513,12 +1514,12 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         }
         int some = 0;
         if (other >= 0) some = count(k, other);
-        else if (gnc == 1) some = count(k, blockIdx.x);
+        else if (gnc == 1) some = count(k, number);
         else
             for (int i = 0; i < gnc; ++i) some += count(k, ds_same(cols[i]));
         if (some) input(l, k);
         for (int i = other >= 0 ? gnc - 1 : 0; i < gnc; ++i)
-            product(k, i ? ds_same(cols[i]) : (int)blockIdx.x);
+            product(k, i ? ds_same(cols[i]) : number);
         if (l == lo && k == DS_QKV) {
             bool on = false;
             if (other < 0) {
@@ -1547,12 +1548,12 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         }
         if (k == DS_QKV) {
             for (int i = 0; i < gnc; ++i)
-                for (int it = i ? ds_same(cols[i]) : (int)blockIdx.x;
+                for (int it = i ? ds_same(cols[i]) : number;
                      it < DS_INT(items); it += DS_WGS)
                     attention(l, it);
             if (DS_INT(Z) > 1)
                 for (int i = 0; i < gnc; ++i)
-                    for (int it = i ? ds_same(cols[i]) : (int)blockIdx.x;
+                    for (int it = i ? ds_same(cols[i]) : number;
                          it < M * DS_INT(nq); it += DS_WGS)
                         combine(l, it);
         }
@@ -1599,7 +1600,7 @@ extern "C" int launch_decode_stack(const StackArgs* args, int hd, int fp8,
     StackArgs a = *args;
     const int layers = a.hi - a.lo;
     if (layers < 1 || layers > DS_LAYERS || a.M < 1) return 1;
-    if (wgs < 1 || wgs > DS_WGS || (hd != 64 && hd != 128)) return 1;
+    if (wgs < 1 || wgs > 2 * DS_WGS || (hd != 64 && hd != 128)) return 1;
     if (a.nkv < 1 || a.nq != a.G * a.nkv || a.G > 16 || a.Z < 1) return 1;
     if (a.items != a.M * a.nkv * a.Z) return 1;
     if (a.Z > DS_SPLITS || !(a.scale > 0.f) || a.patience < 1) return 1;

@@ -281,7 +281,7 @@ int64_t stack_rows(int64_t hidden, int64_t nq, int64_t nkv, int64_t hd,
 // The layers of a decode step, x [M, H] to the last one's result. A layer is 14
 // tensors: w_qkv, w_o, w_up, w_down, their biases, the two norms' weights, their
 // biases (layer norm: all given), pages of keys and of values. wgs: workgroups
-// (DS_WGS; fewer do the work of the others). status: see decode_stack.h, pinned.
+// (DS_WGS; fewer do the work of the others, more find it taken). status: see decode_stack.h, pinned.
 // absent: so many of the last numbers are marked as taken, by nobody.
 Tensor decode_stack(const Tensor& x,
                     const std::vector<std::vector<optional<Tensor>>>& layers,

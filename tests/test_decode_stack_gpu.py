@@ -184,15 +184,48 @@ def test_stack(case, fp8, workgroups):
             assert torch.equal(t, b)           # and nothing else
 
 
-def test_rows_and_workgroups_do_not_change_a_row():
-    """Contexts that are not split: a row is the same to the bit beside others,
-    and whoever computes it."""
+# contexts of one split, and of splits of 128 keys for any number of rows: 1000
+# keys in 8 (8 rows of 4 key heads) or more
+@pytest.mark.parametrize("lens", [[40, 255, 7, 256, 64, 1, 129, 200],
+                                  [40, 1000, 7, 513, 64, 1, 300, 999]])
+def test_rows_and_workgroups_do_not_change_a_row(lens):
+    """Where a context's splits do not depend on the number of rows, a row is the
+    same to the bit beside others, and whoever computes it."""
     spec = _spec(1024, 16, 4, 64, 2816, "rmsnorm")
-    step = _Step(spec, 2, [40, 1000, 7, 513, 64, 1, 300, 999], 16)
+    step = _Step(spec, 2, lens, 16)
     full, _ = step.run()
     for rows in ([3], [5, 2], [7, 0, 1, 4, 6]):
         assert torch.equal(step.run(rows)[0], full[rows])
-        assert torch.equal(step.run(rows, 77)[0], full[rows])
+        for workgroups in (77, 300, 512):
+            assert torch.equal(step.run(rows, workgroups)[0], full[rows])
+
+
+@pytest.mark.parametrize("kind", ["rmsnorm", "layernorm"])
+def test_steps_side_by_side(kind):
+    """Three streams whose steps want all CUs: each has some, its workgroups take
+    over what the others' keep from starting, and those leave when they start."""
+    spec = _spec(768, 12, 4, 64, 3072, kind)
+    steps = [_Step(spec, 6, [300, 40], 16), _Step(spec, 6, [1500], 16),
+             _Step(spec, 6, [7, 257, 64, 90], 16)]
+    status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    want = [s.run() for s in steps]
+    streams = [torch.cuda.Stream() for _ in steps]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        pages = [[[t.clone() for t in kv] for kv in s.pages] for s in steps]
+        torch.cuda.synchronize()
+        got = []
+        for _ in range(4):                     # (the same tokens again)
+            for s, p, stream in zip(steps, pages, streams):
+                with torch.cuda.stream(stream):
+                    got.append(s.run(pages=p, status=status)[0])
+        torch.cuda.synchronize()
+        assert status.item() == 0
+        for i, x in enumerate(got):
+            assert torch.equal(x, want[i % 3][0])
+        for p, (_, w) in zip(pages, want):
+            for kv, kv_want in zip(p, w):
+                assert all(torch.equal(a, b) for a, b in zip(kv, kv_want))
 
 
 def test_more_layers_than_a_launch_takes():

@@ -167,6 +167,69 @@ def test_few_rows_of_wide_stacks(hidden, rows, rings):
     test_steps(spec, rows, "native")
 
 
+DEEP = ModelSpec(name="t-deep", vocab_size=500, hidden_size=256,
+                 intermediate_size=14336, n_layers=2, n_heads=4, n_kv_heads=2,
+                 head_dim=64, max_seq_len=1024)
+
+
+@pytest.mark.parametrize("spec,rows,attention,one", [
+    (SWIGLU, 1, False, True), (SWIGLU, 6, False, True), (SWIGLU, 7, False, False),
+    (GELU, 6, False, True), (GELU, 8, False, False), (DEEP, 2, False, True),
+    (DEEP, 3, False, False), (SWIGLU, 1, True, False)],
+    ids=lambda v: getattr(v, "name", str(v)))
+@torch.no_grad()
+def test_which_steps_are_one_launch(spec, rows, attention, one, monkeypatch):
+    from bee2bee_amd import ops
+
+    W = ModelWeights(spec, DEV, torch.bfloat16).random_init(seed=3)
+    side = _Side(spec, W, DEV, torch.bfloat16, "native")
+    side.prompt(torch.arange(rows), [1] * rows)
+    if attention:
+        side.runner.decode_attn_fn = ops.attn_decode
+    taken, op = [], ops.decode_stack
+    monkeypatch.setattr(ops, "decode_stack", lambda *a, **k: (
+        taken.append(1), op(*a, **k))[1])
+    side.decode(torch.arange(rows), 1)
+    assert len(taken) == one
+
+
+@pytest.mark.parametrize("spec", [SWIGLU, GELU], ids=["swiglu", "gelu"])
+@torch.no_grad()
+def test_captured_steps_of_few_rows(spec, monkeypatch):
+    """One capture, replayed at lengths around a tile, 256 keys (what is not
+    split) and the table's end: as the same step is eagerly, to the bit, and as
+    it is launch by launch (the tolerance above)."""
+    from bee2bee_amd.engine.graphs import DecodeGraphs
+
+    W = ModelWeights(spec, DEV, torch.bfloat16).random_init(seed=3)
+    side = _Side(spec, W, DEV, torch.bfloat16, "native")
+    kv, runner = side.kv, side.runner
+    for t in [*kv.k_cache, *kv.v_cache]:
+        t.normal_()
+    graphs = DecodeGraphs(runner, 2, 64)
+    graphs.block_table.copy_(torch.randperm(600)[:128].int().view(2, 64))
+    held = [t.clone() for t in [*kv.k_cache, *kv.v_cache]]
+
+    def step(run, lens):
+        for t, h in zip([*kv.k_cache, *kv.v_cache], held):
+            t.copy_(h)
+        graphs.input_ids.copy_(torch.tensor([7, 11]))
+        graphs.seq_lens.copy_(torch.tensor(lens))
+        graphs.positions.copy_(torch.tensor(lens) - 1)
+        logits = run().clone()
+        return [logits, *(t.clone() for t in [*kv.k_cache, *kv.v_cache])]
+
+    for lens in ([255, 1], [256, 32], [257, 33], [1000, 1024], [2, 256]):
+        got = step(lambda: graphs.run(2), lens)
+        for a, b in zip(got, step(lambda: graphs._run(2), lens)):
+            assert torch.equal(a, b)
+        with monkeypatch.context() as m:
+            m.setattr(Runner, "_one_launch", lambda self, *a: False)
+            want = step(lambda: graphs._run(2), lens)
+        assert _rel(got[0], want[0]) <= 0.015
+        assert _rel(torch.stack(got[1:]), torch.stack(want[1:])) <= 0.015
+
+
 @torch.no_grad()
 def test_what_few_rows_take_and_refuse():
     """As steps of more rows do: tables and lengths of more rows than there are;
