@@ -223,14 +223,14 @@ rope_store_kernel(const TIN* q, long q_tok, T* q_out, long qo_tok, int H, const 
                   const TIN* __restrict__ v, long v_tok, int G, int D, int Dv,
                   int dims, const int* __restrict__ positions,
                   const float* __restrict__ cos_t,
-                  const float* __restrict__ sin_t, float q_mult,
+                  const float* __restrict__ sin_t, int table, float q_mult,
                   T* __restrict__ k_cache, T* __restrict__ v_cache, int bs,
                   const int* __restrict__ slot_mapping) {
     __shared__ float buf[4][RS_MAXD];
     const long t = blockIdx.x;
     const int wid = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const int pos = positions[t];
     const int half = dims / 2;
+    const long turn = dims ? turn_row(positions[t], table) * half : 0;
     const int slot = slot_mapping[t];
     if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
@@ -269,8 +269,8 @@ rope_store_kernel(const TIN* q, long q_tok, T* q_out, long qo_tok, int H, const 
                 ip = first ? i + half : i - half;
             }
             const float yp = nb[ip];
-            const float cs = cos_t[(long)pos * half + j];
-            const float sn = sin_t[(long)pos * half + j];
+            const float cs = cos_t[turn + j];
+            const float sn = sin_t[turn + j];
             y = first ? y * cs - yp * sn : y * cs + yp * sn;
         }
         stf(dst + i, y * mult);
@@ -573,7 +573,7 @@ extern "C" int launch_rope_store(
     const void* q, long q_tok, void* q_out, long qo_tok, int H, const void* k,
     long k_tok, const void* v, long v_tok, int G, int D, int Dv, int dims,
     int inter, const int* positions, const float* cos_t, const float* sin_t,
-    float q_mult, void* k_cache, void* v_cache, int bs,
+    int table, float q_mult, void* k_cache, void* v_cache, int bs,
     const int* slot_mapping, long T, int in_f32, int c, hipStream_t s) {
     if (D > RS_MAXD) return 1;
     if (T == 0) return 0;
@@ -581,7 +581,7 @@ extern "C" int launch_rope_store(
 #define RS_LAUNCH(TIN, TT, I)                                                 \
     rope_store_kernel<TIN, TT, I><<<grid, 256, 0, s>>>(                       \
         (const TIN*)q, q_tok, (TT*)q_out, qo_tok, H, (const TIN*)k, k_tok,    \
-        (const TIN*)v, v_tok, G, D, Dv, dims, positions, cos_t, sin_t,        \
+        (const TIN*)v, v_tok, G, D, Dv, dims, positions, cos_t, sin_t, table, \
         q_mult, (TT*)k_cache, (TT*)v_cache, bs, slot_mapping)
 #define RS_PICK(TIN, TT)                                                      \
     do {                                                                      \

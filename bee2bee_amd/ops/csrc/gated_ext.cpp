@@ -26,7 +26,7 @@ void launch_slice_rmsnorm(const void*, long, const float*, void*, long, int,
 void launch_gelu_erf(const void*, void*, long, int, hipStream_t);
 int launch_rope_store(const void*, long, void*, long, int, const void*, long,
                       const void*, long, int, int, int, int, int, const int*,
-                      const float*, const float*, float, void*, void*, int,
+                      const float*, const float*, int, float, void*, void*, int,
                       const int*, long, int, int, hipStream_t);
 int min_gru_segment_tokens();
 void launch_min_gru(const void*, long, const void*, long, const void*, long,
@@ -242,20 +242,22 @@ void rope_store(const Tensor& q, const Tensor& k, const Tensor& v,
     TORCH_CHECK(rope_dims >= 0 && rope_dims <= D && rope_dims % 2 == 0);
     TORCH_CHECK(positions.numel() == T && slot_mapping.numel() == T);
     const float *cp = nullptr, *sp = nullptr;
+    int table = 0;
     if (rope_dims > 0) {
         TORCH_CHECK(cos_t.has_value() && sin_t.has_value());
         check_f32(*cos_t, "cos");
         check_f32(*sin_t, "sin");
         TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == rope_dims / 2 &&
-                    sin_t->sizes() == cos_t->sizes());
+                    cos_t->size(0) >= 1 && sin_t->sizes() == cos_t->sizes());
         cp = cos_t->data_ptr<float>();
         sp = sin_t->data_ptr<float>();
+        table = (int)cos_t->size(0);
     }
     const int rc = launch_rope_store(
         q.data_ptr(), q.stride(0), q_out.data_ptr(), q_out.stride(0), H,
         k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), G, D, Dv,
         (int)rope_dims, interleaved ? 1 : 0, positions.data_ptr<int>(), cp,
-        sp, (float)q_mult, k_cache.data_ptr(), v_cache.data_ptr(), bs,
+        sp, table, (float)q_mult, k_cache.data_ptr(), v_cache.data_ptr(), bs,
         slot_mapping.data_ptr<int>(), T, in_f32, c, stream());
     TORCH_CHECK(rc == 0, "rope_store: head dim must be <= 512");
 }

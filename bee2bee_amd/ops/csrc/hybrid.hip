@@ -287,7 +287,7 @@ __global__ void latent_rope_store_kernel(
     T* __restrict__ q_rot, long q_tok_stride, long q_head_stride, int H,
     const T* __restrict__ kv, long kv_stride, const float* __restrict__ w,
     int C, int R, int dims, float eps, const int* __restrict__ positions,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table,
     T* __restrict__ cache, const int* __restrict__ slot_mapping) {
     __shared__ float red[16];
     const long t = blockIdx.x;
@@ -304,9 +304,9 @@ __global__ void latent_rope_store_kernel(
     for (int i = threadIdx.x; i < C; i += blockDim.x)
         stf(dst + i, ldf(row + i) * r * w[i]);
     const int half = dims / 2;
-    const int p = positions[t];
-    const float* cs = cos_t + (long)p * half;
-    const float* sn = sin_t + (long)p * half;
+    const long at = turn_row(positions[t], table) * half;
+    const float* cs = cos_t + at;
+    const float* sn = sin_t + at;
     for (int i = threadIdx.x; i < R; i += blockDim.x) {
         // pair j, its other coordinate ip, and whether i is the first of it
         const bool first = INTER ? (i & 1) == 0 : i < half;
@@ -481,7 +481,7 @@ qk_norm_rope_store_kernel(T* __restrict__ q, long q_tok, int H,
                           const float* __restrict__ wk, float eps, int dims,
                           const int* __restrict__ positions,
                           const float* __restrict__ cos_t,
-                          const float* __restrict__ sin_t,
+                          const float* __restrict__ sin_t, int table,
                           const float* __restrict__ q_mult,
                           T* __restrict__ k_cache, T* __restrict__ v_cache,
                           int bs, const int* __restrict__ slot_mapping,
@@ -489,8 +489,8 @@ qk_norm_rope_store_kernel(T* __restrict__ q, long q_tok, int H,
     __shared__ float buf[4][QKN_MAXD];
     const long t = blockIdx.x;
     const int wid = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const int pos = positions[t];
     const int half = dims / 2;
+    const long turn = dims ? turn_row(positions[t], table) * half : 0;
     const int slot = slot_mapping[t];
     if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
@@ -528,8 +528,8 @@ qk_norm_rope_store_kernel(T* __restrict__ q, long q_tok, int H,
                 const int j = i < half ? i : i - half;
                 const int pi = i < half ? i + half : i - half;
                 const float yp = nb[pi] * r * w[pi];
-                const float c = cos_t[(long)pos * half + j];
-                const float s = sin_t[(long)pos * half + j];
+                const float c = cos_t[turn + j];
+                const float s = sin_t[turn + j];
                 y = i < half ? y * c - yp * s : y * c + yp * s;
             }
             stf(dst + i, y * mul);
@@ -854,7 +854,7 @@ extern "C" void launch_delta_gates(float* qk, long qs, int NQ, int D,
 extern "C" int launch_qk_norm_rope_store(
     void* q, long q_tok, int H, const void* k, long k_tok, int G, int D,
     const float* wq, const float* wk, float eps, int dims,
-    const int* positions, const float* cos_t, const float* sin_t,
+    const int* positions, const float* cos_t, const float* sin_t, int table,
     const float* q_mult, void* k_cache, void* v_cache, int bs,
     const int* slot_mapping, const void* v, long v_tok, int Dv, long T,
     int f32, hipStream_t s) {
@@ -884,12 +884,12 @@ extern "C" int launch_qk_norm_rope_store(
     if (f32)
         qk_norm_rope_store_kernel<float><<<T, 256, 0, s>>>(
             (float*)q, q_tok, H, (const float*)k, k_tok, G, D, wq, wk, eps,
-            dims, positions, cos_t, sin_t, q_mult, (float*)k_cache,
+            dims, positions, cos_t, sin_t, table, q_mult, (float*)k_cache,
             (float*)v_cache, bs, slot_mapping, (const float*)v, v_tok, Dv);
     else
         qk_norm_rope_store_kernel<unsigned short><<<T, 256, 0, s>>>(
             (unsigned short*)q, q_tok, H, (const unsigned short*)k, k_tok, G,
-            D, wq, wk, eps, dims, positions, cos_t, sin_t, q_mult,
+            D, wq, wk, eps, dims, positions, cos_t, sin_t, table, q_mult,
             (unsigned short*)k_cache, (unsigned short*)v_cache, bs,
             slot_mapping, (const unsigned short*)v, v_tok, Dv);
     return 0;
@@ -898,14 +898,15 @@ extern "C" int launch_qk_norm_rope_store(
 extern "C" void launch_latent_rope_store(
     void* q_rot, long q_tok_stride, long q_head_stride, int H, const void* kv,
     long kv_stride, const float* w, int C, int R, int dims, float eps,
-    const int* positions, const float* cos_t, const float* sin_t, void* cache,
-    const int* slot_mapping, int inter, long T, int f32, hipStream_t s) {
+    const int* positions, const float* cos_t, const float* sin_t, int table,
+    void* cache, const int* slot_mapping, int inter, long T, int f32, hipStream_t s) {
     if (T == 0) return;
     const int th = 256;
 #define LRS_LAUNCH(TT, I)                                                     \
     latent_rope_store_kernel<TT, I><<<T, th, 0, s>>>(                         \
         (TT*)q_rot, q_tok_stride, q_head_stride, H, (const TT*)kv, kv_stride, \
-        w, C, R, dims, eps, positions, cos_t, sin_t, (TT*)cache, slot_mapping)
+        w, C, R, dims, eps, positions, cos_t, sin_t, table, (TT*)cache,       \
+        slot_mapping)
     if (f32 && inter) LRS_LAUNCH(float, true);
     else if (f32) LRS_LAUNCH(float, false);
     else if (inter) LRS_LAUNCH(unsigned short, true);

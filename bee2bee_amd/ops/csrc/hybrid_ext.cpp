@@ -28,8 +28,8 @@ void launch_canon_conv(const void*, const float*, void*, const int*,
                        int, int, int, hipStream_t);
 void launch_latent_rope_store(void*, long, long, int, const void*, long,
                               const float*, int, int, int, float, const int*,
-                              const float*, const float*, void*, const int*,
-                              int, long, int, hipStream_t);
+                              const float*, const float*, int, void*,
+                              const int*, int, long, int, hipStream_t);
 int launch_latent_attn(const void*, const void*, long, long, const void*,
                        long, const void*, const int*, int, const int*,
                        const int*, void*, float*, float*, int, int, int, int,
@@ -43,7 +43,7 @@ int lightning_segment_tokens();
 int launch_lightning(const void*, const void*, const void*, long,
                      const float*, float*, const int*, const int*, const int*,
                      float*, float*, int, int, int, int, int, int, int,
-                     const float*, const float*, int, float, hipStream_t);
+                     const float*, const float*, int, int, float, hipStream_t);
 void launch_short_conv(const void*, long, const float*, void*, const int*,
                        const int*, const int*, const int*, void*, long, int,
                        int, int, int, int, int, const float*, int,
@@ -60,7 +60,7 @@ void launch_delta_gates(float*, long, int, int, const void*, long,
                         float*, long, int, int, int, hipStream_t);
 int launch_qk_norm_rope_store(void*, long, int, const void*, long, int, int,
                               const float*, const float*, float, int,
-                              const int*, const float*, const float*,
+                              const int*, const float*, const float*, int,
                               const float*, void*, void*, int, const int*,
                               const void*, long, int, long, int, hipStream_t);
 int launch_delta_rule(const float*, const float*, long, const float*, long,
@@ -237,7 +237,7 @@ void latent_rope_store(Tensor& q_rot, const Tensor& kv, const Tensor& kv_norm,
     TORCH_CHECK(kv_norm.numel() == C);
     TORCH_CHECK(rope_dims >= 0 && rope_dims <= R && rope_dims % 2 == 0);
     TORCH_CHECK(cos_t.dim() == 2 && cos_t.size(1) == rope_dims / 2 &&
-                sin_t.sizes() == cos_t.sizes());
+                cos_t.size(0) >= 1 && sin_t.sizes() == cos_t.sizes());
     TORCH_CHECK(cache.is_contiguous() && cache.dim() == 3 &&
                 cache.size(2) == C + R);
     TORCH_CHECK(positions.numel() == T && slot_mapping.numel() == T);
@@ -246,7 +246,7 @@ void latent_rope_store(Tensor& q_rot, const Tensor& kv, const Tensor& kv_norm,
         (int)q_rot.size(1), kv.data_ptr(), kv.stride(0),
         kv_norm.data_ptr<float>(), C, R, (int)rope_dims, (float)eps,
         positions.data_ptr<int>(), cos_t.data_ptr<float>(),
-        sin_t.data_ptr<float>(), cache.data_ptr(),
+        sin_t.data_ptr<float>(), (int)cos_t.size(0), cache.data_ptr(),
         slot_mapping.data_ptr<int>(), interleaved ? 1 : 0, T, c, stream());
 }
 
@@ -351,8 +351,8 @@ Tensor linear_attn_impl(const Tensor& q, const Tensor& k, const Tensor& v,
                         const Tensor& decay, Tensor& state,
                         const Tensor& state_slots, const Tensor& cu,
                         const Tensor& positions, int64_t max_qlen, int form,
-                        const float* cos_t, const float* sin_t, int rdims,
-                        float k_scale) {
+                        const float* cos_t, const float* sin_t, int table,
+                        int rdims, float k_scale) {
     const int c = act_code(q, "q");
     check_f32(decay, "decay");
     check_f32(state, "state");
@@ -393,7 +393,7 @@ Tensor linear_attn_impl(const Tensor& q, const Tensor& k, const Tensor& v,
         decay.data_ptr<float>(), state.data_ptr<float>(),
         state_slots.data_ptr<int>(), cu.data_ptr<int>(),
         positions.data_ptr<int>(), out.data_ptr<float>(), wsp, (int)n_seg, B,
-        H, D, Dv, c, form, cos_t, sin_t, rdims, k_scale, stream());
+        H, D, Dv, c, form, cos_t, sin_t, table, rdims, k_scale, stream());
     TORCH_CHECK(rc == 0, "linear attention: key dim must be <= 256");
     return out;
 }
@@ -403,7 +403,7 @@ Tensor lightning_attn(const Tensor& q, const Tensor& k, const Tensor& v,
                       const Tensor& state_slots, const Tensor& cu,
                       const Tensor& positions, int64_t max_qlen) {
     return linear_attn_impl(q, k, v, decay, state, state_slots, cu, positions,
-                            max_qlen, 0, nullptr, nullptr, 0, 1.f);
+                            max_qlen, 0, nullptr, nullptr, 0, 0, 1.f);
 }
 
 Tensor retention_attn(const Tensor& q, const Tensor& k, const Tensor& v,
@@ -414,6 +414,7 @@ Tensor retention_attn(const Tensor& q, const Tensor& k, const Tensor& v,
                       const Tensor& cu, const Tensor& positions,
                       int64_t max_qlen) {
     const float *cp = nullptr, *sp = nullptr;
+    int table = 0;
     TORCH_CHECK(rope_dims >= 0 && rope_dims % 2 == 0 &&
                 rope_dims <= q.size(2));
     if (rope_dims > 0) {
@@ -421,12 +422,13 @@ Tensor retention_attn(const Tensor& q, const Tensor& k, const Tensor& v,
         check_f32(*cos_t, "cos");
         check_f32(*sin_t, "sin");
         TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == rope_dims / 2 &&
-                    sin_t->sizes() == cos_t->sizes());
+                    cos_t->size(0) >= 1 && sin_t->sizes() == cos_t->sizes());
         cp = cos_t->data_ptr<float>();
         sp = sin_t->data_ptr<float>();
+        table = (int)cos_t->size(0);
     }
     return linear_attn_impl(q, k, v, decay, state, state_slots, cu, positions,
-                            max_qlen, 1, cp, sp, (int)rope_dims,
+                            max_qlen, 1, cp, sp, table, (int)rope_dims,
                             (float)k_scale);
 }
 
@@ -648,14 +650,16 @@ void qk_norm_rope_store(Tensor& q, const Tensor& k, const Tensor& q_norm,
                 q_mult.numel() == H);
     TORCH_CHECK(rope_dims >= 0 && rope_dims % 2 == 0 && rope_dims <= D);
     const float *cp = nullptr, *sp = nullptr;
+    int table = 0;
     if (rope_dims > 0) {
         TORCH_CHECK(cos_t.has_value() && sin_t.has_value());
         check_f32(*cos_t, "cos");
         check_f32(*sin_t, "sin");
         TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == rope_dims / 2 &&
-                    sin_t->sizes() == cos_t->sizes());
+                    cos_t->size(0) >= 1 && sin_t->sizes() == cos_t->sizes());
         cp = cos_t->data_ptr<float>();
         sp = sin_t->data_ptr<float>();
+        table = (int)cos_t->size(0);
     }
     int Dv = D;
     const void* vp = nullptr;
@@ -679,7 +683,7 @@ void qk_norm_rope_store(Tensor& q, const Tensor& k, const Tensor& q_norm,
     const int rc = launch_qk_norm_rope_store(
         q.data_ptr(), q.stride(0), H, k.data_ptr(), k.stride(0), G, D,
         q_norm.data_ptr<float>(), k_norm.data_ptr<float>(), (float)eps,
-        (int)rope_dims, positions.data_ptr<int>(), cp, sp,
+        (int)rope_dims, positions.data_ptr<int>(), cp, sp, table,
         q_mult.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
         (int)k_cache.size(2), slot_mapping.data_ptr<int>(), vp, v_tok, Dv, T,
         c, stream());

@@ -524,7 +524,8 @@ __global__ void __launch_bounds__(LI_COLS * LI_GROUPS)
 lightning_kernel(const T* __restrict__ q, const T* __restrict__ k,
                  const T* __restrict__ v, long tok_stride,
                  const float* __restrict__ cos_t,
-                 const float* __restrict__ sin_t, int rdims, float k_scale,
+                 const float* __restrict__ sin_t, int table, int rdims,
+                 float k_scale,
                  const float* __restrict__ decay,
                  float* __restrict__ state,        // [slots, H, D, Dv]
                  const int* __restrict__ state_slots,
@@ -574,7 +575,8 @@ lightning_kernel(const T* __restrict__ q, const T* __restrict__ k,
             const float* cs = nullptr;
             const float* sn = nullptr;
             if (FORM == 1 && rdims > 0) {
-                const long pr = (long)positions[t0 + tt] * (rdims / 2);
+                const long pr =
+                    turn_row(positions[t0 + tt], table) * (rdims / 2);
                 cs = cos_t + pr;
                 sn = sin_t + pr;
             }
@@ -1315,8 +1317,8 @@ extern "C" int launch_latent_attn_mfma(
     lightning_kernel<TT, N, MODE, FORM>                                       \
         <<<GRID, LI_COLS * LI_GROUPS, 0, s>>>(                                \
             (const TT*)q, (const TT*)k, (const TT*)v, tok_stride, cos_t,      \
-            sin_t, rdims, k_scale, decay, state, state_slots, cu, positions,  \
-            out, ws, B, H, D, Dv)
+            sin_t, table, rdims, k_scale, decay, state, state_slots, cu,      \
+            positions, out, ws, B, H, D, Dv)
 
 #define LI_CASE(N)                                                            \
     case N:                                                                   \
@@ -1336,8 +1338,8 @@ extern "C" int launch_latent_attn_mfma(
 template <typename TT, int FORM>
 static int lightning_dispatch(const void* q, const void* k, const void* v,
                               long tok_stride, const float* cos_t,
-                              const float* sin_t, int rdims, float k_scale,
-                              const float* decay,
+                              const float* sin_t, int table, int rdims,
+                              float k_scale, const float* decay,
                               float* state, const int* state_slots,
                               const int* cu, const int* positions, float* out,
                               float* ws, int n_seg, int B, int H, int D,
@@ -1367,12 +1369,14 @@ extern "C" int launch_lightning(const void* q, const void* k, const void* v,
                                 float* out, float* ws, int n_seg, int B,
                                 int H, int D, int Dv, int f32, int form,
                                 const float* cos_t, const float* sin_t,
-                                int rdims, float k_scale, hipStream_t s) {
+                                int table, int rdims, float k_scale,
+                                hipStream_t s) {
     if (B == 0) return 0;
 #define LI_DISPATCH(TT, FORM)                                                 \
-    lightning_dispatch<TT, FORM>(q, k, v, tok_stride, cos_t, sin_t, rdims,    \
-                                 k_scale, decay, state, state_slots, cu,      \
-                                 positions, out, ws, n_seg, B, H, D, Dv, s)
+    lightning_dispatch<TT, FORM>(q, k, v, tok_stride, cos_t, sin_t, table,    \
+                                 rdims, k_scale, decay, state, state_slots,   \
+                                 cu, positions, out, ws, n_seg, B, H, D, Dv,  \
+                                 s)
     if (form == 0)
         return f32 ? LI_DISPATCH(float, 0) : LI_DISPATCH(unsigned short, 0);
     return f32 ? LI_DISPATCH(float, 1) : LI_DISPATCH(unsigned short, 1);

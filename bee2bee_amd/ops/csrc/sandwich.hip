@@ -170,14 +170,15 @@ rope_unit_store_kernel(T* __restrict__ q, long q_tok, int H,
                        int Dv, float eps, int dims,
                        const int* __restrict__ positions,
                        const float* __restrict__ cos_t,
-                       const float* __restrict__ sin_t, float q_mult,
+                       const float* __restrict__ sin_t, int table,
+                       float q_mult,
                        T* __restrict__ k_cache, T* __restrict__ v_cache,
                        int bs, const int* __restrict__ slot_mapping) {
     __shared__ float buf[4][RU_MAXD];
     const long t = blockIdx.x;
     const int wid = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const int pos = positions[t];
     const int half = dims / 2;
+    const long turn = dims ? turn_row(positions[t], table) * half : 0;
     const int slot = slot_mapping[t];
     if (slot < 0) return;            // no such position
     const long blk = slot / bs, off = slot % bs;
@@ -211,8 +212,8 @@ rope_unit_store_kernel(T* __restrict__ q, long q_tok, int H,
             if (i < dims) {
                 const int j = i < half ? i : i - half;
                 const float yp = nb[i < half ? i + half : i - half];
-                const float cs = cos_t[(long)pos * half + j];
-                const float sn = sin_t[(long)pos * half + j];
+                const float cs = cos_t[turn + j];
+                const float sn = sin_t[turn + j];
                 y = i < half ? y * cs - yp * sn : y * cs + yp * sn;
             }
         }
@@ -337,7 +338,7 @@ extern "C" int launch_add_group_rmsnorm(float* resid, const void* y,
 extern "C" int launch_rope_unit_store(
     void* q, long q_tok, int H, const void* k, long k_tok, const void* v,
     long v_tok, int G, int D, int Dv, float eps, int dims,
-    const int* positions, const float* cos_t, const float* sin_t,
+    const int* positions, const float* cos_t, const float* sin_t, int table,
     float q_mult, void* k_cache, void* v_cache, int bs,
     const int* slot_mapping, long T, int f32, hipStream_t s) {
     if (D > RU_MAXD) return 1;
@@ -346,13 +347,13 @@ extern "C" int launch_rope_unit_store(
     if (f32)
         rope_unit_store_kernel<float><<<grid, 256, 0, s>>>(
             (float*)q, q_tok, H, (const float*)k, k_tok, (const float*)v,
-            v_tok, G, D, Dv, eps, dims, positions, cos_t, sin_t, q_mult,
+            v_tok, G, D, Dv, eps, dims, positions, cos_t, sin_t, table, q_mult,
             (float*)k_cache, (float*)v_cache, bs, slot_mapping);
     else
         rope_unit_store_kernel<unsigned short><<<grid, 256, 0, s>>>(
             (unsigned short*)q, q_tok, H, (const unsigned short*)k, k_tok,
             (const unsigned short*)v, v_tok, G, D, Dv, eps, dims, positions,
-            cos_t, sin_t, q_mult, (unsigned short*)k_cache,
+            cos_t, sin_t, table, q_mult, (unsigned short*)k_cache,
             (unsigned short*)v_cache, bs, slot_mapping);
     return 0;
 }

@@ -20,8 +20,8 @@ int launch_add_group_rmsnorm(float*, const void*, const float*, const float*,
                              int, hipStream_t);
 int launch_rope_unit_store(void*, long, int, const void*, long, const void*,
                            long, int, int, int, float, int, const int*,
-                           const float*, const float*, float, void*, void*,
-                           int, const int*, long, int, hipStream_t);
+                           const float*, const float*, int, float, void*,
+                           void*, int, const int*, long, int, hipStream_t);
 void launch_polynorm(const void*, const float*, void*, long, int, float, int,
                      hipStream_t);
 void launch_silu_glu(const void*, void*, long, long, int, hipStream_t);
@@ -151,14 +151,16 @@ void rope_unit_store(Tensor& q, const Tensor& k, const Tensor& v, double eps,
                 v.stride(1) == Dv);
     TORCH_CHECK(rope_dims >= 0 && rope_dims % 2 == 0 && rope_dims <= D);
     const float *cp = nullptr, *sp = nullptr;
+    int table = 0;
     if (rope_dims > 0) {
         TORCH_CHECK(cos_t.has_value() && sin_t.has_value());
         check_f32(*cos_t, "cos");
         check_f32(*sin_t, "sin");
         TORCH_CHECK(cos_t->dim() == 2 && cos_t->size(1) == rope_dims / 2 &&
-                    sin_t->sizes() == cos_t->sizes());
+                    cos_t->size(0) >= 1 && sin_t->sizes() == cos_t->sizes());
         cp = cos_t->data_ptr<float>();
         sp = sin_t->data_ptr<float>();
+        table = (int)cos_t->size(0);
     }
     TORCH_CHECK(k_cache.is_cuda() && k_cache.is_contiguous() &&
                 k_cache.dim() == 4 && k_cache.size(1) == G &&
@@ -173,8 +175,8 @@ void rope_unit_store(Tensor& q, const Tensor& k, const Tensor& v, double eps,
     const int rc = launch_rope_unit_store(
         q.data_ptr(), q.stride(0), H, k.data_ptr(), k.stride(0), v.data_ptr(),
         v.stride(0), G, D, Dv, (float)eps, (int)rope_dims,
-        positions.data_ptr<int>(), cp, sp, (float)q_mult, k_cache.data_ptr(),
-        v_cache.data_ptr(), (int)k_cache.size(2),
+        positions.data_ptr<int>(), cp, sp, table, (float)q_mult,
+        k_cache.data_ptr(), v_cache.data_ptr(), (int)k_cache.size(2),
         slot_mapping.data_ptr<int>(), T, c, stream());
     TORCH_CHECK(rc == 0, "rope_unit_store: head dim must be <= 512");
 }

@@ -192,3 +192,56 @@ def test_latent_attention_decode_step(dtype, H, C, R, window):
     o2 = ref.latent_attn(q_abs, q_rot, gate, cache, m["bt"], m["pos"],
                          m["seq"], m["cu"], window, 0.3)
     torch.testing.assert_close(o1.float(), o2.float(), **tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_positions_that_the_rotation_has_not(dtype):
+    """The tables' first row for positions before them, their last for those
+    behind, in each kernel that rotates."""
+    T, H, G, D, C, R, dims, rows = 6, 4, 2, 64, 128, 32, 32, 40
+    g = torch.Generator(device=DEV).manual_seed(3)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device=DEV).to(dtype)
+
+    angles = torch.rand(rows + 24, dims // 2, generator=g, device=DEV) * 6
+    cos, sin = angles.cos()[:rows], angles.sin()[:rows]
+    pos = torch.tensor([5, 39, 40, 63, -2 ** 31, 2 ** 31 - 1],
+                       dtype=torch.int32, device=DEV)
+    slots = torch.arange(T, dtype=torch.int32, device=DEV)
+    q, k, v = rand(T, H, D), rand(T, G, D), rand(T, G, D)
+    kv, q_rot, w = rand(T, C + R), rand(T, H, R), torch.ones(D, device=DEV)
+    mult, decay = torch.ones(H, device=DEV), torch.full((H,), 0.9, device=DEV)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)
+
+    heads = [t.repeat_interleave(H // G, 1) for t in (k, v)]
+
+    def latent(p, inter):
+        rot, cache = q_rot.clone(), torch.zeros(1, 16, C + R, device=DEV,
+                                                dtype=dtype)
+        ops.latent_rope_store(rot, kv, torch.ones(C, device=DEV), 1e-5, C, dims,
+                              p, cos, sin, cache, slots, inter)
+        return rot, cache
+
+    def stored(op):
+        pages = [torch.zeros(1, G, 16, D, device=DEV, dtype=dtype)
+                 for _ in range(2)]
+        rot = q.clone()
+        op(rot, *pages)
+        return rot, *pages
+
+    for op in (
+            lambda p: latent(p, False), lambda p: latent(p, True),
+            lambda p: stored(lambda x, *c: ops.qk_norm_rope_store(
+                x, k, w, w, 1e-5, dims, p, cos, sin, mult, *c, slots, v)),
+            lambda p: stored(lambda x, *c: ops.rope_unit_store(
+                x, k, v, 1e-5, dims, p, cos, sin, 1.0, *c, slots)),
+            lambda p: stored(lambda x, *c: ops.rope_store(
+                x, k, v, x, dims, False, p, cos, sin, 1.0, *c, slots)),
+            lambda p: stored(lambda x, *c: ops.rope_store(
+                x, k, v, x, dims, True, p, cos, sin, 1.0, *c, slots)),
+            lambda p: [ops.retention_attn(
+                q, *heads, decay, dims, cos, sin, 1.0,
+                torch.zeros(1, H, D, D, device=DEV), slots[:1], cu, p, T)]):
+        for a, b in zip(op(pos), op(pos.clamp(0, rows - 1))):
+            assert torch.equal(a, b)
