@@ -4,7 +4,8 @@
 constexpr int DS_WGS = 256;                    // workgroups, a CU each
 constexpr int DS_CLAIMS = DS_WGS + 8 * 32;     // words: a number's, 8 counters
 constexpr int DS_STATE = 64;                   // words: progress; at 32: given up
-constexpr int DS_PATIENCE = 1 << 22;           // polls, of a microsecond or more
+constexpr int DS_PATIENCE = 1 << 22;           // polls, of half a microsecond or
+                                               // more
 constexpr int DS_LAYERS = 31;                  // of a launch: arguments of 4 KB
 constexpr int DS_LAYER_NORM = 1024;            // layer norm: columns at most
 constexpr int DS_ROWS = 8;
@@ -35,7 +36,8 @@ struct StackHead {
     int stride, new_kv, att, o, up, down;    // (queries at 0)
     int turns, pages, area;         // in LDS (launch_decode_stack)
     int turn_rows;                  // of cos_t and sin_t
-    int patience;                   // polls without progress, then given up
+    int patience;                   // 2^n - 1: a wait looks for progress every 2^n
+                                    // polls, and is given up if there is none
     unsigned* words;
     unsigned* parts;                // [M * nkv, Z, G, hd / 16, 18]
     unsigned* claims;               // [DS_CLAIMS]

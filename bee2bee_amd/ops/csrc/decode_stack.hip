@@ -293,29 +293,26 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     if (lane == 0) seen[wid] = DS_EMPTY;
     ds_barrier();                              // (0) all of it is there
 
-    // Has this wait lasted long enough, or has another one?
-    auto enough = [&](int& polls) __attribute__((always_inline)) {
-        unsigned* const state = DS_PTR(state);
-        bool end =
-            ds_same(__hip_atomic_load(&gone, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_WORKGROUP)) ||
-            (unsigned)ds_same(ds_load4(state + 32)) != DS_EMPTY;
-        if (!end && polls >= DS_INT(patience)) {
-            const unsigned now = ds_same(ds_load4(state));
-            end = now == (unsigned)ds_same(seen[wid]);
-            if (lane == 0) seen[wid] = now;
-            polls = 0;
+    // Has this wait lasted long enough, or has another one? (Lane by lane: scalar
+    // registers are what the kernel has too few of. With scalar values a step of six
+    // layers takes 2 us more, for code that does not run.)
+    auto enough = [&](int polls) __attribute__((always_inline)) {
+        typedef __attribute__((address_space(1))) unsigned* global;
+        unsigned* const state = (unsigned*)(global)told_s.state;
+        bool end = __hip_atomic_load(&gone, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP) ||
+                   ds_load4(state + 32) != DS_EMPTY;
+        if ((polls & told_s.patience) == 0) {
+            const unsigned now = ds_load4(state);
+            end = end || now == seen[wid];
+            seen[wid] = now;
         }
-        if (end && lane == 0) {
-            __hip_atomic_store(&gone, 1, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (end) {
+            gone = 1;
             __hip_atomic_store(state + 32, 0u, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-            if (int* const status = DS_PTR(status))
-                __hip_atomic_store(status, 1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_SYSTEM);
         }
-        return end;
+        return (bool)__any(end);
     };
     // Are all lanes' words there? If not, some clocks are left to the others
     // before they are asked for again: eight waves that ask without a pause keep
@@ -472,11 +469,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             if (M > 2 && Q <= 256) rows(std::integral_constant<int, 2>());
             else rows(std::integral_constant<int, 8>());
             return scale;
-        };
-        auto got_on = [&]() __attribute__((always_inline)) {
-            if (lane == 0)
-                __hip_atomic_fetch_add(DS_PTR(state), 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
         };
         bool passed = false;
         int nc = 1, parts = -1;
@@ -672,7 +664,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                     if (start && i == 0 && q == n - 1) decide();
                     if (own) octet(l, k, c + q * DS_WGS, i, q, bias, norm, dst);
                     else ds_barrier();
-                    if (nc > 1) got_on();
                 }
             }
             if (k < 3) fetch(l, k + 1);
@@ -727,7 +718,6 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 for (int i = 0; i < parts; ++i) {
                     ds_barrier();              // (A)
                     ds_barrier();              // (B)
-                    if (nc > 1) got_on();
                 }
             }
             if (++k == 4) k = 0, ++l;
@@ -983,6 +973,12 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     const unsigned slot_end = (wid + 1) * DS_RING * 1024;
     // rows of w 4 (lg & 1) .. + 3, input row lj; places of K apart
     const bool keeps = lj < M && (li >> 3) == (lg >> 1);
+    // (told by a wave that the others do not wait for)
+    auto got_on = [&]() __attribute__((always_inline)) {
+        if (tid == 0)
+            __hip_atomic_fetch_add(told_s.state, 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    };
     // number c's octets of product k, whose first steps are on their way
     auto product = [&](int k, int c) __attribute__((always_inline)) {
         const int n = planned(k, 1) & 0xffff;
@@ -1041,6 +1037,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 *reinterpret_cast<f32x4*>(
                     &part[buf][wid][li >> 3][lj][(lg & 1) * 4]) = acc;
             ds_barrier();
+            if (__builtin_expect(gnc > 1, 0)) got_on();
             buf ^= 1;
             acc = f32x4{0.f, 0.f, 0.f, 0.f};
         }
@@ -1067,7 +1064,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
     long i_base = 0;
     auto attention = [&](int l, int it) __attribute__((always_inline)) {
         const int bs = DS_INT(bs);
-        if (it != i_at) {
+        if (__builtin_expect(it != i_at, 0)) {
             i_at = it;
             i_z = it % DS_INT(Z);
             i_m = it / DS_INT(Z) / DS_INT(nkv);
@@ -1220,7 +1217,8 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
                 *reinterpret_cast<unsigned long*>(fresh_at(first, of) + e2) =
                     fresh_word;
 #pragma unroll 1
-                for (unsigned b = mine & (mine - 1); b; b &= b - 1) {
+                for (unsigned b = mine & (mine - 1); __builtin_expect(b, 0);
+                     b &= b - 1) {
                     const int n = __builtin_ctz(b);
                     polls = 0;
                     do fresh_word = ds_load(fresh_of(n));
@@ -1424,6 +1422,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             }
         }
         ds_barrier();                          // (B): the area is free again
+        if (__builtin_expect(gnc > 1, 0)) got_on();
     };
     // A query head's splits, added up by a wave for 16 of its columns: two a lane,
     // eight lanes a split. Their words are left as they were found, for the next
@@ -1461,7 +1460,7 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
             for (int u = 0; u < U; ++u)
                 ok = ok && ds_there(v[u]) && ds_there(e[u]);
         } while (again(ok, polls));
-        if (!__all(ok)) return;
+        if (__builtin_expect(!__all(ok), 0)) return;
         auto empty = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -1560,6 +1559,9 @@ __global__ __launch_bounds__((DS_WAVES + 1) * 64) void decode_stack_kernel(
         if (++k == 4) k = 0, ++l;
     }
     ds_wait<0>();                              // nothing lands in LDS later
+    if (gone && lane == 0 && told_s.status)
+        __hip_atomic_store(told_s.status, 1, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // LDS of the rings; of the rows of `K` columns or the attention's tiles; of the
@@ -1603,7 +1605,7 @@ extern "C" int launch_decode_stack(const StackArgs* args, int hd, int fp8,
     if (wgs < 1 || wgs > 2 * DS_WGS || (hd != 64 && hd != 128)) return 1;
     if (a.nkv < 1 || a.nq != a.G * a.nkv || a.G > 16 || a.Z < 1) return 1;
     if (a.items != a.M * a.nkv * a.Z) return 1;
-    if (a.Z > DS_SPLITS || !(a.scale > 0.f) || a.patience < 1) return 1;
+    if (a.Z > DS_SPLITS || !(a.scale > 0.f) || a.patience < 31) return 1;
     int deepest = 0;
     for (int k = 0; k < 4; ++k) {
         const long K = a.K[k];

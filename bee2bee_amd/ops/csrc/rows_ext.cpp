@@ -383,7 +383,8 @@ Tensor decode_stack(const Tensor& x,
             work[(long)i * DS_CLAIMS + c].zero_();
             work[(long)i * DS_CLAIMS + DS_WGS + c % 8 * 32].add_(1);
         }
-    a.patience = (int)patience;
+    a.patience = 31;                           // (see decode_stack.h)
+    while (a.patience < patience - 1) a.patience = a.patience * 2 + 1;
     if (status.has_value()) {
         TORCH_CHECK(status->device().is_cpu() && status->numel() == 1 &&
                     status->scalar_type() == torch::kInt32 &&
