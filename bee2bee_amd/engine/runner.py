@@ -102,11 +102,17 @@ class Runner:
     def _few_on_rings(self, rows: int) -> bool:
         """Steps of few rows that run like those of some tens: of wide stacks,
         from where a row more costs more than the launches that it saves. Time of
-        a step of 8 layers, on rows_linear over on the rings:
-          hidden 3584  8 / 9 / 10 / 16 rows   1.00 / 1.03 / 1.06 / 1.10
-          4096         8 / 9 / 10 / 16        0.97 / 1.02 / 1.03 / 1.06
-          3072         8 / 11 / 13 / 16       0.98 / 0.99 / 1.01 / 1.03
-          2048         8 / 10 / 12 / 16       0.88 / 0.95 / 0.97 / 0.99"""
+        a step of 8 layers, 200 keys, on rows_linear over on the rings:
+          hidden 8192  7 / 8 / 9 / 16 rows    1.03 / 1.04 / 1.05 / 1.09
+          5120         7 / 8 / 9 / 16         1.08 / 1.09 / 1.08 / 1.11
+          4096         7 / 8 / 9 / 16         0.98 / 0.99 / 1.05 / 1.08
+          3584         7 / 8 / 9 / 16         1.01 / 1.02 / 1.08 / 1.12
+          3072         8 / 9 / 10 / 11 / 12   1.01 / 1.03 / 1.04 / 1.05 / 1.05
+          2816         8 / 10 / 12 / 16       0.97 / 1.03 / 1.06 / 1.07
+          2560         8 / 10 / 12 / 16       0.93 / 1.04 / 1.04 / 1.07
+          2048         8 / 10 / 12 / 16       0.87 / 0.96 / 0.98 / 1.00
+        The lines are from before the kernels between the rings' products took 10
+        to 15% less time; a few rows below them would gain now."""
         hidden = self.spec.hidden_size
         return (self._mid_dims and hidden >= 3072
                 and rows > (8 if hidden > 3072 else 11))
@@ -116,14 +122,18 @@ class Runner:
         """Decode steps whose layers are one launch (ops.decode_stack); a tensor-
         parallel rank's rows are reduced between its products. What it saves,
         about 2 us a launch, is a layer's; what passes between its workgroups
-        grows with the rows. Time of a step of 8 layers (of 6: 768 columns),
-        launch by launch over one launch:
-          4096 columns, 1 / 2 rows       1.14 / 1.10
-          3584 columns, 1 / 2            1.10 / 1.08
-          3072 columns, 1 / 3 / 4        1.09 / 1.08 / 1.07
-          2048 columns, 1 / 3 / 4        1.15 / 1.12 / 1.11
-          768 columns, 1 / 4 / 6 / 8     1.03 / 1.02 / 1.01 / 1.00
-          768 columns, layer norm, 1 / 4 / 6 / 8   1.21 / 1.16 / 1.03 / 1.00"""
+        grows with the rows, of which a stack takes as many as its deepest product
+        leaves room for in LDS (8192 deep 4, 14336 and 18944 two). Time of a
+        step of 8 layers (of 6: distilgpt2), launch by launch over one launch,
+        1000 keys (5120 columns and fewer than 2048: 300):
+          5120 columns, 1 / 2 rows       1.16 / 1.17
+          4096 columns, 1 / 2            1.13 / 1.10
+          3072 columns, 1 / 2 / 4        1.14 / 1.13 / 1.07
+          2048 columns, 1 / 2 / 4        1.14 / 1.14 / 1.11
+          768 columns, 1 / 2 / 4 / 6     1.07 / 1.02 / 1.07 / 1.05
+          1024 columns, layer norm, 1 / 2 / 4 / 6   1.26 / 1.22 / 1.18 / 1.07
+          768 columns, layer norm, 1 / 2 / 4 / 6    1.23 / 1.18 / 1.16 / 1.04
+        768 columns at 8 rows: 1.00, both."""
         s = self.spec
         return (x.is_cuda and self.decode_attn_fn is None and self._mid_dims
                 and ops.few_rows(x) and self.layer_lo < self.layer_hi

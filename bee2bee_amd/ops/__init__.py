@@ -11,8 +11,9 @@ decode attention, MFMA flash prefill attention, SwiGLU, top-k gating, grouped
 expert GEMM, projections with what stands around them. Other projection GEMMs go
 through hipBLASLt via torch.nn.functional.linear.
 
-Which projections are whose is measured: decode steps of one to six rows are one
-launch of decode_stack.hip; else up to 16 rows (`few_rows`; logits: `head_rows`) the
+Which projections are whose is measured: decode steps of a few rows (one to six in
+small stacks, two in deep ones: `stack_rows`) are one launch of decode_stack.hip;
+else up to 16 rows (`few_rows`; logits: `head_rows`) the
 kernels of linear_rows.hip, one launch for norm, product and what follows; 17 to 256
 rows, of wide stacks fewer (`mid_rows`, `mid_shape`, `mid_gated`) linear_mid.hip,
 split over K or activated; more rows linear_wide.hip where `wide_plan` says so:

@@ -9,8 +9,8 @@
 // stack; weights depend on nothing, so the next product's are asked for under
 // the last steps of this one, and what crosses the chip between products are a
 // few KB of rows. A step with its logits, us, launch by launch / in one: 6 layers
-// of 768 columns, 300 keys 213 / 171; 8 of 2048, 1000 keys 413 / 357; 8 of 4096,
-// 3000 keys 924 / 820; 8 of 3584, two rows of 24000 keys 1057 / 1003.
+// of 768 columns, 300 keys 213 / 172; 8 of 2048, 1000 keys 412 / 360; 8 of 4096,
+// 3000 keys 924 / 810; 8 of 3584, two rows of 24000 keys 1058 / 979.
 //  * Rows pass from workgroup to workgroup as words that say themselves whether
 //    they are there: buffers are filled with DS_EMPTY (a NaN) before, a word is
 //    stored once, and readers load it until it is something else. Every such
