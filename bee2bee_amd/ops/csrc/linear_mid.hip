@@ -8,13 +8,17 @@
 //  rows    bf16, with bias and tanh-gelu where wanted (the output head, the
 //          feed-forward of the GPT-2 family).
 //
-// Bound by reading the weights once, up to about 128 rows; beyond, a CU draws 38
-// to 40 GB/s of weights and input rows together at any number of rows (from L2
-// alone it draws 120; at 200 rows a step takes 1900 clocks, of which products
-// 900). Neither halves that read and multiply in turn (200 rows 3 to 7% faster,
-// fewer 2 to 15% slower), nor weights in registers and the input in all of LDS,
-// nor tiles of 128 rows of w in turns with three buffers of both changed that by
-// more. A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
+// Bound by reading the weights once, up to about 128 rows; beyond, by the steps of
+// the four waves that load the input: at 200 rows 2200 clocks, of which products
+// 900; their seven loads wait up to 1000 for the memory pipe, and the other four
+// waves at the barrier for them. So a step finds out as little as it can: the two
+// kinds of waves have loops of their own, in which the number of loads under way
+// is known (us, with both in one loop / as now: 2x14336x4096 68.6 / 63.4 at 200
+// rows, 81.8 / 72.5 at 256, 51.2 / 50.3 at 128; 4096x14336 38.9 / 36.4 at 200;
+// 2x18944x3584 122 / 107; fewer rows within 2%). Loads spread between the products
+// changed nothing, nor did halves that read and multiply in turn, weights in
+// registers and the input in all of LDS, or tiles of 128 rows of w in turns with
+// three buffers of both. A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
 // workgroup's rows of w, and by all input rows. Four waves fill the one, four
 // the other, straight from memory (global_load_lds: no registers, so 100 KB of
 // loads are under way in each CU), and all eight multiply: the fragments of the
@@ -38,6 +42,8 @@
 // The library's figures are at the rules in ops/__init__.py.
 #include "common.h"
 
+#include <type_traits>
+
 enum { LM_PARTS = 0, LM_GATED = 1, LM_ROWS = 2 };
 
 DEV_INLINE unsigned lm_lds(const void* p) {
@@ -57,16 +63,16 @@ DEV_INLINE void lm_load(const void* base, unsigned off, unsigned to) {
                      "global_load_lds_dwordx4 %0, %1"
                      ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
 }
-// until at most `left` stages (R at most) of PER loads each are under way
-template <int PER, int R>
+// until at most `left` stages, of LO to HI, of PER loads each are under way
+template <int PER, int LO, int HI>
 DEV_INLINE void lm_wait(int left) {
-    if constexpr (R == 0) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (HI <= LO) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (HI > 0 ? HI : 0))
+                     : "memory");
     } else {
-        if (left >= R)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * R) : "memory");
-        else
-            lm_wait<PER, R - 1>(left);
+        constexpr int MID = (LO + HI + 1) / 2;
+        if (left >= MID) lm_wait<PER, MID, HI>(left);
+        else lm_wait<PER, LO, MID - 1>(left);
     }
 }
 
@@ -132,31 +138,35 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     const unsigned to0 = lm_lds(smem) +
                          (of_w ? wid * NLW * 1024
                                : DW * WB + (wid - 4) * NLX * 1024);
+    const char* at = src + (long)(c0 + rot) * 128;     // the next stage's
     int lk = rot, lleft = n, lgrp = g, lslot = 0;
-    auto issue = [&]() {                       // the next stage's loads
-        const char* b = src + (long)(c0 + lk) * 128;
-        if (of_w) {
+    auto issue = [&](auto of) {                // its loads
+        constexpr bool W = decltype(of)::value;
+        if (W || MT > 1 || wid < 6)            // (MT 1: two waves' are all)
 #pragma unroll
-            for (int j = 0; j < NLW; ++j)
-                lm_load<true>(b, off[j], to0 + lslot * WB + j * 1024);
-            if (++lslot == DW) lslot = 0;
-        } else {
-            // (MT 1: two waves' loads are all)
-            if (MT > 1 || wid < 6)
-#pragma unroll
-            for (int j = 0; j < NLX; ++j)
-                lm_load<false>(b, off[j], to0 + lslot * XB + j * 1024);
-            if (++lslot == DX) lslot = 0;
+            for (int j = 0; j < (W ? NLW : NLX); ++j)
+                lm_load<W>(at, off[j], to0 + lslot * (W ? WB : XB) + j * 1024);
+        if (++lslot == (W ? DW : DX)) lslot = 0;
+        at += 128;
+        if (++lk == n) {
+            lk = 0;
+            at -= (long)n * 128;
         }
-        if (++lk == n) lk = 0;
-        if (WK == 1 && --lleft == 0) {
+        if (W && WK == 1 && --lleft == 0) {
             lleft = n;
             lgrp += gridDim.x;
-            if (of_w && lgrp < NG) rows_of(lgrp);
+            if (lgrp < NG) {
+                rows_of(lgrp);
+                at = src + (long)(c0 + lk) * 128;
+            }
         }
     };
-    const int D = of_w ? DW : DX;
-    for (int i = 0; i < D && i < total; ++i) issue();
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (of_w)
+        for (int i = 0; i < DW && i < total; ++i) issue(Yes());
+    else
+        for (int i = 0; i < DX && i < total; ++i) issue(No());
     // 1 / rms of each row, while the weights are on their way: the waves of
     // the input, whose few stages the compiler's wait may include
     __shared__ float inv_s[16];
@@ -208,19 +218,6 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     // (the builtin: the compiler has to know that nothing is under way, or it
     // waits for what was only just asked for)
     auto fragments_here = [&]() { __builtin_amdgcn_s_waitcnt(0xc07f); };
-    // Stage s is read by everyone, so its slot is free; stage s + 1 has come.
-    // (Loads of min(total, s + D) stages have been issued.)
-    auto advance = [&](int s) {
-        if (++ws == DW) ws = 0;
-        if (++xs == DX) xs = 0;
-        if (s + 1 == total) return false;
-        const int left = min(total - 2 - s, D - 2);
-        if (of_w) lm_wait<NLW, DW - 2>(left);
-        else lm_wait<NLX, DX - 2>(left);
-        asm volatile("s_barrier" ::: "memory");
-        if (s + D < total) issue();
-        return true;
-    };
     auto finish = [&](int grp) {
         const float inv = SCALED ? inv_s[min(li, M - 1)] : 1.f;
 #pragma unroll
@@ -271,59 +268,91 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
             }
         }
     };
-    if (of_w) lm_wait<NLW, DW - 1>(min(total, DW) - 1);
-    else lm_wait<NLX, DX - 1>(min(total, DX) - 1);
+    if (of_w) lm_wait<NLW, 0, DW - 1>(min(total, DW) - 1);
+    else lm_wait<NLX, 0, DX - 1>(min(total, DX) - 1);
     fragments_here();                          // (and inv_s is written)
     asm volatile("s_barrier" ::: "memory");
     read(0, WK == 2 ? wk : 0);
-    int left = n;                              // steps of this group
-    auto step = [&](int set, int s) {
+    // Step s of `total`: stages up to s + D - 1 have been asked for, and behind the
+    // barrier all have read stage s, and stage s + 1 has come. fast: there is a
+    // stage s + D, so nothing has to be found out.
+    auto step = [&](auto of, auto fast, int set, int s) {
+        constexpr bool W = decltype(of)::value, FAST = decltype(fast)::value;
+        constexpr int D = W ? DW : DX, PER = W ? NLW : NLX;
         fragments_here();
-        if (WK == 2) {
-            if (advance(s)) read(set ^ 1, wk);
-            products(set);
+        if (WK == 1) {
+            read(1, 1);
+            products(0);
+            fragments_here();
+        }
+        if (FAST || s + 1 < total) {
+            lm_wait<PER, FAST ? D - 2 : 0, D - 2>(min(total - 2 - s, D - 2));
+            asm volatile("s_barrier" ::: "memory");
+            if (++ws == DW) ws = 0;
+            if (++xs == DX) xs = 0;
+            read(WK == 2 ? set ^ 1 : 0, WK == 2 ? wk : 0);
+            if (FAST || s + D < total) issue(of);
+        }
+        products(WK == 2 ? set : 1);
+        // (products that moved into the next step would need registers for three
+        // steps' fragments)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto steps = [&](auto of, int s, int end) {    // (WK 2: all of them)
+        const int fast = min(end, total - (decltype(of)::value ? DW : DX));
+        if (WK == 1) {
+            for (; s < fast; ++s) step(of, Yes(), 0, s);
+            for (; s < end; ++s) step(of, No(), 0, s);
             return;
         }
-        read(1, 1);
-        products(0);
-        fragments_here();
-        if (advance(s)) read(0, 0);
-        products(1);
-        if (--left == 0) {
-            finish(g);
-            g += gridDim.x;
-            left = n;
-            clear();
+        for (; s + 1 < fast; s += 2) {
+            step(of, Yes(), 0, s);
+            step(of, Yes(), 1, s + 1);
+        }
+        for (;;) {
+            step(of, No(), 0, s);
+            if (++s >= end) break;
+            step(of, No(), 1, s);
+            if (++s >= end) break;
         }
     };
-    for (int s = 0;;) {
-        step(0, s);
-        if (++s >= total) break;
-        step(1, s);
-        if (++s >= total) break;
+    if constexpr (WK == 1) {
+        for (int s = 0; s < total; s += n) {
+            if (of_w) steps(Yes(), s, s + n);
+            else steps(No(), s, s + n);
+            finish(g);
+            g += gridDim.x;
+            clear();
+        }
+        return;
     }
-    if (WK == 1) return;
-    // the halves' sums meet in LDS (every load has come, and been read)
-    __syncthreads();
+    // The halves' sums meet in LDS (every load has come, and been read). Waves 0-3
+    // are the first half: the two go their own ways from here, or their sums would
+    // need the same registers.
     f32x4* mg = reinterpret_cast<f32x4*>(smem) +
                 wid % (WN * WM) * TW * MW * 64 + lane;
-    if (wk == 1) {
+    if (of_w) {
+        steps(Yes(), 0, total);
+        __syncthreads();
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int m = 0; m < MW; ++m) {
+                const f32x4 p = mg[(t * MW + m) * 64];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[t][m][r] += p[r];
+            }
+        finish(g);
+    } else {
+        steps(No(), 0, total);
+        __syncthreads();
 #pragma unroll
         for (int t = 0; t < TW; ++t)
 #pragma unroll
             for (int m = 0; m < MW; ++m) mg[(t * MW + m) * 64] = acc[t][m];
+        __syncthreads();
     }
-    __syncthreads();
-    if (wk == 1) return;
-#pragma unroll
-    for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int m = 0; m < MW; ++m) {
-            const f32x4 p = mg[(t * MW + m) * 64];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][m][r] += p[r];
-        }
-    finish(g);
 }
 
 // Tiles of 16 rows of w in a workgroup, as few as a chip of 256 CUs leaves it
@@ -410,8 +439,6 @@ extern "C" int launch_linear_mid(const unsigned short* x,
         if (M <= 96) LM_GO(1, 6, 8, 1, 1, 7, 3, F);                           \
         if (M <= 128) LM_GO(2, 4, 4, 2, 1, 6, 3, F);                          \
         if (M <= 160) LM_GO(2, 5, 4, 2, 1, 6, 3, F);                          \
-        if (M <= 192 && once) LM_GO(4, 6, 2, 2, 2, 5, 3, F);                  \
-        if (M <= 224 && once) LM_GO(4, 7, 2, 2, 2, 4, 3, F);                  \
         if (M <= 192) LM_GO(2, 6, 4, 2, 1, 5, 3, F);                          \
         if (M <= 224) LM_GO(2, 7, 4, 2, 1, 4, 3, F);                          \
         LM_GO(2, 8, 4, 2, 1, 4, 3, F);                                        \
