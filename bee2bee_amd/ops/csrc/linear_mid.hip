@@ -20,25 +20,31 @@
 // registers and the input in all of LDS, or tiles of 128 rows of w in turns with
 // three buffers of both. A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
 // workgroup's rows of w, and by all input rows. Four waves fill the one, four
-// the other, straight from memory (global_load_lds: no registers, so 100 KB of
-// loads are under way in each CU), and all eight multiply: the fragments of the
+// the other, straight from memory (global_load_lds: no registers), and all eight
+// multiply: the fragments of the
 // next half step are read while this one's products run. The weights carry the
 // streaming hint, so that they do not push the input out of L2 (2x14336x4096 at
 // 24 rows 40.8 us without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128
 // bytes in LDS are xor-ed by half their number: no two of a read's 16 rows meet
 // in a bank. Workgroups start at different places of K: in step they would all
 // ask for the same few channels (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 ->
-// 44.5 at 80). The input needs three slots (with two, and more of weights, 44 ->
-// 61 us at 80 rows); more, or its rows apart by an odd number of lines, change
+// 44.5 at 80). The rings hold what
+// covers the memory's latency and no more: 32 KB of weights of narrow products, 64
+// of others. With all of LDS for weights every CU asks for 100 KB at once, and the
+// input that the first step waits for queues behind it (us, rings of 96 to 112 KB /
+// as now: 2048x8192 9.6 / 8.5 at 24 rows, 11.1 / 9.5 at 57; 4096x4096 11.6 / 10.4
+// at 80; 2x8192x2048 16.0 / 14.7 at 57; 2x14336x4096 45.0 / 43.2 at 80; with 48 and
+// 24 KB a third to half more time). The input needs four slots, better six (with
+// two 44 -> 61 us at 80 rows); its rows apart by an odd number of lines change
 // nothing.
 //
-// Measured with the kernel that reads them (us, 24 / 80 / 128 / 200 / 256 rows;
-// in brackets this file's form before, which took weights through registers):
-//   4096x14336 26.2 / 31.9 / 34.9 / 43.1 / 49.1 (30.1 / 36.1 / 43.9 / 56 / 64)
-//   4096x4096  13.1 / 16.8 / 19.6 / 24.1 / 26.0 (14.5 / 17.3 / 20.7 / 25.5 / 29)
-//   6144x4096  15.1 / 21.5 / 25.4 / 31.0 / 33.6 (19.5 / 24.0 / 29.1 / 36.5 / 41)
-//   3584x18944 28.9 / 34.3 / 39.5 / 49.7 / 56.8 (33.7 / 43.1 / 52.2 / 69 / 78)
-//   2048x8192  13.2 / 16.8 / 19.4 / 22.4 / 25.0 (14.4 / 17.1 / 20.3 / 25.5 / 29)
+// Measured (us, launch after launch with weights that no cache holds, 24 / 80 / 128
+// / 200 / 256 rows; in brackets with one loop and the long rings):
+//   4096x14336 20.9 / 25.0 / 28.8 / 36.1 / 42.9 (21.1 / 26.3 / 29.7 / 38.9 / 45.3)
+//   4096x4096  8.3 / 10.4 / 12.4 / 16.8 / 19.1 (9.4 / 11.6 / 13.2 / 17.5 / 19.9)
+//   6144x4096  11.3 / 14.8 / 17.3 / 22.8 / 26.1 (11.4 / 15.8 / 18.6 / 24.5 / 27.9)
+//   3584x18944 23.5 / 29.0 / 33.5 / 43.1 / 50.0 (23.9 / 30.5 / 34.5 / 45.1 / 52.7)
+//   2048x8192  8.5 / 10.5 / 12.5 / 16.7 / 19.5 (9.6 / 11.7 / 13.2 / 18.0 / 20.2)
 // The library's figures are at the rules in ops/__init__.py.
 #include "common.h"
 
@@ -422,24 +428,24 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     } while (0)
 #define LM_4(F)                                                               \
     do {                                                                      \
-        if (M <= 32) LM_GO(1, 2, 4, 1, 2, 12, 6, F);                          \
-        if (M <= 64) LM_GO(1, 4, 4, 1, 2, 12, 6, F);                          \
-        if (M <= 96) LM_GO(2, 3, 2, 2, 2, 10, 5, F);                          \
-        if (M <= 128) LM_GO(2, 4, 2, 2, 2, 10, 4, F);                         \
-        if (M <= 160) LM_GO(2, 5, 2, 2, 2, 8, 4, F);                          \
-        if (M <= 192) LM_GO(2, 6, 2, 2, 2, 8, 4, F);                          \
-        if (M <= 224) LM_GO(2, 7, 2, 2, 2, 7, 3, F);                          \
-        LM_GO(2, 8, 2, 2, 2, 7, 3, F);                                        \
+        if (M <= 32) LM_GO(1, 2, 4, 1, 2, 4, 6, F);                          \
+        if (M <= 64) LM_GO(1, 4, 4, 1, 2, 4, 6, F);                          \
+        if (M <= 96) LM_GO(2, 3, 2, 2, 2, 4, 6, F);                          \
+        if (M <= 128) LM_GO(2, 4, 2, 2, 2, 4, 6, F);                         \
+        if (M <= 160) LM_GO(2, 5, 2, 2, 2, 4, 6, F);                          \
+        if (M <= 192) LM_GO(2, 6, 2, 2, 2, 4, 5, F);                          \
+        if (M <= 224) LM_GO(2, 7, 2, 2, 2, 4, 4, F);                          \
+        LM_GO(2, 8, 2, 2, 2, 4, 4, F);                                        \
     } while (0)
 #define LM_8(F)                                                               \
     do {                                                                      \
-        if (M <= 32) LM_GO(1, 2, 8, 1, 1, 7, 4, F);                           \
-        if (M <= 64) LM_GO(1, 4, 8, 1, 1, 7, 4, F);                           \
-        if (M <= 96 && once) LM_GO(2, 6, 4, 1, 2, 7, 3, F);                   \
-        if (M <= 96) LM_GO(1, 6, 8, 1, 1, 7, 3, F);                           \
-        if (M <= 128) LM_GO(2, 4, 4, 2, 1, 6, 3, F);                          \
-        if (M <= 160) LM_GO(2, 5, 4, 2, 1, 6, 3, F);                          \
-        if (M <= 192) LM_GO(2, 6, 4, 2, 1, 5, 3, F);                          \
+        if (M <= 32) LM_GO(1, 2, 8, 1, 1, 4, 6, F);                           \
+        if (M <= 64) LM_GO(1, 4, 8, 1, 1, 4, 6, F);                           \
+        if (M <= 96 && once) LM_GO(2, 6, 4, 1, 2, 4, 6, F);                   \
+        if (M <= 96) LM_GO(1, 6, 8, 1, 1, 4, 6, F);                           \
+        if (M <= 128) LM_GO(2, 4, 4, 2, 1, 4, 6, F);                          \
+        if (M <= 160) LM_GO(2, 5, 4, 2, 1, 4, 4, F);                          \
+        if (M <= 192) LM_GO(2, 6, 4, 2, 1, 4, 4, F);                          \
         if (M <= 224) LM_GO(2, 7, 4, 2, 1, 4, 3, F);                          \
         LM_GO(2, 8, 4, 2, 1, 4, 3, F);                                        \
     } while (0)
