@@ -356,13 +356,12 @@ def mid_shape(rows: int, width: int, depth: int) -> bool:
     captured (six layers of 768, prompts of 140 / 200 / 256 tokens 490 / 685 / 685
     us, with the library's 770; captured, 332 / 355 / 358 and 329 / 347 / 345).
     Measured with the kernel that reads them
-    (us, the library's in brackets): at 24 / 128 / 200 rows 6144x4096 15.1 (19.1)
-    / 25.4 (30.0) / 31.0 (30.4), 4096x14336 26.2 (32.8) / 34.9 (79) / 43.1
-    (59.6), 3584x18944 28.9 (112) / 39.5 (103) / 49.7 (127), 8192x8192 34.5 (34.6)
-    / 41.2 (52.6) / 49.1 (57), 2048x2048 8.7 (10.9) / 12.3 (11.2) / 15.2 (12.2),
-    3072x2048 9.5 (15.0) / 14.6 (18.1) / 18.2 (16.6), 5120x3072 12.9 (16.4) /
-    21.8 (25.1) / 28.0 (24.1), 768x3072 7.8 (11.9) / 10.6 (10.4) / 13.0
-    (11.3)."""
+    (us, the library's in brackets): at 128 / 160 / 224 rows 6144x4096 25.1 (30.4)
+    / 26.4 (33.2) / 30.3 (42.5), 5120x3072 21.7 (25.5) / 23.4 (28.4) / 26.9
+    (34.7), 4608x3584 22.2 (27.6) / 23.5 (29.6) / 26.9 (37.6), 3072x3072 15.8
+    (23.7) / 17.7 (20.1) / 20.8 (21.5), 3072x2048 13.9 (15.7) / 15.4 (13.0) / 18.4
+    (15.0), 2048x2048 12.0 (11.5) / 13.5 (12.1) at 160, 768x3072 10.6 (10.4) /
+    11.8 (10.7) / 13.6 (11.7)."""
     if width * depth <= 4 << 20 and (rows <= 160 or 2 * depth >= 7 * width):
         return True
     return rows <= MID_MAX or width * depth >= (
@@ -374,10 +373,11 @@ def mid_gated(rows: int, width: int, depth: int) -> bool:
     ends it are the input rows, which each CU draws beside its share of the
     weights; wide_linear takes the others. Measured beside the library's product
     and swiglu (us): 2x14336x4096
-    36.9 (56.7) at 24 rows, 50.8 (57.8) at 128, 64 (69.6) at 200, 78.6 (71.6) at
-    256; 2x18944x3584 44.6 (56.8), 60 (71.6), 68.6 (75.5) at 160, 113 (83) at
-    200; 2x8192x2048 14.2 (19.4), 20 (23.5), 26 (30), 29 (33) at 256; 2x2048x768
-    6.9 (9.4), 9.7 (10.4), 11.9 (10.3). More than 12 tiles of 8 columns a CU go
+    36.9 (56.7) at 24 rows, 49.8 (57.8) at 128, 63 (69.6) at 200, 72.5 (71.6) at
+    256; 2x18944x3584 45.3 (56.8), 57.7 (71.6), 61 (75.5) at 160, 107 (83) at
+    200; 2x8192x2048 14.1 (20.8), 21.7 (23.9), 25 (30.6) at 192, 29 (33) at 256;
+    2x5504x2048 13.0 (18.8), 18.5 (21.6), 23.5 (28.6) at 192, 27.9 (30.7) at 256;
+    2x2048x768 6.9 (9.4), 9.7 (10.4), 11.9 (10.3). More than 12 tiles of 8 columns a CU go
     in rounds, each with a start of its own: 2x27648x5120 96 (100), 107 (105) at
     48, 134 (123) at 128, but 2x28672x8192 141 (181), 153 (186), 194 (211)."""
     tiles = -(-width // 2048)           # of 8 columns, a CU
@@ -389,7 +389,7 @@ def mid_gated(rows: int, width: int, depth: int) -> bool:
         return True
     if tiles > 8:
         return rows <= 160
-    return width * depth >= 16_000_000 and rows <= (256 if tiles <= 4 else 224)
+    return width * depth >= 11_000_000 and rows <= (256 if tiles <= 4 else 224)
 
 
 def mid_gelu(rows: int, width: int, depth: int) -> bool:
@@ -402,15 +402,18 @@ def mid_gelu(rows: int, width: int, depth: int) -> bool:
 def mid_head(rows: int, width: int, depth: int) -> bool:
     """Logits that mid_rows_linear takes. Groups of 8 tiles of 16 columns, a
     CU's one after the other: where the last round leaves more than a twentieth
-    of the chip idle (152064 columns) the library is ahead above 64 rows. Beside
-    the library's product (us): 128256x4096 168 (193) at 24 rows, 195 (218) at
-    80, 230 (245) at 160, 304 (297) at 256; 152064x3584 172 (242), 218 (213);
-    32000x4096 41 (63), 48 (66), 58 (64); 128256x2048 84 (121), 103 (129); of
-    rows of 768 17.0 (18.6), 22.6 (20.8). Few rows (one launch of rows_linear in
-    brackets; a norm takes 2.5 us): 1 / 16 rows 128256x4096 168 (178) / 166
-    (188), 152064x3584 158 (182) / 164 (204), 128256x2048 77 (93) / 81 (101); of
-    rows of 8192 1 / 8 / 12 rows 128256 370 (363) / 371 (359) / 370 (376), 152064
-    454 (427) / 458 (438) / 454 (459)."""
+    of the chip idle (152064 columns) the library is ahead above 64 rows, and of
+    the largest heads wide_linear from 129 rows on. Beside the library's product,
+    and wide_linear's where there is one (us): 128256x4096 159 (193) at 24 rows,
+    188 (218) at 80, 214 (239, 210) at 128, 224 (251, 216) at 160; 32000x4096 41
+    (63), 45 (66), 52 (68), 57 (69), 65 (78) at 200, 73 (79) at 256; 128256x2048
+    82 (121), 102 (129), 120 (134), 129 (141, 137), 143 (178, 144); 152064x3584
+    176 (242), 220 (213), 249 (245, 241); of rows of 768 17.0 (18.6), 22.6
+    (20.8). Few rows (one launch of rows_linear in brackets; a norm takes 2.5
+    us): 1 / 16 rows 128256x4096 155 (178) / 157 (188), 152064x3584 163 (182) /
+    167 (204), 128256x2048 78 (93) / 80 (101); of rows of 8192 1 / 8 / 12 rows
+    128256 370 (363) / 371 (359) / 370 (376), 152064 454 (427) / 458 (438) / 454
+    (459)."""
     if rows <= ROWS_MAX and width * depth < 100_000_000:
         return False
     if rows <= 8 and depth >= 8192:
@@ -418,7 +421,10 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     tiles = -(-width // 16)
     rounds = -(-tiles // 2048)
     full = 256 * rounds * -(-tiles // (256 * rounds))
-    if width % 4 or rows > 160 or (depth < 1024 and rows > 48):
+    if width % 4 or rows > DEEP_MAX or (depth < 1024 and rows > 48):
+        return False
+    if rows > MID_MAX and width * depth > (
+            280_000_000 if rows <= 192 else 150_000_000):
         return False
     return rows <= 64 or tiles * 20 >= full * 19
 

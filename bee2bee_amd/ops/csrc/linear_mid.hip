@@ -28,8 +28,10 @@
 // bytes in LDS are xor-ed by half their number: no two of a read's 16 rows meet
 // in a bank. Workgroups start at different places of K: in step they would all
 // ask for the same few channels (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 ->
-// 44.5 at 80). The rings hold what
-// covers the memory's latency and no more: 32 KB of weights of narrow products, 64
+// 44.5 at 80). Those of output heads, which go round by round, are 5 steps apart
+// and not one: 128256x4096 167 -> 159 us at 24 rows, 193 -> 188 at 80 (gated 2 to
+// 4% slower so, others the same). The rings hold what covers the memory's latency
+// and no more: 32 KB of weights of narrow products, 64
 // of others. With all of LDS for weights every CU asks for 100 KB at once, and the
 // input that the first step waits for queues behind it (us, rings of 96 to 112 KB /
 // as now: 2048x8192 9.6 / 8.5 at 24 rows, 11.1 / 9.5 at 57; 4096x4096 11.6 / 10.4
@@ -105,7 +107,8 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     const int NG = (NT + tiles - 1) / tiles;
     const int CH = K / 64;                     // steps of 64: of them
     const int c0 = CH * blockIdx.y / S, n = CH * (blockIdx.y + 1) / S - c0;
-    const int rot = (blockIdx.x / 8) % n;      // where it starts
+    // where it starts
+    const int rot = blockIdx.x / 8 * (OUT == LM_ROWS ? 5 : 1) % n;
     int g = blockIdx.x;
     const int total = n * ((NG - 1 - g) / (int)gridDim.x + 1);
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -476,6 +479,9 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     if (form == LM_GATED && tiles <= 4) LM_4(LM_GATED);
     if (form == LM_GATED) LM_8(LM_GATED);
     if (form == LM_ROWS && tiles <= 4) LM_4(LM_ROWS);
+    // (half the input: 128256x4096 168 -> 155 us at 1 row with the places of K,
+    // 128256x2048 79.5 -> 77.9, 152064x3584 165 -> 163)
+    if (form == LM_ROWS && M <= 16) LM_GO(1, 1, 8, 1, 1, 4, 6, LM_ROWS);
     if (form == LM_ROWS) LM_8(LM_ROWS);
     if (tiles <= 4) LM_4(LM_PARTS);
     LM_8(LM_PARTS);

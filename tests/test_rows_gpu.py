@@ -277,6 +277,23 @@ def test_activated_rows(M, N, K, act):
             + 1e-6).all()
 
 
+# (five tiles a workgroup, the last one of 12 columns, fewer steps of K than the
+# rings have slots; eight tiles and a second group, more steps)
+@pytest.mark.parametrize("N,K", [(20492, 128), (40004, 960)])
+def test_logits_of_few_rows(N, K):
+    """As above without an activation; a row's logits are the same to the bit
+    whatever rows are beside it."""
+    torch.manual_seed(N)
+    x, w = _rand(16, K), _rand(N, K, std=0.1)
+    got = ops.mid_rows_linear(x, w)
+    want = x.double() @ w.double().t()
+    e = 2 ** -24 * K * (x.double().abs() @ w.double().abs().t())
+    assert ((got.double() - want).abs() <= e + 2 ** -8 * want.abs()
+            + 1e-6).all()
+    for at in (slice(0, 1), slice(3, 5), slice(1, 16)):
+        assert torch.equal(ops.mid_rows_linear(x[at].contiguous(), w), got[at])
+
+
 # (a workgroup's tiles of 8 columns: up to 4, 8, 12, and two groups of 7)
 @pytest.mark.parametrize("N,K", [(8192, 6144), (12560, 4096), (17008, 3008),
                                  (25008, 2048)])
