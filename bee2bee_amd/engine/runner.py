@@ -727,6 +727,8 @@ class Runner:
                 input_ids_or_hidden, positions, slot_mapping, cu, 1,
                 block_table, state_slots)
 
+        order = None
+
         def attn(layer_idx, q, k, v, k_cache, v_cache):
             if self.decode_attn_fn is not None:
                 # injected attention (context parallelism: parallel/cp.py
@@ -735,7 +737,7 @@ class Runner:
                     q, k_cache, v_cache, block_table, seq_lens, self.scale
                 )
             return ops.attn_decode(
-                q, k_cache, v_cache, block_table, seq_lens, self.scale
+                q, k_cache, v_cache, block_table, seq_lens, self.scale, order
             )
 
         hidden = (
@@ -756,8 +758,9 @@ class Runner:
                 slot_mapping, block_table, seq_lens,
                 status=self.step_status)
         if slot_mapping is None:
-            slot_mapping = ops.decode_slots(block_table, positions,
-                                            self.kv.block_size)
+            slot_mapping, order = ops.decode_plan(
+                block_table, positions, self.kv.block_size, seq_lens,
+                self.spec.n_kv_heads)
         return self._run_layers(hidden, positions, slot_mapping, attn)
 
     # --------------------------------------------------------- hybrid stacks

@@ -131,10 +131,12 @@ def attn_decode(
     block_table: torch.Tensor,
     seq_lens: torch.Tensor,
     scale: float,
+    order: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
+    """order: decode_plan's, in which the contexts are read."""
     if _use_hip(q):
         return require_hip().attn_decode(
-            q, k_cache, v_cache, block_table, seq_lens, scale
+            q, k_cache, v_cache, block_table, seq_lens, scale, order
         )
     return reference.attn_decode(q, k_cache, v_cache, block_table, seq_lens, scale)
 
@@ -507,6 +509,27 @@ def decode_slots(block_table, positions, block_size: int):
             and positions.is_contiguous() and block_table.stride(1) == 1):
         return require_hip().decode_slots(block_table, positions, block_size)
     return reference.decode_slots(block_table, positions, block_size)
+
+
+def decode_plan(block_table, positions, block_size: int, seq_lens,
+                kv_heads: int):
+    """-> (decode_slots, the rows' numbers by length, longest first, which
+    attn_decode takes, or None). Workgroups that start last should be short ones:
+    us of attention, as the rows stand / in that order, bf16, 8 key heads of size
+    128, of 250 to 2000 tokens, 16 sequences 19.2 / 19.3, 24 27.8 / 25.3, 48
+    45.6 / 39.4, 128 104 / 95, of 375 to 3000 200 227 / 214 (fp8 118 / 114),
+    of 137 to 1100 400 165 / 160 (fp8 90 / 91), 1536 599 / 615: many workgroups
+    even out by themselves, and neighbours of one length hold each other up."""
+    if (80 <= positions.numel() * kv_heads <= 2048 and _use_hip(positions)
+            and all(t.dtype is torch.int32 for t in (block_table, positions,
+                                                     seq_lens))
+            and positions.dim() == 1 and seq_lens.dim() == 1
+            and positions.is_contiguous() and seq_lens.is_contiguous()
+            and block_table.stride(1) == 1
+            and seq_lens.shape[0] >= positions.shape[0]):
+        return require_hip().decode_plan(block_table, positions, block_size,
+                                         seq_lens)
+    return decode_slots(block_table, positions, block_size), None
 
 
 def embed_positions(ids, table, positions, pos_table):

@@ -9,6 +9,7 @@
 #include <algorithm>
 
 using torch::Tensor;
+using c10::optional;
 
 extern "C" {
 void launch_rmsnorm(const unsigned short*, const unsigned short*,
@@ -43,9 +44,10 @@ int attn_flash_form(long, int, int, int, int, int, int);
 int attn_stream_takes(long, long);
 int attn_stream_splits(long, long, long, int*, int*);
 int launch_attn_stream(const unsigned short*, const void*, const void*,
-                       const int*, const int*, const int*, unsigned short*,
-                       float*, float*, float*, int, int, int, int, int, int,
-                       int, int, int, int, long, float, int, hipStream_t);
+                       const int*, const int*, const int*, const int*,
+                       unsigned short*, float*, float*, float*, int, int, int,
+                       int, int, int, int, int, int, int, long, float, int,
+                       hipStream_t);
 void launch_attn_prefill(const unsigned short*, const unsigned short*,
                          const unsigned short*, const int*, unsigned short*,
                          long, int, int, int, int, long, long, long, int,
@@ -227,7 +229,8 @@ Tensor swiglu(const Tensor& gu) {
 bool attn_stream(const Tensor& q_in, const Tensor& k_cache,
                  const Tensor& v_cache, const int* cu, int nseq,
                  const Tensor& block_table, const Tensor& seq_lens,
-                 Tensor& out, float* out_ml, int max_qlen, double scale) {
+                 const int* order, Tensor& out, float* out_ml, int max_qlen,
+                 double scale) {
     // queries are read 16 bytes at a time
     const bool aligned =
         q_in.stride(0) % 8 == 0 &&
@@ -249,7 +252,7 @@ bool attn_stream(const Tensor& q_in, const Tensor& k_cache,
     }
     return launch_attn_stream(
                bf16p(q), k_cache.data_ptr(), v_cache.data_ptr(), cu,
-               block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),
+               block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), order,
                bf16p_mut(out), out_ml,
                Z > 1 ? part_o.data_ptr<float>() : nullptr,
                Z > 1 ? part_ml.data_ptr<float>() : nullptr, nseq, nkv, G, W,
@@ -261,7 +264,8 @@ std::vector<Tensor> attn_decode_impl(const Tensor& q, const Tensor& k_cache,
                                      const Tensor& v_cache,
                                      const Tensor& block_table,
                                      const Tensor& seq_lens, double scale,
-                                     bool want_lse) {
+                                     bool want_lse,
+                                     const optional<Tensor>& order = {}) {
     check_bf16(q, "q");
     const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
     if (!fp8) check_bf16(k_cache, "k_cache");
@@ -291,7 +295,12 @@ std::vector<Tensor> attn_decode_impl(const Tensor& q, const Tensor& k_cache,
         out_ml = torch::empty({B, nq, 2}, fopt);
         out_ml_p = out_ml.data_ptr<float>();
     }
+    if (order.has_value())
+        TORCH_CHECK(order->is_cuda() && order->is_contiguous() &&
+                    order->scalar_type() == torch::kInt32 &&
+                    order->numel() == B, "order: the rows' numbers");
     if (attn_stream(q, k_cache, v_cache, nullptr, B, block_table, seq_lens,
+                    order.has_value() ? order->data_ptr<int>() : nullptr,
                     out, out_ml_p, 1, scale))
         return want_lse ? std::vector<Tensor>{out, out_ml}
                         : std::vector<Tensor>{out};
@@ -310,9 +319,10 @@ std::vector<Tensor> attn_decode_impl(const Tensor& q, const Tensor& k_cache,
 
 Tensor attn_decode(const Tensor& q, const Tensor& k_cache,
                    const Tensor& v_cache, const Tensor& block_table,
-                   const Tensor& seq_lens, double scale) {
+                   const Tensor& seq_lens, double scale,
+                   const optional<Tensor>& order) {
     return attn_decode_impl(q, k_cache, v_cache, block_table, seq_lens,
-                            scale, false)[0];
+                            scale, false, order)[0];
 }
 
 // out + per-(seq, q-head) (m, l): the flash merge state that context
@@ -381,8 +391,8 @@ Tensor attn_prefill_paged(const Tensor& q, const Tensor& k_cache,
     Tensor out = torch::empty({T, nq, hd}, q.options());
     if (T > 0 && attn_stream_takes((long)nseq * nkv, max_qlen * (nq / nkv)) &&
         attn_stream(q, k_cache, v_cache, cu_q.data_ptr<int>(), nseq,
-                    block_table, seq_lens, out, nullptr, (int)max_qlen,
-                    scale))
+                    block_table, seq_lens, nullptr, out, nullptr,
+                    (int)max_qlen, scale))
         return out;
     launch_attn_prefill_paged(bf16p(q), k_cache.data_ptr(),
                               v_cache.data_ptr(), cu_q.data_ptr<int>(),
@@ -491,7 +501,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fused_add_layernorm", &fused_add_layernorm,
           "residual add + LayerNorm");
     m.def("gelu", &gelu, "gelu_new (tanh approximation)");
-    m.def("attn_decode", &attn_decode, "paged GQA decode attention");
+    m.def("attn_decode", &attn_decode, "paged GQA decode attention",
+          py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+          py::arg("block_table"), py::arg("seq_lens"), py::arg("scale"),
+          py::arg("order") = optional<Tensor>());
     m.def("attn_decode_lse", &attn_decode_lse,
           "paged GQA decode attention + per-head (m, l) merge state");
     m.def("attn_prefill", &attn_prefill, "varlen causal flash prefill");

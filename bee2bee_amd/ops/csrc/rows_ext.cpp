@@ -40,6 +40,8 @@ extern "C" int launch_qkv_rope_store(
     const float*, const float*, int, void*, void*, const int*, long, int, int,
     int, int, int, hipStream_t);
 
+extern "C" int launch_decode_plan(const int*, const int*, int*, const int*,
+                                  int*, int, int, long, int, hipStream_t);
 extern "C" void launch_decode_slots(const int*, const int*, int*, int, int,
                                     long, int, hipStream_t);
 extern "C" void launch_embed_positions(const long*, const unsigned short*,
@@ -601,17 +603,37 @@ Tensor rope_store_qkv(const Tensor& qkv, const optional<Tensor>& bias,
     return out;
 }
 
-Tensor decode_slots(const Tensor& table, const Tensor& pos, int64_t bs) {
+void check_decode(const Tensor& table, const Tensor& pos, int64_t bs) {
     TORCH_CHECK(table.is_cuda() && table.scalar_type() == torch::kInt32 &&
                 table.dim() == 2 && table.stride(1) == 1);
     TORCH_CHECK(pos.is_cuda() && pos.scalar_type() == torch::kInt32 &&
                 pos.is_contiguous() && pos.dim() == 1 &&
                 pos.size(0) <= table.size(0) && bs > 0);
+}
+
+Tensor decode_slots(const Tensor& table, const Tensor& pos, int64_t bs) {
+    check_decode(table, pos, bs);
     Tensor slots = torch::empty_like(pos);
     launch_decode_slots(table.data_ptr<int>(), pos.data_ptr<int>(),
                         slots.data_ptr<int>(), pos.size(0), table.size(1),
                         table.stride(0), bs, stream());
     return slots;
+}
+
+// the same, and the rows by length, longest first
+std::vector<Tensor> decode_plan(const Tensor& table, const Tensor& pos,
+                                int64_t bs, const Tensor& lens) {
+    check_decode(table, pos, bs);
+    TORCH_CHECK(lens.is_cuda() && lens.scalar_type() == torch::kInt32 &&
+                lens.is_contiguous() && lens.dim() == 1 &&
+                lens.size(0) >= pos.size(0), "lengths of the rows");
+    Tensor slots = torch::empty_like(pos), order = torch::empty_like(pos);
+    TORCH_CHECK(launch_decode_plan(table.data_ptr<int>(), pos.data_ptr<int>(),
+                                   slots.data_ptr<int>(), lens.data_ptr<int>(),
+                                   order.data_ptr<int>(), pos.size(0),
+                                   table.size(1), table.stride(0), bs,
+                                   stream()) == 0, "1 to 2048 rows");
+    return {slots, order};
 }
 
 // [T, H] bf16 = embed[ids] + pos_embed[pos]
@@ -656,6 +678,8 @@ void register_rows_ops(pybind11::module_& m) {
     m.def("add_norm_parts", &add_norm_parts,
           "residual add of a projection's parts, and the next norm");
     m.def("decode_slots", &decode_slots, "page slots of a decode step's rows");
+    m.def("decode_plan", &decode_plan,
+          "page slots of a decode step's rows, and the rows by length");
     m.def("embed_positions", &embed_positions,
           "token and learned position embeddings, added");
     m.def("rope_store_qkv", &rope_store_qkv,

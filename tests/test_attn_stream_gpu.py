@@ -196,3 +196,71 @@ def test_weights_add_up_to_one(nseq, hd):
             scale = 0.6931471805599453
         got = ops.attn_decode(q, kc, vc, table, lens, scale)
         assert (got == 1).all(), (far, got.float().min().item())
+
+
+# contexts at the edges of a tile, of what eight waves take at once and of splits
+EDGES = [0, 1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 287, 288, 289, 383, 384,
+         385, 511, 512, 513, 767, 768, 769, 900]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("nq,nkv,hd,total,bs,width", [
+    (16, 8, 128, EDGES[:12], 256, 4),        # 288 workgroups, 3 splits
+    (16, 8, 64, EDGES, 64, 0),               # 384, 2 splits
+    (8, 4, 128, EDGES * 4, 128, 0),          # 384 of whole contexts
+    (8, 8, 128, EDGES[1::2] * 6, 32, 64),    # more than eight waves take; fp8 too
+    (8, 8, 64, EDGES[::3] + [2500], 256, 16),
+    (8, 8, 128, EDGES[:12] * 2, 24, 0),      # pages that tiles cross
+])
+def test_decode_by_length(nq, nkv, hd, total, bs, width, fp8):
+    """Four and eight waves a context, in the order of lengths and as the rows
+    stand: the same to the bit."""
+    kc, vc, table, lens = _pages(nkv, hd, bs, total, fp8, 4, width)
+    q = torch.randn(len(total), nq, hd, device=DEV).bfloat16()
+    pos = (lens - 1).clamp(0)
+    slots, order = ops.decode_plan(table, pos, bs, lens, nkv)
+    assert torch.equal(slots, ops.decode_slots(table, pos, bs))
+    if 80 <= len(total) * nkv <= 2048:
+        want = sorted(range(len(total)), key=lambda b: (-total[b], b))
+        assert order.tolist() == want
+    else:
+        assert order is None
+    got = ops.attn_decode(q, kc, vc, table, lens, 0.1, order)
+    assert torch.equal(got, ops.attn_decode(q, kc, vc, table, lens, 0.1))
+    qf = q.float()
+    if fp8:
+        qf = (qf * 0.1).bfloat16().to(torch.float8_e4m3fn).float() / 0.1
+    keep = lens > 0
+    assert not got[~keep].any()
+    want = reference.attn_decode(qf[keep], _wide(kc), _wide(vc), table[keep],
+                                 lens[keep], 0.1)
+    _check(got[keep], want, _wide(vc))
+
+
+@pytest.mark.parametrize("B", [10, 64, 65, 2048])
+def test_rows_by_length(B):
+    """Equal lengths stay as they stand; more lengths and tables than rows."""
+    lens = torch.randint(0, 40, (B + 3,), device=DEV, dtype=torch.int32)
+    table = torch.randint(0, 99, (B + 3, 2), device=DEV, dtype=torch.int32)
+    pos = torch.randint(-1, 70, (B,), device=DEV, dtype=torch.int32)
+    nkv = 8 if B < 100 else 1
+    slots, order = ops.decode_plan(table, pos, 32, lens, nkv)
+    assert torch.equal(slots, ops.decode_slots(table, pos, 32))
+    assert torch.equal(order.long(), lens[:B].sort(descending=True,
+                                                   stable=True).indices)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_chunks_of_eight_waves(fp8):
+    """Two and three row tiles of a chunk, 8 waves a context."""
+    for new, old in ([4, 5, 1] * 4, [300, 0, 255] * 4), ([9] * 13, [600] * 13):
+        total = [a + b for a, b in zip(new, old)]
+        kc, vc, table, lens = _pages(8, 128, 256, total, fp8, 2)
+        q = torch.randn(sum(new), 32, 128, device=DEV).bfloat16()
+        cu = torch.tensor([0] + torch.tensor(new).cumsum(0).tolist(),
+                          dtype=torch.int32, device=DEV)
+        got = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, max(new), 0.1)
+        want = reference.attn_decode_with_history(
+            q.float(), _wide(kc), _wide(vc), table, lens,
+            torch.tensor(new, dtype=torch.int32), 0.1)
+        _check(got, want, _wide(vc))
