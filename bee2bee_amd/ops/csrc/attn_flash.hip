@@ -32,7 +32,7 @@
 // before it (16-row tiles, weights and V transposed through LDS by 2-byte
 // writes) reached 97-170 TFLOP/s on the same shapes; this one: 4096 queries
 // of 28 heads on 16384 keys 728 us (1155 TFLOP/s; 890 without turns), four
-// prompts of 512 to 4096 tokens of 28 heads 245 (284 as 128 rows without
+// prompts of 512 to 4096 tokens of 28 heads 215 (284 as 128 rows without
 // turns), 2048 tokens of 32 heads 55 (59), nine prompts of 112 to 901 tokens
 // 35. Without s_setprio for the multiplying waves 1 to 2% are lost.
 #include "common.h"
@@ -73,6 +73,81 @@ DEV_INLINE void fl_load(const char* base, unsigned off, unsigned to) {
                  ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
 }
 
+// A block: a sequence, its first query and their number, the tokens that it has
+// with them, and which of its rows of tiles
+struct FlBlock {
+    int seq, s0, QL, L, tile;
+};
+
+// The j-th block of a key head, those with many keys first, of sequences of up to
+// `most` blocks of `rows` query rows; false: there is none. The chip deals a die's
+// workgroups out to its four parts in turn, and one that finds its part full holds
+// up those behind it. If a sequence has the same turn all along, as the number of
+// sequences and key heads may make it, a long one's blocks are all on one part or
+// two. An odd number of sequences goes round by itself; of an even one the order is
+// turned from one row of tiles to the next, so that it meets other parts, and dies
+// where they share a key head (`apart`: they do not). Of two, four and six, where
+// that is not enough, and of portions, whose histories differ, each workgroup finds
+// the j-th block by the number of keys: a microsecond or two, 3 to 12% of prompts
+// of 9 to 30 that gain nothing. us, before / now, 32/8 and 28/4 heads of size 128, 32/8 of
+// 64: by keys, 2 prompts of 375 and 3000 tokens 140 / 90, 121 / 85, 86 / 67, 4 of 500 to
+// 4000 394 / 235, 242 / 201, 255 / 144, 6 of 250 to 2000 161 / 115, 108 / 99, 87 / 63, portions
+// of 300 on 500, 1000 on 4000 and 2000 on 100 163 / 140, 155 / 131; turned, 12 of 250 to
+// 2000 294 / 213 (28/4 as before); odd, 17 of 110 to 900 of 28/4 86 / 72, 9 of 210 to
+// 1700 153 / 105.
+DEV_INLINE bool fl_block(const int* cu, const int* seq_lens, int nseq, int G,
+                         int rows, int j, int most, bool apart, FlBlock& b) {
+    if (nseq == 1 || nseq > 8 || (!seq_lens && (nseq % 2 || nseq > 6))) {
+        const int up = j / nseq;
+        const int turn = nseq % 2 ? 0 : apart ? up + up / nseq : up;
+        b.tile = most - 1 - up;
+        b.seq = (j + turn) % nseq;
+        b.s0 = cu[b.seq];
+        b.QL = cu[b.seq + 1] - b.s0;
+        b.L = seq_lens ? seq_lens[b.seq] : b.QL;
+        return b.tile * rows < b.QL * G;
+    }
+    const int lane = threadIdx.x & 63, at = min(lane, nseq - 1);
+    const int s0 = cu[at], len = cu[at + 1] - s0;
+    const int L = seq_lens ? seq_lens[at] : len;
+    const int mine =
+        lane < nseq ? min((max(len, 0) * G + rows - 1) / rows, most) : 0;
+    // a block's level: rows of tiles before it, as if the history were queries
+    const int low = max(L - len, 0) * G / rows;
+    // blocks at level x and above, a lane a level: 64 at a time
+    auto from = [&](int x) {
+        int n = 0;
+        for (int i = 0; i < nseq; ++i) {
+            const int m = __builtin_amdgcn_readlane(mine, i);
+            n += min(max(m + __builtin_amdgcn_readlane(low, i) - x, 0), m);
+        }
+        return n;
+    };
+    int span = 1, lo = 0, above = 0;
+    for (int i = 0; i < nseq; ++i)
+        span = max(span, __builtin_amdgcn_readlane(mine + low, i));
+    for (bool first = true; first || span > 1; first = false) {
+        const int step = (span + 63) / 64, n = from(lo + lane * step);
+        const unsigned long higher = __ballot(n > j);
+        if (!higher) return false;             // (the first time)
+        const int last = 63 - __builtin_clzl(higher);
+        if (last < 63) above = __builtin_amdgcn_readlane(n, last + 1);
+        lo += last * step;
+        span = step;
+    }
+    // the (j - above)-th sequence that has one there
+    const bool has = lo >= low && lo < low + mine;
+    const unsigned long all = __ballot(has);
+    const int before = __builtin_amdgcn_mbcnt_hi(
+        (unsigned)(all >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)all, 0));
+    b.seq = __builtin_ctzl(__ballot(has && before == j - above));
+    b.s0 = __builtin_amdgcn_readlane(s0, b.seq);
+    b.QL = __builtin_amdgcn_readlane(len, b.seq);
+    b.L = __builtin_amdgcn_readlane(L, b.seq);
+    b.tile = lo - __builtin_amdgcn_readlane(low, b.seq);
+    return true;
+}
+
 template <int HD, int RW, int KSP, bool PAGED, bool TURNS, typename KVT>
 __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k,
@@ -94,19 +169,19 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     static_assert(FL_KT % RPT == 0, "whole staging steps");
 
     // workgroups go round the 8 dies in turn: heads fastest, so that a key
-    // head stays on few of them, long rows of tiles first, and the sequences
-    // rotated from one tile to the next, so that a long one is on all
+    // head stays on few of them, and long rows of tiles first
     const int nseq = pairs / nkv;
-    const int up = blockIdx.x / pairs, tile = gridDim.x / pairs - 1 - up;
-    const int seq =
-        (blockIdx.x % pairs / nkv + (nkv % 8 ? up : 0)) % nseq;
-    const int kvh = blockIdx.x % nkv;
     const int G = nq / nkv;
-    const int s0 = cu[seq], QL = cu[seq + 1] - s0;
-    const int L = PAGED ? seq_lens[seq] : QL;
-    const int hist = L - QL;
-    const int row0 = tile * ROWS;
-    if (row0 >= QL * G) return;
+    const int kvh = blockIdx.x % nkv;
+    FlBlock at;
+    if (!fl_block(cu, PAGED ? seq_lens : nullptr, nseq, G, ROWS,
+                  blockIdx.x / nkv, gridDim.x / pairs, nkv % 8 == 0, at))
+        return;
+    // (or what depends on them would be vectors: up to 9% of a step)
+    auto same = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    const int seq = same(at.seq), s0 = same(at.s0), QL = same(at.QL);
+    const int L = same(at.L), hist = L - QL;
+    const int row0 = same(at.tile) * ROWS;
     const int* bt = PAGED ? block_table + (long)seq * W : nullptr;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -319,7 +394,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             asm volatile("s_barrier" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
         };
-        auto at = [&](int t) { return smem + (t & 3) * 2 * TILE; };
+        auto tile_at = [&](int t) { return smem + (t & 3) * 2 * TILE; };
         // bf16 goes straight to LDS: a wave's loads are 4 rows of 256 bytes,
         // lane l the 16 bytes that belong at l * 16
         const int nt = (kv_end + FL_KT - 1) / FL_KT;
@@ -490,9 +565,9 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             }
             turn();
             if (wid >= 4) turn();
-            read_k(at(0), 0);
-            read_k(at(0), 1);
-            make_s(at(0));
+            read_k(tile_at(0), 0);
+            read_k(tile_at(0), 1);
+            make_s(tile_at(0));
             turn();
             for (int t = 0; t + 1 < nt; ++t) {
                 // V of tile t + 2 takes the place of t - 2's, K of t + 3 that
@@ -507,8 +582,8 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 }
                 first_weights(t * FL_KT);
                 if (!DIRECT) __builtin_amdgcn_s_waitcnt(0xc07f);
-                read_v(at(t), 0);
-                read_v(at(t), 1);
+                read_v(tile_at(t), 0);
+                read_v(tile_at(t), 1);
                 if (DIRECT) {
                     if (t + 3 < nt)
                         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NST)
@@ -518,15 +593,15 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 }
                 turn();
                 __builtin_amdgcn_s_setprio(1);
-                make_o(at(t), std::true_type(), at(t + 1));
-                make_s(at(t + 1));
+                make_o(tile_at(t), std::true_type(), tile_at(t + 1));
+                make_s(tile_at(t + 1));
                 __builtin_amdgcn_s_setprio(0);
                 turn();
             }
             first_weights((nt - 1) * FL_KT);
-            read_v(at(nt - 1), 0);
-            read_v(at(nt - 1), 1);
-            make_o(at(nt - 1), std::false_type(), nullptr);
+            read_v(tile_at(nt - 1), 0);
+            read_v(tile_at(nt - 1), 1);
+            make_o(tile_at(nt - 1), std::false_type(), nullptr);
             if (wid < 4) turn();
         }
     } else {

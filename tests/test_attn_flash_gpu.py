@@ -215,3 +215,39 @@ def test_weights_add_up_to_one(hd, T):
     q, k, _ = _qkv(T, 8, 8, hd, 5)
     got = ops.attn_prefill(q, k, v, _cu([T]), T, hd ** -0.5)
     assert (got == 1).all(), got.float().min().item()
+
+
+@pytest.mark.parametrize("nkv", [4, 8])
+@pytest.mark.parametrize("lens", [
+    [700, 90], [33, 0, 650, 1], [1, 600, 40, 300, 64, 65], [500, 20] * 4,
+    [257, 1, 900], [150, 31, 400, 90, 7], [260, 30, 129] * 3 + [500],
+    [90, 40, 128, 20, 300] * 4])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_blocks_of_every_sequence(hd, lens, nkv):
+    """Every row of tiles of every sequence is taken, however many of them there
+    are and whatever the lengths and histories."""
+    nq = 4 * nkv
+    q, k, v = _qkv(sum(lens), nq, nkv, hd, len(lens))
+    cu, scale = _cu(lens), hd ** -0.5
+    got = ops.attn_prefill(q, k, v, cu, max(lens), scale)
+    want = reference.attn_prefill(q.float(), k.float(), v.float(), cu,
+                                  max(lens), scale)
+    _check(got, want, v)
+    # portions: every second sequence has a history
+    bs, old = 64, [(i % 2) * (40 + 97 * i) for i in range(len(lens))]
+    total = [a + b for a, b in zip(old, lens)]
+    counts = [-(-n // bs) for n in total]
+    table = torch.zeros(len(lens), max(counts), dtype=torch.int32, device=DEV)
+    pages = torch.randperm(sum(counts) + 1, device=DEV).int()
+    at = 0
+    for i, c in enumerate(counts):
+        table[i, :c] = pages[at : at + c]
+        at += c
+    kc, vc = (torch.randn(sum(counts) + 1, nkv, bs, hd, device=DEV).bfloat16()
+              for _ in range(2))
+    sl = torch.tensor(total, dtype=torch.int32, device=DEV)
+    got = ops.attn_prefill_paged(q, kc, vc, table, sl, cu, max(lens), scale)
+    want = reference.attn_decode_with_history(
+        q.float(), kc.float(), vc.float(), table, sl,
+        torch.tensor(lens, dtype=torch.int32), scale)
+    _check(got, want, vc)
