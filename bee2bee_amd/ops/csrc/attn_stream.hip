@@ -514,8 +514,8 @@ static long stream_groups(long pairs, long rows) {
 // / 101), so that verified tokens attend as decoded ones do in steps of more
 // rows than decode_stack.hip takes; to the bit only the last token of each
 // sequence, beside as many sequences in a table as wide (the splits' borders
-// follow from them) and on bf16 pages (decoding rounds its queries on 8-bit
-// ones).
+// follow from them), on bf16 pages (decoding rounds its queries on 8-bit ones)
+// and where decoding has four waves a context, too.
 extern "C" int attn_stream_takes(long pairs, long rows) {
     return rows <= 32 || stream_groups(pairs, rows) <= 448;
 }
@@ -582,10 +582,12 @@ extern "C" int launch_attn_stream(
     // of lengths: bf16 of 250 to 2000 tokens, 16 sequences 19.2 / 20.3, 24 27.4 /
     // 25.3, 48 45.0 / 39.4, 96 74.7 / 74.0, of 500 to 4000 12 28.7 / 26.3, 40
     // 68.6 / 68.3, 64 105.7 / 98.0; fp8 16 16.7 / 15.3, 24 18.7 / 19.3, 32 23.6 /
-    // 21.1, 12 20.8 / 18.8, 64 56.7 / 60.8.
+    // 21.1, 12 20.8 / 18.8, 64 56.7 / 60.8. Chunks, of about one length and in no
+    // such order, stay with four (64 sequences' 2 tokens on 2000 84.0 / 85.7).
     const long wgs = (long)grid.x * grid.z * even;
     const bool wide =
-        whole && (fp8 ? wgs <= 320 : wgs > 256 && wgs / even <= 512);
+        whole && !cu &&
+        (fp8 ? wgs <= 320 : wgs > 256 && wgs / even <= 512);
     const int waves = wide ? 8 : 4;
     const int smem = waves * 2 * ST_KEYS * hd * 2 +
                      qt * 16 * waves * 2 * (int)sizeof(float);

@@ -251,8 +251,9 @@ def test_rows_by_length(B):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-def test_chunks_of_eight_waves(fp8):
-    """Two and three row tiles of a chunk, 8 waves a context."""
+def test_chunks_of_many_contexts(fp8):
+    """Two and three row tiles of a chunk, as many contexts as decoding would
+    have eight waves for."""
     for new, old in ([4, 5, 1] * 4, [300, 0, 255] * 4), ([9] * 13, [600] * 13):
         total = [a + b for a, b in zip(new, old)]
         kc, vc, table, lens = _pages(8, 128, 256, total, fp8, 2)
