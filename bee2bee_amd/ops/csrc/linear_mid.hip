@@ -38,7 +38,11 @@
 // at 80; 2x8192x2048 16.0 / 14.7 at 57; 2x14336x4096 45.0 / 43.2 at 80; with 48 and
 // 24 KB a third to half more time). The input needs four slots, better six (with
 // two 44 -> 61 us at 80 rows); its rows apart by an odd number of lines change
-// nothing.
+// nothing. A CU takes in 57 GB/s from memory, 50 to 60 of weights and input
+// together, so what a slot has past the rows and tiles that there are is not loaded
+// (loaded / not: 2x18944x3584 47.5 / 46.4 at 24 rows, 54.8 / 52.4 at 80, 103 / 96 at
+// 200, 123 / 109 at 256; 2x14336x4096 40.2 / 39.2 at 57, 43.8 / 42.4 at 80, 63.0 / 62.2
+// at 200; 6144x4096 14.4 / 13.9 at 80; others within 1%).
 //
 // Measured (us, launch after launch with weights that no cache holds, 24 / 80 / 128
 // / 200 / 256 rows; in brackets with one loop and the long rings):
@@ -58,18 +62,24 @@ DEV_INLINE unsigned lm_lds(const void* p) {
     return (unsigned)(unsigned long)(
         __attribute__((address_space(3))) const char*)p;
 }
-// 16 bytes a lane from base + off to LDS at `to` + lane * 16. The compiler does
-// not see these loads: lm_wait counts them. (M0 is set where it is used.)
+// 16 bytes a lane of `lanes` from base + off to LDS at `to` + lane * 16 (all lanes
+// are active before and after). The compiler does not see these loads: lm_wait
+// counts them, those of no lane too. (M0 is set where it is used.)
 template <bool STREAM>
-DEV_INLINE void lm_load(const void* base, unsigned off, unsigned to) {
+DEV_INLINE void lm_load(const void* base, unsigned off, unsigned to,
+                        unsigned long lanes) {
     if constexpr (STREAM)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %1 nt"
-                     ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\t"
+                     "global_load_lds_dwordx4 %0, %1 nt\n\t"
+                     "s_mov_b64 exec, -1"
+                     ::"v"(off), "s"(base), "s"(to), "s"(lanes)
+                     : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, %1"
-                     ::"v"(off), "s"(base), "s"(to) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\t"
+                     "global_load_lds_dwordx4 %0, %1\n\t"
+                     "s_mov_b64 exec, -1"
+                     ::"v"(off), "s"(base), "s"(to), "s"(lanes)
+                     : "memory", "m0");
 }
 // until at most `left` stages, of LO to HI, of PER loads each are under way
 template <int PER, int LO, int HI>
@@ -118,6 +128,13 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     const bool of_w = wid < 4;
     const int r8 = lane >> 3, p8 = lane & 7;
     unsigned off[NLW > NLX ? NLW : NLX];
+    // of the tiles and rows that there are: others' places in LDS hold anything,
+    // and only their own sums come of it
+    unsigned lanes[NLW > NLX ? NLW : NLX][2];
+    auto only = [&](int j, unsigned long of) {
+        lanes[j][0] = __builtin_amdgcn_readfirstlane((unsigned)of);
+        lanes[j][1] = __builtin_amdgcn_readfirstlane((unsigned)(of >> 32));
+    };
     const char* src = reinterpret_cast<const char*>(of_w ? w : x);
     auto rows_of = [&](int grp) {              // (tiles past the last: its)
         const int t0 = grp * tiles;
@@ -128,6 +145,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
             const int i = wid * NLW + j;
             const int r = (i & 1) * 8 + r8;
             const int t = min(t0 + min(i >> 1, tiles - 1), NT - 1);
+            only(j, (i >> 1) < tiles && t0 + (i >> 1) < NT ? ~0ul : 0ul);
             const long row = OUT == LM_GATED
                                  ? (long)t * 8 + r8 + (i & 1) * (long)N
                                  : min(t * 16 + r, N - 1) - t0 * 16;
@@ -142,6 +160,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
             const int r = ((wid - 4) * NLX + j) * 8 + r8;
             off[j] = (unsigned)(((long)min(r, M - 1) * K +
                                  (p8 ^ (r >> 1 & 7)) * 8) * 2);
+            only(j, __ballot(r < M));
         }
     }
     const unsigned to0 = lm_lds(smem) +
@@ -154,7 +173,8 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
         if (W || MT > 1 || wid < 6)            // (MT 1: two waves' are all)
 #pragma unroll
             for (int j = 0; j < (W ? NLW : NLX); ++j)
-                lm_load<W>(at, off[j], to0 + lslot * (W ? WB : XB) + j * 1024);
+                lm_load<W>(at, off[j], to0 + lslot * (W ? WB : XB) + j * 1024,
+                           lanes[j][0] | (unsigned long)lanes[j][1] << 32);
         if (++lslot == (W ? DW : DX)) lslot = 0;
         at += 128;
         if (++lk == n) {
