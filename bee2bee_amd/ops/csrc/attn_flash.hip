@@ -148,13 +148,39 @@ DEV_INLINE bool fl_block(const int* cu, const int* seq_lens, int nseq, int G,
     return true;
 }
 
-template <int HD, int RW, int KSP, bool PAGED, bool TURNS, typename KVT>
+// What one sequence's blocks beyond whole rounds of 256 workgroups are shared by
+struct FlShare {
+    int from;                  // the first of the 256 workgroups that share them
+    float *o, *ml;             // [512, 256, 128], [512, 256, 2]: a block's pieces
+};
+constexpr int FL_SHARERS = 256;
+
+// Whether `rest` blocks of a sequence of L tokens are shared: what it saves is half
+// of the chip's idle part of a last round, as long as a block of all keys; pieces
+// and their sums cost 50 us. us, whole / shared, 32/8 heads: 2100 on 2200 147 / 154
+// (264 blocks), on 4000 232 / 206, on 8000 418 / 310, on 16000 808 / 555; 2500 (320) on 2600
+// 185 / 188, on 8000 442 / 381; 28/4: 3150 (348) on 3200 228 / 252, on 8000 459 / 435, 5000
+// (548) on 14000 1246 / 1035; 4096 (448) on 12288 779 / 845.
+__host__ __device__ inline bool fl_worth(int rest, long L) {
+    return rest > 0 && rest <= 96 && (256 - rest) * L >= 5800L * 256;
+}
+
+// tiles of 64 keys that the block `tile` of a sequence has
+DEV_INLINE int fl_tiles(int tile, int rows, int G, int QL, int hist) {
+    if (tile * rows >= QL * G) return 0;
+    return (hist + min((tile + 1) * rows - 1, QL * G - 1) / G + FL_KT) / FL_KT;
+}
+
+// SHARE: one sequence; workgroups from share.from on take parts of the last blocks
+template <int HD, int RW, int KSP, bool PAGED, bool TURNS, bool SHARE,
+          typename KVT>
 __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k,
     const KVT* __restrict__ v, const int* __restrict__ cu,
     const int* __restrict__ block_table, const int* __restrict__ seq_lens,
-    unsigned short* __restrict__ out, int nq, int nkv, long s_q, long s_k,
-    long s_v, int W, int bs, int pairs, float scale_log2) {
+    unsigned short* __restrict__ out, int blocks, int nq, int nkv, long s_q,
+    long s_k, long s_v, int W, int bs, int pairs, float scale_log2,
+    const FlShare share) {
     constexpr int NW = RW * KSP;           // waves
     constexpr int ROWS = RW * 32;          // query rows of a workgroup
     constexpr int NF = 2 / KSP;            // 32-key tiles of a wave's step
@@ -168,20 +194,20 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     static_assert(!TURNS || (HD == 128 && RW == 8 && KSP == 1), "");
     static_assert(FL_KT % RPT == 0, "whole staging steps");
 
-    // workgroups go round the 8 dies in turn: heads fastest, so that a key
-    // head stays on few of them, and long rows of tiles first
-    const int nseq = pairs / nkv;
-    const int G = nq / nkv;
-    const int kvh = blockIdx.x % nkv;
-    FlBlock at;
-    if (!fl_block(cu, PAGED ? seq_lens : nullptr, nseq, G, ROWS,
-                  blockIdx.x / nkv, gridDim.x / pairs, nkv % 8 == 0, at))
-        return;
-    // (or what depends on them would be vectors: up to 9% of a step)
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    // two buffers, or four, of a K and a V tile each
+    // (numbers that are scalars, or what depends on them would be vectors: up to 9%
+    // of a step)
     auto same = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
-    const int seq = same(at.seq), s0 = same(at.s0), QL = same(at.QL);
-    const int L = same(at.L), hist = L - QL;
-    const int row0 = same(at.tile) * ROWS;
+    const int G = nq / nkv, kvh = blockIdx.x % nkv;
+
+    // The tiles t0 .. t1 - 1 (t1 0: all) of a block; piece: where its sums go, -1:
+    // they are the result
+    auto block = [&](const int seq, const int s0, const int QL, const int L,
+                     const int tile, const int t0, const int t1,
+                     const int piece) __attribute__((always_inline)) {
+    const int hist = L - QL;
+    const int row0 = tile * ROWS;
     const int* bt = PAGED ? block_table + (long)seq * W : nullptr;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -189,9 +215,6 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const int lr = lane & 31, hi = lane >> 5;
     const int rw = KSP == 1 ? wid : wid % RW;     // row block of the wave
     const int f0 = KSP == 1 ? 0 : wid / RW;       // its first 32-key tile
-
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    // two buffers, or four, of a K and a V tile each
 
     // ---- this lane's query row
     const int R = row0 + rw * 32 + lr;
@@ -397,7 +420,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         auto tile_at = [&](int t) { return smem + (t & 3) * 2 * TILE; };
         // bf16 goes straight to LDS: a wave's loads are 4 rows of 256 bytes,
         // lane l the 16 bytes that belong at l * 16
-        const int nt = (kv_end + FL_KT - 1) / FL_KT;
+        const int nt = (kv_end + FL_KT - 1) / FL_KT, te = SHARE ? t1 : nt;
         unsigned off[2][2][NST];               // K, V; a whole tile, the last
 #pragma unroll
         for (int i = 0; i < NST; ++i) {
@@ -419,17 +442,18 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         // Tiles are asked for in order, K's one ahead of V's: where the next
         // ones lie in memory and in LDS, and what is left of K's page.
         const char *k_src = nullptr, *v_src = nullptr, *v_next = nullptr;
-        int k_to = 0, v_to = TILE, k_left = 0, k_at = 0;
+        int k_to = (t0 & 3) * 2 * TILE, v_to = k_to + TILE, k_left = 0, k_at = 0;
         auto page_of = [&](const KVT* pool, int b) {
             return reinterpret_cast<const char*>(
                 pool + ((long)b * nkv + kvh) * bs * HD);
         };
         if (DIRECT && nt > 0) {
             if (PAGED) {
-                const int b = bt[0];
-                k_src = page_of(k, b);
-                v_src = page_of(v, b);
-                k_left = bs;
+                k_at = t0 * FL_KT / bs;
+                const int b = bt[k_at], in = t0 * FL_KT - k_at * bs;
+                k_src = page_of(k, b) + in * RB;
+                v_src = page_of(v, b) + in * RB;
+                k_left = bs - in;
             } else {
                 k_src = reinterpret_cast<const char*>(
                     k + (long)s0 * s_k + (long)kvh * HD);
@@ -440,7 +464,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         }
         int new_page = 0;                      // asked for a turn ahead
         auto load_k = [&](int t) {
-            if (t >= nt) return;
+            if (t >= te) return;
             if (t + 1 == nt)
 #pragma unroll
                 for (int i = 0; i < NST; ++i) off[0][0][i] = off[0][1][i];
@@ -458,7 +482,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 new_page = bt[++k_at];
         };
         auto load_v = [&](int t) {
-            if (t >= nt) return;
+            if (t >= te) return;
             if (t + 1 == nt)
 #pragma unroll
                 for (int i = 0; i < NST; ++i) off[1][0][i] = off[1][1][i];
@@ -547,11 +571,11 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         };
         if (nt > 0) {
             if (DIRECT) {
-                load_k(0);
-                load_v(0);
-                load_k(1);
-                load_v(1);
-                load_k(2);
+                load_k(t0);
+                load_v(t0);
+                load_k(t0 + 1);
+                load_v(t0 + 1);
+                load_k(t0 + 2);
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
                 load_tile(0);
@@ -565,11 +589,11 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             }
             turn();
             if (wid >= 4) turn();
-            read_k(tile_at(0), 0);
-            read_k(tile_at(0), 1);
-            make_s(tile_at(0));
+            read_k(tile_at(t0), 0);
+            read_k(tile_at(t0), 1);
+            make_s(tile_at(t0));
             turn();
-            for (int t = 0; t + 1 < nt; ++t) {
+            for (int t = t0; t + 1 < te; ++t) {
                 // V of tile t + 2 takes the place of t - 2's, K of t + 3 that
                 // of t - 1's: their last readers were in the turn before. What
                 // the last such turn asked for has come by the end of this.
@@ -585,7 +609,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 read_v(tile_at(t), 0);
                 read_v(tile_at(t), 1);
                 if (DIRECT) {
-                    if (t + 3 < nt)
+                    if (t + 3 < te)
                         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NST)
                                      : "memory");
                     else
@@ -598,10 +622,10 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 __builtin_amdgcn_s_setprio(0);
                 turn();
             }
-            first_weights((nt - 1) * FL_KT);
-            read_v(tile_at(nt - 1), 0);
-            read_v(tile_at(nt - 1), 1);
-            make_o(tile_at(nt - 1), std::false_type(), nullptr);
+            first_weights((te - 1) * FL_KT);
+            read_v(tile_at(te - 1), 0);
+            read_v(tile_at(te - 1), 1);
+            make_o(tile_at(te - 1), std::false_type(), nullptr);
             if (wid < 4) turn();
         }
     } else {
@@ -652,6 +676,22 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             for (int r = 0; r < 16; ++r)
                 o[d][r] = o[d][r] * a0 + mg[(d * 16 + r) * 64] * a1;
     }
+    if (SHARE && piece >= 0) {
+        const int row = rw * 32 + lr;
+        float* to = share.o + ((long)piece * ROWS + row) * HD;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                *reinterpret_cast<f32x4*>(to + d * 32 + r4 * 8 + hi * 4) =
+                    f32x4{o[d][r4 * 4], o[d][r4 * 4 + 1], o[d][r4 * 4 + 2],
+                          o[d][r4 * 4 + 3]};
+        if (hi == 0) {
+            share.ml[((long)piece * ROWS + row) * 2] = m;
+            share.ml[((long)piece * ROWS + row) * 2 + 1] = l;
+        }
+        return;
+    }
     if (!row_ok) return;
     const float inv = l == 0.f ? 0.f : 1.f / l;
     unsigned short* orow = out + ((long)(s0 + pos) * nq + head) * HD;
@@ -665,6 +705,103 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
                 w[e] = (short)f2bf(o[d][r4 * 4 + e] * inv);
             *reinterpret_cast<short4v*>(orow + d * 32 + r4 * 8 + hi * 4) = w;
         }
+    };
+
+    const bool shared =
+        SHARE && fl_worth(blocks - share.from, seq_lens[0]);
+    if (SHARE && !shared && blockIdx.x >= (unsigned)blocks) return;
+    if (!shared || blockIdx.x < (unsigned)share.from) {
+        // workgroups go round the 8 dies in turn: heads fastest, so that a key
+        // head stays on few of them, and long rows of tiles first
+        FlBlock at;
+        if (SHARE) {
+            at.seq = 0;
+            at.s0 = cu[0];
+            at.QL = cu[1] - at.s0;
+            at.L = seq_lens[0];
+            at.tile = blocks / nkv - 1 - blockIdx.x / nkv;
+            if (at.tile * ROWS >= at.QL * G) return;
+        } else if (!fl_block(cu, PAGED ? seq_lens : nullptr, pairs / nkv, G, ROWS,
+                             blockIdx.x / nkv, blocks / pairs, nkv % 8 == 0,
+                             at)) {
+            return;
+        }
+        const int QL = same(at.QL), L = same(at.L), tile = same(at.tile);
+        const int hist = L - QL;
+        block(same(at.seq), same(at.s0), QL, L, tile, 0,
+              SHARE ? fl_tiles(tile, ROWS, G, QL, hist) : 0, -1);
+        return;
+    }
+    if constexpr (SHARE) {
+        const int s0 = cu[0], QL = cu[1] - s0, L = seq_lens[0], hist = L - QL;
+        const int rest = (blocks - share.from) / nkv;
+        const int sharers = FL_SHARERS / nkv;
+        const int w = blockIdx.x - share.from, mine = w / nkv;
+        int total = 0;
+        for (int t = 0; t < rest; ++t) total += fl_tiles(t, ROWS, G, QL, hist);
+        const int lo = (long)total * mine / sharers;
+        const int hi_ = (long)total * (mine + 1) / sharers;
+        int before = 0;
+        for (int t = 0; t < rest && before < hi_; ++t) {
+            const int n = fl_tiles(t, ROWS, G, QL, hist);
+            const int a = max(lo - before, 0), b = min(hi_ - before, n);
+            before += n;
+            if (a >= b) continue;
+            block(0, s0, QL, L, t, a, b,
+                  a == 0 && b == n ? -1 : w * 2 + (a == 0));
+            __syncthreads();                   // the tiles are read
+        }
+    }
+}
+
+// The pieces of shared blocks: workgroup = (block, 8 of its rows), 32 threads a
+// row, 4 coordinates each
+__global__ __launch_bounds__(256) void attn_flash_join_kernel(
+    const FlShare share, const int* __restrict__ cu,
+    const int* __restrict__ seq_lens, unsigned short* __restrict__ out, int nq,
+    int nkv, int blocks) {
+    constexpr int ROWS = 256, HD = 128;
+    const int G = nq / nkv;
+    if (!fl_worth(blocks - share.from, seq_lens[0])) return;
+    const int s0 = cu[0], QL = cu[1] - s0, hist = seq_lens[0] - QL;
+    const int kvh = blockIdx.x / 32 % nkv, tile = blockIdx.x / 32 / nkv;
+    const int rest = (blocks - share.from) / nkv, sharers = FL_SHARERS / nkv;
+    int total = 0, before = 0;
+    for (int t = 0; t < rest; ++t) {
+        if (t == tile) before = total;
+        total += fl_tiles(t, ROWS, G, QL, hist);
+    }
+    const int n = fl_tiles(tile, ROWS, G, QL, hist);
+    const int row = blockIdx.x % 32 * 8 + threadIdx.x / 32;
+    const int c = threadIdx.x % 32 * 4, R = tile * ROWS + row;
+    if (n == 0 || R >= QL * G) return;
+    // who has the block's first tile
+    int w = (long)before * sharers / total;
+    while ((long)total * (w + 1) / sharers <= before) ++w;
+    if ((long)total * (w + 1) / sharers >= before + n) return;   // and all others
+    float M = -1e30f, sum = 0.f;
+    f32x4 acc{0.f, 0.f, 0.f, 0.f};
+    for (bool first = true; (long)total * w / sharers < before + n;
+         ++w, first = false) {
+        if ((long)total * (w + 1) / sharers == (long)total * w / sharers)
+            continue;                          // (fewer tiles than sharers)
+        const long at = ((long)(w * nkv + kvh) * 2 + first) * ROWS + row;
+        const float m = share.ml[at * 2], l = share.ml[at * 2 + 1];
+        const f32x4 o = *reinterpret_cast<const f32x4*>(share.o + at * HD + c);
+        const float mn = fmaxf(M, m);
+        const float old = __builtin_amdgcn_exp2f(M - mn);
+        const float now = __builtin_amdgcn_exp2f(m - mn);
+        M = mn;
+        sum = sum * old + l * now;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = acc[e] * old + o[e] * now;
+    }
+    const float inv = sum == 0.f ? 0.f : 1.f / sum;
+    short4v y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = (short)f2bf(acc[e] * inv);
+    *reinterpret_cast<short4v*>(
+        out + ((long)(s0 + R / G) * nq + kvh * G + R % G) * HD + c) = y;
 }
 
 // ------------------------------------------------------------- launchers
@@ -754,13 +891,40 @@ extern "C" int attn_flash_form(long T, int nseq, int nq, int nkv, int hd,
     return (256 >> shape) + (shape == 0 && turns);
 }
 
-#define FL_ONE(HDV, RWV, KSPV, PG, TU, KVT)                                     \
-    hipLaunchKernelGGL(                                                       \
-        (attn_flash_kernel<HDV, RWV, KSPV, PG, TU, KVT>),                        \
-        dim3((unsigned)((rows + RWV * 32 - 1) / (RWV * 32) * pairs)),         \
-        dim3(RWV * KSPV * 64), flash_smem(HDV, RWV, KSPV, TU), stream, q,     \
-        (const KVT*)k, (const KVT*)v, cu, block_table, seq_lens, out, nq,     \
-        nkv, s_q, s_k, s_v, W, bs, pairs, scale * LOG2E)
+// Workgroups of a step that take whole blocks where 256 more share the rest, 0:
+// all take whole ones. One portion, of bf16 pages: its blocks are about as long as
+// each other, and what is left over whole rounds of 256 takes as long as a round.
+// W * bs: the most tokens that it may have; the kernel looks at those it has.
+extern "C" int attn_flash_share(int nseq, int nq, int nkv, int hd, int max_qlen,
+                                int W, int bs, int fp8, int shape256) {
+    if (nseq != 1 || hd != 128 || fp8 || !shape256 || FL_SHARERS % nkv) return 0;
+    const long blocks = ((long)max_qlen * (nq / nkv) + 255) / 256 * nkv;
+    const long rest = blocks % 256;
+    if (blocks < 256 || blocks > 1 << 20 || !fl_worth(rest, (long)W * bs))
+        return 0;
+    return (int)(blocks - rest);
+}
+
+// fp32 numbers that a step's pieces take, 0: it has none
+extern "C" long attn_flash_pieces(long T, int nseq, int nq, int nkv, int hd,
+                                  int max_qlen, int W, int bs, int fp8) {
+    const bool turns = flash_turns(hd, true, bs, true);
+    if (nseq != 1 || max_qlen < 1 || !turns) return 0;
+    const int shape = flash_shape(hd, T, nseq, nq, nkv, max_qlen, true, turns);
+    return attn_flash_share(nseq, nq, nkv, hd, max_qlen, W, bs, fp8, shape == 0)
+               ? 512L * 256 * (128 + 2) : 0;
+}
+
+#define FL_ONE(HDV, RWV, KSPV, PG, TU, KVT)                                   \
+    do {                                                                      \
+        const int blocks = (rows + RWV * 32 - 1) / (RWV * 32) * pairs;        \
+        hipLaunchKernelGGL(                                                   \
+            (attn_flash_kernel<HDV, RWV, KSPV, PG, TU, false, KVT>),          \
+            dim3((unsigned)blocks), dim3(RWV * KSPV * 64),                    \
+            flash_smem(HDV, RWV, KSPV, TU), stream, q, (const KVT*)k,         \
+            (const KVT*)v, cu, block_table, seq_lens, out, blocks, nq, nkv,   \
+            s_q, s_k, s_v, W, bs, pairs, scale * LOG2E, FlShare{});           \
+    } while (0)
 #define FL_HD(HDV, PG, KVT)                                                   \
     do {                                                                      \
         if (shape == 0 && HDV == 128 && turns)                                \
@@ -779,9 +943,10 @@ constexpr float LOG2E = 1.44269504088896340736f;
 // below 2^24 (a tile's offsets are of 32 bits). Nonzero for any other.
 extern "C" int launch_attn_flash(
     const unsigned short* q, const void* k, const void* v, const int* cu,
-    const int* block_table, const int* seq_lens, unsigned short* out, long T,
-    int nseq, int nq, int nkv, int hd, long s_q, long s_k, long s_v, int W,
-    int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
+    const int* block_table, const int* seq_lens, unsigned short* out,
+    float* pieces, long T, int nseq, int nq, int nkv, int hd, long s_q, long s_k,
+    long s_v, int W, int bs, int max_qlen, float scale, int fp8,
+    hipStream_t stream) {
     if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
     const bool aligned = ((unsigned long)k | (unsigned long)v) % 16 == 0;
     if (!block_table && (!aligned || s_k % 8 || s_v % 8 || s_k >= 1 << 24 ||
@@ -793,6 +958,23 @@ extern "C" int launch_attn_flash(
     const bool turns = flash_turns(hd, block_table, bs, aligned);
     const int shape =
         flash_shape(hd, T, nseq, nq, nkv, max_qlen, block_table, turns);
+    const int from = pieces ? attn_flash_share(nseq, nq, nkv, hd, max_qlen, W, bs,
+                                               fp8, shape == 0 && turns)
+                            : 0;
+    if (from && block_table) {
+        const int blocks = (int)((rows + 255) / 256 * pairs);
+        const FlShare share{from, pieces + 512 * 256 * 2, pieces};
+        hipLaunchKernelGGL(
+            (attn_flash_kernel<128, 8, 1, true, true, true, unsigned short>),
+            dim3(from + FL_SHARERS), dim3(512), flash_smem(128, 8, 1, true),
+            stream, q, (const unsigned short*)k, (const unsigned short*)v, cu,
+            block_table, seq_lens, out, blocks, nq, nkv, s_q, s_k, s_v, W, bs,
+            pairs, scale * LOG2E, share);
+        hipLaunchKernelGGL(attn_flash_join_kernel, dim3((blocks - from) * 32),
+                           dim3(256), 0, stream, share, cu, seq_lens, out, nq,
+                           nkv, blocks);
+        return 0;
+    }
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

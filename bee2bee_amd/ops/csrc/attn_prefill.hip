@@ -456,17 +456,18 @@ static int prefill_mfma_smem(int hd) {
 // attn_flash.hip: head size 64 or 128 and a positive scale, nonzero otherwise
 extern "C" int launch_attn_flash(
     const unsigned short* q, const void* k, const void* v, const int* cu,
-    const int* block_table, const int* seq_lens, unsigned short* out, long T,
-    int nseq, int nq, int nkv, int hd, long s_q, long s_k, long s_v, int W,
-    int bs, int max_qlen, float scale, int fp8, hipStream_t stream);
+    const int* block_table, const int* seq_lens, unsigned short* out,
+    float* pieces, long T, int nseq, int nq, int nkv, int hd, long s_q, long s_k,
+    long s_v, int W, int bs, int max_qlen, float scale, int fp8,
+    hipStream_t stream);
 
 extern "C" void launch_attn_prefill(
     const unsigned short* q, const unsigned short* k, const unsigned short* v,
     const int* cu, unsigned short* out, long T, int nseq, int nq, int nkv,
     int hd, long s_q, long s_k, long s_v, int max_seqlen, float scale,
     int causal, hipStream_t stream) {
-    if (causal && launch_attn_flash(q, k, v, cu, nullptr, nullptr, out, T,
-                                    nseq, nq, nkv, hd, s_q, s_k, s_v, 0, 1,
+    if (causal && launch_attn_flash(q, k, v, cu, nullptr, nullptr, out, nullptr,
+                                    T, nseq, nq, nkv, hd, s_q, s_k, s_v, 0, 1,
                                     max_seqlen, scale, 0, stream) == 0)
         return;
     dim3 grid(nq, nseq);
@@ -483,10 +484,11 @@ extern "C" void launch_attn_prefill(
 extern "C" void launch_attn_prefill_paged(
     const unsigned short* q, const void* k_cache, const void* v_cache,
     const int* cu, const int* block_table, const int* seq_lens,
-    unsigned short* out, long T, int nseq, int nq, int nkv, int hd, long s_q,
-    int W, int bs, int max_qlen, float scale, int fp8, hipStream_t stream) {
+    unsigned short* out, float* pieces, long T, int nseq, int nq, int nkv,
+    int hd, long s_q, int W, int bs, int max_qlen, float scale, int fp8,
+    hipStream_t stream) {
     if (launch_attn_flash(q, k_cache, v_cache, cu, block_table, seq_lens, out,
-                          T, nseq, nq, nkv, hd, s_q, 0, 0, W, bs, max_qlen,
+                          pieces, T, nseq, nq, nkv, hd, s_q, 0, 0, W, bs, max_qlen,
                           scale, fp8, stream) == 0)
         return;
 #define PFP_LAUNCH(KVT)                                                       \

@@ -54,9 +54,10 @@ void launch_attn_prefill(const unsigned short*, const unsigned short*,
                          float, int, hipStream_t);
 void launch_attn_prefill_paged(const unsigned short*, const void*,
                                const void*, const int*, const int*,
-                               const int*, unsigned short*, long, int, int,
-                               int, int, long, int, int, int, float, int,
+                               const int*, unsigned short*, float*, long, int,
+                               int, int, int, long, int, int, int, float, int,
                                hipStream_t);
+long attn_flash_pieces(long, int, int, int, int, int, int, int, int);
 void launch_mfma_probe(const unsigned short*, const unsigned short*, float*,
                        hipStream_t);
 void launch_mfma_probe_fp8(const unsigned char*, const unsigned char*,
@@ -394,11 +395,18 @@ Tensor attn_prefill_paged(const Tensor& q, const Tensor& k_cache,
                     block_table, seq_lens, nullptr, out, nullptr,
                     (int)max_qlen, scale))
         return out;
+    Tensor pieces;
+    if (const long n = attn_flash_pieces(T, nseq, nq, nkv, hd, (int)max_qlen, W,
+                                         bs, fp8))
+        pieces = torch::empty({n}, q.options().dtype(torch::kFloat32));
     launch_attn_prefill_paged(bf16p(q), k_cache.data_ptr(),
                               v_cache.data_ptr(), cu_q.data_ptr<int>(),
                               block_table.data_ptr<int>(),
-                              seq_lens.data_ptr<int>(), bf16p_mut(out), T,
-                              nseq, nq, nkv, hd, q.stride(0), W, bs, (int)max_qlen,
+                              seq_lens.data_ptr<int>(), bf16p_mut(out),
+                              pieces.defined() ? pieces.data_ptr<float>()
+                                               : nullptr,
+                              T, nseq, nq, nkv, hd, q.stride(0), W, bs,
+                              (int)max_qlen,
                               (float)scale, fp8 ? 1 : 0, stream());
     return out;
 }

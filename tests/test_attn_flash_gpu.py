@@ -251,3 +251,34 @@ def test_blocks_of_every_sequence(hd, lens, nkv):
         q.float(), kc.float(), vc.float(), table, sl,
         torch.tensor(lens, dtype=torch.int32), scale)
     _check(got, want, vc)
+
+
+@pytest.mark.parametrize("nq,nkv,new,old,bs", [
+    (32, 8, 2100, 4200, 256),       # 33 rows of blocks of 8 heads: 8 are shared
+    (32, 8, 2049, 3991, 64), (28, 4, 2900, 6000, 256),
+    (16, 1, 4200, 4300, 128),       # 7 blocks, 256 that share them
+    (64, 16, 1090, 6001, 256), (24, 8, 2800, 100, 256),
+])
+def test_a_portion_whose_last_blocks_are_shared(nq, nkv, new, old, bs):
+    """Blocks that are more than whole rounds of 256 are cut by keys and joined;
+    blocks that no cut meets, and rows that see no key of a piece, among them."""
+    hd, total = 128, new + old
+    pages = -(-max(total, 6400) // bs)  # (room for more: the kernel finds out)
+    g = torch.Generator(device=DEV).manual_seed(new)
+    table = torch.randperm(pages, generator=g, device=DEV).int()[None]
+    kc, vc = (torch.randn(pages, nkv, bs, hd, generator=g,
+                          device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(new, nq, hd, generator=g, device=DEV).bfloat16()
+    sl = torch.tensor([total], dtype=torch.int32, device=DEV)
+    got = ops.attn_prefill_paged(q, kc, vc, table, sl, _cu([new]), new, 0.1)
+    at = torch.cat([torch.arange(0, 80), torch.randint(0, new, (200,)),
+                    torch.arange(new - 80, new)]).to(DEV)
+    k = kc[table[0].long()].transpose(1, 2).reshape(-1, nkv, hd)[:total].float()
+    v = vc[table[0].long()].transpose(1, 2).reshape(-1, nkv, hd)[:total].float()
+    k, v = (t.repeat_interleave(nq // nkv, 1).transpose(0, 1).contiguous()
+            for t in (k, v))
+    sc = q[at].float().transpose(0, 1) @ k.transpose(1, 2).contiguous() * 0.1
+    ahead = torch.arange(total, device=DEV) > (old + at)[:, None]
+    want = torch.softmax(sc.masked_fill(ahead, -torch.inf), -1) @ v
+    _check(got[at], want.transpose(0, 1), vc)
+    assert torch.isfinite(got).all()
