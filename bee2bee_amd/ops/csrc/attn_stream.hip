@@ -25,21 +25,26 @@
 // one of 3000 8.5 instead of 15.3; 16 sequences' 5 tokens on 1500 24 instead
 // of 166. Loads two tiles ahead gain nothing on fp8 rows (121) and spill on
 // others. A CU draws 45 to 57 GB/s of what no cache holds, from 32 KB under way on,
-// so that what is left to gain are CUs without work: contexts of up to 512
-// workgroups have eight waves each, and longer ones start first (figures at
-// launch_attn_stream and decode_plan). Whole pages are told at compile time: with
-// the look-up of a key's page in the loop, for pages that tiles cross, a step of a
-// wave was 697 instructions, of which 300 are left (200 sequences of up to 3000 fp8
-// 121 -> 118 us, 16 sequences' 5 tokens on 1500 23.8 -> 23.5, 8 of 4000 20.7 -> 20.0).
+// so that what is left to gain are CUs without work: longer contexts start first
+// (figures at decode_plan). Whole pages are told at compile time: with the look-up of
+// a key's page in the loop, for pages that tiles cross, a step of a wave was 697
+// instructions, of which 300 are left (200 sequences of up to 3000 fp8 121 -> 118 us,
+// 16 sequences' 5 tokens on 1500 23.8 -> 23.5, 8 of 4000 20.7 -> 20.0).
 #include "common.h"
-
-#include <type_traits>
 
 typedef __attribute__((ext_vector_type(4))) short short4v;
 typedef __attribute__((address_space(3))) short4v lds_short4v;
 
+// Eight waves of a context gain 3 to 16% in uneven batches that start in the order
+// of their lengths, and lose elsewhere: such a workgroup has a CU to itself. us, four /
+// eight waves, 8 key heads of size 128, 24, 40 and 64 sequences: of 250 to 2000 tokens
+// by length 27.4 / 24.1, 38.6 / 35.4, 52.3 / 49.0; of 2000 38.2 / 40.5, 64.7 / 67.4,
+// 82.5 / 83.8; of 200 10.1 / 11.8, 11.8 / 13.6, 13.6 / 16.4; of 5 to 40 6.1 / 6.0, 6.8 /
+// 8.9, 7.4 / 10.4; fp8 pages, 17 of 2000 21.3 / 25.7, 20 of 200 9.8 / 12.4, 40 of 250 to
+// 2000 by length 25.5 / 22.0. The lengths are on the GPU, so no rule tells them apart.
+constexpr int ST_WAVES = 4;
 constexpr int ST_KEYS = 32;                      // keys of a wave's tile
-constexpr int ST_UNIT = 4 * ST_KEYS;             // splits are of so many keys
+constexpr int ST_STEP = ST_WAVES * ST_KEYS;      // keys of a workgroup's step
 constexpr float ST_LOG2E = 1.44269504088896340736f;
 
 // 16 bytes of a row, as read
@@ -90,12 +95,12 @@ DEV_INLINE bf16x8 st_round_fp8(bf16x8 x, float scale) {
 // keys per split, the same for every reader: a context in `even` parts of whole
 // steps of a workgroup, none above `most` keys (whole steps too)
 DEV_INLINE int split_keys(int L, int even, int most) {
-    return min(((L + even - 1) / even + ST_UNIT - 1) / ST_UNIT * ST_UNIT, most);
+    return min(((L + even - 1) / even + ST_STEP - 1) / ST_STEP * ST_STEP, most);
 }
 
 // WHOLE: bs is a multiple of ST_KEYS, so that no tile crosses pages
-template <int WAVES, int HD, int QT, typename KVT, bool STREAM, bool WHOLE>
-__global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
+template <int HD, int QT, typename KVT, bool STREAM, bool WHOLE>
+__global__ __launch_bounds__(ST_WAVES * 64, 2) void attn_stream_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k_cache,
     const KVT* __restrict__ v_cache, const int* __restrict__ cu,
     const int* __restrict__ block_table, const int* __restrict__ seq_lens,
@@ -103,11 +108,6 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
     float* __restrict__ out_ml, float* __restrict__ part_o,
     float* __restrict__ part_ml, int nkv, int G, int W, int bs, int Z, int even,
     int most, int max_rows, long s_q, float scale) {
-    constexpr int STEP = WAVES * ST_KEYS;  // keys of a workgroup's step
-    // a tile's values are waited for behind its scores (24 sequences of up to 2000
-    // 24.5 us, 25.7 with both before them, 64 of 4000 97.7 and 100.3; of four waves
-    // fp8 takes 124 so, 118 not)
-    constexpr bool APART = WAVES == 8;
     constexpr int KS = HD / 32;          // k steps of a score tile
     constexpr int DT = HD / 16;          // output tiles of 16 coordinates
     constexpr int PC = 2 / sizeof(KVT);  // chunks of 8 elements of a load
@@ -176,18 +176,11 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
     // the chip (query rows past 32 aside), so it is only streamed through L2.
     const int ld_row = lane / CPR, ld_c = lane % CPR * PC;
     st_raw rk[NL], rv[NL];
-    using Yes = std::true_type;
-    using No = std::false_type;
-    auto load_tile = [&](int kb, auto keys, auto values) {
-        constexpr bool K = decltype(keys)::value, V = decltype(values)::value;
-        auto load = [&](int i, const KVT* k, const KVT* v, long off) {
-            if constexpr (K)
-                rk[i] = st_load<STREAM>(
-                    reinterpret_cast<const st_raw*>(k + off));
-            if constexpr (V)
-                rv[i] = st_load<STREAM>(
-                    reinterpret_cast<const st_raw*>(v + off));
-        };
+    auto load = [&](int i, const KVT* k, const KVT* v, long off) {
+        rk[i] = st_load<STREAM>(reinterpret_cast<const st_raw*>(k + off));
+        rv[i] = st_load<STREAM>(reinterpret_cast<const st_raw*>(v + off));
+    };
+    auto load_tile = [&](int kb) {
         if constexpr (WHOLE) {
             // a tile inside one page: the page is a scalar look-up, and a lane's
             // rows lie at 32-bit offsets from it
@@ -212,25 +205,6 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
             }
         }
     };
-    // registers -> LDS, 16-byte chunks xor-ed by the key
-    auto stage = [&](auto keys, auto values) {
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int row = ld_row + i * RPI;
-#pragma unroll
-            for (int p = 0; p < PC; ++p) {
-                if constexpr (decltype(keys)::value)
-                    *reinterpret_cast<short8*>(
-                        kd + row * RB + (((ld_c + p) ^ k_swz(row)) << 4)) =
-                        st_piece<KVT>(rk[i], p);
-                if constexpr (decltype(values)::value)
-                    *reinterpret_cast<short8*>(
-                        kd + TILE + row * RB +
-                        (((ld_c + p) ^ v_swz(row)) << 4)) =
-                        st_piece<KVT>(rv[i], p);
-            }
-        }
-    };
 
     // ---- fragment addresses: K row li (+ 16), chunk ks * 4 + lg; V through
     // the transposing read, 16 lanes on 4 keys x 16 coordinates
@@ -251,23 +225,24 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
     }
 
     int kb = k0 + wid * ST_KEYS;
-    if constexpr (APART) {
-        if (kb < k1) load_tile(kb, Yes(), No());
-        if (kb < k1) load_tile(kb, No(), Yes());
-    } else if (kb < k1) {
-        load_tile(kb, Yes(), Yes());
-    }
-    for (; kb < k1; kb += STEP) {
-        // ---- the tile into LDS, and the next one's loads on their way over
-        // this one's products
-        const bool more = kb + STEP < k1;
-        if constexpr (APART) stage(Yes(), No());
-        else stage(Yes(), Yes());
-        if constexpr (APART) {
-            if (more) load_tile(kb + STEP, Yes(), No());
-        } else if (more) {
-            load_tile(kb + STEP, Yes(), Yes());
+    if (kb < k1) load_tile(kb);
+    for (; kb < k1; kb += ST_STEP) {
+        // ---- registers -> LDS (16-byte chunks xor-ed by the key), and the
+        // next tile's loads on their way over this tile's products
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int row = ld_row + i * RPI;
+#pragma unroll
+            for (int p = 0; p < PC; ++p) {
+                *reinterpret_cast<short8*>(
+                    kd + row * RB + (((ld_c + p) ^ k_swz(row)) << 4)) =
+                    st_piece<KVT>(rk[i], p);
+                *reinterpret_cast<short8*>(
+                    kd + TILE + row * RB + (((ld_c + p) ^ v_swz(row)) << 4)) =
+                    st_piece<KVT>(rv[i], p);
+            }
         }
+        if (kb + ST_STEP < k1) load_tile(kb + ST_STEP);
         WAVE_LDS_SYNC();
 
         // ---- S^T = K Q^T: column = query row, rows = 16 keys
@@ -329,11 +304,6 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
             // what rounding does to both cancels
             l[t] = add_bf16x8(bp[t], l[t]);
         }
-        if constexpr (APART) {
-            stage(No(), Yes());
-            if (more) load_tile(kb + STEP, No(), Yes());
-            WAVE_LDS_SYNC();
-        }
         // ---- O^T += V^T P^T; keys in the order the score tiles hold them:
         // lane group lg has 4 lg + {0..3}, then 16 + 4 lg + {0..3}
 #pragma unroll
@@ -354,7 +324,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
         WAVE_LDS_SYNC();
     }
 
-    // ---- the waves' sums meet in LDS: each leaves m, l and O in its
+    // ---- the four waves' sums meet in LDS: each leaves m, l and O in its
     // own tiles
     float* mine = reinterpret_cast<float*>(kd);
 #pragma unroll
@@ -365,28 +335,28 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
             *reinterpret_cast<f32x4*>(mine + ((t * DT + d) * 64 + lane) * 4) =
                 o[d][t];
     }
-    float* ml_s = reinterpret_cast<float*>(smem + WAVES * 2 * TILE);
+    float* ml_s = reinterpret_cast<float*>(smem + ST_WAVES * 2 * TILE);
     if (lg == 0) {
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
-            ml_s[((t * 16 + li) * WAVES + wid) * 2] = m[t];
-            ml_s[((t * 16 + li) * WAVES + wid) * 2 + 1] = l[t];
+            ml_s[((t * 16 + li) * ST_WAVES + wid) * 2] = m[t];
+            ml_s[((t * 16 + li) * ST_WAVES + wid) * 2 + 1] = l[t];
         }
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         if (row0 + t * 16 + li >= live) continue;
-        float wm[WAVES], M = -1e30f, lsum = 0.f;
+        float wm[ST_WAVES], M = -1e30f, lsum = 0.f;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            wm[w] = ml_s[((t * 16 + li) * WAVES + w) * 2];
+        for (int w = 0; w < ST_WAVES; ++w) {
+            wm[w] = ml_s[((t * 16 + li) * ST_WAVES + w) * 2];
             M = fmaxf(M, wm[w]);
         }
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
+        for (int w = 0; w < ST_WAVES; ++w) {
             wm[w] = __builtin_amdgcn_exp2f(wm[w] - M);
-            lsum += wm[w] * ml_s[((t * 16 + li) * WAVES + w) * 2 + 1];
+            lsum += wm[w] * ml_s[((t * 16 + li) * ST_WAVES + w) * 2 + 1];
         }
         const long part =
             (((long)b * nkv + kvh) * Z + blockIdx.y) * max_rows + row0 +
@@ -402,10 +372,10 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void attn_stream_kernel(
         }
         // (no keys: zeros; a NaN is neither less nor greater and stays one)
         const float inv = lsum == 0.f ? 0.f : 1.f / lsum;
-        for (int d = wid; d < DT; d += WAVES) {
+        for (int d = wid; d < DT; d += ST_WAVES) {
             f32x4 a{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
+            for (int w = 0; w < ST_WAVES; ++w) {
                 const f32x4 x = *reinterpret_cast<const f32x4*>(
                     smem + w * 2 * TILE + ((t * DT + d) * 64 + lane) * 16);
 #pragma unroll
@@ -514,8 +484,8 @@ static long stream_groups(long pairs, long rows) {
 // / 101), so that verified tokens attend as decoded ones do in steps of more
 // rows than decode_stack.hip takes; to the bit only the last token of each
 // sequence, beside as many sequences in a table as wide (the splits' borders
-// follow from them), on bf16 pages (decoding rounds its queries on 8-bit ones)
-// and where decoding has four waves a context, too.
+// follow from them) and on bf16 pages (decoding rounds its queries on 8-bit
+// ones).
 extern "C" int attn_stream_takes(long pairs, long rows) {
     return rows <= 32 || stream_groups(pairs, rows) <= 448;
 }
@@ -541,7 +511,7 @@ constexpr long ST_GRID = 1536;
 extern "C" int attn_stream_splits(long pairs, long rows, long keys, int* even,
                                   int* most) {
     const long groups = pairs > 0 ? stream_groups(pairs, rows) : 1;
-    const long steps = (keys + ST_UNIT - 1) / ST_UNIT;
+    const long steps = (keys + ST_STEP - 1) / ST_STEP;
     long e = (256 + groups - 1) / groups;
     if (e > 32) e = 32;                        // the combine's lanes
     if (e > steps) e = steps;
@@ -555,7 +525,7 @@ extern "C" int attn_stream_splits(long pairs, long rows, long keys, int* even,
     }
     *even = (int)e;
     // (a split of no more than its share of `keys`: never more than z)
-    *most = z > e ? (int)((steps + z - 1) / z) * ST_UNIT : 1 << 30;
+    *most = z > e ? (int)((steps + z - 1) / z) * ST_STEP : 1 << 30;
     return (int)z;
 }
 
@@ -567,45 +537,30 @@ extern "C" int launch_attn_stream(
     const unsigned short* q, const void* k_cache, const void* v_cache,
     const int* cu, const int* block_table, const int* seq_lens,
     const int* order, unsigned short* out, float* out_ml, float* part_o,
-    float* part_ml, int nseq, int nkv, int G, int W, int bs, int hd, int Z, int even, int most,
-    int max_qlen, long s_q, float scale, int fp8, hipStream_t stream) {
+    float* part_ml, int nseq, int nkv, int G, int W, int bs, int hd, int Z,
+    int even, int most, int max_qlen, long s_q, float scale, int fp8,
+    hipStream_t stream) {
     if ((hd != 64 && hd != 128) || !(scale > 0.f)) return 1;
     if (nseq == 0 || max_qlen <= 0) return 0;
     const int max_rows = max_qlen * G;
     const int qt = max_rows <= 16 ? 1 : 2;
     const dim3 grid(nseq * nkv, Z, (max_rows + qt * 16 - 1) / (qt * 16));
     const bool whole = bs % ST_KEYS == 0;
-    // Eight waves of a context where a CU would have more than one workgroup of
-    // four, but not two: their lengths differ, and the longest then have a CU
-    // each. fp8 tiles are half the bytes, so that four waves alone draw less than a
-    // CU can. us, four / eight waves, 8 key heads of size 128 and the order
-    // of lengths: bf16 of 250 to 2000 tokens, 16 sequences 19.2 / 20.3, 24 27.4 /
-    // 25.3, 48 45.0 / 39.4, 96 74.7 / 74.0, of 500 to 4000 12 28.7 / 26.3, 40
-    // 68.6 / 68.3, 64 105.7 / 98.0; fp8 16 16.7 / 15.3, 24 18.7 / 19.3, 32 23.6 /
-    // 21.1, 12 20.8 / 18.8, 64 56.7 / 60.8. Chunks, of about one length and in no
-    // such order, stay with four (64 sequences' 2 tokens on 2000 84.0 / 85.7).
-    const long wgs = (long)grid.x * grid.z * even;
-    const bool wide =
-        whole && !cu &&
-        (fp8 ? wgs <= 320 : wgs > 256 && wgs / even <= 512);
-    const int waves = wide ? 8 : 4;
-    const int smem = waves * 2 * ST_KEYS * hd * 2 +
-                     qt * 16 * waves * 2 * (int)sizeof(float);
+    const int smem = ST_WAVES * 2 * ST_KEYS * hd * 2 +
+                     qt * 16 * ST_WAVES * 2 * (int)sizeof(float);
     const bool streamed =
         (long)nseq * nkv * W * bs * hd * (fp8 ? 2 : 4) > 6 << 20;
 #define ST_ONE(HDV, QTV, KVT)                                                 \
     do {                                                                      \
-        if (wide && streamed) ST_GO(8, HDV, QTV, KVT, true, true);      \
-        else if (wide) ST_GO(8, HDV, QTV, KVT, false, true);            \
-        else if (streamed && whole) ST_GO(4, HDV, QTV, KVT, true, true);      \
-        else if (streamed) ST_GO(4, HDV, QTV, KVT, true, false);              \
-        else if (whole) ST_GO(4, HDV, QTV, KVT, false, true);                 \
-        else ST_GO(4, HDV, QTV, KVT, false, false);                           \
+        if (streamed && whole) ST_GO(HDV, QTV, KVT, true, true);              \
+        else if (streamed) ST_GO(HDV, QTV, KVT, true, false);                 \
+        else if (whole) ST_GO(HDV, QTV, KVT, false, true);                    \
+        else ST_GO(HDV, QTV, KVT, false, false);                              \
     } while (0)
-#define ST_GO(WV, HDV, QTV, KVT, STR, WHOLE)                                  \
+#define ST_GO(HDV, QTV, KVT, STR, WHOLE)                                      \
     hipLaunchKernelGGL(                                                       \
-        (attn_stream_kernel<WV, HDV, QTV, KVT, STR, WHOLE>), grid,            \
-        dim3(WV * 64), smem, stream, q, (const KVT*)k_cache,                  \
+        (attn_stream_kernel<HDV, QTV, KVT, STR, WHOLE>), grid,                \
+        dim3(ST_WAVES * 64), smem, stream, q, (const KVT*)k_cache,            \
         (const KVT*)v_cache, cu, block_table, seq_lens, order, out, out_ml,   \
         part_o, part_ml, nkv, G, W, bs, Z, even, most, max_rows, s_q, scale)
 #define ST_COMBINE(HDV, P, I)                                                 \

@@ -392,8 +392,8 @@ __global__ void decode_slots_kernel(const int* __restrict__ table,
 
 // The same, and order: the B <= ORDER_MAX rows by their lengths, longest first (of
 // the same length: as they stand). A row's place is the number of rows before it:
-// four waves count a quarter of the others each, for 64 rows. 2 us up to 100 rows,
-// 4 at 2000.
+// four waves count a quarter of the others each, for 64 rows. 2.1 us at 24 rows, 3.0
+// at 100, 4.0 at 200, 7.3 at 512, 23 at 2048.
 constexpr int ORDER_MAX = 2048;
 __global__ __launch_bounds__(256) void decode_plan_kernel(
     const int* __restrict__ table, const int* __restrict__ pos,

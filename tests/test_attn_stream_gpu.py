@@ -123,6 +123,23 @@ def test_the_last_verified_token_gets_the_sums_of_decoding():
     assert torch.equal(rows[new - 1 :: new], last)
 
 
+# (96, 192 and 320 (sequence, key head) pairs: three splits, two, none)
+@pytest.mark.parametrize("nseq", [12, 24, 40])
+def test_last_verified_tokens_of_many_sequences(nseq):
+    """As above, whatever the number of sequences and the order in which decoding
+    reads them."""
+    total, new = [130 + 57 * i for i in range(nseq)], 4
+    kc, vc, table, lens = _pages(8, 128, 256, total, False, 3)
+    q = torch.randn(nseq * new, 32, 128, device=DEV).bfloat16()
+    cu = torch.arange(nseq + 1, dtype=torch.int32, device=DEV) * new
+    rows = ops.attn_prefill_paged(q, kc, vc, table, lens, cu, new, 0.1)
+    last = q[new - 1 :: new].contiguous()
+    _, order = ops.decode_plan(table, lens - 1, 256, lens, 8)
+    for o in (None, order):
+        got = ops.attn_decode(last, kc, vc, table, lens, 0.1, o)
+        assert torch.equal(rows[new - 1 :: new], got)
+
+
 def test_queries_at_odd_addresses_and_other_scales():
     kc, vc, table, lens = _pages(2, 64, 32, [70, 5], False, 4)
     flat = torch.randn(2 * (4 * 64 + 1) + 1, device=DEV).bfloat16()
@@ -198,7 +215,7 @@ def test_weights_add_up_to_one(nseq, hd):
         assert (got == 1).all(), (far, got.float().min().item())
 
 
-# contexts at the edges of a tile, of what eight waves take at once and of splits
+# contexts at the edges of a tile, of a workgroup's steps and of splits
 EDGES = [0, 1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 287, 288, 289, 383, 384,
          385, 511, 512, 513, 767, 768, 769, 900]
 
@@ -208,13 +225,12 @@ EDGES = [0, 1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 287, 288, 289, 383, 384
     (16, 8, 128, EDGES[:12], 256, 4),        # 288 workgroups, 3 splits
     (16, 8, 64, EDGES, 64, 0),               # 384, 2 splits
     (8, 4, 128, EDGES * 4, 128, 0),          # 384 of whole contexts
-    (8, 8, 128, EDGES[1::2] * 6, 32, 64),    # more than eight waves take; fp8 too
+    (8, 8, 128, EDGES[1::2] * 6, 32, 64),    # 384, tables wider than contexts
     (8, 8, 64, EDGES[::3] + [2500], 256, 16),
     (8, 8, 128, EDGES[:12] * 2, 24, 0),      # pages that tiles cross
 ])
 def test_decode_by_length(nq, nkv, hd, total, bs, width, fp8):
-    """Four and eight waves a context, in the order of lengths and as the rows
-    stand: the same to the bit."""
+    """In the order of lengths and as the rows stand: the same to the bit."""
     kc, vc, table, lens = _pages(nkv, hd, bs, total, fp8, 4, width)
     q = torch.randn(len(total), nq, hd, device=DEV).bfloat16()
     pos = (lens - 1).clamp(0)
@@ -252,8 +268,7 @@ def test_rows_by_length(B):
 
 @pytest.mark.parametrize("fp8", [False, True])
 def test_chunks_of_many_contexts(fp8):
-    """Two and three row tiles of a chunk, as many contexts as decoding would
-    have eight waves for."""
+    """Two and three row tiles of a chunk, in 12 and 13 contexts."""
     for new, old in ([4, 5, 1] * 4, [300, 0, 255] * 4), ([9] * 13, [600] * 13):
         total = [a + b for a, b in zip(new, old)]
         kc, vc, table, lens = _pages(8, 128, 256, total, fp8, 2)
