@@ -151,9 +151,18 @@ DEV_INLINE bool fl_block(const int* cu, const int* seq_lens, int nseq, int G,
 // What one sequence's blocks beyond whole rounds of 256 workgroups are shared by
 struct FlShare {
     int from;                  // the first of the 256 workgroups that share them
-    float *o, *ml;             // [512, 256, 128], [512, 256, 2]: a block's pieces
+    float *o, *ml;             // [pieces, 256, 128], [pieces, 256, 2]
 };
 constexpr int FL_SHARERS = 256;
+
+// Workgroup w of a key head's has tiles of its block t: from one such pair to the
+// next w + t grows, so that this many places hold the pieces of `rest` blocks
+__host__ __device__ constexpr long fl_pieces(long rest) {
+    return FL_SHARERS + rest;
+}
+DEV_INLINE long fl_piece(int w, int t, int nkv, int kvh) {
+    return (long)(w + t) * nkv + kvh;
+}
 
 // Whether `rest` blocks of a sequence of L tokens are shared: what it saves is half
 // of the chip's idle part of a last round, as long as a block of all keys; pieces
@@ -736,7 +745,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
         const int s0 = cu[0], QL = cu[1] - s0, L = seq_lens[0], hist = L - QL;
         const int rest = (blocks - share.from) / nkv;
         const int sharers = FL_SHARERS / nkv;
-        const int w = blockIdx.x - share.from, mine = w / nkv;
+        const int mine = (blockIdx.x - share.from) / nkv;
         int total = 0;
         for (int t = 0; t < rest; ++t) total += fl_tiles(t, ROWS, G, QL, hist);
         const int lo = (long)total * mine / sharers;
@@ -748,7 +757,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             before += n;
             if (a >= b) continue;
             block(0, s0, QL, L, t, a, b,
-                  a == 0 && b == n ? -1 : w * 2 + (a == 0));
+                  a == 0 && b == n ? -1 : (int)fl_piece(mine, t, nkv, kvh));
             __syncthreads();                   // the tiles are read
         }
     }
@@ -781,11 +790,10 @@ __global__ __launch_bounds__(256) void attn_flash_join_kernel(
     if ((long)total * (w + 1) / sharers >= before + n) return;   // and all others
     float M = -1e30f, sum = 0.f;
     f32x4 acc{0.f, 0.f, 0.f, 0.f};
-    for (bool first = true; (long)total * w / sharers < before + n;
-         ++w, first = false) {
+    for (; (long)total * w / sharers < before + n; ++w) {
         if ((long)total * (w + 1) / sharers == (long)total * w / sharers)
             continue;                          // (fewer tiles than sharers)
-        const long at = ((long)(w * nkv + kvh) * 2 + first) * ROWS + row;
+        const long at = fl_piece(w, tile, nkv, kvh) * ROWS + row;
         const float m = share.ml[at * 2], l = share.ml[at * 2 + 1];
         const f32x4 o = *reinterpret_cast<const f32x4*>(share.o + at * HD + c);
         const float mn = fmaxf(M, m);
@@ -911,8 +919,10 @@ extern "C" long attn_flash_pieces(long T, int nseq, int nq, int nkv, int hd,
     const bool turns = flash_turns(hd, true, bs, true);
     if (nseq != 1 || max_qlen < 1 || !turns) return 0;
     const int shape = flash_shape(hd, T, nseq, nq, nkv, max_qlen, true, turns);
-    return attn_flash_share(nseq, nq, nkv, hd, max_qlen, W, bs, fp8, shape == 0)
-               ? 512L * 256 * (128 + 2) : 0;
+    const int from =
+        attn_flash_share(nseq, nq, nkv, hd, max_qlen, W, bs, fp8, shape == 0);
+    const long blocks = ((long)max_qlen * (nq / nkv) + 255) / 256 * nkv;
+    return from ? fl_pieces(blocks - from) * 256 * (128 + 2) : 0;
 }
 
 #define FL_ONE(HDV, RWV, KSPV, PG, TU, KVT)                                   \
@@ -963,7 +973,8 @@ extern "C" int launch_attn_flash(
                             : 0;
     if (from && block_table) {
         const int blocks = (int)((rows + 255) / 256 * pairs);
-        const FlShare share{from, pieces + 512 * 256 * 2, pieces};
+        const FlShare share{from, pieces + fl_pieces(blocks - from) * 256 * 2,
+                            pieces};
         hipLaunchKernelGGL(
             (attn_flash_kernel<128, 8, 1, true, true, true, unsigned short>),
             dim3(from + FL_SHARERS), dim3(512), flash_smem(128, 8, 1, true),

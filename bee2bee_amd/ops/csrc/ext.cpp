@@ -395,10 +395,15 @@ Tensor attn_prefill_paged(const Tensor& q, const Tensor& k_cache,
                     block_table, seq_lens, nullptr, out, nullptr,
                     (int)max_qlen, scale))
         return out;
+    // (34 to 47 MB that a call can do without: blocks are not shared then)
     Tensor pieces;
     if (const long n = attn_flash_pieces(T, nseq, nq, nkv, hd, (int)max_qlen, W,
-                                         bs, fp8))
-        pieces = torch::empty({n}, q.options().dtype(torch::kFloat32));
+                                         bs, fp8)) {
+        try {
+            pieces = torch::empty({n}, q.options().dtype(torch::kFloat32));
+        } catch (const c10::OutOfMemoryError&) {
+        }
+    }
     launch_attn_prefill_paged(bf16p(q), k_cache.data_ptr(),
                               v_cache.data_ptr(), cu_q.data_ptr<int>(),
                               block_table.data_ptr<int>(),

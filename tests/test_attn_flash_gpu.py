@@ -282,3 +282,50 @@ def test_a_portion_whose_last_blocks_are_shared(nq, nkv, new, old, bs):
     want = torch.softmax(sc.masked_fill(ahead, -torch.inf), -1) @ v
     _check(got[at], want.transpose(0, 1), vc)
     assert torch.isfinite(got).all()
+
+
+def _portion(nq, nkv, new, total, bs=256):
+    """A portion of `new` tokens of a sequence of `total`, on pages in order."""
+    pages = -(-total // bs)
+    kc, vc = (torch.randn(pages, nkv, bs, 128, device=DEV).bfloat16()
+              for _ in range(2))
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+    sl = torch.tensor([total], dtype=torch.int32, device=DEV)
+    q = torch.randn(new, nq, 128, device=DEV).bfloat16()
+    cu = _cu([new])
+    return lambda: ops.attn_prefill_paged(q, kc, vc, table, sl, cu, new, 0.1), vc
+
+
+# (8 blocks that 256 workgroups share, and 92)
+@pytest.mark.parametrize("nq,nkv,new,places", [(32, 8, 2100, 264),
+                                               (28, 4, 3150, 348)])
+def test_shared_blocks_without_memory_for_their_pieces(nq, nkv, new, places):
+    """The pieces take the places that they need, and where there is no memory for
+    these, blocks are taken whole."""
+    call, v = _portion(nq, nkv, new, new + 8000)
+    want = call()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    held = torch.cuda.memory_allocated()
+    assert torch.equal(call(), want)
+    room = (torch.cuda.max_memory_allocated() - held
+            - want.numel() * want.element_size())
+    assert 0 <= room - places * 256 * 130 * 4 < 2 << 20
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    limit = torch.cuda.memory_reserved() + (want.numel() * 2) + (8 << 20)
+    whole = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.reset_peak_memory_stats()
+    held = torch.cuda.memory_allocated()
+    torch.cuda.set_per_process_memory_fraction(limit / whole)
+    try:
+        got = call()
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert (torch.cuda.max_memory_allocated() - held
+            < want.numel() * want.element_size() + (8 << 20))
+    # (each is off the exact result by up to _check's bound)
+    assert ((got.float() - want.float()).abs().max()
+            <= v.float().abs().max() * 2 ** -7)
