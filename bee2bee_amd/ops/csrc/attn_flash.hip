@@ -79,27 +79,20 @@ struct FlBlock {
     int seq, s0, QL, L, tile;
 };
 
-// The j-th block of a key head, those with many keys first, of sequences of up to
-// `most` blocks of `rows` query rows; false: there is none. The chip deals a die's
-// workgroups out to its four parts in turn, and one that finds its part full holds
-// up those behind it. If a sequence has the same turn all along, as the number of
-// sequences and key heads may make it, a long one's blocks are all on one part or
-// two. An odd number of sequences goes round by itself; of an even one the order is
-// turned from one row of tiles to the next, so that it meets other parts, and dies
-// where they share a key head (`apart`: they do not). Of two, four and six, where
-// that is not enough, and of portions, whose histories differ, each workgroup finds
-// the j-th block by the number of keys: a microsecond or two, 3 to 12% of prompts
-// of 9 to 30 that gain nothing. us, before / now, 32/8 and 28/4 heads of size 128, 32/8 of
-// 64: by keys, 2 prompts of 375 and 3000 tokens 140 / 90, 121 / 85, 86 / 67, 4 of 500 to
-// 4000 394 / 235, 242 / 201, 255 / 144, 6 of 250 to 2000 161 / 115, 108 / 99, 87 / 63, portions
-// of 300 on 500, 1000 on 4000 and 2000 on 100 163 / 140, 155 / 131; turned, 12 of 250 to
-// 2000 294 / 213 (28/4 as before); odd, 17 of 110 to 900 of 28/4 86 / 72, 9 of 210 to
-// 1700 153 / 105.
+// The order of a key head's blocks, those with many keys first (figures at
+// attn_flash_order): row of tiles by row of tiles, the sequences as they stand, or
+// turned by one from each row to the next, or by one more every `nseq` rows; or by the
+// number of keys, which each workgroup works out, of up to 64 sequences.
+enum { FL_STRAIGHT = 0, FL_TURNED = 1, FL_TURNED_MORE = 2, FL_BY_KEYS = 3 };
+
+// The j-th block in that order, of sequences of up to `most` blocks of `rows` query
+// rows; false: there is none
 DEV_INLINE bool fl_block(const int* cu, const int* seq_lens, int nseq, int G,
-                         int rows, int j, int most, bool apart, FlBlock& b) {
-    if (nseq == 1 || nseq > 8 || (!seq_lens && (nseq % 2 || nseq > 6))) {
+                         int rows, int j, int most, int order, FlBlock& b) {
+    if (order != FL_BY_KEYS) {
         const int up = j / nseq;
-        const int turn = nseq % 2 ? 0 : apart ? up + up / nseq : up;
+        const int turn = order == FL_STRAIGHT ? 0
+                         : order == FL_TURNED ? up : up + up / nseq;
         b.tile = most - 1 - up;
         b.seq = (j + turn) % nseq;
         b.s0 = cu[b.seq];
@@ -123,6 +116,17 @@ DEV_INLINE bool fl_block(const int* cu, const int* seq_lens, int nseq, int G,
         }
         return n;
     };
+    // (as many blocks behind as much history each: the search is 0.5 us more)
+    const auto first_of = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    if (!__ballot(lane < nseq &&
+                  (mine != first_of(mine) || low != first_of(low)))) {
+        b.seq = j % nseq;
+        b.s0 = __builtin_amdgcn_readlane(s0, b.seq);
+        b.QL = __builtin_amdgcn_readlane(len, b.seq);
+        b.L = __builtin_amdgcn_readlane(L, b.seq);
+        b.tile = first_of(mine) - 1 - j / nseq;
+        return b.tile >= 0;
+    }
     int span = 1, lo = 0, above = 0;
     for (int i = 0; i < nseq; ++i)
         span = max(span, __builtin_amdgcn_readlane(mine + low, i));
@@ -187,8 +191,8 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
     const unsigned short* __restrict__ q, const KVT* __restrict__ k,
     const KVT* __restrict__ v, const int* __restrict__ cu,
     const int* __restrict__ block_table, const int* __restrict__ seq_lens,
-    unsigned short* __restrict__ out, int blocks, int nq, int nkv, long s_q,
-    long s_k, long s_v, int W, int bs, int pairs, float scale_log2,
+    unsigned short* __restrict__ out, int blocks, int order, int nq, int nkv,
+    long s_q, long s_k, long s_v, int W, int bs, int pairs, float scale_log2,
     const FlShare share) {
     constexpr int NW = RW * KSP;           // waves
     constexpr int ROWS = RW * 32;          // query rows of a workgroup
@@ -731,8 +735,7 @@ __global__ __launch_bounds__(RW * KSP * 64, 2) void attn_flash_kernel(
             at.tile = blocks / nkv - 1 - blockIdx.x / nkv;
             if (at.tile * ROWS >= at.QL * G) return;
         } else if (!fl_block(cu, PAGED ? seq_lens : nullptr, pairs / nkv, G, ROWS,
-                             blockIdx.x / nkv, blocks / pairs, nkv % 8 == 0,
-                             at)) {
+                             blockIdx.x / nkv, blocks / pairs, order, at)) {
             return;
         }
         const int QL = same(at.QL), L = same(at.L), tile = same(at.tile);
@@ -899,6 +902,40 @@ extern "C" int attn_flash_form(long T, int nseq, int nq, int nkv, int hd,
     return (256 >> shape) + (shape == 0 && turns);
 }
 
+// The order of a step's blocks. The chip deals workgroups out to its eight dies in
+// turn and a die's to its four parts, and one that finds its part full holds up those
+// behind it: a long sequence's blocks should be on all parts, and a sequence's on one
+// die, whose L2 then has its keys. From one row of tiles to the next a sequence moves
+// on by nseq * nkv workgroups, turned by (nseq - 1) * nkv. Where that is an odd number
+// of times 8, its die stays and its part changes: turned; an odd number of sequences of
+// other sizes moves on by itself. Even ones are turned, where a row of tiles goes round
+// all dies (nkv a multiple of 8) by one more each time round; of twelve and more, which
+// share parts by threes, only in large steps.
+// By keys, each workgroup looks at all sequences, 0.3 to 1 us of its time: two, four and
+// six prompts of different lengths, for which turning is not enough, and portions, whose
+// histories the host does not know, of up to eight sequences; not small steps, nor
+// prompts of about one length.
+// us, straight / turned (by one more) / by keys, an eighth of the longest up to it: 2
+// prompts of up to 2500 tokens of 32/8 heads 94.9 / 67.7 / 67.4, 4 175 / 106 / 99, 6 157 / 149
+// / 144, 8 of up to 1000 60.0 / 46.6 / 48.3, 12 80.6 / 67.9 / 71.5; 28/4, 9 of up to 1600 93 /
+// 137 / 96, 7 of up to 700 27.3 / 25.2 / 26.0; 12/12 of 64, 7 of up to 2500 71.6 / 59.1 / 57.6,
+// 5 56.1 / 62.5 / 53.1; small and level ones of 32/8, 4 of up to 64 6.1 / 6.2 / 6.6, 2 of 200
+// 8.5 / 8.4 / 8.7; portions of 32/8, 1000 tokens on 0 to 4000, 3 168 / - / 135, 4 218 / 211 / 161, 4
+// on 4000 269 / 269 / 271, 8 of 64 on 100 9.1 / 9.1 / 9.9.
+extern "C" int attn_flash_order(long T, int nseq, int nq, int nkv, int max_qlen,
+                                bool pages) {
+    const long full = T * nq / 256;
+    const bool level = 4 * T >= 3L * nseq * max_qlen;
+    if (nseq == 1) return FL_STRAIGHT;
+    if (pages ? nseq <= 8 && full >= 80
+              : nseq % 2 == 0 && nseq <= 6 && !level && full >= 40)
+        return FL_BY_KEYS;
+    if (nkv % 8 == 0)
+        return nseq % 2 || full < (nseq >= 12 ? 600 : pages ? 80 : 0)
+                   ? FL_STRAIGHT : FL_TURNED_MORE;
+    return nseq % 2 == 0 || (nseq - 1) * nkv % 16 == 8 ? FL_TURNED : FL_STRAIGHT;
+}
+
 // Workgroups of a step that take whole blocks where 256 more share the rest, 0:
 // all take whole ones. One portion, of bf16 pages: its blocks are about as long as
 // each other, and what is left over whole rounds of 256 takes as long as a round.
@@ -932,8 +969,8 @@ extern "C" long attn_flash_pieces(long T, int nseq, int nq, int nkv, int hd,
             (attn_flash_kernel<HDV, RWV, KSPV, PG, TU, false, KVT>),          \
             dim3((unsigned)blocks), dim3(RWV * KSPV * 64),                    \
             flash_smem(HDV, RWV, KSPV, TU), stream, q, (const KVT*)k,         \
-            (const KVT*)v, cu, block_table, seq_lens, out, blocks, nq, nkv,   \
-            s_q, s_k, s_v, W, bs, pairs, scale * LOG2E, FlShare{});           \
+            (const KVT*)v, cu, block_table, seq_lens, out, blocks, order, nq, \
+            nkv, s_q, s_k, s_v, W, bs, pairs, scale * LOG2E, FlShare{});      \
     } while (0)
 #define FL_HD(HDV, PG, KVT)                                                   \
     do {                                                                      \
@@ -979,13 +1016,15 @@ extern "C" int launch_attn_flash(
             (attn_flash_kernel<128, 8, 1, true, true, true, unsigned short>),
             dim3(from + FL_SHARERS), dim3(512), flash_smem(128, 8, 1, true),
             stream, q, (const unsigned short*)k, (const unsigned short*)v, cu,
-            block_table, seq_lens, out, blocks, nq, nkv, s_q, s_k, s_v, W, bs,
-            pairs, scale * LOG2E, share);
+            block_table, seq_lens, out, blocks, FL_STRAIGHT, nq, nkv, s_q, s_k,
+            s_v, W, bs, pairs, scale * LOG2E, share);
         hipLaunchKernelGGL(attn_flash_join_kernel, dim3((blocks - from) * 32),
                            dim3(256), 0, stream, share, cu, seq_lens, out, nq,
                            nkv, blocks);
         return 0;
     }
+    const int order =
+        attn_flash_order(T, nseq, nq, nkv, max_qlen, block_table != nullptr);
     if (!block_table) {
         if (hd == 128) FL_HD(128, false, unsigned short);
         else FL_HD(64, false, unsigned short);

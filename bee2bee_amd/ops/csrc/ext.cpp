@@ -41,6 +41,7 @@ void launch_attn_decode(const unsigned short*, const void*, const void*,
                         float*, unsigned short*, float*, int, int, int, int,
                         int, int, int, long, float, int, hipStream_t);
 int attn_flash_form(long, int, int, int, int, int, int);
+int attn_flash_order(long, int, int, int, int, bool);
 int attn_stream_takes(long, long);
 int attn_stream_splits(long, long, long, int*, int*);
 int launch_attn_stream(const unsigned short*, const void*, const void*,
@@ -525,6 +526,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "chunked prefill vs paged history");
     m.def("attn_flash_form", &attn_flash_form,
           "rows of prompt attention's workgroups, + 1 where waves take turns");
+    m.def("attn_flash_order", &attn_flash_order,
+          "order of a step's blocks (attn_flash.hip)");
     m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA layout probe");
     m.def("mfma_probe_fp8", &mfma_probe_fp8,
           "16x16x32 fp8 MFMA layout probe");

@@ -51,3 +51,29 @@ def test_shapes_follow_what_was_measured(n, longest, nq, nkv, rows256, rows128):
 def test_prompts_of_one_length(n, each, nq, nkv, rows256, rows128):
     want = 257 if rows256 < rows128 else 128
     assert _form([each] * n, nq, nkv, 128) == want
+
+
+# us, row of tiles by row of tiles as the sequences stand / turned / by the number of
+# keys; of prompts of an eighth of the longest up to it
+@pytest.mark.parametrize("n,longest,nq,nkv,straight,turned,keys", [
+    (2, 2500, 32, 8, 94.9, 67.7, 67.4), (4, 2500, 32, 8, 175, 106, 99),
+    (6, 2500, 32, 8, 157, 149, 144), (8, 1000, 32, 8, 60.0, 46.6, 48.3),
+    (12, 1600, 32, 8, 164, 140, 143), (9, 1600, 28, 4, 93, 137, 96),
+    (7, 700, 28, 4, 27.3, 25.2, 26.0), (7, 2500, 12, 12, 71.6, 59.1, 57.6),
+    (4, 64, 32, 8, 6.1, 6.2, 6.6), (2, 64, 12, 12, 4.5, 4.5, 4.8)])
+def test_orders_follow_what_was_measured(n, longest, nq, nkv, straight, turned,
+                                         keys):
+    """The fastest, or within 4% of it."""
+    order = ops.require_hip().attn_flash_order(
+        sum(_spread(n, longest)), n, nq, nkv, longest, False)
+    took = (straight, turned, turned, keys)[order]
+    assert took <= 1.04 * min(straight, turned, keys)
+
+
+def test_only_few_large_and_uneven_steps_search():
+    """A workgroup's search costs 0.3 to 1 us."""
+    order = ops.require_hip().attn_flash_order
+    for n, each, pages in ((1, 4000, False), (2, 2000, False), (4, 1000, False),
+                           (3, 20, True), (8, 64, True), (9, 1000, True)):
+        assert order(n * each, n, 32, 8, each, pages) != 3
+    assert order(4 * 1000, 4, 32, 8, 1000, True) == 3    # (histories may differ)

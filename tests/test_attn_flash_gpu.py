@@ -221,7 +221,10 @@ def test_weights_add_up_to_one(hd, T):
 @pytest.mark.parametrize("lens", [
     [700, 90], [33, 0, 650, 1], [1, 600, 40, 300, 64, 65], [500, 20] * 4,
     [257, 1, 900], [150, 31, 400, 90, 7], [260, 30, 129] * 3 + [500],
-    [90, 40, 128, 20, 300] * 4])
+    [90, 40, 128, 20, 300] * 4,
+    # as many blocks of each, of one length and not; rows of tiles turned by their
+    # dies; twelve sequences whose parts even out
+    [300, 290, 310], [257] * 4, [200, 150, 40] * 2 + [700], [60, 200, 130] * 4])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_blocks_of_every_sequence(hd, lens, nkv):
     """Every row of tiles of every sequence is taken, however many of them there
@@ -251,6 +254,41 @@ def test_blocks_of_every_sequence(hd, lens, nkv):
         q.float(), kc.float(), vc.float(), table, sl,
         torch.tensor(lens, dtype=torch.int32), scale)
     _check(got, want, vc)
+
+
+def _check_portions(lens, old, nq, nkv, hd, bs=64):
+    total = [a + b for a, b in zip(old, lens)]
+    counts = [-(-n // bs) for n in total]
+    table = torch.zeros(len(lens), max(counts), dtype=torch.int32, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(sum(total))
+    pages = torch.randperm(sum(counts), generator=g, device=DEV).int()
+    at = 0
+    for i, c in enumerate(counts):
+        table[i, :c] = pages[at : at + c]
+        at += c
+    kc, vc = (torch.randn(sum(counts), nkv, bs, hd, generator=g,
+                          device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(sum(lens), nq, hd, generator=g, device=DEV).bfloat16()
+    sl = torch.tensor(total, dtype=torch.int32, device=DEV)
+    scale = hd ** -0.5
+    got = ops.attn_prefill_paged(q, kc, vc, table, sl, _cu(lens), max(lens),
+                                 scale)
+    want = reference.attn_decode_with_history(
+        q.float(), kc.float(), vc.float(), table, sl,
+        torch.tensor(lens, dtype=torch.int32), scale)
+    _check(got, want, vc)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("lens,old", [
+    ([300, 290, 310], [70, 100, 64]), ([520] * 2, [600] * 2),
+    ([200, 193, 256, 250, 210, 256, 255, 199], [0] * 8)])
+def test_portions_of_as_many_blocks(hd, lens, old):
+    """Sequences whose blocks and histories count the same, their lengths do not."""
+    order = ops.require_hip().attn_flash_order(sum(lens), len(lens), 32, 8,
+                                               max(lens), True)
+    assert order == 3
+    _check_portions(lens, old, 32, 8, hd)
 
 
 @pytest.mark.parametrize("nq,nkv,new,old,bs", [
