@@ -291,6 +291,35 @@ def test_portions_of_as_many_blocks(hd, lens, old):
     _check_portions(lens, old, 32, 8, hd)
 
 
+# (the last: rows of tiles of the longest, its history's among them)
+@pytest.mark.parametrize("nq,nkv,hd,form,lens,old,levels", [
+    (32, 8, 64, 64, [1024, 30], None, 64), (32, 8, 64, 64, [1025, 30], None, 65),
+    (28, 4, 128, 257, [2341, 40], None, 65), (28, 4, 128, 257, [4681, 900], None,
+                                              128),
+    (28, 4, 128, 257, [4682, 30], None, 129),
+    (32, 8, 64, 128, [2100, 20, 700, 1], None, 66),
+    (32, 8, 64, 128, [2050, 0, 90, 800, 33, 64], None, 65),
+    (28, 4, 128, 64, [64, 700], [5800, 0], 641),
+    (32, 8, 128, 64, [300, 65, 300], [0, 4800, 1900], 305),
+])
+def test_blocks_found_in_two_passes(nq, nkv, hd, form, lens, old, levels):
+    """The search by keys looks at 64 levels (rows of tiles) at a time."""
+    hip = ops.require_hip()
+    T, n, most = sum(lens), len(lens), max(lens)
+    bs, G, rows = 64 if old else 0, nq // nkv, form & ~1
+    assert max(-(-a * G // rows) + b * G // rows
+               for a, b in zip(lens, old or [0] * n)) == levels
+    assert hip.attn_flash_form(T, n, nq, nkv, hd, most, bs) == form
+    assert hip.attn_flash_order(T, n, nq, nkv, most, bool(old)) == 3
+    if old:
+        return _check_portions(lens, old, nq, nkv, hd, bs)
+    q, k, v = _qkv(T, nq, nkv, hd, n)
+    got = ops.attn_prefill(q, k, v, _cu(lens), most, hd ** -0.5)
+    want = reference.attn_prefill(q.float(), k.float(), v.float(), _cu(lens),
+                                  most, hd ** -0.5)
+    _check(got, want, v)
+
+
 @pytest.mark.parametrize("nq,nkv,new,old,bs", [
     (32, 8, 2100, 4200, 256),       # 33 rows of blocks of 8 heads: 8 are shared
     (32, 8, 2049, 3991, 64), (28, 4, 2900, 6000, 256),
