@@ -379,7 +379,10 @@ def mid_gated(rows: int, width: int, depth: int) -> bool:
     256; 2x18944x3584 45.3 (56.8), 57.7 (71.6), 61 (75.5) at 160, 107 (83) at
     200; 2x8192x2048 14.1 (20.8), 21.7 (23.9), 25 (30.6) at 192, 29 (33) at 256;
     2x5504x2048 13.0 (18.8), 18.5 (21.6), 23.5 (28.6) at 192, 27.9 (30.7) at 256;
-    2x2048x768 6.9 (9.4), 9.7 (10.4), 11.9 (10.3). More than 12 tiles of 8 columns a CU go
+    2x2048x768 6.9 (9.4), 9.7 (10.4), 11.9 (10.3). Beside wide_linear at 160 / 192 /
+    224 rows: 2x5504x2048 20.4 (27.4) / 22.9 (28.9) / 25.5 (30.2), 2x9216x1408 22.1
+    (26.8) / 23.9 (22.6) / 25.8 (23.7), 2x12288x1024 19.0 (20.4) / 21.1 (18.3) / 23.2
+    (18.9), 2x16384x768 18.4 (17.6) / 20.5 (17.3) / 22.6 (17.6). More than 12 tiles of 8 columns a CU go
     in rounds, each with a start of its own: 2x27648x5120 96 (100), 107 (105) at
     48, 134 (123) at 128, but 2x28672x8192 141 (181), 153 (186), 194 (211)."""
     tiles = -(-width // 2048)           # of 8 columns, a CU
@@ -391,7 +394,11 @@ def mid_gated(rows: int, width: int, depth: int) -> bool:
         return True
     if tiles > 8:
         return rows <= 160
-    return width * depth >= 11_000_000 and rows <= (256 if tiles <= 4 else 224)
+    if width * depth < 11_000_000:
+        return False
+    if tiles > 4 and width * depth < 16_000_000:
+        return rows <= 160 and depth >= 1024
+    return rows <= (256 if tiles <= 4 else 224)
 
 
 def mid_gelu(rows: int, width: int, depth: int) -> bool:
@@ -405,13 +412,20 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     """Logits that mid_rows_linear takes. Groups of 8 tiles of 16 columns, a
     CU's one after the other: where the last round leaves more than a twentieth
     of the chip idle (152064 columns) the library is ahead above 64 rows, and of
-    the largest heads wide_linear from 129 rows on. Beside the library's product,
+    the largest heads wide_linear from 129 rows on; above 160 rows it is also where
+    rounds are short (few steps of K) or have fewer than 8 tiles for the waves that
+    take two each. Beside the library's product,
     and wide_linear's where there is one (us): 128256x4096 159 (193) at 24 rows,
     188 (218) at 80, 214 (239, 210) at 128, 224 (251, 216) at 160; 32000x4096 41
     (63), 45 (66), 52 (68), 57 (69), 65 (78) at 200, 73 (79) at 256; 128256x2048
     82 (121), 102 (129), 120 (134), 129 (141, 137), 143 (178, 144); 152064x3584
     176 (242), 220 (213), 249 (245, 241); of rows of 768 17.0 (18.6), 22.6
-    (20.8). Few rows (one launch of rows_linear in brackets; a norm takes 2.5
+    (20.8). At 160 / 192 / 224 / 256 rows: 65536x8192 190 (211, 204) / 209 (212, 205);
+    64000x4096 110 (136, 131) at 161, 112 (138, 133); 28672x4096 53 (56) / 56 (60) / 60
+    (64) / 67 (67); 32000x2048 33 (39) / 34 (39) / 37 (40) / 42 (40); 32000x1024 22 (21)
+    / 22 (22) / 25 (23) / 27 (24); 65536x2048 67 (77) at 161, 67 (77) / 73 (78) / 80 (78);
+    57344x2048 59 (59) / 64 (59) / 68 (62) / 73 (60), 49152x2048 57 (56) at 161, 60 (55)
+    / 65 (57) / 75 (56); 65536x1536 54 (54) / 55 (48) / 59 (50) / 65 (52). Few rows (one launch of rows_linear in brackets; a norm takes 2.5
     us): 1 / 16 rows 128256x4096 155 (178) / 157 (188), 152064x3584 163 (182) /
     167 (204), 128256x2048 78 (93) / 80 (101); of rows of 8192 1 / 8 / 12 rows
     128256 370 (363) / 371 (359) / 370 (376), 152064 454 (427) / 458 (438) / 454
@@ -425,9 +439,16 @@ def mid_head(rows: int, width: int, depth: int) -> bool:
     full = 256 * rounds * -(-tiles // (256 * rounds))
     if width % 4 or rows > DEEP_MAX or (depth < 1024 and rows > 48):
         return False
-    if rows > MID_MAX and width * depth > (
-            280_000_000 if rows <= 192 else 150_000_000):
+    if rows > MID_MAX and depth < 8192 and width * depth > 280_000_000:
         return False
+    if rows > 160:
+        each = full // (256 * rounds)
+        if width * depth > (280_000_000 if rows <= 192 else 150_000_000):
+            return False
+        if rounds > 1 and not (rows <= 192 and each == 8 and depth >= 2048):
+            return False
+        if depth < 1536 or (rows > 224 and (depth < 4096 or each < 7)):
+            return False
     return rows <= 64 or tiles * 20 >= full * 19
 
 

@@ -249,3 +249,33 @@ def test_small_products_of_129_to_256_rows(rows, width, depth, own):
     (8, 128256, 4096, 174, 187), (1, 32000, 4096, 48, 50)])
 def test_output_heads_of_few_rows(rows, width, depth, rings, alone):
     assert ops.mid_head(rows, width, depth) == (rings < alone)
+
+
+# us as measured: the rings, the fastest of the library and linear_wide.hip
+@pytest.mark.parametrize("rows,width,depth,rings,other", [
+    (128, 128256, 4096, 214, 239), (129, 131072, 4096, 217, 202),
+    (160, 131072, 4096, 225, 205), (129, 65536, 8192, 191, 207),
+    (160, 65536, 8192, 190, 204), (160, 128256, 8192, 412, 424),
+    (161, 64000, 4096, 110, 131), (192, 64000, 4096, 112, 133),
+    (192, 65536, 2048, 67, 77), (193, 64000, 2048, 69, 67),
+    (161, 49152, 2048, 57.4, 56.1), (192, 49152, 2048, 60, 55),
+    (256, 49152, 2048, 75, 56), (192, 57344, 2048, 64, 59),
+    (192, 65536, 1536, 55, 48), (161, 32000, 1024, 21.5, 21.1),
+    (256, 32000, 1024, 27, 24), (224, 32000, 2048, 37, 40),
+    (256, 32000, 2048, 41.9, 40.3), (224, 32000, 3072, 51, 53),
+    (225, 32000, 3072, 59, 54), (256, 32000, 4096, 71, 72),
+    (224, 24576, 4096, 58, 60), (225, 24576, 4096, 64, 60)])
+def test_output_heads_of_129_to_256_rows(rows, width, depth, rings, other):
+    assert ops.mid_head(rows, width, depth) == (rings < other)
+
+
+# us as measured: the rings, linear_wide.hip
+@pytest.mark.parametrize("rows,width,depth,rings,wide", [
+    (160, 5504, 2048, 20.4, 27.4), (256, 5504, 2048, 27.8, 31.1),
+    (256, 8192, 1536, 25, 27), (256, 4096, 3072, 37, 47),
+    (160, 9216, 1408, 22.1, 26.8), (161, 9216, 1408, 23.2, 21.7),
+    (224, 9216, 1408, 25.8, 23.7), (160, 12288, 1024, 19.0, 20.4),
+    (161, 12288, 1024, 20.5, 17.7), (224, 14336, 1024, 24.3, 19.8),
+    (160, 16384, 768, 18.4, 17.6), (224, 16384, 768, 22.6, 17.6)])
+def test_gated_projections_of_129_to_256_rows(rows, width, depth, rings, wide):
+    assert ops.mid_gated(rows, width, depth) == (rings < wide)
