@@ -757,7 +757,12 @@ class Runner:
                 self.rope_cos if s.pos_type == "rope" else None, self.rope_sin,
                 slot_mapping, block_table, seq_lens,
                 status=self.step_status)
-        if slot_mapping is None:
+        if slot_mapping is None and (self.decode_attn_fn is not None
+                                     or self.spec.head_dim not in (64, 128)):
+            # (attention that does not take an order)
+            slot_mapping = ops.decode_slots(block_table, positions,
+                                            self.kv.block_size)
+        elif slot_mapping is None:
             slot_mapping, order = ops.decode_plan(
                 block_table, positions, self.kv.block_size, seq_lens,
                 self.spec.n_kv_heads)

@@ -279,3 +279,32 @@ def test_output_heads_of_129_to_256_rows(rows, width, depth, rings, other):
     (160, 16384, 768, 18.4, 17.6), (224, 16384, 768, 22.6, 17.6)])
 def test_gated_projections_of_129_to_256_rows(rows, width, depth, rings, wide):
     assert ops.mid_gated(rows, width, depth) == (rings < wide)
+
+
+@pytest.mark.parametrize("head_dim,own,ordered", [
+    (64, False, True), (64, True, False), (32, False, False)])
+@torch.no_grad()
+def test_rows_are_ordered_for_attention_that_takes_it(head_dim, own, ordered,
+                                                      monkeypatch):
+    """Steps that are not told their slots: an attention of the caller's, and
+    head sizes that attn_stream.hip does not have, get no order of the rows."""
+    spec = dataclasses.replace(PRESETS["tiny"], head_dim=head_dim)
+    kv = PagedKV(spec, CPU, torch.float32, n_blocks=16, block_size=16)
+    r = Runner(spec, _weights(spec), kv, CPU, torch.float32)
+    if own:
+        r.decode_attn_fn = ops.attn_decode
+    kv.new_seq(0)
+    kv.extend_seq(0, 3)
+    taken, op = [], ops.decode_plan
+    monkeypatch.setattr(ops, "decode_plan", lambda *a: (
+        taken.append(1), op(*a))[1])
+    table, pos = kv.block_table([0]), torch.tensor([2], dtype=torch.int32)
+    ids = torch.tensor([7])
+    kv_before = [t.clone() for t in [*kv.k_cache, *kv.v_cache]]
+    got = r.forward_decode(ids, pos, None, table, pos + 1)
+    assert bool(taken) == ordered
+    for t, old in zip([*kv.k_cache, *kv.v_cache], kv_before):
+        t.copy_(old)
+    want = r.forward_decode(ids, pos, decode_slot_mapping(table, pos, 16), table,
+                            pos + 1)
+    assert torch.equal(got, want)
