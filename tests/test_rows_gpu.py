@@ -252,7 +252,8 @@ def test_parts_over_k(M, N, K):
 @pytest.mark.parametrize("N,K,act", [
     (8, 64, "swiglu"), (2056, 1088, "swiglu"), (9000, 192, "swiglu"),
     (17000, 704, "swiglu"), (25000, 128, "swiglu"), (4, 64, None),
-    (3072, 768, "gelu"), (8204, 320, "gelu"), (33004, 576, None)])
+    (3072, 768, "gelu"), (8204, 320, "gelu"), (33004, 576, None),
+    (32004, 320, None)])     # (eight tiles each, the last workgroup one)
 def test_activated_rows(M, N, K, act):
     """Products are exact in fp32, their sums off by K roundings at most; an
     activation's slope is below 1.13, and the result is rounded to bf16."""
@@ -277,9 +278,11 @@ def test_activated_rows(M, N, K, act):
             + 1e-6).all()
 
 
-# (five tiles a workgroup, the last one of 12 columns, fewer steps of K than the
-# rings have slots; eight tiles and a second group, more steps)
-@pytest.mark.parametrize("N,K", [(20492, 128), (40004, 960)])
+# (tiles a workgroup: six, the last of 12 columns, fewer steps of K than the rings
+# have slots; five and a second group, more steps; eight, and in the last workgroup
+# one; eight and a second group)
+@pytest.mark.parametrize("N,K", [(20492, 128), (40004, 960), (32004, 320),
+                                 (65524, 192)])
 def test_logits_of_few_rows(N, K):
     """As above without an activation; a row's logits are the same to the bit
     whatever rows are beside it."""
