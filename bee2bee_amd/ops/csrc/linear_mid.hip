@@ -9,40 +9,41 @@
 //          feed-forward of the GPT-2 family).
 //
 // Bound by reading the weights once, up to about 128 rows; beyond, by the steps of
-// the four waves that load the input: at 200 rows 2200 clocks, of which products
-// 900; their seven loads wait up to 1000 for the memory pipe, and the other four
-// waves at the barrier for them. So a step finds out as little as it can: the two
-// kinds of waves have loops of their own, in which the number of loads under way
-// is known (us, with both in one loop / as now: 2x14336x4096 68.6 / 63.4 at 200
-// rows, 81.8 / 72.5 at 256, 51.2 / 50.3 at 128; 4096x14336 38.9 / 36.4 at 200;
-// 2x18944x3584 122 / 107; fewer rows within 2%). Loads spread between the products
-// changed nothing, nor did halves that read and multiply in turn, weights in
-// registers and the input in all of LDS, or tiles of 128 rows of w in turns with
-// three buffers of both. A workgroup a CU, 160 KB of LDS as two rings: 64 of K by the
-// workgroup's rows of w, and by all input rows. Four waves fill the one, four
-// the other, straight from memory (global_load_lds: no registers), and all eight
-// multiply: the fragments of the
-// next half step are read while this one's products run. The weights carry the
-// streaming hint, so that they do not push the input out of L2 (2x14336x4096 at
-// 24 rows 40.8 us without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128
-// bytes in LDS are xor-ed by half their number: no two of a read's 16 rows meet
-// in a bank. Workgroups start at different places of K: in step they would all
-// ask for the same few channels (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 ->
-// 44.5 at 80). Those of output heads, which go round by round, are 5 steps apart
-// and not one: 128256x4096 167 -> 159 us at 24 rows, 193 -> 188 at 80 (gated 2 to
-// 4% slower so, others the same). The rings hold what covers the memory's latency
-// and no more: 32 KB of weights of narrow products, 64
-// of others. With all of LDS for weights every CU asks for 100 KB at once, and the
-// input that the first step waits for queues behind it (us, rings of 96 to 112 KB /
-// as now: 2048x8192 9.6 / 8.5 at 24 rows, 11.1 / 9.5 at 57; 4096x4096 11.6 / 10.4
-// at 80; 2x8192x2048 16.0 / 14.7 at 57; 2x14336x4096 45.0 / 43.2 at 80; with 48 and
-// 24 KB a third to half more time). The input needs four slots, better six (with
-// two 44 -> 61 us at 80 rows); its rows apart by an odd number of lines change
-// nothing. A CU takes in 57 GB/s from memory, 50 to 60 of weights and input
-// together, so what a slot has past the rows and tiles that there are is not loaded
-// (loaded / not: 2x18944x3584 47.5 / 46.4 at 24 rows, 54.8 / 52.4 at 80, 103 / 96 at
-// 200, 123 / 109 at 256; 2x14336x4096 40.2 / 39.2 at 57, 43.8 / 42.4 at 80, 63.0 / 62.2
-// at 200; 6144x4096 14.4 / 13.9 at 80; others within 1%).
+// the four waves that load the input: at 200 rows 2200 clocks, of which products 900;
+// their seven loads wait up to 1000 for the memory pipe, and the other four waves at
+// the barrier for them. So a step finds out as little as it can: the two kinds of
+// waves have loops of their own, in which the number of loads under way is known (us,
+// with both in one loop / as now: 2x14336x4096 68.6 / 63.4 at 200 rows, 81.8 / 72.5
+// at 256, 51.2 / 50.3 at 128; 4096x14336 38.9 / 36.4 at 200; 2x18944x3584 122 / 107;
+// fewer rows within 2%). Loads spread between the products changed nothing, nor did
+// halves that read and multiply in turn, weights in registers and the input in all of
+// LDS, or tiles of 128 rows of w in turns with three buffers of both. A workgroup a
+// CU, with two rings in LDS: 64 of K by the workgroup's rows of w, and by all input
+// rows. Four waves fill the one, four the other, straight from memory
+// (global_load_lds: no registers), and all eight multiply: the fragments of the next
+// half step are read while this one's products run. The weights carry the streaming
+// hint, so that they do not push the input out of L2 (2x14336x4096 at 24 rows 40.8 us
+// without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128 bytes in LDS are xor-ed by
+// half their number: no two of a read's 16 rows meet in a bank. Workgroups start at
+// different places of K: in step they would all ask for the same few channels
+// (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 -> 44.5 at 80). Those of output heads,
+// which go round by round, are 5 steps apart and not one: 128256x4096 167 -> 159 us
+// at 24 rows, 193 -> 188 at 80 (gated 2 to 4% slower so, others the same). The rings
+// of up to 8 tiles hold what covers the memory's latency and no more: four slots of
+// weights, 32 KB up to 4 tiles and 64 above. With all of LDS for weights every CU
+// asks for 100 KB at once, and the input that the first step waits for queues behind
+// it (us, rings of 96 to 112 KB / as now: 2048x8192 9.6 / 8.5 at 24 rows, 11.1 / 9.5
+// at 57; 4096x4096 11.6 / 10.4 at 80; 2x8192x2048 16.0 / 14.7 at 57; 2x14336x4096
+// 45.0 / 43.2 at 80; with 48 and 24 KB a third to half more time). The input has six
+// slots there, fewer from 129 rows on, down to the three that LDS has room for above
+// 192 (with two 44 -> 61 us at 80 rows). Gated products of 9 to 12 tiles and those of
+// scaled rows (LM_SCALED) still have the long rings, 96 to 144 KB of weights; shorter
+// ones were not measured there. Input rows apart by an odd number of lines change
+// nothing. A CU takes in 57 GB/s from memory, 50 to 60 of weights and input together,
+// so what a slot has past the rows and tiles that there are is not loaded (loaded /
+// not: 2x18944x3584 47.5 / 46.4 at 24 rows, 54.8 / 52.4 at 80, 103 / 96 at 200, 123 /
+// 109 at 256; 2x14336x4096 40.2 / 39.2 at 57, 43.8 / 42.4 at 80, 63.0 / 62.2 at 200;
+// 6144x4096 14.4 / 13.9 at 80; others within 1%).
 //
 // Measured (us, launch after launch with weights that no cache holds, 24 / 80 / 128
 // / 200 / 256 rows; in brackets with one loop and the long rings):
@@ -451,10 +452,10 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     } while (0)
 #define LM_4(F)                                                               \
     do {                                                                      \
-        if (M <= 32) LM_GO(1, 2, 4, 1, 2, 4, 6, F);                          \
-        if (M <= 64) LM_GO(1, 4, 4, 1, 2, 4, 6, F);                          \
-        if (M <= 96) LM_GO(2, 3, 2, 2, 2, 4, 6, F);                          \
-        if (M <= 128) LM_GO(2, 4, 2, 2, 2, 4, 6, F);                         \
+        if (M <= 32) LM_GO(1, 2, 4, 1, 2, 4, 6, F);                           \
+        if (M <= 64) LM_GO(1, 4, 4, 1, 2, 4, 6, F);                           \
+        if (M <= 96) LM_GO(2, 3, 2, 2, 2, 4, 6, F);                           \
+        if (M <= 128) LM_GO(2, 4, 2, 2, 2, 4, 6, F);                          \
         if (M <= 160) LM_GO(2, 5, 2, 2, 2, 4, 6, F);                          \
         if (M <= 192) LM_GO(2, 6, 2, 2, 2, 4, 5, F);                          \
         if (M <= 224) LM_GO(2, 7, 2, 2, 2, 4, 4, F);                          \
