@@ -98,9 +98,10 @@ DEV_INLINE void lm_wait(int left) {
 // Waves: WN groups of TW tiles of 16 rows of w, by WM groups of MW tiles of 16
 // input rows, by WK halves of a step. DW, DX: slots of the rings. `tiles` of
 // the TW * WN are used. WK 1: a workgroup takes every gridDim.x-th group of
-// tiles, loading the next one's first steps under this one's last.
+// tiles, loading the next one's first steps under this one's last. APART: the two
+// halves of K's steps have sums of their own, as with WK 2.
 template <int TW, int MW, int WN, int WM, int WK, int DW, int DX, int OUT,
-          bool SCALED = false>
+          bool SCALED = false, bool APART = false>
 __global__ __launch_bounds__(512) void linear_mid_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias, void* __restrict__ out, int M,
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     const float* __restrict__ squares, float eps) {
     constexpr int T = TW * WN, MT = MW * WM;
     static_assert(WN * WM * WK == 8 && DW >= 2 && DX >= 2, "");
+    static_assert(WK == 1 || !APART, "");
     constexpr int NLW = T / 2, NLX = (MT + 1) / 2;  // loads of a wave a step
     constexpr int WB = NLW * 4096, XB = NLX * 4096; // bytes of a slot
     const int tid = threadIdx.x, lane = tid & 63;
@@ -214,12 +216,15 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     }
 
     // ---- products
-    f32x4 acc[TW][MW];
+    f32x4 acc[TW][MW], other[APART ? TW : 1][APART ? MW : 1];
     auto clear = [&]() {
 #pragma unroll
         for (int t = 0; t < TW; ++t)
 #pragma unroll
-            for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MW; ++m) {
+                acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if constexpr (APART) other[t][m] = acc[t][m];
+            }
     };
     clear();
     bf16x8 fw[2][TW], fx[2][MW];
@@ -241,9 +246,12 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
 #pragma unroll
         for (int m = 0; m < MW; ++m)
 #pragma unroll
-            for (int t = 0; t < TW; ++t)
-                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    fw[set][t], fx[set][m], acc[t][m], 0, 0, 0);
+            for (int t = 0; t < TW; ++t) {
+                f32x4& to = APART && set ? other[APART ? t : 0][APART ? m : 0]
+                                         : acc[t][m];
+                to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    fw[set][t], fx[set][m], to, 0, 0, 0);
+            }
     };
     // (the builtin: the compiler has to know that nothing is under way, or it
     // waits for what was only just asked for)
@@ -350,6 +358,14 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
         for (int s = 0; s < total; s += n) {
             if (of_w) steps(Yes(), s, s + n);
             else steps(No(), s, s + n);
+            if constexpr (APART)
+#pragma unroll
+                for (int t = 0; t < TW; ++t)
+#pragma unroll
+                    for (int m = 0; m < MW; ++m)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            acc[t][m][r] += other[t][m][r];
             finish(g);
             g += gridDim.x;
             clear();
@@ -438,13 +454,15 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     const int NG = (NT + tiles - 1) / tiles;
     const bool once = NG * S <= 256;           // no second group of tiles
 #define LM_GO(TW, MW, WN, WM, WK, DW, DX, F)                                  \
+    LM_SUMS(TW, MW, WN, WM, WK, DW, DX, F, false)
+#define LM_SUMS(TW, MW, WN, WM, WK, DW, DX, F, APART)                         \
     do {                                                                      \
         constexpr int lds =                                                   \
             DW * (TW * WN / 2) * 4096 + DX * ((MW * WM + 1) / 2) * 4096;      \
         static_assert(lds <= 163840, "LDS of a CU");                          \
         static_assert(WK == 1 || TW * MW * 1024 * 4 <= lds, "halves");        \
         hipLaunchKernelGGL(                                                   \
-            (linear_mid_kernel<TW, MW, WN, WM, WK, DW, DX, F>),               \
+            (linear_mid_kernel<TW, MW, WN, WM, WK, DW, DX, F, false, APART>), \
             dim3(WK == 1 && !once ? 256 / S : NG, S), dim3(512),              \
             lds, stream, x, w, bias, out, M, N, K, S, tiles, gelu, nullptr,   \
             0.f);                                                             \
@@ -473,6 +491,11 @@ extern "C" int launch_linear_mid(const unsigned short* x,
         if (M <= 224) LM_GO(2, 7, 4, 2, 1, 4, 3, F);                          \
         LM_GO(2, 8, 4, 2, 1, 4, 3, F);                                        \
     } while (0)
+#define LM_APART(F)                                                           \
+    do {                                                                      \
+        if (M <= 192) LM_SUMS(2, 6, 4, 2, 1, 4, 4, F, true);                  \
+        LM_SUMS(2, 7, 4, 2, 1, 4, 3, F, true);                                \
+    } while (0)
 #define LM_SCALED(TW, MW, WN, WM, WK, DW, DX)                                 \
     do {                                                                      \
         constexpr int lds =                                                   \
@@ -497,7 +520,13 @@ extern "C" int launch_linear_mid(const unsigned short* x,
         if (M <= 128) LM_GO(3, 4, 4, 2, 1, 4, 3, LM_GATED);
         LM_GO(3, 5, 4, 2, 1, 4, 3, LM_GATED);
     }
+    // Sums of all of K in one chain are half as far off again (parts of 4096x14336 from
+    // 64 bits 2.5e-7 of their norm, in two chains 1.7e-7); where registers allow it they
+    // are two. us, one chain / two, at 192 rows: 4096x14336 33.7 / 34.8, 2x14336x4096 58.2
+    // / 58.7; 224: 36.4 / 36.7, 65.9 / 63.7.
+    const bool apart = tiles > 4 && once && M > 160 && M <= 224;
     if (form == LM_GATED && tiles <= 4) LM_4(LM_GATED);
+    if (form == LM_GATED && apart) LM_APART(LM_GATED);
     if (form == LM_GATED) LM_8(LM_GATED);
     if (form == LM_ROWS && tiles <= 4) LM_4(LM_ROWS);
     // (half the input: 128256x4096 168 -> 155 us at 1 row with the places of K,
@@ -505,10 +534,13 @@ extern "C" int launch_linear_mid(const unsigned short* x,
     if (form == LM_ROWS && M <= 16) LM_GO(1, 1, 8, 1, 1, 4, 6, LM_ROWS);
     if (form == LM_ROWS) LM_8(LM_ROWS);
     if (tiles <= 4) LM_4(LM_PARTS);
+    if (apart) LM_APART(LM_PARTS);
     LM_8(LM_PARTS);
 #undef LM_SCALED
+#undef LM_APART
 #undef LM_8
 #undef LM_4
+#undef LM_SUMS
 #undef LM_GO
     return 1;
 }

@@ -278,6 +278,23 @@ def test_activated_rows(M, N, K, act):
             + 1e-6).all()
 
 
+# (five to eight tiles a workgroup)
+@pytest.mark.parametrize("N,K,act", [
+    (4096, 14336, None), (6144, 2048, None), (3588, 4160, None),
+    (14336, 512, "swiglu"), (9000, 320, "swiglu")])
+def test_sums_of_k_in_halves(N, K, act):
+    """161 to 224 rows sum K in two chains as 65 to 96 do: a row is the same to the
+    bit among them."""
+    torch.manual_seed(N)
+    x = _rand(224, K)
+    w = _rand(2 * N if act else N, K, std=0.05)
+    run = (lambda rows: ops.mid_rows_linear(x[:rows], w, None, act)) if act else (
+        lambda rows: ops.mid_linear(x[:rows], w))
+    want = run(96)
+    for rows in (161, 192, 193, 224):
+        assert torch.equal(run(rows)[..., :96, :], want)
+
+
 # (tiles a workgroup: six, the last of 12 columns, fewer steps of K than the rings
 # have slots; five and a second group, more steps; eight, and in the last workgroup
 # one; eight and a second group)
