@@ -26,9 +26,10 @@
 // without, 36.8 with; 4096x14336 24.8 / 22.2). Rows of 128 bytes in LDS are xor-ed by
 // half their number: no two of a read's 16 rows meet in a bank. Workgroups start at
 // different places of K: in step they would all ask for the same few channels
-// (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 -> 44.5 at 80). Those of output heads,
-// which go round by round, are 5 steps apart and not one: 128256x4096 167 -> 159 us
-// at 24 rows, 193 -> 188 at 80 (gated 2 to 4% slower so, others the same). The rings
+// (2x14336x4096 44.8 -> 41.3 us at 24 rows, 53 -> 44.5 at 80). Rows of more than four
+// tiles a workgroup, which output heads are, start 5 steps apart and not one:
+// 128256x4096 167 -> 159 us at 24 rows, 193 -> 188 at 80, 32000x4096 43.5 -> 41.8 at
+// 24, 32000x2048 23.6 -> 22.6 (gated 2 to 4% slower so, others the same). The rings
 // of up to 8 tiles hold what covers the memory's latency and no more: four slots of
 // weights, 32 KB up to 4 tiles and 64 above. With all of LDS for weights every CU
 // asks for 100 KB at once, and the input that the first step waits for queues behind
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(512) void linear_mid_kernel(
     const int CH = K / 64;                     // steps of 64: of them
     const int c0 = CH * blockIdx.y / S, n = CH * (blockIdx.y + 1) / S - c0;
     // where it starts
-    const int rot = blockIdx.x / 8 * (OUT == LM_ROWS ? 5 : 1) % n;
+    const int rot = blockIdx.x / 8 * (OUT == LM_ROWS && tiles > 4 ? 5 : 1) % n;
     int g = blockIdx.x;
     const int total = n * ((NG - 1 - g) / (int)gridDim.x + 1);
     extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -295,6 +295,18 @@ def test_sums_of_k_in_halves(N, K, act):
         assert torch.equal(run(rows)[..., :96, :], want)
 
 
+@pytest.mark.parametrize("M", [1, 17, 57, 129, 256])
+@pytest.mark.parametrize("N,K", [(8192, 704), (3588, 640), (512, 320)])
+def test_rows_are_parts_rounded(N, K, M):
+    """Rows of narrow projections (tails of many rows, gelu) and their parts, of
+    which these have one, sum K in the same order."""
+    torch.manual_seed(N + M)
+    x, w = _rand(M, K), _rand(N, K, std=0.1)
+    parts = ops.mid_linear(x, w)
+    assert parts.shape[0] == 1
+    assert torch.equal(ops.mid_rows_linear(x, w), parts[0].bfloat16())
+
+
 # (tiles a workgroup: six, the last of 12 columns, fewer steps of K than the rings
 # have slots; five and a second group, more steps; eight, and in the last workgroup
 # one; eight and a second group)
